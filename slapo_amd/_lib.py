@@ -1,7 +1,8 @@
-"""ctypes binding of libslapo_amd.so (the C ABI declared in include/slapo_amd.h).
+"""Loaders of the native pieces: the ctypes binding of libslapo_amd.so (the C ABI declared in
+include/slapo_amd.h) and `host()`, the extension module that the ops call.
 
-The library is loaded lazily on first use and never built at import time.  If it is missing
-the loader raises: there is no eager / CPU substitute for the kernels in this package.
+Both are loaded lazily on first use and never built at import time.  If one is missing the loader
+raises: there is no eager / CPU substitute for the kernels in this package.
 """
 from __future__ import annotations
 
@@ -177,6 +178,25 @@ def load():
             fn.argtypes = argtypes
         _lib = lib
     return _lib
+
+
+_host = None
+
+
+def host():
+    """The extension module behind the ops (csrc/host_ops.cpp).  Raises if it is not built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError(
+                "slapo_amd/_host.so is missing or was built for another torch: build it with "
+                f"`python -m slapo_amd.build` ({e})"
+            ) from e
+        _host = module
+    return _host
 
 
 def check(status: int, what: str):

@@ -1,7 +1,9 @@
-"""Build recipe for libslapo_amd.so: hipcc cross-compiles every csrc/*.hip for gfx950.
+"""Build recipe of the two native pieces: libslapo_amd.so (hipcc cross-compiles every csrc/*.hip
+for gfx950) and the extension module _host.so (g++ compiles csrc/host_ops.cpp against torch's
+headers; it calls the kernels through the C ABI of the library beside it).
 
-The library is built in-tree (slapo_amd/libslapo_amd.so) so that it travels with the source
-tree; nothing is compiled at import time.  `python -m slapo_amd.build` rebuilds it.
+Both are built in-tree (slapo_amd/) so that they travel with the source tree; nothing is compiled
+at import time.  `python -m slapo_amd.build` rebuilds them.
 """
 from __future__ import annotations
 
@@ -10,11 +12,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(PKG_DIR, "csrc")
 OBJ_DIR = os.path.join(CSRC_DIR, "build")
 LIB_PATH = os.path.join(PKG_DIR, "libslapo_amd.so")
+HOST_PATH = os.path.join(PKG_DIR, "_host.so")
 
 ARCH = "gfx950"
 
@@ -74,14 +78,46 @@ def _compile_one(src: str, extra: list[str]) -> str:
     return obj
 
 
+def _compile_host() -> str:
+    """Object file of the extension module: host code only, no device pass."""
+    from torch.utils.cpp_extension import include_paths
+
+    obj = os.path.join(OBJ_DIR, "host_ops.o")
+    dirs = [*include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM", *[f for d in dirs for f in ("-isystem", d)], "-c",
+           os.path.join(CSRC_DIR, "host_ops.cpp"), "-o", obj]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed for host_ops.cpp:\n{proc.stdout}\n{proc.stderr}")
+    return obj
+
+
+def _link_host(obj: str) -> str:
+    """torch's libraries are loaded by `import torch` before the module is; libslapo_amd.so is found
+    beside it."""
+    from torch.utils.cpp_extension import library_paths
+
+    tmp = HOST_PATH + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, obj, f"-L{PKG_DIR}", "-lslapo_amd",
+           *[f"-L{d}" for d in library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu",
+           "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, HOST_PATH)
+    return HOST_PATH
+
+
 def build_library(verbose: bool = False, extra_flags: list[str] | None = None) -> str:
-    """Compile all kernels and link the shared library; always recompiles."""
+    """Compile all kernels and the host module and link both; always recompiles."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     extra = list(extra_flags or [])
     srcs = sources()
     if verbose:
         print(f"[slapo_amd.build] compiling {len(srcs)} files for {ARCH}", flush=True)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=8) as pool:
+        host_obj = pool.submit(_compile_host)
         objs = list(pool.map(lambda s: _compile_one(s, extra), srcs))
     tmp = LIB_PATH + ".tmp"
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
@@ -89,8 +125,9 @@ def build_library(verbose: bool = False, extra_flags: list[str] | None = None) -
     if proc.returncode != 0:
         raise RuntimeError(f"link failed:\n{proc.stdout}\n{proc.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_host(host_obj.result())
     if verbose:
-        print(f"[slapo_amd.build] wrote {LIB_PATH}", flush=True)
+        print(f"[slapo_amd.build] wrote {LIB_PATH} and {HOST_PATH}", flush=True)
     return LIB_PATH
 
 

@@ -1,0 +1,813 @@
+// Host path of the ops: argument checks, output / workspace allocation, kernel launches through the
+// C ABI and the autograd nodes, as a CPython extension module (slapo_amd/_host.so).
+//
+// Why native: a training step calls these ops hundreds of times and most calls are shorter than the
+// host work around them.  With torch.autograd.Function and ctypes a forward + backward pair cost
+// 100-175 us of Python on the launching and the engine thread whatever the kernels took (fp16
+// 1537 x 768 bias + dropout + residual + LayerNorm: 175-187 us per pair against 22 us of kernels).
+// The nodes here derive from torch::autograd::Node directly: the backward runs on the engine's
+// thread without the interpreter lock, and a call allocates its outputs and nothing else.
+//
+// Nothing in this file computes: every number comes from a kernel behind include/slapo_amd.h.
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/grad_mode.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/pybind.h>
+
+#include <ATen/ATen.h>
+#include <ATen/core/Generator.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
+#include <c10/hip/HIPStream.h>
+
+#include <cstring>
+#include <mutex>
+
+#include "../../include/slapo_amd.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::Node;
+using torch::autograd::SavedVariable;
+using torch::autograd::variable_list;
+
+// ---- errors -------------------------------------------------------------------------------------
+
+// A negative status of the C ABI becomes the exception that slapo_amd._lib.check raises.
+void check(int status, const char* what) {
+    if (status == SLAPO_OK) return;
+    const std::string text = std::string(what) + " failed: " + slapo_amd_status_string(status) +
+                             " (status " + std::to_string(status) + ")";
+    if (status >= SLAPO_ERR_ARG) TORCH_CHECK_VALUE(false, text);
+    pybind11::gil_scoped_acquire gil;
+    PyObject* mod = PyImport_ImportModule("slapo_amd._lib");
+    PyObject* cls = mod ? PyObject_GetAttrString(mod, "SlapoAmdError") : nullptr;
+    if (cls) PyErr_SetString(cls, text.c_str());
+    Py_XDECREF(cls);
+    Py_XDECREF(mod);
+    python_error err;
+    err.persist();
+    throw std::move(err);
+}
+
+void require_device(std::initializer_list<const Tensor*> tensors) {
+    for (const Tensor* t : tensors)
+        if (t->defined() && !t->is_cuda())
+            TORCH_CHECK(false,
+                        "slapo_amd kernels run on a gfx950 device only; got a tensor on '",
+                        t->device().str(),
+                        "'.  There is no CPU implementation in this package.");
+}
+
+// Tangents of forward-mode differentiation would be dropped without a word: refuse them, as
+// torch.autograd.Function does for a function without `jvp`.
+void refuse_tangents(std::initializer_list<const Tensor*> tensors) {
+    for (const Tensor* t : tensors)
+        if (t->defined() && t->_fw_grad(0).defined())
+            TORCH_CHECK(false, "slapo_amd ops do not implement forward-mode differentiation");
+}
+
+int dtype_code(at::ScalarType t) {
+    switch (t) {
+        case at::kFloat: return SLAPO_F32;
+        case at::kHalf: return SLAPO_F16;
+        case at::kBFloat16: return SLAPO_BF16;
+        default:
+            TORCH_CHECK_VALUE(false, "unsupported dtype ", t,
+                              "; expected float32, float16 or bfloat16");
+    }
+}
+
+// ---- small helpers ------------------------------------------------------------------------------
+
+void* stream_of(const Tensor& t) {
+    return c10::hip::getCurrentHIPStream(t.device().index()).stream();
+}
+bool capturing() {
+    return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
+
+const void* cptr(const Tensor& t) { return t.defined() ? t.const_data_ptr() : nullptr; }
+void* mptr(const Tensor& t) { return t.defined() ? t.mutable_data_ptr() : nullptr; }
+bool aligned(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15) == 0; }
+
+Tensor floats(int64_t n, const Tensor& like) {
+    return at::empty({n > 0 ? n : 1}, like.options().dtype(at::kFloat));
+}
+
+Tensor cast(const Tensor& t, at::ScalarType dt) {
+    return !t.defined() || t.scalar_type() == dt ? t : t.to(dt);
+}
+// contiguous and of dtype `dt`
+Tensor dense(const Tensor& t, at::ScalarType dt) {
+    return t.defined() ? cast(t.contiguous(), dt) : t;
+}
+
+SavedVariable keep(const Tensor& t, bool is_output = false) {
+    return t.defined() ? SavedVariable(t, is_output) : SavedVariable();
+}
+
+// Dropout of one call: probability, the (seed, offset) pair drawn for it -- by value, or in the
+// device memory of `state` while a graph is being captured -- and the launch plan.
+struct Dropout {
+    double p = 0.0;
+    uint64_t seed = 0, offset = 0;
+    Tensor state;
+    slapo_dropout_plan plan = {};
+
+    const slapo_dropout_plan* plan_ptr() const { return p > 0.0 ? &plan : nullptr; }
+    void set_plan(int64_t numel, int elem_bytes, const at::Device& dev) {
+        if (!(p > 0.0)) return;
+        check(slapo_amd_dropout_plan(numel, elem_bytes, 256, dev.index(), &plan),
+              "slapo_amd_dropout_plan");
+        if (state.defined()) {
+            TORCH_CHECK_VALUE(
+                state.is_cuda() && state.numel() == 2 && state.is_contiguous() &&
+                    (state.scalar_type() == at::kLong || state.scalar_type() == at::kUInt64),
+                "rng_state must be a contiguous device tensor of two 64-bit integers");
+            plan.rng_state = state.const_data_ptr();
+        }
+    }
+};
+
+template <typename T, typename... Inputs>
+std::shared_ptr<T> make_node(bool wanted, const Inputs&... inputs) {
+    if (!wanted) return nullptr;
+    std::shared_ptr<T> node(new T(), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(inputs...));
+    return node;
+}
+
+// ---- attention ----------------------------------------------------------------------------------
+
+// Four-dimensional [batch, seqlen, heads, head_dim] operand as the kernels address it.
+struct Operand {
+    Tensor t;
+    int64_t strides[3];
+
+    void take(const Tensor& in) {
+        t = in;
+        const auto st = t.strides();
+        bool usable = t.size(3) <= 1 || st[3] == 1;
+        if (usable) {
+            const int64_t esz = t.element_size();
+            usable = aligned(t) && st[0] * esz % 16 == 0 && st[1] * esz % 16 == 0 &&
+                     st[2] * esz % 16 == 0;
+        }
+        if (!usable) t = t.contiguous();
+        const auto s2 = t.strides();
+        strides[0] = s2[0], strides[1] = s2[1], strides[2] = s2[2];
+    }
+};
+
+struct AttnProblem {
+    slapo_attn_params prm = {};
+    Tensor bias;  // fp32, addressed with prm.bias_strides (0 on broadcast dims)
+    Dropout drop;
+    at::ScalarType dtype = at::kFloat;
+
+    int64_t b() const { return prm.batch; }
+    int64_t h() const { return prm.heads; }
+    int64_t sq() const { return prm.seqlen_q; }
+    int64_t sk() const { return prm.seqlen_k; }
+    int64_t d() const { return prm.head_dim; }
+    bool empty() const { return b() * h() * sq() * d() == 0; }
+
+    void describe(const Tensor& q, const Tensor& k, bool causal, int64_t window, double scale) {
+        dtype = q.scalar_type();
+        prm.dtype = dtype_code(dtype);
+        prm.batch = (int32_t)q.size(0);
+        prm.seqlen_q = (int32_t)q.size(1);
+        prm.heads = (int32_t)q.size(2);
+        prm.head_dim = (int32_t)q.size(3);
+        prm.seqlen_k = (int32_t)k.size(1);
+        prm.causal = causal ? 1 : 0;
+        prm.window = (int32_t)window;
+        prm.scale = (float)scale;
+    }
+    // Additive mask -> fp32, broadcast dims with stride 0.
+    void set_bias(const Tensor& mask) {
+        if (!mask.defined()) return;
+        TORCH_CHECK_VALUE(mask.dim() == 4,
+                          "attention_mask must be 4-D ([B,1,1,Sk] or [B,H,Sq,Sk])");
+        bias = cast(mask, at::kFloat);
+        const int64_t want[4] = {b(), h(), sq(), sk()};
+        for (int i = 0; i < 4; ++i) {
+            const int64_t n = bias.size(i);
+            TORCH_CHECK(n == want[i] || n == 1, "attention_mask of shape ", mask.sizes(),
+                        " does not broadcast to [", b(), ", ", h(), ", ", sq(), ", ", sk(), "]");
+            prm.bias_strides[i] = n == 1 && want[i] != 1 ? 0 : bias.stride(i);
+        }
+    }
+    // Draws, once the geometry is known: F.dropout leaves the generator alone for an empty tensor.
+    void set_dropout(Dropout&& in, const at::Device& dev) {
+        drop = std::move(in);
+        const int64_t scores = b() * h() * sq() * sk();
+        if (scores == 0) drop.p = 0.0;
+        drop.set_plan(scores, 4, dev);
+        prm.p_drop = (float)drop.p;
+        prm.seed = drop.seed;
+        prm.offset = drop.offset;
+        if (drop.p > 0.0) prm.plan = drop.plan;
+    }
+};
+
+void check_operands(const Tensor& q, const Tensor& k, const Tensor& v) {
+    TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4 && v.dim() == 4,
+                      "q, k, v must be [batch, seqlen, heads, head_dim]");
+    TORCH_CHECK_VALUE(k.sizes() == v.sizes() && q.size(0) == k.size(0) && q.size(2) == k.size(2) &&
+                          q.size(3) == k.size(3),
+                      "inconsistent q/k/v shapes ", q.sizes(), " ", k.sizes(), " ", v.sizes());
+    TORCH_CHECK_VALUE(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(),
+                      "q, k, v must share a dtype");
+    require_device({&q, &k, &v});
+}
+
+struct AttnResult {
+    Tensor out, lse, keep_mask;
+};
+
+AttnResult launch_attn_fwd(AttnProblem& a, const Tensor& q, const Tensor& k, const Tensor& v,
+                           bool save_mask, int64_t save_mask_max) {
+    AttnResult r;
+    slapo_attn_params& prm = a.prm;
+    r.out = at::empty({a.b(), a.sq(), a.h(), a.d()}, q.options());
+    r.lse = at::empty({a.b(), a.h(), a.sq()}, q.options().dtype(at::kFloat));
+    prm.o_strides[0] = a.sq() * a.h() * a.d();
+    prm.o_strides[1] = a.h() * a.d();
+    prm.o_strides[2] = a.d();
+    if (a.empty()) return r;
+    if (save_mask) {
+        const int64_t bytes = (int64_t)slapo_amd_attn_keep_mask_bytes(&prm);
+        if (bytes > 0 && bytes <= save_mask_max) {
+            r.keep_mask = at::empty({bytes / 4}, q.options().dtype(at::kInt));
+            prm.keep_mask = r.keep_mask.mutable_data_ptr();
+        }
+    }
+    check(slapo_amd_attn_fwd(&prm, cptr(q), cptr(k), cptr(v),
+                             static_cast<const float*>(cptr(a.bias)), mptr(r.out),
+                             static_cast<float*>(mptr(r.lse)), stream_of(q)),
+          "slapo_amd_attn_fwd");
+    return r;
+}
+
+// dq / dk / dv: destinations with their three outer strides.
+void launch_attn_bwd(AttnProblem& a, const Tensor& q, const Tensor& k, const Tensor& v,
+                     const Tensor& out, const Tensor& lse, const Tensor& keep_mask,
+                     const Tensor& grad, const Tensor (&dst)[3], const int64_t (&ds)[3][3]) {
+    Tensor dout = grad.scalar_type() == a.dtype ? grad.contiguous()
+                                                : grad.to(a.dtype).contiguous();
+    if (!aligned(dout)) dout = dout.clone();
+    a.prm.keep_mask = mptr(keep_mask);
+    const size_t ws_bytes = slapo_amd_attn_bwd_workspace_bytes(&a.prm);
+    const Tensor ws = floats((int64_t)(ws_bytes / 4), q);
+    check(slapo_amd_attn_bwd(&a.prm, cptr(q), cptr(k), cptr(v),
+                             static_cast<const float*>(cptr(a.bias)), cptr(out), cptr(dout),
+                             static_cast<const float*>(cptr(lse)), mptr(dst[0]), mptr(dst[1]),
+                             mptr(dst[2]), ds[0], ds[1], ds[2], mptr(ws), ws_bytes, stream_of(q)),
+          "slapo_amd_attn_bwd");
+}
+
+// Forward saves q, k, v, bias, out, lse, the (seed, offset) pair and, with dropout, the keep bits;
+// the backward recomputes the probabilities from lse and reads (or regenerates) the dropout mask --
+// it never draws.
+struct AttnBackward : Node {
+    AttnProblem a;
+    SavedVariable q, k, v, bias, out, lse, keep_mask, state;
+
+    std::string name() const override { return "HipAttentionBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (SavedVariable* s : {&q, &k, &v, &bias, &out, &lse, &keep_mask, &state})
+            s->reset_data();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list res(3);
+        if (!grads[0].defined()) return res;
+        const Tensor tq = q.unpack(), tk = k.unpack(), tv = v.unpack();
+        const Tensor tout = out.unpack(getptr()), tlse = lse.unpack();
+        AttnProblem call = a;
+        call.bias = bias.unpack();
+        call.drop.state = state.unpack();
+        if (call.drop.state.defined()) call.prm.plan.rng_state = call.drop.state.const_data_ptr();
+        const c10::OptionalDeviceGuard guard(tq.device());
+        const Tensor dst[3] = {at::empty(tq.sizes(), tq.options()),
+                               at::empty(tk.sizes(), tk.options()),
+                               at::empty(tv.sizes(), tv.options())};
+        if (dst[0].numel() == 0 || dst[1].numel() == 0) {
+            for (const Tensor& t : dst) t.zero_();
+        } else {
+            int64_t ds[3][3];
+            for (int i = 0; i < 3; ++i)
+                for (int j = 0; j < 3; ++j) ds[i][j] = dst[i].stride(j);
+            launch_attn_bwd(call, tq, tk, tv, tout, tlse, keep_mask.unpack(), grads[0], dst, ds);
+        }
+        for (int i = 0; i < 3; ++i)
+            if (task_should_compute_output(i)) res[i] = dst[i];
+        return res;
+    }
+};
+
+Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask,
+                 bool causal, int64_t window, std::optional<double> scale, Dropout&& drop,
+                 bool save_mask, int64_t save_mask_max) {
+    check_operands(q, k, v);
+    require_device({&mask});
+    refuse_tangents({&q, &k, &v});
+    const bool need = torch::autograd::compute_requires_grad(q, k, v);
+    auto node = make_node<AttnBackward>(need, q, k, v);
+    AttnProblem a;
+    AttnResult r;
+    Operand oq, ok, ov;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(q.device());
+        a.describe(q, k, causal, window,
+                   scale ? *scale : 1.0 / std::sqrt((double)q.size(3)));
+        oq.take(q), ok.take(k), ov.take(v);
+        std::memcpy(a.prm.q_strides, oq.strides, sizeof oq.strides);
+        std::memcpy(a.prm.k_strides, ok.strides, sizeof ok.strides);
+        std::memcpy(a.prm.v_strides, ov.strides, sizeof ov.strides);
+        a.set_bias(mask);
+        a.set_dropout(std::move(drop), q.device());
+        r = launch_attn_fwd(a, oq.t, ok.t, ov.t, save_mask && need && a.drop.p < 1.0,
+                            save_mask_max);
+    }
+    if (node) {
+        torch::autograd::set_history(r.out, node);
+        node->q = keep(oq.t), node->k = keep(ok.t), node->v = keep(ov.t);
+        node->bias = keep(a.bias), node->lse = keep(r.lse), node->keep_mask = keep(r.keep_mask);
+        node->state = keep(a.drop.state);
+        node->out = keep(r.out, true);
+        a.bias = Tensor(), a.drop.state = Tensor();
+        node->a = a;
+    }
+    return r.out;
+}
+
+// ---- bias + GeLU --------------------------------------------------------------------------------
+
+// rows x cols of x, with a bias of shape [cols]
+std::pair<int64_t, int64_t> rows_cols(const Tensor& x, const Tensor& bias) {
+    TORCH_CHECK_VALUE(x.dim() > 0, "the input needs at least one dimension");
+    const int64_t cols = x.size(-1);
+    TORCH_CHECK_VALUE(!bias.defined() || (bias.dim() == 1 && bias.size(0) == cols),
+                      "bias must have shape [", cols, "], got ", bias.sizes());
+    return {cols > 0 ? x.numel() / cols : 0, cols};
+}
+
+Tensor colsum_workspace(int64_t rows, int64_t cols, const Tensor& like, size_t* bytes) {
+    *bytes = slapo_amd_colsum_workspace_bytes(rows, cols);
+    return floats((int64_t)(*bytes / 4), like);
+}
+
+struct BiasGeluBackward : Node {
+    SavedVariable y, bias;
+    at::ScalarType bias_dtype = at::kFloat;
+
+    std::string name() const override { return "HipBiasGeLUBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        y.reset_data(), bias.reset_data();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list res(2);
+        if (!grads[0].defined()) return res;
+        const bool need_bias = task_should_compute_output(1);
+        const Tensor ty = y.unpack(), tb = bias.unpack();
+        const c10::OptionalDeviceGuard guard(ty.device());
+        const Tensor g = dense(grads[0], ty.scalar_type());
+        const auto [rows, cols] = rows_cols(ty, tb);
+        Tensor dx = at::empty_like(ty), db, ws;
+        if (need_bias) db = at::empty({cols}, ty.options());
+        if (ty.numel() == 0) {
+            if (need_bias) db.zero_();
+        } else {
+            size_t ws_bytes = 0;
+            if (need_bias) ws = colsum_workspace(rows, cols, ty, &ws_bytes);
+            check(slapo_amd_bias_gelu_bwd(cptr(g), cptr(ty), cptr(tb), mptr(dx), mptr(db), mptr(ws),
+                                          ws_bytes, rows, cols, dtype_code(ty.scalar_type()),
+                                          stream_of(ty)),
+                  "slapo_amd_bias_gelu_bwd");
+        }
+        if (task_should_compute_output(0)) res[0] = dx;
+        if (need_bias) res[1] = cast(db, bias_dtype);
+        return res;
+    }
+};
+
+// gelu_tanh(inp + bias); without a bias (an undefined tensor) a row of zeros stands in
+Tensor bias_gelu(const Tensor& inp, const Tensor& bias_in) {
+    require_device({&inp, &bias_in});
+    refuse_tangents({&inp, &bias_in});
+    auto node = make_node<BiasGeluBackward>(
+        torch::autograd::compute_requires_grad(inp, bias_in), inp, bias_in);
+    Tensor y, bias, out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(inp.device());
+        const auto [rows, cols] = rows_cols(inp, bias_in);
+        y = inp.contiguous();
+        bias = bias_in.defined() ? dense(bias_in, y.scalar_type()) : at::zeros({cols}, y.options());
+        out = at::empty_like(y);
+        const int code = dtype_code(y.scalar_type());
+        if (y.numel() != 0)
+            check(slapo_amd_bias_gelu_fwd(cptr(y), cptr(bias), mptr(out), rows, cols, code,
+                                          stream_of(y)),
+                  "slapo_amd_bias_gelu_fwd");
+    }
+    if (node) {
+        torch::autograd::set_history(out, node);
+        node->y = keep(y), node->bias = keep(bias);
+        node->bias_dtype = bias_in.defined() ? bias_in.scalar_type() : y.scalar_type();
+    }
+    return out;
+}
+
+// ---- bias + dropout (+ residual) ----------------------------------------------------------------
+
+struct BiasDropoutBackward : Node {
+    Dropout drop;
+    SavedVariable state;
+    at::ScalarType bias_dtype = at::kFloat;
+    bool has_residual = false;
+
+    std::string name() const override { return "HipBiasDropoutResidualBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        state.reset_data();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list res(3);
+        if (!grads[0].defined()) return res;
+        const bool need_x = task_should_compute_output(0), need_bias = task_should_compute_output(1);
+        if (has_residual && task_should_compute_output(2)) res[2] = grads[0];
+        // without dropout the gradient of x is the incoming one: only its column sum is left to do
+        const bool pass_x = drop.p == 0.0;
+        if (need_x && pass_x) res[0] = grads[0];
+        const bool write_x = need_x && !pass_x;
+        if (!write_x && !need_bias) return res;
+        const c10::OptionalDeviceGuard guard(grads[0].device());
+        const Tensor g = grads[0].contiguous();
+        const auto [rows, cols] = rows_cols(g, Tensor());
+        Tensor dx, db, ws;
+        if (write_x) dx = at::empty_like(g);
+        if (need_bias) db = at::empty({cols}, g.options());
+        if (g.numel() == 0) {
+            if (need_bias) db.zero_();
+        } else {
+            Dropout d = drop;
+            d.state = state.unpack();
+            if (d.state.defined()) d.plan.rng_state = d.state.const_data_ptr();
+            size_t ws_bytes = 0;
+            if (need_bias) ws = colsum_workspace(rows, cols, g, &ws_bytes);
+            check(slapo_amd_bias_dropout_residual_bwd(
+                      cptr(g), mptr(dx), mptr(db), mptr(ws), ws_bytes, rows, cols,
+                      dtype_code(g.scalar_type()), d.p, d.seed, d.offset, d.plan_ptr(),
+                      stream_of(g)),
+                  "slapo_amd_bias_dropout_residual_bwd");
+        }
+        if (write_x) res[0] = dx;
+        if (need_bias) res[1] = cast(db, bias_dtype);
+        return res;
+    }
+};
+
+Tensor bias_dropout_residual(const Tensor& x_in, const Tensor& bias_in, const Tensor& res_in,
+                             Dropout&& drop) {
+    require_device({&x_in, &bias_in, &res_in});
+    refuse_tangents({&x_in, &bias_in, &res_in});
+    TORCH_CHECK_VALUE(!res_in.defined() || res_in.sizes() == x_in.sizes(),
+                      "residual must have the shape of x");
+    auto node = make_node<BiasDropoutBackward>(
+        torch::autograd::compute_requires_grad(x_in, bias_in, res_in), x_in, bias_in, res_in);
+    Tensor out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(x_in.device());
+        const auto [rows, cols] = rows_cols(x_in, bias_in);
+        const Tensor x = x_in.contiguous();
+        const at::ScalarType dt = x.scalar_type();
+        const Tensor bias = dense(bias_in, dt), res = dense(res_in, dt);
+        const int code = dtype_code(dt);
+        out = at::empty_like(x);
+        if (x.numel() == 0) drop.p = 0.0;
+        drop.set_plan(x.numel(), (int)x.element_size(), x.device());
+        if (x.numel() != 0)
+            check(slapo_amd_bias_dropout_residual_fwd(
+                      cptr(x), cptr(bias), cptr(res), mptr(out), rows, cols, code, drop.p,
+                      drop.seed, drop.offset, drop.plan_ptr(), stream_of(x)),
+                  "slapo_amd_bias_dropout_residual_fwd");
+    }
+    if (node) {
+        torch::autograd::set_history(out, node);
+        node->state = keep(drop.state);
+        drop.state = Tensor();
+        node->drop = drop;
+        node->bias_dtype = bias_in.scalar_type();
+        node->has_residual = res_in.defined();
+    }
+    return out;
+}
+
+// ---- bias + dropout + residual + LayerNorm ------------------------------------------------------
+
+struct LayerNormBackward : Node {
+    Dropout drop;
+    SavedVariable z, stats, weight, state;  // stats: mean and rstd, [2, rows]
+    at::ScalarType dtypes[3];               // bias, weight, ln_bias
+    bool has_bias = false, has_residual = false;
+
+    std::string name() const override { return "HipBiasDropoutResidualLayerNormBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (SavedVariable* s : {&z, &stats, &weight, &state}) s->reset_data();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list res(5);  // x, bias, residual, weight, ln_bias
+        if (!grads[0].defined()) return res;
+        const Tensor tz = z.unpack(), tstats = stats.unpack(), tw = weight.unpack();
+        const c10::OptionalDeviceGuard guard(tz.device());
+        const at::ScalarType dt = tz.scalar_type();
+        const Tensor g = dense(grads[0], dt);
+        const auto [rows, cols] = rows_cols(tz, Tensor());
+        const bool need[5] = {task_should_compute_output(0),
+                              has_bias && task_should_compute_output(1),
+                              has_residual && task_should_compute_output(2),
+                              task_should_compute_output(3), task_should_compute_output(4)};
+        Tensor dx, dres, vec[3];  // vec: dbias, dweight, dln_bias
+        // without dropout dx and dresidual are the same values: one tensor serves both
+        const bool same = drop.p == 0.0 && need[0] && need[2];
+        if (need[0]) dx = at::empty_like(tz);
+        if (need[2] && !same) dres = at::empty_like(tz);
+        const bool need_vec[3] = {need[1], need[3], need[4]};
+        for (int i = 0; i < 3; ++i)
+            if (need_vec[i]) vec[i] = at::empty({cols}, tz.options());
+        if (tz.numel() == 0) {
+            for (Tensor& t : vec)
+                if (t.defined()) t.zero_();
+        } else if (need[0] || need[1] || need[2] || need[3] || need[4]) {
+            Dropout d = drop;
+            d.state = state.unpack();
+            if (d.state.defined()) d.plan.rng_state = d.state.const_data_ptr();
+            Tensor ws;
+            size_t ws_bytes = 0;
+            if (need[1] || need[3] || need[4]) {
+                ws_bytes = slapo_amd_ln_bwd_workspace_bytes(rows, cols);
+                ws = floats((int64_t)(ws_bytes / 4), tz);
+            }
+            const float* mean = static_cast<const float*>(cptr(tstats));
+            check(slapo_amd_bias_dropout_residual_ln_bwd(
+                      cptr(g), cptr(tz), mean, mean + rows, cptr(tw), mptr(dx), mptr(dres),
+                      mptr(vec[1]), mptr(vec[2]), mptr(vec[0]), mptr(ws), ws_bytes, rows, cols,
+                      dtype_code(dt), d.p, d.seed, d.offset, d.plan_ptr(), stream_of(tz)),
+                  "slapo_amd_bias_dropout_residual_ln_bwd");
+        }
+        res[0] = dx;
+        res[1] = cast(vec[0], dtypes[0]);
+        res[2] = same ? dx : dres;
+        res[3] = cast(vec[1], dtypes[1]);
+        res[4] = cast(vec[2], dtypes[2]);
+        return res;
+    }
+};
+
+Tensor bias_dropout_residual_layer_norm(const Tensor& x_in, const Tensor& bias_in,
+                                        const Tensor& res_in, const Tensor& weight_in,
+                                        const Tensor& ln_bias_in, double eps, Dropout&& drop) {
+    require_device({&x_in, &bias_in, &res_in, &weight_in, &ln_bias_in});
+    refuse_tangents({&x_in, &bias_in, &res_in, &weight_in, &ln_bias_in});
+    TORCH_CHECK_VALUE(!res_in.defined() || res_in.sizes() == x_in.sizes(),
+                      "residual must have the shape of x");
+    for (const Tensor* t : {&bias_in, &weight_in, &ln_bias_in})
+        TORCH_CHECK_VALUE(
+            !t->defined() || (t->dim() == 1 && x_in.dim() > 0 && t->size(0) == x_in.size(-1)),
+            "bias, weight and ln_bias must be 1-D of the last dimension of x");
+    const bool need = torch::autograd::compute_requires_grad(x_in, bias_in, res_in, weight_in,
+                                                             ln_bias_in);
+    auto node =
+        make_node<LayerNormBackward>(need, x_in, bias_in, res_in, weight_in, ln_bias_in);
+    Tensor y, z, stats, weight;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(x_in.device());
+        const auto [rows, cols] = rows_cols(x_in, Tensor());
+        const Tensor x = x_in.contiguous();
+        const at::ScalarType dt = x.scalar_type();
+        const Tensor bias = dense(bias_in, dt), res = dense(res_in, dt);
+        weight = dense(weight_in, dt);
+        const Tensor ln_bias = dense(ln_bias_in, dt);
+        const int code = dtype_code(dt);
+        y = at::empty_like(x);
+        if (need) {
+            z = at::empty_like(x);
+            stats = floats(2 * rows, x);
+        }
+        if (x.numel() == 0) drop.p = 0.0;
+        drop.set_plan(x.numel(), (int)x.element_size(), x.device());
+        float* mean = static_cast<float*>(mptr(stats));
+        if (x.numel() != 0)
+            check(slapo_amd_bias_dropout_residual_ln_fwd(
+                      cptr(x), cptr(bias), cptr(res), cptr(weight), cptr(ln_bias), mptr(z),
+                      mptr(y), mean, mean ? mean + rows : nullptr, rows, cols, code, eps, drop.p,
+                      drop.seed, drop.offset, drop.plan_ptr(), stream_of(x)),
+                  "slapo_amd_bias_dropout_residual_ln_fwd");
+    }
+    if (node) {
+        torch::autograd::set_history(y, node);
+        node->z = keep(z), node->stats = keep(stats), node->weight = keep(weight);
+        node->state = keep(drop.state);
+        drop.state = Tensor();
+        node->drop = drop;
+        node->has_bias = bias_in.defined(), node->has_residual = res_in.defined();
+        node->dtypes[0] = bias_in.defined() ? bias_in.scalar_type() : at::kFloat;
+        node->dtypes[1] = weight_in.scalar_type();
+        node->dtypes[2] = ln_bias_in.scalar_type();
+    }
+    return y;
+}
+
+// ---- random numbers -----------------------------------------------------------------------------
+
+// (seed, offset) for one launch from the default generator of device `index`, whose offset moves
+// on by `increment`, as an ATen random kernel would have it.
+std::pair<uint64_t, uint64_t> draw(int64_t increment, c10::DeviceIndex index) {
+    at::Generator gen = at::globalContext().defaultGenerator(at::Device(at::kCUDA, index));
+    std::lock_guard<std::mutex> lock(gen.mutex());
+    const uint64_t seed = gen.current_seed(), offset = gen.get_offset();
+    gen.set_offset(offset + (uint64_t)increment);
+    return {seed, offset};
+}
+
+// ---- Python -------------------------------------------------------------------------------------
+
+const Tensor& tensor_arg(PyObject* o, const char* name) {
+    TORCH_CHECK_TYPE(THPVariable_Check(o), name, " must be a tensor, got ", Py_TYPE(o)->tp_name);
+    return THPVariable_Unpack(o);
+}
+const Tensor& optional_tensor_arg(PyObject* o, const char* name) {
+    static const Tensor none;
+    return o == Py_None ? none : tensor_arg(o, name);
+}
+double double_arg(PyObject* o) {
+    const double v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) throw python_error();
+    return v;
+}
+int64_t int_arg(PyObject* o) {
+    const long long v = PyLong_AsLongLong(o);
+    if (v == -1 && PyErr_Occurred()) throw python_error();
+    return v;
+}
+uint64_t uint_arg(PyObject* o) {
+    const unsigned long long v = PyLong_AsUnsignedLongLong(o);
+    if (v == (unsigned long long)-1 && PyErr_Occurred()) throw python_error();
+    return v;
+}
+bool bool_arg(PyObject* o) {
+    const int v = PyObject_IsTrue(o);
+    if (v < 0) throw python_error();
+    return v != 0;
+}
+// p, seed, offset, state
+Dropout dropout_args(PyObject* const* a) {
+    Dropout d;
+    d.p = double_arg(a[0]);
+    d.seed = uint_arg(a[1]);
+    d.offset = uint_arg(a[2]);
+    d.state = optional_tensor_arg(a[3], "rng_state");
+    return d;
+}
+void want(Py_ssize_t n, Py_ssize_t expected, const char* name) {
+    TORCH_CHECK_TYPE(n == expected, name, " takes ", expected, " arguments, got ", n);
+}
+
+// attention(q, k, v, mask, causal, window, scale, p, seed, offset, state, save_mask, save_max)
+PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 13, "attention");
+    const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v");
+    const Tensor& mask = optional_tensor_arg(a[3], "attention_mask");
+    const bool causal = bool_arg(a[4]), save_mask = bool_arg(a[11]);
+    const int64_t window = int_arg(a[5]), save_max = int_arg(a[12]);
+    std::optional<double> scale;
+    if (a[6] != Py_None) scale = double_arg(a[6]);
+    Dropout drop = dropout_args(a + 7);
+    Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = attention(q, k, v, mask, causal, window, scale, std::move(drop), save_mask, save_max);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// attention_scores(q, k, v): checks the operands, returns the number of scores B * H * Sq * Sk
+PyObject* py_attention_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 3, "attention_scores");
+    const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v");
+    check_operands(q, k, v);
+    return PyLong_FromLongLong(q.size(0) * q.size(1) * q.size(2) * k.size(1));
+    END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_bias_gelu(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 2, "bias_gelu");
+    const Tensor& x = tensor_arg(a[0], "inp");
+    const Tensor& bias = optional_tensor_arg(a[1], "bias");
+    Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = bias_gelu(x, bias);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// bias_dropout_residual(x, bias, residual, p, seed, offset, state)
+PyObject* py_bias_dropout_residual(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 7, "bias_dropout_residual");
+    const Tensor &x = tensor_arg(a[0], "x"), &bias = tensor_arg(a[1], "bias");
+    const Tensor& residual = optional_tensor_arg(a[2], "residual");
+    Dropout drop = dropout_args(a + 3);
+    Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = bias_dropout_residual(x, bias, residual, std::move(drop));
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// bias_dropout_residual_layer_norm(x, bias, residual, weight, ln_bias, eps, p, seed, offset, state)
+PyObject* py_layer_norm(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 10, "bias_dropout_residual_layer_norm");
+    const Tensor& x = tensor_arg(a[0], "x");
+    const Tensor& bias = optional_tensor_arg(a[1], "bias");
+    const Tensor& residual = optional_tensor_arg(a[2], "residual");
+    const Tensor &weight = tensor_arg(a[3], "weight"), &ln_bias = tensor_arg(a[4], "ln_bias");
+    const double eps = double_arg(a[5]);
+    Dropout drop = dropout_args(a + 6);
+    Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = bias_dropout_residual_layer_norm(x, bias, residual, weight, ln_bias, eps,
+                                               std::move(drop));
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// philox_increment(numel, elem_bytes, device_index): how far F.dropout would advance the generator
+PyObject* py_philox_increment(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 3, "philox_increment");
+    slapo_dropout_plan plan;
+    check(slapo_amd_dropout_plan(int_arg(a[0]), (int)int_arg(a[1]), 256, (int)int_arg(a[2]), &plan),
+          "slapo_amd_dropout_plan");
+    return PyLong_FromLongLong(plan.offset_increment);
+    END_HANDLE_TH_ERRORS
+}
+
+// draw(increment, device_index): (seed, offset), or None while the current stream is capturing
+PyObject* py_draw(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 2, "draw");
+    const int64_t increment = int_arg(a[0]), index = int_arg(a[1]);
+    if (capturing()) Py_RETURN_NONE;
+    const auto [seed, offset] = draw(increment, (c10::DeviceIndex)index);
+    return Py_BuildValue("KK", (unsigned long long)seed, (unsigned long long)offset);
+    END_HANDLE_TH_ERRORS
+}
+
+#define SLAPO_METHOD(name, fn) \
+    { name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr }
+PyMethodDef methods[] = {
+    SLAPO_METHOD("attention", py_attention),
+    SLAPO_METHOD("attention_scores", py_attention_scores),
+    SLAPO_METHOD("bias_gelu", py_bias_gelu),
+    SLAPO_METHOD("bias_dropout_residual", py_bias_dropout_residual),
+    SLAPO_METHOD("bias_dropout_residual_layer_norm", py_layer_norm),
+    SLAPO_METHOD("philox_increment", py_philox_increment),
+    SLAPO_METHOD("draw", py_draw),
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_host",
+                          "Native host path of the slapo_amd ops", -1, methods,
+                          nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&module_def); }

@@ -51,10 +51,23 @@ extern "C" int slapo_amd_dropout_plan_for(int64_t numel, int elem_bytes, int64_t
 
 extern "C" int slapo_amd_dropout_plan(int64_t numel, int elem_bytes, int64_t ptr_align,
                                       int device, slapo_dropout_plan* plan) {
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) != hipSuccess) return SLAPO_ERR_DEVICE;
-    return slapo_amd_dropout_plan_for(numel, elem_bytes, ptr_align, prop.multiProcessorCount,
-                                      prop.maxThreadsPerMultiProcessor, plan);
+    // The two properties of a device are asked once (the query is slow beside a launch) and kept as
+    // one word: compute units in the upper half, threads per unit in the lower.
+    static std::atomic<uint64_t> known[64];
+    const bool cached = device >= 0 && device < 64;
+    uint64_t dims = cached ? known[device].load(std::memory_order_relaxed) : 0;
+    if (dims == 0) {
+        int cus = 0, threads = 0;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) !=
+                hipSuccess ||
+            hipDeviceGetAttribute(&threads, hipDeviceAttributeMaxThreadsPerMultiProcessor,
+                                  device) != hipSuccess)
+            return SLAPO_ERR_DEVICE;
+        dims = ((uint64_t)(uint32_t)cus << 32) | (uint32_t)threads;
+        if (cached) known[device].store(dims, std::memory_order_relaxed);
+    }
+    return slapo_amd_dropout_plan_for(numel, elem_bytes, ptr_align, (int)(dims >> 32),
+                                      (int)(uint32_t)dims, plan);
 }
 
 static inline float uniform_of(uint32_t v) {

@@ -1,5 +1,7 @@
-"""Tensor-level wrappers over the C ABI: argument checking, output/workspace allocation with
-torch's caching allocator, stream selection.  No arithmetic happens here."""
+"""Launch-level wrappers over the C ABI for direct use of single kernels, with an explicit (seed,
+offset) pair and explicit intermediate results (tests, benchmarks, the cross entropy): argument
+checking, output / workspace allocation with torch's caching allocator, stream selection.  No
+arithmetic happens here.  The ops go through csrc/host_ops.cpp instead."""
 from __future__ import annotations
 
 import ctypes
@@ -20,8 +22,7 @@ def _require_device(*tensors):
             )
 
 
-# The wrappers below sit on the critical path of every training step, so the per-call host work
-# is kept small: raw stream and data pointers as plain integers (ctypes converts them through the
+# Per-call host work is kept small: raw stream and data pointers as plain integers (ctypes converts them through the
 # declared argtypes), a device switch only when the tensor lives on another device than the
 # current one, and parameter structs cached per problem geometry.
 def _stream():

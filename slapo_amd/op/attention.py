@@ -28,9 +28,9 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from .._lib import host
 from ..random import draw_philox  # noqa: F401  (kept importable from here for direct launches)
 from ..random import draw_philox_state
-from . import _kernels as K
 from .fused_bias import bias_dropout
 
 logger = logging.getLogger("slapo_amd")
@@ -57,64 +57,24 @@ SAVE_DROPOUT_MASK = True
 SAVE_DROPOUT_MASK_MAX_BYTES = 512 << 20
 
 
-class _HipAttention(torch.autograd.Function):
-    """Forward saves (q, k, v, bias, out, lse), the Philox (seed, offset) and, with dropout, the
-    keep bits; backward recomputes the probabilities from lse and reads (or regenerates) the
-    dropout mask -- it never draws."""
-
-    # pylint: disable=arguments-differ, abstract-method
-    @staticmethod
-    def forward(ctx, q, k, v, bias, causal, window, scale, p):
-        b, sq, h, _ = q.shape
-        sk = k.shape[1]
-        plan, seed, offset, rng_state = None, 0, 0, None
-        if b * h * sq * sk == 0:
-            p = 0.0  # nothing to drop, and F.dropout leaves the generator alone for an empty tensor
-        if p > 0.0:
-            plan = K.dropout_plan(b * h * sq * sk, 4, q.device)
-            if p < 1.0:
-                seed, offset, rng_state = draw_philox_state(plan.offset_increment, q.device)
-        save_mask = SAVE_DROPOUT_MASK and 0.0 < p < 1.0 and any(ctx.needs_input_grad[:3])
-        if save_mask:
-            mask_bytes = b * h * ((sk + 31) // 32) * ((sq + 3) // 4 * 4) * 4
-            save_mask = mask_bytes <= SAVE_DROPOUT_MASK_MAX_BYTES
-        out, lse, (q, k, v), keep_mask = K.attn_fwd(q, k, v, bias, causal, window, scale, p, seed,
-                                                    offset, plan, save_mask=save_mask,
-                                                    rng_state=rng_state)
-        ctx.save_for_backward(q, k, v, bias, out, lse, keep_mask, rng_state)
-        ctx.cfg = (causal, window, scale, p, seed, offset, plan)
-        return out
-
-    @staticmethod
-    def backward(ctx, dout):
-        q, k, v, bias, out, lse, keep_mask, rng_state = ctx.saved_tensors
-        causal, window, scale, p, seed, offset, plan = ctx.cfg
-        dq, dk, dv = K.attn_bwd(dout, q, k, v, bias, out, lse, causal, window, scale, p, seed,
-                                offset, plan, keep_mask, rng_state)
-        return dq, dk, dv, None, None, None, None, None
-
-
 def hip_attention(q, k, v, attention_mask=None, causal=False, p=0.0, scale=None, window=0):
     """q, k, v: [B, S, H, D] (head_dim contiguous; outer dims may be strided views).
     attention_mask: additive, 4-D, broadcastable to [B, H, Sq, Sk].  Returns [B, Sq, H, D]."""
-    if q.ndim != 4 or k.ndim != 4 or v.ndim != 4:
-        raise ValueError("q, k, v must be [batch, seqlen, heads, head_dim]")
-    if k.shape != v.shape or q.shape[0] != k.shape[0] or q.shape[2:] != k.shape[2:]:
-        raise ValueError(f"inconsistent q/k/v shapes {tuple(q.shape)} {tuple(k.shape)} "
-                         f"{tuple(v.shape)}")
-    if not (q.dtype == k.dtype == v.dtype):
-        raise ValueError("q, k, v must share a dtype")
-    if p < 0.0 or p > 1.0:
-        raise ValueError(f"dropout probability has to be between 0 and 1, but got {p}")
-    b, sq, h, d = q.shape
-    bias = None
-    if attention_mask is not None:
-        if attention_mask.requires_grad:
-            warning_once("WARNING: bias gradient is not supported yet. "
-                         "The mask is applied but receives no gradient")
-        bias = K.prepare_bias(attention_mask.detach(), b, h, sq, k.shape[1])
-    scale = float(scale) if scale is not None else float(d) ** -0.5
-    return _HipAttention.apply(q, k, v, bias, bool(causal), int(window or 0), scale, float(p))
+    native = host()
+    seed, offset, rng_state = 0, 0, None
+    if p != 0.0:
+        if not 0.0 <= p <= 1.0:
+            raise ValueError(f"dropout probability has to be between 0 and 1, but got {p}")
+        scores = native.attention_scores(q, k, v)
+        # nothing is drawn for p = 1, nor for an empty tensor (F.dropout leaves the generator alone)
+        if p < 1.0 and scores:
+            seed, offset, rng_state = draw_philox_state(
+                native.philox_increment(scores, 4, q.device.index), q.device)
+    if attention_mask is not None and attention_mask.requires_grad:
+        warning_once("WARNING: bias gradient is not supported yet. "
+                     "The mask is applied but receives no gradient")
+    return native.attention(q, k, v, attention_mask, causal, window or 0, scale, p, seed, offset,
+                            rng_state, SAVE_DROPOUT_MASK, SAVE_DROPOUT_MASK_MAX_BYTES)
 
 
 class FlashAttentionOp(nn.Module):
@@ -156,10 +116,9 @@ class FlashAttentionOp(nn.Module):
         self.bias_layout = "b11k"
 
     def forward(self, query_layer, key_layer, value_layer, attention_mask, p):
-        ret = self.attn_fn(query_layer, key_layer, value_layer, attention_mask,
-                           causal=self.apply_causal_mask, p=p, scale=self.scale,
-                           window=self.window or 0)
-        return ret.to(query_layer.dtype)
+        return self.attn_fn(query_layer, key_layer, value_layer, attention_mask,
+                            causal=self.apply_causal_mask, p=p, scale=self.scale,
+                            window=self.window or 0)
 
     def extra_repr(self):
         return (f"attn_op_name={self.attn_op_name}, causal={self.apply_causal_mask}, "

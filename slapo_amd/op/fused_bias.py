@@ -12,93 +12,42 @@ from __future__ import annotations
 import torch
 from torch import nn
 
+from .._lib import host
 from ..random import draw_philox_state
-from . import _kernels as K
-
-
-class BiasGeLUFunction(torch.autograd.Function):
-    """gelu_tanh(inp + bias); backward is the closed form of fused_bias.py:26-34 and returns the
-    bias gradient already reduced to the bias shape."""
-
-    # pylint: disable=arguments-differ, abstract-method
-    @staticmethod
-    def forward(ctx, inp, bias):
-        ctx.save_for_backward(inp, bias)
-        return K.bias_gelu_fwd(inp, bias)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        inp, bias = ctx.saved_tensors
-        dx, dbias = K.bias_gelu_bwd(grad_output, inp, bias, need_dbias=ctx.needs_input_grad[1])
-        if dbias is not None and dbias.dtype != bias.dtype:
-            dbias = dbias.to(bias.dtype)
-        return (dx if ctx.needs_input_grad[0] else None), dbias
 
 
 def bias_gelu(inp: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
-    return BiasGeLUFunction.apply(inp, bias)
+    """gelu_tanh(inp + bias); backward is the closed form of fused_bias.py:26-34 and returns the
+    bias gradient already reduced to the bias shape."""
+    return host().bias_gelu(inp, bias)
 
 
-class _NewGeLU(torch.autograd.Function):
-    """The same kernels with a zero bias and no bias gradient."""
+class BiasGeLUFunction(torch.autograd.Function):
+    """The reference's name for `bias_gelu`: `BiasGeLUFunction.apply(inp, bias)`."""
 
-    # pylint: disable=arguments-differ, abstract-method
-    @staticmethod
-    def forward(ctx, inp):
-        zero = inp.new_zeros(inp.shape[-1])
-        ctx.save_for_backward(inp, zero)
-        return K.bias_gelu_fwd(inp, zero)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        inp, zero = ctx.saved_tensors
-        dx, _ = K.bias_gelu_bwd(grad_output, inp, zero, need_dbias=False)
-        return dx
+    # pylint: disable=abstract-method
+    apply = staticmethod(bias_gelu)
 
 
 def new_gelu(inp: torch.Tensor) -> torch.Tensor:
     """HF `gelu_new` (fused_bias.py:49-60) as one kernel per direction."""
-    return _NewGeLU.apply(inp)
+    return host().bias_gelu(inp, None)
 
 
 def bias_new_gelu(inp: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     """HF `gelu_new` on inp + bias.  Its constant sqrt(2/pi) equals the 0.79788456 of
     `BiasGeLUFunction` to 8 digits, so both names share one kernel."""
-    return BiasGeLUFunction.apply(inp, bias)
+    return bias_gelu(inp, bias)
 
 
-class _BiasDropoutResidual(torch.autograd.Function):
-    # pylint: disable=arguments-differ, abstract-method
-    @staticmethod
-    def forward(ctx, x, bias, residual, p):
-        plan, seed, offset, rng_state = None, 0, 0, None
-        if x.numel() == 0:
-            p = 0.0  # nothing to drop, and F.dropout leaves the generator alone for an empty tensor
-        if 0.0 < p:
-            plan = K.dropout_plan(x.numel(), x.element_size(), x.device)
-            if p < 1.0:
-                # The generator moves exactly as it would for F.dropout on this tensor.
-                seed, offset, rng_state = draw_philox_state(plan.offset_increment, x.device)
-        ctx.p, ctx.seed, ctx.offset, ctx.plan = p, seed, offset, plan
-        ctx.rng_state = rng_state  # a non-differentiable two-element tensor, or None
-        ctx.bias_like = bias
-        ctx.has_residual = residual is not None
-        return K.bias_dropout_residual_fwd(x, bias, residual, p, seed, offset, plan,
-                                           rng_state=rng_state)
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        need_dx, need_dbias = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
-        dx = dbias = None
-        if need_dx or need_dbias:
-            if ctx.p == 0.0 and not need_dbias:
-                dx = grad_output
-            else:
-                dx, dbias = K.bias_dropout_residual_bwd(
-                    grad_output, ctx.bias_like, ctx.p, ctx.seed, ctx.offset, ctx.plan,
-                    need_dx=need_dx, need_dbias=need_dbias, rng_state=ctx.rng_state)
-        dres = grad_output if (ctx.has_residual and ctx.needs_input_grad[2]) else None
-        return dx, dbias, dres, None
+def _draw(x, p):
+    """(seed, offset, state) of the mask F.dropout(x, p) would draw; the generator moves exactly as
+    it would there.  Nothing is drawn for p of 0 or 1, nor for an empty tensor."""
+    n = x.numel()
+    if not 0.0 < p < 1.0 or n == 0 or not x.is_cuda:
+        return 0, 0, None
+    return draw_philox_state(host().philox_increment(n, x.element_size(), x.device.index),
+                             x.device)
 
 
 def bias_dropout(x: torch.Tensor, bias: torch.Tensor, p: float = 0.5, training: bool = True,
@@ -107,50 +56,16 @@ def bias_dropout(x: torch.Tensor, bias: torch.Tensor, p: float = 0.5, training: 
     in-place target is the temporary x + bias, which this kernel never materialises."""
     del inplace
     _check_p(p)
-    return _BiasDropoutResidual.apply(x, bias, None, float(p) if training else 0.0)
+    p = p if training else 0.0
+    return host().bias_dropout_residual(x, bias, None, p, *_draw(x, p))
 
 
 def bias_dropout_residual(x: torch.Tensor, bias: torch.Tensor, residual: torch.Tensor,
                           p: float = 0.5, training: bool = True) -> torch.Tensor:
     """dropout(x + bias) + residual, the pattern of tests/test_fusion.py:179-180."""
     _check_p(p)
-    return _BiasDropoutResidual.apply(x, bias, residual, float(p) if training else 0.0)
-
-
-class _BiasDropoutResidualLayerNorm(torch.autograd.Function):
-    # pylint: disable=arguments-differ, abstract-method
-    @staticmethod
-    def forward(ctx, x, bias, residual, weight, ln_bias, p, eps):
-        plan, seed, offset, rng_state = None, 0, 0, None
-        if x.numel() == 0:
-            p = 0.0  # nothing to drop, and F.dropout leaves the generator alone for an empty tensor
-        if 0.0 < p:
-            plan = K.dropout_plan(x.numel(), x.element_size(), x.device)
-            if p < 1.0:
-                # The generator moves exactly as it would for F.dropout on this tensor.
-                seed, offset, rng_state = draw_philox_state(plan.offset_increment, x.device)
-        need_grad = any(ctx.needs_input_grad[:5])
-        y, z, mean, rstd = K.bias_dropout_residual_ln_fwd(
-            x, bias, residual, weight, ln_bias, eps, p, seed, offset, plan,
-            save_for_backward=need_grad, rng_state=rng_state)
-        ctx.rng_state = rng_state  # a non-differentiable two-element tensor, or None
-        ctx.cfg = (p, seed, offset, plan, bias is not None, residual is not None)
-        ctx.dtypes = tuple(t.dtype if t is not None else None for t in (bias, weight, ln_bias))
-        ctx.save_for_backward(z, mean, rstd, weight)
-        return y
-
-    @staticmethod
-    def backward(ctx, grad_output):
-        z, mean, rstd, weight = ctx.saved_tensors
-        p, seed, offset, plan, has_bias, has_residual = ctx.cfg
-        need = ctx.needs_input_grad
-        dx, dres, dw, dlb, db = K.bias_dropout_residual_ln_bwd(
-            grad_output, z, mean, rstd, weight, p, seed, offset, plan, need_dx=need[0],
-            need_dres=has_residual and need[2], need_dweight=need[3], need_dln_bias=need[4],
-            need_dbias=has_bias and need[1], rng_state=ctx.rng_state)
-        cast = lambda t, dt: t if t is None or t.dtype == dt else t.to(dt)
-        return (dx, cast(db, ctx.dtypes[0]), dres, cast(dw, ctx.dtypes[1]),
-                cast(dlb, ctx.dtypes[2]), None, None)
+    p = p if training else 0.0
+    return host().bias_dropout_residual(x, bias, residual, p, *_draw(x, p))
 
 
 def bias_dropout_residual_layer_norm(x: torch.Tensor, bias, residual, weight: torch.Tensor,
@@ -159,8 +74,9 @@ def bias_dropout_residual_layer_norm(x: torch.Tensor, bias, residual, weight: to
     """layer_norm(dropout(x + bias) + residual) over the last dimension, the pattern of
     tests/test_fusion.py:184-185 (bias and residual may be None)."""
     _check_p(p)
-    return _BiasDropoutResidualLayerNorm.apply(x, bias, residual, weight, ln_bias,
-                                               float(p) if training else 0.0, float(eps))
+    p = p if training else 0.0
+    return host().bias_dropout_residual_layer_norm(x, bias, residual, weight, ln_bias, eps, p,
+                                                   *_draw(x, p))
 
 
 def _check_p(p):
@@ -172,7 +88,7 @@ class HipBiasGeLU(nn.Module):
     """Replacement payload for a matched `gelu(x + bias)` subgraph."""
 
     def forward(self, x, bias):
-        return BiasGeLUFunction.apply(x, bias)
+        return bias_gelu(x, bias)
 
 
 class HipBiasDropoutResidual(nn.Module):

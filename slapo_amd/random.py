@@ -19,6 +19,8 @@ import random as _py_random
 import numpy as np
 import torch
 
+from ._lib import host
+
 _MODEL_PARALLEL_RNG_TRACKER_NAME = "model-parallel-rng"
 
 
@@ -132,24 +134,27 @@ def set_random_seed(seed=2013, dp_rank=None, pp_rank=None, tp_rank=None,
     return seed
 
 
+def _draw(offset_increment: int, device):
+    """(seed, offset), or None while the current stream is being captured into a graph."""
+    if offset_increment % 4 != 0:
+        raise ValueError("Philox offset increments are multiples of 4")
+    idx = None if device is None else torch.device(device).index
+    return host().draw(offset_increment, torch.cuda.current_device() if idx is None else idx)
+
+
 def draw_philox(offset_increment: int, device=None):
     """Take (seed, offset) for one kernel launch from the device's default generator and advance
     its offset by `offset_increment` (a multiple of 4), exactly as an ATen random kernel would.
     Must be called from forward only; backward re-uses the pair saved in the autograd context."""
-    if offset_increment % 4 != 0:
-        raise ValueError("Philox offset increments are multiples of 4")
-    if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
+    pair = _draw(offset_increment, device)
+    if pair is None:
         # The pair is read on the host and baked into the launch: a captured graph would replay
         # one and the same mask.  `draw_philox_state` is the capturable form.
         raise RuntimeError(
             "slapo_amd: draw_philox reads (seed, offset) from the device generator on the host "
             "and cannot be captured into a graph; use draw_philox_state"
         )
-    gen = DeviceGeneratorBackend._gen(device)
-    seed = gen.initial_seed()
-    offset = gen.get_offset()
-    gen.set_offset(offset + offset_increment)
-    return seed, offset
+    return pair
 
 
 def draw_philox_state(offset_increment: int, device=None):
@@ -164,11 +169,8 @@ def draw_philox_state(offset_increment: int, device=None):
     seed and offset are 0 and unused.  A replay's mask is then a function of the generator's
     state at that replay -- fresh per replay, repeatable after `torch.cuda.manual_seed` -- though
     not the mask an eager call would draw from the same state."""
-    if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
-        if offset_increment % 4 != 0:
-            raise ValueError("Philox offset increments are multiples of 4")
+    pair = _draw(offset_increment, device)
+    if pair is None:
         dev = torch.device("cuda", torch.cuda.current_device()) if device is None else device
-        state = torch.randint(0, 2 ** 62, (2,), dtype=torch.int64, device=dev)
-        return 0, 0, state
-    seed, offset = draw_philox(offset_increment, device)
-    return seed, offset, None
+        return 0, 0, torch.randint(0, 2 ** 62, (2,), dtype=torch.int64, device=dev)
+    return pair[0], pair[1], None
