@@ -77,7 +77,10 @@ __global__ __launch_bounds__(256) void attn_delta_scalar_kernel(const AttnArgs a
 // hold does not matter and they are left as they are.  With a local window the grid's second
 // dimension counts words from the first one of the row's window (window / 32 + 1 of them, not
 // seqlen_k / 32: every thread then has a word to draw); without one it is the word itself.
-// kExact: any launch geometry of the dropout plan and any seqlen_k (one Philox block per bit).
+// kExact: any launch geometry of the dropout plan and any seqlen_k (dropout_keep32).  Drawn per
+// word this costs 9 Philox blocks per 32 scores where the forward kernel, whose lanes hold single
+// groups of four, drew one block per score: bf16 B3 S777 H12 D64 without a causal mask, p 0.1,
+// forward 147 us before, @MASK_US@ us with this kernel ahead of it.
 template <bool kExact>
 __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in) {
     AttnArgs a = a_in;
@@ -88,19 +91,22 @@ __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in) {
     int w = blockIdx.y;
     if (a.window > 0) w += max(i - a.window + 1, 0) >> 5;
     if (w >= a.mask_words) return;
-    if (a.causal && 32 * w > i) return;
-    if (a.window > 0 && i - (32 * w + 31) >= a.window) return;
+    if (a.window > 0) {
+        if (a.causal && 32 * w > i) return;
+        if (i - (32 * w + 31) >= a.window) return;
+    } else if (a.causal && 64 * (w >> 1) > (i | 31)) {
+        return;  // (without a window: every word of a 64-key tile that the row's group visits)
+    }
     const uint64_t row_base = ((uint64_t)bh * a.sq + (uint64_t)i) * (uint64_t)a.sk;
     uint32_t word = 0;
+    if constexpr (kExact) {
+        word = dropout_keep32(a.rng, row_base + 32 * (uint64_t)w);
+    } else {
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk) {
-        const int key0 = 32 * w + 4 * blk;
-        if (key0 < a.sk) {
-            const uint64_t e0 = row_base + (uint64_t)key0;
-            if constexpr (kExact)
-                word |= dropout_keep_any(a.rng, e0, min(4, a.sk - key0)) << (4 * blk);
-            else
-                word |= dropout_keep4_pow2(a.rng, e0 >> 2) << (4 * blk);
+        for (int blk = 0; blk < 8; ++blk) {
+            const int key0 = 32 * w + 4 * blk;
+            if (key0 < a.sk)
+                word |= dropout_keep4_pow2(a.rng, (row_base + (uint64_t)key0) >> 2) << (4 * blk);
         }
     }
     a.keep_mask[((int64_t)bh * a.mask_words + w) * a.mask_pitch + i] = word;
@@ -238,10 +244,11 @@ extern "C" int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, c
     hipStream_t st = (hipStream_t)stream;
     if (prm->dtype == SLAPO_F32) return attn_fwd_f32(a, st);
     if (!half_ptrs_ok({q, k, v, o})) return SLAPO_ERR_ALIGN;
-    if (a.dropout && a.keep_mask && a.window > 0 && keep_mask_kernel_fits(a)) {
-        // Local window with a buffer for the keep bits: draw them first, the forward kernel
-        // then reads them like the backward kernels do (bf16 B4 S2048 H16 D128, window 256,
-        // p 0.1: 88 against 127 us).  Without a window the forward draws them itself and
+    if (a.dropout && a.keep_mask && (a.window > 0 || a.dropout == 2) && keep_mask_kernel_fits(a)) {
+        // Local window, or a mask geometry without whole Philox blocks per aligned group of keys,
+        // with a buffer for the keep bits: draw them first, the forward kernel then reads them
+        // like the backward kernels do (bf16 B4 S2048 H16 D128, window 256, p 0.1: 88 against 127
+        // us; the geometry: see keep_mask_kernel).  Otherwise the forward draws them itself and
         // stores them as it goes: there the Philox arithmetic overlaps the matrix instructions
         // and a separate pass measured slower (239 against 199 us at the same shape, 116
         // against 87 us at fp16 B8 S1024 H16 D64).

@@ -139,8 +139,10 @@ __global__ __launch_bounds__(kThreads, (DPAD <= 64 && kDrop == 0 ? 3 : 2)) void 
     // keep bits, and gain 9 % at head_dim 128 where the kernel draws its dropout bits (bf16 B4
     // S2048 H16 causal, p 0.1: 209 -> 190 us): that build has the most live registers, and the
     // subtractions' operands are what it no longer keeps.  Only that build uses it.  (Builds with
-    // a bias could not: the masking value -FLT_MAX is no number of T.)
-    constexpr bool kRefInMma = kBias == 0 && (kDrop == 1 || kDrop == 2) && kWin == 0 && DPAD > 96;
+    // a bias could not: the masking value -FLT_MAX is no number of T; and the build for the other mask
+    // geometries rounds as the one that reads stored bits does, which stands in for it wherever
+    // there is a buffer for them.)
+    constexpr bool kRefInMma = kBias == 0 && kDrop == 1 && kWin == 0 && DPAD > 96;
     constexpr float kRefUnit = std::is_same<T, f16_t>::value ? 64.f : 1.f;
     frag_t ones_frag, ref_frag;
 #pragma unroll
@@ -538,12 +540,7 @@ template <typename T, int DPAD, int kWin, int kSteps>
 int dispatch_nobias(const AttnArgs& a, hipStream_t st) {
     if (a.dropout == 1) return launch<T, DPAD, 0, 1, kWin, kSteps>(a, st);
     if (a.dropout == 2) return launch<T, DPAD, 0, 2, kWin, kSteps>(a, st);
-    if (a.dropout == 3) {  // stored keep bits: local-window calls only, see attn_capi.hip
-        if constexpr (kWin != 0)
-            return launch<T, DPAD, 0, 3, kWin, kSteps>(a, st);
-        else
-            return SLAPO_ERR_ARG;
-    }
+    if (a.dropout == 3) return launch<T, DPAD, 0, 3, kWin, kSteps>(a, st);
     return launch<T, DPAD, 0, 0, kWin, kSteps>(a, st);
 }
 template <typename T, int DPAD, int kSteps = DPAD / 16>

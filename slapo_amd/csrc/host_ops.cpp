@@ -335,8 +335,14 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor
         std::memcpy(a.prm.v_strides, ov.strides, sizeof ov.strides);
         a.set_bias(mask);
         a.set_dropout(std::move(drop), q.device());
-        r = launch_attn_fwd(a, oq.t, ok.t, ov.t, save_mask && need && a.drop.p < 1.0,
-                            save_mask_max);
+        // a mask geometry that the forward kernel would draw score by score is drawn ahead of it,
+        // which takes the buffer also where no backward will read it
+        const slapo_dropout_plan& plan = a.drop.plan;
+        const bool per_score = a.drop.p > 0.0 &&
+                               (plan.vec < 4 || a.sk() % 4 != 0 ||
+                                (plan.total_threads & (plan.total_threads - 1)) != 0);
+        r = launch_attn_fwd(a, oq.t, ok.t, ov.t,
+                            save_mask && a.drop.p < 1.0 && (need || per_score), save_mask_max);
     }
     if (node) {
         torch::autograd::set_history(r.out, node);

@@ -166,6 +166,39 @@ SLAPO_HD uint32_t dropout_keep4_pow2(const DropoutState& s, uint64_t group) {
            (keep_word(s, r.z) ? 4u : 0u) | (keep_word(s, r.w) ? 8u : 0u);
 }
 
+// Keep-bits of the 32 consecutive elements starting at elem (bit j <-> element elem + j), for any
+// thread count and alignment and vec <= 4 (the plan of a 4-byte tensor).  The element -> (thread,
+// trip) split costs a division where the thread count is no power of two: it is taken once and
+// stepped from there.  A Philox block serves `vec` of the elements: 9 blocks at vec 4 (8 where the
+// run is aligned), 17 at vec 2, 32 at vec 1.
+SLAPO_HD uint32_t dropout_keep32(const DropoutState& s, uint64_t elem) {
+    const uint32_t shift = s.vec == 4 ? 2u : s.vec == 2 ? 1u : 0u;
+    uint64_t thread, trip;
+    const uint64_t v = elem >> shift;
+    if (((v | s.total_threads) >> 32) == 0 && s.t_shift < 0) {
+        const uint32_t q = (uint32_t)v / (uint32_t)s.total_threads;
+        trip = q;
+        thread = (uint32_t)v - q * (uint32_t)s.total_threads;
+    } else {
+        split_by_threads(s, v, thread, trip);
+    }
+    const int skip = (int)(elem & ((1u << shift) - 1u));  // elements of the first block before elem
+    uint32_t bits = 0;
+#if defined(__HIPCC__)
+#pragma unroll 1
+#endif
+    for (int at = -skip; at < 32; at += 1 << shift) {
+        const u32x4 r = philox_block(s, thread, shift ? trip : trip >> 2);
+        uint32_t four = (keep_word(s, r.x) ? 1u : 0u) | (keep_word(s, r.y) ? 2u : 0u) |
+                        (keep_word(s, r.z) ? 4u : 0u) | (keep_word(s, r.w) ? 8u : 0u);
+        if (shift == 0) four = (four >> (trip & 3)) & 1u;
+        if (shift == 1) four &= 3u;
+        bits |= at < 0 ? four >> -at : four << at;
+        if (++thread == s.total_threads) thread = 0, ++trip;
+    }
+    return bits;
+}
+
 // Keep-bits of the n (1..4) consecutive elements starting at elem, for any launch geometry and
 // alignment.  Deliberately a rolled loop: this path is rare and must stay small.
 SLAPO_HD uint32_t dropout_keep_any(const DropoutState& s, uint64_t elem, int n) {
