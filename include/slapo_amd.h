@@ -257,6 +257,15 @@ size_t slapo_amd_attn_keep_mask_bytes(const slapo_attn_params* prm);
 int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* k, const void* v,
                        const float* bias, void* o, float* lse, void* stream);
 
+/* The same call with a workspace (16-byte aligned, slapo_amd_attn_fwd_workspace_bytes of it, may be
+ * NULL where that is 0): with one query per sequence and no dropout the keys of a (batch, head) are
+ * shared by several workgroups, whose partial results meet there.  Without it such a call runs with
+ * one workgroup per (batch, head). */
+size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm);
+int slapo_amd_attn_fwd_ws(const slapo_attn_params* prm, const void* q, const void* k,
+                          const void* v, const float* bias, void* o, float* lse, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* Workspace (bytes) the backward needs: fp32 delta = rowsum(dO * O), one value per query row. */
 size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* prm);
 

@@ -127,6 +127,11 @@ PROTOTYPES = {
     "slapo_amd_attn_fwd": (
         ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]
     ),
+    "slapo_amd_attn_fwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
+    "slapo_amd_attn_fwd_ws": (
+        ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
+                       ctypes.c_size_t, c_vp]
+    ),
     "slapo_amd_attn_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
     "slapo_amd_attn_keep_mask_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
     "slapo_amd_attn_bwd": (

@@ -14,6 +14,8 @@ int attn_bwd_dq_mfma_bf16(const AttnArgs& a, hipStream_t st);
 int attn_fwd_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_f32(const AttnArgs& a, hipStream_t st);
+int attn_decode_shares(int64_t n_bh, int n_keys);
+int attn_decode(const AttnArgs& a, int dtype, int n_shares, float* part, hipStream_t st);
 }  // namespace slapo
 
 using namespace slapo;
@@ -186,18 +188,47 @@ extern "C" size_t slapo_amd_attn_keep_mask_bytes(const slapo_attn_params* p) {
     return (size_t)p->batch * p->heads * words * sizeof(uint32_t);
 }
 
-extern "C" int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* k,
-                                  const void* v, const float* bias, void* o, float* lse,
-                                  void* stream) {
+namespace {
+
+// One query per sequence without dropout: attn_decode.hip.  How many workgroups share the keys of one
+// (batch, head), 0 where that kernel does not apply.
+int decode_shares(const slapo_attn_params* p) {
+    if (!p || p->seqlen_q != 1 || p->p_drop > 0.f || p->batch <= 0 || p->heads <= 0 ||
+        p->seqlen_k <= 0)
+        return 0;
+    return attn_decode_shares((int64_t)p->batch * p->heads, p->causal ? 1 : p->seqlen_k);
+}
+
+}  // namespace
+
+extern "C" size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm) {
+    const int shares = decode_shares(prm);
+    if (shares <= 1) return 0;
+    return (size_t)shares * prm->batch * prm->heads * (2 + prm->head_dim) * sizeof(float);
+}
+
+extern "C" int slapo_amd_attn_fwd_ws(const slapo_attn_params* prm, const void* q, const void* k,
+                                     const void* v, const float* bias, void* o, float* lse,
+                                     void* workspace, size_t workspace_bytes, void* stream) {
     AttnArgs a = {};
     int rc = fill_args(prm, &a, false);
     if (rc != SLAPO_OK) return rc;
     if (!q || !k || !v || !o || !lse) return SLAPO_ERR_ARG;
+    if (workspace && !aligned16(workspace)) return SLAPO_ERR_ALIGN;
     a.q = q, a.k = k, a.v = v, a.o = o, a.lse = lse;
     set_bias(&a, bias);
     hipStream_t st = (hipStream_t)stream;
-    if (prm->dtype == SLAPO_F32) return attn_fwd_f32(a, st);
-    if (!half_ptrs_ok({q, k, v, o})) return SLAPO_ERR_ALIGN;
+    const bool f32 = prm->dtype == SLAPO_F32;
+    if (!f32 && !half_ptrs_ok({q, k, v, o})) return SLAPO_ERR_ALIGN;
+    if (int shares = decode_shares(prm)) {
+        // 16-byte reads of whole rows (16-bit types: checked above)
+        const bool rows_ok = !f32 || (a.d % 4 == 0 && strides_ok(prm->q_strides, 4) &&
+                                      strides_ok(prm->k_strides, 4) &&
+                                      strides_ok(prm->v_strides, 4) && half_ptrs_ok({q, k, v}));
+        if (!workspace || workspace_bytes < slapo_amd_attn_fwd_workspace_bytes(prm)) shares = 1;
+        if (rows_ok) return attn_decode(a, prm->dtype, shares, static_cast<float*>(workspace), st);
+    }
+    if (f32) return attn_fwd_f32(a, st);
     if (a.dropout && a.keep_mask && (a.window > 0 || a.dropout == 2) && keep_mask_kernel_fits(a)) {
         // Local window, or a mask geometry without whole Philox blocks per aligned group of keys,
         // with a buffer for the keep bits: draw them first, the forward kernel then reads them
@@ -211,6 +242,12 @@ extern "C" int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, c
         a.dropout = 3;
     }
     return prm->dtype == SLAPO_F16 ? attn_fwd_mfma_f16(a, st) : attn_fwd_mfma_bf16(a, st);
+}
+
+extern "C" int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* k,
+                                  const void* v, const float* bias, void* o, float* lse,
+                                  void* stream) {
+    return slapo_amd_attn_fwd_ws(prm, q, k, v, bias, o, lse, nullptr, 0, stream);
 }
 
 extern "C" size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* prm) {

@@ -3,6 +3,7 @@
 `-m "not gpu"` runs the oracle pins, host logic and C-ABI export checks (no device needed);
 `-m gpu` runs the parity tests proper, which call the HIP kernels through the C ABI.
 """
+import gc
 import os
 import sys
 
@@ -59,3 +60,10 @@ def assert_parity(actual, expected, dtype, what=""):
         err = max_abs_err(actual, expected)
         bound = HALF_RTOL * expected.detach().double().abs().max().item() + 1e-5
         assert err <= bound, f"{what}: max-abs {err:.3e} > {bound:.3e} (= {HALF_RTOL} relative)"
+
+
+def pytest_runtest_teardown(item, nextitem):
+    """Reference cycles that a module leaves behind (traced graph modules hold device tensors) are
+    collected at its end, not somewhere inside a later test that watches device memory."""
+    if nextitem is None or nextitem.fspath != item.fspath:
+        gc.collect()

@@ -631,6 +631,28 @@ def test_fp32_kernels_at_the_edges_of_tiles(shape, sk, causal, window, p):
     _check(q, k, v, do, mask, causal, window, torch.float32, p=p)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b,h,d,sk,layout", [
+    (1, 1, 8, 1, None),            # one key
+    (2, 3, 64, 127, "padding"),    # one share of the keys
+    (2, 3, 72, 129, None),         # two shares, the second with one key
+    (1, 5, 128, 3001, "padding"),  # many shares, some of them nothing but padding
+    (3, 2, 32, 640, "left"),       # key 0 masked: nothing may be skipped
+    (40, 30, 80, 200, None),       # more (batch, head) pairs than the chip needs workgroups
+])
+def test_one_query_per_sequence(dtype, b, h, d, sk, layout):
+    """The kernel for a generation step, forward and (through the ordinary kernels) backward."""
+    q, k, v, do, g = _inputs(b, 1, h, d, dtype, sk=sk)
+    mask = None
+    if layout == "padding":
+        mask, _ = _padding_mask(b, sk, dtype, g, max(1, sk // 8))
+    elif layout == "left":
+        mask = torch.zeros(b, 1, 1, sk, dtype=dtype)
+        mask[..., :sk // 2] = torch.finfo(dtype).min
+    _check(q, k, v, do, mask, False, 0, dtype)
+    _check(q, k, v, do, mask, True, 0, dtype)
+
+
 # ---- seeded sweep over the whole call surface --------------------------------------------------
 @pytest.mark.parametrize("seed", range(40))
 def test_random_configurations_against_the_oracle(seed):
