@@ -257,14 +257,32 @@ size_t slapo_amd_attn_keep_mask_bytes(const slapo_attn_params* prm);
 int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* k, const void* v,
                        const float* bias, void* o, float* lse, void* stream);
 
-/* The same call with a workspace (16-byte aligned, slapo_amd_attn_fwd_workspace_bytes of it, may be
- * NULL where that is 0): with one query per sequence and no dropout the keys of a (batch, head) are
- * shared by several workgroups, whose partial results meet there.  Without it such a call runs with
- * one workgroup per (batch, head). */
+/* The same call with two more freedoms.
+ * Bias type: SLAPO_F32 / F16 / BF16 name the element type that `bias` is stored in (with 16-bit
+ * q / k / v a 16-bit bias must have stride 0 over the queries, and neither a call with dropout nor
+ * the backward takes one);
+ * SLAPO_BIAS_PREPARED says that it is the output of slapo_amd_attn_prepare_bias, with strides
+ * {batch, head, rounded seqlen_k, 1}.
+ * Workspace: 16-byte aligned, slapo_amd_attn_fwd_workspace_bytes of it (may be NULL where that is
+ * 0).  With one query per sequence and no dropout the keys of a (batch, head) are shared by several
+ * workgroups, whose partial results meet there; without it such a call runs with one workgroup
+ * per (batch, head). */
+#define SLAPO_BIAS_PREPARED 3
 size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm);
-int slapo_amd_attn_fwd_ws(const slapo_attn_params* prm, const void* q, const void* k,
-                          const void* v, const float* bias, void* o, float* lse, void* workspace,
-                          size_t workspace_bytes, void* stream);
+int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
+                          const void* v, const void* bias, int bias_type, void* o, float* lse,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
+/* An additive bias with values of its own per query, laid out as the 16-bit kernels read it fastest:
+ * fp32 [batch][heads][rounded seqlen_q][rounded seqlen_k] (both rounded up to 64), in log2 units.
+ * batch / heads are those of the bias itself (1 where it is broadcast: the calls that read the
+ * result then pass stride 0).  _bytes is 0 where the layout does not serve: seqlen_q x seqlen_k
+ * (rounded) of 2^30 and more. */
+size_t slapo_amd_attn_prepared_bias_bytes(int64_t batch, int64_t heads, int64_t seqlen_q,
+                                          int64_t seqlen_k);
+int slapo_amd_attn_prepare_bias(const void* bias, int bias_type, const int64_t bias_strides[4],
+                                int64_t batch, int64_t heads, int64_t seqlen_q, int64_t seqlen_k,
+                                float* out, void* stream);
 
 /* Workspace (bytes) the backward needs: fp32 delta = rowsum(dO * O), one value per query row. */
 size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* prm);
@@ -276,6 +294,14 @@ int slapo_amd_attn_bwd(const slapo_attn_params* prm, const void* q, const void* 
                        void* dq, void* dk, void* dv, const int64_t dq_strides[3],
                        const int64_t dk_strides[3], const int64_t dv_strides[3], void* workspace,
                        size_t workspace_bytes, void* stream);
+
+/* The same call with the bias type of slapo_amd_attn_fwd_ex. */
+int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
+                          const void* v, const void* bias, int bias_type, const void* o,
+                          const void* dout, const float* lse, void* dq, void* dk, void* dv,
+                          const int64_t dq_strides[3], const int64_t dk_strides[3],
+                          const int64_t dv_strides[3], void* workspace, size_t workspace_bytes,
+                          void* stream);
 
 /* The backward runs as stages on `stream`, in this order:
  *   PREPARE  nothing to do;

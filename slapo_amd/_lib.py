@@ -128,9 +128,20 @@ PROTOTYPES = {
         ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]
     ),
     "slapo_amd_attn_fwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
-    "slapo_amd_attn_fwd_ws": (
-        ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
-                       ctypes.c_size_t, c_vp]
+    "slapo_amd_attn_fwd_ex": (
+        ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, ctypes.c_int, c_vp,
+                       c_vp, c_vp, ctypes.c_size_t, c_vp]
+    ),
+    "slapo_amd_attn_prepared_bias_bytes": (ctypes.c_size_t, [c_i64, c_i64, c_i64, c_i64]),
+    "slapo_amd_attn_prepare_bias": (
+        ctypes.c_int, [c_vp, ctypes.c_int, ctypes.POINTER(c_i64), c_i64, c_i64, c_i64, c_i64,
+                       c_vp, c_vp]
+    ),
+    "slapo_amd_attn_bwd_ex": (
+        ctypes.c_int,
+        [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, ctypes.c_int, c_vp, c_vp, c_vp, c_vp,
+         c_vp, c_vp, ctypes.POINTER(c_i64), ctypes.POINTER(c_i64), ctypes.POINTER(c_i64), c_vp,
+         ctypes.c_size_t, c_vp],
     ),
     "slapo_amd_attn_bwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
     "slapo_amd_attn_keep_mask_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),

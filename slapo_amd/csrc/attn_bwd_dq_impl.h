@@ -95,10 +95,12 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     // kBias == 2: thread (x & 63) carries key row0 + (x & 63) of the requested tile (all four
     // wavefronts alike, so that neither request nor store needs a branch)
     const float* bias_keys = nullptr;
-    if constexpr (kBias == 2) bias_keys = a.bias + b * a.bs[0] + h * a.bs[1];
+    if constexpr (kBias == 2)
+        bias_keys = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1];
     float bias_stage = 0.f;
     auto store_bias = [&](int slot) __attribute__((always_inline)) {
-        if constexpr (kBias == 2) bias_lds[slot * kBN + row_slot(lane)] = bias_log2(bias_stage);
+        if constexpr (kBias == 2)
+            bias_lds[slot * kBN + row_slot(lane)] = bias_log2(bias_stage);
     };
     const float* bias_tile = bias_lds;  // the slot of the tile in process
     auto request = [&](int row0) __attribute__((always_inline)) {
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     int j_lo, j_hi;
     key_range(a, q0, min(q0 + kBM, a.sq), j_lo, j_hi);
     if constexpr (kBias)  // skip the tiles that hold nothing but padded keys
-        j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads>(
+        j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads, false>(
                                            a, b, h, reinterpret_cast<float*>(smem_raw))));
     const int t_lo = j_lo / kBN;
     const int t_hi = (j_hi + kBN - 1) / kBN;
@@ -197,8 +199,9 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     if constexpr (kDrop != 0)
         drop_row_base = ((uint64_t)bh * a.sq + (uint64_t)q_row) * (uint64_t)a.sk;
     const float* bias_row = nullptr;
-    if constexpr (kBias)
-        bias_row = a.bias + b * a.bs[0] + h * a.bs[1] + (int64_t)min(q_row, a.sq - 1) * a.bs[2];
+    if constexpr (kBias == 1 || kBias == 3)  // (prepared rows exist past the end)
+        bias_row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] +
+                   (int64_t)(kBias == 3 ? q_row : min(q_row, a.sq - 1)) * a.bs[2];
 
     // per-lane LDS offsets (elements) that do not change from tile to tile
     const int row_off = pi_row(i_loc) * kPitch + 8 * g;
@@ -293,11 +296,16 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
                                                                      quad_slot(r4, g));
                 bv[0] = t4.x, bv[1] = t4.y, bv[2] = t4.z, bv[3] = t4.w;
             }
+            if constexpr (kBias == 3) {
+                const f32x4_t t4 =
+                    *reinterpret_cast<const f32x4_t*>(bias_row + j0 + 16 * g + 4 * r4);
+                bv[0] = t4.x, bv[1] = t4.y, bv[2] = t4.z, bv[3] = t4.w;
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 float x = s[4 * r4 + e];  // the scale is in already
                 if constexpr (!kAccInit) x -= lse_sub;
-                if constexpr (kBias == 2) x += bv[e];
+                if constexpr (kBias == 2 || kBias == 3) x += bv[e];
                 float p = fast_exp2(x);
                 if constexpr (kMask != 0) {
                     const int c = acc_row(4 * r4 + e, 0);
@@ -555,6 +563,12 @@ int launch(const AttnArgs& a, hipStream_t st) {
 template <typename T, int DPAD, bool kStagger, int kSteps = DPAD / 16>
 int dispatch_flags(const AttnArgs& a, hipStream_t st) {
     if (a.has_bias) {
+        if (a.bias_type == SLAPO_BIAS_PREPARED) {
+            if (a.dropout == 1) return launch<T, DPAD, 3, 1, kStagger, kSteps>(a, st);
+            if (a.dropout == 2) return launch<T, DPAD, 3, 2, kStagger, kSteps>(a, st);
+            if (a.dropout == 3) return launch<T, DPAD, 3, 3, kStagger, kSteps>(a, st);
+            return launch<T, DPAD, 3, 0, kStagger, kSteps>(a, st);
+        }
         if (a.bs[2] == 0) {  // the bias depends on the key only
             if (a.dropout == 1) return launch<T, DPAD, 2, 1, kStagger, kSteps>(a, st);
             if (a.dropout == 2) return launch<T, DPAD, 2, 2, kStagger, kSteps>(a, st);

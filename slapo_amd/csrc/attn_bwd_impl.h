@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     int i_lo, i_hi;
     query_range(a, k0, min(k0 + kBN, a.sk), i_lo, i_hi);
     if constexpr (kBias) {  // a workgroup that owns nothing but padded keys has dK = dV = 0
-        if (k0 >= padded_key_limit<kBwdThreads>(a, b, h, reinterpret_cast<float*>(smem_raw)))
+        if (k0 >= padded_key_limit<kBwdThreads, false>(a, b, h, reinterpret_cast<float*>(smem_raw)))
             i_hi = i_lo;
     }
     const int t_lo = i_lo / kBwdBM;
@@ -142,7 +142,15 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     // kBias: 0 = none, 1 = any layout (read from memory per score), 2 = the launcher guarantees a
     // bias that does not depend on the query (stride 0 over the queries, the compact [B,1,1,Sk]
     // layout): one register per lane and key block.
+    // 3 = a prepared bias (bias_prepare_kernel): register r of a lane reads row i at the slot of the
+    // lane's key, a whole 128-byte block per row and lane-group.
     constexpr bool bias_per_key = kBias == 2;
+    const float* bias_tile = nullptr;
+    uint32_t bias_lane = 0;
+    if constexpr (kBias == 3) {
+        bias_tile = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] + kw0;
+        bias_lane = (uint32_t)(kAccGroupStep * g * (int)a.bs[2] + prepared_slot(c_loc));
+    }
     float bias_k[KB];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
@@ -150,7 +158,8 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
         if constexpr (kBias) {
             if (bias_per_key && key[kb] < a.sk)
                 bias_k[kb] =
-                    bias_log2(a.bias[b * a.bs[0] + h * a.bs[1] + (int64_t)key[kb] * a.bs[3]]);
+                    bias_log2(reinterpret_cast<const float*>(
+                        a.bias)[b * a.bs[0] + h * a.bs[1] + (int64_t)key[kb] * a.bs[3]]);
         }
     }
     // per-lane LDS offsets (elements) that do not change from tile to tile
@@ -357,8 +366,13 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
                 } else if constexpr (kBias == 1) {
                     const int i = ih0 + acc_row(r, g);
                     if (i < a.sq && key[kb] < a.sk)
-                        x += bias_log2(a.bias[b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] +
-                                              (int64_t)key[kb] * a.bs[3]]);
+                        x += bias_log2(reinterpret_cast<const float*>(
+                            a.bias)[b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] +
+                                    (int64_t)key[kb] * a.bs[3]]);
+                } else if constexpr (kBias == 3) {
+                    static_assert(KB == 1, "one key block per wavefront");
+                    const float* row = bias_tile + (int64_t)(ih0 + acc_row(r, 0)) * a.bs[2];
+                    x += row[bias_lane];
                 }
                 float p = fast_exp2(x);
                 if constexpr (kMask != 0) {
@@ -674,6 +688,7 @@ int dispatch_drop(const AttnArgs& a, hipStream_t st) {
 template <typename T, int DPAD, int kSteps = DPAD / 16>
 int dispatch_flags(const AttnArgs& a, hipStream_t st) {
     if (!a.has_bias) return dispatch_drop<T, DPAD, 0, kSteps>(a, st);
+    if (a.bias_type == SLAPO_BIAS_PREPARED) return dispatch_drop<T, DPAD, 3, kSteps>(a, st);
     return a.bs[2] == 0 ? dispatch_drop<T, DPAD, 2, kSteps>(a, st)
                         : dispatch_drop<T, DPAD, 1, kSteps>(a, st);
 }

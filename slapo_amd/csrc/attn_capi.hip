@@ -163,14 +163,62 @@ int fill_args(const slapo_attn_params* p, AttnArgs* a, bool backward) {
     return SLAPO_OK;
 }
 
-void set_bias(AttnArgs* a, const float* bias) {
+// The additive bias of a call: SLAPO_ERR_DTYPE for a type that its layout is not read in.
+int set_bias(AttnArgs* a, const void* bias, int type, bool f32, bool backward) {
     a->bias = bias;
     a->has_bias = bias ? 1 : 0;
     a->bias_vec4 = 0;
-    if (bias && a->bs[3] == 1 && aligned16(bias) && a->bs[0] % 4 == 0 && a->bs[1] % 4 == 0 &&
+    a->bias_type = type;
+    if (!bias) return SLAPO_OK;
+    if (a->sq == 1 && type != SLAPO_BIAS_PREPARED) a->bs[2] = 0;
+    if (type == SLAPO_BIAS_PREPARED) {
+        if (f32) return SLAPO_ERR_DTYPE;
+        return aligned16(bias) ? SLAPO_OK : SLAPO_ERR_ALIGN;
+    }
+    if (type != SLAPO_F32 && type != SLAPO_F16 && type != SLAPO_BF16) return SLAPO_ERR_DTYPE;
+    // the kernels address the values of a row with 32-bit offsets
+    if (a->bs[3] < 0 || a->bs[3] * a->sk >= int64_t(1) << 30) return SLAPO_ERR_SHAPE;
+    // 16-bit biases of the 16-bit kernels: one value per key in a forward without dropout, or
+    // prepared
+    if (type != SLAPO_F32 && !f32 && (backward || a->dropout || a->bs[2] != 0))
+        return SLAPO_ERR_DTYPE;
+    if (a->bs[3] == 1 && aligned16(bias) && a->bs[0] % 4 == 0 && a->bs[1] % 4 == 0 &&
         a->bs[2] % 4 == 0)
         a->bias_vec4 = 1;
+    return SLAPO_OK;
 }
+
+// Additive bias with values of its own per query -> fp32 rows in log2 units, masking values
+// canonical, rows and row length padded to 64 with zeros, the keys of a 32-key block in
+// accumulator order (prepared_slot).  One thread per four slots; bound by reading the mask and
+// writing the rows once (bf16 [B,1,Sq,Sk]: 6 bytes per value), which stands in for the conversion
+// to fp32 that such a mask would need anyway.  The matrix kernels then add a bias with four
+// 16-byte loads per 32 scores and lane: fp16 B21 S1512 H11 D72 with a [B,1,Sq,Sk] causal and
+// padding mask, forward + backward 2.50 -> 1.37 ms.
+__global__ __launch_bounds__(256) void bias_prepare_kernel(const AttnArgs a, int64_t heads,
+                                                           int rows, int pitch,
+                                                           float* __restrict__ out) {
+    const int64_t quad = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int per_row = pitch / 4;
+    const int64_t row = quad / per_row;
+    const int x = (int)(quad - row * per_row) * 4;  // first slot
+    const int64_t bh = row / rows;
+    const int i = (int)(row - bh * rows);
+    const int64_t b = bh / heads, h = bh - b * heads;
+    if (b >= a.batch) return;
+    const int g = (x >> 4) & 1, r = x & 15;
+    f32x4_t v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int j = (x & ~31) + acc_row(r + e, g);
+        if (i < a.sq && j < a.sk)
+            v[e] = bias_log2(bias_load(a, b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] +
+                                              (int64_t)j * a.bs[3]));
+    }
+    *reinterpret_cast<f32x4_t*>(out + row * pitch + x) = v;
+}
+
+int64_t prepared_rows(int64_t n) { return (n + 63) & ~int64_t(63); }
 
 bool half_ptrs_ok(std::initializer_list<const void*> ptrs) {
     for (const void* p : ptrs)
@@ -207,18 +255,52 @@ extern "C" size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* pr
     return (size_t)shares * prm->batch * prm->heads * (2 + prm->head_dim) * sizeof(float);
 }
 
-extern "C" int slapo_amd_attn_fwd_ws(const slapo_attn_params* prm, const void* q, const void* k,
-                                     const void* v, const float* bias, void* o, float* lse,
-                                     void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" size_t slapo_amd_attn_prepared_bias_bytes(int64_t batch, int64_t heads,
+                                                     int64_t seqlen_q, int64_t seqlen_k) {
+    if (batch <= 0 || heads <= 0 || seqlen_q <= 0 || seqlen_k <= 0) return 0;
+    // the kernels address the rows of one (batch, head) with 32-bit byte offsets
+    const int64_t one = prepared_rows(seqlen_q) * prepared_rows(seqlen_k);
+    if (one >= int64_t(1) << 30) return 0;
+    return (size_t)(batch * heads * one) * sizeof(float);
+}
+
+extern "C" int slapo_amd_attn_prepare_bias(const void* bias, int bias_type,
+                                           const int64_t bias_strides[4], int64_t batch,
+                                           int64_t heads, int64_t seqlen_q, int64_t seqlen_k,
+                                           float* out, void* stream) {
+    if (!bias || !bias_strides || !out) return SLAPO_ERR_ARG;
+    if (bias_type != SLAPO_F32 && bias_type != SLAPO_F16 && bias_type != SLAPO_BF16)
+        return SLAPO_ERR_DTYPE;
+    if (!aligned16(out)) return SLAPO_ERR_ALIGN;
+    if (!slapo_amd_attn_prepared_bias_bytes(batch, heads, seqlen_q, seqlen_k))
+        return SLAPO_ERR_SHAPE;
+    AttnArgs a = {};
+    a.bias = bias, a.bias_type = bias_type;
+    for (int i = 0; i < 4; ++i) a.bs[i] = bias_strides[i];
+    a.batch = (int)batch, a.sq = (int)seqlen_q, a.sk = (int)seqlen_k;
+    const int rows = (int)prepared_rows(seqlen_q), pitch = (int)prepared_rows(seqlen_k);
+    const int64_t quads = batch * heads * rows * (pitch / 4);
+    const int64_t blocks = (quads + 255) / 256;
+    if (blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
+    hipLaunchKernelGGL(bias_prepare_kernel, dim3((unsigned)blocks), dim3(256), 0,
+                       (hipStream_t)stream, a, heads, rows, pitch, out);
+    return check_launch();
+}
+
+extern "C" int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
+                                     const void* v, const void* bias, int bias_type, void* o,
+                                     float* lse, void* workspace, size_t workspace_bytes,
+                                     void* stream) {
     AttnArgs a = {};
     int rc = fill_args(prm, &a, false);
     if (rc != SLAPO_OK) return rc;
     if (!q || !k || !v || !o || !lse) return SLAPO_ERR_ARG;
     if (workspace && !aligned16(workspace)) return SLAPO_ERR_ALIGN;
     a.q = q, a.k = k, a.v = v, a.o = o, a.lse = lse;
-    set_bias(&a, bias);
-    hipStream_t st = (hipStream_t)stream;
     const bool f32 = prm->dtype == SLAPO_F32;
+    rc = set_bias(&a, bias, bias_type, f32, false);
+    if (rc != SLAPO_OK) return rc;
+    hipStream_t st = (hipStream_t)stream;
     if (!f32 && !half_ptrs_ok({q, k, v, o})) return SLAPO_ERR_ALIGN;
     if (int shares = decode_shares(prm)) {
         // 16-byte reads of whole rows (16-bit types: checked above)
@@ -226,7 +308,8 @@ extern "C" int slapo_amd_attn_fwd_ws(const slapo_attn_params* prm, const void* q
                                       strides_ok(prm->k_strides, 4) &&
                                       strides_ok(prm->v_strides, 4) && half_ptrs_ok({q, k, v}));
         if (!workspace || workspace_bytes < slapo_amd_attn_fwd_workspace_bytes(prm)) shares = 1;
-        if (rows_ok) return attn_decode(a, prm->dtype, shares, static_cast<float*>(workspace), st);
+        if (rows_ok && bias_type != SLAPO_BIAS_PREPARED)
+            return attn_decode(a, prm->dtype, shares, static_cast<float*>(workspace), st);
     }
     if (f32) return attn_fwd_f32(a, st);
     if (a.dropout && a.keep_mask && (a.window > 0 || a.dropout == 2) && keep_mask_kernel_fits(a)) {
@@ -247,7 +330,7 @@ extern "C" int slapo_amd_attn_fwd_ws(const slapo_attn_params* prm, const void* q
 extern "C" int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* k,
                                   const void* v, const float* bias, void* o, float* lse,
                                   void* stream) {
-    return slapo_amd_attn_fwd_ws(prm, q, k, v, bias, o, lse, nullptr, 0, stream);
+    return slapo_amd_attn_fwd_ex(prm, q, k, v, bias, SLAPO_F32, o, lse, nullptr, 0, stream);
 }
 
 extern "C" size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* prm) {
@@ -257,13 +340,12 @@ extern "C" size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* pr
     return rows * sizeof(float);  // delta
 }
 
-extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const void* q,
-                                         const void* k, const void* v, const float* bias,
-                                         const void* o, const void* dout, const float* lse,
-                                         void* dq, void* dk, void* dv,
-                                         const int64_t dq_strides[3], const int64_t dk_strides[3],
-                                         const int64_t dv_strides[3], void* workspace,
-                                         size_t workspace_bytes, int stages, void* stream) {
+namespace {
+int run_backward(const slapo_attn_params* prm, const void* q, const void* k, const void* v,
+                 const void* bias, int bias_type, const void* o, const void* dout,
+                 const float* lse, void* dq, void* dk, void* dv, const int64_t dq_strides[3],
+                 const int64_t dk_strides[3], const int64_t dv_strides[3], void* workspace,
+                 size_t workspace_bytes, int stages, void* stream) {
     AttnArgs a = {};
     int rc = fill_args(prm, &a, true);
     if (rc != SLAPO_OK) return rc;
@@ -282,7 +364,8 @@ extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const voi
     a.q = q, a.k = k, a.v = v, a.o = const_cast<void*>(o), a.dout = dout;
     a.lse = const_cast<float*>(lse);
     a.dk = dk, a.dv = dv;
-    set_bias(&a, bias);
+    rc = set_bias(&a, bias, bias_type, prm->dtype == SLAPO_F32, true);
+    if (rc != SLAPO_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
 
     a.delta = reinterpret_cast<float*>(workspace);
@@ -311,6 +394,29 @@ extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const voi
         rc = prm->dtype == SLAPO_F16 ? attn_bwd_mfma_f16(a, st) : attn_bwd_mfma_bf16(a, st);
     }
     return rc;
+}
+
+}  // namespace
+
+extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const void* q,
+                                         const void* k, const void* v, const float* bias,
+                                         const void* o, const void* dout, const float* lse,
+                                         void* dq, void* dk, void* dv,
+                                         const int64_t dq_strides[3], const int64_t dk_strides[3],
+                                         const int64_t dv_strides[3], void* workspace,
+                                         size_t workspace_bytes, int stages, void* stream) {
+    return run_backward(prm, q, k, v, bias, SLAPO_F32, o, dout, lse, dq, dk, dv, dq_strides,
+                        dk_strides, dv_strides, workspace, workspace_bytes, stages, stream);
+}
+
+extern "C" int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
+                                     const void* v, const void* bias, int bias_type,
+                                     const void* o, const void* dout, const float* lse, void* dq,
+                                     void* dk, void* dv, const int64_t dq_strides[3],
+                                     const int64_t dk_strides[3], const int64_t dv_strides[3],
+                                     void* workspace, size_t workspace_bytes, void* stream) {
+    return run_backward(prm, q, k, v, bias, bias_type, o, dout, lse, dq, dk, dv, dq_strides,
+                        dk_strides, dv_strides, workspace, workspace_bytes, SLAPO_BWD_ALL, stream);
 }
 
 extern "C" int slapo_amd_attn_bwd(const slapo_attn_params* prm, const void* q, const void* k,

@@ -227,7 +227,7 @@ struct AttnArgs {
     void* dq;  // element type of the tensors
     void* dk;
     void* dv;
-    const float* bias;
+    const void* bias;
     float* lse;
     float* delta;
     int64_t qs[3], ks[3], vs[3], os[3], dqs[3], dks[3], dvs[3];
@@ -235,6 +235,7 @@ struct AttnArgs {
     int batch, heads, sq, sk, d;
     int causal, window;
     int has_bias, bias_vec4;  // bias_vec4: s3 == 1, s2 == 0 rows 16B-aligned
+    int bias_type;            // SLAPO_F32 / F16 / BF16, or SLAPO_BIAS_PREPARED
     // dropout: 0 = off, 1 = fast mask geometry (plan.vec >= 4, power-of-two thread count and
     // sk % 4 == 0: one Philox block per aligned group of four keys), 2 = any geometry,
     // 3 = keep bits read from keep_mask (drawn by keep_mask_kernel ahead of the forward)
@@ -253,6 +254,43 @@ struct AttnArgs {
     int head_group;
     int n_cus;
 };
+
+// One value of the additive bias in the type it is stored in.  Split into the read -- one aligned
+// dword whatever the type, so that a request stays straight-line code -- and the conversion, which
+// belongs where the value is used and is a pair of selects, not a branch.
+__device__ __forceinline__ float bias_value(const AttnArgs& a, uint32_t raw) {
+    const float half = (float)__builtin_bit_cast(f16_t, (uint16_t)raw);
+    const uint32_t half_bits = __builtin_bit_cast(uint32_t, half);
+    const uint32_t bits16 = a.bias_type == SLAPO_BF16 ? raw << 16 : half_bits;
+    return __builtin_bit_cast(float, a.bias_type == SLAPO_F32 ? raw : bits16);
+}
+// at element index idx
+__device__ __forceinline__ float bias_load(const AttnArgs& a, int64_t idx) {
+    const uintptr_t at =
+        reinterpret_cast<uintptr_t>(a.bias) + ((uint64_t)idx << (a.bias_type == SLAPO_F32 ? 2 : 1));
+    return bias_value(a, *reinterpret_cast<const uint32_t*>(at & ~(uintptr_t)3) >> ((at & 2) * 8));
+}
+// A row of values, one per key: a wavefront-uniform base and 32-bit byte offsets per lane.
+struct BiasKeys {
+    const char* base;
+    uint32_t mis, shift, step;
+    __device__ __forceinline__ BiasKeys(const AttnArgs& a, int64_t row) {
+        shift = a.bias_type == SLAPO_F32 ? 2 : 1;
+        const uintptr_t at = reinterpret_cast<uintptr_t>(a.bias) + ((uint64_t)row << shift);
+        base = reinterpret_cast<const char*>(at & ~(uintptr_t)3);
+        mis = (uint32_t)at & 2u;
+        step = (uint32_t)a.bs[3];
+    }
+    __device__ __forceinline__ uint32_t raw(int j) const {
+        const uint32_t off = (((uint32_t)j * step) << shift) + mis;
+        return *reinterpret_cast<const uint32_t*>(base + (off & ~3u)) >> ((off & 2u) * 8);
+    }
+};
+// Position of key `key` (0..31) of a 32-key block in a prepared bias row: the sixteen values of
+// lane-group 0 in accumulator order, then those of lane-group 1.
+__device__ __forceinline__ constexpr int prepared_slot(int key) {
+    return ((key >> 1) & 1) * 16 + ((key >> 4) << 3) + ((key & 1) << 2) + ((key >> 2) & 3);
+}
 
 // Which unit of work a workgroup takes.  The kernels order their work heaviest first (under a
 // causal mask a workgroup's loop has 2 to 2 S / 128 tiles), and the hardware hands the
@@ -350,14 +388,23 @@ __device__ __forceinline__ void query_range(const AttnArgs& a, int k_lo, int k_h
 // Called by all threads of the workgroup; `scratch` is 4 floats of LDS that nothing else uses
 // until the call returns.
 constexpr float kMaskedBias = -30000.f;  // below fp16's most negative value, far beyond any score
-template <int THREADS>
+// kTyped: the bias may be of any type; the 16-bit backward kernels take fp32 only (their registers are
+// all spoken for: the selects of bias_value cost them 10 %).
+template <int THREADS, bool kTyped>
 __device__ __forceinline__ int padded_key_limit(const AttnArgs& a, int b, int h, float* scratch) {
-    if (!a.has_bias || a.bs[2] != 0 || a.window > 0) return a.sk;
-    const float* brow = a.bias + b * a.bs[0] + h * a.bs[1];
-    if (!(brow[0] > kMaskedBias)) return a.sk;
+    if (!a.has_bias || a.bs[2] != 0 || a.window > 0) return a.sk;  // (a prepared one: pitch)
     int last = 0;
-    for (int j = threadIdx.x; j < a.sk; j += THREADS)
-        if (brow[(int64_t)j * a.bs[3]] > kMaskedBias) last = j;
+    if constexpr (kTyped) {
+        const BiasKeys row(a, b * a.bs[0] + h * a.bs[1]);
+        if (!(bias_value(a, row.raw(0)) > kMaskedBias)) return a.sk;
+        for (int j = threadIdx.x; j < a.sk; j += THREADS)
+            if (bias_value(a, row.raw(j)) > kMaskedBias) last = j;
+    } else {
+        const float* row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1];
+        if (!(row[0] > kMaskedBias)) return a.sk;
+        for (int j = threadIdx.x; j < a.sk; j += THREADS)
+            if (row[(int64_t)j * a.bs[3]] > kMaskedBias) last = j;
+    }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
     if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = __int_as_float(last);

@@ -11,7 +11,7 @@
 // groups, then wavefronts, are merged once at the end.  With more than one share per (batch, head)
 // the unnormalised results go to a workspace and attn_decode_merge_kernel adds them in order (no
 // atomics).  Scores, probabilities and sums are fp32; q, k, v enter as they are stored.
-// bf16 B8 H16 Sk2000 D128 (131 MB): 54.6 us with the tile kernel, @STEP@ here.
+// bf16 B8 H16 Sk2000 D128 (131 MB): 54.6 us with the tile kernel, 27.5 us here (4.8 TB/s).
 //
 // Reference semantics: slapo/op/attention.py:163-181 (attention_bmk).
 #include <type_traits>
@@ -122,16 +122,17 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a,
     const T* qp = reinterpret_cast<const T*>(a.q) + b * a.qs[0] + h * a.qs[2];
     const T* kp = reinterpret_cast<const T*>(a.k) + b * a.ks[0] + h * a.ks[2];
     const T* vp = reinterpret_cast<const T*>(a.v) + b * a.vs[0] + h * a.vs[2];
-    const float* bias = a.has_bias ? a.bias + b * a.bs[0] + h * a.bs[1] : nullptr;
+    const bool bias = a.has_bias != 0;
+    const int64_t bias_at = b * a.bs[0] + h * a.bs[1];
     const bool col_ok = sub * kN < a.d;
     const int col = min(sub * kN, a.d - kN);
 
-    if (bias && bias[0] > kMaskedBias) {
+    if (bias && bias_load(a, bias_at) > kMaskedBias) {
         // Padding at the end of the share contributes exactly zero to a row that sees key 0 (see
         // padded_key_limit): its keys are not read.
         int last = k_lo - 1;
         for (int j = k_lo + (int)threadIdx.x; j < k_hi; j += kThreads)
-            if (bias[(int64_t)j * a.bs[3]] > kMaskedBias) last = j;
+            if (bias_load(a, bias_at + (int64_t)j * a.bs[3]) > kMaskedBias) last = j;
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
         if (lane == 0) sh_m[wave] = __int_as_float(last);
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a,
                 __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(kp + j * a.ks[1] + col));
             *reinterpret_cast<u32x4_t*>(&vv[u]) =
                 __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(vp + j * a.vs[1] + col));
-            s[u] = bias ? bias[j * a.bs[3]] : 0.f;
+            s[u] = bias ? bias_load(a, bias_at + j * a.bs[3]) : 0.f;
         }
         float mx = m;
 #pragma unroll

@@ -49,8 +49,8 @@ __device__ __forceinline__ float column_sum(float v) {
 }
 
 __device__ __forceinline__ float bias_at(const AttnArgs& a, int b, int h, int i, int j) {
-    return canonical_bias(
-        a.bias[b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] + (int64_t)j * a.bs[3]]);
+    return canonical_bias(bias_load(
+        a, b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] + (int64_t)j * a.bs[3]));
 }
 
 // LDS row pitch of a tile, in floats
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(kThreads, DB <= 4 ? 3 : 2) void attn_f32_fwd_kernel
 
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
-    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads>(a, at.b, at.h, lds) : a.sk));
+    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk));
     const int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
 
     Tile<DB, kVec> kt, vt;
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
 
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
-    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads>(a, at.b, at.h, lds) : a.sk));
+    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk));
     const int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
 
     Tile<DB, kVec> kt, vt;
@@ -452,7 +452,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
     int i_lo, i_hi;
     query_range(a, at.row0, min(at.row0 + kRows, a.sk), i_lo, i_hi);
     // keys past the last unpadded one get no probability from any row
-    if (at.row0 >= (has_bias ? padded_key_limit<kThreads>(a, at.b, at.h, lds) : a.sk)) i_hi = i_lo;
+    if (at.row0 >= (has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk)) i_hi = i_lo;
     const int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
 
     Tile<DB, kVec> qt, gt;

@@ -32,19 +32,29 @@ constexpr int kBM = kWaves * 32;
 constexpr int kBN = 64;
 constexpr float kMaxSlack = 8.0f;  // hysteresis of the softmax reference, log2 units
 
+// Workgroups per CU: three in 168 registers without dropout or a per-score bias up to head_dim 64.
+constexpr int fwd_per_cu(int dpad, int bias, int drop) {
+    return dpad <= 64 && drop == 0 && bias != 3 ? 3 : 2;
+}
+
 template <typename T, int DPAD, int kBias, int kDrop, int kWin, int kSteps>
-__global__ __launch_bounds__(kThreads, (DPAD <= 64 && kDrop == 0 ? 3 : 2)) void attn_fwd_kernel(
+__global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn_fwd_kernel(
     const AttnArgs a_in) {
     // kBias: 0 = no additive bias, 1 = any layout (read from memory per score), 2 = the bias
     // depends on the key only (stride 0 over the queries, e.g. a [B,1,1,Sk] padding mask): the 64
     // values of a key tile travel through LDS beside the K / V tile and the tile body has neither
     // global loads nor branches for them (bf16 B4 S2048 H32 D80 causal, every key valid: 241 us
-    // with the per-score reads against 169 us without a bias).
+    // with the per-score reads against 169 us without a bias), 3 = a prepared bias
+    // (bias_prepare_kernel): fp32 rows in log2 units, padded and in accumulator order, so that a
+    // lane reads its sixteen values of a half with four 16-byte loads and nothing else.
     // kWin: 0 = the launcher guarantees window <= 0, 1 = it guarantees window > 0, 2 = either.
     // Folding "no window" in removes the two-sided mask body and the window tests from the
     // kernel, and with them the register spills of the bias-free builds (head_dim 64: 24 spilled
     // registers -> none, 37.8 -> 35.7 us at fp16 B8 S1024 H16 causal; head_dim 128: 69 -> 4,
     // 116 -> 96-109 us at bf16 B4 S2048 H16 causal); folding "window" in leaves one masked body.
+    // 4 = like 2 for a bias of any type (16-bit masks at inference; the selects of the conversion cost
+    // the forward 2 %, so that training, whose backward kernels read fp32 anyway, keeps 2).
+    constexpr bool kKeyBias = kBias == 2 || kBias == 4;
     AttnArgs a = a_in;
     if constexpr (kWin == 0) a.window = 0;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
@@ -60,7 +70,7 @@ __global__ __launch_bounds__(kThreads, (DPAD <= 64 && kDrop == 0 ? 3 : 2)) void 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* k_lds = reinterpret_cast<T*>(smem_raw);  // K[2][tile]
     T* v_lds = k_lds + 2 * kTileElems;          // V[2][tile]
-    float* bias_lds = reinterpret_cast<float*>(v_lds + 2 * kTileElems);  // [2][kBN], kBias == 2
+    float* bias_lds = reinterpret_cast<float*>(v_lds + 2 * kTileElems);  // [2][kBN], kKeyBias
 
     const int n_bh = a.batch * a.heads;
     const int n_qt = (a.sq + kBM - 1) / kBM;
@@ -85,7 +95,7 @@ __global__ __launch_bounds__(kThreads, (DPAD <= 64 && kDrop == 0 ? 3 : 2)) void 
     int j_lo, j_hi;
     key_range(a, q0, min(q0 + kBM, a.sq), j_lo, j_hi);
     if constexpr (kBias)  // skip the tiles that hold nothing but padded keys
-        j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads>(
+        j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads, kBias == 4>(
                                            a, b, h, reinterpret_cast<float*>(smem_raw))));
     const int t_lo = j_lo / kBN;
     const int t_hi = (j_hi + kBN - 1) / kBN;
@@ -154,19 +164,25 @@ __global__ __launch_bounds__(kThreads, (DPAD <= 64 && kDrop == 0 ? 3 : 2)) void 
     if constexpr (kDrop != 0)
         drop_row_base = ((uint64_t)bh * a.sq + (uint64_t)q_row) * (uint64_t)a.sk;
     const float* bias_row = nullptr;
-    if constexpr (kBias)
-        bias_row = a.bias + b * a.bs[0] + h * a.bs[1] + (int64_t)min(q_row, a.sq - 1) * a.bs[2];
-    // kBias == 2: thread (x & 63) carries key j0 + (x & 63) of the requested tile (all four
+    if constexpr (kBias == 1 || kBias == 3)  // (prepared rows exist past the end)
+        bias_row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] +
+                   (int64_t)(kBias == 3 ? q_row : min(q_row, a.sq - 1)) * a.bs[2];
+    // kKeyBias: thread (x & 63) carries key j0 + (x & 63) of the requested tile (all four
     // wavefronts alike, so that neither request nor store needs a branch)
     const float* bias_keys = nullptr;
-    if constexpr (kBias == 2) bias_keys = a.bias + b * a.bs[0] + h * a.bs[1];
+    if constexpr (kBias == 2)
+        bias_keys = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1];
+    const BiasKeys bias_typed(a, kBias == 4 ? b * a.bs[0] + h * a.bs[1] : 0);
     float bias_stage = 0.f;
+    uint32_t bias_raw = 0;
     auto request_bias = [&](int j0) __attribute__((always_inline)) {
         if constexpr (kBias == 2)
             bias_stage = bias_keys[(int64_t)min(j0 + lane, a.sk - 1) * a.bs[3]];
+        if constexpr (kBias == 4) bias_raw = bias_typed.raw(min(j0 + lane, a.sk - 1));
     };
     auto store_bias = [&](int slot) __attribute__((always_inline)) {
-        if constexpr (kBias == 2) bias_lds[slot * kBN + row_slot(lane)] = bias_log2(bias_stage);
+        if constexpr (kBias == 4) bias_stage = bias_value(a, bias_raw);
+        if constexpr (kKeyBias) bias_lds[slot * kBN + row_slot(lane)] = bias_log2(bias_stage);
     };
     const float* bias_tile = bias_lds;  // the slot of the tile in process
     request_bias(t_lo * kBN);
@@ -235,7 +251,13 @@ __global__ __launch_bounds__(kThreads, (DPAD <= 64 && kDrop == 0 ? 3 : 2)) void 
         float mx = -INFINITY;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
-            if constexpr (kBias == 2) {
+            if constexpr (kBias == 3) {
+                const f32x4_t t4 =
+                    *reinterpret_cast<const f32x4_t*>(bias_row + j0 + 16 * g + 4 * r4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s[4 * r4 + e] += t4[e];
+            }
+            if constexpr (kKeyBias) {
                 const f32x4_t t4 = *reinterpret_cast<const f32x4_t*>(bias_tile + 32 * kb +
                                                                      quad_slot(r4, g));
                 s[4 * r4 + 0] += t4.x;
@@ -519,7 +541,7 @@ template <typename T, int DPAD, int kBias, int kDrop, int kWin, int kSteps>
 int launch(const AttnArgs& a, hipStream_t st) {
     typedef TileStage<T, DPAD, kBN, kThreads> Stage;
     const size_t smem = (size_t)4 * kBN * Stage::kPitch * sizeof(T) +
-                        (kBias == 2 ? 2 * kBN * sizeof(float) : 0);
+                        (kBias == 2 || kBias == 4 ? 2 * kBN * sizeof(float) : 0);
     const int n_qt = (a.sq + kBM - 1) / kBM;
     const int64_t blocks = (int64_t)n_qt * a.batch * a.heads;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
@@ -531,7 +553,7 @@ int launch(const AttnArgs& a, hipStream_t st) {
     // (head groups: not where the kernel draws or applies dropout bits -- its workgroups run twice as
     // long there and a group's late heavy ones become the tail: 314 -> 350 us at bf16 B4 S2048 H32
     // D80 causal, p 0.1, 588 -> 667 us at fp16 B2 S4096 H32 D96)
-    set_dispatch_order(&ordered, blocks, (DPAD <= 64 && kDrop == 0) ? 3 : 2, kDrop == 0);
+    set_dispatch_order(&ordered, blocks, fwd_per_cu(DPAD, kBias, kDrop), kDrop == 0);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, ordered);
     return check_launch();
 }
@@ -548,6 +570,15 @@ int dispatch_flags(const AttnArgs& a, hipStream_t st) {
     if (a.has_bias) {
         // one build for both: with a bias the window-free build measured slower (it spills more
         // at head_dim 64 and 96: 266 against 185 us at bf16 B4 S2048 H32 D80 with a padding mask)
+        if (a.bias_type == SLAPO_BIAS_PREPARED) {
+            if (a.dropout == 1) return launch<T, DPAD, 3, 1, 2, kSteps>(a, st);
+            if (a.dropout == 2) return launch<T, DPAD, 3, 2, 2, kSteps>(a, st);
+            if (a.dropout == 3) return launch<T, DPAD, 3, 3, 2, kSteps>(a, st);
+            return launch<T, DPAD, 3, 0, 2, kSteps>(a, st);
+        }
+        if (a.bias_type != SLAPO_F32)  // one value per key, no dropout (checked by the caller)
+            return a.window <= 0 ? launch<T, DPAD, 4, 0, 0, kSteps>(a, st)
+                                 : launch<T, DPAD, 4, 0, 2, kSteps>(a, st);
         if (a.bs[2] == 0) {  // the bias depends on the key only
             if (a.dropout == 1) return launch<T, DPAD, 2, 1, 2, kSteps>(a, st);
             if (a.dropout == 2) return launch<T, DPAD, 2, 2, 2, kSteps>(a, st);

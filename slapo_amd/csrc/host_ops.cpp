@@ -174,7 +174,8 @@ struct Operand {
 
 struct AttnProblem {
     slapo_attn_params prm = {};
-    Tensor bias;  // fp32, addressed with prm.bias_strides (0 on broadcast dims)
+    Tensor bias;  // of type bias_type, addressed with prm.bias_strides (0 on broadcast dims)
+    int bias_type = SLAPO_F32;
     Dropout drop;
     at::ScalarType dtype = at::kFloat;
 
@@ -197,19 +198,50 @@ struct AttnProblem {
         prm.window = (int32_t)window;
         prm.scale = (float)scale;
     }
-    // Additive mask -> fp32, broadcast dims with stride 0.
-    void set_bias(const Tensor& mask) {
+    // Additive mask, broadcast dims with stride 0.  The fp32 kernels read any layout and type.  The
+    // 16-bit ones read one value per key, in the mask's own type at inference (no backward to follow,
+    // no dropout); a
+    // mask with values per query is prepared for them -- a pass over it that replaces the
+    // conversion to fp32 -- unless it is fp32 already and every (batch, head) has values of its
+    // own: then it is read once per direction, in place.
+    void set_bias(const Tensor& mask, bool infer) {
         if (!mask.defined()) return;
         TORCH_CHECK_VALUE(mask.dim() == 4,
                           "attention_mask must be 4-D ([B,1,1,Sk] or [B,H,Sq,Sk])");
-        bias = cast(mask, at::kFloat);
-        const int64_t want[4] = {b(), h(), sq(), sk()};
+        const at::ScalarType mt = mask.scalar_type();
+        const bool known = mt == at::kFloat || mt == at::kHalf || mt == at::kBFloat16;
+        const bool per_key = mask.size(2) == 1;
+        bias = known && (infer || !per_key || dtype == at::kFloat) ? mask : cast(mask, at::kFloat);
+        bias_type = dtype_code(bias.scalar_type());
+        const int64_t wanted[4] = {b(), h(), sq(), sk()};
         for (int i = 0; i < 4; ++i) {
             const int64_t n = bias.size(i);
-            TORCH_CHECK(n == want[i] || n == 1, "attention_mask of shape ", mask.sizes(),
+            TORCH_CHECK(n == wanted[i] || n == 1, "attention_mask of shape ", mask.sizes(),
                         " does not broadcast to [", b(), ", ", h(), ", ", sq(), ", ", sk(), "]");
-            prm.bias_strides[i] = n == 1 && want[i] != 1 ? 0 : bias.stride(i);
+            prm.bias_strides[i] = n == 1 && wanted[i] != 1 ? 0 : bias.stride(i);
         }
+        if (dtype == at::kFloat || per_key || empty() || sk() == 0) return;
+        const int64_t mb = prm.bias_strides[0] ? b() : 1, mh = prm.bias_strides[1] ? h() : 1;
+        const int64_t bytes =
+            (int64_t)slapo_amd_attn_prepared_bias_bytes(mb, mh, sq(), sk());
+        if (bytes == 0 || (bias_type == SLAPO_F32 && mb * mh == b() * h())) {
+            bias = cast(bias, at::kFloat);
+            for (int i = 0; i < 4; ++i)
+                if (prm.bias_strides[i]) prm.bias_strides[i] = bias.stride(i);
+            bias_type = SLAPO_F32;
+            return;
+        }
+        const Tensor rows = fresh({bytes / 4}, at::kFloat);
+        check(slapo_amd_attn_prepare_bias(cptr(bias), bias_type, prm.bias_strides, mb, mh, sq(),
+                                          sk(), static_cast<float*>(mptr(rows)), stream_of(bias)),
+              "slapo_amd_attn_prepare_bias");
+        bias = rows;
+        bias_type = SLAPO_BIAS_PREPARED;
+        const int64_t pitch = (sk() + 63) / 64 * 64, plane = (sq() + 63) / 64 * 64 * pitch;
+        prm.bias_strides[0] = mb > 1 ? mh * plane : 0;
+        prm.bias_strides[1] = mh > 1 ? plane : 0;
+        prm.bias_strides[2] = pitch;
+        prm.bias_strides[3] = 1;
     }
     // Draws, once the geometry is known: F.dropout leaves the generator alone for an empty tensor.
     void set_dropout(Dropout&& in, const at::Device& dev) {
@@ -258,11 +290,10 @@ AttnResult launch_attn_fwd(AttnProblem& a, const Tensor& q, const Tensor& k, con
     }
     const size_t ws_bytes = slapo_amd_attn_fwd_workspace_bytes(&prm);
     const Tensor ws = ws_bytes ? floats((int64_t)(ws_bytes / 4)) : Tensor();
-    check(slapo_amd_attn_fwd_ws(&prm, cptr(q), cptr(k), cptr(v),
-                                static_cast<const float*>(cptr(a.bias)), mptr(r.out),
-                                static_cast<float*>(mptr(r.lse)), mptr(ws), ws_bytes,
+    check(slapo_amd_attn_fwd_ex(&prm, cptr(q), cptr(k), cptr(v), cptr(a.bias), a.bias_type,
+                                mptr(r.out), static_cast<float*>(mptr(r.lse)), mptr(ws), ws_bytes,
                                 stream_of(q)),
-          "slapo_amd_attn_fwd_ws");
+          "slapo_amd_attn_fwd_ex");
     return r;
 }
 
@@ -276,11 +307,11 @@ void launch_attn_bwd(AttnProblem& a, const Tensor& q, const Tensor& k, const Ten
     a.prm.keep_mask = mptr(keep_mask);
     const size_t ws_bytes = slapo_amd_attn_bwd_workspace_bytes(&a.prm);
     const Tensor ws = floats((int64_t)(ws_bytes / 4));
-    check(slapo_amd_attn_bwd(&a.prm, cptr(q), cptr(k), cptr(v),
-                             static_cast<const float*>(cptr(a.bias)), cptr(out), cptr(dout),
-                             static_cast<const float*>(cptr(lse)), mptr(dst[0]), mptr(dst[1]),
-                             mptr(dst[2]), ds[0], ds[1], ds[2], mptr(ws), ws_bytes, stream_of(q)),
-          "slapo_amd_attn_bwd");
+    check(slapo_amd_attn_bwd_ex(&a.prm, cptr(q), cptr(k), cptr(v), cptr(a.bias), a.bias_type,
+                                cptr(out), cptr(dout), static_cast<const float*>(cptr(lse)),
+                                mptr(dst[0]), mptr(dst[1]), mptr(dst[2]), ds[0], ds[1], ds[2],
+                                mptr(ws), ws_bytes, stream_of(q)),
+          "slapo_amd_attn_bwd_ex");
 }
 
 // Forward saves q, k, v, bias, out, lse, the (seed, offset) pair and, with dropout, the keep bits;
@@ -342,7 +373,7 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor
         std::memcpy(a.prm.q_strides, oq.strides, sizeof oq.strides);
         std::memcpy(a.prm.k_strides, ok.strides, sizeof ok.strides);
         std::memcpy(a.prm.v_strides, ov.strides, sizeof ov.strides);
-        a.set_bias(mask);
+        a.set_bias(mask, !need && drop.p == 0.0);
         a.set_dropout(std::move(drop), q.device());
         // a mask geometry that the forward kernel would draw score by score is drawn ahead of it,
         // which takes the buffer also where no backward will read it
