@@ -172,6 +172,14 @@ int slapo_amd_bias_dropout_residual_ln_bwd(const void* grad_y, const void* z, co
                                            const slapo_dropout_plan* plan, void* stream);
 
 /* ------------------------------------------------------------------------------------------
+ * FusedQKV's re-layout (slapo/op/linear.py:41-57): packed[3 i + {0, 1, 2}] <-> q[i], k[i], v[i],
+ * i < n, all dense; any dtype of SLAPO_*. */
+int slapo_amd_qkv_split(const void* packed, void* q, void* k, void* v, int64_t n, int dtype,
+                        void* stream);
+int slapo_amd_qkv_join(const void* q, const void* k, const void* v, void* packed, int64_t n,
+                       int dtype, void* stream);
+
+/* ------------------------------------------------------------------------------------------
  * Vocab-parallel cross entropy, the part computed on one shard [rows, vocab] of the logits
  * (vocabulary ids vocab_start .. vocab_start + vocab - 1).  Replaces the tensor passes of
  * _VocabParallelCrossEntropy.forward / .backward (slapo/op/cross_entropy.py:21-124).
@@ -188,6 +196,11 @@ int slapo_amd_bias_dropout_residual_ln_bwd(const void* grad_y, const void* z, co
 int slapo_amd_vocab_ce_fwd(const void* logits, const int64_t* target, float* row_max,
                            float* sum_exp, float* predicted, float* sum_logits, int64_t rows,
                            int64_t vocab, int64_t vocab_start, int dtype, void* stream);
+/* The forward where the shard is the whole vocabulary: the loss [rows] itself (label-smoothed where
+ * label_smoothing > 0: :79-88), and row_max and 1 / sum_exp for the backward. */
+int slapo_amd_vocab_ce_loss(const void* logits, const int64_t* target, float* loss,
+                            float* row_max, float* inv_sum_exp, int64_t rows, int64_t vocab,
+                            double label_smoothing, int dtype, void* stream);
 int slapo_amd_vocab_ce_bwd(const void* logits, const int64_t* target, const float* row_max,
                            const float* inv_sum_exp, const float* grad_loss, void* grad_logits,
                            int64_t rows, int64_t vocab, int64_t vocab_start,

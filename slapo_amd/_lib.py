@@ -119,6 +119,12 @@ PROTOTYPES = {
         ctypes.c_int,
         [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, ctypes.c_int, c_vp],
     ),
+    "slapo_amd_vocab_ce_loss": (
+        ctypes.c_int,
+        [c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, ctypes.c_double, ctypes.c_int, c_vp],
+    ),
+    "slapo_amd_qkv_split": (ctypes.c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, ctypes.c_int, c_vp]),
+    "slapo_amd_qkv_join": (ctypes.c_int, [c_vp, c_vp, c_vp, c_vp, c_i64, ctypes.c_int, c_vp]),
     "slapo_amd_vocab_ce_bwd": (
         ctypes.c_int,
         [c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, ctypes.c_double, ctypes.c_int,

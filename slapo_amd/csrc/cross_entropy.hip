@@ -68,12 +68,34 @@ struct CeVec {
     T v[V];
 };
 
-// Forward: m[row], s[row], predicted[row], sum_x[row] of one shard.  target may be any integer;
-// it counts when vocab_start <= target < vocab_start + n.
-template <typename T, int V, int kCeThreads>
+// Where a row's results go.  Of a shard: maximum, sum of exponentials, target's logit, sum of logits.
+// Of the whole vocabulary: the loss, maximum and 1 / sum that the backward reads, in place of five
+// elementwise launches over [tokens] (23 us beside the 134 us of the row pass at 8192 x 50257).
+struct ShardStats {
+    float *m, *s, *predicted, *sum_x;
+    __device__ __forceinline__ void put(int64_t row, float mm, float ss, float pred, float xx,
+                                        int) const {
+        m[row] = mm, s[row] = ss, predicted[row] = pred, sum_x[row] = xx;
+    }
+};
+struct LossStats {
+    float *loss, *m, *inv_s;
+    float smoothing;  // slapo/op/cross_entropy.py:79-88: alpha K / (K - 1), 0 without smoothing
+    __device__ __forceinline__ void put(int64_t row, float mm, float ss, float pred, float xx,
+                                        int n) const {
+        const float log_s = logf(ss);
+        float v = log_s + (mm - pred);  // mm - pred first: exact where the logits sit far from zero
+        if (smoothing > 0.f)
+            v = (1.0f - smoothing) * v - smoothing * ((xx / (float)n - mm) - log_s);
+        loss[row] = v, m[row] = mm, inv_s[row] = 1.0f / ss;
+    }
+};
+
+// Forward: one block per row.  target may be any integer; it counts when vocab_start <= target <
+// vocab_start + n.
+template <typename T, int V, int kCeThreads, typename Out>
 __global__ __launch_bounds__(kCeThreads) void ce_fwd_kernel(
-    const T* __restrict__ logits, const int64_t* __restrict__ target, float* __restrict__ m_out,
-    float* __restrict__ s_out, float* __restrict__ pred_out, float* __restrict__ sumx_out, int n,
+    const T* __restrict__ logits, const int64_t* __restrict__ target, Out out, int n,
     int64_t vocab_start) {
     const int64_t row = blockIdx.x;
     const T* x = logits + row * (int64_t)n;
@@ -149,11 +171,8 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd_kernel(
             ce_merge(mm, ss, red[0][w], red[1][w]);
             xx += red[2][w];
         }
-        m_out[row] = mm;
-        s_out[row] = ss;
-        sumx_out[row] = xx;
         const int64_t t = target[row] - vocab_start;
-        pred_out[row] = (t >= 0 && t < n) ? Elem<T>::to_f32(x[t]) : 0.f;
+        out.put(row, mm, ss, (t >= 0 && t < n) ? Elem<T>::to_f32(x[t]) : 0.f, xx, n);
     }
 }
 
@@ -229,19 +248,36 @@ inline bool ce_dims_ok(int64_t rows, int64_t n) {
     return rows > 0 && n > 0 && rows <= 0x7FFFFFFF && n <= 0x7FFFFFFF;
 }
 
-template <typename T>
-int ce_fwd_dispatch(const void* logits, const int64_t* target, float* m, float* s, float* pred,
-                    float* sumx, int64_t rows, int64_t n, int64_t vocab_start, hipStream_t st) {
-#define SLAPO_CE_FWD(THREADS)                                                                   \
-    hipLaunchKernelGGL((ce_fwd_kernel<T, Elem<T>::kPerVec, THREADS>), dim3((unsigned)rows),     \
-                       dim3(THREADS), 0, st, (const T*)logits, target, m, s, pred, sumx, (int)n, \
-                       vocab_start)
+template <typename T, typename Out>
+int ce_fwd_dispatch(const void* logits, const int64_t* target, const Out& out, int64_t rows,
+                    int64_t n, int64_t vocab_start, hipStream_t st) {
+    if (reinterpret_cast<uintptr_t>(logits) & (sizeof(T) - 1)) return SLAPO_ERR_ALIGN;
+#define SLAPO_CE_FWD(THREADS)                                                                    \
+    hipLaunchKernelGGL((ce_fwd_kernel<T, Elem<T>::kPerVec, THREADS, Out>), dim3((unsigned)rows), \
+                       dim3(THREADS), 0, st, (const T*)logits, target, out, (int)n, vocab_start)
     if (n >= 16384)
         SLAPO_CE_FWD(512);
     else
         SLAPO_CE_FWD(256);
 #undef SLAPO_CE_FWD
     return check_launch();
+}
+template <typename Out>
+int ce_fwd_typed(const void* logits, const int64_t* target, const Out& out, int64_t rows, int64_t n,
+                 int64_t vocab_start, int dtype, void* stream) {
+    if (!ce_dims_ok(rows, n)) return SLAPO_ERR_SHAPE;
+    hipStream_t st = (hipStream_t)stream;
+    switch (dtype) {
+        case SLAPO_F32: return ce_fwd_dispatch<float>(logits, target, out, rows, n, vocab_start, st);
+        case SLAPO_F16: return ce_fwd_dispatch<f16_t>(logits, target, out, rows, n, vocab_start, st);
+        case SLAPO_BF16:
+            return ce_fwd_dispatch<bf16_t>(logits, target, out, rows, n, vocab_start, st);
+        default: return SLAPO_ERR_DTYPE;
+    }
+}
+// slapo/op/cross_entropy.py:112-116: smoothing = alpha K / (K - 1) with K the shard's size
+double effective_smoothing(double label_smoothing, int64_t vocab) {
+    return label_smoothing > 0.0 ? label_smoothing * (double)vocab / (double)(vocab - 1) : 0.0;
 }
 
 template <typename T>
@@ -277,24 +313,20 @@ extern "C" int slapo_amd_vocab_ce_fwd(const void* logits, const int64_t* target,
                                       void* stream) {
     if (!logits || !target || !row_max || !sum_exp || !predicted || !sum_logits)
         return SLAPO_ERR_ARG;
-    if (!ce_dims_ok(rows, vocab)) return SLAPO_ERR_SHAPE;
-    hipStream_t st = (hipStream_t)stream;
-    switch (dtype) {
-        case SLAPO_F32:
-            if (reinterpret_cast<uintptr_t>(logits) & 3) return SLAPO_ERR_ALIGN;
-            return ce_fwd_dispatch<float>(logits, target, row_max, sum_exp, predicted, sum_logits,
-                                          rows, vocab, vocab_start, st);
-        case SLAPO_F16:
-            if (reinterpret_cast<uintptr_t>(logits) & 1) return SLAPO_ERR_ALIGN;
-            return ce_fwd_dispatch<f16_t>(logits, target, row_max, sum_exp, predicted, sum_logits,
-                                          rows, vocab, vocab_start, st);
-        case SLAPO_BF16:
-            if (reinterpret_cast<uintptr_t>(logits) & 1) return SLAPO_ERR_ALIGN;
-            return ce_fwd_dispatch<bf16_t>(logits, target, row_max, sum_exp, predicted,
-                                           sum_logits, rows, vocab, vocab_start, st);
-        default:
-            return SLAPO_ERR_DTYPE;
-    }
+    const ShardStats out{row_max, sum_exp, predicted, sum_logits};
+    return ce_fwd_typed(logits, target, out, rows, vocab, vocab_start, dtype, stream);
+}
+
+extern "C" int slapo_amd_vocab_ce_loss(const void* logits, const int64_t* target, float* loss,
+                                       float* row_max, float* inv_sum_exp, int64_t rows,
+                                       int64_t vocab, double label_smoothing, int dtype,
+                                       void* stream) {
+    if (!logits || !target || !loss || !row_max || !inv_sum_exp) return SLAPO_ERR_ARG;
+    if (!(label_smoothing >= 0.0 && label_smoothing < 1.0)) return SLAPO_ERR_ARG;
+    if (label_smoothing > 0.0 && vocab < 2) return SLAPO_ERR_SHAPE;
+    const LossStats out{loss, row_max, inv_sum_exp,
+                        (float)effective_smoothing(label_smoothing, vocab)};
+    return ce_fwd_typed(logits, target, out, rows, vocab, 0, dtype, stream);
 }
 
 extern "C" int slapo_amd_vocab_ce_bwd(const void* logits, const int64_t* target,
@@ -307,9 +339,7 @@ extern "C" int slapo_amd_vocab_ce_bwd(const void* logits, const int64_t* target,
     if (!ce_dims_ok(rows, vocab)) return SLAPO_ERR_SHAPE;
     if (!(label_smoothing >= 0.0 && label_smoothing < 1.0)) return SLAPO_ERR_ARG;
     if (label_smoothing > 0.0 && vocab < 2) return SLAPO_ERR_SHAPE;
-    // slapo/op/cross_entropy.py:112-116: smoothing = alpha K / (K - 1) with K the shard's size
-    const double smoothing =
-        label_smoothing > 0.0 ? label_smoothing * (double)vocab / (double)(vocab - 1) : 0.0;
+    const double smoothing = effective_smoothing(label_smoothing, vocab);
     const float onehot_scale = (float)(1.0 - smoothing);
     const float flat = (float)(smoothing / (double)vocab);
     hipStream_t st = (hipStream_t)stream;

@@ -382,7 +382,15 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const float* __restr
 // unfused modules compute from the stored sum; z is also what the backward reads.
 // ----------------------------------------------------------------------------------------
 constexpr int kLnChunks = 4;         // 16-byte chunks per thread and row (guarded against cols)
-constexpr int kLnRowsPerBlock = 16;  // backward: rows walked by one block (column partial sums)
+// Backward: rows that one block walks before it writes its column sums.  16, or fewer where that would
+// leave the device less than two blocks per CU -- the rows of a block run one after the other (a
+// block-wide row at a time above 64 V * 2 columns, eight wavefront rows at a time below): fp16
+// 384 x 2560 in 24 blocks took @LNB@.
+inline int ln_rows_per_block(int64_t rows, bool wide) {
+    int rpb = 16;
+    while (rpb > (wide ? 2 : 8) && (rows + rpb - 1) / rpb < 512) rpb /= 2;
+    return rpb;
+}
 
 // Sum over the 64 lanes, on every lane, without LDS traffic: butterflies inside the 16-lane
 // rows through DPP (quad permutes, row rotations), then the four row sums through v_readlane.
@@ -519,7 +527,7 @@ __global__ __launch_bounds__(256) void bias_dropout_residual_ln_fwd_kernel(
 // Backward of the above.  With xh = (z - mean) rstd and g = dy gamma:
 //   dz = rstd (g - mean_c(g) - xh mean_c(g xh)),  dresidual = dz,  dx = dz keep / (1 - p),
 //   dgamma = sum_r dy xh,  dbeta = sum_r dy,  dbias = sum_r dx.
-// A block walks kLnRowsPerBlock rows and keeps the three column sums of its threads in
+// A block walks rows_per_block rows and keeps the three column sums of its threads in
 // registers; they leave as one fp32 partial row triple per block ([block][3][cols]: dgamma, dbeta,
 // dbias) for ln_finish_kernel.  No atomics: the result does not depend on scheduling.
 // NV = 16-byte chunks per thread and row (1, 2 or 4, the smallest that covers cols): the column
@@ -530,12 +538,13 @@ __global__ __launch_bounds__(kThreads, (kThreads == 512 && kDrop != 2) ? 4 : 1)
 void bias_dropout_residual_ln_bwd_kernel(
     const T* __restrict__ dy, const T* __restrict__ z, const float* __restrict__ mean,
     const float* __restrict__ rstd, const T* __restrict__ gamma, T* __restrict__ dx,
-    T* __restrict__ dres, float* __restrict__ partial, int64_t rows, int cols, DropoutState s) {
+    T* __restrict__ dres, float* __restrict__ partial, int64_t rows, int cols, int rows_per_block,
+    DropoutState s) {
     if constexpr (kDrop != 0) resolve_device_state(s);
     static_assert(TPR == 256 ? kThreads == 256 : (kThreads == 256 || kThreads == 512),
                   "a block is one wide row, or four or eight wavefront rows");
     constexpr int kRows = kThreads / TPR;  // rows in flight per block
-    constexpr int kIters = kLnRowsPerBlock / kRows;
+    const int n_iters = rows_per_block / kRows;
     constexpr int kCombCols = TPR == 64 ? 64 * V * NV : 1;
     __shared__ float red[2][2][4];
     __shared__ float comb[4 * 3 * kCombCols];
@@ -551,7 +560,7 @@ void bias_dropout_residual_ln_bwd_kernel(
         for (int i = 0; i < V; ++i) acc_g[u][i] = 0.f, acc_b[u][i] = 0.f, acc_x[u][i] = 0.f;
     }
     const float inv_n = 1.0f / (float)cols;
-    const int64_t row0 = (int64_t)blockIdx.x * kLnRowsPerBlock + rr;
+    const int64_t row0 = (int64_t)blockIdx.x * rows_per_block + rr;
 
     // rows it + 1 and it + 2 are in flight while row it is processed
     Chunk<T, V> gy[NV], zz[NV], gy_n1[NV], zz_n1[NV], gy_n2[NV], zz_n2[NV];
@@ -572,12 +581,12 @@ void bias_dropout_residual_ln_bwd_kernel(
         }
     };
     request(row0, gy, zz, m, rs);
-    if (kIters > 1) request(row0 + kRows, gy_n1, zz_n1, m_n1, rs_n1);
+    if (n_iters > 1) request(row0 + kRows, gy_n1, zz_n1, m_n1, rs_n1);
 #pragma unroll 1
-    for (int it = 0; it < kIters; ++it) {
+    for (int it = 0; it < n_iters; ++it) {
         const int64_t row = row0 + it * kRows;
         const bool row_ok = row < rows;  // uniform per wavefront
-        if (it + 2 < kIters) request(row + 2 * kRows, gy_n2, zz_n2, m_n2, rs_n2);
+        if (it + 2 < n_iters) request(row + 2 * kRows, gy_n2, zz_n2, m_n2, rs_n2);
         float s1 = 0.f, s2 = 0.f;
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
@@ -973,14 +982,15 @@ int ln_bwd_dispatch(const void* dy, const void* z, const float* mean, const floa
     for (const void* p : {dy, z, gamma, (const void*)dx, (const void*)dres})
         if (p && !aligned16(p)) return SLAPO_ERR_ALIGN;
     const bool want_sums = dgamma || dbeta || dbias;
-    const int64_t n_blocks = (rows + kLnRowsPerBlock - 1) / kLnRowsPerBlock;
+    const int rpb = ln_rows_per_block(rows, wide);
+    const int64_t n_blocks = (rows + rpb - 1) / rpb;
     float* partial = want_sums ? (float*)ws : nullptr;
     const int mode = !dropout ? 0 : (s.g_shift >= 0 && s.t_shift >= 0) ? 1 : 2;
 #define SLAPO_LAUNCH_LNB(NV, TPR, MODE)                                                         \
     hipLaunchKernelGGL(                                                                         \
         (bias_dropout_residual_ln_bwd_kernel<T, V, NV, TPR, MODE, (TPR == 64 ? 512 : 256)>),    \
         dim3((unsigned)n_blocks), dim3(TPR == 64 ? 512 : 256), 0, st, (const T*)dy,             \
-        (const T*)z, mean, rstd, (const T*)gamma, (T*)dx, (T*)dres, partial, rows, (int)cols, s)
+        (const T*)z, mean, rstd, (const T*)gamma, (T*)dx, (T*)dres, partial, rows, (int)cols, rpb, s)
 #define SLAPO_LAUNCH_LNB_MODE(NV, TPR)            \
     do {                                          \
         if (mode == 0) SLAPO_LAUNCH_LNB(NV, TPR, 0); \
@@ -1107,7 +1117,8 @@ extern "C" int slapo_amd_bias_dropout_residual_bwd(const void* grad, void* dx, v
 
 extern "C" size_t slapo_amd_ln_bwd_workspace_bytes(int64_t rows, int64_t cols) {
     if (rows <= 0 || cols <= 0) return 0;
-    const int64_t n_blocks = (rows + kLnRowsPerBlock - 1) / kLnRowsPerBlock;
+    const int rpb = ln_rows_per_block(rows, true);  // the most partial rows, whatever the type
+    const int64_t n_blocks = (rows + rpb - 1) / rpb;
     return (size_t)n_blocks * 3 * (size_t)cols * sizeof(float);
 }
 

@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
@@ -25,8 +26,12 @@
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
+#include <array>
+#include <cmath>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
+#include <vector>
 
 #include "../../include/slapo_amd.h"
 
@@ -152,26 +157,6 @@ std::shared_ptr<T> make_node(bool wanted, const Inputs&... inputs) {
 
 // ---- attention ----------------------------------------------------------------------------------
 
-// Four-dimensional [batch, seqlen, heads, head_dim] operand as the kernels address it.
-struct Operand {
-    Tensor t;
-    int64_t strides[3];
-
-    void take(const Tensor& in) {
-        t = in;
-        const auto st = t.strides();
-        bool usable = t.size(3) <= 1 || st[3] == 1;
-        if (usable) {
-            const int64_t esz = t.element_size();
-            usable = aligned(t) && st[0] * esz % 16 == 0 && st[1] * esz % 16 == 0 &&
-                     st[2] * esz % 16 == 0;
-        }
-        if (!usable) t = t.contiguous();
-        const auto s2 = t.strides();
-        strides[0] = s2[0], strides[1] = s2[1], strides[2] = s2[2];
-    }
-};
-
 struct AttnProblem {
     slapo_attn_params prm = {};
     Tensor bias;  // of type bias_type, addressed with prm.bias_strides (0 on broadcast dims)
@@ -186,17 +171,15 @@ struct AttnProblem {
     int64_t d() const { return prm.head_dim; }
     bool empty() const { return b() * h() * sq() * d() == 0; }
 
-    void describe(const Tensor& q, const Tensor& k, bool causal, int64_t window, double scale) {
-        dtype = q.scalar_type();
+    void describe(at::ScalarType type, int64_t b, int64_t sq, int64_t sk, int64_t h, int64_t d,
+                  bool causal, int64_t window, std::optional<double> scale) {
+        dtype = type;
         prm.dtype = dtype_code(dtype);
-        prm.batch = (int32_t)q.size(0);
-        prm.seqlen_q = (int32_t)q.size(1);
-        prm.heads = (int32_t)q.size(2);
-        prm.head_dim = (int32_t)q.size(3);
-        prm.seqlen_k = (int32_t)k.size(1);
+        prm.batch = (int32_t)b, prm.heads = (int32_t)h, prm.head_dim = (int32_t)d;
+        prm.seqlen_q = (int32_t)sq, prm.seqlen_k = (int32_t)sk;
         prm.causal = causal ? 1 : 0;
         prm.window = (int32_t)window;
-        prm.scale = (float)scale;
+        prm.scale = (float)(scale ? *scale : 1.0 / std::sqrt((double)d));
     }
     // Additive mask, broadcast dims with stride 0.  The fp32 kernels read any layout and type.  The
     // 16-bit ones read one value per key, in the mask's own type at inference (no backward to follow,
@@ -271,11 +254,58 @@ struct AttnResult {
     Tensor out, lse, keep_mask;
 };
 
-AttnResult launch_attn_fwd(AttnProblem& a, const Tensor& q, const Tensor& k, const Tensor& v,
+// The three operands of a call: tensors of their own, or views of one packed [B, S, H, 3 D] tensor.
+struct Operands {
+    Tensor t[3];
+    const void* ptr[3] = {nullptr, nullptr, nullptr};
+    bool packed = false;
+
+    void take(AttnProblem& a, const Tensor& q, const Tensor& k, const Tensor& v) {
+        const Tensor* in[3] = {&q, &k, &v};
+        int64_t* strides[3] = {a.prm.q_strides, a.prm.k_strides, a.prm.v_strides};
+        for (int i = 0; i < 3; ++i) {
+            t[i] = usable(*in[i]);
+            ptr[i] = cptr(t[i]);
+            for (int j = 0; j < 3; ++j) strides[i][j] = t[i].stride(j);
+        }
+    }
+    void take_packed(AttnProblem& a, const Tensor& qkv) {
+        packed = true;
+        t[0] = qkv.contiguous();
+        if (!aligned(t[0])) t[0] = t[0].clone();
+        packed_views(a, cptr(t[0]), ptr, a.prm.q_strides, a.prm.k_strides, a.prm.v_strides);
+    }
+    // q, k, v (or their gradients) inside a dense packed buffer
+    template <typename P>
+    static void packed_views(const AttnProblem& a, P* base, P* (&at)[3], int64_t* qs, int64_t* ks,
+                             int64_t* vs) {
+        const int64_t esz = a.prm.dtype == SLAPO_F32 ? 4 : 2, row = 3 * a.h() * a.d();
+        const int64_t st[3] = {a.sq() * row, row, 3 * a.d()};
+        for (int64_t* s : {qs, ks, vs}) std::memcpy(s, st, sizeof st);
+        typedef std::conditional_t<std::is_const<P>::value, const char, char> byte;
+        for (int i = 0; i < 3; ++i)
+            at[i] = base ? reinterpret_cast<byte*>(base) + i * a.d() * esz : nullptr;
+    }
+
+ private:
+    // Strided [B, S, H, D] views are read as they are while their rows stay 16-byte aligned.
+    static Tensor usable(const Tensor& in) {
+        const auto st = in.strides();
+        bool ok = in.size(3) <= 1 || st[3] == 1;
+        if (ok) {
+            const int64_t esz = in.element_size();
+            ok = aligned(in) && st[0] * esz % 16 == 0 && st[1] * esz % 16 == 0 &&
+                 st[2] * esz % 16 == 0;
+        }
+        return ok ? in : in.contiguous();
+    }
+};
+
+AttnResult launch_attn_fwd(AttnProblem& a, const Operands& x, at::IntArrayRef out_sizes,
                            bool save_mask, int64_t save_mask_max) {
     AttnResult r;
     slapo_attn_params& prm = a.prm;
-    r.out = fresh({a.b(), a.sq(), a.h(), a.d()}, q.scalar_type());
+    r.out = fresh(out_sizes, a.dtype);
     r.lse = fresh({a.b(), a.h(), a.sq()}, at::kFloat);
     prm.o_strides[0] = a.sq() * a.h() * a.d();
     prm.o_strides[1] = a.h() * a.d();
@@ -290,68 +320,108 @@ AttnResult launch_attn_fwd(AttnProblem& a, const Tensor& q, const Tensor& k, con
     }
     const size_t ws_bytes = slapo_amd_attn_fwd_workspace_bytes(&prm);
     const Tensor ws = ws_bytes ? floats((int64_t)(ws_bytes / 4)) : Tensor();
-    check(slapo_amd_attn_fwd_ex(&prm, cptr(q), cptr(k), cptr(v), cptr(a.bias), a.bias_type,
+    check(slapo_amd_attn_fwd_ex(&prm, x.ptr[0], x.ptr[1], x.ptr[2], cptr(a.bias), a.bias_type,
                                 mptr(r.out), static_cast<float*>(mptr(r.lse)), mptr(ws), ws_bytes,
-                                stream_of(q)),
+                                stream_of(r.out)),
           "slapo_amd_attn_fwd_ex");
     return r;
 }
 
-// dq / dk / dv: destinations with their three outer strides.
-void launch_attn_bwd(AttnProblem& a, const Tensor& q, const Tensor& k, const Tensor& v,
-                     const Tensor& out, const Tensor& lse, const Tensor& keep_mask,
-                     const Tensor& grad, const Tensor (&dst)[3], const int64_t (&ds)[3][3]) {
-    Tensor dout = grad.scalar_type() == a.dtype ? grad.contiguous()
-                                                : grad.to(a.dtype).contiguous();
+// dst, ds: where dq / dk / dv go and their three outer strides.
+void launch_attn_bwd(AttnProblem& a, const Operands& x, const Tensor& out, const Tensor& lse,
+                     const Tensor& keep_mask, const Tensor& grad, void* const (&dst)[3],
+                     const int64_t (&ds)[3][3]) {
+    Tensor dout = cast(grad, a.dtype).contiguous();
     if (!aligned(dout)) dout = dout.clone();
     a.prm.keep_mask = mptr(keep_mask);
     const size_t ws_bytes = slapo_amd_attn_bwd_workspace_bytes(&a.prm);
     const Tensor ws = floats((int64_t)(ws_bytes / 4));
-    check(slapo_amd_attn_bwd_ex(&a.prm, cptr(q), cptr(k), cptr(v), cptr(a.bias), a.bias_type,
+    check(slapo_amd_attn_bwd_ex(&a.prm, x.ptr[0], x.ptr[1], x.ptr[2], cptr(a.bias), a.bias_type,
                                 cptr(out), cptr(dout), static_cast<const float*>(cptr(lse)),
-                                mptr(dst[0]), mptr(dst[1]), mptr(dst[2]), ds[0], ds[1], ds[2],
-                                mptr(ws), ws_bytes, stream_of(q)),
+                                dst[0], dst[1], dst[2], ds[0], ds[1], ds[2], mptr(ws), ws_bytes,
+                                stream_of(out)),
           "slapo_amd_attn_bwd_ex");
 }
 
-// Forward saves q, k, v, bias, out, lse, the (seed, offset) pair and, with dropout, the keep bits;
-// the backward recomputes the probabilities from lse and reads (or regenerates) the dropout mask --
-// it never draws.
+// Forward saves q, k, v (or the packed tensor), bias, out, lse, the (seed, offset) pair and, with
+// dropout, the keep bits; the backward recomputes the probabilities from lse and reads (or
+// regenerates) the dropout mask -- it never draws.  The gradient of a packed tensor is written in
+// place as three strided views: no concatenation afterwards.
 struct AttnBackward : Node {
     AttnProblem a;
-    SavedVariable q, k, v, bias, out, lse, keep_mask, state;
+    SavedVariable x[3], bias, out, lse, keep_mask, state;
+    bool packed = false;
 
     std::string name() const override { return "HipAttentionBackward"; }
     void release_variables() override {
         std::lock_guard<std::mutex> lock(mutex_);
-        for (SavedVariable* s : {&q, &k, &v, &bias, &out, &lse, &keep_mask, &state})
+        for (SavedVariable* s : {&x[0], &x[1], &x[2], &bias, &out, &lse, &keep_mask, &state})
             s->reset_data();
+    }
+    void save(const Operands& in, AttnProblem& problem, const AttnResult& r) {
+        torch::autograd::set_history(r.out, getptr());
+        packed = in.packed;
+        for (int i = 0; i < (packed ? 1 : 3); ++i) x[i] = keep(in.t[i]);
+        bias = keep(problem.bias), lse = keep(r.lse), keep_mask = keep(r.keep_mask);
+        state = keep(problem.drop.state);
+        out = keep(r.out, true);
+        problem.bias = Tensor(), problem.drop.state = Tensor();
+        a = problem;
     }
     variable_list apply(variable_list&& grads) override {
         std::lock_guard<std::mutex> lock(mutex_);
-        variable_list res(3);
+        variable_list res(packed ? 1 : 3);
         if (!grads[0].defined()) return res;
-        const Tensor tq = q.unpack(), tk = k.unpack(), tv = v.unpack();
-        const Tensor tout = out.unpack(getptr()), tlse = lse.unpack();
         AttnProblem call = a;
-        call.bias = bias.unpack();
-        call.drop.state = state.unpack();
-        if (call.drop.state.defined()) call.prm.plan.rng_state = call.drop.state.const_data_ptr();
-        const c10::OptionalDeviceGuard guard(tq.device());
-        const Tensor dst[3] = {fresh_like(tq), fresh_like(tk), fresh_like(tv)};
-        if (dst[0].numel() == 0 || dst[1].numel() == 0) {
-            for (const Tensor& t : dst) t.zero_();
+        Operands in;
+        Tensor dst[3];
+        void* dst_ptr[3];
+        int64_t ds[3][3];
+        const Tensor tout = out.unpack(getptr()), tlse = lse.unpack();
+        const c10::OptionalDeviceGuard guard(tout.device());
+        if (packed) {
+            in.take_packed(call, x[0].unpack());
+            dst[0] = fresh_like(in.t[0]);
+            Operands::packed_views<void>(call, mptr(dst[0]), dst_ptr, ds[0], ds[1], ds[2]);
         } else {
-            int64_t ds[3][3];
-            for (int i = 0; i < 3; ++i)
+            in.take(call, x[0].unpack(), x[1].unpack(), x[2].unpack());
+            for (int i = 0; i < 3; ++i) {
+                dst[i] = fresh_like(in.t[i]);
+                dst_ptr[i] = mptr(dst[i]);
                 for (int j = 0; j < 3; ++j) ds[i][j] = dst[i].stride(j);
-            launch_attn_bwd(call, tq, tk, tv, tout, tlse, keep_mask.unpack(), grads[0], dst, ds);
+            }
         }
-        for (int i = 0; i < 3; ++i)
+        if (call.empty() || call.sk() == 0) {
+            for (const Tensor& t : dst)
+                if (t.defined()) t.zero_();
+        } else {
+            call.bias = bias.unpack();
+            call.drop.state = state.unpack();
+            if (call.drop.state.defined())
+                call.prm.plan.rng_state = call.drop.state.const_data_ptr();
+            launch_attn_bwd(call, in, tout, tlse, keep_mask.unpack(), grads[0], dst_ptr, ds);
+        }
+        for (size_t i = 0; i < res.size(); ++i)
             if (task_should_compute_output(i)) res[i] = dst[i];
         return res;
     }
 };
+
+// What the two forms of the call share once the problem is described and the operands are taken.
+AttnResult run_attention(AttnProblem& a, const Operands& x, at::IntArrayRef out_sizes,
+                         const Tensor& mask, Dropout&& drop, bool need, bool save_mask,
+                         int64_t save_mask_max) {
+    a.set_bias(mask, !need && drop.p == 0.0);
+    a.set_dropout(std::move(drop), x.t[0].device());
+    // a mask geometry that the forward kernel would draw score by score is drawn ahead of it, which
+    // takes the buffer also where no backward will read it
+    const slapo_dropout_plan& plan = a.drop.plan;
+    const bool per_score = a.drop.p > 0.0 &&
+                           (plan.vec < 4 || a.sk() % 4 != 0 ||
+                            (plan.total_threads & (plan.total_threads - 1)) != 0);
+    return launch_attn_fwd(a, x, out_sizes, save_mask && a.drop.p < 1.0 && (need || per_score),
+                           save_mask_max);
+}
 
 Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask,
                  bool causal, int64_t window, std::optional<double> scale, Dropout&& drop,
@@ -363,37 +433,170 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor
     auto node = make_node<AttnBackward>(need, q, k, v);
     AttnProblem a;
     AttnResult r;
-    Operand oq, ok, ov;
+    Operands x;
     {
         at::AutoDispatchBelowADInplaceOrView below;
         const c10::OptionalDeviceGuard guard(q.device());
-        a.describe(q, k, causal, window,
-                   scale ? *scale : 1.0 / std::sqrt((double)q.size(3)));
-        oq.take(q), ok.take(k), ov.take(v);
-        std::memcpy(a.prm.q_strides, oq.strides, sizeof oq.strides);
-        std::memcpy(a.prm.k_strides, ok.strides, sizeof ok.strides);
-        std::memcpy(a.prm.v_strides, ov.strides, sizeof ov.strides);
-        a.set_bias(mask, !need && drop.p == 0.0);
-        a.set_dropout(std::move(drop), q.device());
-        // a mask geometry that the forward kernel would draw score by score is drawn ahead of it,
-        // which takes the buffer also where no backward will read it
-        const slapo_dropout_plan& plan = a.drop.plan;
-        const bool per_score = a.drop.p > 0.0 &&
-                               (plan.vec < 4 || a.sk() % 4 != 0 ||
-                                (plan.total_threads & (plan.total_threads - 1)) != 0);
-        r = launch_attn_fwd(a, oq.t, ok.t, ov.t,
-                            save_mask && a.drop.p < 1.0 && (need || per_score), save_mask_max);
+        a.describe(q.scalar_type(), q.size(0), q.size(1), k.size(1), q.size(2), q.size(3), causal,
+                   window, scale);
+        x.take(a, q, k, v);
+        r = run_attention(a, x, {a.b(), a.sq(), a.h(), a.d()}, mask, std::move(drop), need,
+                          save_mask, save_mask_max);
+    }
+    if (node) node->save(x, a, r);
+    return r.out;
+}
+
+// Self-attention on the output of a fused projection: qkv is [B, S, heads * 3 * head_dim] with q, k, v
+// of one head side by side, the result [B, S, heads * head_dim].
+Tensor attention_packed(const Tensor& qkv, int64_t head_dim, const Tensor& mask, bool causal,
+                        int64_t window, std::optional<double> scale, Dropout&& drop, bool save_mask,
+                        int64_t save_mask_max) {
+    require_device({&qkv, &mask});
+    refuse_tangents({&qkv});
+    TORCH_CHECK_VALUE(qkv.dim() == 3 && head_dim > 0 && qkv.size(2) % (3 * head_dim) == 0,
+                      "qkv must be [batch, seqlen, heads * 3 * head_dim]");
+    const bool need = torch::autograd::compute_requires_grad(qkv);
+    auto node = make_node<AttnBackward>(need, qkv);
+    AttnProblem a;
+    AttnResult r;
+    Operands x;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(qkv.device());
+        a.describe(qkv.scalar_type(), qkv.size(0), qkv.size(1), qkv.size(1),
+                   qkv.size(2) / (3 * head_dim), head_dim, causal, window, scale);
+        x.take_packed(a, qkv);
+        r = run_attention(a, x, {a.b(), a.sq(), a.h() * a.d()}, mask, std::move(drop), need,
+                          save_mask, save_mask_max);
+    }
+    if (node) node->save(x, a, r);
+    return r.out;
+}
+
+// ---- FusedQKV -----------------------------------------------------------------------------------
+
+struct QkvSplitBackward : Node {
+    std::vector<int64_t> sizes;  // of the packed tensor
+    at::ScalarType dtype = at::kFloat;
+    c10::Device device = at::kCPU;
+
+    std::string name() const override { return "HipQKVSplitBackward"; }
+    variable_list apply(variable_list&& grads) override {
+        variable_list res(1);
+        if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return res;
+        const c10::OptionalDeviceGuard guard(device);
+        Tensor g[3];
+        const Tensor packed = fresh(sizes, dtype);
+        for (int i = 0; i < 3; ++i) {
+            if (grads[i].defined())
+                g[i] = dense(grads[i], dtype);
+            else
+                g[i] = fresh({packed.numel() / 3}, dtype).zero_();
+        }
+        if (packed.numel() > 0)
+            check(slapo_amd_qkv_join(cptr(g[0]), cptr(g[1]), cptr(g[2]), mptr(packed),
+                                     packed.numel() / 3, dtype_code(dtype), stream_of(packed)),
+                  "slapo_amd_qkv_join");
+        res[0] = packed;
+        return res;
+    }
+};
+
+// [.., heads * head_size * 3] -> three [.., heads, head_size]
+std::array<Tensor, 3> qkv_split(const Tensor& packed_in, int64_t heads, int64_t head_size) {
+    require_device({&packed_in});
+    refuse_tangents({&packed_in});
+    TORCH_CHECK(packed_in.dim() > 0 && packed_in.size(-1) == heads * head_size * 3,
+                "expected ", heads * head_size * 3, " columns, got ", packed_in.sizes());
+    auto node = make_node<QkvSplitBackward>(torch::autograd::compute_requires_grad(packed_in),
+                                            packed_in);
+    std::array<Tensor, 3> out;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(packed_in.device());
+        const Tensor packed = packed_in.contiguous();
+        const int code = dtype_code(packed.scalar_type());
+        std::vector<int64_t> sizes(packed.sizes().begin(), packed.sizes().end() - 1);
+        sizes.push_back(heads), sizes.push_back(head_size);
+        for (Tensor& t : out) t = fresh(sizes, packed.scalar_type());
+        if (packed.numel() > 0)
+            check(slapo_amd_qkv_split(cptr(packed), mptr(out[0]), mptr(out[1]), mptr(out[2]),
+                                      packed.numel() / 3, code, stream_of(packed)),
+                  "slapo_amd_qkv_split");
     }
     if (node) {
-        torch::autograd::set_history(r.out, node);
-        node->q = keep(oq.t), node->k = keep(ok.t), node->v = keep(ov.t);
-        node->bias = keep(a.bias), node->lse = keep(r.lse), node->keep_mask = keep(r.keep_mask);
-        node->state = keep(a.drop.state);
-        node->out = keep(r.out, true);
-        a.bias = Tensor(), a.drop.state = Tensor();
-        node->a = a;
+        node->sizes.assign(packed_in.sizes().begin(), packed_in.sizes().end());
+        node->dtype = packed_in.scalar_type();
+        node->device = packed_in.device();
+        for (const Tensor& t : out) torch::autograd::set_history(t, node);
     }
-    return r.out;
+    return out;
+}
+
+// ---- cross entropy ------------------------------------------------------------------------------
+
+struct CrossEntropyBackward : Node {
+    SavedVariable logits, target, stats;  // stats: row maximum and 1 / sum, [2, rows]
+    double smoothing = 0.0;
+
+    std::string name() const override { return "HipCrossEntropyBackward"; }
+    void release_variables() override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        for (SavedVariable* s : {&logits, &target, &stats}) s->reset_data();
+    }
+    variable_list apply(variable_list&& grads) override {
+        std::lock_guard<std::mutex> lock(mutex_);
+        variable_list res(1);
+        if (!grads[0].defined()) return res;
+        const Tensor x = logits.unpack(), t = target.unpack(), st = stats.unpack();
+        const c10::OptionalDeviceGuard guard(x.device());
+        const Tensor g = dense(grads[0], at::kFloat);
+        res[0] = fresh_like(x);
+        const int64_t rows = t.numel();
+        if (x.numel() == 0) return res;
+        const float* m = static_cast<const float*>(cptr(st));
+        check(slapo_amd_vocab_ce_bwd(cptr(x), static_cast<const int64_t*>(cptr(t)), m, m + rows,
+                                     static_cast<const float*>(cptr(g)), mptr(res[0]), rows,
+                                     x.size(-1), 0, smoothing, dtype_code(x.scalar_type()),
+                                     stream_of(x)),
+              "slapo_amd_vocab_ce_bwd");
+        return res;
+    }
+};
+
+Tensor cross_entropy(const Tensor& logits_in, const Tensor& target_in, double smoothing) {
+    require_device({&logits_in, &target_in});
+    refuse_tangents({&logits_in});
+    TORCH_CHECK_VALUE(logits_in.dim() > 0, "logits need a vocabulary dimension");
+    const int64_t vocab = logits_in.size(-1), rows = vocab > 0 ? logits_in.numel() / vocab : 0;
+    TORCH_CHECK_VALUE(target_in.numel() == rows,
+                      "target must have the shape of the logits without the vocabulary dim");
+    TORCH_CHECK_VALUE(smoothing == 0.0 || vocab >= 2, "label smoothing needs at least two classes");
+    auto node = make_node<CrossEntropyBackward>(torch::autograd::compute_requires_grad(logits_in),
+                                                logits_in);
+    Tensor logits, target, loss, stats;
+    {
+        at::AutoDispatchBelowADInplaceOrView below;
+        const c10::OptionalDeviceGuard guard(logits_in.device());
+        logits = logits_in.contiguous();
+        target = dense(target_in, at::kLong);
+        const int code = dtype_code(logits.scalar_type());
+        loss = fresh(target_in.sizes(), at::kFloat);
+        stats = floats(2 * rows);
+        float* m = static_cast<float*>(mptr(stats));
+        if (rows > 0)
+            check(slapo_amd_vocab_ce_loss(cptr(logits), static_cast<const int64_t*>(cptr(target)),
+                                          static_cast<float*>(mptr(loss)), m, m + rows, rows, vocab,
+                                          smoothing, code, stream_of(logits)),
+                  "slapo_amd_vocab_ce_loss");
+    }
+    if (node) {
+        torch::autograd::set_history(loss, node);
+        node->logits = keep(logits), node->target = keep(target), node->stats = keep(stats);
+        node->smoothing = smoothing;
+    }
+    return loss;
 }
 
 // ---- bias + GeLU --------------------------------------------------------------------------------
@@ -756,6 +959,63 @@ PyObject* py_attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// attention_packed(qkv, head_dim, mask, causal, window, scale, p, seed, offset, state, save_mask,
+// save_max)
+PyObject* py_attention_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 12, "attention_packed");
+    const Tensor& qkv = tensor_arg(a[0], "qkv");
+    const int64_t head_dim = int_arg(a[1]);
+    const Tensor& mask = optional_tensor_arg(a[2], "attention_mask");
+    const bool causal = bool_arg(a[3]), save_mask = bool_arg(a[10]);
+    const int64_t window = int_arg(a[4]), save_max = int_arg(a[11]);
+    std::optional<double> scale;
+    if (a[5] != Py_None) scale = double_arg(a[5]);
+    Dropout drop = dropout_args(a + 6);
+    Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = attention_packed(qkv, head_dim, mask, causal, window, scale, std::move(drop),
+                               save_mask, save_max);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// qkv_split(packed, heads, head_size): [q, k, v]
+PyObject* py_qkv_split(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 3, "qkv_split");
+    const Tensor& packed = tensor_arg(a[0], "packed");
+    const int64_t heads = int_arg(a[1]), head_size = int_arg(a[2]);
+    std::array<Tensor, 3> out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = qkv_split(packed, heads, head_size);
+    }
+    THPObjectPtr list(PyList_New(3));
+    if (!list) throw python_error();
+    for (int i = 0; i < 3; ++i)
+        PyList_SET_ITEM(list.get(), i, THPVariable_Wrap(std::move(out[i])));
+    return list.release();
+    END_HANDLE_TH_ERRORS
+}
+
+// cross_entropy(logits, target, smoothing)
+PyObject* py_cross_entropy(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 3, "cross_entropy");
+    const Tensor &logits = tensor_arg(a[0], "logits"), &target = tensor_arg(a[1], "target");
+    const double smoothing = double_arg(a[2]);
+    Tensor out;
+    {
+        pybind11::gil_scoped_release no_gil;
+        out = cross_entropy(logits, target, smoothing);
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
 // attention_scores(q, k, v): checks the operands, returns the number of scores B * H * Sq * Sk
 PyObject* py_attention_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -842,7 +1102,10 @@ PyObject* py_draw(PyObject*, PyObject* const* a, Py_ssize_t n) {
     { name, (PyCFunction)(void (*)(void))fn, METH_FASTCALL, nullptr }
 PyMethodDef methods[] = {
     SLAPO_METHOD("attention", py_attention),
+    SLAPO_METHOD("attention_packed", py_attention_packed),
     SLAPO_METHOD("attention_scores", py_attention_scores),
+    SLAPO_METHOD("qkv_split", py_qkv_split),
+    SLAPO_METHOD("cross_entropy", py_cross_entropy),
     SLAPO_METHOD("bias_gelu", py_bias_gelu),
     SLAPO_METHOD("bias_dropout_residual", py_bias_dropout_residual),
     SLAPO_METHOD("bias_dropout_residual_layer_norm", py_layer_norm),

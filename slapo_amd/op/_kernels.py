@@ -1,5 +1,5 @@
 """Launch-level wrappers over the C ABI for direct use of single kernels, with an explicit (seed,
-offset) pair and explicit intermediate results (tests, benchmarks, the cross entropy): argument
+offset) pair and explicit intermediate results (tests, benchmarks, vocabulary shards): argument
 checking, output / workspace allocation with torch's caching allocator, stream selection.  No
 arithmetic happens here.  The ops go through csrc/host_ops.cpp instead."""
 from __future__ import annotations

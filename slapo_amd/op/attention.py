@@ -57,24 +57,46 @@ SAVE_DROPOUT_MASK = True
 SAVE_DROPOUT_MASK_MAX_BYTES = 512 << 20
 
 
+def _draw(p, scores, device):
+    """(seed, offset, state) for the mask F.dropout would draw for `scores` fp32 probabilities.
+    Nothing is drawn for p of 0 or 1, nor for an empty tensor (F.dropout leaves the generator
+    alone)."""
+    if not 0.0 <= p <= 1.0:
+        raise ValueError(f"dropout probability has to be between 0 and 1, but got {p}")
+    if not 0.0 < p < 1.0 or not scores:
+        return 0, 0, None
+    return draw_philox_state(host().philox_increment(scores, 4, device.index), device)
+
+
+def _note_bias_gradient(attention_mask):
+    if attention_mask is not None and attention_mask.requires_grad:
+        warning_once("WARNING: bias gradient is not supported yet. "
+                     "The mask is applied but receives no gradient")
+
+
 def hip_attention(q, k, v, attention_mask=None, causal=False, p=0.0, scale=None, window=0):
     """q, k, v: [B, S, H, D] (head_dim contiguous; outer dims may be strided views).
     attention_mask: additive, 4-D, broadcastable to [B, H, Sq, Sk].  Returns [B, Sq, H, D]."""
     native = host()
-    seed, offset, rng_state = 0, 0, None
+    seed, offset, state = 0, 0, None
     if p != 0.0:
-        if not 0.0 <= p <= 1.0:
-            raise ValueError(f"dropout probability has to be between 0 and 1, but got {p}")
-        scores = native.attention_scores(q, k, v)
-        # nothing is drawn for p = 1, nor for an empty tensor (F.dropout leaves the generator alone)
-        if p < 1.0 and scores:
-            seed, offset, rng_state = draw_philox_state(
-                native.philox_increment(scores, 4, q.device.index), q.device)
-    if attention_mask is not None and attention_mask.requires_grad:
-        warning_once("WARNING: bias gradient is not supported yet. "
-                     "The mask is applied but receives no gradient")
+        seed, offset, state = _draw(p, native.attention_scores(q, k, v), q.device)
+    _note_bias_gradient(attention_mask)
     return native.attention(q, k, v, attention_mask, causal, window or 0, scale, p, seed, offset,
-                            rng_state, SAVE_DROPOUT_MASK, SAVE_DROPOUT_MASK_MAX_BYTES)
+                            state, SAVE_DROPOUT_MASK, SAVE_DROPOUT_MASK_MAX_BYTES)
+
+
+def _packed_attention(qkv, head_dim, attention_mask, causal, p, scale, window):
+    """`hip_attention` on the output [B, S, heads * 3 * head_dim] of a fused projection; returns
+    [B, S, heads * head_dim].  The backward writes the gradient of `qkv` as one tensor."""
+    seed, offset, state = 0, 0, None
+    if p != 0.0:
+        b, s, width = qkv.shape
+        seed, offset, state = _draw(p, b * (width // (3 * head_dim)) * s * s, qkv.device)
+    _note_bias_gradient(attention_mask)
+    return host().attention_packed(qkv, head_dim, attention_mask, causal, window or 0, scale, p,
+                                   seed, offset, state, SAVE_DROPOUT_MASK,
+                                   SAVE_DROPOUT_MASK_MAX_BYTES)
 
 
 class FlashAttentionOp(nn.Module):
@@ -183,16 +205,26 @@ class FlashAttention(nn.Module):
         """[B, S, heads*head_size] -> [B, S, heads, head_size]; -1 covers sharded head counts."""
         return x.view(x.size()[:-1] + (-1, self.attention_head_size))
 
+    def _split_packed(self, packed):
+        # Head-interleaved packing [.., heads, 3*head_size]: q, k, v of one head are adjacent,
+        # which keeps a tensor-parallel shard of the weight a set of whole heads.  The three
+        # results are strided views; the kernel reads them in place.
+        packed = packed.view(packed.size()[:-1] + (-1, 3 * self.attention_head_size))
+        return packed.split(self.attention_head_size, dim=-1)
+
     def _project_qkv(self, hidden_states):
-        if self.fused_qkv:
-            # Head-interleaved packing [.., heads, 3*head_size]: q, k, v of one head are adjacent,
-            # which keeps a tensor-parallel shard of the weight a set of whole heads.  The three
-            # results are strided views; the kernel reads them in place.
-            packed = self.qkv(hidden_states)
-            packed = packed.view(packed.size()[:-1] + (-1, 3 * self.attention_head_size))
-            return packed.split(self.attention_head_size, dim=-1)
         return tuple(self.reshape_for_scores(proj(hidden_states))
                      for proj in (self.query, self.key, self.value))
+
+    def _core_takes_packed(self, packed):
+        """The packed form stands in for splitting the projection and calling `attn_op` only when
+        nothing could tell the difference: the child is the plain op (a schedule's `.fork_rng`
+        wraps its `forward`, primitives/tensor_parallel.py:185-191; `.replace` swaps it) without
+        hooks, and the input a real device tensor."""
+        core = self.attn_op
+        return (type(packed) is torch.Tensor and packed.is_cuda and packed.ndim == 3
+                and type(core) is FlashAttentionOp and core.attn_fn is hip_attention
+                and "forward" not in core.__dict__ and not _has_hooks(core))
 
     def _tail_can_fuse(self, x):
         """The fused out_proj-bias + resid_dropout pass stands in for the two child calls only when
@@ -224,7 +256,17 @@ class FlashAttention(nn.Module):
         if head_mask is not None:
             raise NotImplementedError("FlashAttention does not support head mask yet.")
 
-        query_layer, key_layer, value_layer = self._project_qkv(hidden_states)
+        if self.fused_qkv:
+            packed = self.qkv(hidden_states)
+            if layer_past is None and not use_cache and self._core_takes_packed(packed):
+                core = self.attn_op
+                context_layer = _packed_attention(
+                    packed, self.attention_head_size, attention_mask, core.apply_causal_mask,
+                    self.attn_pdrop, core.scale, core.window)
+                return (self._project_context(context_layer), None)
+            query_layer, key_layer, value_layer = self._split_packed(packed)
+        else:
+            query_layer, key_layer, value_layer = self._project_qkv(hidden_states)
 
         if layer_past is not None:
             past_key, past_value = layer_past
@@ -239,15 +281,17 @@ class FlashAttention(nn.Module):
         context_layer = context_layer.contiguous()
         context_layer = context_layer.view(context_layer.size()[:-2] + (-1,))
 
-        if self.output_proj:
-            if self._tail_can_fuse(context_layer):
-                # out_proj's bias and resid_dropout ride on one pass over [B, S, hidden] (the
-                # reference runs the GEMM with bias, then nn.Dropout: slapo/op/attention.py:514-516).
-                # The mask is the one nn.Dropout would draw; p and training are read from the child.
-                context_layer = bias_dropout(
-                    F.linear(context_layer, self.out_proj.weight, None), self.out_proj.bias,
-                    self.resid_dropout.p, self.resid_dropout.training)
-            else:
-                context_layer = self.resid_dropout(self.out_proj(context_layer))
+        return (self._project_context(context_layer),
+                (key_layer, value_layer) if use_cache else None)
 
-        return (context_layer, (key_layer, value_layer) if use_cache else None)
+    def _project_context(self, context_layer):
+        if not self.output_proj:
+            return context_layer
+        if self._tail_can_fuse(context_layer):
+            # out_proj's bias and resid_dropout ride on one pass over [B, S, hidden] (the
+            # reference runs the GEMM with bias, then nn.Dropout: slapo/op/attention.py:514-516).
+            # The mask is the one nn.Dropout would draw; p and training are read from the child.
+            return bias_dropout(
+                F.linear(context_layer, self.out_proj.weight, None), self.out_proj.bias,
+                self.resid_dropout.p, self.resid_dropout.training)
+        return self.resid_dropout(self.out_proj(context_layer))

@@ -13,6 +13,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor, nn
 
+from .._lib import host
 from .fused_bias import BiasGeLUFunction, bias_dropout, bias_new_gelu
 
 
@@ -33,7 +34,10 @@ class FusedQKV(nn.Module):
         return x.view(shape).contiguous()
 
     def forward(self, hidden_states):
-        packed = self.reshape_for_scores(self.fused_linear(hidden_states))
+        packed = self.fused_linear(hidden_states)
+        if type(packed) is Tensor and packed.is_cuda:  # one pass instead of three strided copies
+            return host().qkv_split(packed, self.num_heads // self.world_size, self.head_size)
+        packed = self.reshape_for_scores(packed)
         return [t.squeeze(-1).contiguous() for t in torch.split(packed, 1, dim=-1)]
 
 

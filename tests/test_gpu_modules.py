@@ -202,3 +202,44 @@ def test_ops_on_side_streams_from_two_threads():
     for i in range(2):
         for a, b_ in zip(got[i], want[i]):
             assert torch.equal(a, b_)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("tokens,heads,head_size", [(5, 3, 8), (33, 2, 20), (7, 1, 3)])
+def test_fused_qkv_layout_and_gradient(dtype, tokens, heads, head_size):
+    """One pass in each direction, 16-byte runs and element by element, against torch's own
+    splitting of the same projection output; a result that is not used gives no gradient."""
+    m = op.FusedQKV(heads * head_size, heads, 1).to(device="cuda", dtype=dtype)
+    x = torch.randn(2, tokens, heads * head_size, device="cuda", dtype=dtype, requires_grad=True)
+    go = [torch.randn(2, tokens, heads, head_size, device="cuda", dtype=dtype) for _ in range(3)]
+    packed = m.fused_linear(x)
+    ref = [t.squeeze(-1) for t in m.reshape_for_scores(packed).split(1, dim=-1)]
+    out = m(x)
+    for used in (3, 2):
+        for a, r in zip(out, ref):
+            assert a.shape == r.shape and a.is_contiguous() and torch.equal(a, r)
+        ga, = torch.autograd.grad(out[:used], x, go[:used], retain_graph=True)
+        gr, = torch.autograd.grad(ref[:used], x, go[:used], retain_graph=True)
+        assert torch.equal(ga, gr)
+
+
+@pytest.mark.parametrize("dtype,head_dim,p", [(torch.float16, 64, 0.0), (torch.bfloat16, 80, 0.1),
+                                              (torch.float32, 12, 0.1)])
+def test_packed_attention_equals_the_split_call(dtype, head_dim, p):
+    """FlashAttention hands the fused projection to the kernel in one piece: same output and the
+    same gradient, bit for bit, as splitting it and calling the op."""
+    torch.manual_seed(4)
+    heads, b, s = 3, 2, 75
+    m = op.FlashAttention(heads * head_dim, heads, attn_pdrop=p, output_proj=True, fused_qkv=True,
+                          attn_op_name="hip_cdna4").to(device="cuda", dtype=dtype)
+    x = torch.randn(b, s, heads * head_dim, device="cuda", dtype=dtype, requires_grad=True)
+    mask = torch.zeros(b, 1, 1, s, device="cuda", dtype=dtype)
+    mask[1, ..., 50:] = torch.finfo(dtype).min
+    results = []
+    for use_cache in (False, True):  # the cache asks for k and v: the split form
+        torch.cuda.manual_seed(9)
+        out, _ = m(x, mask, use_cache=use_cache)
+        results.append([out, *torch.autograd.grad(out, [x, *m.qkv.parameters()],
+                                                  torch.ones_like(out))])
+    for a, r in zip(*results):
+        assert torch.equal(a, r)
