@@ -277,9 +277,9 @@ int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* 
  * SLAPO_BIAS_PREPARED says that it is the output of slapo_amd_attn_prepare_bias, with strides
  * {batch, head, rounded seqlen_k, 1}.
  * Workspace: 16-byte aligned, slapo_amd_attn_fwd_workspace_bytes of it (may be NULL where that is
- * 0).  With one query per sequence and no dropout the keys of a (batch, head) are shared by several
- * workgroups, whose partial results meet there; without it such a call runs with one workgroup
- * per (batch, head). */
+ * 0).  Where a call has too few rows to fill the device, the keys of a block of rows are dealt to
+ * several workgroups, whose partial results meet there; with a smaller one or none every block of
+ * rows keeps to one workgroup. */
 #define SLAPO_BIAS_PREPARED 3
 size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm);
 int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
@@ -308,7 +308,10 @@ int slapo_amd_attn_bwd(const slapo_attn_params* prm, const void* q, const void* 
                        const int64_t dk_strides[3], const int64_t dv_strides[3], void* workspace,
                        size_t workspace_bytes, void* stream);
 
-/* The same call with the bias type of slapo_amd_attn_fwd_ex. */
+/* The same call with the bias type of slapo_amd_attn_fwd_ex.  A workspace of
+ * slapo_amd_attn_bwd_ex_workspace_bytes (at least slapo_amd_attn_bwd_workspace_bytes is needed)
+ * also holds the partial results of a call that is dealt to more workgroups as described there. */
+size_t slapo_amd_attn_bwd_ex_workspace_bytes(const slapo_attn_params* prm);
 int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
                           const void* v, const void* bias, int bias_type, const void* o,
                           const void* dout, const float* lse, void* dq, void* dk, void* dv,

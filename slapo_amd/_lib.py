@@ -143,6 +143,7 @@ PROTOTYPES = {
         ctypes.c_int, [c_vp, ctypes.c_int, ctypes.POINTER(c_i64), c_i64, c_i64, c_i64, c_i64,
                        c_vp, c_vp]
     ),
+    "slapo_amd_attn_bwd_ex_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
     "slapo_amd_attn_bwd_ex": (
         ctypes.c_int,
         [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, ctypes.c_int, c_vp, c_vp, c_vp, c_vp,

@@ -62,7 +62,11 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
 
     const int n_bh = a.batch * a.heads;
     const int n_qt = (a.sq + kBM - 1) / kBM;
-    const int work = work_index(a);
+    int work = work_index(a), split = 0;
+    if (a.n_split > 1) {
+        split = work / (n_bh * n_qt);
+        work -= split * n_bh * n_qt;
+    }
     const int bh = work % n_bh;
     const int qt = n_qt - 1 - work / n_bh;  // heaviest (latest) query tiles first
     const int b = bh / a.heads;
@@ -119,8 +123,9 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     if constexpr (kBias)  // skip the tiles that hold nothing but padded keys
         j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads, false>(
                                            a, b, h, reinterpret_cast<float*>(smem_raw))));
-    const int t_lo = j_lo / kBN;
-    const int t_hi = (j_hi + kBN - 1) / kBN;
+    int t_lo = j_lo / kBN;
+    int t_hi = (j_hi + kBN - 1) / kBN;
+    if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
     const int n_tiles = t_hi - t_lo;
 
     frag_t qf[DK], gf[DK];
@@ -525,7 +530,7 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     if (a.window <= 0 && q0 + kBM <= a.sq) {
         n_fast = a.sk / kBN;
         if (a.causal) n_fast = min(n_fast, (q0 + 1) / kBN);
-        n_fast = min(n_fast, n_tiles);
+        n_fast = min(n_fast - t_lo, n_tiles);
     }
     int r = 0;
     for (; r < n_fast; ++r) iteration(r, std::true_type{});
@@ -537,6 +542,11 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
         T* dq_row0 =
             reinterpret_cast<T*>(a.dq) + b * a.dqs[0] + (int64_t)wq0 * a.dqs[1] + h * a.dqs[2];
         const float out_scale = (kDrop != 0 ? a.scale * a.rng.inv_keep : a.scale) * inv_n;
+        if (a.n_split > 1) {
+            const int64_t row0 = ((int64_t)split * n_bh + bh) * a.sq + wq0;
+            store_partial<DPAD>(dq_acc, out_scale, a.part + row0 * a.d, a.sq - wq0, a.d);
+            return;
+        }
         store_block_via_lds<T, DPAD, kPitch>(dq_acc, out_scale, k_lds + wave * 32 * kPitch,
                                              dq_row0, a.dqs[1], a.sq - wq0, a.d);
     }
@@ -548,14 +558,14 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const size_t smem = (size_t)(kKRing + kVRing) * kBN * Stage::kPitch * sizeof(T) +
                         (kBias == 2 ? 2 * kBN * sizeof(float) : 0);
     const int n_qt = (a.sq + kBM - 1) / kBM;
-    const int64_t blocks = (int64_t)n_qt * a.batch * a.heads;
+    const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
     auto kern = attn_bwd_dq_kernel<T, DPAD, kBias, kDrop, kStagger, kSteps>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
-    set_dispatch_order(&ordered, blocks, (kStagger && DPAD > 64) ? 1 : 2);
+    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, (kStagger && DPAD > 64) ? 1 : 2);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, ordered);
     return check_launch();
 }

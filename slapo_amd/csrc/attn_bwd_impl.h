@@ -80,7 +80,12 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     uint32_t* mask_lds = reinterpret_cast<uint32_t*>(smem_raw + 2 * SM::kQBytes + SM::kStatBytes);
 
     const int n_bh = a.batch * a.heads;
-    const int work = work_index(a);
+    int work = work_index(a), split = 0;
+    if (a.n_split > 1) {
+        const int base = (int)gridDim.x / a.n_split;
+        split = work / base;
+        work -= split * base;
+    }
     const int bh = work % n_bh;
     const int kt = work / n_bh;  // low key tiles see the most queries under a causal mask
     const int b = bh / a.heads;
@@ -136,8 +141,9 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
         if (k0 >= padded_key_limit<kBwdThreads, false>(a, b, h, reinterpret_cast<float*>(smem_raw)))
             i_hi = i_lo;
     }
-    const int t_lo = i_lo / kBwdBM;
-    const int t_hi = (i_hi + kBwdBM - 1) / kBwdBM;
+    int t_lo = i_lo / kBwdBM;
+    int t_hi = (i_hi + kBwdBM - 1) / kBwdBM;
+    if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
 
     // kBias: 0 = none, 1 = any layout (read from memory per score), 2 = the launcher guarantees a
     // bias that does not depend on the query (stride 0 over the queries, the compact [B,1,1,Sk]
@@ -636,6 +642,15 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     // through the dO buffers)
     static_assert(KB == 1, "the output staging assumes 32 keys per wavefront");
     if (kw0 < a.sk) {
+        if (a.n_split > 1) {
+            const int64_t rows = (int64_t)n_bh * a.sk;
+            float* part = a.part + (split * rows + (int64_t)bh * a.sk + kw0) * a.d;
+            store_partial<DPAD>(dk_acc[0], kDrop != 0 ? a.scale * a.rng.inv_keep : a.scale, part,
+                                a.sk - kw0, a.d);
+            store_partial<DPAD>(dv_acc[0], kDrop != 0 ? a.rng.inv_keep : 1.0f,
+                                part + a.n_split * rows * a.d, a.sk - kw0, a.d);
+            return;
+        }
         T* dk_row0 =
             reinterpret_cast<T*>(a.dk) + b * a.dks[0] + (int64_t)kw0 * a.dks[1] + h * a.dks[2];
         T* dv_row0 =
@@ -657,14 +672,14 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const size_t smem = SM::kBytes;
     constexpr int kBN = kBwdWaves * 32 * KB;
     const int n_kt = (a.sk + kBN - 1) / kBN;
-    const int64_t blocks = (int64_t)n_kt * a.batch * a.heads;
+    const int64_t blocks = (int64_t)n_kt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
     auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
-    set_dispatch_order(&ordered, blocks, bwd_two_per_cu(DPAD, kDrop, KB) ? 2 : 1);
+    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, bwd_two_per_cu(DPAD, kDrop, KB) ? 2 : 1);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBwdThreads), smem, st, ordered);
     return check_launch();
 }

@@ -14,6 +14,10 @@ int attn_bwd_dq_mfma_bf16(const AttnArgs& a, hipStream_t st);
 int attn_fwd_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_f32(const AttnArgs& a, hipStream_t st);
+int attn_splits(int64_t blocks, int64_t cus, int64_t tiles, bool f32, bool causal);
+int attn_merge_fwd(const AttnArgs& a, int dtype, hipStream_t st);
+int attn_merge_bwd(const AttnArgs& a, int dtype, const float* dq_part, int n_dq,
+                   const float* dkv_part, int n_dkv, hipStream_t st);
 int attn_decode_shares(int64_t n_bh, int n_keys);
 int attn_decode(const AttnArgs& a, int dtype, int n_shares, float* part, hipStream_t st);
 }  // namespace slapo
@@ -152,6 +156,8 @@ int fill_args(const slapo_attn_params* p, AttnArgs* a, bool backward) {
     }
     a->snake_len = 0, a->snake_rows = 0;
     a->n_cus = half ? cus_of_current_device() : 0;
+    a->n_split = 1;
+    a->part = nullptr;
     a->keep_mask = nullptr;
     a->mask_words = (p->seqlen_k + 31) / 32;
     a->mask_pitch = (p->seqlen_q + 3) & ~3;
@@ -249,10 +255,52 @@ int decode_shares(const slapo_attn_params* p) {
 
 }  // namespace
 
+namespace {
+
+// Splits of the three kernels of a call (attn_splits), for the current device.
+struct Splits {
+    int fwd = 1, dq = 1, dkv = 1;
+};
+Splits plan_splits(const slapo_attn_params* p) {
+    Splits s;
+    if (!p || p->batch <= 0 || p->heads <= 0 || p->seqlen_q <= 0 || p->seqlen_k <= 0 ||
+        p->head_dim <= 0)
+        return s;
+    const int64_t cus = cus_of_current_device();
+    const bool f32 = p->dtype == SLAPO_F32;
+    const int64_t n_bh = (int64_t)p->batch * p->heads, rows = f32 ? 64 : 128, tile = f32 ? 32 : 64;
+    auto blocks = [&](int64_t n) { return n_bh * ((n + rows - 1) / rows); };
+    auto tiles = [&](int64_t n) {
+        return ((p->window > 0 && p->window + rows < n ? p->window + rows : n) + tile - 1) / tile;
+    };
+    const bool causal = p->causal && p->window <= 0;
+    s.fwd = s.dq = attn_splits(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), f32, causal);
+    s.dkv = attn_splits(blocks(p->seqlen_k), cus, tiles(p->seqlen_q), f32, causal);
+    return s;
+}
+size_t delta_bytes(const slapo_attn_params* p) {  // rounded: the partial results follow
+    return (slapo_amd_attn_bwd_workspace_bytes(p) + 255) & ~size_t(255);
+}
+
+}  // namespace
+
 extern "C" size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm) {
-    const int shares = decode_shares(prm);
-    if (shares <= 1) return 0;
-    return (size_t)shares * prm->batch * prm->heads * (2 + prm->head_dim) * sizeof(float);
+    if (const int shares = decode_shares(prm))
+        return shares == 1 ? 0
+                           : (size_t)shares * prm->batch * prm->heads * (2 + prm->head_dim) *
+                                 sizeof(float);
+    const Splits s = plan_splits(prm);
+    if (s.fwd == 1) return 0;
+    return (size_t)s.fwd * prm->batch * prm->heads * prm->seqlen_q * (2 + prm->head_dim) *
+           sizeof(float);
+}
+
+extern "C" size_t slapo_amd_attn_bwd_ex_workspace_bytes(const slapo_attn_params* prm) {
+    const Splits s = plan_splits(prm);
+    if (s.dq == 1 && s.dkv == 1) return slapo_amd_attn_bwd_workspace_bytes(prm);
+    const size_t row = (size_t)prm->batch * prm->heads * prm->head_dim * sizeof(float);
+    return delta_bytes(prm) + (s.dq > 1 ? row * prm->seqlen_q * s.dq : 0) +
+           (s.dkv > 1 ? 2 * row * prm->seqlen_k * s.dkv : 0);
 }
 
 extern "C" size_t slapo_amd_attn_prepared_bias_bytes(int64_t batch, int64_t heads,
@@ -311,7 +359,16 @@ extern "C" int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q
         if (rows_ok && bias_type != SLAPO_BIAS_PREPARED)
             return attn_decode(a, prm->dtype, shares, static_cast<float*>(workspace), st);
     }
-    if (f32) return attn_fwd_f32(a, st);
+    const size_t split_bytes = slapo_amd_attn_fwd_workspace_bytes(prm);
+    if (workspace && split_bytes > 0 && workspace_bytes >= split_bytes &&
+        decode_shares(prm) == 0) {
+        a.n_split = plan_splits(prm).fwd;
+        a.part = static_cast<float*>(workspace);
+    }
+    auto merged = [&](int status) {
+        return status == SLAPO_OK && a.n_split > 1 ? attn_merge_fwd(a, prm->dtype, st) : status;
+    };
+    if (f32) return merged(attn_fwd_f32(a, st));
     if (a.dropout && a.keep_mask && (a.window > 0 || a.dropout == 2) && keep_mask_kernel_fits(a)) {
         // Local window, or a mask geometry without whole Philox blocks per aligned group of keys,
         // with a buffer for the keep bits: draw them first, the forward kernel then reads them
@@ -324,7 +381,7 @@ extern "C" int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q
         if (rc != SLAPO_OK) return rc;
         a.dropout = 3;
     }
-    return prm->dtype == SLAPO_F16 ? attn_fwd_mfma_f16(a, st) : attn_fwd_mfma_bf16(a, st);
+    return merged(prm->dtype == SLAPO_F16 ? attn_fwd_mfma_f16(a, st) : attn_fwd_mfma_bf16(a, st));
 }
 
 extern "C" int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* k,
@@ -371,29 +428,46 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
     a.delta = reinterpret_cast<float*>(workspace);
     a.dq = dq;
 
-    // PREPARE has nothing to do (the dQ kernel computes delta for its own rows and stores it for
-    // the dK / dV kernel), so DQ runs before DKDV.
-    if (prm->dtype == SLAPO_F32) {
-        if (stages & SLAPO_BWD_DQ) {
-            rc = attn_bwd_dq_f32(a, st);
-            if (rc != SLAPO_OK) return rc;
+    const bool f32 = prm->dtype == SLAPO_F32;
+    if (!f32) {
+        if (!half_ptrs_ok({q, k, v, o, dout, dq, dk, dv})) return SLAPO_ERR_ALIGN;
+        if (!strides_ok(dq_strides, 8) || !strides_ok(dk_strides, 8) || !strides_ok(dv_strides, 8))
+            return SLAPO_ERR_ALIGN;
+    }
+    // Partial results need room, and a caller that runs all stages: both kernels' are merged in one
+    // launch at the end.
+    Splits splits;
+    float *dq_part = nullptr, *dkv_part = nullptr;
+    if (stages == SLAPO_BWD_ALL &&
+        workspace_bytes >= slapo_amd_attn_bwd_ex_workspace_bytes(prm)) {
+        splits = plan_splits(prm);
+        float* next = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(prm));
+        if (splits.dq > 1) {
+            dq_part = next;
+            next += (int64_t)splits.dq * a.batch * a.heads * a.sq * a.d;
         }
-        if (stages & SLAPO_BWD_DKDV) rc = attn_bwd_f32(a, st);
-        return rc;
+        if (splits.dkv > 1) dkv_part = next;
     }
 
-    if (!half_ptrs_ok({q, k, v, o, dout, dq, dk, dv})) return SLAPO_ERR_ALIGN;
-    if (!strides_ok(dq_strides, 8) || !strides_ok(dk_strides, 8) || !strides_ok(dv_strides, 8))
-        return SLAPO_ERR_ALIGN;
-
+    // PREPARE has nothing to do (the dQ kernel computes delta for its own rows and stores it for
+    // the dK / dV kernel), so DQ runs before DKDV.
     if (stages & SLAPO_BWD_DQ) {
-        rc = prm->dtype == SLAPO_F16 ? attn_bwd_dq_mfma_f16(a, st) : attn_bwd_dq_mfma_bf16(a, st);
+        a.n_split = splits.dq, a.part = dq_part;
+        rc = f32                        ? attn_bwd_dq_f32(a, st)
+             : prm->dtype == SLAPO_F16 ? attn_bwd_dq_mfma_f16(a, st)
+                                       : attn_bwd_dq_mfma_bf16(a, st);
         if (rc != SLAPO_OK) return rc;
     }
     if (stages & SLAPO_BWD_DKDV) {
-        rc = prm->dtype == SLAPO_F16 ? attn_bwd_mfma_f16(a, st) : attn_bwd_mfma_bf16(a, st);
+        a.n_split = splits.dkv, a.part = dkv_part;
+        rc = f32                        ? attn_bwd_f32(a, st)
+             : prm->dtype == SLAPO_F16 ? attn_bwd_mfma_f16(a, st)
+                                       : attn_bwd_mfma_bf16(a, st);
+        if (rc != SLAPO_OK) return rc;
     }
-    return rc;
+    return dq_part || dkv_part
+               ? attn_merge_bwd(a, prm->dtype, dq_part, splits.dq, dkv_part, splits.dkv, st)
+               : SLAPO_OK;
 }
 
 }  // namespace

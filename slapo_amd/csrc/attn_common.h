@@ -253,7 +253,18 @@ struct AttnArgs {
     // group before the next group), so that the K / V of the heads in flight fit its L2
     int head_group;
     int n_cus;
+    // The tiles of a workgroup's rows dealt to n_split workgroups (consecutive shares, the split is the
+    // slowest index of the grid), which leave fp32 partial results in `part`; see attn_split.hip.
+    int n_split;
+    float* part;
 };
+
+// The share of tiles [t_lo, t_hi) that workgroup number `split` of its row block takes.
+__device__ __forceinline__ void split_tiles(const AttnArgs& a, int split, int& t_lo, int& t_hi) {
+    const int n = t_hi - t_lo;
+    t_hi = t_lo + n * (split + 1) / a.n_split;
+    t_lo += n * split / a.n_split;
+}
 
 // One value of the additive bias in the type it is stored in.  Split into the read -- one aligned
 // dword whatever the type, so that a request stays straight-line code -- and the conversion, which
@@ -449,6 +460,24 @@ __device__ __forceinline__ void store_block_via_lds(const f32x16_t (&acc)[DPAD /
         if (row < n_rows && 8 * c < d)
             *reinterpret_cast<u32x4_t*>(out_row0 + (int64_t)row * row_stride + 8 * c) = v;
     }
+}
+
+// The same block as fp32 to a dense partial result (rows of d floats).
+template <int DPAD>
+__device__ __forceinline__ void store_partial(const f32x16_t (&acc)[DPAD / 32], float mul,
+                                              float* out_row0, int n_rows, int d) {
+    const int lane = threadIdx.x & 63;
+    const int i = lane & 31, g = lane >> 5;
+    if (i >= n_rows) return;
+#pragma unroll
+    for (int x = 0; x < DPAD / 32; ++x)
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const int col = 32 * x + 8 * r4 + 4 * g;
+            const f32x4_t v = {acc[x][4 * r4] * mul, acc[x][4 * r4 + 1] * mul,
+                               acc[x][4 * r4 + 2] * mul, acc[x][4 * r4 + 3] * mul};
+            if (col < d) *reinterpret_cast<f32x4_t*>(out_row0 + (int64_t)i * d + col) = v;
+        }
 }
 
 // Stage a [ROWS x DPAD] tile of T (rows row0.., zero beyond n_rows / beyond d) through registers.

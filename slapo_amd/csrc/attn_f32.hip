@@ -193,12 +193,16 @@ __device__ __forceinline__ uint32_t keep_queries(const AttnArgs& a, int bh, int 
 // What a workgroup of the query-owning kernels works on: heaviest query tiles first, the heads as
 // the fast index so that the tiles of one head share an XCD's L2.
 struct Place {
-    int b, h, bh, row0;
+    int b, h, bh, row0, split;
+    int64_t part_row0;  // of the split's partial result, rows of all (batch, head) pairs
     __device__ __forceinline__ Place(const AttnArgs& a, int n_rows, bool last_first) {
         const int n_bh = a.batch * a.heads;
         const int n_t = (n_rows + kRows - 1) / kRows;
         bh = (int)(blockIdx.x % (unsigned)n_bh);
-        const int t = (int)(blockIdx.x / (unsigned)n_bh);
+        int t = (int)(blockIdx.x / (unsigned)n_bh);
+        split = t / n_t;
+        t -= split * n_t;
+        part_row0 = ((int64_t)split * n_bh + bh) * n_rows;
         b = bh / a.heads, h = bh % a.heads;
         row0 = (last_first ? n_t - 1 - t : t) * kRows;
     }
@@ -246,7 +250,8 @@ __global__ __launch_bounds__(kThreads, DB <= 4 ? 3 : 2) void attn_f32_fwd_kernel
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
     j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk));
-    const int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
+    int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
+    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
     Tile<DB, kVec> kt, vt;
     f32x4_t qf[DB], o[DB];
@@ -320,6 +325,15 @@ __global__ __launch_bounds__(kThreads, DB <= 4 ? 3 : 2) void attn_f32_fwd_kernel
     }
     const float l_tot = column_sum(l);
     if (i >= a.sq) return;
+    if (a.n_split > 1) {
+        store_row<kVec>(o, 1.0f, a.part + (at.part_row0 + i) * a.d, a.d);
+        if (g == 0) {
+            float* ml = a.part + (int64_t)a.n_split * a.batch * a.heads * a.sq * a.d +
+                        2 * (at.part_row0 + i);
+            ml[0] = m, ml[1] = l_tot;
+        }
+        return;
+    }
     float* op = reinterpret_cast<float*>(a.o) + at.b * a.os[0] + (int64_t)i * a.os[1] +
                 at.h * a.os[2];
     store_row<kVec>(o, 1.0f / l_tot, op, a.d);
@@ -354,7 +368,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
     j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk));
-    const int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
+    int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
+    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
     Tile<DB, kVec> kt, vt;
     f32x4_t qf[DB], gf[DB], dq[DB];
@@ -421,6 +436,10 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
         __syncthreads();
     }
     if (i >= a.sq) return;
+    if (a.n_split > 1) {
+        store_row<kVec>(dq, a.scale, a.part + (at.part_row0 + i) * a.d, a.d);
+        return;
+    }
     float* dqp = reinterpret_cast<float*>(a.dq) + at.b * a.dqs[0] + (int64_t)i * a.dqs[1] +
                  at.h * a.dqs[2];
     store_row<kVec>(dq, a.scale, dqp, a.d);
@@ -453,7 +472,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
     query_range(a, at.row0, min(at.row0 + kRows, a.sk), i_lo, i_hi);
     // keys past the last unpadded one get no probability from any row
     if (at.row0 >= (has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk)) i_hi = i_lo;
-    const int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
+    int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
+    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
     Tile<DB, kVec> qt, gt;
     f32x4_t kf[DB], vf[DB], dk[DB], dv[DB];
@@ -531,6 +551,13 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
         __syncthreads();
     }
     if (j >= a.sk) return;
+    if (a.n_split > 1) {
+        float* part = a.part + (at.part_row0 + j) * a.d;
+        store_row<kVec>(dk, a.scale, part, a.d);
+        store_row<kVec>(dv, 1.0f,
+                        part + (int64_t)a.n_split * a.batch * a.heads * a.sk * a.d, a.d);
+        return;
+    }
     float* dkp = reinterpret_cast<float*>(a.dk) + at.b * a.dks[0] + (int64_t)j * a.dks[1] +
                  at.h * a.dks[2];
     float* dvp = reinterpret_cast<float*>(a.dv) + at.b * a.dvs[0] + (int64_t)j * a.dvs[1] +
@@ -545,7 +572,8 @@ enum class Which { kFwd, kDq, kDkv };
 template <int DB, Which kWhich, int kMode>
 int launch(const AttnArgs& a, hipStream_t st) {
     const int n_rows = kWhich == Which::kDkv ? a.sk : a.sq;
-    const int64_t blocks = (int64_t)((n_rows + kRows - 1) / kRows) * a.batch * a.heads;
+    const int64_t blocks =
+        (int64_t)((n_rows + kRows - 1) / kRows) * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
     const size_t smem = (4 * kTile * kPitchOf<DB> + (kWhich == Which::kDkv ? 6 * kTile : 0)) *
                         sizeof(float);

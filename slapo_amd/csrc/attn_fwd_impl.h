@@ -74,7 +74,11 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
 
     const int n_bh = a.batch * a.heads;
     const int n_qt = (a.sq + kBM - 1) / kBM;
-    const int work = work_index(a);
+    int work = work_index(a), split = 0;
+    if (a.n_split > 1) {
+        split = work / (n_bh * n_qt);
+        work -= split * n_bh * n_qt;
+    }
     const int bh = work % n_bh;
     const int qt = n_qt - 1 - work / n_bh;  // heaviest (latest) query tiles first
     const int b = bh / a.heads;
@@ -97,8 +101,9 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     if constexpr (kBias)  // skip the tiles that hold nothing but padded keys
         j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads, kBias == 4>(
                                            a, b, h, reinterpret_cast<float*>(smem_raw))));
-    const int t_lo = j_lo / kBN;
-    const int t_hi = (j_hi + kBN - 1) / kBN;
+    int t_lo = j_lo / kBN;
+    int t_hi = (j_hi + kBN - 1) / kBN;
+    if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
     const int n_tiles = t_hi - t_lo;
 
     // Start-up loads, all issued before any is used: the Q^T fragments (column i = this lane's
@@ -494,7 +499,7 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
         if (a.window <= 0 && q0 + kBM <= a.sq) {
             n_fast = a.sk / kBN;
             if (a.causal) n_fast = min(n_fast, (q0 + 1) / kBN);
-            n_fast = min(n_fast, n_tiles);
+            n_fast = min(n_fast - t_lo, n_tiles);
         }
         int r = 0;
         for (; r < n_fast; ++r) iteration(r, std::true_type{});
@@ -519,6 +524,17 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
 
     // ---- epilogue ----
     const float l_tot = sum_xor32(l_run);
+    if (a.n_split > 1) {
+        const int64_t rows = (int64_t)n_bh * a.sq;
+        const int64_t row0 = (int64_t)bh * a.sq + wq0;
+        if (wq0 < a.sq)
+            store_partial<DPAD>(o_acc, 1.0f, a.part + (split * rows + row0) * a.d, a.sq - wq0, a.d);
+        if (q_row < a.sq && g == 0) {
+            float* ml = a.part + a.n_split * rows * a.d + 2 * (split * rows + row0 + i_loc);
+            ml[0] = m_run, ml[1] = l_tot;
+        }
+        return;
+    }
     const float inv_l = kDrop != 0 ? a.rng.inv_keep / l_tot : 1.0f / l_tot;
     // every wavefront is past the last barrier of the loop: the K buffers are free, and each
     // wavefront routes its 32 output rows through its own quarter of them
@@ -543,7 +559,7 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const size_t smem = (size_t)4 * kBN * Stage::kPitch * sizeof(T) +
                         (kBias == 2 || kBias == 4 ? 2 * kBN * sizeof(float) : 0);
     const int n_qt = (a.sq + kBM - 1) / kBM;
-    const int64_t blocks = (int64_t)n_qt * a.batch * a.heads;
+    const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
     auto kern = attn_fwd_kernel<T, DPAD, kBias, kDrop, kWin, kSteps>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
@@ -553,7 +569,8 @@ int launch(const AttnArgs& a, hipStream_t st) {
     // (head groups: not where the kernel draws or applies dropout bits -- its workgroups run twice as
     // long there and a group's late heavy ones become the tail: 314 -> 350 us at bf16 B4 S2048 H32
     // D80 causal, p 0.1, 588 -> 667 us at fp16 B2 S4096 H32 D96)
-    set_dispatch_order(&ordered, blocks, fwd_per_cu(DPAD, kBias, kDrop), kDrop == 0);
+    if (a.n_split == 1)
+        set_dispatch_order(&ordered, blocks, fwd_per_cu(DPAD, kBias, kDrop), kDrop == 0);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, ordered);
     return check_launch();
 }
@@ -574,15 +591,20 @@ int dispatch_flags(const AttnArgs& a, hipStream_t st) {
             if (a.dropout == 1) return launch<T, DPAD, 3, 1, 2, kSteps>(a, st);
             if (a.dropout == 2) return launch<T, DPAD, 3, 2, 2, kSteps>(a, st);
             if (a.dropout == 3) return launch<T, DPAD, 3, 3, 2, kSteps>(a, st);
-            return launch<T, DPAD, 3, 0, 2, kSteps>(a, st);
+            return a.window <= 0 ? launch<T, DPAD, 3, 0, 0, kSteps>(a, st)
+                                 : launch<T, DPAD, 3, 0, 2, kSteps>(a, st);
         }
         if (a.bias_type != SLAPO_F32)  // one value per key, no dropout (checked by the caller)
             return a.window <= 0 ? launch<T, DPAD, 4, 0, 0, kSteps>(a, st)
                                  : launch<T, DPAD, 4, 0, 2, kSteps>(a, st);
         if (a.bs[2] == 0) {  // the bias depends on the key only
-            if (a.dropout == 1) return launch<T, DPAD, 2, 1, 2, kSteps>(a, st);
+            if (a.dropout == 1)
+                return a.window <= 0 ? launch<T, DPAD, 2, 1, 0, kSteps>(a, st)
+                                     : launch<T, DPAD, 2, 1, 2, kSteps>(a, st);
             if (a.dropout == 2) return launch<T, DPAD, 2, 2, 2, kSteps>(a, st);
-            if (a.dropout == 3) return launch<T, DPAD, 2, 3, 2, kSteps>(a, st);
+            if (a.dropout == 3)
+                return a.window <= 0 ? launch<T, DPAD, 2, 3, 0, kSteps>(a, st)
+                                     : launch<T, DPAD, 2, 3, 2, kSteps>(a, st);
             if (a.window <= 0) return launch<T, DPAD, 2, 0, 0, kSteps>(a, st);
             return launch<T, DPAD, 2, 0, 2, kSteps>(a, st);
         }

@@ -334,7 +334,7 @@ void launch_attn_bwd(AttnProblem& a, const Operands& x, const Tensor& out, const
     Tensor dout = cast(grad, a.dtype).contiguous();
     if (!aligned(dout)) dout = dout.clone();
     a.prm.keep_mask = mptr(keep_mask);
-    const size_t ws_bytes = slapo_amd_attn_bwd_workspace_bytes(&a.prm);
+    const size_t ws_bytes = slapo_amd_attn_bwd_ex_workspace_bytes(&a.prm);
     const Tensor ws = floats((int64_t)(ws_bytes / 4));
     check(slapo_amd_attn_bwd_ex(&a.prm, x.ptr[0], x.ptr[1], x.ptr[2], cptr(a.bias), a.bias_type,
                                 cptr(out), cptr(dout), static_cast<const float*>(cptr(lse)),

@@ -653,6 +653,25 @@ def test_one_query_per_sequence(dtype, b, h, d, sk, layout):
     _check(q, k, v, do, mask, True, 0, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,sk,causal,window,p,layout", [
+    ((1, 1536, 1, 64), None, True, 0, 0.0, None),        # fewest tiles, causal: unequal shares
+    ((1, 1665, 1, 128), None, False, 0, 0.0, None),      # one row in the last block
+    ((1, 1540, 2, 72), None, True, 0, 0.1, "padding"),   # padded keys: shares that hold nothing else
+    ((1, 1800, 1, 80), None, True, 1600, 0.1, None),     # local window
+    ((1, 700, 1, 32), 1600, False, 0, 0.0, "square"),    # per-query mask, more keys than queries
+])
+def test_few_rows_dealt_to_many_workgroups(dtype, shape, sk, causal, window, p, layout):
+    """Calls too small to fill the device: partial results of shares of the tiles, merged."""
+    q, k, v, do, g = _inputs(*shape, dtype, sk=sk)
+    mask = None
+    if layout == "padding":
+        mask, _ = _padding_mask(shape[0], shape[1], dtype, g, shape[1] // 4)
+    elif layout == "square":
+        mask = torch.randn(1, 1, shape[1], sk, generator=g).to(dtype)
+    _check(q, k, v, do, mask, causal, window, dtype, p=p)
+
+
 # ---- seeded sweep over the whole call surface --------------------------------------------------
 @pytest.mark.parametrize("seed", range(40))
 def test_random_configurations_against_the_oracle(seed):
