@@ -120,6 +120,11 @@ Tensor dense(const Tensor& t, at::ScalarType dt) {
     return t.defined() ? cast(t.contiguous(), dt) : t;
 }
 
+// What saved-tensor hooks hand back has the values of what was saved; the kernels need it dense too.
+Tensor unpack_dense(const SavedVariable& s, std::shared_ptr<Node> owner = nullptr) {
+    const Tensor t = s.unpack(std::move(owner));
+    return t.defined() ? t.contiguous() : t;
+}
 SavedVariable keep(const Tensor& t, bool is_output = false) {
     return t.defined() ? SavedVariable(t, is_output) : SavedVariable();
 }
@@ -181,6 +186,13 @@ struct AttnProblem {
         prm.window = (int32_t)window;
         prm.scale = (float)(scale ? *scale : 1.0 / std::sqrt((double)d));
     }
+    // The strides of a mask that is read as it is, 0 on broadcast dims.  Also of the one that the
+    // backward gets back: saved-tensor hooks keep its values, not its layout.
+    void address_bias() {
+        const int64_t wanted[4] = {b(), h(), sq(), sk()};
+        for (int i = 0; i < 4; ++i)
+            prm.bias_strides[i] = bias.size(i) == 1 && wanted[i] != 1 ? 0 : bias.stride(i);
+    }
     // Additive mask, broadcast dims with stride 0.  The fp32 kernels read any layout and type.  The
     // 16-bit ones read one value per key, in the mask's own type at inference (no backward to follow,
     // no dropout); a
@@ -197,20 +209,18 @@ struct AttnProblem {
         bias = known && (infer || !per_key || dtype == at::kFloat) ? mask : cast(mask, at::kFloat);
         bias_type = dtype_code(bias.scalar_type());
         const int64_t wanted[4] = {b(), h(), sq(), sk()};
-        for (int i = 0; i < 4; ++i) {
-            const int64_t n = bias.size(i);
-            TORCH_CHECK(n == wanted[i] || n == 1, "attention_mask of shape ", mask.sizes(),
-                        " does not broadcast to [", b(), ", ", h(), ", ", sq(), ", ", sk(), "]");
-            prm.bias_strides[i] = n == 1 && wanted[i] != 1 ? 0 : bias.stride(i);
-        }
+        for (int i = 0; i < 4; ++i)
+            TORCH_CHECK(bias.size(i) == wanted[i] || bias.size(i) == 1, "attention_mask of shape ",
+                        mask.sizes(), " does not broadcast to [", b(), ", ", h(), ", ", sq(), ", ",
+                        sk(), "]");
+        address_bias();
         if (dtype == at::kFloat || per_key || empty() || sk() == 0) return;
         const int64_t mb = prm.bias_strides[0] ? b() : 1, mh = prm.bias_strides[1] ? h() : 1;
         const int64_t bytes =
             (int64_t)slapo_amd_attn_prepared_bias_bytes(mb, mh, sq(), sk());
         if (bytes == 0 || (bias_type == SLAPO_F32 && mb * mh == b() * h())) {
             bias = cast(bias, at::kFloat);
-            for (int i = 0; i < 4; ++i)
-                if (prm.bias_strides[i]) prm.bias_strides[i] = bias.stride(i);
+            address_bias();
             bias_type = SLAPO_F32;
             return;
         }
@@ -377,7 +387,7 @@ struct AttnBackward : Node {
         Tensor dst[3];
         void* dst_ptr[3];
         int64_t ds[3][3];
-        const Tensor tout = out.unpack(getptr()), tlse = lse.unpack();
+        const Tensor tout = unpack_dense(out, getptr()), tlse = unpack_dense(lse);
         const c10::OptionalDeviceGuard guard(tout.device());
         if (packed) {
             in.take_packed(call, x[0].unpack());
@@ -396,10 +406,16 @@ struct AttnBackward : Node {
                 if (t.defined()) t.zero_();
         } else {
             call.bias = bias.unpack();
-            call.drop.state = state.unpack();
+            if (call.bias.defined()) {
+                if (call.bias_type == SLAPO_BIAS_PREPARED)
+                    call.bias = call.bias.contiguous();
+                else
+                    call.address_bias();
+            }
+            call.drop.state = unpack_dense(state);
             if (call.drop.state.defined())
                 call.prm.plan.rng_state = call.drop.state.const_data_ptr();
-            launch_attn_bwd(call, in, tout, tlse, keep_mask.unpack(), grads[0], dst_ptr, ds);
+            launch_attn_bwd(call, in, tout, tlse, unpack_dense(keep_mask), grads[0], dst_ptr, ds);
         }
         for (size_t i = 0; i < res.size(); ++i)
             if (task_should_compute_output(i)) res[i] = dst[i];
@@ -549,7 +565,7 @@ struct CrossEntropyBackward : Node {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list res(1);
         if (!grads[0].defined()) return res;
-        const Tensor x = logits.unpack(), t = target.unpack(), st = stats.unpack();
+        const Tensor x = unpack_dense(logits), t = unpack_dense(target), st = unpack_dense(stats);
         const c10::OptionalDeviceGuard guard(x.device());
         const Tensor g = dense(grads[0], at::kFloat);
         res[0] = fresh_like(x);
@@ -629,7 +645,7 @@ struct BiasGeluBackward : Node {
         variable_list res(2);
         if (!grads[0].defined()) return res;
         const bool need_bias = task_should_compute_output(1);
-        const Tensor ty = y.unpack(), tb = bias.unpack();
+        const Tensor ty = unpack_dense(y), tb = unpack_dense(bias);
         const c10::OptionalDeviceGuard guard(ty.device());
         const Tensor g = dense(grads[0], ty.scalar_type());
         const auto [rows, cols] = rows_cols(ty, tb);
@@ -713,7 +729,7 @@ struct BiasDropoutBackward : Node {
             if (need_bias) db.zero_();
         } else {
             Dropout d = drop;
-            d.state = state.unpack();
+            d.state = unpack_dense(state);
             if (d.state.defined()) d.plan.rng_state = d.state.const_data_ptr();
             size_t ws_bytes = 0;
             if (need_bias) ws = colsum_workspace(rows, cols, &ws_bytes);
@@ -783,7 +799,7 @@ struct LayerNormBackward : Node {
         std::lock_guard<std::mutex> lock(mutex_);
         variable_list res(5);  // x, bias, residual, weight, ln_bias
         if (!grads[0].defined()) return res;
-        const Tensor tz = z.unpack(), tstats = stats.unpack(), tw = weight.unpack();
+        const Tensor tz = unpack_dense(z), tstats = unpack_dense(stats), tw = unpack_dense(weight);
         const c10::OptionalDeviceGuard guard(tz.device());
         const at::ScalarType dt = tz.scalar_type();
         const Tensor g = dense(grads[0], dt);
@@ -805,7 +821,7 @@ struct LayerNormBackward : Node {
                 if (t.defined()) t.zero_();
         } else if (need[0] || need[1] || need[2] || need[3] || need[4]) {
             Dropout d = drop;
-            d.state = state.unpack();
+            d.state = unpack_dense(state);
             if (d.state.defined()) d.plan.rng_state = d.state.const_data_ptr();
             Tensor ws;
             size_t ws_bytes = 0;

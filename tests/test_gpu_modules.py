@@ -243,3 +243,23 @@ def test_packed_attention_equals_the_split_call(dtype, head_dim, p):
                                                   torch.ones_like(out))])
     for a, r in zip(*results):
         assert torch.equal(a, r)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("layout", ["expanded", "sliced"])
+def test_attention_backward_with_saved_tensors_kept_on_the_host(dtype, layout):
+    # the hooks bring a saved mask back dense, whatever its strides were in the forward
+    torch.manual_seed(0)
+    b, s, h, d = 2, 96, 2, 64
+    q, k, v = (torch.randn(b, s, h, d, dtype=dtype, device="cuda", requires_grad=True)
+               for _ in range(3))
+    if layout == "expanded":
+        mask = torch.randn(1, 1, 1, s, device="cuda").expand(b, h, 1, s)
+    else:
+        mask = torch.randn(b, h, s, 2 * s, device="cuda")[..., ::2]
+    g = torch.randn(b, s, h, d, dtype=dtype, device="cuda")
+    plain = torch.autograd.grad(op.hip_attention(q, k, v, mask, causal=True), (q, k, v), g)
+    with torch.autograd.graph.save_on_cpu():
+        out = op.hip_attention(q, k, v, mask, causal=True)
+    for a, r in zip(torch.autograd.grad(out, (q, k, v), g), plain):
+        assert torch.equal(a, r)
