@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -23,6 +24,7 @@
 #include <ATen/core/Generator.h>
 #include <ATen/detail/CUDAHooksInterface.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 
@@ -502,6 +504,15 @@ struct QkvSplitBackward : Node {
         variable_list res(1);
         if (!grads[0].defined() && !grads[1].defined() && !grads[2].defined()) return res;
         const c10::OptionalDeviceGuard guard(device);
+        if (c10::GradMode::is_enabled()) {  // create_graph: of operations that can be derived again
+            Tensor like;
+            for (const Tensor& t : grads)
+                if (t.defined()) like = t;
+            std::vector<Tensor> parts;
+            for (const Tensor& t : grads) parts.push_back(t.defined() ? t : at::zeros_like(like));
+            res[0] = at::stack(parts, -1).reshape(sizes);
+            return res;
+        }
         Tensor g[3];
         const Tensor packed = fresh(sizes, dtype);
         for (int i = 0; i < 3; ++i) {
@@ -518,6 +529,20 @@ struct QkvSplitBackward : Node {
         return res;
     }
 };
+
+// Whether qkv_split stands in for the torch operations: not where something watches those (vmap and
+// the other function transforms, forward-mode differentiation, tracing, a dispatch mode) and not for
+// types that the kernel does not move.
+bool qkv_plain(const Tensor& packed) {
+    const auto t = packed.scalar_type();
+    return packed.is_cuda() && (t == at::kFloat || t == at::kHalf || t == at::kBFloat16) &&
+           !packed.key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::FuncTorchBatched,
+                                                          c10::DispatchKey::FuncTorchGradWrapper,
+                                                          c10::DispatchKey::Functionalize,
+                                                          c10::DispatchKey::Python})) &&
+           !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+           !torch::jit::tracer::isTracing() && !packed._fw_grad(0).defined();
+}
 
 // [.., heads * head_size * 3] -> three [.., heads, head_size]
 std::array<Tensor, 3> qkv_split(const Tensor& packed_in, int64_t heads, int64_t head_size) {
@@ -998,6 +1023,14 @@ PyObject* py_attention_packed(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
+// qkv_plain(packed)
+PyObject* py_qkv_plain(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 1, "qkv_plain");
+    return PyBool_FromLong(qkv_plain(tensor_arg(a[0], "packed")));
+    END_HANDLE_TH_ERRORS
+}
+
 // qkv_split(packed, heads, head_size): [q, k, v]
 PyObject* py_qkv_split(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
@@ -1120,6 +1153,7 @@ PyMethodDef methods[] = {
     SLAPO_METHOD("attention", py_attention),
     SLAPO_METHOD("attention_packed", py_attention_packed),
     SLAPO_METHOD("attention_scores", py_attention_scores),
+    SLAPO_METHOD("qkv_plain", py_qkv_plain),
     SLAPO_METHOD("qkv_split", py_qkv_split),
     SLAPO_METHOD("cross_entropy", py_cross_entropy),
     SLAPO_METHOD("bias_gelu", py_bias_gelu),

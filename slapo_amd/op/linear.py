@@ -35,7 +35,8 @@ class FusedQKV(nn.Module):
 
     def forward(self, hidden_states):
         packed = self.fused_linear(hidden_states)
-        if type(packed) is Tensor and packed.is_cuda:  # one pass instead of three strided copies
+        if (type(packed) is Tensor and packed.is_cuda and not torch.compiler.is_compiling()
+                and host().qkv_plain(packed)):  # one pass instead of three strided copies
             return host().qkv_split(packed, self.num_heads // self.world_size, self.head_size)
         packed = self.reshape_for_scores(packed)
         return [t.squeeze(-1).contiguous() for t in torch.split(packed, 1, dim=-1)]

@@ -263,3 +263,33 @@ def test_attention_backward_with_saved_tensors_kept_on_the_host(dtype, layout):
         out = op.hip_attention(q, k, v, mask, causal=True)
     for a, r in zip(torch.autograd.grad(out, (q, k, v), g), plain):
         assert torch.equal(a, r)
+
+
+def test_fused_qkv_where_its_operations_are_watched():
+    torch.manual_seed(0)
+    m = op.FusedQKV(32, 4, 1).cuda().double()
+    x = torch.randn(2, 6, 32, device="cuda", dtype=torch.float64)
+
+    def ref(x):
+        packed = m.fused_linear(x).view(*x.shape[:-1], 4, 8, 3)
+        return [t.squeeze(-1) for t in packed.split(1, dim=-1)]
+
+    def check(got, want):
+        for a, r in zip(got, want):
+            assert torch.equal(a, r)
+
+    check(m(x), ref(x))  # a type that the kernel does not move
+    m, x = m.float(), x.float()
+    check(m(x), ref(x))
+    batched = torch.func.vmap(lambda t: tuple(m(t)))(x)
+    assert all(a.shape == (2, 6, 4, 8) for a in batched)
+    _, tangents = torch.func.jvp(lambda t: tuple(m(t)), (x,), (x,))
+    _, wanted = torch.func.jvp(lambda t: tuple(ref(t)), (x,), (x,))
+    check(tangents, wanted)
+    x = x.requires_grad_()  # a second derivative reaches the incoming gradient
+    g = torch.randn(2, 6, 4, 8, device="cuda", requires_grad=True)
+    seconds = []
+    for f in (m, ref):
+        first, = torch.autograd.grad(f(x)[1], x, g, create_graph=True)
+        seconds.append(torch.autograd.grad(first.square().sum(), g)[0])
+    torch.testing.assert_close(*seconds)
