@@ -162,6 +162,11 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a,
                 __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(vp + j * a.vs[1] + col));
             s[u] = bias ? bias_load(a, bias_at + j * a.bs[3]) : 0.f;
         }
+        if (j0 + kSpan > k_hi) {  // rows past the end: zeros, as 0 * inf would not be one
+#pragma unroll
+            for (int u = 0; u < kStrip; ++u)
+                if (j0 + u * kGroups + group >= k_hi) vv[u] = Row16<T>{};
+        }
         float mx = m;
 #pragma unroll
         for (int u = 0; u < kStrip; ++u) {

@@ -215,6 +215,8 @@ struct AttnProblem {
             TORCH_CHECK(bias.size(i) == wanted[i] || bias.size(i) == 1, "attention_mask of shape ",
                         mask.sizes(), " does not broadcast to [", b(), ", ", h(), ", ", sq(), ", ",
                         sk(), "]");
+        // (the kernels address a row's values with 32-bit offsets)
+        if (bias.size(3) > 1 && bias.stride(3) * sk() >= int64_t(1) << 30) bias = bias.contiguous();
         address_bias();
         if (dtype == at::kFloat || per_key || empty() || sk() == 0) return;
         const int64_t mb = prm.bias_strides[0] ? b() : 1, mh = prm.bias_strides[1] ? h() : 1;

@@ -653,6 +653,17 @@ def test_one_query_per_sequence(dtype, b, h, d, sk, layout):
     _check(q, k, v, do, mask, True, 0, dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_one_query_with_an_infinite_value_at_the_last_key(dtype):
+    q, k, v, _, _ = _inputs(1, 1, 2, 64, dtype, sk=333)
+    clean = op.hip_attention(q.cuda(), k.cuda(), v.cuda())
+    v[0, -1, 1, 5] = float("inf")
+    out = op.hip_attention(q.cuda(), k.cuda(), v.cuda())
+    assert out[0, 0, 1, 5].item() == float("inf")
+    out[0, 0, 1, 5] = clean[0, 0, 1, 5]
+    assert torch.equal(out, clean)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("shape,sk,causal,window,p,layout", [
     ((1, 1536, 1, 64), None, True, 0, 0.0, None),        # fewest tiles, causal: unequal shares
