@@ -382,16 +382,6 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const float* __restr
 // unfused modules compute from the stored sum; z is also what the backward reads.
 // ----------------------------------------------------------------------------------------
 constexpr int kLnChunks = 4;         // 16-byte chunks per thread and row (guarded against cols)
-// Backward: rows that one block walks before it writes its column sums.  16, or fewer where that would
-// leave the device less than two blocks per CU -- the rows of a block run one after the other (a
-// block-wide row at a time above 64 V * 2 columns, eight wavefront rows at a time below): fp16
-// 384 x 2560 in 24 blocks took @LNB@.
-inline int ln_rows_per_block(int64_t rows, bool wide) {
-    int rpb = 16;
-    while (rpb > (wide ? 2 : 8) && (rows + rpb - 1) / rpb < 512) rpb /= 2;
-    return rpb;
-}
-
 // Sum over the 64 lanes, on every lane, without LDS traffic: butterflies inside the 16-lane
 // rows through DPP (quad permutes, row rotations), then the four row sums through v_readlane.
 template <int kCtrl>
@@ -527,66 +517,104 @@ __global__ __launch_bounds__(256) void bias_dropout_residual_ln_fwd_kernel(
 // Backward of the above.  With xh = (z - mean) rstd and g = dy gamma:
 //   dz = rstd (g - mean_c(g) - xh mean_c(g xh)),  dresidual = dz,  dx = dz keep / (1 - p),
 //   dgamma = sum_r dy xh,  dbeta = sum_r dy,  dbias = sum_r dx.
-// A block walks rows_per_block rows and keeps the three column sums of its threads in
-// registers; they leave as one fp32 partial row triple per block ([block][3][cols]: dgamma, dbeta,
-// dbias) for ln_finish_kernel.  No atomics: the result does not depend on scheduling.
-// NV = 16-byte chunks per thread and row (1, 2 or 4, the smallest that covers cols): the column
-// sums cost 3 * NV * V registers, and registers decide how many rows a CU has in flight.  The
-// loads of the next two rows are issued before the current row is reduced.
-template <typename T, int V, int NV, int TPR, int kDrop, int kThreads>
-__global__ __launch_bounds__(kThreads, (kThreads == 512 && kDrop != 2) ? 4 : 1)
-void bias_dropout_residual_ln_bwd_kernel(
+// A block of eight wavefronts holds 512 / TPR rows at a time, TPR threads each, and walks
+// rows_per_block of them; a thread keeps the three column sums of its columns in registers, the block
+// adds those of its row groups through LDS, and they leave as one fp32 partial row triple per block
+// ([block][3][cols]: dgamma, dbeta, dbias) for ln_finish_kernel.  No atomics: the result does not
+// depend on scheduling.
+// Bound by vector instructions and memory about equally (some 40 instructions per element with
+// dropout, 15 of them the mask's Philox rounds, against 8 bytes), so what counts is how many
+// wavefronts a SIMD has to overlap the two with: TPR is the smallest width at which a thread has one
+// 16-byte chunk per row (NV = 1; 2 above 512 chunks only), which leaves room for four wavefronts per
+// SIMD and for the loads of the next kAhead rows.  With a
+// wavefront per row up to 1024 columns the build for two chunks spilled 52 registers, and the wide
+// rows had one or two wavefronts per SIMD.  Both kernels together, before -> after (p 0.1): fp16
+// 1537 x 768 18.0 -> 9.4 us, bf16 4096 x 1024 34.4 -> 13.2, 4096 x 2048 31.3 -> 22.7, 8192 x 4096
+// 81.5 -> 66.8 (4.0 TB/s), fp16 2000 x 8000 115 -> 53.
+constexpr int kLnbThreads = 512;
+// Blocks of a launch: one for each of the 256 CUs, which walk the rows that fall to them, so that the
+// partial rows -- 24 bytes per block and column, written and read again -- stay few (bf16 4096 x 1024,
+// p 0: 10.7 us with 256 blocks, 14.0 with 512, 21.1 with 1024).  Two per CU where the launch is long
+// enough to pay for them and dropout makes it wait for vector instructions more than for partial rows
+// (bf16, p 0.1, 256 / 512 blocks: 4096 x 1024 13.3 / 15.4 us, 8192 x 768 20.0 / 18.5, 8192 x 2560
+// 65.0 / 49.8).
+inline int64_t lnb_blocks(int64_t rows, int64_t cols, bool dropout) {
+    const int64_t most = dropout && rows * cols >= 5 << 20 ? 512 : 256;
+    return rows < most ? rows : most;
+}
+
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// Sums of a and b over the TPR threads of a row; red: LDS of this iteration, [wavefront][2].
+template <int TPR>
+__device__ __forceinline__ void row_sums(float& a, float& b, float (*red)[2]) {
+    a = wave_sum(a), b = wave_sum(b);
+    if constexpr (TPR > 64) {
+        const int w = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 0) red[w][0] = a, red[w][1] = b;
+        __syncthreads();
+        const int first = w & ~(TPR / 64 - 1);
+        a = b = 0.f;
+#pragma unroll
+        for (int i = 0; i < TPR / 64; ++i) a += red[first + i][0], b += red[first + i][1];
+    }
+}
+
+template <typename T, int V, int NV, int TPR, int kDrop>
+__global__ __launch_bounds__(kLnbThreads, NV == 1 ? 4 : 2) void bias_dropout_residual_ln_bwd_kernel(
     const T* __restrict__ dy, const T* __restrict__ z, const float* __restrict__ mean,
     const float* __restrict__ rstd, const T* __restrict__ gamma, T* __restrict__ dx,
     T* __restrict__ dres, float* __restrict__ partial, int64_t rows, int cols, int rows_per_block,
     DropoutState s) {
     if constexpr (kDrop != 0) resolve_device_state(s);
-    static_assert(TPR == 256 ? kThreads == 256 : (kThreads == 256 || kThreads == 512),
-                  "a block is one wide row, or four or eight wavefront rows");
-    constexpr int kRows = kThreads / TPR;  // rows in flight per block
+    constexpr int kRows = kLnbThreads / TPR;  // rows in flight per block
+    constexpr int kAhead = kDrop == 2 || NV > 1 ? 1 : 2;
+    constexpr int kQuads = 3 * V / 4;  // of a thread's column sums per chunk
+    static_assert(kRows == 1 || NV == 1, "several rows per block: one chunk per thread");
     const int n_iters = rows_per_block / kRows;
-    constexpr int kCombCols = TPR == 64 ? 64 * V * NV : 1;
-    __shared__ float red[2][2][4];
-    __shared__ float comb[4 * 3 * kCombCols];
+    __shared__ float red[2][kLnbThreads / 64][2];
+    __shared__ f32x4_t comb[kRows > 1 ? kQuads * kLnbThreads : 1];
     const int sub = threadIdx.x % TPR;
     const int rr = threadIdx.x / TPR;
     Chunk<T, V> gm[NV];
-    float acc_g[NV][V], acc_b[NV][V], acc_x[NV][V];
+    float acc[NV][3][V];
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
         const int col0 = (sub + u * TPR) * V;
         if (col0 < cols) gm[u] = load_chunk_cached<T, V>(gamma + col0);
 #pragma unroll
-        for (int i = 0; i < V; ++i) acc_g[u][i] = 0.f, acc_b[u][i] = 0.f, acc_x[u][i] = 0.f;
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int i = 0; i < V; ++i) acc[u][k][i] = 0.f;
     }
     const float inv_n = 1.0f / (float)cols;
     const int64_t row0 = (int64_t)blockIdx.x * rows_per_block + rr;
 
-    // rows it + 1 and it + 2 are in flight while row it is processed
-    Chunk<T, V> gy[NV], zz[NV], gy_n1[NV], zz_n1[NV], gy_n2[NV], zz_n2[NV];
-    float m = 0.f, rs = 0.f, m_n1 = 0.f, rs_n1 = 0.f, m_n2 = 0.f, rs_n2 = 0.f;
-    auto request = [&](int64_t row, Chunk<T, V> (&g)[NV], Chunk<T, V> (&zc)[NV], float& mm,
-                       float& rr_) __attribute__((always_inline)) {
-        if (row < rows) {  // uniform per wavefront
-            mm = mean[row];
-            rr_ = rstd[row];
+    // slot 0 holds the row in process, slot k the k-th after it
+    Chunk<T, V> gy[kAhead + 1][NV], zz[kAhead + 1][NV];
+    float m[kAhead + 1], rs[kAhead + 1];
+    auto request = [&](int it, int slot) __attribute__((always_inline)) {
+        const int64_t row = row0 + (int64_t)it * kRows;
+        if (it < n_iters && row < rows) {  // uniform per wavefront
+            m[slot] = mean[row];
+            rs[slot] = rstd[row];
 #pragma unroll
             for (int u = 0; u < NV; ++u) {
                 const int col0 = (sub + u * TPR) * V;
                 if (col0 < cols) {
-                    g[u] = load_chunk<T, V>(dy + row * cols + col0);
-                    zc[u] = load_chunk<T, V>(z + row * cols + col0);
+                    gy[slot][u] = load_chunk<T, V>(dy + row * cols + col0);
+                    zz[slot][u] = load_chunk<T, V>(z + row * cols + col0);
                 }
             }
         }
     };
-    request(row0, gy, zz, m, rs);
-    if (n_iters > 1) request(row0 + kRows, gy_n1, zz_n1, m_n1, rs_n1);
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) request(k, k);
 #pragma unroll 1
     for (int it = 0; it < n_iters; ++it) {
-        const int64_t row = row0 + it * kRows;
+        const int64_t row = row0 + (int64_t)it * kRows;
         const bool row_ok = row < rows;  // uniform per wavefront
-        if (it + 2 < n_iters) request(row + 2 * kRows, gy_n2, zz_n2, m_n2, rs_n2);
+        request(it + kAhead, kAhead);
         float s1 = 0.f, s2 = 0.f;
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
@@ -594,18 +622,18 @@ void bias_dropout_residual_ln_bwd_kernel(
             if (row_ok && col0 < cols) {
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const float d = Elem<T>::to_f32(gy[u].v[i]);
-                    const float xh = (Elem<T>::to_f32(zz[u].v[i]) - m) * rs;
+                    const float d = Elem<T>::to_f32(gy[0][u].v[i]);
+                    const float xh = (Elem<T>::to_f32(zz[0][u].v[i]) - m[0]) * rs[0];
                     const float g = d * Elem<T>::to_f32(gm[u].v[i]);
                     s1 += g;
                     s2 = __builtin_fmaf(g, xh, s2);
-                    acc_g[u][i] = __builtin_fmaf(d, xh, acc_g[u][i]);
-                    acc_b[u][i] += d;
+                    acc[u][0][i] = __builtin_fmaf(d, xh, acc[u][0][i]);
+                    acc[u][1][i] += d;
                 }
             }
         }
-        const float c1 = row_sum<TPR>(s1, red[it & 1][0]) * inv_n;
-        const float c2 = row_sum<TPR>(s2, red[it & 1][1]) * inv_n;
+        row_sums<TPR>(s1, s2, red[it & 1]);
+        const float c1 = s1 * inv_n, c2 = s2 * inv_n;
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
             const int col0 = (sub + u * TPR) * V;
@@ -616,140 +644,98 @@ void bias_dropout_residual_ln_bwd_kernel(
                 Chunk<T, V> oz, ox;
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const float xh = (Elem<T>::to_f32(zz[u].v[i]) - m) * rs;
-                    const float g = Elem<T>::to_f32(gy[u].v[i]) * Elem<T>::to_f32(gm[u].v[i]);
-                    const float dz = rs * (g - c1 - xh * c2);
+                    const float xh = (Elem<T>::to_f32(zz[0][u].v[i]) - m[0]) * rs[0];
+                    const float g = Elem<T>::to_f32(gy[0][u].v[i]) * Elem<T>::to_f32(gm[u].v[i]);
+                    const float dz = rs[0] * (g - c1 - xh * c2);
                     float d = dz;
                     if constexpr (kDrop != 0) d = ((bits >> i) & 1u) ? dz * s.inv_keep : 0.0f;
                     oz.v[i] = Elem<T>::from_f32(dz);
                     ox.v[i] = Elem<T>::from_f32(d);
-                    acc_x[u][i] += d;
+                    acc[u][2][i] += d;
                 }
                 if (dres) store_chunk<T, V>(dres + off, oz);
                 if (dx) store_chunk<T, V>(dx + off, ox);
             }
         }
 #pragma unroll
-        for (int u = 0; u < NV; ++u) {
-            gy[u] = gy_n1[u], zz[u] = zz_n1[u];
-            gy_n1[u] = gy_n2[u], zz_n1[u] = zz_n2[u];
+        for (int k = 0; k < kAhead; ++k) {
+#pragma unroll
+            for (int u = 0; u < NV; ++u) gy[k][u] = gy[k + 1][u], zz[k][u] = zz[k + 1][u];
+            m[k] = m[k + 1], rs[k] = rs[k + 1];
         }
-        m = m_n1, rs = rs_n1, m_n1 = m_n2, rs_n1 = rs_n2;
     }
     if (!partial) return;
     float* out = partial + (int64_t)blockIdx.x * 3 * cols;
-    if constexpr (TPR == 256) {
+    // quad q of a chunk: values 4 (q % (V / 4)) .. + 3 of column sum q / (V / 4)
+    auto put = [&](int col0, int q, const f32x4_t& v) __attribute__((always_inline)) {
+        *reinterpret_cast<f32x4_any*>(out + (int64_t)(q / (V / 4)) * cols + col0 + q % (V / 4) * 4) = v;
+    };
+    auto mine = [&](int u, int q) __attribute__((always_inline)) {
+        const float* a = &acc[u][q / (V / 4)][q % (V / 4) * 4];
+        return f32x4_t{a[0], a[1], a[2], a[3]};
+    };
+    if constexpr (kRows == 1) {
 #pragma unroll
         for (int u = 0; u < NV; ++u) {
             const int col0 = (sub + u * TPR) * V;
             if (col0 < cols) {
 #pragma unroll
-                for (int i = 0; i < V; ++i) {
-                    out[col0 + i] = acc_g[u][i];
-                    out[cols + col0 + i] = acc_b[u][i];
-                    out[2 * cols + col0 + i] = acc_x[u][i];
-                }
+                for (int q = 0; q < kQuads; ++q) put(col0, q, mine(u, q));
             }
         }
     } else {
-        // every wavefront (row group) parks its sums in LDS, then the block adds the four copies
-        // column by column and writes the partial row with consecutive lanes on consecutive
-        // columns
-        float* mine = comb + (rr & 3) * 3 * kCombCols;
-        if constexpr (kRows == 8) {
-            // the upper four wavefronts hand their sums to the lower four first, so that the
-            // parking area stays at four copies
-            if (rr >= 4) {
 #pragma unroll
-                for (int u = 0; u < NV; ++u) {
-                    const int col0 = (sub + u * TPR) * V;
-                    if (col0 < cols) {
-#pragma unroll
-                        for (int i = 0; i < V; ++i) {
-                            mine[col0 + i] = acc_g[u][i];
-                            mine[kCombCols + col0 + i] = acc_b[u][i];
-                            mine[2 * kCombCols + col0 + i] = acc_x[u][i];
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-            if (rr < 4) {
-#pragma unroll
-                for (int u = 0; u < NV; ++u) {
-                    const int col0 = (sub + u * TPR) * V;
-                    if (col0 < cols) {
-#pragma unroll
-                        for (int i = 0; i < V; ++i) {
-                            acc_g[u][i] += mine[col0 + i];
-                            acc_b[u][i] += mine[kCombCols + col0 + i];
-                            acc_x[u][i] += mine[2 * kCombCols + col0 + i];
-                        }
-                    }
-                }
-            }
-            __syncthreads();
-        }
-        if (rr < 4) {
-#pragma unroll
-            for (int u = 0; u < NV; ++u) {
-                const int col0 = (sub + u * TPR) * V;
-                if (col0 < cols) {
-#pragma unroll
-                    for (int i = 0; i < V; ++i) {
-                        mine[col0 + i] = acc_g[u][i];
-                        mine[kCombCols + col0 + i] = acc_b[u][i];
-                        mine[2 * kCombCols + col0 + i] = acc_x[u][i];
-                    }
-                }
-            }
-        }
+        for (int q = 0; q < kQuads; ++q) comb[q * kLnbThreads + threadIdx.x] = mine(0, q);
         __syncthreads();
-        for (int c = threadIdx.x; c < 3 * cols; c += kThreads) {
-            const int which = c / cols;
-            const int idx = which * kCombCols + (c - which * cols);
-            out[c] = (comb[idx] + comb[3 * kCombCols + idx]) +
-                     (comb[6 * kCombCols + idx] + comb[9 * kCombCols + idx]);
+        // row group rr adds up quads rr, rr + kRows, ... of all groups
+        if (sub * V < cols) {
+            for (int q = rr; q < kQuads; q += kRows) {
+                f32x4_t v = comb[q * kLnbThreads + sub];
+#pragma unroll
+                for (int r = 1; r < kRows; ++r) v += comb[q * kLnbThreads + r * TPR + sub];
+                put(sub * V, q, v);
+            }
         }
     }
 }
 
 // Second stage: partial is [n_partials][3 * cols]; column c of it belongs to dgamma (c < cols),
-// dbeta or dbias.  A block owns kFC columns and kFR row-lanes (kFC * kFR = 256): narrow tiles for
-// small matrices (many blocks, the stage is a chain of L2 round trips), 256-byte segments for
-// large ones (the stage is then bound by reading the partials).
-template <typename T, int kFC, int kFR>
+// dbeta or dbias.  A block owns 32 columns and eight row-lanes: 128-byte segments, and with 256 partial
+// rows one round of 32 loads per thread (16 columns x 16 row-lanes and 64 x 4 take 0.5-1 us longer
+// at 768 to 2048 columns).
+constexpr int kLnFinCols = 32, kLnFinLanes = 8;
+template <typename T>
 __global__ __launch_bounds__(256) void ln_finish_kernel(const float* __restrict__ partial,
                                                         T* __restrict__ dgamma,
                                                         T* __restrict__ dbeta,
                                                         T* __restrict__ dbias, int64_t n_partials,
                                                         int cols) {
-    static_assert(kFC * kFR == 256, "one thread per (column, row-lane)");
-    __shared__ float red[kFR][kFC + 1];
-    const int cx = threadIdx.x % kFC;
-    const int ry = threadIdx.x / kFC;
+    static_assert(kLnFinCols * kLnFinLanes == 256, "one thread per (column, row-lane)");
+    __shared__ float red[kLnFinLanes][kLnFinCols + 1];
+    const int cx = threadIdx.x % kLnFinCols;
+    const int ry = threadIdx.x / kLnFinCols;
     const int64_t cols3 = 3 * (int64_t)cols;
-    const int64_t c = (int64_t)blockIdx.x * kFC + cx;
+    const int64_t c = (int64_t)blockIdx.x * kLnFinCols + cx;
     float t = 0.f;
     if (c < cols3) {
         // 32 loads in flight per thread while that many rows are left, then eight
         float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         int64_t k = ry;
-        for (; k + (kFinWide - 1) * kFR < n_partials; k += kFinWide * kFR) {
+        for (; k + (kFinWide - 1) * kLnFinLanes < n_partials; k += kFinWide * kLnFinLanes) {
             float v[kFinWide];
 #pragma unroll
-            for (int j = 0; j < kFinWide; ++j) v[j] = partial[(k + j * kFR) * cols3 + c];
+            for (int j = 0; j < kFinWide; ++j) v[j] = partial[(k + j * kLnFinLanes) * cols3 + c];
 #pragma unroll
             for (int j = 0; j < kFinWide; ++j) acc[j & 7] += v[j];
         }
-        for (; k + 7 * kFR < n_partials; k += 8 * kFR) {
+        for (; k + 7 * kLnFinLanes < n_partials; k += 8 * kLnFinLanes) {
             float v[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = partial[(k + j * kFR) * cols3 + c];
+            for (int j = 0; j < 8; ++j) v[j] = partial[(k + j * kLnFinLanes) * cols3 + c];
 #pragma unroll
             for (int j = 0; j < 8; ++j) acc[j] += v[j];
         }
-        for (; k < n_partials; k += kFR) acc[0] += partial[k * cols3 + c];
+        for (; k < n_partials; k += kLnFinLanes) acc[0] += partial[k * cols3 + c];
         t = ((acc[0] + acc[1]) + (acc[2] + acc[3])) + ((acc[4] + acc[5]) + (acc[6] + acc[7]));
     }
     red[ry][cx] = t;
@@ -757,7 +743,7 @@ __global__ __launch_bounds__(256) void ln_finish_kernel(const float* __restrict_
     if (ry == 0 && c < cols3) {
         float sum = 0.f;
 #pragma unroll
-        for (int r = 0; r < kFR; ++r) sum += red[r][cx];
+        for (int r = 0; r < kLnFinLanes; ++r) sum += red[r][cx];
         const int which = (int)(c / cols);
         T* dst = which == 0 ? dgamma : which == 1 ? dbeta : dbias;
         if (dst) dst[c - (int64_t)which * cols] = Elem<T>::from_f32(sum);
@@ -982,49 +968,45 @@ int ln_bwd_dispatch(const void* dy, const void* z, const float* mean, const floa
     for (const void* p : {dy, z, gamma, (const void*)dx, (const void*)dres})
         if (p && !aligned16(p)) return SLAPO_ERR_ALIGN;
     const bool want_sums = dgamma || dbeta || dbias;
-    const int rpb = ln_rows_per_block(rows, wide);
+    const int chunks = (int)(cols / V);  // per row
+    const int tpr = chunks <= 64 ? 64 : chunks <= 128 ? 128 : chunks <= 256 ? 256 : kLnbThreads;
+    const int in_flight = kLnbThreads / tpr;
+    const int64_t most_blocks = lnb_blocks(rows, cols, dropout);
+    const int64_t per_block = (rows + most_blocks - 1) / most_blocks;
+    const int64_t rpb64 = (per_block + in_flight - 1) / in_flight * in_flight;
+    if (rpb64 > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
+    const int rpb = (int)rpb64;
     const int64_t n_blocks = (rows + rpb - 1) / rpb;
     float* partial = want_sums ? (float*)ws : nullptr;
     const int mode = !dropout ? 0 : (s.g_shift >= 0 && s.t_shift >= 0) ? 1 : 2;
-#define SLAPO_LAUNCH_LNB(NV, TPR, MODE)                                                         \
-    hipLaunchKernelGGL(                                                                         \
-        (bias_dropout_residual_ln_bwd_kernel<T, V, NV, TPR, MODE, (TPR == 64 ? 512 : 256)>),    \
-        dim3((unsigned)n_blocks), dim3(TPR == 64 ? 512 : 256), 0, st, (const T*)dy,             \
-        (const T*)z, mean, rstd, (const T*)gamma, (T*)dx, (T*)dres, partial, rows, (int)cols, rpb, s)
-#define SLAPO_LAUNCH_LNB_MODE(NV, TPR)            \
-    do {                                          \
+#define SLAPO_LAUNCH_LNB(NV, TPR, MODE)                                                        \
+    hipLaunchKernelGGL((bias_dropout_residual_ln_bwd_kernel<T, V, NV, TPR, MODE>),             \
+                       dim3((unsigned)n_blocks), dim3(kLnbThreads), 0, st, (const T*)dy,       \
+                       (const T*)z, mean, rstd, (const T*)gamma, (T*)dx, (T*)dres, partial, rows, \
+                       (int)cols, rpb, s)
+#define SLAPO_LAUNCH_LNB_MODE(NV, TPR)               \
+    do {                                             \
         if (mode == 0) SLAPO_LAUNCH_LNB(NV, TPR, 0); \
         if (mode == 1) SLAPO_LAUNCH_LNB(NV, TPR, 1); \
         if (mode == 2) SLAPO_LAUNCH_LNB(NV, TPR, 2); \
     } while (0)
-    const int tpr = wide ? 256 : 64;
-    const int chunks = (int)((cols / V + tpr - 1) / tpr);  // per thread and row, 1..kLnChunks
-    if (wide) {
-        if (chunks <= 1)
-            SLAPO_LAUNCH_LNB_MODE(1, 256);
-        else if (chunks <= 2)
-            SLAPO_LAUNCH_LNB_MODE(2, 256);
-        else
-            SLAPO_LAUNCH_LNB_MODE(4, 256);
-    } else {
-        if (chunks <= 1)
-            SLAPO_LAUNCH_LNB_MODE(1, 64);
-        else
-            SLAPO_LAUNCH_LNB_MODE(2, 64);
-    }
+    if (tpr == 64)
+        SLAPO_LAUNCH_LNB_MODE(1, 64);
+    else if (tpr == 128)
+        SLAPO_LAUNCH_LNB_MODE(1, 128);
+    else if (tpr == 256)
+        SLAPO_LAUNCH_LNB_MODE(1, 256);
+    else if (chunks <= kLnbThreads)
+        SLAPO_LAUNCH_LNB_MODE(1, 512);
+    else
+        SLAPO_LAUNCH_LNB_MODE(2, 512);
 #undef SLAPO_LAUNCH_LNB_MODE
 #undef SLAPO_LAUNCH_LNB
     rc = check_launch();
     if (rc != SLAPO_OK || !want_sums) return rc;
-    if (3 * cols >= 6144) {
-        hipLaunchKernelGGL((ln_finish_kernel<T, 64, 4>), dim3((unsigned)((3 * cols + 63) / 64)),
-                           dim3(256), 0, st, partial, (T*)dgamma, (T*)dbeta, (T*)dbias, n_blocks,
-                           (int)cols);
-    } else {
-        hipLaunchKernelGGL((ln_finish_kernel<T, 16, 16>), dim3((unsigned)((3 * cols + 15) / 16)),
-                           dim3(256), 0, st, partial, (T*)dgamma, (T*)dbeta, (T*)dbias, n_blocks,
-                           (int)cols);
-    }
+    hipLaunchKernelGGL(ln_finish_kernel<T>, dim3((unsigned)((3 * cols + kLnFinCols - 1) / kLnFinCols)),
+                       dim3(256), 0, st, partial, (T*)dgamma, (T*)dbeta, (T*)dbias, n_blocks,
+                       (int)cols);
     return check_launch();
 }
 
@@ -1117,8 +1099,7 @@ extern "C" int slapo_amd_bias_dropout_residual_bwd(const void* grad, void* dx, v
 
 extern "C" size_t slapo_amd_ln_bwd_workspace_bytes(int64_t rows, int64_t cols) {
     if (rows <= 0 || cols <= 0) return 0;
-    const int rpb = ln_rows_per_block(rows, true);  // the most partial rows, whatever the type
-    const int64_t n_blocks = (rows + rpb - 1) / rpb;
+    const int64_t n_blocks = lnb_blocks(rows, cols, true);  // the most of any call
     return (size_t)n_blocks * 3 * (size_t)cols * sizeof(float);
 }
 

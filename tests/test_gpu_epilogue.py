@@ -160,6 +160,32 @@ def test_bias_dropout_residual_layer_norm(dtype, shape, p):
             assert_parity(got, want, dtype, name)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols", [(1, 512), (9, 520), (255, 1024), (257, 1032), (513, 2048),
+                                       (6, 2056), (258, 4096), (300, 8), (5300, 992)])
+def test_layer_norm_backward_at_the_edges_of_its_row_widths(dtype, rows, cols):
+    """Widths at which the threads per row change, rows that do not fill the blocks, and the size at
+    which the number of blocks changes; the parameter sums against float64."""
+    g = torch.Generator().manual_seed(rows * cols)
+    x, r, go = (torch.randn(rows, cols, generator=g).to(dtype).cuda() for _ in range(3))
+    b, w, lb = (torch.randn(cols, generator=g).to(dtype).cuda() for _ in range(3))
+    leaves = [t.requires_grad_() for t in (x, b, r, w, lb)]
+    torch.cuda.manual_seed(3)
+    y = op.bias_dropout_residual_layer_norm(*leaves, p=0.1)
+    grads = torch.autograd.grad(y, leaves, go)
+    torch.cuda.manual_seed(3)
+    keep = F.dropout(torch.ones_like(x), 0.1) != 0
+    x6, b6, r6, w6, lb6 = (t.detach().double().requires_grad_() for t in leaves)
+    z = torch.where(keep, (x6 + b6) / 0.9, torch.zeros((), dtype=torch.double, device="cuda")) + r6
+    z = z + (z.to(dtype).double() - z).detach()  # z is stored in the tensors' type
+    ref = torch.autograd.grad(F.layer_norm(z, (cols,), w6, lb6), (x6, b6, r6, w6, lb6), go.double())
+    # fp32: a sum of `rows` products in any order; 16 bits: one rounding of the result
+    bar = 2e-6 * max(1.0, rows ** 0.5 / 4) if dtype == torch.float32 else \
+        {torch.float16: 1e-3, torch.bfloat16: 8e-3}[dtype]
+    for got, want in zip(grads, ref):
+        assert ((got.double() - want).norm() / want.norm().clamp_min(1e-30)).item() <= bar
+
+
 def test_layer_norm_fusion_module_and_optional_operands():
     """The module against nn.LayerNorm on the same parameters; bias / residual left out; no
     gradient requested (nothing saved); argument errors."""
