@@ -375,13 +375,18 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const float* __restr
 // bias + dropout + residual + LayerNorm (the fusion pattern of tests/test_fusion.py:157-204:
 // layer_norm(dropout(x + bias) + residual)).
 //
-// A row is owned by TPR threads: one wavefront (TPR = 64) up to 64 * V * 2 columns, the
-// whole block (TPR = 256) above, so that every row value stays in registers between the two
-// passes of the statistics and is read from memory once.  z = dropout(x + bias) + residual is
+// A row is owned by TPR threads with NV 16-byte chunks each, so that every row value stays in
+// registers between the two passes of the statistics and is read from memory once.  One chunk per
+// thread (TPR 64 to 512) leaves the most wavefronts in flight and no guarded instructions for chunks
+// that a row does not have: against one wavefront up to 1024 columns and a block above, both with
+// up to four chunks, p 0.1: fp16 1537 x 768 5.7 -> 5.0 us, bf16 4096 x 1024 10.3 -> 9.2 (p 0: 7.9 ->
+// 6.6), 4096 x 2048 16.2 -> 15.0, fp16 2000 x 8000 30.5 -> 29.3.  Two chunks per thread at half the
+// width where many rows leave a quarter of the threads idle (bf16 8192 x 2560 39.9 us with one, 36.5
+// with two; 8192 x 768, p 0, 11.5 and 10.0).  z = dropout(x + bias) + residual is
 // rounded to T first and the statistics are taken from the rounded values, i.e. exactly what the
 // unfused modules compute from the stored sum; z is also what the backward reads.
 // ----------------------------------------------------------------------------------------
-constexpr int kLnChunks = 4;         // 16-byte chunks per thread and row (guarded against cols)
+constexpr int kLnMaxChunks = 1024;  // 16-byte chunks of a row
 // Sum over the 64 lanes, on every lane, without LDS traffic: butterflies inside the 16-lane
 // rows through DPP (quad permutes, row rotations), then the four row sums through v_readlane.
 template <int kCtrl>
@@ -404,43 +409,47 @@ __device__ __forceinline__ float wave_sum(float v) {
         float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
     return (r0 + r1) + (r2 + r3);
 }
-// Sum over the TPR threads of a row.  red: 4 floats of LDS that no other reduction in flight uses
-// (TPR == 256 only; every thread of the block has to call).
+// Sum over the TPR threads of a row.  red: a float of LDS per wavefront that no other reduction in
+// flight uses (TPR > 64 only; every thread of the block has to call).
 template <int TPR>
 __device__ __forceinline__ float row_sum(float v, float* red) {
     v = wave_sum(v);
-    if constexpr (TPR == 256) {
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    if constexpr (TPR > 64) {
+        const int w = threadIdx.x >> 6;
+        if ((threadIdx.x & 63) == 0) red[w] = v;
         __syncthreads();
-        v = (red[0] + red[1]) + (red[2] + red[3]);
+        const int first = w & ~(TPR / 64 - 1);
+        v = red[first] + red[first + 1];
+#pragma unroll
+        for (int i = 2; i < TPR / 64; i += 2) v += red[first + i] + red[first + i + 1];
     }
     return v;
 }
 
-template <typename T, int V, int TPR, int kDrop>
-__global__ __launch_bounds__(256) void bias_dropout_residual_ln_fwd_kernel(
+template <typename T, int V, int NV, int TPR, int kDrop>
+__global__ __launch_bounds__(TPR > 256 ? TPR : 256) void bias_dropout_residual_ln_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ bias, const T* __restrict__ residual,
     const T* __restrict__ gamma, const T* __restrict__ beta, T* __restrict__ z_out,
     T* __restrict__ y, float* __restrict__ mean_out, float* __restrict__ rstd_out, int64_t rows,
     int cols, float eps, DropoutState s) {
     if constexpr (kDrop != 0) resolve_device_state(s);
-    constexpr int kRows = 256 / TPR;  // rows per block
-    __shared__ float red[2][4];
+    constexpr int kRows = TPR > 256 ? 1 : 256 / TPR;  // rows per block
+    __shared__ float red[2][8];
     const int sub = threadIdx.x % TPR;
     const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / TPR;
     const bool row_ok = row < rows;  // uniform per wavefront
-    float zf[kLnChunks][V];
+    float zf[NV][V];
     float sum = 0.f;
     // odd wavefronts draw their dropout bits before they request their data, even ones after (see
     // bias_dropout_residual_fwd_kernel)
-    uint32_t bits_u[kLnChunks];
+    uint32_t bits_u[NV];
 #pragma unroll
-    for (int u = 0; u < kLnChunks; ++u) bits_u[u] = 0xFFFFFFFFu;
+    for (int u = 0; u < NV; ++u) bits_u[u] = 0xFFFFFFFFu;
     const bool draw_first = (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 1) != 0;
     if constexpr (kDrop != 0) {
         if (draw_first) {
 #pragma unroll
-            for (int u = 0; u < kLnChunks; ++u) {
+            for (int u = 0; u < NV; ++u) {
                 const int col0 = (sub + u * TPR) * V;
                 if (row_ok && col0 < cols)
                     bits_u[u] = keep_bits<V, kDrop>(s, (uint64_t)(row * cols + col0));
@@ -449,7 +458,7 @@ __global__ __launch_bounds__(256) void bias_dropout_residual_ln_fwd_kernel(
         }
     }
 #pragma unroll
-    for (int u = 0; u < kLnChunks; ++u) {
+    for (int u = 0; u < NV; ++u) {
         const int col0 = (sub + u * TPR) * V;
 #pragma unroll
         for (int i = 0; i < V; ++i) zf[u][i] = 0.f;
@@ -481,7 +490,7 @@ __global__ __launch_bounds__(256) void bias_dropout_residual_ln_fwd_kernel(
     const float mean = row_sum<TPR>(sum, red[0]) * inv_n;
     float sq = 0.f;
 #pragma unroll
-    for (int u = 0; u < kLnChunks; ++u) {
+    for (int u = 0; u < NV; ++u) {
         if ((sub + u * TPR) * V < cols) {
 #pragma unroll
             for (int i = 0; i < V; ++i) {
@@ -494,7 +503,7 @@ __global__ __launch_bounds__(256) void bias_dropout_residual_ln_fwd_kernel(
     const float rstd = 1.0f / __builtin_sqrtf(var + eps);
     if (!row_ok) return;
 #pragma unroll
-    for (int u = 0; u < kLnChunks; ++u) {
+    for (int u = 0; u < NV; ++u) {
         const int col0 = (sub + u * TPR) * V;
         if (col0 < cols) {
             const Chunk<T, V> g = load_chunk_cached<T, V>(gamma + col0);
@@ -917,11 +926,10 @@ int dropres_bwd_dispatch(const void* grad, void* dx, void* dbias, void* ws, int6
 }
 
 template <typename T>
-inline int ln_geometry(int64_t rows, int64_t cols, bool* wide) {
+inline int ln_geometry(int64_t rows, int64_t cols) {
     constexpr int V = Elem<T>::kPerVec;
     if (cols % V != 0) return SLAPO_ERR_ALIGN;
-    if (cols > 256 * V * kLnChunks) return SLAPO_ERR_SHAPE;
-    *wide = cols > 64 * V * 2;  // a wavefront per row up to two chunks per lane, a block above
+    if (cols > kLnMaxChunks * V) return SLAPO_ERR_SHAPE;
     if (rows > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
     return SLAPO_OK;
 }
@@ -932,26 +940,47 @@ int ln_fwd_dispatch(const void* x, const void* bias, const void* residual, const
                     int64_t cols, float eps, bool dropout, const DropoutState& s,
                     hipStream_t st) {
     constexpr int V = Elem<T>::kPerVec;
-    bool wide = false;
-    int rc = ln_geometry<T>(rows, cols, &wide);
+    int rc = ln_geometry<T>(rows, cols);
     if (rc != SLAPO_OK) return rc;
     for (const void* p : {x, bias, residual, gamma, beta, (const void*)z, (const void*)y})
         if (p && !aligned16(p)) return SLAPO_ERR_ALIGN;
     const int mode = !dropout ? 0 : (s.g_shift >= 0 && s.t_shift >= 0) ? 1 : 2;
-#define SLAPO_LAUNCH_LN(TPR, MODE)                                                              \
-    hipLaunchKernelGGL((bias_dropout_residual_ln_fwd_kernel<T, V, TPR, MODE>),                  \
-                       dim3((unsigned)((rows + (256 / TPR) - 1) / (256 / TPR))), dim3(256), 0,  \
-                       st, (const T*)x, (const T*)bias, (const T*)residual, (const T*)gamma,    \
-                       (const T*)beta, (T*)z, (T*)y, mean, rstd, rows, (int)cols, eps, s)
-    if (wide) {
-        if (mode == 0) SLAPO_LAUNCH_LN(256, 0);
-        if (mode == 1) SLAPO_LAUNCH_LN(256, 1);
-        if (mode == 2) SLAPO_LAUNCH_LN(256, 2);
+#define SLAPO_LAUNCH_LN(NV, TPR, MODE)                                                         \
+    hipLaunchKernelGGL((bias_dropout_residual_ln_fwd_kernel<T, V, NV, TPR, MODE>),            \
+                       dim3((unsigned)((rows + in_flight - 1) / in_flight)),                  \
+                       dim3(TPR > 256 ? TPR : 256), 0, st, (const T*)x, (const T*)bias,       \
+                       (const T*)residual, (const T*)gamma, (const T*)beta, (T*)z, (T*)y, mean, \
+                       rstd, rows, (int)cols, eps, s)
+#define SLAPO_LAUNCH_LN_MODE(NV, TPR)               \
+    do {                                            \
+        constexpr int in_flight = TPR > 256 ? 1 : 256 / TPR; \
+        if (mode == 0) SLAPO_LAUNCH_LN(NV, TPR, 0); \
+        if (mode == 1) SLAPO_LAUNCH_LN(NV, TPR, 1); \
+        if (mode == 2) SLAPO_LAUNCH_LN(NV, TPR, 2); \
+    } while (0)
+    const int chunks = (int)(cols / V);  // per row
+    int tpr = 64;
+    while (tpr < 512 && tpr < chunks) tpr *= 2;
+    // many rows that leave a quarter of their threads idle: two chunks per thread of half the width
+    if (rows >= 4096 && tpr > 64 && 4 * chunks <= 3 * tpr) {
+        if (tpr == 128)
+            SLAPO_LAUNCH_LN_MODE(2, 64);
+        else if (tpr == 256)
+            SLAPO_LAUNCH_LN_MODE(2, 128);
+        else
+            SLAPO_LAUNCH_LN_MODE(2, 256);
+    } else if (tpr == 64) {
+        SLAPO_LAUNCH_LN_MODE(1, 64);
+    } else if (tpr == 128) {
+        SLAPO_LAUNCH_LN_MODE(1, 128);
+    } else if (tpr == 256) {
+        SLAPO_LAUNCH_LN_MODE(1, 256);
+    } else if (chunks <= tpr) {
+        SLAPO_LAUNCH_LN_MODE(1, 512);
     } else {
-        if (mode == 0) SLAPO_LAUNCH_LN(64, 0);
-        if (mode == 1) SLAPO_LAUNCH_LN(64, 1);
-        if (mode == 2) SLAPO_LAUNCH_LN(64, 2);
+        SLAPO_LAUNCH_LN_MODE(2, 512);
     }
+#undef SLAPO_LAUNCH_LN_MODE
 #undef SLAPO_LAUNCH_LN
     return check_launch();
 }
@@ -962,8 +991,7 @@ int ln_bwd_dispatch(const void* dy, const void* z, const float* mean, const floa
                     void* dbias, void* ws, int64_t rows, int64_t cols, bool dropout,
                     const DropoutState& s, hipStream_t st) {
     constexpr int V = Elem<T>::kPerVec;
-    bool wide = false;
-    int rc = ln_geometry<T>(rows, cols, &wide);
+    int rc = ln_geometry<T>(rows, cols);
     if (rc != SLAPO_OK) return rc;
     for (const void* p : {dy, z, gamma, (const void*)dx, (const void*)dres})
         if (p && !aligned16(p)) return SLAPO_ERR_ALIGN;
