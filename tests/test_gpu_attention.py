@@ -683,6 +683,19 @@ def test_few_rows_dealt_to_many_workgroups(dtype, shape, sk, causal, window, p, 
     _check(q, k, v, do, mask, causal, window, dtype, p=p)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("b,sq,sk,valid", [
+    (1, 65, 131, 64),    # the second tile of keys is padding, one row in the last unit of 64
+    (3, 333, 333, 90),   # tiles of padding behind tiles with a valid key, seqlen_k % 4 != 0
+    (2, 64, 257, 257),   # nothing padded in the longest sequence, one key in the last word
+])
+def test_keep_bits_drawn_ahead_beside_a_padding_mask(b, sq, sk, valid, causal):
+    """Masks drawn before the forward: words of tiles that hold nothing but padding are not drawn."""
+    q, k, v, do, g = _inputs(b, sq, 2, 64, torch.float16, sk=sk)
+    mask, _ = _padding_mask(b, sk, torch.float16, g, valid)
+    _check(q, k, v, do, mask, causal, 0, torch.float16, p=0.1)
+
+
 # ---- seeded sweep over the whole call surface --------------------------------------------------
 @pytest.mark.parametrize("seed", range(40))
 def test_random_configurations_against_the_oracle(seed):
