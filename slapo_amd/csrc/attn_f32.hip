@@ -20,8 +20,8 @@
 // matrix pipe: 256 FLOP per cycle and CU (157 TFLOP/s nominal; a large fp32 library product reaches
 // 138 on this card).  A wavefront spends 32 DB x 16 matrix cycles per tile and product against about
 // 200 vector instructions, and needs few registers, so several wavefronts share a SIMD and hide each
-// other's vector work.  B4 S512 H16 D64 without a mask, forward: 56 us = 76 TFLOP/s (one thread per row on
-// plain FMAs: 686 us, 6.3 TFLOP/s).
+// other's vector work.  B4 S512 H16 D64 without a mask, forward: 51.5 us = 83 TFLOP/s (one thread per row
+// on plain FMAs: 686 us, 6.3 TFLOP/s); B2 S2048 H16 D128 696 us = 99 TFLOP/s.
 //
 // Reference semantics: slapo/op/attention.py:163-181 (attention_bmk) and its autograd.
 #include "attn_common.h"
@@ -34,6 +34,13 @@ constexpr int kWaves = 4;
 constexpr int kThreads = kWaves * 64;
 constexpr int kRows = kWaves * 16;  // rows owned by a workgroup
 constexpr int kTile = 32;           // streamed rows per LDS tile
+// Forward calls that give a CU two workgroups at most run kHalves = 2: eight wavefronts, two per 16
+// query rows, each with one half of a tile of 64 keys and a softmax state of its own, merged at the end
+// through LDS.  Four wavefronts per SIMD then hide the vector work of a launch that has no more rows
+// (B4 S512 H16 D64 56.6 -> 51.5 us, D80 83.7 -> 72.6, B1 S4096 H2 D64 causal 113 -> 102); with more
+// workgroups the other ones do that and the merge only costs (B16 S512 H16 D64 184 -> 191 us, B2 S2048
+// H16 D128 696 -> 750).
+constexpr int64_t kHalvesBlocks = 512;  // two for each of 256 CUs
 
 __device__ __forceinline__ f32x4_t mma(float a, float b, f32x4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -62,23 +69,23 @@ constexpr int kPitchOf = 16 * DB + 4;
 // about bias and dropout when it runs.
 constexpr int kGeneral = 4;
 
-// A tile of kTile rows of 16 DB floats on its way from global memory to LDS.  Rows past the end are
+// A tile of kTileRows rows of 16 DB floats on its way from global memory to LDS.  Rows past the end are
 // clamped, columns past d read as zero.
-template <int DB, bool kVec>
+template <int DB, bool kVec, int kTileRows = kTile, int kBlock = kThreads>
 struct Tile {
     static constexpr int kPitch = kPitchOf<DB>;
-    static constexpr int kElems = kTile * kPitch;
+    static constexpr int kElems = kTileRows * kPitch;
     static constexpr int kPerRow = 4 * DB;
-    static constexpr int kChunks = kTile * kPerRow;
-    static constexpr int kPer = (kChunks + kThreads - 1) / kThreads;
+    static constexpr int kChunks = kTileRows * kPerRow;
+    static constexpr int kPer = (kChunks + kBlock - 1) / kBlock;
     f32x4_t r[kPer];
 
     __device__ __forceinline__ void load(const float* base, int64_t stride, int row0, int n_rows,
                                          int d) {
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int c = threadIdx.x + u * kThreads;
-            if (kChunks % kThreads != 0 && c >= kChunks) continue;
+            const int c = threadIdx.x + u * kBlock;
+            if (kChunks % kBlock != 0 && c >= kChunks) continue;
             const float* row = base + (int64_t)min(row0 + c / kPerRow, n_rows - 1) * stride;
             const int col = 4 * (c % kPerRow);
             if constexpr (kVec) {
@@ -92,8 +99,8 @@ struct Tile {
     __device__ __forceinline__ void store(float* lds, int row0, int n_rows, int d) const {
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int c = threadIdx.x + u * kThreads;
-            if (kChunks % kThreads != 0 && c >= kChunks) continue;
+            const int c = threadIdx.x + u * kBlock;
+            if (kChunks % kBlock != 0 && c >= kChunks) continue;
             const int row = c / kPerRow, col = 4 * (c % kPerRow);
             f32x4_t v = r[u];
 #pragma unroll
@@ -227,21 +234,25 @@ __device__ __forceinline__ Visible queries_of_key(const AttnArgs& a, int j, int 
             (a.window > 0 ? min(j + a.window, a.sq) - 1 : a.sq - 1) - first};
 }
 
-template <int DB, int kMode>
-__global__ __launch_bounds__(kThreads, DB <= 4 ? 3 : 2) void attn_f32_fwd_kernel(
+template <int DB, int kMode, int kHalves>
+__global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void attn_f32_fwd_kernel(
     const AttnArgs a_in) {
+    constexpr int kFwdThreads = kHalves * kThreads, kFwdTile = kHalves * kTile;
     AttnArgs a = a_in;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
     if (dropout) resolve_device_state(a.rng);
     extern __shared__ __align__(16) float lds[];
-    constexpr int kElems = Tile<DB, kVec>::kElems;
+    typedef Tile<DB, kVec, kFwdTile, kFwdThreads> tile_t;
+    constexpr int kElems = tile_t::kElems;
     float* ks = lds;               // K[2][tile]
     float* vs = lds + 2 * kElems;  // V[2][tile]
     const Place at(a, a.sq, true);
     const int lane = threadIdx.x & 63, g = lane >> 4;
-    const int wq0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wq0 = at.row0 + 16 * (wave % kWaves);
+    const int half = wave / kWaves;  // of every tile's keys
     const int i = wq0 + (lane & 15);
     const float* qp = reinterpret_cast<const float*>(a.q) + at.b * a.qs[0] + at.h * a.qs[2];
     const float* kp = reinterpret_cast<const float*>(a.k) + at.b * a.ks[0] + at.h * a.ks[2];
@@ -249,32 +260,33 @@ __global__ __launch_bounds__(kThreads, DB <= 4 ? 3 : 2) void attn_f32_fwd_kernel
 
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
-    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk));
-    int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
+    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kFwdThreads, true>(a, at.b, at.h, lds) : a.sk));
+    int t_lo = j_lo / kFwdTile, t_hi = (j_hi + kFwdTile - 1) / kFwdTile;
     if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
-    Tile<DB, kVec> kt, vt;
+    tile_t kt, vt;
     f32x4_t qf[DB], o[DB];
-    kt.load(kp, a.ks[1], t_lo * kTile, a.sk, a.d);
-    vt.load(vp, a.vs[1], t_lo * kTile, a.sk, a.d);
+    kt.load(kp, a.ks[1], t_lo * kFwdTile, a.sk, a.d);
+    vt.load(vp, a.vs[1], t_lo * kFwdTile, a.sk, a.d);
     load_frags<kVec>(qf, qp, a.qs[1], i, a.sq, a.d, a.scale);
 #pragma unroll
     for (int x = 0; x < DB; ++x) o[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;  // l: this lane's share of the row sum
-    kt.store(ks, t_lo * kTile, a.sk, a.d);
-    vt.store(vs, t_lo * kTile, a.sk, a.d);
+    kt.store(ks, t_lo * kFwdTile, a.sk, a.d);
+    vt.store(vs, t_lo * kFwdTile, a.sk, a.d);
     __syncthreads();
 
     const int wq_last = min(wq0 + 15, a.sq - 1);
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
-        const float *kb = ks + slot * kElems, *vb = vs + slot * kElems;
+        const int part = half * kTile * tile_t::kPitch;
+        const float *kb = ks + slot * kElems + part, *vb = vs + slot * kElems + part;
         if (t + 1 < t_hi) {
-            kt.load(kp, a.ks[1], (t + 1) * kTile, a.sk, a.d);
-            vt.load(vp, a.vs[1], (t + 1) * kTile, a.sk, a.d);
+            kt.load(kp, a.ks[1], (t + 1) * kFwdTile, a.sk, a.d);
+            vt.load(vp, a.vs[1], (t + 1) * kFwdTile, a.sk, a.d);
         }
-        const int j0 = t * kTile;
-        const bool active = wq0 < a.sq && (!a.causal || j0 <= wq_last) &&
+        const int j0 = t * kFwdTile + half * kTile;
+        const bool active = wq0 < a.sq && j0 < a.sk && (!a.causal || j0 <= wq_last) &&
                             (a.window <= 0 || wq0 - (j0 + kTile - 1) < a.window);
         if (active) {  // uniform per wavefront
             f32x4_t s[2];
@@ -318,12 +330,35 @@ __global__ __launch_bounds__(kThreads, DB <= 4 ? 3 : 2) void attn_f32_fwd_kernel
             }
         }
         if (t + 1 < t_hi) {
-            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d);
-            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d);
+            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d);
+            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d);
         }
         __syncthreads();
     }
-    const float l_tot = column_sum(l);
+    float l_tot = column_sum(l);
+    if constexpr (kHalves == 2) {
+        // the second half's state joins the first's through LDS (every wavefront is past the loop's
+        // last barrier): lane by lane, the two hold the same rows and columns
+        float* state = lds + (wave % kWaves) * (4 * DB + 2) * 64 + lane;
+        if (half != 0) {
+#pragma unroll
+            for (int x = 0; x < DB; ++x)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) state[(4 * x + e) * 64] = o[x][e];
+            state[4 * DB * 64] = m, state[(4 * DB + 1) * 64] = l_tot;
+        }
+        __syncthreads();
+        if (half != 0) return;
+        const float m2 = state[4 * DB * 64], m_all = fmaxf(m, m2);
+        const float w1 = m == -INFINITY ? 0.f : expf(m - m_all);
+        const float w2 = m2 == -INFINITY ? 0.f : expf(m2 - m_all);
+        l_tot = l_tot * w1 + state[(4 * DB + 1) * 64] * w2;
+        m = m_all;
+#pragma unroll
+        for (int x = 0; x < DB; ++x)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[x][e] = o[x][e] * w1 + state[(4 * x + e) * 64] * w2;
+    }
     if (i >= a.sq) return;
     if (a.n_split > 1) {
         store_row<kVec>(o, 1.0f, a.part + (at.part_row0 + i) * a.d, a.d);
@@ -569,21 +604,25 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
 enum class Which { kFwd, kDq, kDkv };
 
 // DB = 16-wide blocks of the head dimension
-template <int DB, Which kWhich, int kMode>
+template <int DB, Which kWhich, int kMode, int kHalves = 1>
 int launch(const AttnArgs& a, hipStream_t st) {
     const int n_rows = kWhich == Which::kDkv ? a.sk : a.sq;
     const int64_t blocks =
         (int64_t)((n_rows + kRows - 1) / kRows) * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    const size_t smem = (4 * kTile * kPitchOf<DB> + (kWhich == Which::kDkv ? 6 * kTile : 0)) *
+    if constexpr (kWhich == Which::kFwd && kHalves == 1) {
+        if (blocks <= kHalvesBlocks) return launch<DB, kWhich, kMode, 2>(a, st);
+    }
+    const size_t smem = (4 * kHalves * kTile * kPitchOf<DB> +
+                         (kWhich == Which::kDkv ? 6 * kTile : 0)) *
                         sizeof(float);
-    auto kern = kWhich == Which::kFwd  ? attn_f32_fwd_kernel<DB, kMode>
+    auto kern = kWhich == Which::kFwd  ? attn_f32_fwd_kernel<DB, kMode, kHalves>
                 : kWhich == Which::kDq ? attn_f32_dq_kernel<DB, kMode>
                                        : attn_f32_dkv_kernel<DB, kMode>;
     static std::atomic<uint64_t> lds_ready{0};
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kHalves * kThreads), smem, st, a);
     return check_launch();
 }
 
