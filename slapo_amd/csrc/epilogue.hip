@@ -6,6 +6,8 @@
 //
 // Formulas follow slapo/op/fused_bias.py:18-34 (bias_gelu / bias_gelu_back) and :67-74
 // (bias_dropout); math is fp32 inside, storage in the tensor dtype.
+#include <type_traits>
+
 #include "common.h"
 
 using namespace slapo;
@@ -202,32 +204,36 @@ __global__ __launch_bounds__(256) void bias_dropout_residual_fwd_kernel(
 }
 
 // ----------------------------------------------------------------------------------------
-// Backward kernels: a block is 64 column-chunks x 4 row-lanes and walks kRowsPerBlock rows,
-// keeping per-thread fp32 column sums; the 4 row-lanes are combined through LDS and written
-// as one fp32 partial row per block.
+// Backward kernels: a block of 512 threads is kCols column-chunks (64, or 32 for matrices that
+// have no more) x 512 / kCols row-lanes and walks rows_per_block rows, keeping per-thread fp32 column
+// sums; the row-lanes are combined through LDS and written as one fp32 partial row per block.
 // ----------------------------------------------------------------------------------------
-constexpr int kRowsPerBlock = 64;  // at most; see colsum_rows_per_block
-constexpr int kRowLanes = 4;
-constexpr int kColLanes = 64;
+constexpr int kWalkThreads = 512;
 
-// Rows that one block walks: 64 where that still gives the device four blocks per CU or more,
-// else 32 or 16 (a block's rows run one after the other, so a narrow matrix in few blocks is
-// bound by latency: bf16 8192 x 1024 in 256 blocks of 64 rows took 15.7 us for 33.6 MB).  The
+// Rows that one block walks: 128 where that still gives the device two blocks per CU or more,
+// else 64 or 32 (a block's rows run one after the other, so a narrow matrix in few blocks is
+// bound by latency), 16 where even 32 leave CUs without a block.  With eight row-lanes (sixteen of 32
+// chunks) instead of four of 64, the rows in flight and the chain of a thread are the same, but half
+// the partial rows are left for the finishing kernel, and matrices of up to 32 chunks have no idle
+// lanes.  Bias-GeLU backward with its finish, before -> after: bf16 4096 x 1024 10.1 -> 9.6 us, fp16
+// 2000 x 8000 24.0 -> 19.9, 20000 x 256 16.4 -> 12.6, 32000 x 128 20.8 -> 15.5; bias-dropout backward
+// 20.4 -> 17.7, 15.2 -> 10.8, 19.0 -> 13.2 at the last three.  The
 // choice depends on the shape alone, so that the workspace size and the finishing kernel agree
 // with the launch.
 inline int colsum_rows_per_block(int64_t rows, int64_t cols) {
-    const int64_t col_blocks = (cols + 8 * kColLanes - 1) / (8 * kColLanes);
-    int rpb = kRowsPerBlock;
-    while (rpb > 16 && col_blocks * ((rows + rpb - 1) / rpb) < 1024) rpb /= 2;
+    const int64_t col_blocks = (cols + 511) / 512;
+    int rpb = 128;
+    while (rpb > 16 && col_blocks * ((rows + rpb - 1) / rpb) < (rpb > 32 ? 512 : 256)) rpb /= 2;
     return rpb;
 }
 
-template <typename T, int V, typename F>
+template <typename T, int V, int kCols, typename F>
 __device__ __forceinline__ void colsum_walk(int64_t rows, int64_t cols, float* __restrict__ partial,
                                             bool want_sum, int rows_per_block, F&& body) {
-    const int cx = threadIdx.x % kColLanes;
-    const int ry = threadIdx.x / kColLanes;
-    const int64_t chunk_col = (int64_t)blockIdx.x * kColLanes + cx;
+    constexpr int kLanes = kWalkThreads / kCols;  // rows at a time
+    const int cx = threadIdx.x % kCols;
+    const int ry = threadIdx.x / kCols;
+    const int64_t chunk_col = (int64_t)blockIdx.x * kCols + cx;
     const int64_t col0 = chunk_col * V;
     const bool active = col0 < cols;
     float acc[V];
@@ -239,33 +245,32 @@ __device__ __forceinline__ void colsum_walk(int64_t rows, int64_t cols, float* _
             // a whole block of rows: no test between the iterations, so that the loads of an
             // unrolled group of four rows are requested together
 #pragma unroll 4
-            for (int it = 0; it < rows_per_block / kRowLanes; ++it)
-                body(r_begin + ry + (int64_t)it * kRowLanes, col0, acc);
+            for (int it = 0; it < rows_per_block / kLanes; ++it)
+                body(r_begin + ry + (int64_t)it * kLanes, col0, acc);
         } else {
-            for (int it = 0; it < rows_per_block / kRowLanes; ++it) {
-                const int64_t r = r_begin + ry + (int64_t)it * kRowLanes;
+            for (int it = 0; it < rows_per_block / kLanes; ++it) {
+                const int64_t r = r_begin + ry + (int64_t)it * kLanes;
                 if (r < rows) body(r, col0, acc);
             }
         }
     }
     if (!want_sum) return;
-    __shared__ float red[kRowLanes][kColLanes][V + 1];
+    __shared__ float red[V][kLanes][kCols];
 #pragma unroll
-    for (int i = 0; i < V; ++i) red[ry][cx][i] = acc[i];
+    for (int i = 0; i < V; ++i) red[i][ry][cx] = acc[i];
     __syncthreads();
-    if (ry == 0 && active) {
+    // thread (cx, i): value i of the chunk, all row-lanes
+    for (int i = ry; i < V; i += kLanes) {
+        if (!active) break;
+        float t = red[i][0][cx];
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
-            float t = red[0][cx][i];
-#pragma unroll
-            for (int k = 1; k < kRowLanes; ++k) t += red[k][cx][i];
-            partial[(int64_t)blockIdx.y * cols + col0 + i] = t;
-        }
+        for (int k = 1; k < kLanes; ++k) t += red[i][k][cx];
+        partial[(int64_t)blockIdx.y * cols + col0 + i] = t;
     }
 }
 
-template <typename T, int V>
-__global__ __launch_bounds__(256) void bias_gelu_bwd_kernel(const T* __restrict__ grad,
+template <typename T, int V, int kCols>
+__global__ __launch_bounds__(kWalkThreads) void bias_gelu_bwd_kernel(const T* __restrict__ grad,
                                                             const T* __restrict__ y,
                                                             const T* __restrict__ bias,
                                                             T* __restrict__ dx,
@@ -274,10 +279,10 @@ __global__ __launch_bounds__(256) void bias_gelu_bwd_kernel(const T* __restrict_
                                                             int want_sum, int rows_per_block) {
     Chunk<T, V> b;
     {
-        const int64_t col0 = ((int64_t)blockIdx.x * kColLanes + threadIdx.x % kColLanes) * V;
+        const int64_t col0 = ((int64_t)blockIdx.x * kCols + threadIdx.x % kCols) * V;
         if (col0 < cols) b = load_chunk_cached<T, V>(bias + col0);
     }
-    colsum_walk<T, V>(rows, cols, partial, want_sum != 0, rows_per_block,
+    colsum_walk<T, V, kCols>(rows, cols, partial, want_sum != 0, rows_per_block,
                       [&](int64_t r, int64_t col0, float* acc) {
                           const int64_t off = r * cols + col0;
                           const Chunk<T, V> g = load_chunk<T, V>(grad + off);
@@ -295,8 +300,8 @@ __global__ __launch_bounds__(256) void bias_gelu_bwd_kernel(const T* __restrict_
                       });
 }
 
-template <typename T, int V, int kDrop>
-__global__ __launch_bounds__(256) void bias_dropout_bwd_kernel(const T* __restrict__ grad,
+template <typename T, int V, int kDrop, int kCols>
+__global__ __launch_bounds__(kWalkThreads) void bias_dropout_bwd_kernel(const T* __restrict__ grad,
                                                                T* __restrict__ dx,
                                                                float* __restrict__ partial,
                                                                int64_t rows, int64_t cols,
@@ -304,7 +309,7 @@ __global__ __launch_bounds__(256) void bias_dropout_bwd_kernel(const T* __restri
                                                                int rows_per_block,
                                                                DropoutState s) {
     if constexpr (kDrop != 0) resolve_device_state(s);
-    colsum_walk<T, V>(rows, cols, partial, want_sum != 0, rows_per_block,
+    colsum_walk<T, V, kCols>(rows, cols, partial, want_sum != 0, rows_per_block,
                       [&](int64_t r, int64_t col0, float* acc) {
                           const int64_t off = r * cols + col0;
                           const Chunk<T, V> g = load_chunk<T, V>(grad + off);
@@ -839,14 +844,21 @@ int dropres_fwd_launch(const void* x, const void* bias, const void* residual, vo
     return check_launch();
 }
 
-inline bool bwd_grid(int64_t rows, int64_t cols, int v, dim3* grid) {
+// Calls launch(grid, rows per block, kCols) for a column-sum walk over chunks of v columns.
+template <typename Launch>
+inline int walk_launch(int64_t rows, int64_t cols, int v, Launch&& launch) {
     const int64_t chunk_cols = (cols + v - 1) / v;
-    const int64_t gx = (chunk_cols + kColLanes - 1) / kColLanes;
+    const int width = chunk_cols <= 32 ? 32 : 64;
+    const int64_t gx = (chunk_cols + width - 1) / width;
     const int rpb = colsum_rows_per_block(rows, cols);
     const int64_t gy = (rows + rpb - 1) / rpb;
-    if (gx > 0x7FFFFFFF || gy > 65535) return false;
-    *grid = dim3((unsigned)gx, (unsigned)gy);
-    return true;
+    if (gx > 0x7FFFFFFF || gy > 65535) return SLAPO_ERR_SHAPE;
+    const dim3 grid((unsigned)gx, (unsigned)gy);
+    if (width == 32)
+        launch(grid, rpb, std::integral_constant<int, 32>{});
+    else
+        launch(grid, rpb, std::integral_constant<int, 64>{});
+    return check_launch();
 }
 
 template <typename T>
@@ -862,21 +874,18 @@ int finish_colsum(const float* partial, void* dbias, int64_t rows, int64_t cols,
 template <typename T>
 int gelu_bwd_dispatch(const void* grad, const void* y, const void* bias, void* dx, void* dbias,
                       void* ws, int64_t rows, int64_t cols, hipStream_t st) {
-    dim3 grid;
     const int want = dbias ? 1 : 0;
-    if (vector_ok<T>(cols, {grad, y, bias, dx})) {
-        constexpr int V = Elem<T>::kPerVec;
-        if (!bwd_grid(rows, cols, V, &grid)) return SLAPO_ERR_SHAPE;
-        hipLaunchKernelGGL((bias_gelu_bwd_kernel<T, V>), grid, dim3(256), 0, st, (const T*)grad,
-                           (const T*)y, (const T*)bias, (T*)dx, (float*)ws, rows, cols, want,
-                           colsum_rows_per_block(rows, cols));
-    } else {
-        if (!bwd_grid(rows, cols, 1, &grid)) return SLAPO_ERR_SHAPE;
-        hipLaunchKernelGGL((bias_gelu_bwd_kernel<T, 1>), grid, dim3(256), 0, st, (const T*)grad,
-                           (const T*)y, (const T*)bias, (T*)dx, (float*)ws, rows, cols, want,
-                           colsum_rows_per_block(rows, cols));
-    }
-    int rc = check_launch();
+    auto run = [&](auto v_tag) {
+        constexpr int V = decltype(v_tag)::value;
+        return walk_launch(rows, cols, V, [&](dim3 grid, int rpb, auto cols_tag) {
+            hipLaunchKernelGGL((bias_gelu_bwd_kernel<T, V, decltype(cols_tag)::value>), grid,
+                               dim3(kWalkThreads), 0, st, (const T*)grad, (const T*)y,
+                               (const T*)bias, (T*)dx, (float*)ws, rows, cols, want, rpb);
+        });
+    };
+    const int rc = vector_ok<T>(cols, {grad, y, bias, dx})
+                       ? run(std::integral_constant<int, Elem<T>::kPerVec>{})
+                       : run(std::integral_constant<int, 1>{});
     if (rc != SLAPO_OK || !dbias) return rc;
     return finish_colsum<T>((const float*)ws, dbias, rows, cols, st);
 }
@@ -884,21 +893,20 @@ int gelu_bwd_dispatch(const void* grad, const void* y, const void* bias, void* d
 template <typename T, int V>
 int dropres_bwd_launch(const void* grad, void* dx, void* ws, int64_t rows, int64_t cols,
                        bool dropout, int want, const DropoutState& s, hipStream_t st) {
-    dim3 grid;
-    if (!bwd_grid(rows, cols, V, &grid)) return SLAPO_ERR_SHAPE;
     const int write_dx = dx ? 1 : 0;
-#define SLAPO_LAUNCH_DB(MODE)                                                                  \
-    hipLaunchKernelGGL((bias_dropout_bwd_kernel<T, V, MODE>), grid, dim3(256), 0, st,          \
-                       (const T*)grad, (T*)dx, (float*)ws, rows, cols, want, write_dx,            \
-                       colsum_rows_per_block(rows, cols), s)
     const int mode = !dropout ? 0 : (V % 4 == 0 && s.g_shift >= 0 && s.t_shift >= 0) ? 1 : 2;
-    if (mode == 0) SLAPO_LAUNCH_DB(0);
-    if constexpr (V % 4 == 0) {
-        if (mode == 1) SLAPO_LAUNCH_DB(1);
-    }
-    if (mode == 2) SLAPO_LAUNCH_DB(2);
+    return walk_launch(rows, cols, V, [&](dim3 grid, int rpb, auto cols_tag) {
+#define SLAPO_LAUNCH_DB(MODE)                                                                     \
+    hipLaunchKernelGGL((bias_dropout_bwd_kernel<T, V, MODE, decltype(cols_tag)::value>), grid,    \
+                       dim3(kWalkThreads), 0, st, (const T*)grad, (T*)dx, (float*)ws, rows, cols, \
+                       want, write_dx, rpb, s)
+        if (mode == 0) SLAPO_LAUNCH_DB(0);
+        if constexpr (V % 4 == 0) {
+            if (mode == 1) SLAPO_LAUNCH_DB(1);
+        }
+        if (mode == 2) SLAPO_LAUNCH_DB(2);
 #undef SLAPO_LAUNCH_DB
-    return check_launch();
+    });
 }
 
 template <typename T>

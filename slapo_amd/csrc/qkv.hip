@@ -4,7 +4,7 @@
 // round.  torch takes three strided copies forward and, backward, three zero-filled packed tensors
 // and their sum.  Bound by memory: 2 x the packed bytes.  A thread owns V consecutive elements of
 // each of q, k, v = 3 V consecutive packed elements: 16-byte accesses on both sides.
-// fp16 tokens 8192, hidden 1024 (100 MB): @QKV@.
+// fp16 tokens 8192, hidden 1024 (100 MB): 16.1 us, 6.2 TB/s; forward + backward 122 -> 54 us.
 #include "common.h"
 
 using namespace slapo;

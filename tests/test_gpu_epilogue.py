@@ -161,6 +161,31 @@ def test_bias_dropout_residual_layer_norm(dtype, shape, p):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,cols", [(1, 8), (17, 256), (4100, 256), (33, 264), (129, 512),
+                                       (8200, 520), (31, 4104), (77, 333)])
+def test_bias_gradients_at_the_edges_of_the_column_walk(dtype, rows, cols):
+    """Rows that do not fill a block, both widths of a block, one chunk more, scalar chunks."""
+    g = torch.Generator().manual_seed(rows + cols)
+    x, go = (torch.randn(rows, cols, generator=g).to(dtype).cuda() for _ in range(2))
+    b = torch.randn(cols, generator=g).to(dtype).cuda().requires_grad_()
+    x.requires_grad_()
+    torch.cuda.manual_seed(3)
+    out = op.bias_dropout(x, b, 0.1, True)
+    dx, db = torch.autograd.grad(out, (x, b), go)
+    torch.cuda.manual_seed(3)
+    want = torch.where(F.dropout(torch.ones_like(go), 0.1) != 0, go.double() / 0.9, 0.0)
+    dy, dyb = torch.autograd.grad(op.bias_gelu(x, b), (x, b), go)
+    x6, b6 = x.detach().double().requires_grad_(), b.detach().double().requires_grad_()
+    ref = torch.autograd.grad(F.gelu(x6 + b6, approximate="tanh"), (x6, b6), go.double())
+    # fp32: sums of `rows` terms in any order, exp2 and reciprocal of the GeLU at 1 ulp each;
+    # 16 bits: one rounding of the result
+    bar = 4e-6 * max(1.0, rows ** 0.5 / 4) if dtype == torch.float32 else \
+        {torch.float16: 1e-3, torch.bfloat16: 8e-3}[dtype]
+    for got, r in ((dx, want), (db, want.sum(0)), (dy, ref[0]), (dyb, ref[1])):
+        assert ((got.double() - r).norm() / r.norm().clamp_min(1e-30)).item() <= bar
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,cols", [(1, 512), (9, 520), (255, 1024), (257, 1032), (513, 2048),
                                        (6, 2056), (258, 4096), (300, 8), (5300, 992)])
 def test_layer_norm_backward_at_the_edges_of_its_row_widths(dtype, rows, cols):
