@@ -156,7 +156,7 @@ int slapo_amd_bias_dropout_residual_ln_fwd(const void* x, const void* bias, cons
                                            void* stream);
 
 /* Bytes of fp32 workspace the backward below needs when any of dgamma / dbeta / dbias is asked
- * for: one partial row triple per 16 rows. */
+ * for: one partial row triple per block of its launch, 512 blocks at most. */
 size_t slapo_amd_ln_bwd_workspace_bytes(int64_t rows, int64_t cols);
 
 /* Backward of slapo_amd_bias_dropout_residual_ln_fwd from grad_y and the saved z, mean, rstd:

@@ -1062,7 +1062,8 @@ inline bool dims_ok(int64_t rows, int64_t cols) {
 
 extern "C" size_t slapo_amd_colsum_workspace_bytes(int64_t rows, int64_t cols) {
     if (rows <= 0 || cols <= 0) return 0;
-    const int rpb = colsum_rows_per_block(rows, cols);
+    // never less than a partial row per 64 rows, the size that callers of this ABI know
+    const int most = colsum_rows_per_block(rows, cols), rpb = most < 64 ? most : 64;
     const int64_t n_partials = (rows + rpb - 1) / rpb;
     return (size_t)n_partials * (size_t)cols * sizeof(float);
 }
