@@ -164,6 +164,15 @@ std::shared_ptr<T> make_node(bool wanted, const Inputs&... inputs) {
 
 // ---- attention ----------------------------------------------------------------------------------
 
+// wanted: batch, heads, seqlen_q, seqlen_k
+void check_mask(const Tensor& mask, const std::array<int64_t, 4>& wanted) {
+    if (!mask.defined()) return;
+    TORCH_CHECK_VALUE(mask.dim() == 4, "attention_mask must be 4-D ([B,1,1,Sk] or [B,H,Sq,Sk])");
+    for (int i = 0; i < 4; ++i)
+        TORCH_CHECK(mask.size(i) == wanted[i] || mask.size(i) == 1, "attention_mask of shape ",
+                    mask.sizes(), " does not broadcast to ", at::IntArrayRef(wanted));
+}
+
 struct AttnProblem {
     slapo_attn_params prm = {};
     Tensor bias;  // of type bias_type, addressed with prm.bias_strides (0 on broadcast dims)
@@ -203,18 +212,12 @@ struct AttnProblem {
     // own: then it is read once per direction, in place.
     void set_bias(const Tensor& mask, bool infer) {
         if (!mask.defined()) return;
-        TORCH_CHECK_VALUE(mask.dim() == 4,
-                          "attention_mask must be 4-D ([B,1,1,Sk] or [B,H,Sq,Sk])");
+        check_mask(mask, {b(), h(), sq(), sk()});
         const at::ScalarType mt = mask.scalar_type();
         const bool known = mt == at::kFloat || mt == at::kHalf || mt == at::kBFloat16;
         const bool per_key = mask.size(2) == 1;
         bias = known && (infer || !per_key || dtype == at::kFloat) ? mask : cast(mask, at::kFloat);
         bias_type = dtype_code(bias.scalar_type());
-        const int64_t wanted[4] = {b(), h(), sq(), sk()};
-        for (int i = 0; i < 4; ++i)
-            TORCH_CHECK(bias.size(i) == wanted[i] || bias.size(i) == 1, "attention_mask of shape ",
-                        mask.sizes(), " does not broadcast to [", b(), ", ", h(), ", ", sq(), ", ",
-                        sk(), "]");
         // (the kernels address a row's values with 32-bit offsets)
         if (bias.size(3) > 1 && bias.stride(3) * sk() >= int64_t(1) << 30) bias = bias.contiguous();
         address_bias();
@@ -262,6 +265,11 @@ void check_operands(const Tensor& q, const Tensor& k, const Tensor& v) {
     TORCH_CHECK_VALUE(q.scalar_type() == k.scalar_type() && q.scalar_type() == v.scalar_type(),
                       "q, k, v must share a dtype");
     require_device({&q, &k, &v});
+}
+
+void check_packed(const Tensor& qkv, int64_t head_dim) {
+    TORCH_CHECK_VALUE(qkv.dim() == 3 && head_dim > 0 && qkv.size(2) % (3 * head_dim) == 0,
+                      "qkv must be [batch, seqlen, heads * 3 * head_dim]");
 }
 
 struct AttnResult {
@@ -474,8 +482,7 @@ Tensor attention_packed(const Tensor& qkv, int64_t head_dim, const Tensor& mask,
                         int64_t save_mask_max) {
     require_device({&qkv, &mask});
     refuse_tangents({&qkv});
-    TORCH_CHECK_VALUE(qkv.dim() == 3 && head_dim > 0 && qkv.size(2) % (3 * head_dim) == 0,
-                      "qkv must be [batch, seqlen, heads * 3 * head_dim]");
+    check_packed(qkv, head_dim);
     const bool need = torch::autograd::compute_requires_grad(qkv);
     auto node = make_node<AttnBackward>(need, qkv);
     AttnProblem a;
@@ -1067,13 +1074,29 @@ PyObject* py_cross_entropy(PyObject*, PyObject* const* a, Py_ssize_t n) {
     END_HANDLE_TH_ERRORS
 }
 
-// attention_scores(q, k, v): checks the operands, returns the number of scores B * H * Sq * Sk
+// attention_scores(q, k, v, mask): checks the operands -- before anything is drawn for them -- and
+// returns the number of scores B * H * Sq * Sk
 PyObject* py_attention_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
-    want(n, 3, "attention_scores");
+    want(n, 4, "attention_scores");
     const Tensor &q = tensor_arg(a[0], "q"), &k = tensor_arg(a[1], "k"), &v = tensor_arg(a[2], "v");
     check_operands(q, k, v);
+    check_mask(optional_tensor_arg(a[3], "attention_mask"),
+               {q.size(0), q.size(2), q.size(1), k.size(1)});
     return PyLong_FromLongLong(q.size(0) * q.size(1) * q.size(2) * k.size(1));
+    END_HANDLE_TH_ERRORS
+}
+
+// packed_scores(qkv, head_dim, mask): the same for the packed form
+PyObject* py_packed_scores(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    want(n, 3, "packed_scores");
+    const Tensor& qkv = tensor_arg(a[0], "qkv");
+    const int64_t head_dim = int_arg(a[1]);
+    check_packed(qkv, head_dim);
+    const int64_t b = qkv.size(0), s = qkv.size(1), h = qkv.size(2) / (3 * head_dim);
+    check_mask(optional_tensor_arg(a[2], "attention_mask"), {b, h, s, s});
+    return PyLong_FromLongLong(b * h * s * s);
     END_HANDLE_TH_ERRORS
 }
 
@@ -1155,6 +1178,7 @@ PyMethodDef methods[] = {
     SLAPO_METHOD("attention", py_attention),
     SLAPO_METHOD("attention_packed", py_attention_packed),
     SLAPO_METHOD("attention_scores", py_attention_scores),
+    SLAPO_METHOD("packed_scores", py_packed_scores),
     SLAPO_METHOD("qkv_plain", py_qkv_plain),
     SLAPO_METHOD("qkv_split", py_qkv_split),
     SLAPO_METHOD("cross_entropy", py_cross_entropy),

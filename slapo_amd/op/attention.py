@@ -80,7 +80,7 @@ def hip_attention(q, k, v, attention_mask=None, causal=False, p=0.0, scale=None,
     native = host()
     seed, offset, state = 0, 0, None
     if p != 0.0:
-        seed, offset, state = _draw(p, native.attention_scores(q, k, v), q.device)
+        seed, offset, state = _draw(p, native.attention_scores(q, k, v, attention_mask), q.device)
     _note_bias_gradient(attention_mask)
     return native.attention(q, k, v, attention_mask, causal, window or 0, scale, p, seed, offset,
                             state, SAVE_DROPOUT_MASK, SAVE_DROPOUT_MASK_MAX_BYTES)
@@ -91,8 +91,8 @@ def _packed_attention(qkv, head_dim, attention_mask, causal, p, scale, window):
     [B, S, heads * head_dim].  The backward writes the gradient of `qkv` as one tensor."""
     seed, offset, state = 0, 0, None
     if p != 0.0:
-        b, s, width = qkv.shape
-        seed, offset, state = _draw(p, b * (width // (3 * head_dim)) * s * s, qkv.device)
+        scores = host().packed_scores(qkv, head_dim, attention_mask)
+        seed, offset, state = _draw(p, scores, qkv.device)
     _note_bias_gradient(attention_mask)
     return host().attention_packed(qkv, head_dim, attention_mask, causal, window or 0, scale, p,
                                    seed, offset, state, SAVE_DROPOUT_MASK,

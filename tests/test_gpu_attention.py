@@ -696,6 +696,20 @@ def test_keep_bits_drawn_ahead_beside_a_padding_mask(b, sq, sk, valid, causal):
     _check(q, k, v, do, mask, causal, 0, torch.float16, p=0.1)
 
 
+def test_a_refused_mask_draws_nothing():
+    q = torch.randn(2, 16, 2, 64, dtype=torch.float16, device="cuda")
+    m = op.FlashAttention(128, 2, 0.1, 0.1, "hip_cdna4", fused_qkv=True).half().cuda()
+    x = torch.randn(2, 16, 128, dtype=torch.float16, device="cuda")
+    before = torch.cuda.get_rng_state()
+    for shape, error in (((2, 1, 1, 15), RuntimeError), ((2, 16), ValueError)):
+        mask = torch.zeros(shape, dtype=torch.float16, device="cuda")
+        with pytest.raises(error):
+            op.hip_attention(q, q, q, mask, p=0.1)
+        with pytest.raises(error):
+            m(x, mask)
+    assert torch.equal(before, torch.cuda.get_rng_state())
+
+
 # ---- seeded sweep over the whole call surface --------------------------------------------------
 @pytest.mark.parametrize("seed", range(40))
 def test_random_configurations_against_the_oracle(seed):
