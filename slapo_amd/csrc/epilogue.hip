@@ -414,6 +414,14 @@ __device__ __forceinline__ float wave_sum(float v) {
         float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
     return (r0 + r1) + (r2 + r3);
 }
+// The same over each half of the wavefront.
+__device__ __forceinline__ float half_sum(float v) {
+    v += dpp_move<0xB1>(v);   // quad_perm [1,0,3,2]
+    v += dpp_move<0x4E>(v);   // quad_perm [2,3,0,1]
+    v += dpp_move<0x124>(v);  // row_ror 4
+    v += dpp_move<0x128>(v);  // row_ror 8
+    return v + __shfl_xor(v, 16, 64);
+}
 // Sum over the TPR threads of a row.  red: a float of LDS per wavefront that no other reduction in
 // flight uses (TPR > 64 only; every thread of the block has to call).
 template <int TPR>
@@ -545,6 +553,8 @@ __global__ __launch_bounds__(TPR > 256 ? TPR : 256) void bias_dropout_residual_l
 // rows had one or two wavefronts per SIMD.  Both kernels together, before -> after (p 0.1): fp16
 // 1537 x 768 18.0 -> 9.4 us, bf16 4096 x 1024 34.4 -> 13.2, 4096 x 2048 31.3 -> 22.7, 8192 x 4096
 // 81.5 -> 66.8 (4.0 TB/s), fp16 2000 x 8000 115 -> 53.
+// Rows of 32 chunks at most take half a wavefront: fp16 20000 x 256 21.6 us with a whole one, 16.4 with
+// half; 32000 x 128 27.4 and 18.0.
 constexpr int kLnbThreads = 512;
 // Blocks of a launch: one for each of the 256 CUs, which walk the rows that fall to them, so that the
 // partial rows -- 24 bytes per block and column, written and read again -- stay few (bf16 4096 x 1024,
@@ -562,6 +572,10 @@ typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 // Sums of a and b over the TPR threads of a row; red: LDS of this iteration, [wavefront][2].
 template <int TPR>
 __device__ __forceinline__ void row_sums(float& a, float& b, float (*red)[2]) {
+    if constexpr (TPR == 32) {
+        a = half_sum(a), b = half_sum(b);
+        return;
+    }
     a = wave_sum(a), b = wave_sum(b);
     if constexpr (TPR > 64) {
         const int w = threadIdx.x >> 6;
@@ -609,7 +623,7 @@ __global__ __launch_bounds__(kLnbThreads, NV == 1 ? 4 : 2) void bias_dropout_res
     float m[kAhead + 1], rs[kAhead + 1];
     auto request = [&](int it, int slot) __attribute__((always_inline)) {
         const int64_t row = row0 + (int64_t)it * kRows;
-        if (it < n_iters && row < rows) {  // uniform per wavefront
+        if (it < n_iters && row < rows) {  // uniform per wavefront (TPR 64 and more)
             m[slot] = mean[row];
             rs[slot] = rstd[row];
 #pragma unroll
@@ -1005,7 +1019,7 @@ int ln_bwd_dispatch(const void* dy, const void* z, const float* mean, const floa
         if (p && !aligned16(p)) return SLAPO_ERR_ALIGN;
     const bool want_sums = dgamma || dbeta || dbias;
     const int chunks = (int)(cols / V);  // per row
-    const int tpr = chunks <= 64 ? 64 : chunks <= 128 ? 128 : chunks <= 256 ? 256 : kLnbThreads;
+    const int tpr = chunks <= 32 ? 32 : chunks <= 64 ? 64 : chunks <= 128 ? 128 : chunks <= 256 ? 256 : kLnbThreads;
     const int in_flight = kLnbThreads / tpr;
     const int64_t most_blocks = lnb_blocks(rows, cols, dropout);
     const int64_t per_block = (rows + most_blocks - 1) / most_blocks;
@@ -1026,7 +1040,9 @@ int ln_bwd_dispatch(const void* dy, const void* z, const float* mean, const floa
         if (mode == 1) SLAPO_LAUNCH_LNB(NV, TPR, 1); \
         if (mode == 2) SLAPO_LAUNCH_LNB(NV, TPR, 2); \
     } while (0)
-    if (tpr == 64)
+    if (tpr == 32)
+        SLAPO_LAUNCH_LNB_MODE(1, 32);
+    else if (tpr == 64)
         SLAPO_LAUNCH_LNB_MODE(1, 64);
     else if (tpr == 128)
         SLAPO_LAUNCH_LNB_MODE(1, 128);

@@ -187,7 +187,8 @@ def test_bias_gradients_at_the_edges_of_the_column_walk(dtype, rows, cols):
 
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("rows,cols", [(1, 512), (9, 520), (255, 1024), (257, 1032), (513, 2048),
-                                       (6, 2056), (258, 4096), (300, 8), (5300, 992)])
+                                       (6, 2056), (258, 4096), (300, 8), (5300, 992),
+                                       (47, 256), (5001, 128), (33, 264)])
 def test_layer_norm_backward_at_the_edges_of_its_row_widths(dtype, rows, cols):
     """Widths at which the threads per row change, rows that do not fill the blocks, and the size at
     which the number of blocks changes; the parameter sums against float64."""
