@@ -31,6 +31,7 @@ from torch import nn
 from .._lib import host
 from ..random import draw_philox  # noqa: F401  (kept importable from here for direct launches)
 from ..random import draw_philox_state
+from ._tracing import record, tracing_state
 from .fused_bias import bias_dropout
 
 logger = logging.getLogger("slapo_amd")
@@ -77,6 +78,8 @@ def _note_bias_gradient(attention_mask):
 def hip_attention(q, k, v, attention_mask=None, causal=False, p=0.0, scale=None, window=0):
     """q, k, v: [B, S, H, D] (head_dim contiguous; outer dims may be strided views).
     attention_mask: additive, 4-D, broadcastable to [B, H, Sq, Sk].  Returns [B, Sq, H, D]."""
+    if tracing_state() is not None:
+        return record(hip_attention, q, k, v, attention_mask, causal, p, scale, window)
     native = host()
     seed, offset, state = 0, 0, None
     if p != 0.0:
@@ -220,9 +223,10 @@ class FlashAttention(nn.Module):
         """The packed form stands in for splitting the projection and calling `attn_op` only when
         nothing could tell the difference: the child is the plain op (a schedule's `.fork_rng`
         wraps its `forward`, primitives/tensor_parallel.py:185-191; `.replace` swaps it) without
-        hooks, and the input a real device tensor."""
+        hooks, the input a real device tensor and no `torch.jit.trace` watching."""
         core = self.attn_op
-        return (type(packed) is torch.Tensor and packed.is_cuda and packed.ndim == 3
+        return (tracing_state() is None
+                and type(packed) is torch.Tensor and packed.is_cuda and packed.ndim == 3
                 and type(core) is FlashAttentionOp and core.attn_fn is hip_attention
                 and "forward" not in core.__dict__ and not _has_hooks(core))
 

@@ -15,6 +15,7 @@ import torch
 from torch import nn
 
 from .._lib import host
+from ._tracing import record, tracing_state
 
 
 def vocab_range_from_per_partition_vocab_size(per_partition_vocab_size, rank, _):
@@ -33,6 +34,9 @@ def _group_rank_and_size(group):
 def vocab_parallel_cross_entropy(vocab_parallel_logits, target, label_smoothing=0.0, group=None):
     """Per-token loss log(sum exp(logits)) - logits[target], optionally label-smoothed; logits
     [..., vocab/p], target [...] (slapo/op/cross_entropy.py:128-150).  The loss is fp32."""
+    if tracing_state() is not None:
+        return record(vocab_parallel_cross_entropy, vocab_parallel_logits, target, label_smoothing,
+                      group)
     if _group_rank_and_size(group)[1] != 1:
         raise NotImplementedError(
             "vocab-parallel cross entropy over more than one rank: the per-shard statistics "

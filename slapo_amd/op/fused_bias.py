@@ -14,11 +14,14 @@ from torch import nn
 
 from .._lib import host
 from ..random import draw_philox_state
+from ._tracing import record, tracing_state
 
 
 def bias_gelu(inp: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
     """gelu_tanh(inp + bias); backward is the closed form of fused_bias.py:26-34 and returns the
     bias gradient already reduced to the bias shape."""
+    if tracing_state() is not None:
+        return record(bias_gelu, inp, bias)
     return host().bias_gelu(inp, bias)
 
 
@@ -31,6 +34,8 @@ class BiasGeLUFunction(torch.autograd.Function):
 
 def new_gelu(inp: torch.Tensor) -> torch.Tensor:
     """HF `gelu_new` (fused_bias.py:49-60) as one kernel per direction."""
+    if tracing_state() is not None:
+        return record(new_gelu, inp)
     return host().bias_gelu(inp, None)
 
 
@@ -55,6 +60,8 @@ def bias_dropout(x: torch.Tensor, bias: torch.Tensor, p: float = 0.5, training: 
     """dropout(x + bias).  `inplace` is accepted for signature compatibility; the reference's
     in-place target is the temporary x + bias, which this kernel never materialises."""
     del inplace
+    if tracing_state() is not None:
+        return record(bias_dropout, x, bias, p, training)
     _check_p(p)
     p = p if training else 0.0
     return host().bias_dropout_residual(x, bias, None, p, *_draw(x, p))
@@ -63,6 +70,8 @@ def bias_dropout(x: torch.Tensor, bias: torch.Tensor, p: float = 0.5, training: 
 def bias_dropout_residual(x: torch.Tensor, bias: torch.Tensor, residual: torch.Tensor,
                           p: float = 0.5, training: bool = True) -> torch.Tensor:
     """dropout(x + bias) + residual, the pattern of tests/test_fusion.py:179-180."""
+    if tracing_state() is not None:
+        return record(bias_dropout_residual, x, bias, residual, p, training)
     _check_p(p)
     p = p if training else 0.0
     return host().bias_dropout_residual(x, bias, residual, p, *_draw(x, p))
@@ -73,6 +82,9 @@ def bias_dropout_residual_layer_norm(x: torch.Tensor, bias, residual, weight: to
                                      training: bool = True) -> torch.Tensor:
     """layer_norm(dropout(x + bias) + residual) over the last dimension, the pattern of
     tests/test_fusion.py:184-185 (bias and residual may be None)."""
+    if tracing_state() is not None:
+        return record(bias_dropout_residual_layer_norm, x, bias, residual, weight, ln_bias, p, eps,
+                      training)
     _check_p(p)
     p = p if training else 0.0
     return host().bias_dropout_residual_layer_norm(x, bias, residual, weight, ln_bias, eps, p,

@@ -293,3 +293,67 @@ def test_fused_qkv_where_its_operations_are_watched():
         first, = torch.autograd.grad(f(x)[1], x, g, create_graph=True)
         seconds.append(torch.autograd.grad(first.square().sum(), g)[0])
     torch.testing.assert_close(*seconds)
+
+
+class _AmongTorchOperations(torch.nn.Module):
+    """An op of [2, 24, 64] values between two torch operations."""
+
+    def __init__(self, name):
+        super().__init__()
+        self.name = name
+        vec = lambda: torch.nn.Parameter(torch.randn(64))
+        self.bias, self.weight, self.shift = vec(), vec(), vec()
+        self.register_buffer("mask", torch.randn(2, 1, 1, 24))
+        self.register_buffer("target", torch.randint(0, 64, (2, 24)))
+        if name == "flash_attention":
+            self.child = op.FlashAttention(64, 4, 0.1, 0.1, "hip_cdna4", fused_qkv=True)
+        elif name == "fused_mlp":
+            self.child = op.FusedMLP(64, 64, "gelu_new", 0.1)
+
+    def forward(self, x):
+        x = x * 1.5
+        if self.name == "attention":
+            q = x.view(2, 24, 4, 16)
+            y = op.hip_attention(q, q.flip(1), q - 1, self.mask, causal=True, p=0.1).flatten(2)
+        elif self.name == "flash_attention":
+            y = self.child(x, self.mask)[0]
+        elif self.name == "fused_mlp":
+            y = self.child(x)
+        elif self.name == "bias_gelu":
+            y = op.bias_gelu(x, self.bias)
+        elif self.name == "new_gelu":
+            y = op.new_gelu(x)
+        elif self.name == "bias_dropout":
+            y = op.bias_dropout(x, self.bias, 0.1)
+        elif self.name == "bias_dropout_residual":
+            y = op.bias_dropout_residual(x, self.bias, x.flip(1), 0.1)
+        elif self.name == "layer_norm":
+            y = op.bias_dropout_residual_layer_norm(x, self.bias, x.flip(1), self.weight,
+                                                    self.shift, 0.1)
+        else:
+            y = op.vocab_parallel_cross_entropy(x, self.target, 0.1)
+        return y * 0.5 + 1
+
+
+@pytest.mark.parametrize("grad", [True, False])
+@pytest.mark.parametrize("name", ["attention", "flash_attention", "fused_mlp", "bias_gelu",
+                                  "new_gelu", "bias_dropout", "bias_dropout_residual",
+                                  "layer_norm", "cross_entropy"])
+def test_traced_ops_compute_on_their_inputs(name, grad):
+    """`torch.jit.trace` keeps an op as an operation: the traced module gives what the module gives
+    on other inputs than the example, its dropout draws again, and gradients flow through it."""
+    m = _AmongTorchOperations(name).cuda()
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(m, torch.randn(2, 24, 64, device="cuda"), check_trace=False)
+        x = torch.randn(2, 24, 64, device="cuda", requires_grad=grad)
+        torch.cuda.manual_seed(3)
+        wanted = m(x)
+        torch.cuda.manual_seed(3)
+        got = traced(x)
+    assert torch.equal(got, wanted)
+    if grad:
+        into = [x, *m.parameters()]
+        up = torch.randn_like(wanted)
+        for a, r in zip(torch.autograd.grad(got, into, up, allow_unused=True),
+                        torch.autograd.grad(wanted, into, up, allow_unused=True)):
+            assert (a is None) == (r is None) and (a is None or torch.equal(a, r))

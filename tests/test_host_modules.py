@@ -327,3 +327,50 @@ def test_fused_tail_is_taken_only_for_plain_hook_free_children():
     h = m.out_proj.register_full_backward_hook(lambda mod, gi, go: None)
     assert _has_hooks(m.out_proj)
     h.remove()
+
+
+def test_an_op_that_the_tracer_cannot_see_is_recorded_as_a_call():
+    """`record` on the host, with numpy in the kernels' place: the graph holds a call, not its
+    result, and gradients flow both while the trace is taken and when it runs."""
+    from slapo_amd.op import _tracing as T
+
+    class _Scale(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, x, bias, factor):
+            assert T.tracing_state() is None
+            ctx.factor = factor
+            return torch.from_numpy(x.detach().numpy() * factor + bias.detach().numpy())
+
+        @staticmethod
+        def backward(ctx, grad):
+            return grad * ctx.factor, grad.sum(0), None
+
+    def scale(x, bias, factor):
+        if T.tracing_state() is not None:
+            return T.record(scale, x, bias, factor)
+        return _Scale.apply(x, bias, factor)
+
+    bias = torch.nn.Parameter(torch.randn(4))
+    seen = []
+
+    class _Model(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.bias = bias
+
+        def forward(self, x):
+            y = scale(x + 1, self.bias, 3.0)
+            if T.tracing_state() is not None and y.requires_grad:
+                seen.append(torch.autograd.grad(y.sum(), self.bias)[0])
+            return y * 2
+
+    x = torch.randn(7, 4, requires_grad=True)
+    for grad in (False, True):
+        with torch.set_grad_enabled(grad):
+            traced = torch.jit.trace(_Model(), torch.randn(5, 4), check_trace=False)
+            got = traced(x)
+        assert torch.equal(got, ((x + 1) * 3 + bias) * 2)
+    assert len(seen) == 1 and torch.equal(seen[0], torch.full((4,), 5.0))
+    got.sum().backward()
+    assert torch.equal(x.grad, torch.full((7, 4), 6.0))
+    assert torch.equal(bias.grad, torch.full((4,), 14.0))
