@@ -49,8 +49,8 @@ __global__ __launch_bounds__(kThreads) void merge_fwd_kernel(const AttnArgs a) {
     const int n = min(4, a.d - c);
     for (int s = 0; s < a.n_split; ++s) {
         const float ms = ml[2 * s * n_rows];
-        if (ms == -INFINITY) continue;
-        const float w = kLog2 ? fast_exp2(ms - m) : expf(ms - m);
+        // (no maximum: nothing seen, or nothing but NaN scores, whose sum and values are NaN and stay)
+        const float w = ms == -INFINITY ? 0.f : kLog2 ? fast_exp2(ms - m) : expf(ms - m);
         l = __builtin_fmaf(ml[2 * s * n_rows + 1], w, l);
         const float* p = a.part + s * plane + row * a.d + c;
 #pragma unroll

@@ -683,6 +683,26 @@ def test_few_rows_dealt_to_many_workgroups(dtype, shape, sk, causal, window, p, 
     _check(q, k, v, do, mask, causal, window, dtype, p=p)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("causal", [False, True])
+def test_nan_keys_reach_every_row_that_sees_them(dtype, causal):
+    """Dealt tiles: a share whose visible scores are all NaN has no maximum and still counts.  One
+    key at a time, the first of every share of every block among them, and whole shares; the call
+    without a workspace, which deals nothing, gives the same."""
+    from slapo_amd.op import _kernels as K
+    s, d = 1536, 64
+    q, k, v, _, _ = _inputs(1, s, 1, d, dtype)
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    for lo, hi in [(j, j + 1) for j in range(0, s, 32)] + [(0, 192), (384, 768), (0, s)]:
+        bad = k.clone()
+        bad[:, lo:hi] = float("nan")
+        sees = (torch.arange(s, device="cuda") >= (lo if causal else 0)).view(1, s, 1, 1)
+        dealt = op.hip_attention(q, bad, v, causal=causal)
+        alone = K.attn_fwd(q, bad, v, None, causal, 0, d ** -0.5, 0.0, 0, 0, None)[0]
+        for out in (dealt, alone):
+            assert torch.equal(out.isnan(), sees.expand_as(out)), (lo, hi)
+
+
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("b,sq,sk,valid", [
     (1, 65, 131, 64),    # the second tile of keys is padding, one row in the last unit of 64
