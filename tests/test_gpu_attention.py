@@ -124,6 +124,31 @@ def test_key_only_bias_per_batch_and_head(dtype, shape, sk, causal, window, p):
     _check(q, k, v, do, mask, causal, window, dtype, p)
 
 
+@pytest.mark.parametrize("layout", ["dense", "sliced"])
+def test_an_fp32_per_query_mask_is_shared_by_the_calls_that_train_with_it(layout):
+    """The 16-bit kernels read such a mask in a layout of their own; between forward and backward a
+    call keeps the caller's tensor, not a copy, wherever the saved tensors are kept."""
+    b, s, h, d = 2, 200, 2, 64
+    q, k, v, do, g = _inputs(b, s, h, d, torch.float16)
+    mask = torch.randn(b, 1, s, s, generator=g)
+    _check(q, k, v, do, mask, True, 0, torch.float16, p=0.1)
+    q, k, v, do, mask = (t.cuda() for t in (q, k, v, do, mask))
+    if layout == "sliced":
+        mask = mask.repeat_interleave(2, dim=-1)[..., ::2]
+    q.requires_grad_()
+
+    def held(m):
+        before = torch.cuda.memory_allocated()
+        out = op.hip_attention(q, k, v, m, causal=True)
+        return out, torch.cuda.memory_allocated() - before
+
+    bare, masked = held(None), held(mask)
+    assert masked[1] == bare[1]
+    with torch.autograd.graph.save_on_cpu():
+        hooked = op.hip_attention(q, k, v, mask, causal=True)
+    assert torch.equal(*(torch.autograd.grad(out, q, do)[0] for out in (masked[0], hooked)))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("kind", ["short", "left", "holes"])
