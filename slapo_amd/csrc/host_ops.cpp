@@ -278,6 +278,9 @@ void check_packed(const Tensor& qkv, int64_t head_dim) {
                       "qkv must be [batch, seqlen, heads * 3 * head_dim]");
 }
 
+// A mask receives no gradient: what is saved of it must not hold on to how it was computed.
+Tensor detached(const Tensor& t) { return t.defined() && t.requires_grad() ? t.detach() : t; }
+
 struct AttnResult {
     Tensor out, lse, keep_mask;
 };
@@ -461,11 +464,12 @@ AttnResult run_attention(AttnProblem& a, const Operands& x, at::IntArrayRef out_
                            save_mask_max);
 }
 
-Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask,
+Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask_in,
                  bool causal, int64_t window, std::optional<double> scale, Dropout&& drop,
                  bool save_mask, int64_t save_mask_max) {
     check_operands(q, k, v);
-    require_device({&mask});
+    require_device({&mask_in});
+    const Tensor mask = detached(mask_in);
     refuse_tangents({&q, &k, &v});
     const bool need = torch::autograd::compute_requires_grad(q, k, v);
     auto node = make_node<AttnBackward>(need, q, k, v);
@@ -487,10 +491,11 @@ Tensor attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor
 
 // Self-attention on the output of a fused projection: qkv is [B, S, heads * 3 * head_dim] with q, k, v
 // of one head side by side, the result [B, S, heads * head_dim].
-Tensor attention_packed(const Tensor& qkv, int64_t head_dim, const Tensor& mask, bool causal,
+Tensor attention_packed(const Tensor& qkv, int64_t head_dim, const Tensor& mask_in, bool causal,
                         int64_t window, std::optional<double> scale, Dropout&& drop, bool save_mask,
                         int64_t save_mask_max) {
-    require_device({&qkv, &mask});
+    require_device({&qkv, &mask_in});
+    const Tensor mask = detached(mask_in);
     refuse_tangents({&qkv});
     check_packed(qkv, head_dim);
     const bool need = torch::autograd::compute_requires_grad(qkv);

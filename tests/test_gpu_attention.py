@@ -149,6 +149,29 @@ def test_an_fp32_per_query_mask_is_shared_by_the_calls_that_train_with_it(layout
     assert torch.equal(*(torch.autograd.grad(out, q, do)[0] for out in (masked[0], hooked)))
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows", [1, 96])
+def test_a_computed_mask_is_saved_without_its_history(dtype, rows, packed):
+    """The mask receives no gradient, so its graph is not kept until the backward."""
+    b, s, h, d = 2, 96, 2, 64
+    q, k, v, _, _ = _inputs(b, s, h, d, dtype)
+    q, k, v = (t.cuda().requires_grad_() for t in (q, k, v))
+    m = op.FlashAttention(h * d, h, fused_qkv=True).to("cuda", dtype)
+
+    def held(graph):
+        before = torch.cuda.memory_allocated()
+        source = torch.randn(1 << 20, device="cuda", requires_grad=graph)
+        mask = source.square()[:b * rows * s].clone().view(b, 1, rows, s)
+        out = m(q.flatten(2), mask)[0] if packed else op.hip_attention(q, k, v, mask)
+        del source, mask
+        return out, torch.cuda.memory_allocated() - before
+
+    held(False)  # (the workspace of the first matrix product)
+    without = held(False)
+    assert held(True)[1] == without[1]
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("kind", ["short", "left", "holes"])
