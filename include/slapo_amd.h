@@ -272,8 +272,8 @@ int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* 
 
 /* The same call with two more freedoms.
  * Bias type: SLAPO_F32 / F16 / BF16 name the element type that `bias` is stored in (with 16-bit
- * q / k / v a 16-bit bias must have stride 0 over the queries, and neither a call with dropout nor
- * the backward takes one);
+ * q / k / v a 16-bit bias must have stride 0 over the queries and a stride s3 >= 0 over the keys with
+ * s3 * seqlen_k < 2^30, and neither a call with dropout nor the backward takes one);
  * SLAPO_BIAS_PREPARED says that it is the output of slapo_amd_attn_prepare_bias, with strides
  * {batch, head, rounded seqlen_k, 1}.
  * Workspace: 16-byte aligned, slapo_amd_attn_fwd_workspace_bytes of it (may be NULL where that is

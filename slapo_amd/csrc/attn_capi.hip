@@ -201,12 +201,13 @@ int set_bias(AttnArgs* a, const void* bias, int type, bool f32, bool backward) {
         return aligned16(bias) ? SLAPO_OK : SLAPO_ERR_ALIGN;
     }
     if (type != SLAPO_F32 && type != SLAPO_F16 && type != SLAPO_BF16) return SLAPO_ERR_DTYPE;
-    // the kernels address the values of a row with 32-bit offsets
-    if (a->bs[3] < 0 || a->bs[3] * a->sk >= int64_t(1) << 30) return SLAPO_ERR_SHAPE;
-    // 16-bit biases of the 16-bit kernels: one value per key in a forward without dropout, or
-    // prepared
-    if (type != SLAPO_F32 && !f32 && (backward || a->dropout || a->bs[2] != 0))
-        return SLAPO_ERR_DTYPE;
+    if (type != SLAPO_F32 && !f32) {
+        // 16-bit biases of the 16-bit kernels: one value per key in a forward without dropout, or
+        // prepared
+        if (backward || a->dropout || a->bs[2] != 0) return SLAPO_ERR_DTYPE;
+        // (addressed with 32-bit offsets: BiasKeys)
+        if (a->bs[3] < 0 || a->bs[3] * a->sk >= int64_t(1) << 30) return SLAPO_ERR_SHAPE;
+    }
     if (a->bs[3] == 1 && aligned16(bias) && a->bs[0] % 4 == 0 && a->bs[1] % 4 == 0 &&
         a->bs[2] % 4 == 0)
         a->bias_vec4 = 1;

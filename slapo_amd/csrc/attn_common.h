@@ -281,7 +281,8 @@ __device__ __forceinline__ float bias_load(const AttnArgs& a, int64_t idx) {
         reinterpret_cast<uintptr_t>(a.bias) + ((uint64_t)idx << (a.bias_type == SLAPO_F32 ? 2 : 1));
     return bias_value(a, *reinterpret_cast<const uint32_t*>(at & ~(uintptr_t)3) >> ((at & 2) * 8));
 }
-// A row of values, one per key: a wavefront-uniform base and 32-bit byte offsets per lane.
+// A row of values, one per key: a wavefront-uniform base and 32-bit byte offsets per lane (a key
+// stride >= 0 whose seqlen_k-fold is below 2^30, checked by the dispatcher).
 struct BiasKeys {
     const char* base;
     uint32_t mis, shift, step;
@@ -406,10 +407,10 @@ __device__ __forceinline__ int padded_key_limit(const AttnArgs& a, int b, int h,
     if (!a.has_bias || a.bs[2] != 0 || a.window > 0) return a.sk;  // (a prepared one: pitch)
     int last = 0;
     if constexpr (kTyped) {
-        const BiasKeys row(a, b * a.bs[0] + h * a.bs[1]);
-        if (!(bias_value(a, row.raw(0)) > kMaskedBias)) return a.sk;
+        const int64_t row = b * a.bs[0] + h * a.bs[1];
+        if (!(bias_load(a, row) > kMaskedBias)) return a.sk;
         for (int j = threadIdx.x; j < a.sk; j += THREADS)
-            if (bias_value(a, row.raw(j)) > kMaskedBias) last = j;
+            if (bias_load(a, row + j * a.bs[3]) > kMaskedBias) last = j;
     } else {
         const float* row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1];
         if (!(row[0] > kMaskedBias)) return a.sk;

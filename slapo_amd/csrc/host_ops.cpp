@@ -223,8 +223,10 @@ struct AttnProblem {
         const bool per_key = mask.size(2) == 1;
         bias = known && (infer || !per_key || dtype == at::kFloat) ? mask : cast(mask, at::kFloat);
         bias_type = dtype_code(bias.scalar_type());
-        // (the kernels address a row's values with 32-bit offsets)
-        if (bias.size(3) > 1 && bias.stride(3) * sk() >= int64_t(1) << 30) bias = bias.contiguous();
+        // (the 16-bit kernels address a row of 16-bit values with 32-bit offsets)
+        if (bias_type != SLAPO_F32 && per_key && dtype != at::kFloat && bias.size(3) > 1 &&
+            bias.stride(3) * sk() >= int64_t(1) << 30)
+            bias = bias.contiguous();
         address_bias();
         if (dtype == at::kFloat || per_key || empty() || sk() == 0) return;
         const int64_t mb = prm.bias_strides[0] ? b() : 1, mh = prm.bias_strides[1] ? h() : 1;

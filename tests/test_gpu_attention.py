@@ -778,6 +778,50 @@ def test_a_refused_mask_draws_nothing():
     assert torch.equal(before, torch.cuda.get_rng_state())
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("s,rows,step", [
+    (70, 1, -1), (70, 70, -1),   # values per key and per query, backwards
+    (5, 5, -3),
+    (5, 1, 1 << 28),             # the last key's value 4 GB behind the first's
+])
+def test_bias_strides_of_the_c_abi(dtype, s, rows, step):
+    """An fp32 bias is addressed with 64-bit strides of either sign, forward and backward: the same
+    bits as from a dense one."""
+    import ctypes
+
+    from slapo_amd import _lib
+    from slapo_amd.op import _kernels as K
+
+    lib = _lib.load()
+    b, h, d = 1, 2, 64
+    q, k, v, do, g = _inputs(b, s, h, d, dtype)
+    q, k, v, do = (t.cuda() for t in (q, k, v, do))
+    dense = torch.randn(rows, s, generator=g)
+    dense[:, s - 2:] = -1e9  # padded keys: the walk that looks for them reads the bias as well
+    dense = dense.cuda()
+    span = (s - 1) * abs(step) + 1
+    spread = torch.empty(rows, span, device="cuda")
+    spread[:, ::abs(step)] = dense.flip(-1) if step < 0 else dense
+    first = spread.data_ptr() + (4 * (span - 1) if step < 0 else 0)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    ws = torch.empty(b * h * s, device="cuda")
+    results = []
+    for bias, row, key in ((dense.data_ptr(), s, 1), (first, span, step)):
+        o, lse = torch.empty_like(q), torch.empty(b, h, s, device="cuda")
+        grads = [torch.empty_like(q) for _ in range(3)]
+        prm = K.make_attn_params(q, k, v, o, None, True, 0, d ** -0.5, 0.0, 0, 0, None)
+        prm.bias_strides = (ctypes.c_int64 * 4)(0, 0, row if rows > 1 else 0, key)
+        assert lib.slapo_amd_attn_fwd(ctypes.byref(prm), P(q), P(k), P(v), bias, P(o), P(lse),
+                                      st) == 0
+        assert lib.slapo_amd_attn_bwd(
+            ctypes.byref(prm), P(q), P(k), P(v), bias, P(o), P(do), P(lse), *map(P, grads),
+            *(K._bshd_strides(t) for t in grads), P(ws), ws.numel() * 4, st) == 0
+        results.append([o, lse, *grads])
+    for a, r in zip(*results):
+        assert torch.equal(a, r)
+
+
 # ---- seeded sweep over the whole call surface --------------------------------------------------
 @pytest.mark.parametrize("seed", range(40))
 def test_random_configurations_against_the_oracle(seed):
