@@ -310,7 +310,9 @@ int slapo_amd_attn_bwd(const slapo_attn_params* prm, const void* q, const void* 
 
 /* The same call with the bias type of slapo_amd_attn_fwd_ex.  A workspace of
  * slapo_amd_attn_bwd_ex_workspace_bytes (at least slapo_amd_attn_bwd_workspace_bytes is needed)
- * also holds the partial results of a call that is dealt to more workgroups as described there. */
+ * also holds the partial results of a call that is dealt to more workgroups as described there;
+ * the sums of such a call are formed in another order than slapo_amd_attn_bwd's, which deals nothing
+ * whatever its workspace holds. */
 size_t slapo_amd_attn_bwd_ex_workspace_bytes(const slapo_attn_params* prm);
 int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
                           const void* v, const void* bias, int bias_type, const void* o,

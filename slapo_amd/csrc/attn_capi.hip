@@ -422,7 +422,7 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
                  const void* bias, int bias_type, const void* o, const void* dout,
                  const float* lse, void* dq, void* dk, void* dv, const int64_t dq_strides[3],
                  const int64_t dk_strides[3], const int64_t dv_strides[3], void* workspace,
-                 size_t workspace_bytes, int stages, void* stream) {
+                 size_t workspace_bytes, int stages, bool deal, void* stream) {
     AttnArgs a = {};
     int rc = fill_args(prm, &a, true);
     if (rc != SLAPO_OK) return rc;
@@ -454,12 +454,10 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
         if (!strides_ok(dq_strides, 8) || !strides_ok(dk_strides, 8) || !strides_ok(dv_strides, 8))
             return SLAPO_ERR_ALIGN;
     }
-    // Partial results need room, and a caller that runs all stages: both kernels' are merged in one
-    // launch at the end.
+    // Partial results need room.  Both kernels' are merged in one launch at the end.
     Splits splits;
     float *dq_part = nullptr, *dkv_part = nullptr;
-    if (stages == SLAPO_BWD_ALL &&
-        workspace_bytes >= slapo_amd_attn_bwd_ex_workspace_bytes(prm)) {
+    if (deal && workspace_bytes >= slapo_amd_attn_bwd_ex_workspace_bytes(prm)) {
         splits = plan_splits(prm);
         float* next = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(prm));
         if (splits.dq > 1) {
@@ -500,7 +498,7 @@ extern "C" int slapo_amd_attn_bwd_stages(const slapo_attn_params* prm, const voi
                                          const int64_t dv_strides[3], void* workspace,
                                          size_t workspace_bytes, int stages, void* stream) {
     return run_backward(prm, q, k, v, bias, SLAPO_F32, o, dout, lse, dq, dk, dv, dq_strides,
-                        dk_strides, dv_strides, workspace, workspace_bytes, stages, stream);
+                        dk_strides, dv_strides, workspace, workspace_bytes, stages, false, stream);
 }
 
 extern "C" int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
@@ -510,7 +508,8 @@ extern "C" int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q
                                      const int64_t dk_strides[3], const int64_t dv_strides[3],
                                      void* workspace, size_t workspace_bytes, void* stream) {
     return run_backward(prm, q, k, v, bias, bias_type, o, dout, lse, dq, dk, dv, dq_strides,
-                        dk_strides, dv_strides, workspace, workspace_bytes, SLAPO_BWD_ALL, stream);
+                        dk_strides, dv_strides, workspace, workspace_bytes, SLAPO_BWD_ALL, true,
+                        stream);
 }
 
 extern "C" int slapo_amd_attn_bwd(const slapo_attn_params* prm, const void* q, const void* k,

@@ -661,6 +661,48 @@ def test_backward_is_bitwise_reproducible_and_stages_compose():
         assert torch.equal(a, c)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_backward_forms_agree_where_tiles_could_be_dealt(dtype):
+    """A call of few rows, with room for the partial results of dealt tiles: slapo_amd_attn_bwd
+    equals its own stages and the form with a workspace inside the library, bit for bit;
+    slapo_amd_attn_bwd_ex deals, and agrees to rounding."""
+    import ctypes
+
+    from slapo_amd import _lib
+    from slapo_amd.op import _kernels as K
+
+    lib = _lib.load()
+    s, d = 1536, 16
+    q, k, v, do, _ = _inputs(1, s, 1, d, dtype)
+    q, k, v, do = (t.cuda() for t in (q, k, v, do))
+    o, lse, _ = K.attn_fwd(q, k, v, None, True, 0, d ** -0.5, 0.0, 0, 0, None)
+    prm = K.make_attn_params(q, k, v, o, None, True, 0, d ** -0.5, 0.0, 0, 0, None)
+    nb = lib.slapo_amd_attn_bwd_ex_workspace_bytes(ctypes.byref(prm))
+    assert lib.slapo_amd_attn_bwd_workspace_bytes(ctypes.byref(prm)) < nb <= 4 << 20
+    ws = torch.empty(nb // 4, device="cuda")
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+
+    def run(*calls):
+        grads = [torch.full_like(q, float("nan")) for _ in range(3)]
+        strides = [K._bshd_strides(t) for t in grads]
+        into = [P(o), P(do), P(lse), *map(P, grads), *strides]
+        for fn, bias, tail in calls:
+            assert fn(ctypes.byref(prm), P(q), P(k), P(v), *bias, *into, *tail, st) == 0
+        return grads
+
+    whole = run((lib.slapo_amd_attn_bwd, [None], [P(ws), nb]))
+    for other in (run(*((lib.slapo_amd_attn_bwd_stages, [None], [P(ws), nb, stage])
+                        for stage in (_lib.BWD_PREPARE, _lib.BWD_DQ, _lib.BWD_DKDV))),
+                  run((lib.slapo_amd_attn_bwd_static_scratch, [None], []))):
+        for a, r in zip(other, whole):
+            assert torch.equal(a, r)
+    dealt = run((lib.slapo_amd_attn_bwd_ex, [None, _lib.SLAPO_F32], [P(ws), nb]))
+    assert not all(torch.equal(a, r) for a, r in zip(dealt, whole))
+    for a, r in zip(dealt, whole):
+        assert_parity(a, r, dtype)
+
+
 @pytest.mark.parametrize("shape,sk,causal,window,p", [
     ((1, 1, 2, 20), 33, False, 0, 0.0),       # one query, head_dim no multiple of four
     ((1, 15, 1, 72), 16, True, 0, 0.0),       # less than a wavefront's rows
