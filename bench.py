@@ -264,27 +264,26 @@ def bench_epilogues(device, iters=40):
                                            "frac_of_hbm_peak": nbytes / sec / 1e9 / HBM_PEAK_GBS}
     del xs, rs, os_, zs
 
-    # vocab-parallel cross entropy on one shard: GPT-2's unpadded vocabulary, fp16 logits
+    # cross entropy with the whole vocabulary on one device: GPT-2's unpadded one, fp16 logits
     V = 50257
     logits = torch.randn(T, V, device=device, dtype=torch.float16)
     grad = torch.empty_like(logits)
     tgt = torch.randint(0, V, (T,), device=device)
-    stats = torch.empty(4, T, device=device, dtype=torch.float32)
-    gl = torch.ones(T, device=device, dtype=torch.float32)
+    loss, row_max, inv_s, gl = (torch.ones(T, device=device, dtype=torch.float32)
+                                for _ in range(4))
 
-    def ce_fwd(i):
-        rc = lib.slapo_amd_vocab_ce_fwd(P(logits), P(tgt), P(stats[0]), P(stats[1]), P(stats[2]),
-                                        P(stats[3]), T, V, 0, _lib.SLAPO_F16, st)
+    def ce_fwd(i):  # the loss, and what the backward needs of a row: what the op launches
+        rc = lib.slapo_amd_vocab_ce_loss(P(logits), P(tgt), P(loss), P(row_max), P(inv_s), T, V,
+                                         0.0, _lib.SLAPO_F16, st)
         assert rc == 0
 
     sec = timed(ce_fwd, 1)
-    nbytes = T * V * 2 + T * (8 + 16)
+    nbytes = T * V * 2 + T * (8 + 12)
     out["vocab_ce_fwd"] = {"bytes": nbytes, "us": sec * 1e6, "GBps": nbytes / sec / 1e9,
                            "frac_of_hbm_peak": nbytes / sec / 1e9 / HBM_PEAK_GBS}
-    inv_s = 1.0 / stats[1]
 
     def ce_bwd(i):
-        rc = lib.slapo_amd_vocab_ce_bwd(P(logits), P(tgt), P(stats[0]), P(inv_s), P(gl), P(grad),
+        rc = lib.slapo_amd_vocab_ce_bwd(P(logits), P(tgt), P(row_max), P(inv_s), P(gl), P(grad),
                                         T, V, 0, 0.0, _lib.SLAPO_F16, st)
         assert rc == 0
 
@@ -517,21 +516,24 @@ def bench_other_attention(device, iters=20, with_cpu=True):
                                      save_mask=True)
         prm = K.make_attn_params(q, k, v, o, bias, True, w, scale, cfg["p"], 2013, 0, plan, keep)
         dq, dk, dv = (torch.empty_like(q) for _ in range(3))
-        nbytes = lib.slapo_amd_attn_bwd_workspace_bytes(ctypes.byref(prm))
-        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
+        nfwd = lib.slapo_amd_attn_fwd_workspace_bytes(ctypes.byref(prm))
+        nbytes = lib.slapo_amd_attn_bwd_ex_workspace_bytes(ctypes.byref(prm))
+        ws = torch.empty(max(nfwd, nbytes) // 4, dtype=torch.float32, device=device)
         strides = [K._bshd_strides(t) for t in (dq, dk, dv)]
 
+        # the calls that the op makes, with the workspaces it gives them
         def fwd():
-            rc = lib.slapo_amd_attn_fwd(ctypes.byref(prm), P(q), P(k), P(v), P(bias), P(o), P(lse),
-                                        st)
+            rc = lib.slapo_amd_attn_fwd_ex(ctypes.byref(prm), P(q), P(k), P(v), P(bias),
+                                           _lib.SLAPO_F32, P(o), P(lse), P(ws), nfwd, st)
             if rc:
-                raise RuntimeError(f"slapo_amd_attn_fwd failed with status {rc}")
+                raise RuntimeError(f"slapo_amd_attn_fwd_ex failed with status {rc}")
 
         def bwd():
-            rc = lib.slapo_amd_attn_bwd(ctypes.byref(prm), P(q), P(k), P(v), P(bias), P(o), P(do),
-                                        P(lse), P(dq), P(dk), P(dv), *strides, P(ws), nbytes, st)
+            rc = lib.slapo_amd_attn_bwd_ex(ctypes.byref(prm), P(q), P(k), P(v), P(bias),
+                                           _lib.SLAPO_F32, P(o), P(do), P(lse), P(dq), P(dk),
+                                           P(dv), *strides, P(ws), nbytes, st)
             if rc:
-                raise RuntimeError(f"slapo_amd_attn_bwd failed with status {rc}")
+                raise RuntimeError(f"slapo_amd_attn_bwd_ex failed with status {rc}")
 
         def timed(fn):
             for _ in range(3):
