@@ -215,7 +215,7 @@ int slapo_amd_vocab_ce_bwd(const void* logits, const int64_t* target, const floa
  * restatements xformers_ref (:134-196) and flash_attn_ref (:39-131).
  * ---------------------------------------------------------------------------------------- */
 typedef struct slapo_attn_params {
-    int32_t dtype;    /* SLAPO_F16 / SLAPO_BF16 (MFMA kernels) or SLAPO_F32 (fp32 FMA kernels)  */
+    int32_t dtype;    /* SLAPO_F16 / SLAPO_BF16 or SLAPO_F32: MFMA kernels of that type         */
     int32_t batch;
     int32_t heads;
     int32_t seqlen_q;
@@ -246,13 +246,15 @@ typedef struct slapo_attn_params {
     slapo_dropout_plan plan;
     /* Optional (may be NULL), 16-bit types with p_drop > 0 only: device buffer of
      * slapo_amd_attn_keep_mask_bytes(prm) bytes.  The forward call stores the dropout keep bits
-     * in it (one bit per score; with window > 0 a kernel launched ahead of the forward kernel on
-     * the same stream draws them and the forward kernel reads them), and a backward that is given
+     * in it (one bit per score; with window > 0, and where the plan's geometry has no whole Philox
+     * block per aligned group of four keys, a kernel launched ahead of the forward kernel on the
+     * same stream draws them and the forward kernel reads them), and a backward that is given
      * the same buffer reads them instead of drawing every Philox block again in both of its
      * kernels.  The results are bitwise the same with and without it.  Words whose keys no query
      * of the row's 32-query group can see under the causal mask are not written; with a window,
-     * only the words that hold a key the row itself can see are (the rest is never applied to a
-     * non-zero probability).  Layout: uint32 words [batch*heads][ceil(seqlen_k/32)][pitch],
+     * only the words that hold a key the row itself can see are, and words drawn ahead beside a
+     * per-key bias not where their key tile and all behind it are padding (the rest is never
+     * applied to a non-zero probability).  Layout: uint32 words [batch*heads][ceil(seqlen_k/32)][pitch],
      * pitch = seqlen_q rounded up to 4; bit j of word (bh, w, i) = keep(query i, key 32 w + j). */
     void* keep_mask;
 } slapo_attn_params;

@@ -30,8 +30,8 @@ namespace {
 // kernels: thread (row i, word w) draws the eight Philox blocks of keys 32 w .. 32 w + 31 of
 // query i and stores them as one word, keep_mask[(bh * mask_words + w) * mask_pitch + i], bit j =
 // keep(i, 32 w + j).  The matrix kernels then only test bits; drawing inside the forward kernel
-// costs about forty vector-ALU cycles per score beside thirty-two (head_dim 128) or sixteen (64)
-// of matrix work.  Only words that hold a key the row itself can see are drawn: the kernels read
+// costs about seventy vector-ALU cycles per score (61 instructions per block of four) beside
+// thirty-two (head_dim 128) or sixteen (64) of matrix work.  Only words that hold a key the row itself can see are drawn: the kernels read
 // whole words of every 64-key tile that some query of a 32-query group sees, but a bit that
 // belongs to a pair outside the row's own mask meets a probability of zero, so what such words
 // hold does not matter and they are left as they are.  With a local window the word columns count
@@ -40,10 +40,10 @@ namespace {
 // kExact: any launch geometry of the dropout plan and any seqlen_k (dropout_keep32).  Drawn per
 // word this costs 9 Philox blocks per 32 scores where the forward kernel, whose lanes hold single
 // groups of four, drew one block per score: bf16 B3 S777 H12 D64 without a causal mask, p 0.1,
-// forward and backward 199 us before, 92 us with this kernel ahead of the forward.  The words of
+// forward and backward 199 us before, 89 us with this kernel ahead of the forward.  The words of
 // padded keys are left as they are too where the other kernels skip their tiles (a third of them in
 // that call's mask).  Units of 64 rows and a word, dealt to the wavefronts one after the other: blocks
-// of 256 rows left a quarter of the launch to nine rows at S777.  That call: 22.1 -> 17.5 us.
+// of 256 rows left a quarter of the launch to nine rows at S777.  That call: 22.1 -> 17.3 us.
 template <bool kExact>
 __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in, int words) {
     AttnArgs a = a_in;

@@ -134,11 +134,11 @@ namespace slapo {
 // all below 24 (12) tiles: partial results and their merging cost about 10 us, a tile of 64 keys
 // takes a workgroup about 0.6 us at head_dim 64 and 1.1 us at 128.  1: no split.
 // A CU is busy with one workgroup of the 16-bit kernels (one wavefront per SIMD does 92 % of what
-// two do), with two of the fp32 ones.  bf16, causal: B1 S2304 H3 D128 forward 50 -> 35 us, forward +
-// backward 207 -> 113 us; at B2 S1024 H8 D64 the same split costs (19 -> 26 us).  fp32 B1 S1971 H2
-// D72 forward + backward 712 -> 169 us.
+// two do), with two of the fp32 ones.  Kernels, merging included, bf16, causal: B1 S2304 H3 D128
+// forward 49 -> 29 us, forward + backward 206 -> 109 us; at B2 S1024 H8 D64 the same split costs
+// (forward 19 -> 26 us).  fp32 B1 S1971 H2 D72 forward + backward 629 -> 170 us.
 // Under a causal mask the blocks have half the longest one's tiles on average, so that even a launch
-// with a workgroup for every CU gains from two shares (bf16 B1 S8192 H4 D64: 375 -> 313 us).
+// with a workgroup for every CU gains from two shares (bf16 B1 S8192 H4 D64: 378 -> 315 us).
 int attn_splits(int64_t blocks, int64_t cus, int64_t tiles, bool f32, bool causal) {
     const int64_t slots = f32 ? 2 * cus : cus, least = f32 ? 4 : 6;
     if (blocks <= 0 || tiles < (f32 ? 12 : 24)) return 1;

@@ -451,7 +451,7 @@ def test_scale_one_with_unscaled_queries_against_the_fp32_kernels(dtype):
     deviation 11 and row maxima near 40.  The MFMA kernels fold scale * log2(e) into Q (forward,
     dQ) or K (dK/dV) and round the product back to the 16-bit type, so forward and backward do not
     round the same operand: with |s| around 40 the recomputed probabilities differ from the
-    forward's by about 2^-9 |s| relative.  The fp32 FMA kernels of this library (oracle-checked at
+    forward's by about 2^-9 |s| relative.  The fp32 kernels of this library (oracle-checked at
     1e-5) run on the same 16-bit values and give the reference.  Softmax rows are nearly one-hot
     here, so the comparison is made at the parity bar relative to the largest reference magnitude,
     as for every other 16-bit case; the measured errors are recorded in the design notes."""
@@ -498,7 +498,7 @@ def test_cfg5_gpt_neo_at_seq_2048_against_the_oracle(window):
 def test_full_size_cfg2_properties():
     """fp16, B 8, S 1024, 16 x 64, causal, at full size: (1) V = const gives that const back
     (rows of P sum to one); (2) query 0 returns V[0]; (3) linearity in V; (4) agreement with the
-    independent fp32 FMA kernels of this library run on the same fp16 values; (5) dV, dK vanish
+    independent fp32 kernels of this library run on the same fp16 values; (5) dV, dK vanish
     for no key and sum rules: sum_i dQ.q = sum_j dK.k (softmax shift invariance gives
     sum_j dS_ij = 0 hence dQ_i . q_i = sum_j ds_ij s_ij = ... checked as a scalar identity)."""
     b, s, h, d = 8, 1024, 16, 64
@@ -527,7 +527,7 @@ def test_full_size_cfg2_properties():
 
 
 def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
-    """The library's independent fp32 FMA kernels on the same 16-bit values and the same seed."""
+    """The library's independent fp32 kernels on the same 16-bit values and the same seed."""
     qf, kf, vf = (t.float().requires_grad_(True) for t in (q, k, v))
     torch.cuda.manual_seed(seed)
     ref = op.hip_attention(qf, kf, vf, mask, causal=causal, p=p, window=window)
@@ -539,7 +539,7 @@ def test_full_size_cfg4_properties():
     """bf16, B 4, S 2048, 32 x 80, causal + key padding with valid lengths ~ U[512, 2048], at full
     size: rows of P sum to one (V = 1 returns 1, also for queries in the padded region); query 0
     returns V[0]; linearity in V; padded keys receive exactly zero dK, dV; agreement of all four
-    outputs with the fp32 FMA kernels run on the same bf16 values; sum_i dQ.q = sum_j dK.k."""
+    outputs with the fp32 kernels run on the same bf16 values; sum_i dQ.q = sum_j dK.k."""
     b, s, h, d = 4, 2048, 32, 80
     g = torch.Generator().manual_seed(2013)
     q, k, v, do = (torch.randn(b, s, h, d, generator=g).bfloat16().cuda() for _ in range(4))
@@ -572,7 +572,7 @@ def test_full_size_cfg5_properties(window):
     """bf16, B 4, S 2048, 16 x 128, causal (global and window 256), dropout 0.1, at full size
     (268 M scores: 128 Philox loop trips).  The keep bits that the forward stores are torch's
     mask for the dense fp32 [B*H, Sq, Sk] tensor wherever the forward visits; outputs and
-    gradients agree with the fp32 FMA kernels run under the same seed; with V = 1 every row
+    gradients agree with the fp32 kernels run under the same seed; with V = 1 every row
     returns the kept share of its probabilities, which averages to 1 over a head."""
     import ctypes
 
@@ -905,7 +905,7 @@ def test_random_configurations_against_the_oracle(seed):
                                                  ((1, 12288, 1, 128), True, 1000)])
 def test_long_sequences_against_the_fp32_kernels(shape, causal, window):
     """Sequence lengths well beyond the benchmark's (16 to 256 key tiles per workgroup, offsets
-    past 2^24 elements within a head): the MFMA kernels against the fp32 FMA kernels of this
+    past 2^24 elements within a head): the MFMA kernels against the fp32 kernels of this
     library (oracle-checked at 1e-5 on small shapes) on the same bf16 values, at the 2e-2 bar."""
     g = torch.Generator().manual_seed(77)
     mk = lambda: torch.randn(*shape, generator=g).to(torch.bfloat16)
