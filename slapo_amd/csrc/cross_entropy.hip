@@ -26,14 +26,33 @@ namespace {
 constexpr int kCeMaxThreads = 1024;
 constexpr int kCeAlign = 128;  // bytes: alignment of a row's vector body
 
-// (m, s) pairs combine as  m = max(m1, m2),  s = s1 exp(m1 - m) + s2 exp(m2 - m); an empty
-// partner is (-inf, 0).
+// (m, s) pairs combine as  m = max(m1, m2),  s = s1 exp(m1 - m) + s2 exp(m2 - m).  A pair without a
+// maximum has weight 0: it has met nothing or nothing but -inf, (-inf, 0), or a NaN as well, which
+// no maximum takes and the sum passes on, (-inf, NaN).
+__device__ __forceinline__ float ce_weight(float m, float mn) {
+    return m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f((m - mn) * 1.4426950408889634f);
+}
 __device__ __forceinline__ void ce_merge(float& m, float& s, float m2, float s2) {
     const float mn = fmaxf(m, m2);
-    if (mn == -INFINITY) return;  // both empty
-    s = s * __builtin_amdgcn_exp2f((m - mn) * 1.4426950408889634f) +
-        s2 * __builtin_amdgcn_exp2f((m2 - mn) * 1.4426950408889634f);
+    s = s * ce_weight(m, mn) + s2 * ce_weight(m2, mn);
     m = mn;
+}
+// N logits, vm their maximum, join a pair
+template <int N>
+__device__ __forceinline__ void ce_add(float& m, float& s, const float (&f)[N], float vm) {
+    // rescale the running sum only when the maximum moves
+    const float mn = fmaxf(m, vm);
+    if (mn > m) {
+        s *= __builtin_amdgcn_exp2f((m - mn) * 1.4426950408889634f);  // exp2(-inf) = 0
+        m = mn;
+    }
+    if (m != -INFINITY) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) s += __builtin_amdgcn_exp2f((f[j] - m) * 1.4426950408889634f);
+    } else {
+#pragma unroll
+        for (int j = 0; j < N; ++j) s += f[j] == f[j] ? 0.f : f[j];
+    }
 }
 
 template <typename T>
@@ -103,7 +122,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd_kernel(
     float m = -INFINITY, s = 0.f, sx = 0.f;
     auto add1 = [&](float v) __attribute__((always_inline)) {
         sx += v;
-        ce_merge(m, s, v, 1.0f);
+        ce_add<1>(m, s, {v}, v);
     };
     if ((int)threadIdx.x < sp.head) add1(Elem<T>::to_f32(x[threadIdx.x]));
     for (int e = sp.tail0 + threadIdx.x; e < n; e += kCeThreads) add1(Elem<T>::to_f32(x[e]));
@@ -127,17 +146,7 @@ __global__ __launch_bounds__(kCeThreads) void ce_fwd_kernel(
             vm = fmaxf(vm, f[j]);
             sx += f[j];
         }
-        // rescale the running sum only when the maximum moves
-        const float mn = fmaxf(m, vm);
-        if (mn > m) {
-            s *= __builtin_amdgcn_exp2f((m - mn) * 1.4426950408889634f);  // exp2(-inf) = 0
-            m = mn;
-        }
-        if (m != -INFINITY) {
-#pragma unroll
-            for (int j = 0; j < V; ++j)
-                s += __builtin_amdgcn_exp2f((f[j] - m) * 1.4426950408889634f);
-        }
+        ce_add<V>(m, s, f, vm);
     };
     // four loads in flight per thread
     int i = threadIdx.x;

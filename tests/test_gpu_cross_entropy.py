@@ -148,3 +148,30 @@ def test_rows_that_start_anywhere_relative_to_a_cache_line(off_x, off_g):
     assert_parity(grad, OC.backward(softmax, target, go.double()), torch.float16, "grad")
     # nothing outside the gradient's own elements was written
     assert bool((buf_g[:off_g] == 7.0).all()) and bool((buf_g[off_g + rows * vocab:] == 7.0).all())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("offset", [0, 3])
+def test_a_nan_logit_reaches_the_loss(dtype, offset):
+    """One NaN per row, in the head, the body, the tail or as a thread's whole vector, with finite
+    or -inf neighbours: the row's loss and gradient are NaN, the other rows' are not; the op's
+    kernel on buffers that start anywhere."""
+    vocab = 1237
+    spots = [(0, 1), (1, 2), (40, 41), (63, 64), (64, 65), (64, 72), (128, 192), (700, 701),
+             (1230, 1237), (1236, 1237)]
+    logits, target, go = _case((3 * len(spots),), vocab, dtype)
+    for i, (lo, hi) in enumerate(spots):
+        logits[3 * i, lo:hi] = float("nan")
+        logits[3 * i + 1, max(0, lo - 70):lo + 70] = float("-inf")
+        logits[3 * i + 1, lo:hi] = float("nan")
+    buf = torch.zeros(logits.numel() + offset, dtype=dtype, device="cuda")
+    x = buf[offset:].view_as(logits)
+    x.copy_(logits)
+    x.requires_grad_()
+    loss = op.vocab_parallel_cross_entropy(x, target.cuda())
+    loss.backward(go.cuda())
+    bad = torch.arange(3 * len(spots), device="cuda") % 3 != 2
+    assert torch.equal(loss.isnan(), bad)
+    assert torch.equal(x.grad.isnan().all(-1), bad) and torch.equal(x.grad.isnan().any(-1), bad)
+    ref, _ = OC.forward(logits[2::3], target[2::3])
+    assert max_abs_err(loss[2::3], ref) <= 1e-4 * max(1.0, float(ref.abs().max()))
