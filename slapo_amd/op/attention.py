@@ -141,9 +141,11 @@ class FlashAttentionOp(nn.Module):
         self.bias_layout = "b11k"
 
     def forward(self, query_layer, key_layer, value_layer, attention_mask, p):
-        return self.attn_fn(query_layer, key_layer, value_layer, attention_mask,
-                            causal=self.apply_causal_mask, p=p, scale=self.scale,
-                            window=self.window or 0)
+        ret = self.attn_fn(query_layer, key_layer, value_layer, attention_mask,
+                           causal=self.apply_causal_mask, p=p, scale=self.scale,
+                           window=self.window or 0)
+        # (the kernel keeps the type; a function put in its place may not)
+        return ret if self.attn_fn is hip_attention else ret.to(query_layer.dtype)
 
     def extra_repr(self):
         return (f"attn_op_name={self.attn_op_name}, causal={self.apply_causal_mask}, "

@@ -374,3 +374,11 @@ def test_an_op_that_the_tracer_cannot_see_is_recorded_as_a_call():
     got.sum().backward()
     assert torch.equal(x.grad, torch.full((7, 4), 6.0))
     assert torch.equal(bias.grad, torch.full((4,), 14.0))
+
+
+def test_a_replaced_attention_function_keeps_the_type_of_the_queries():
+    core = op.FlashAttentionOp("hip_cdna4", True)
+    core.attn_fn = lambda q, k, v, mask, causal, p, scale, window: q.float() * 2
+    q = torch.randn(1, 4, 2, 8, dtype=torch.float16)
+    out = core(q, q, q, None, 0.0)
+    assert out.dtype == torch.float16 and torch.equal(out, q * 2)
