@@ -37,7 +37,7 @@ namespace {
 // hold does not matter and they are left as they are.  With a local window the word columns count
 // from the first word of the row's window (window / 32 + 1 of them, not seqlen_k / 32: every thread
 // then has a word to draw); without one they are the words themselves.
-// kExact: any launch geometry of the dropout plan and any seqlen_k (dropout_keep32).  Drawn per
+// kExact: any launch geometry of the dropout plan and any seqlen_k (dropout_keep_run).  Drawn per
 // word this costs 9 Philox blocks per 32 scores where the forward kernel, whose lanes hold single
 // groups of four, drew one block per score: bf16 B3 S777 H12 D64 without a causal mask, p 0.1,
 // forward and backward 199 us before, 89 us with this kernel ahead of the forward.  The words of
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in, int
     const uint64_t row_base = ((uint64_t)bh * a.sq + (uint64_t)i) * (uint64_t)a.sk;
     uint32_t word = 0;
     if constexpr (kExact) {
-        word = dropout_keep32(a.rng, row_base + 32 * (uint64_t)w);
+        word = dropout_keep_run(a.rng, row_base + 32 * (uint64_t)w, 32);
     } else {
 #pragma unroll
         for (int blk = 0; blk < 8; ++blk) {

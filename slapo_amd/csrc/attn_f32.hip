@@ -1,27 +1,36 @@
-// Attention forward and backward for fp32 tensors on the fp32 matrix instructions
-// (v_mfma_f32_16x16x4_f32: fp32 operands, fp32 products and sums -- no reduced-precision input
-// anywhere), the kernels behind dtype == SLAPO_F32, whose parity bar is 1e-5 absolute.
+// Attention forward and backward for fp32 tensors, the kernels behind dtype == SLAPO_F32, whose
+// parity bar is 1e-5 absolute.
 //
-// v_mfma_f32_16x16x4_f32 (one wavefront, lane l, i = l % 16, g = l / 16):
-//   A operand: lane holds A[row i][k-slot g];   B operand: lane holds B[k-slot g][column i];
+// Products run on the bf16 matrix instructions without giving up fp32: an operand is the exact sum
+// of three bf16 numbers, x = h + m + l (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 8 + 8 + 8
+// mantissa bits, fp32's exponent range), and x y = hh + (hm + mh) + (mm + hl + lh) + O(2^-25 |x y|),
+// six v_mfma_f32_16x16x32_bf16 with exact products and fp32 sums.
+//
+// v_mfma_f32_16x16x32_bf16 (one wavefront, lane l, i = l % 16, g = l / 16):
+//   A operand: lane holds A[row i][k-slots 8 g .. 8 g + 7];   B operand: the same slots of column i;
 //   C/D:       register r of lane l is element (row 4 g + r, column i).
-// The k-slots may stand for any data as long as A and B agree.  Two choices keep every operand a
-// plain LDS read or a register:
-//  * products over the head dimension (S = QK^T, dP = dO V^T): slot g of step 4 t + e is element
-//    16 t + 4 g + e, so that one 16-byte read of a row serves four steps;
-//  * products over keys or queries (PV, dS K, P^T dO, dS^T Q): an accumulator register r of the
-//    previous product holds row 4 g + r of its column -- exactly slot g of step r -- so
-//    probabilities never leave registers, and the other operand is row 4 g + r of the row-major
-//    tile in LDS, sixteen lanes on consecutive elements.
-// With a row pitch of 16 DB + 4 floats both access patterns touch all 64 banks once.
+// The k-slots may stand for any data as long as A and B agree, and so may the rows of A:
+//  * products over the head dimension (S = QK^T, dP = dO V^T): slot 8 g + e of step t is element
+//    32 t + 8 g + e, a 16-byte read per plane; MFMA row 4 g + r is tile row 4 r + lane_row(g) of a
+//    group of 16 (lane_row swaps the two bits of g);
+//  * products over keys or queries (PV, dS K, P^T dO, dS^T Q): the accumulator registers r of two
+//    such groups are slots r and 4 + r, so probabilities never leave registers, and the other
+//    operand comes from the row-major tile by two transposing reads per plane.
+// With that row order and a pitch of an odd number of 16-byte units both kinds of read touch every
+// bank once.
 //
-// One workgroup = 4 wavefronts x 16 rows (queries in forward and dQ, keys in dK/dV); the other side
-// streams through LDS in tiles of 32 rows, double buffered, staged through registers.  Bound by the
-// matrix pipe: 256 FLOP per cycle and CU (157 TFLOP/s nominal; a large fp32 library product reaches
-// 138 on this card).  A wavefront spends 32 DB x 16 matrix cycles per tile and product against about
-// 200 vector instructions, and needs few registers, so several wavefronts share a SIMD and hide each
-// other's vector work.  B4 S512 H16 D64 without a mask, forward: 51.5 us = 83 TFLOP/s (one thread per row
-// on plain FMAs: 686 us, 6.3 TFLOP/s); B2 S2048 H16 D128 696 us = 99 TFLOP/s.
+// A workgroup owns 16 rows per wavefront (queries in forward and dQ, keys in dK/dV); the other side
+// streams through LDS in tiles of 32 rows, double buffered, staged through registers and split into its
+// planes on the way.  Per 16 x 32 scores and wavefront (forward, head_dim 64) that is 768 matrix
+// cycles -- the fp32 matrix instructions take 2048 --, about 200 vector instructions (half of them
+// the splitting of the tile and of the probabilities) and 24 KB of LDS reads: no one of the three
+// binds, their sum does.  fp32 matrix instructions in the same layout -> these: forward B4 S512
+// H16 D64 50.9 -> 33.2 us (83 -> 129 TFLOP/s), B16 S512 H16 D64 184 -> 103, B2 S2048 H16 D128 701 -> 356
+// (193 TFLOP/s; the fp32 instructions stop at 157); forward and backward B4 S512 H16 D64 210 -> 125, B4
+// S1024 H8 D80 554 -> 337, B1 S1024 H8 D128 causal 233 -> 146.  Errors against 64 bits (2-norm) at B4
+// S512 H16 D64: output 4.1e-7 -> 2.0e-7, gradients 6.2e-7 -> 5.3e-7; at B2 S2048 H16 D128 output
+// 9.3e-7 -> 3.7e-7.
+//
 //
 // Reference semantics: slapo/op/attention.py:163-181 (attention_bmk) and its autograd.
 #include "attn_common.h"
@@ -30,52 +39,137 @@ using namespace slapo;
 
 namespace {
 
-constexpr int kWaves = 4;
-constexpr int kThreads = kWaves * 64;
-constexpr int kRows = kWaves * 16;  // rows owned by a workgroup
-constexpr int kTile = 32;           // streamed rows per LDS tile
-// Forward calls that give a CU two workgroups at most run kHalves = 2: eight wavefronts, two per 16
-// query rows, each with one half of a tile of 64 keys and a softmax state of its own, merged at the end
-// through LDS.  Four wavefronts per SIMD then hide the vector work of a launch that has no more rows
-// (B4 S512 H16 D64 56.6 -> 51.5 us, D80 83.7 -> 72.6, B1 S4096 H2 D64 causal 113 -> 102); with more
-// workgroups the other ones do that and the merge only costs (B16 S512 H16 D64 184 -> 191 us, B2 S2048
-// H16 D128 696 -> 750).
-constexpr int64_t kHalvesBlocks = 512;  // two for each of 256 CUs
+constexpr int kTile = 32;  // streamed rows per LDS tile
+// Wavefronts per workgroup (16 rows each).  Eight split a tile once for 128 rows where four do it for
+// 64, and let head_dim 128, whose 104 KB of tiles leave a CU one workgroup, have two wavefronts per
+// SIMD (B1 S1024 H8 D128 causal, forward and backward: 146 against 198 us).  At head_dim 65-96
+// two workgroups of four fit a CU and balance causal and windowed calls better (B2 S1000 H6 D96
+// window 200: 87 against 127 us; without a mask equal).  Up to 64 it takes workgroups enough:
+constexpr int64_t kWideFwd = 128;   // in units of 64 rows: forward B3 S500 H12 D64 (288) 32.8 against
+                                    // 34.8 us, below that kHalves
+constexpr int64_t kWideBwd = 512;   // B4 S512 H16 D64 (512) 125 against 132 us forward and backward,
+                                    // B2 S777 H12 D64 (312) padded, p 0.1: 305 against 283
+// Smaller forward calls up to head_dim 64 run kHalves = 2: eight wavefronts, two per 16 query rows, each
+// with one half of a tile of 64 keys and a softmax state of its own, merged at the end through LDS (B1
+// S256 H8 D64, 32 units: 12.3 us against 15.6 with four wavefronts and 18.1 with eight times 16 rows).
+// LDS and registers leave a SIMD four of a forward's wavefronts up to head_dim 64, else two.
+constexpr int per_simd(int db, int waves) { return db <= 4 && waves >= 8 ? 4 : 2; }
+constexpr float kReserve = 8.0f;  // of the softmax reference above the maximum, log2 units
 
-__device__ __forceinline__ f32x4_t mma(float a, float b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+typedef Mma<bf16_t>::frag frag_t;
+__device__ __forceinline__ f32x4_t splat(float v) { return f32x4_t{v, v, v, v}; }
+// Eight fp32 numbers as their bf16 parts.
+struct Split8 {
+    u32x4_t h, m, l;
+};
+__device__ __forceinline__ frag_t frag(u32x4_t v) { return __builtin_bit_cast(frag_t, v); }
+// c (and, in `small`, the five smaller products) += A B of fp32 operands
+__device__ __forceinline__ void mma(const Split8& a, const Split8& b, f32x4_t& c, f32x4_t& small) {
+    small = Mma<bf16_t>::mma16(frag(a.l), frag(b.h), small);
+    small = Mma<bf16_t>::mma16(frag(a.h), frag(b.l), small);
+    small = Mma<bf16_t>::mma16(frag(a.m), frag(b.m), small);
+    small = Mma<bf16_t>::mma16(frag(a.m), frag(b.h), small);
+    small = Mma<bf16_t>::mma16(frag(a.h), frag(b.m), small);
+    c = Mma<bf16_t>::mma16(frag(a.h), frag(b.h), c);
 }
+__device__ __forceinline__ float low_half(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
+__device__ __forceinline__ float high_half(uint32_t v) {
+    return __builtin_bit_cast(float, v & 0xFFFF0000u);
+}
+// The parts of two finite numbers below 3.38e38 (NaN: stays one)
+__device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = pack2<bf16_t>(x, y);
+    x -= low_half(h), y -= high_half(h);
+    m = pack2<bf16_t>(x, y);
+    l = pack2<bf16_t>(x - low_half(m), y - high_half(m));
+}
+// ... of any two.  What bf16 would round to infinity is cut instead; an infinity stands in the last
+// part alone, which meets nothing but the other operand's first one (its rest may have any sign).
+__device__ __forceinline__ void split2_any(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const float v[2] = {x, y};
+    float hi[2], mid[2], lo[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const bool inf = __builtin_isinf(v[e]);
+        const float finite = inf ? 0.f : v[e];
+        hi[e] = low_half(pack2<bf16_t>(finite, 0.f));
+        if (__builtin_isinf(hi[e])) hi[e] = high_half(__builtin_bit_cast(uint32_t, finite));
+        mid[e] = low_half(pack2<bf16_t>(finite - hi[e], 0.f));
+        lo[e] = inf ? v[e] : finite - hi[e] - mid[e];
+    }
+    h = pack2<bf16_t>(hi[0], hi[1]);
+    m = pack2<bf16_t>(mid[0], mid[1]);
+    l = pack2<bf16_t>(lo[0], lo[1]);
+}
+__device__ __forceinline__ void split4(const f32x4_t& v, uint32_t* h, uint32_t* m, uint32_t* l) {
+    const float top = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(top > 3.38e38f) != 0, 0)) {
+        split2_any(v[0], v[1], h[0], m[0], l[0]);
+        split2_any(v[2], v[3], h[1], m[1], l[1]);
+    } else {
+        split2(v[0], v[1], h[0], m[0], l[0]);
+        split2(v[2], v[3], h[1], m[1], l[1]);
+    }
+}
+// kSmall: probabilities, whose size needs no look
+template <bool kSmall = false>
+__device__ __forceinline__ Split8 split8(const f32x4_t& a, const f32x4_t& b) {
+    uint32_t h[4], m[4], l[4];
+    if constexpr (kSmall) {
+        split2(a[0], a[1], h[0], m[0], l[0]);
+        split2(a[2], a[3], h[1], m[1], l[1]);
+        split2(b[0], b[1], h[2], m[2], l[2]);
+        split2(b[2], b[3], h[3], m[3], l[3]);
+    } else {
+        split4(a, h, m, l);
+        split4(b, h + 2, m + 2, l + 2);
+    }
+    return {u32x4_t{h[0], h[1], h[2], h[3]}, u32x4_t{m[0], m[1], m[2], m[3]},
+            u32x4_t{l[0], l[1], l[2], l[3]}};
+}
+// Tile row (of a group of 16) of accumulator register r of lane-group g: 4 r + lane_row(g).
+__device__ __forceinline__ int lane_row(int g) { return (g & 1) * 2 + (g >> 1); }
 // Across the four lanes that share a column (l, l ^ 16, l ^ 32, l ^ 48)
+__device__ __forceinline__ void swap16(float v, float& even, float& odd) {
+    float a = v, b = v;  // the odd rows of 16 lanes of one against the even rows of the other
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    even = a, odd = b;
+}
 __device__ __forceinline__ float column_max(float v) {
-    v = fmaxf(v, __shfl_xor(v, 16, 64));
-    return fmaxf(v, __shfl_xor(v, 32, 64));
+    float a, b;
+    swap16(v, a, b);
+    return max_xor32(fmaxf(a, b));
 }
 __device__ __forceinline__ float column_sum(float v) {
-    v += __shfl_xor(v, 16, 64);
-    return v + __shfl_xor(v, 32, 64);
+    float a, b;
+    swap16(v, a, b);
+    return sum_xor32(a + b);
 }
 
 __device__ __forceinline__ float bias_at(const AttnArgs& a, int b, int h, int i, int j) {
-    return canonical_bias(bias_load(
+    return bias_log2(bias_load(
         a, b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] + (int64_t)j * a.bs[3]));
 }
 
-// LDS row pitch of a tile, in floats
+// Steps of 32 over the head dimension, and the LDS row pitch of a tile's plane in elements
 template <int DB>
-constexpr int kPitchOf = 16 * DB + 4;
+constexpr int kStepsOf = (DB + 1) / 2;
+template <int DB>
+constexpr int kPitchOf = 32 * kStepsOf<DB> + 8;
 
 // Builds of each kernel: kMode & 1 = with a bias, kMode & 2 = with dropout, for tensors whose rows are
 // 16-byte aligned with d % 4 == 0; kGeneral serves every other layout element by element and decides
 // about bias and dropout when it runs.
 constexpr int kGeneral = 4;
 
-// A tile of kTileRows rows of 16 DB floats on its way from global memory to LDS.  Rows past the end are
-// clamped, columns past d read as zero.
-template <int DB, bool kVec, int kTileRows = kTile, int kBlock = kThreads>
+// A tile of kTileRows rows on its way from global memory to LDS, where it stands as three bf16 planes.
+// Rows past the end are clamped, columns past d read as zero.
+template <int DB, bool kVec, int kTileRows, int kBlock>
 struct Tile {
     static constexpr int kPitch = kPitchOf<DB>;
-    static constexpr int kElems = kTileRows * kPitch;
-    static constexpr int kPerRow = 4 * DB;
+    static constexpr int kPlane = kTileRows * kPitch;
+    static constexpr int kElems = 3 * kPlane;
+    static constexpr int kPerRow = 8 * kStepsOf<DB>;
     static constexpr int kChunks = kTileRows * kPerRow;
     static constexpr int kPer = (kChunks + kBlock - 1) / kBlock;
     f32x4_t r[kPer];
@@ -96,30 +190,40 @@ struct Tile {
             }
         }
     }
-    __device__ __forceinline__ void store(float* lds, int row0, int n_rows, int d) const {
+    __device__ __forceinline__ void store(bf16_t* lds, int row0, int n_rows, int d) {
+        if (row0 + kTileRows > n_rows || d < 32 * kStepsOf<DB>) {  // uniform
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const int c = threadIdx.x + u * kBlock;
+                const int row = c / kPerRow, col = 4 * (c % kPerRow);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (row0 + row >= n_rows || col + e >= d) r[u][e] = 0.f;
+            }
+        }
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
             const int c = threadIdx.x + u * kBlock;
             if (kChunks % kBlock != 0 && c >= kChunks) continue;
-            const int row = c / kPerRow, col = 4 * (c % kPerRow);
-            f32x4_t v = r[u];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (row0 + row >= n_rows || col + e >= d) v[e] = 0.f;
-            *reinterpret_cast<f32x4_t*>(lds + row * kPitch + col) = v;
+            uint32_t h[2], m[2], l[2];
+            split4(r[u], h, m, l);
+            bf16_t* p = lds + c / kPerRow * kPitch + 4 * (c % kPerRow);
+            *reinterpret_cast<u32x2_t*>(p) = u32x2_t{h[0], h[1]};
+            *reinterpret_cast<u32x2_t*>(p + kPlane) = u32x2_t{m[0], m[1]};
+            *reinterpret_cast<u32x2_t*>(p + 2 * kPlane) = u32x2_t{l[0], l[1]};
         }
     }
 };
 
-// Register fragments of row `row` (16 DB elements, 4 per step group): element 16 t + 4 g + e.
-template <bool kVec, int DB>
-__device__ __forceinline__ void load_frags(f32x4_t (&f)[DB], const float* base, int64_t stride,
-                                           int row, int n_rows, int d, float scale) {
+// Row `row` of a tensor as this lane holds it: elements 32 t + 8 g .. + 7 in f[2 t], f[2 t + 1].
+template <bool kVec, int KS>
+__device__ __forceinline__ void load_row(f32x4_t (&f)[2 * KS], const float* base, int64_t stride,
+                                         int row, int n_rows, int d, float scale) {
     const int g = (threadIdx.x & 63) >> 4;
     const float* p = base + (int64_t)min(row, n_rows - 1) * stride;
 #pragma unroll
-    for (int t = 0; t < DB; ++t) {
-        const int col = 16 * t + 4 * g;
+    for (int t = 0; t < 2 * KS; ++t) {
+        const int col = 32 * (t >> 1) + 8 * g + 4 * (t & 1);
         if constexpr (kVec) {
             f[t] = *reinterpret_cast<const f32x4_t*>(p + min(col, d - 4));
         } else {
@@ -131,32 +235,48 @@ __device__ __forceinline__ void load_frags(f32x4_t (&f)[DB], const float* base, 
             f[t][e] = (row < n_rows && col + e < d) ? f[t][e] * scale : 0.f;
     }
 }
+template <int KS>
+__device__ __forceinline__ void split_row(Split8 (&f)[KS], const f32x4_t (&v)[2 * KS]) {
+#pragma unroll
+    for (int t = 0; t < KS; ++t) f[t] = split8(v[2 * t], v[2 * t + 1]);
+}
 
-// c += A B over the head dimension: A = 16 tile rows from row `r0` on, B = this lane's fragments.
-template <int DB>
-__device__ __forceinline__ f32x4_t dot_rows(const float* tile, int r0, const f32x4_t (&f)[DB]) {
-    const int lane = threadIdx.x & 63;
-    const float* p = tile + (r0 + (lane & 15)) * kPitchOf<DB> + 4 * (lane >> 4);
+// small + A B over the head dimension: A = 16 tile rows from row `r0` on, B = this lane's fragments.
+template <int DB, int kPlane>
+__device__ __forceinline__ f32x4_t dot_rows(const bf16_t* tile, int r0,
+                                            const Split8 (&f)[kStepsOf<DB>],
+                                            f32x4_t small = f32x4_t{0.f, 0.f, 0.f, 0.f}) {
+    const int lane = threadIdx.x & 63, i = lane & 15;
+    const bf16_t* p = tile + (r0 + 4 * (i & 3) + lane_row(i >> 2)) * kPitchOf<DB> + 8 * (lane >> 4);
     f32x4_t c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < DB; ++t) {
-        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(p + 16 * t);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c = mma(v[e], f[t][e], c);
+    for (int t = 0; t < kStepsOf<DB>; ++t) {
+        const bf16_t* q = p + 32 * t;
+        const Split8 v = {*reinterpret_cast<const u32x4_t*>(q),
+                          *reinterpret_cast<const u32x4_t*>(q + kPlane),
+                          *reinterpret_cast<const u32x4_t*>(q + 2 * kPlane)};
+        mma(v, f[t], c, small);
     }
-    return c;
+    return c + small;
 }
-// acc[x] += A B over the 16 tile rows from r0 on: A = columns 16 x .. 16 x + 15 of those rows
-// (transposed), B = w, register r of it being row 4 g + r of this lane's column.
-template <int DB>
-__device__ __forceinline__ void add_rows(const float* tile, int r0, const f32x4_t& w,
-                                         f32x4_t (&acc)[DB]) {
+// acc[x] += A B over the 32 tile rows: A = columns 16 x .. 16 x + 15 of those rows (transposed), B =
+// w, slots r and 4 + r of it being rows 4 r + lane_row(g) and 16 more of this lane's column.
+template <int DB, int kPlane>
+__device__ __forceinline__ void add_rows(const bf16_t* tile, const Split8& w, f32x4_t (&acc)[DB],
+                                         f32x4_t (&small)[DB]) {
     const int lane = threadIdx.x & 63;
-    const float* p = tile + (r0 + 4 * (lane >> 4)) * kPitchOf<DB> + (lane & 15);
+    const bf16_t* p = tile +
+                      (4 * ((lane & 15) >> 2) + lane_row(lane >> 4)) * kPitchOf<DB> + 4 * (lane & 3);
+    auto columns = [&](const bf16_t* q) __attribute__((always_inline)) {
+        const u32x2_t a = lds_read_tr16(q), b = lds_read_tr16(q + 16 * kPitchOf<DB>);
+        return u32x4_t{a.x, a.y, b.x, b.y};
+    };
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int x = 0; x < DB; ++x) acc[x] = mma(p[r * kPitchOf<DB> + 16 * x], w[r], acc[x]);
+    for (int x = 0; x < DB; ++x) {
+        const bf16_t* q = p + 16 * x;
+        const Split8 v = {columns(q), columns(q + kPlane), columns(q + 2 * kPlane)};
+        mma(v, w, acc[x], small[x]);
+    }
 }
 
 // Writes this lane's column of acc (element 16 x + 4 g + r in acc[x][r]) times mul as row `row`.
@@ -176,23 +296,37 @@ __device__ __forceinline__ void store_row(const f32x4_t (&acc)[DB], float mul, f
     }
 }
 
-// Keep bits (bit r: key j + r) of query i and the four keys from j on, j % 4 == 0.
+// Keep bits (bit r: key j + r) of query i and the kKeys keys from j on, j % 4 == 0.
+template <int kKeys>
 __device__ __forceinline__ uint32_t keep_keys(const AttnArgs& a, int bh, int i, int j) {
     const uint64_t e = ((uint64_t)bh * a.sq + (uint64_t)i) * (uint64_t)a.sk + (uint64_t)j;
     if (i >= a.sq || j >= a.sk) return 0;
-    if (a.dropout == 1) return dropout_keep4_pow2(a.rng, e >> 2);
-    return dropout_keep_any(a.rng, e, min(4, a.sk - j));
+    if (a.dropout != 1)
+        return dropout_keep_run(a.rng, e, min(kKeys, a.sk - j)) & ((1u << kKeys) - 1u);
+    uint32_t bits = dropout_keep4_pow2(a.rng, e >> 2);
+#pragma unroll
+    for (int k = 4; k < kKeys; k += 4)
+        if (j + k < a.sk) bits |= dropout_keep4_pow2(a.rng, (e + (uint64_t)k) >> 2) << k;
+    return bits;
+}
+// Keep bits of query i (the lane's column) and the 32 keys from j0 on: a Philox block covers four
+// consecutive keys, so each of the four lanes of a query draws eight keys and they exchange them.
+__device__ __forceinline__ uint32_t keep_keys32(const AttnArgs& a, int bh, int i, int j0) {
+    const int at = 8 * ((threadIdx.x & 63) >> 4);
+    uint32_t bits = keep_keys<8>(a, bh, i, j0 + at) << at;
+    bits |= (uint32_t)__shfl_xor((int)bits, 16, 64);
+    return bits | (uint32_t)__shfl_xor((int)bits, 32, 64);
 }
 template <int kCtrl>
 __device__ __forceinline__ uint32_t dpp(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xF, 0xF, false);
 }
-// The same for a lane whose registers are the queries i .. i + 3 and whose key is j0 + l % 16 (bit
-// r: query i + r): a Philox block covers four consecutive keys, i.e. the four lanes of a quad, so
-// lane c of a quad draws the block of query i + c and the quad exchanges them.
+// The same for a lane whose registers are the queries i + 4 r and whose key is j0 + l % 16 (bit r:
+// query i + 4 r): a Philox block covers four consecutive keys, i.e. the four lanes of a quad, so
+// lane c of a quad draws the block of query i + 4 c and the quad exchanges them.
 __device__ __forceinline__ uint32_t keep_queries(const AttnArgs& a, int bh, int i, int j0) {
     const int c = threadIdx.x & 3, j = j0 + (threadIdx.x & 15);
-    const uint32_t mine = keep_keys(a, bh, i + c, j - c);
+    const uint32_t mine = keep_keys<4>(a, bh, i + 4 * c, j - c);
     return ((dpp<0x00>(mine) >> c) & 1u) | (((dpp<0x55>(mine) >> c) & 1u) << 1) |
            (((dpp<0xAA>(mine) >> c) & 1u) << 2) | (((dpp<0xFF>(mine) >> c) & 1u) << 3);
 }
@@ -202,7 +336,8 @@ __device__ __forceinline__ uint32_t keep_queries(const AttnArgs& a, int bh, int 
 struct Place {
     int b, h, bh, row0, split;
     int64_t part_row0;  // of the split's partial result, rows of all (batch, head) pairs
-    __device__ __forceinline__ Place(const AttnArgs& a, int n_rows, bool last_first) {
+    // kRows rows per workgroup
+    __device__ __forceinline__ Place(const AttnArgs& a, int n_rows, int kRows, bool last_first) {
         const int n_bh = a.batch * a.heads;
         const int n_t = (n_rows + kRows - 1) / kRows;
         bh = (int)(blockIdx.x % (unsigned)n_bh);
@@ -221,23 +356,21 @@ struct Visible {
     __device__ __forceinline__ bool operator()(int c) const { return c >= lo && c <= hi; }
 };
 // the run starts at key `first` of query i
-__device__ __forceinline__ Visible keys_of_query(const AttnArgs& a, int i, int first, bool masked) {
-    if (!masked) return {0, kTile};
+__device__ __forceinline__ Visible keys_of_query(const AttnArgs& a, int i, int first) {
     return {(a.window > 0 ? i - a.window + 1 : 0) - first,
             (a.causal ? min(i, a.sk - 1) : a.sk - 1) - first};
 }
 // the run starts at query `first` of key j
-__device__ __forceinline__ Visible queries_of_key(const AttnArgs& a, int j, int first,
-                                                  bool masked) {
-    if (!masked) return {0, kTile};
+__device__ __forceinline__ Visible queries_of_key(const AttnArgs& a, int j, int first) {
     return {(a.causal ? j : 0) - first,
             (a.window > 0 ? min(j + a.window, a.sq) - 1 : a.sq - 1) - first};
 }
 
-template <int DB, int kMode, int kHalves>
-__global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void attn_f32_fwd_kernel(
-    const AttnArgs a_in) {
-    constexpr int kFwdThreads = kHalves * kThreads, kFwdTile = kHalves * kTile;
+template <int DB, int kMode, int kWaves, int kHalves>
+__global__ __launch_bounds__(kHalves* kWaves * 64, per_simd(DB, kHalves* kWaves)) void
+attn_f32_fwd_kernel(const AttnArgs a_in) {
+    constexpr int kFwdThreads = kHalves * kWaves * 64, kFwdTile = kHalves * kTile;
+    constexpr int kRows = 16 * kWaves, KS = kStepsOf<DB>;
     AttnArgs a = a_in;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
@@ -245,14 +378,15 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
     if (dropout) resolve_device_state(a.rng);
     extern __shared__ __align__(16) float lds[];
     typedef Tile<DB, kVec, kFwdTile, kFwdThreads> tile_t;
-    constexpr int kElems = tile_t::kElems;
-    float* ks = lds;               // K[2][tile]
-    float* vs = lds + 2 * kElems;  // V[2][tile]
-    const Place at(a, a.sq, true);
+    constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
+    bf16_t* ks = reinterpret_cast<bf16_t*>(lds);  // K[2][tile]
+    bf16_t* vs = ks + 2 * kElems;                 // V[2][tile]
+    const Place at(a, a.sq, kRows, true);
     const int lane = threadIdx.x & 63, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wq0 = at.row0 + 16 * (wave % kWaves);
     const int half = wave / kWaves;  // of every tile's keys
+    const int row_g = lane_row(g);
     const int i = wq0 + (lane & 15);
     const float* qp = reinterpret_cast<const float*>(a.q) + at.b * a.qs[0] + at.h * a.qs[2];
     const float* kp = reinterpret_cast<const float*>(a.k) + at.b * a.ks[0] + at.h * a.ks[2];
@@ -265,13 +399,18 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
     if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
     tile_t kt, vt;
-    f32x4_t qf[DB], o[DB];
+    Split8 qf[KS];
+    f32x4_t o[DB], o_small[DB];  // (mma)
     kt.load(kp, a.ks[1], t_lo * kFwdTile, a.sk, a.d);
     vt.load(vp, a.vs[1], t_lo * kFwdTile, a.sk, a.d);
-    load_frags<kVec>(qf, qp, a.qs[1], i, a.sq, a.d, a.scale);
+    {
+        f32x4_t q[2 * KS];
+        load_row<kVec, KS>(q, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
+        split_row<KS>(qf, q);
+    }
 #pragma unroll
-    for (int x = 0; x < DB; ++x) o[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;  // l: this lane's share of the row sum
+    for (int x = 0; x < DB; ++x) o[x] = o_small[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;  // m: in log2 units, as the scores are; l: this lane's share of the row sum
     kt.store(ks, t_lo * kFwdTile, a.sk, a.d);
     vt.store(vs, t_lo * kFwdTile, a.sk, a.d);
     __syncthreads();
@@ -280,7 +419,7 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
         const int part = half * kTile * tile_t::kPitch;
-        const float *kb = ks + slot * kElems + part, *vb = vs + slot * kElems + part;
+        const bf16_t *kb = ks + slot * kElems + part, *vb = vs + slot * kElems + part;
         if (t + 1 < t_hi) {
             kt.load(kp, a.ks[1], (t + 1) * kFwdTile, a.sk, a.d);
             vt.load(vp, a.vs[1], (t + 1) * kFwdTile, a.sk, a.d);
@@ -290,44 +429,53 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
                             (a.window <= 0 || wq0 - (j0 + kTile - 1) < a.window);
         if (active) {  // uniform per wavefront
             f32x4_t s[2];
-            s[0] = dot_rows<DB>(kb, 0, qf);
-            s[1] = dot_rows<DB>(kb, 16, qf);
+            s[0] = dot_rows<DB, kPlane>(kb, 0, qf);
+            s[1] = dot_rows<DB, kPlane>(kb, 16, qf);
             const bool masked = j0 + kTile > a.sk || (a.causal && j0 + kTile - 1 > wq0) ||
                                 (a.window > 0 && wq_last - j0 >= a.window);
-            const Visible vis = keys_of_query(a, i, j0 + 4 * g, masked);
+            if (has_bias) {
+#pragma unroll
+                for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        s[h2][r] += bias_at(a, at.b, at.h, min(i, a.sq - 1),
+                                            min(j0 + 16 * h2 + 4 * r + row_g, a.sk - 1));
+            }
+            if (masked) {  // uniform
+                const Visible vis = keys_of_query(a, i, j0 + row_g);
+#pragma unroll
+                for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (!vis(16 * h2 + 4 * r)) s[h2][r] = -INFINITY;
+            }
             float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx = fmaxf(mx, fmaxf(s[0][r], s[1][r]));
+            mx = column_max(mx);
+            // moved lazily, to kReserve above the maximum: probabilities stay at or below 1
+            const bool move = mx > m;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(move) != 0, 0)) {
+                const float m_new = move ? mx + kReserve : m;
+                const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - m_new);
+                m = m_new;
+                l *= alpha;
+#pragma unroll
+                for (int x = 0; x < DB; ++x) o[x] *= alpha, o_small[x] *= alpha;
+            }
+            const float m_ref = m == -INFINITY ? 0.f : m;
+            uint32_t bits = 0u;
+            if (dropout) bits = keep_keys32(a, at.bh, i, j0) >> row_g;
 #pragma unroll
             for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int j = j0 + 16 * h2 + 4 * g + r;
-                    if (has_bias)
-                        s[h2][r] += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
-                    s[h2][r] = vis(16 * h2 + r) ? s[h2][r] : -INFINITY;
-                    mx = fmaxf(mx, s[h2][r]);
-                }
-            const float m_new = fmaxf(m, column_max(mx));
-            if (__builtin_amdgcn_ballot_w64(m_new > m) != 0) {
-                const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
-                m = m_new;
-                l *= alpha;
-#pragma unroll
-                for (int x = 0; x < DB; ++x) o[x] *= alpha;
-            }
-            const float m_ref = m == -INFINITY ? 0.f : m;
-#pragma unroll
-            for (int h2 = 0; h2 < 2; ++h2) {
-                uint32_t bits = 0xFu;
-                if (dropout) bits = keep_keys(a, at.bh, i, j0 + 16 * h2 + 4 * g);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float p = expf(s[h2][r] - m_ref);
+                    float p = fast_exp2(s[h2][r] - m_ref);
                     l += p;
-                    if (dropout) p = (bits >> r) & 1u ? p * a.rng.inv_keep : 0.f;
+                    if (dropout) p = (bits >> (16 * h2 + 4 * r)) & 1u ? p * a.rng.inv_keep : 0.f;
                     s[h2][r] = p;
                 }
-                add_rows<DB>(vb, 16 * h2, s[h2], o);
-            }
+            add_rows<DB, kPlane>(vb, split8<true>(s[0], s[1]), o, o_small);
         }
         if (t + 1 < t_hi) {
             kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d);
@@ -336,6 +484,8 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
         __syncthreads();
     }
     float l_tot = column_sum(l);
+#pragma unroll
+    for (int x = 0; x < DB; ++x) o[x] += o_small[x];
     if constexpr (kHalves == 2) {
         // the second half's state joins the first's through LDS (every wavefront is past the loop's
         // last barrier): lane by lane, the two hold the same rows and columns
@@ -350,8 +500,8 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
         __syncthreads();
         if (half != 0) return;
         const float m2 = state[4 * DB * 64], m_all = fmaxf(m, m2);
-        const float w1 = m == -INFINITY ? 0.f : expf(m - m_all);
-        const float w2 = m2 == -INFINITY ? 0.f : expf(m2 - m_all);
+        const float w1 = m == -INFINITY ? 0.f : fast_exp2(m - m_all);
+        const float w2 = m2 == -INFINITY ? 0.f : fast_exp2(m2 - m_all);
         l_tot = l_tot * w1 + state[(4 * DB + 1) * 64] * w2;
         m = m_all;
 #pragma unroll
@@ -374,24 +524,27 @@ __global__ __launch_bounds__(kHalves* kThreads, DB <= 4 ? kHalves + 2 : 2) void 
     store_row<kVec>(o, 1.0f / l_tot, op, a.d);
     // a row that saw nothing but masked keys: see canonical_bias
     if (g == 0)
-        a.lse[(int64_t)at.bh * a.sq + i] = m == -kFltMax ? l_tot * kMaskedRowLse : m + logf(l_tot);
+        a.lse[(int64_t)at.bh * a.sq + i] = m == -kFltMax ? l_tot * kMaskedRowLse
+                                                         : __builtin_fmaf(m, kLn2, logf(l_tot));
 }
 
 // dQ: dq_i = scale * sum_j ds_ij k_j,  ds = p (dp - delta),  dp = dO_i . v_j.  Also computes
 // delta = rowsum(dO * O) of its rows and stores it for the dK / dV kernel, which runs second.
-template <int DB, int kMode>
-__global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs a_in) {
+template <int DB, int kMode, int kWaves>
+__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnArgs a_in) {
+    constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves, KS = kStepsOf<DB>;
     AttnArgs a = a_in;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
     if (dropout) resolve_device_state(a.rng);
     extern __shared__ __align__(16) float lds[];
-    constexpr int kElems = Tile<DB, kVec>::kElems;
-    float* ks = lds;
-    float* vs = lds + 2 * kElems;
-    const Place at(a, a.sq, true);
-    const int lane = threadIdx.x & 63, g = lane >> 4;
+    typedef Tile<DB, kVec, kTile, kThreads> tile_t;
+    constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
+    bf16_t* ks = reinterpret_cast<bf16_t*>(lds);
+    bf16_t* vs = ks + 2 * kElems;
+    const Place at(a, a.sq, kRows, true);
+    const int lane = threadIdx.x & 63, g = lane >> 4, row_g = lane_row(g);
     const int wq0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = wq0 + (lane & 15);
     const float* qp = reinterpret_cast<const float*>(a.q) + at.b * a.qs[0] + at.h * a.qs[2];
@@ -406,26 +559,30 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
     int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
     if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
-    Tile<DB, kVec> kt, vt;
-    f32x4_t qf[DB], gf[DB], dq[DB];
+    tile_t kt, vt;
+    Split8 qf[KS], gf[KS];
+    f32x4_t dq[DB];
     kt.load(kp, a.ks[1], t_lo * kTile, a.sk, a.d);
     vt.load(vp, a.vs[1], t_lo * kTile, a.sk, a.d);
-    load_frags<kVec>(qf, qp, a.qs[1], i, a.sq, a.d, a.scale);
-    load_frags<kVec>(gf, gp, a.os[1], i, a.sq, a.d, 1.0f);
     float delta = 0.f;
     {
-        f32x4_t of[DB];
-        load_frags<kVec>(of, op, a.os[1], i, a.sq, a.d, 1.0f);
+        f32x4_t row[2 * KS], out[2 * KS];
+        load_row<kVec, KS>(row, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
+        split_row<KS>(qf, row);
+        load_row<kVec, KS>(row, gp, a.os[1], i, a.sq, a.d, 1.0f);
+        load_row<kVec, KS>(out, op, a.os[1], i, a.sq, a.d, 1.0f);
+        split_row<KS>(gf, row);
 #pragma unroll
-        for (int x = 0; x < DB; ++x) {
-            dq[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int x = 0; x < 2 * KS; ++x)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) delta = __builtin_fmaf(of[x][e], gf[x][e], delta);
-        }
+            for (int e = 0; e < 4; ++e) delta = __builtin_fmaf(out[x][e], row[x][e], delta);
         delta = column_sum(delta);
+#pragma unroll
+        for (int x = 0; x < DB; ++x) dq[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
     const float lse_raw = i < a.sq ? a.lse[(int64_t)at.bh * a.sq + i] : 0.f;
-    const float lse = lse_reference(lse_raw, 1.0f), inv_n = lse_row_factor(lse_raw);
+    const float lse = lse_reference(lse_raw, kLog2e), inv_n = lse_row_factor(lse_raw);
+    const float rest = masked_row_lse(lse_raw) ? 0.f : __builtin_fmaf(lse_raw, -kLog2e, lse);
     if (g == 0 && i < a.sq) a.delta[(int64_t)at.bh * a.sq + i] = delta;
     kt.store(ks, t_lo * kTile, a.sk, a.d);
     vt.store(vs, t_lo * kTile, a.sk, a.d);
@@ -434,7 +591,7 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
     const int wq_last = min(wq0 + 15, a.sq - 1);
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
-        const float *kb = ks + slot * kElems, *vb = vs + slot * kElems;
+        const bf16_t *kb = ks + slot * kElems, *vb = vs + slot * kElems;
         if (t + 1 < t_hi) {
             kt.load(kp, a.ks[1], (t + 1) * kTile, a.sk, a.d);
             vt.load(vp, a.vs[1], (t + 1) * kTile, a.sk, a.d);
@@ -445,24 +602,34 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
         if (active) {
             const bool masked = j0 + kTile > a.sk || (a.causal && j0 + kTile - 1 > wq0) ||
                                 (a.window > 0 && wq_last - j0 >= a.window);
-            const Visible vis = keys_of_query(a, i, j0 + 4 * g, masked);
+            uint32_t bits = 0u;
+            if (dropout) bits = keep_keys32(a, at.bh, i, j0) >> row_g;
+            f32x4_t ds[2];
 #pragma unroll
             for (int h2 = 0; h2 < 2; ++h2) {
-                f32x4_t s = dot_rows<DB>(kb, 16 * h2, qf);
-                f32x4_t dp = dot_rows<DB>(vb, 16 * h2, gf);
-                uint32_t bits = 0xFu;
-                if (dropout) bits = keep_keys(a, at.bh, i, j0 + 16 * h2 + 4 * g);
+                const f32x4_t s = dot_rows<DB, kPlane>(kb, 16 * h2, qf, splat(rest));
+                const f32x4_t dp = dot_rows<DB, kPlane>(vb, 16 * h2, gf);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int j = j0 + 16 * h2 + 4 * g + r;
+                    const int j = j0 + 16 * h2 + 4 * r + row_g;
+                    float x = s[r], y = dp[r];
                     if (has_bias)
-                        s[r] += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
-                    if (dropout) dp[r] = (bits >> r) & 1u ? dp[r] * a.rng.inv_keep : 0.f;
-                    const float ds = expf(s[r] - lse) * inv_n * (dp[r] - delta);
-                    s[r] = vis(16 * h2 + r) ? ds : 0.f;
+                        x += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
+                    if (dropout) y = (bits >> (16 * h2 + 4 * r)) & 1u ? y * a.rng.inv_keep : 0.f;
+                    y -= delta;
+                    if (has_bias) y *= inv_n;  // (1 without a bias)
+                    ds[h2][r] = fast_exp2(x - lse) * y;
                 }
-                add_rows<DB>(kb, 16 * h2, s, dq);
             }
+            if (masked) {  // uniform
+                const Visible vis = keys_of_query(a, i, j0 + row_g);
+#pragma unroll
+                for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (!vis(16 * h2 + 4 * r)) ds[h2][r] = 0.f;
+            }
+            add_rows<DB, kPlane>(kb, split8(ds[0], ds[1]), dq, dq);
         }
         if (t + 1 < t_hi) {
             kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d);
@@ -482,20 +649,24 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dq_kernel(const AttnArgs
 
 // dK and dV: a wavefront owns 16 keys, queries stream through LDS.
 //   dv_j = sum_i pdrop_ij dO_i          dk_j = scale * sum_i ds_ij q_i
-template <int DB, int kMode>
-__global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArgs a_in) {
+template <int DB, int kMode, int kWaves>
+__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const AttnArgs a_in) {
+    constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves, KS = kStepsOf<DB>;
     AttnArgs a = a_in;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
     if (dropout) resolve_device_state(a.rng);
     extern __shared__ __align__(16) float lds[];
-    constexpr int kElems = Tile<DB, kVec>::kElems;
-    float* qs = lds;
-    float* gs = lds + 2 * kElems;
-    float* rows = lds + 4 * kElems;  // [2][3][kTile]: lse reference, its factor, delta
-    const Place at(a, a.sk, false);
-    const int lane = threadIdx.x & 63, g = lane >> 4;
+    typedef Tile<DB, kVec, kTile, kThreads> tile_t;
+    constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
+    bf16_t* qs = reinterpret_cast<bf16_t*>(lds);
+    bf16_t* gs = qs + 2 * kElems;
+    // [2][4][kTile]: lse reference and its rest, its factor, delta; rows in the order of the accumulators (row
+    // 16 h + 4 r + e at 16 h + 4 e + r)
+    float* rows = reinterpret_cast<float*>(gs + 2 * kElems);
+    const Place at(a, a.sk, kRows, false);
+    const int lane = threadIdx.x & 63, g = lane >> 4, row_g = lane_row(g);
     const int wk0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = wk0 + (lane & 15);
     const float* qp = reinterpret_cast<const float*>(a.q) + at.b * a.qs[0] + at.h * a.qs[2];
@@ -510,8 +681,9 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
     int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
     if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
 
-    Tile<DB, kVec> qt, gt;
-    f32x4_t kf[DB], vf[DB], dk[DB], dv[DB];
+    tile_t qt, gt;
+    Split8 kf[KS], vf[KS];
+    f32x4_t dk[DB], dv[DB];
     float lse_r = 0.f, delta_r = 0.f;  // thread x < kTile: row x of the tile on its way
     auto request = [&](int t) __attribute__((always_inline)) {
         qt.load(qp, a.qs[1], t * kTile, a.sq, a.d);
@@ -526,14 +698,22 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
         qt.store(qs + slot * kElems, t * kTile, a.sq, a.d);
         gt.store(gs + slot * kElems, t * kTile, a.sq, a.d);
         if (threadIdx.x < kTile) {
-            float* r = rows + slot * 3 * kTile + threadIdx.x;
-            r[0] = lse_reference(lse_r, 1.0f);
-            r[kTile] = lse_row_factor(lse_r);
+            const int x = threadIdx.x;
+            float* r = rows + slot * 4 * kTile + ((x & 16) | (x & 3) << 2 | (x >> 2 & 3));
+            const float lse = lse_reference(lse_r, kLog2e);
+            r[0] = lse;
+            r[kTile] = masked_row_lse(lse_r) ? 0.f : __builtin_fmaf(lse_r, -kLog2e, lse);
             r[2 * kTile] = delta_r;
+            r[3 * kTile] = lse_row_factor(lse_r);
         }
     };
-    load_frags<kVec>(kf, kp, a.ks[1], j, a.sk, a.d, a.scale);
-    load_frags<kVec>(vf, vp, a.vs[1], j, a.sk, a.d, 1.0f);
+    {
+        f32x4_t row[2 * KS];
+        load_row<kVec, KS>(row, kp, a.ks[1], j, a.sk, a.d, a.scale_log2);
+        split_row<KS>(kf, row);
+        load_row<kVec, KS>(row, vp, a.vs[1], j, a.sk, a.d, 1.0f);
+        split_row<KS>(vf, row);
+    }
 #pragma unroll
     for (int x = 0; x < DB; ++x) dk[x] = dv[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     if (t_lo < t_hi) {
@@ -545,8 +725,8 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
     const int wk_last = min(wk0 + 15, a.sk - 1);
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
-        const float *qb = qs + slot * kElems, *gb = gs + slot * kElems;
-        const float* rb = rows + slot * 3 * kTile;
+        const bf16_t *qb = qs + slot * kElems, *gb = gs + slot * kElems;
+        const float* rb = rows + slot * 4 * kTile;
         if (t + 1 < t_hi) request(t + 1);
         const int i0 = t * kTile;
         const bool active = wk0 < a.sk && (!a.causal || i0 + kTile - 1 >= wk0) &&
@@ -555,32 +735,40 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
             const bool masked = i0 + kTile > a.sq || wk0 + 16 > a.sk ||
                                 (a.causal && i0 < wk0 + 15) ||
                                 (a.window > 0 && i0 + kTile - 1 - wk0 >= a.window);
-            const Visible vis = queries_of_key(a, j, i0 + 4 * g, masked);
+            f32x4_t pd[2], ds[2];
 #pragma unroll
             for (int h2 = 0; h2 < 2; ++h2) {
-                f32x4_t s = dot_rows<DB>(qb, 16 * h2, kf);
-                f32x4_t dp = dot_rows<DB>(gb, 16 * h2, vf);
-                const int r0 = 16 * h2 + 4 * g;
+                const int r0 = 16 * h2 + 4 * row_g;
                 const f32x4_t lse = *reinterpret_cast<const f32x4_t*>(rb + r0);
-                const f32x4_t inv_n = *reinterpret_cast<const f32x4_t*>(rb + kTile + r0);
+                const f32x4_t rest = *reinterpret_cast<const f32x4_t*>(rb + kTile + r0);
                 const f32x4_t delta = *reinterpret_cast<const f32x4_t*>(rb + 2 * kTile + r0);
-                uint32_t bits = 0xFu;
-                if (dropout) bits = keep_queries(a, at.bh, i0 + r0, wk0);
-                f32x4_t pd;
+                const f32x4_t s = dot_rows<DB, kPlane>(qb, 16 * h2, kf, rest);
+                const f32x4_t dp = dot_rows<DB, kPlane>(gb, 16 * h2, vf);
+                uint32_t bits = 0u;
+                if (dropout) bits = keep_queries(a, at.bh, i0 + 16 * h2 + row_g, wk0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int i = i0 + r0 + r;
+                    const int i = i0 + 16 * h2 + 4 * r + row_g;
+                    float x = s[r];
                     if (has_bias)
-                        s[r] += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
-                    const float p = expf(s[r] - lse[r]) * inv_n[r];
+                        x += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
+                    float p = fast_exp2(x - lse[r]);
+                    if (has_bias) p *= rb[3 * kTile + r0 + r];  // (1 without a bias)
                     const float keep = dropout ? ((bits >> r) & 1u ? a.rng.inv_keep : 0.f) : 1.f;
-                    const bool seen = vis(16 * h2 + r);
-                    pd[r] = seen ? p * keep : 0.f;
-                    s[r] = seen ? p * (dp[r] * keep - delta[r]) : 0.f;
+                    pd[h2][r] = p * keep;
+                    ds[h2][r] = p * (dp[r] * keep - delta[r]);
                 }
-                add_rows<DB>(gb, 16 * h2, pd, dv);
-                add_rows<DB>(qb, 16 * h2, s, dk);
             }
+            if (masked) {  // uniform
+                const Visible vis = queries_of_key(a, j, i0 + row_g);
+#pragma unroll
+                for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (!vis(16 * h2 + 4 * r)) pd[h2][r] = ds[h2][r] = 0.f;
+            }
+            add_rows<DB, kPlane>(gb, split8<true>(pd[0], pd[1]), dv, dv);
+            add_rows<DB, kPlane>(qb, split8(ds[0], ds[1]), dk, dk);
         }
         if (t + 1 < t_hi) publish(t + 1, slot ^ 1);
         __syncthreads();
@@ -604,26 +792,36 @@ __global__ __launch_bounds__(kThreads, 2) void attn_f32_dkv_kernel(const AttnArg
 enum class Which { kFwd, kDq, kDkv };
 
 // DB = 16-wide blocks of the head dimension
-template <int DB, Which kWhich, int kMode, int kHalves = 1>
-int launch(const AttnArgs& a, hipStream_t st) {
+template <int DB, Which kWhich, int kMode, int kWaves, int kHalves = 1>
+int launch_build(const AttnArgs& a, hipStream_t st) {
     const int n_rows = kWhich == Which::kDkv ? a.sk : a.sq;
+    constexpr int kRows = 16 * kWaves;
     const int64_t blocks =
         (int64_t)((n_rows + kRows - 1) / kRows) * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    if constexpr (kWhich == Which::kFwd && kHalves == 1) {
-        if (blocks <= kHalvesBlocks) return launch<DB, kWhich, kMode, 2>(a, st);
-    }
-    const size_t smem = (4 * kHalves * kTile * kPitchOf<DB> +
-                         (kWhich == Which::kDkv ? 6 * kTile : 0)) *
-                        sizeof(float);
-    auto kern = kWhich == Which::kFwd  ? attn_f32_fwd_kernel<DB, kMode, kHalves>
-                : kWhich == Which::kDq ? attn_f32_dq_kernel<DB, kMode>
-                                       : attn_f32_dkv_kernel<DB, kMode>;
+    const size_t smem = 4 * 3 * kHalves * kTile * kPitchOf<DB> * sizeof(bf16_t) +
+                        (kWhich == Which::kDkv ? 8 * kTile * sizeof(float) : 0);
+    auto kern = [] {
+        if constexpr (kWhich == Which::kFwd) return attn_f32_fwd_kernel<DB, kMode, kWaves, kHalves>;
+        else if constexpr (kWhich == Which::kDq) return attn_f32_dq_kernel<DB, kMode, kWaves>;
+        else return attn_f32_dkv_kernel<DB, kMode, kWaves>;
+    }();
     static std::atomic<uint64_t> lds_ready{0};
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kHalves * kThreads), smem, st, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kHalves * kWaves * 64), smem, st, a);
     return check_launch();
+}
+template <int DB, Which kWhich, int kMode>
+int launch(const AttnArgs& a, hipStream_t st) {
+    const int n_rows = kWhich == Which::kDkv ? a.sk : a.sq;
+    const int64_t units = (int64_t)((n_rows + 63) / 64) * a.batch * a.heads * a.n_split;
+    if constexpr (DB > 6) return launch_build<DB, kWhich, kMode, 8>(a, st);
+    else if constexpr (DB > 4) return launch_build<DB, kWhich, kMode, 4>(a, st);
+    else if (units >= (kWhich == Which::kFwd ? kWideFwd : kWideBwd))
+        return launch_build<DB, kWhich, kMode, 8>(a, st);
+    else if constexpr (kWhich == Which::kFwd) return launch_build<DB, kWhich, kMode, 4, 2>(a, st);
+    else return launch_build<DB, kWhich, kMode, 4>(a, st);
 }
 
 template <Which kWhich, int DB>

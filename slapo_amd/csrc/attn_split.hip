@@ -29,11 +29,9 @@ __device__ __forceinline__ void store4(T* p, const f32x4_t& v) {
     }
 }
 
-// Forward: a thread owns four columns of one query row.  m in log2 units for the 16-bit kernels and
-// in natural units for fp32.
+// Forward: a thread owns four columns of one query row.  m in log2 units.
 template <typename T>
 __global__ __launch_bounds__(kThreads) void merge_fwd_kernel(const AttnArgs a) {
-    constexpr bool kLog2 = sizeof(T) != 4;
     const int quads = (a.d + 3) / 4;
     const int64_t n_rows = (int64_t)a.batch * a.heads * a.sq;
     const int64_t at = (int64_t)blockIdx.x * kThreads + threadIdx.x;
@@ -50,7 +48,7 @@ __global__ __launch_bounds__(kThreads) void merge_fwd_kernel(const AttnArgs a) {
     for (int s = 0; s < a.n_split; ++s) {
         const float ms = ml[2 * s * n_rows];
         // (no maximum: nothing seen, or nothing but NaN scores, whose sum and values are NaN and stay)
-        const float w = ms == -INFINITY ? 0.f : kLog2 ? fast_exp2(ms - m) : expf(ms - m);
+        const float w = ms == -INFINITY ? 0.f : fast_exp2(ms - m);
         l = __builtin_fmaf(ml[2 * s * n_rows + 1], w, l);
         const float* p = a.part + s * plane + row * a.d + c;
 #pragma unroll
@@ -58,7 +56,8 @@ __global__ __launch_bounds__(kThreads) void merge_fwd_kernel(const AttnArgs a) {
             if (e < n) o[e] = __builtin_fmaf(p[e], w, o[e]);
     }
     // the 16-bit kernels leave the factor of the kept probabilities to the output rows
-    const float inv = (kLog2 && a.dropout ? a.rng.inv_keep : 1.0f) / l;
+    constexpr bool kF32 = sizeof(T) == 4;
+    const float inv = (!kF32 && a.dropout ? a.rng.inv_keep : 1.0f) / l;
     const int i = (int)(row % a.sq);
     const int64_t bh = row / a.sq, b = bh / a.heads, h = bh - b * a.heads;
     T* out = reinterpret_cast<T*>(a.o) + b * a.os[0] + (int64_t)i * a.os[1] + h * a.os[2] + c;
@@ -68,8 +67,8 @@ __global__ __launch_bounds__(kThreads) void merge_fwd_kernel(const AttnArgs a) {
         for (int e = 0; e < n; ++e) out[e] = Elem<T>::from_f32(o[e] * inv);
     }
     if (c == 0) {
-        const float log_l = kLog2 ? __builtin_log2f(l) : logf(l);
-        a.lse[row] = m == -kFltMax ? l * kMaskedRowLse : (m + log_l) * (kLog2 ? kLn2 : 1.0f);
+        const float lse = kF32 ? __builtin_fmaf(m, kLn2, logf(l)) : (m + __builtin_log2f(l)) * kLn2;
+        a.lse[row] = m == -kFltMax ? l * kMaskedRowLse : lse;
     }
 }
 

@@ -166,12 +166,25 @@ SLAPO_HD uint32_t dropout_keep4_pow2(const DropoutState& s, uint64_t group) {
            (keep_word(s, r.z) ? 4u : 0u) | (keep_word(s, r.w) ? 8u : 0u);
 }
 
-// Keep-bits of the 32 consecutive elements starting at elem (bit j <-> element elem + j), for any
-// thread count and alignment and vec <= 4 (the plan of a 4-byte tensor).  The element -> (thread,
+// Keep-bits of the n (1..32) consecutive elements starting at elem, for any launch geometry and
+// alignment.  Deliberately a rolled loop: this path is rare and must stay small.
+SLAPO_HD uint32_t dropout_keep_any(const DropoutState& s, uint64_t elem, int n) {
+    uint32_t bits = 0;
+#if defined(__HIPCC__)
+#pragma unroll 1
+#endif
+    for (int e = 0; e < n; ++e) bits |= (dropout_keep1(s, elem + (uint64_t)e) ? 1u : 0u) << e;
+    return bits;
+}
+
+// Keep-bits of the n <= 32 consecutive elements starting at elem (bit j <-> element elem + j; bits from
+// n on are not zero), for any thread count and alignment, fast at vec <= 4 (the plan of a 4-byte
+// tensor).  The element -> (thread,
 // trip) split costs a division where the thread count is no power of two: it is taken once and
-// stepped from there.  A Philox block serves `vec` of the elements: 9 blocks at vec 4 (8 where the
-// run is aligned), 17 at vec 2, 32 at vec 1.
-SLAPO_HD uint32_t dropout_keep32(const DropoutState& s, uint64_t elem) {
+// stepped from there.  A Philox block serves `vec` of the elements: 9 blocks for 32 at vec 4 (8 where
+// the run is aligned), 17 at vec 2, 32 at vec 1.
+SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem, int n) {
+    if (s.vec > 4) return dropout_keep_any(s, elem, n);
     const uint32_t shift = s.vec == 4 ? 2u : s.vec == 2 ? 1u : 0u;
     uint64_t thread, trip;
     const uint64_t v = elem >> shift;
@@ -187,7 +200,7 @@ SLAPO_HD uint32_t dropout_keep32(const DropoutState& s, uint64_t elem) {
 #if defined(__HIPCC__)
 #pragma unroll 1
 #endif
-    for (int at = -skip; at < 32; at += 1 << shift) {
+    for (int at = -skip; at < n; at += 1 << shift) {
         const u32x4 r = philox_block(s, thread, shift ? trip : trip >> 2);
         uint32_t four = (keep_word(s, r.x) ? 1u : 0u) | (keep_word(s, r.y) ? 2u : 0u) |
                         (keep_word(s, r.z) ? 4u : 0u) | (keep_word(s, r.w) ? 8u : 0u);
@@ -196,17 +209,6 @@ SLAPO_HD uint32_t dropout_keep32(const DropoutState& s, uint64_t elem) {
         bits |= at < 0 ? four >> -at : four << at;
         if (++thread == s.total_threads) thread = 0, ++trip;
     }
-    return bits;
-}
-
-// Keep-bits of the n (1..4) consecutive elements starting at elem, for any launch geometry and
-// alignment.  Deliberately a rolled loop: this path is rare and must stay small.
-SLAPO_HD uint32_t dropout_keep_any(const DropoutState& s, uint64_t elem, int n) {
-    uint32_t bits = 0;
-#if defined(__HIPCC__)
-#pragma unroll 1
-#endif
-    for (int e = 0; e < n; ++e) bits |= (dropout_keep1(s, elem + (uint64_t)e) ? 1u : 0u) << e;
     return bits;
 }
 

@@ -721,6 +721,36 @@ def test_fp32_kernels_at_the_edges_of_tiles(shape, sk, causal, window, p):
     _check(q, k, v, do, mask, causal, window, torch.float32, p=p)
 
 
+@pytest.mark.parametrize("shape", [(2, 1037, 4, 64), (4, 1025, 8, 24), (1, 257, 3, 128)])
+def test_fp32_workgroups_of_eight_wavefronts(shape):
+    """Calls large enough (or wide enough) for workgroups of 128 rows, with remainders of the rows."""
+    q, k, v, do, g = _inputs(*shape, torch.float32)
+    _check(q, k, v, do, None, True, 0, torch.float32)
+
+
+@pytest.mark.parametrize("head_dim", [64, 80, 128])
+def test_fp32_values_at_the_ends_of_the_range(head_dim):
+    """The kernels split fp32 numbers into bf16 parts: values that bf16 rounds to infinity, whose rest
+    is subnormal, infinities and NaN come out as fp32 arithmetic has them."""
+    q, k, v, _, g = _inputs(1, 70, 2, head_dim, torch.float32)
+    top = torch.finfo(torch.float32).max
+    v[0, 60, 0, 0] = top           # weight below 1: finite
+    v[0, 4, 0, 1] = float("inf")
+    v[0, 5, 0, 2] = -float("inf")
+    v[0, 6, 0, 3] = float("nan")
+    v[0, :, 0, 4] *= 1e-36
+    k[0, 7, 1, 5] = float("inf")   # scores of -inf (weight 0) and of +inf (a row of NaN)
+    out = op.hip_attention(q.cuda(), k.cuda(), v.cuda(), None, causal=False).cpu().double()
+    ref = OA.xformers_ref(q, k, v, None, False, compute_dtype=torch.float64)
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    assert torch.equal(torch.isinf(out), torch.isinf(ref))
+    ok = torch.isfinite(ref)
+    assert ok[..., 5:].any(dim=1).all()
+    scale = v.double().abs().nan_to_num(0.0, 0.0, 0.0).amax(dim=1, keepdim=True).clamp(min=1e-37)
+    err = ((out - ref).where(ok, torch.zeros_like(ref)).abs() / scale).max().item()
+    assert err <= 1e-5, err  # the fp32 bar of unit-scale values, per column
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("b,h,d,sk,layout", [
     (1, 1, 8, 1, None),            # one key
