@@ -45,13 +45,14 @@ constexpr int kTile = 32;  // streamed rows per LDS tile
 // SIMD (B1 S1024 H8 D128 causal, forward and backward: 146 against 198 us).  At head_dim 65-96
 // two workgroups of four fit a CU and balance causal and windowed calls better (B2 S1000 H6 D96
 // window 200: 87 against 127 us; without a mask equal).  Up to 64 it takes workgroups enough:
-constexpr int64_t kWideFwd = 128;   // in units of 64 rows: forward B3 S500 H12 D64 (288) 32.8 against
-                                    // 34.8 us, below that kHalves
-constexpr int64_t kWideBwd = 512;   // B4 S512 H16 D64 (512) 125 against 132 us forward and backward,
-                                    // B2 S777 H12 D64 (312) padded, p 0.1: 305 against 283
-// Smaller forward calls up to head_dim 64 run kHalves = 2: eight wavefronts, two per 16 query rows, each
+constexpr int64_t kWideBwd = 512;   // in units of 64 rows: B4 S512 H16 D64 (512) 125 against 132 us
+                                    // forward and backward, B2 S777 H12 D64 (312) padded, p 0.1 305
+                                    // against 283; a forward gains at once (288: 32.8 against 34.8)
+// Small forward calls up to head_dim 96 run kHalves = 2: eight wavefronts, two per 16 query rows, each
 // with one half of a tile of 64 keys and a softmax state of its own, merged at the end through LDS (B1
-// S256 H8 D64, 32 units: 12.3 us against 15.6 with four wavefronts and 18.1 with eight times 16 rows).
+// S256 H8 D64, 32 units: 12.3 us against 15.6 with four wavefronts and 18.1 with eight times 16 rows;
+// B4 S292 H4 D72, 80 units: 19.2 against 25.7; B2 S512 H8 D72, 128 units: 32.2 against 27.6).
+constexpr int64_t kHalvesBelow = 128;
 // LDS and registers leave a SIMD four of a forward's wavefronts up to head_dim 64, else two.
 constexpr int per_simd(int db, int waves) { return db <= 4 && waves >= 8 ? 4 : 2; }
 constexpr float kReserve = 8.0f;  // of the softmax reference above the maximum, log2 units
@@ -816,12 +817,16 @@ template <int DB, Which kWhich, int kMode>
 int launch(const AttnArgs& a, hipStream_t st) {
     const int n_rows = kWhich == Which::kDkv ? a.sk : a.sq;
     const int64_t units = (int64_t)((n_rows + 63) / 64) * a.batch * a.heads * a.n_split;
-    if constexpr (DB > 6) return launch_build<DB, kWhich, kMode, 8>(a, st);
-    else if constexpr (DB > 4) return launch_build<DB, kWhich, kMode, 4>(a, st);
-    else if (units >= (kWhich == Which::kFwd ? kWideFwd : kWideBwd))
+    if constexpr (DB > 6) {
         return launch_build<DB, kWhich, kMode, 8>(a, st);
-    else if constexpr (kWhich == Which::kFwd) return launch_build<DB, kWhich, kMode, 4, 2>(a, st);
-    else return launch_build<DB, kWhich, kMode, 4>(a, st);
+    } else {
+        if constexpr (kWhich == Which::kFwd)
+            if (units < kHalvesBelow) return launch_build<DB, kWhich, kMode, 4, 2>(a, st);
+        if constexpr (DB <= 4)
+            if (kWhich == Which::kFwd || units >= kWideBwd)
+                return launch_build<DB, kWhich, kMode, 8>(a, st);
+        return launch_build<DB, kWhich, kMode, 4>(a, st);
+    }
 }
 
 template <Which kWhich, int DB>
