@@ -35,14 +35,14 @@ constexpr int kBN = 64;
 constexpr int kKRing = 2;
 constexpr int kVRing = 2;
 
-// kStagger: see the tile bodies below.  Staggered halves need one workgroup per CU above
-// head_dim 64; sequential halves fit two.
+// kStagger (see the tile bodies below): up to head_dim 64; above, sequential halves are what fits two
+// workgroups per CU.
 // kBias: 0 = no additive bias, 1 = any layout (read from memory per score), 2 = the bias depends on
 // the key only (stride 0 over the queries): its 64 values per key tile travel through LDS beside
 // the K / V tile, and the tile bodies have neither global loads nor branches for them.
-template <typename T, int DPAD, int kBias, int kDrop, bool kStagger, int kSteps>
-__global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void attn_bwd_dq_kernel(
-    const AttnArgs a_in) {
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
+__global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(const AttnArgs a_in) {
+    constexpr bool kStagger = DPAD <= 64;
     AttnArgs a = a_in;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     typedef typename Mma<T>::frag frag_t;
@@ -127,6 +127,7 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     int t_hi = (j_hi + kBN - 1) / kBN;
     if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
     const int n_tiles = t_hi - t_lo;
+    const TileOrder order = TileOrder::of<kBM, kBN>(a, q0, t_lo, t_hi);
 
     frag_t qf[DK], gf[DK];
     float lse2, delta, inv_n = 1.0f;
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
             ov[t] = *reinterpret_cast<const u32x4_t*>(o_base + (int64_t)qr * a.os[1] + dc);
         }
         const float lse_raw = a.lse[(int64_t)bh * a.sq + qr];
-        request(t_lo * kBN);
+        request(order.first() * kBN);
         const bool row_ok = q_row < a.sq;
 #pragma unroll
         for (int t = 0; t < DK; ++t) {
@@ -204,9 +205,9 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     if constexpr (kDrop != 0)
         drop_row_base = ((uint64_t)bh * a.sq + (uint64_t)q_row) * (uint64_t)a.sk;
     const float* bias_row = nullptr;
-    if constexpr (kBias == 1 || kBias == 3)  // (prepared rows exist past the end)
+    if constexpr (kBias == 1 || kBias == 3)  // (rows past the end: the last one)
         bias_row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] +
-                   (int64_t)(kBias == 3 ? q_row : min(q_row, a.sq - 1)) * a.bs[2];
+                   (int64_t)min(q_row, a.sq - 1) * a.bs[2];
 
     // per-lane LDS offsets (elements) that do not change from tile to tile
     const int row_off = pi_row(i_loc) * kPitch + 8 * g;
@@ -219,19 +220,14 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
         if (a.window > 0 && wq0 - (j0 + kBN - 1) >= a.window) return false;
         return true;
     };
-    auto tile_needs_mask = [&](int t) __attribute__((always_inline)) {
-        const int j0 = t * kBN;
-        return (j0 + kBN > a.sk) || (a.causal && j0 + kBN - 1 > wq0) ||
-               (a.window > 0 && wq_last - j0 >= a.window);
-    };
-
     // The tile is processed as two halves of 32 keys.  With kStagger their stages are staggered,
     // so that the matrix instructions of one half always have independent vector work of the
     // other half around them (a wavefront overlaps the two only when they are interleaved in its
     // instruction stream).  Without it the halves run one after the other: above head_dim 64 that
     // is what fits two workgroups per CU into the register file, and the second resident workgroup
     // hides more latency than the stagger does (measured: 28 % faster at head_dim 80, 2-12 % at
-    // 128; only the masked tile bodies of a local window lose, to register spills, at 128).
+    // 128; with one masked body for all bounds also where a window or stored dropout bits spilled
+    // registers before: 90.6 -> 71.3 us at bf16 B4 S2048 H16 D128 window 256, p 0.1).
 
     // S^T half = K_half Q^T (log2 units)
     auto half_s = [&](const T* kt, int kb, f32x16_t& s) __attribute__((always_inline)) {
@@ -261,17 +257,19 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
         }
     };
     // scores -> probabilities, in place
-    // mask_tag: 0 = every key visible, 1 = upper bound only (causal / key tail), 2 = both bounds
+    // mask_tag: 0 = every key visible, 1 = the causal, window and tail bounds, as one bit per key:
+    // two instructions per score whatever the bounds are (a compare and a select for each bound
+    // before), so that one masked tile body serves every call
     auto half_exp = [&](f32x16_t& s, int t, int kb, auto mask_tag) __attribute__((always_inline)) {
         constexpr int kMask = decltype(mask_tag)::value;
         const int j0 = t * kBN + kb * 32;
-        // register r is key j0 + acc_row(r, g) = j0 + kAccGroupStep g + c with c = acc_row(r, 0);
-        // visible iff c_lo <= c <= c_hi
-        int c_lo = 0, c_hi = 0;
+        // register r is key j0 + acc_row(r, g) = j0 + kAccGroupStep g + c with c = acc_row(r, 0)
+        uint32_t visible = 0u;
         if constexpr (kMask != 0) {
             const int k_max = a.causal ? min(a.sk - 1, q_row) : a.sk - 1;
-            c_hi = k_max - j0 - kAccGroupStep * g;
-            if constexpr (kMask == 2) c_lo = q_row - a.window + 1 - j0 - kAccGroupStep * g;
+            const int k_min = a.window > 0 ? q_row - a.window + 1 : 0;
+            const int at = j0 + kAccGroupStep * g;
+            visible = visible_bits(k_min - at, k_max - at);
         }
         if constexpr (kBias == 1) {
             // Registers 8 h + e and 8 h + 4 + e are keys 2 g and 2 g + 1 of the aligned group of
@@ -312,14 +310,7 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
                 if constexpr (!kAccInit) x -= lse_sub;
                 if constexpr (kBias == 2 || kBias == 3) x += bv[e];
                 float p = fast_exp2(x);
-                if constexpr (kMask != 0) {
-                    const int c = acc_row(4 * r4 + e, 0);
-                    if constexpr (kMask == 2) {
-                        if (c > c_hi || c < c_lo) p = 0.f;
-                    } else {
-                        if (c > c_hi) p = 0.f;
-                    }
-                }
+                if constexpr (kMask != 0) p = keep_or_zero(p, visible, acc_row(4 * r4 + e, 0));
                 s[4 * r4 + e] = p;
             }
         }
@@ -406,8 +397,8 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     // Hand-scheduled version of tile_body for tiles without masks: the LDS operands of each group
     // of matrix instructions are requested one phase before the group runs, and scheduling fences
     // keep the compiler from sinking the requests back down to their uses.
-    auto tile_body_fast = [&](const T* kt, const T* vt, int t, auto mask_tag)
-                              __attribute__((always_inline)) {
+    auto tile_body_fast = [&](const T* kt, const T* vt, int t) __attribute__((always_inline)) {
+        constexpr std::integral_constant<int, 0> mask_tag{};
         frag_t kr0[DK], vr0[DK], kr1[DK], vr1[DK], kq0[2 * DV], kq1[2 * DV];
         f32x16_t s0, s1, p0, p1;
         uint32_t dw0[8], dw1[8];
@@ -468,72 +459,48 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
 
     // ---- prologue: tile 0 into LDS ----
     if (n_tiles > 0) {
-        ks.fix(t_lo * kBN, a.sk, a.d);
-        vs.fix(t_lo * kBN, a.sk, a.d);
+        ks.fix(order.first() * kBN, a.sk, a.d);
+        vs.fix(order.first() * kBN, a.sk, a.d);
         ks.store(k_lds);
         vs.store(v_lds);
         store_bias(0);
     }
     __syncthreads();
 
-    // Iteration r: request tile r+1, process tile r, write tile r+1 into the other ring slot.
-    // kFast iterations hold tiles that every wavefront of the workgroup sees in full, so their body
-    // is one straight block; the others test activity and masks per wavefront.
+    // Iteration r: request the next tile, process tile r of the order, write the next tile into the
+    // other ring slot.  kFast iterations hold tiles that every wavefront of the workgroup sees in
+    // full; the others test activity per wavefront and mask.
+    int t = order.first();
     auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
         constexpr bool kFast = decltype(fast_tag)::value;
-        const int t = t_lo + r;
+        const int next = kFast ? order.after_fast(t) : order.after(t);
         const bool have_next = r + 1 < n_tiles;
         if (have_next) {
-            request((t + 1) * kBN);
+            request(next * kBN);
         }
         const T* kt = k_lds + (r % kKRing) * kTileElems;
         const T* vt = v_lds + (r % kVRing) * kTileElems;
         bias_tile = bias_lds + (r & 1) * kBN;
         if constexpr (kFast) {
             if constexpr (kStagger)
-                tile_body_fast(kt, vt, t, std::integral_constant<int, 0>{});
+                tile_body_fast(kt, vt, t);
             else
                 tile_body(kt, vt, t, std::integral_constant<int, 0>{});
         } else if (tile_active(t)) {
-            // One wavefront per SIMD (head_dim 128, 412-484 registers): nothing else hides the
-            // latencies of a masked tile, so it runs the hand-scheduled body as well (dQ at bf16 B4
-            // S2048 H16 D128, window 256, p 0.1: 90.8 -> 86.5 us).  With two wavefronts per SIMD
-            // the extra copies of that body cost registers (246 -> 256 and 16 spilled at head_dim
-            // 64) and gain nothing.
-            if constexpr (kStagger && DPAD > 96 && kDrop != 2) {
-                if (!tile_needs_mask(t))
-                    tile_body_fast(kt, vt, t, std::integral_constant<int, 0>{});
-                else if (a.window > 0)
-                    tile_body_fast(kt, vt, t, std::integral_constant<int, 2>{});
-                else
-                    tile_body_fast(kt, vt, t, std::integral_constant<int, 1>{});
-            } else {
-                if (!tile_needs_mask(t))
-                    tile_body(kt, vt, t, std::integral_constant<int, 0>{});
-                else if (a.window > 0)
-                    tile_body(kt, vt, t, std::integral_constant<int, 2>{});
-                else
-                    tile_body(kt, vt, t, std::integral_constant<int, 1>{});
-            }
+            tile_body(kt, vt, t, std::integral_constant<int, 1>{});
         }
         if (have_next) {
-            ks.fix((t + 1) * kBN, a.sk, a.d);
-            vs.fix((t + 1) * kBN, a.sk, a.d);
+            ks.fix(next * kBN, a.sk, a.d);
+            vs.fix(next * kBN, a.sk, a.d);
             ks.store(k_lds + ((r + 1) % kKRing) * kTileElems);
             vs.store(v_lds + ((r + 1) % kVRing) * kTileElems);
             store_bias((r + 1) & 1);
         }
         __syncthreads();
+        t = next;
     };
-    // leading tiles that need neither mask nor activity test for any of the 128 queries
-    int n_fast = 0;
-    if (a.window <= 0 && q0 + kBM <= a.sq) {
-        n_fast = a.sk / kBN;
-        if (a.causal) n_fast = min(n_fast, (q0 + 1) / kBN);
-        n_fast = min(n_fast - t_lo, n_tiles);
-    }
     int r = 0;
-    for (; r < n_fast; ++r) iteration(r, std::true_type{});
+    for (; r < order.end - order.begin; ++r) iteration(r, std::true_type{});
     for (; r < n_tiles; ++r) iteration(r, std::false_type{});
     // ---- epilogue: dQ = scale * dQ^T^T ----
     // every wavefront is past the last barrier of the loop: the K buffers are free, and each
@@ -552,7 +519,7 @@ __global__ __launch_bounds__(kThreads, (kStagger && DPAD > 64 ? 1 : 2)) void att
     }
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, bool kStagger, int kSteps>
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
 int launch(const AttnArgs& a, hipStream_t st) {
     typedef TileStage<T, DPAD, kBN, kThreads> Stage;
     const size_t smem = (size_t)(kKRing + kVRing) * kBN * Stage::kPitch * sizeof(T) +
@@ -560,54 +527,48 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const int n_qt = (a.sq + kBM - 1) / kBM;
     const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    auto kern = attn_bwd_dq_kernel<T, DPAD, kBias, kDrop, kStagger, kSteps>;
+    auto kern = attn_bwd_dq_kernel<T, DPAD, kBias, kDrop, kSteps>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
-    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, (kStagger && DPAD > 64) ? 1 : 2);
+    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, 2);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, ordered);
     return check_launch();
 }
 
-template <typename T, int DPAD, bool kStagger, int kSteps = DPAD / 16>
+template <typename T, int DPAD, int kSteps = DPAD / 16>
 int dispatch_flags(const AttnArgs& a, hipStream_t st) {
     if (a.has_bias) {
         if (a.bias_type == SLAPO_BIAS_PREPARED) {
-            if (a.dropout == 1) return launch<T, DPAD, 3, 1, kStagger, kSteps>(a, st);
-            if (a.dropout == 2) return launch<T, DPAD, 3, 2, kStagger, kSteps>(a, st);
-            if (a.dropout == 3) return launch<T, DPAD, 3, 3, kStagger, kSteps>(a, st);
-            return launch<T, DPAD, 3, 0, kStagger, kSteps>(a, st);
+            if (a.dropout == 1) return launch<T, DPAD, 3, 1, kSteps>(a, st);
+            if (a.dropout == 2) return launch<T, DPAD, 3, 2, kSteps>(a, st);
+            if (a.dropout == 3) return launch<T, DPAD, 3, 3, kSteps>(a, st);
+            return launch<T, DPAD, 3, 0, kSteps>(a, st);
         }
         if (a.bs[2] == 0) {  // the bias depends on the key only
-            if (a.dropout == 1) return launch<T, DPAD, 2, 1, kStagger, kSteps>(a, st);
-            if (a.dropout == 2) return launch<T, DPAD, 2, 2, kStagger, kSteps>(a, st);
-            if (a.dropout == 3) return launch<T, DPAD, 2, 3, kStagger, kSteps>(a, st);
-            return launch<T, DPAD, 2, 0, kStagger, kSteps>(a, st);
+            if (a.dropout == 1) return launch<T, DPAD, 2, 1, kSteps>(a, st);
+            if (a.dropout == 2) return launch<T, DPAD, 2, 2, kSteps>(a, st);
+            if (a.dropout == 3) return launch<T, DPAD, 2, 3, kSteps>(a, st);
+            return launch<T, DPAD, 2, 0, kSteps>(a, st);
         }
-        if (a.dropout == 1) return launch<T, DPAD, 1, 1, kStagger, kSteps>(a, st);
-        if (a.dropout == 2) return launch<T, DPAD, 1, 2, kStagger, kSteps>(a, st);
-        if (a.dropout == 3) return launch<T, DPAD, 1, 3, kStagger, kSteps>(a, st);
-        return launch<T, DPAD, 1, 0, kStagger, kSteps>(a, st);
+        if (a.dropout == 1) return launch<T, DPAD, 1, 1, kSteps>(a, st);
+        if (a.dropout == 2) return launch<T, DPAD, 1, 2, kSteps>(a, st);
+        if (a.dropout == 3) return launch<T, DPAD, 1, 3, kSteps>(a, st);
+        return launch<T, DPAD, 1, 0, kSteps>(a, st);
     }
-    if (a.dropout == 1) return launch<T, DPAD, 0, 1, kStagger, kSteps>(a, st);
-    if (a.dropout == 2) return launch<T, DPAD, 0, 2, kStagger, kSteps>(a, st);
-    if (a.dropout == 3) return launch<T, DPAD, 0, 3, kStagger, kSteps>(a, st);
-    return launch<T, DPAD, 0, 0, kStagger, kSteps>(a, st);
+    if (a.dropout == 1) return launch<T, DPAD, 0, 1, kSteps>(a, st);
+    if (a.dropout == 2) return launch<T, DPAD, 0, 2, kSteps>(a, st);
+    if (a.dropout == 3) return launch<T, DPAD, 0, 3, kSteps>(a, st);
+    return launch<T, DPAD, 0, 0, kSteps>(a, st);
 }
 
 template <typename T>
 int dispatch(const AttnArgs& a, hipStream_t st) {
-    if (a.d <= 64) return dispatch_flags<T, 64, true>(a, st);
-    if (a.d <= 80) return dispatch_flags<T, 96, false, 5>(a, st);  // five k-steps cover head_dim 80
-    if (a.d <= 96) return dispatch_flags<T, 96, false>(a, st);
-    if (a.d <= 128) {
-        // a local window leaves mostly masked tiles, whose bodies spill at two workgroups per CU;
-        // so does the body that applies stored dropout bits (163 spilled registers: 188 against
-        // 158 us at bf16 B4 S2048 H16 causal, p 0.1)
-        if (a.window > 0 || a.dropout == 3) return dispatch_flags<T, 128, true>(a, st);
-        return dispatch_flags<T, 128, false>(a, st);
-    }
+    if (a.d <= 64) return dispatch_flags<T, 64>(a, st);
+    if (a.d <= 80) return dispatch_flags<T, 96, 5>(a, st);  // five k-steps cover head_dim 80
+    if (a.d <= 96) return dispatch_flags<T, 96>(a, st);
+    if (a.d <= 128) return dispatch_flags<T, 128>(a, st);
     return SLAPO_ERR_SHAPE;
 }
 

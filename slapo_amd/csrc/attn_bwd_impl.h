@@ -47,17 +47,19 @@ struct BwdSmem {
     static constexpr size_t kBytes = 2 * kQBytes + kStatBytes + kMaskBytes;
 };
 
-constexpr bool bwd_two_per_cu(int dpad, int drop, int kb) {
-    return kb == 1 && (dpad <= 64 || (dpad == 96 && drop != 3));
-}
+// Two workgroups per CU up to DPAD 96, one at 128 (192 resident accumulator / fragment registers).  At
+// 96 with the forward's keep bits both are built: two where a call has more key blocks than CUs
+// (fp16 B5 S920 H31 D80 window 356, p 0.1, forward and backward 256 -> 226 us; bf16 B4 S2048 H12 D96
+// causal, p 0.1 322 -> 292), else one, whose staggered body is the faster of the two (fp16 B2 S1600 H8
+// D96 padded, p 0.1, 208 blocks dealt to 416 workgroups: 168 against 173 us; B1 S2048 H12 D96 175
+// against 181).
+constexpr bool bwd_two_per_cu(int dpad, int kb) { return kb == 1 && dpad <= 96; }
 
 // KB = blocks of 32 keys per wavefront.  KB = 2 halves the LDS operand traffic per matrix
 // instruction (every Q / dO fragment read feeds two MFMAs) at the price of twice the resident
 // fragments and accumulators, i.e. one wavefront per SIMD instead of two.
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps>
-// Two workgroups per CU up to DPAD 96, one at 128 (192 resident accumulator / fragment registers)
-// and at 96 with the forward's keep bits (measured 23-35 % slower with two than with one).
-__global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 : 1)) void attn_bwd_kernel(
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, bool kTwo>
+__global__ __launch_bounds__(kBwdThreads, (kTwo ? 2 : 1)) void attn_bwd_kernel(
     const AttnArgs a_in) {
     AttnArgs a = a_in;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
@@ -154,7 +156,9 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     const float* bias_tile = nullptr;
     uint32_t bias_lane = 0;
     if constexpr (kBias == 3) {
-        bias_tile = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] + kw0;
+        // (prepared rows end at a multiple of 64 keys: a wavefront past that reads the last block)
+        bias_tile = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] +
+                    min(kw0, (a.sk - 1) & ~31);
         bias_lane = (uint32_t)(kAccGroupStep * g * (int)a.bs[2] + prepared_slot(c_loc));
     }
     float bias_k[KB];
@@ -272,9 +276,10 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     };
     auto tile_fast = [&](int t) __attribute__((always_inline)) {
         const int i0 = t * kBwdBM;
-        // every (query, key) pair of the tile is visible: the first query sees the last key
-        // (causal), the last query still sees the first key (local window)
-        return k0 + kBN <= a.sk && i0 + kBwdBM <= a.sq && (!a.causal || i0 >= k0 + kBN - 1) &&
+        // the first query sees the last key (causal), the last query still sees the first key (local
+        // window).  What lies past the end needs no masks: queries there have P = 0 (a -inf among
+        // the values that the scores start from), keys there yield rows that are not written.
+        return (!a.causal || i0 >= k0 + kBN - 1) &&
                (a.window <= 0 || i0 + kBwdBM - 1 - k0 < a.window);
     };
     // Two generic (diagonal / tail) tiles in a row are processed together, see generic_step; when
@@ -312,9 +317,8 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
         return true;
     };
     auto half_needs_mask = [&](int ih0) __attribute__((always_inline)) {
-        const int i_last = min(ih0 + 32, a.sq) - 1;
-        return (kw0 + kWaveKeys > a.sk) || (a.causal && kw0 + kWaveKeys - 1 > ih0) ||
-               (a.window > 0 && i_last - kw0 >= a.window);
+        return (a.causal && kw0 + kWaveKeys - 1 > ih0) ||
+               (a.window > 0 && ih0 + 31 - kw0 >= a.window);
     };
 
     // ---- stages of one half tile (32 queries at ih0 = i0 + 32 hf) ----
@@ -343,25 +347,19 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
             }
         }
     };
-    // scores -> probabilities in place.  mask_tag: 0 = all visible, 1 = lower bound on the query
-    // only (causal / key tail), 2 = both bounds (local window)
+    // scores -> probabilities in place.  mask_tag: 0 = all visible, 1 = the causal and window bounds, as
+    // one bit per query: two instructions per score whatever they are
     auto half_exp = [&](f32x16_t (&s)[KB], const float* lse_h, int ih0, auto mask_tag)
                         __attribute__((always_inline)) {
         constexpr int kMask = decltype(mask_tag)::value;
-        // register r is query ih0 + acc_row(r, g) = ih0 + kAccGroupStep g + c with
-        // c = acc_row(r, 0); visible iff c_lo <= c <= c_hi
-        int c_lo[KB], c_hi[KB];
+        // register r is query ih0 + acc_row(r, g) = at + acc_row(r, 0)
+        const int at = ih0 + kAccGroupStep * g;
+        uint32_t visible[KB];
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-            c_lo[kb] = 0, c_hi[kb] = 0;
-            if constexpr (kMask != 0) {
-                c_lo[kb] = (key[kb] < a.sk)
-                               ? (a.causal ? key[kb] - ih0 - kAccGroupStep * g : -1)
-                               : 64;
-                if constexpr (kMask == 2)
-                    c_hi[kb] = key[kb] + a.window - 1 - ih0 - kAccGroupStep * g;
-            }
-        }
+        for (int kb = 0; kb < KB; ++kb)
+            visible[kb] = kMask == 0 ? 0u
+                                     : visible_bits(a.causal ? key[kb] - at : 0,
+                                                    a.window > 0 ? key[kb] + a.window - 1 - at : 31);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
 #pragma unroll
@@ -381,14 +379,7 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
                     x += row[bias_lane];
                 }
                 float p = fast_exp2(x);
-                if constexpr (kMask != 0) {
-                    const int c = acc_row(r, 0);
-                    if constexpr (kMask == 2) {
-                        if (c < c_lo[kb] || c > c_hi[kb]) p = 0.f;
-                    } else {
-                        if (c < c_lo[kb]) p = 0.f;
-                    }
-                }
+                if constexpr (kMask != 0) p = keep_or_zero(p, visible[kb], acc_row(r, 0));
                 s[kb][r] = p;
             }
         }
@@ -506,11 +497,9 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
         }
     };
 
-    // The two halves of a fast tile one after the other.  At DPAD 96 this is what fits two
-    // workgroups per CU (11-51 spilled registers); the second resident workgroup is worth more
-    // than the stagger: 319 -> 287 us at bf16 B4 S2048 H32 D80 causal, 638 -> 503 us when the
-    // backward regenerates the dropout mask.  With the forward's keep bits it is the other way
-    // round (370 -> 455 us), so that variant keeps one workgroup and the staggered body.
+    // The two halves of a fast tile one after the other: at DPAD 96 this is what fits two workgroups
+    // per CU, and the second one is worth more than the stagger (319 -> 287 us at bf16 B4 S2048 H32 D80
+    // causal, 638 -> 503 us when the backward regenerates the dropout mask).
     auto sequential_tile = [&](int t) __attribute__((always_inline)) {
         const int buf = (t - t_lo) & 1;
         const T* qt = q_lds + buf * SM::kQTile;
@@ -568,7 +557,7 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     auto fast_iteration = [&](int t) __attribute__((always_inline)) {
         constexpr bool kLateRequest = DPAD <= 64;  // two workgroups share a CU: registers scarce
         if constexpr (!kLateRequest) request_tile(regs, t + 1);
-        if constexpr (DPAD == 96 && bwd_two_per_cu(DPAD, kDrop, KB))
+        if constexpr (DPAD == 96 && kTwo)
             sequential_tile(t);
         else
             staggered_tile(t, std::integral_constant<int, 0>{},
@@ -595,10 +584,11 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
             f32x16_t s[KB], dp[KB];
             uint32_t pw[KB][8], dw[KB][8];
             half_sp(qt, gt, lse_h, delta_h, hf, s, dp);
-            if (!half_needs_mask(ih0))
+            // (a second copy without masks pays only up to head_dim 64, where registers are left: fp16
+            // B8 S1024 H16 D64 causal 120.4 -> 119.9 us forward and backward; bf16 B4 S2048 H16 D128
+            // window 256, p 0.1 224 -> 229)
+            if (DPAD <= 64 && !half_needs_mask(ih0))
                 half_exp(s, lse_h, ih0, std::integral_constant<int, 0>{});
-            else if (a.window > 0)
-                half_exp(s, lse_h, ih0, std::integral_constant<int, 2>{});
             else
                 half_exp(s, lse_h, ih0, std::integral_constant<int, 1>{});
             half_ds(s, dp, delta_h, mask_h, ih0, pw, dw);
@@ -611,30 +601,27 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     // both tiles in LDS no wavefront waits at a barrier in between for the busiest one.
     auto generic_step = [&](int t) __attribute__((always_inline)) -> int {
         const bool pair = kPairGeneric && t + 1 < t_hi && !tile_fast(t + 1);
-        if (!pair) {
-            request_tile(regs, t + 1);
-            generic_tiles(t, 1);
-            if (t + 1 < t_hi) stage_tile(regs, t + 1);
-            sync_staged();
-            return 1;
-        }
-        if (!(pair_first && t == t_lo)) {  // otherwise the start-up has staged tile t+1 already
+        const int n = pair ? 2 : 1;
+        if (pair && !(pair_first && t == t_lo)) {  // otherwise the start-up has staged tile t+1
             request_tile(regs, t + 1);
             stage_tile(regs, t + 1);  // the other buffer: last read before the previous barrier
             sync_staged();
         }
-        request_tile(regs, t + 2);
-        generic_tiles(t, 2);
-        __syncthreads();  // tile t+2 goes where tile t was
-        if (t + 2 < t_hi) stage_tile(regs, t + 2);
+        request_tile(regs, t + n);
+        generic_tiles(t, n);
+        if (pair) __syncthreads();  // tile t+2 goes where tile t was
+        if (t + n < t_hi) stage_tile(regs, t + n);
         sync_staged();
-        return 2;
+        return n;
     };
-    {
-        int t = t_lo;
+    // Generic tiles stand before and after the fast ones.  One copy of their body, in a loop of two
+    // rounds: with a copy for each side, three ways to mask in each, the live values of all of
+    // them cost registers in the fast body too.
+    int t = t_lo;
+#pragma unroll 1
+    for (int round = 0; round < 2; ++round) {
         while (t < t_hi && !tile_fast(t)) t += generic_step(t);
         for (; t < t_hi && tile_fast(t); ++t) fast_iteration(t);
-        while (t < t_hi) t += generic_step(t);
     }
     // ---- write dK, dV ----
     // every wavefront is past the last barrier of the loop: the tile buffers are free, and each
@@ -666,7 +653,7 @@ __global__ __launch_bounds__(kBwdThreads, (bwd_two_per_cu(DPAD, kDrop, KB) ? 2 :
     }
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps>
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, bool kTwo>
 int launch(const AttnArgs& a, hipStream_t st) {
     typedef BwdSmem<T, DPAD> SM;
     const size_t smem = SM::kBytes;
@@ -674,12 +661,12 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const int n_kt = (a.sk + kBN - 1) / kBN;
     const int64_t blocks = (int64_t)n_kt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps>;
+    auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps, kTwo>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
-    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, bwd_two_per_cu(DPAD, kDrop, KB) ? 2 : 1);
+    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, kTwo ? 2 : 1);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBwdThreads), smem, st, ordered);
     return check_launch();
 }
@@ -689,7 +676,12 @@ int launch(const AttnArgs& a, hipStream_t st) {
 // resident wavefront hides more latency than the halved LDS traffic saves.  Only KB = 1 is built.
 template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
 int launch_kb(const AttnArgs& a, hipStream_t st) {
-    return launch<T, DPAD, kBias, kDrop, 1, kSteps>(a, st);
+    if constexpr (DPAD == 96 && kDrop == 3) {
+        const int64_t blocks =
+            (int64_t)((a.sk + kBwdWaves * 32 - 1) / (kBwdWaves * 32)) * a.batch * a.heads;
+        if (blocks <= a.n_cus) return launch<T, DPAD, kBias, kDrop, 1, kSteps, false>(a, st);
+    }
+    return launch<T, DPAD, kBias, kDrop, 1, kSteps, bwd_two_per_cu(DPAD, 1)>(a, st);
 }
 
 template <typename T, int DPAD, int kBias, int kSteps>

@@ -217,6 +217,12 @@ __device__ __forceinline__ float keep_or_zero(float v, uint32_t bits, uint32_t p
     return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, v) & m);
 }
 
+// v where bit `pos` of `bits` is set, -inf elsewhere.
+__device__ __forceinline__ float keep_or_hide(float v, uint32_t bits, uint32_t pos) {
+    const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)bits, pos, 1u);
+    return __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, v) & m) | (~m & 0xFF800000u));
+}
+
 // Kernel argument block (filled by the host dispatcher from slapo_attn_params).
 struct AttnArgs {
     const void* q;
@@ -384,6 +390,37 @@ __device__ __forceinline__ void key_range(const AttnArgs& a, int q_lo, int q_hi,
     j_hi = a.causal ? min(a.sk, q_hi) : a.sk;
     j_lo = a.window > 0 ? max(0, q_lo - a.window + 1) : 0;
 }
+// The order in which a workgroup with queries [q0, q0 + kRows) takes its key tiles of kKeys: first
+// those that every query sees in full (the leading ones, with a local window a run in the middle),
+// then the others in ascending order.  Two loops, then, with one tile body each: a loop that chose
+// between bodies kept the live values of all of them apart (dQ at head_dim 128: 151 spilled
+// registers, none with one body per loop).
+struct TileOrder {
+    int t_lo, begin, end;  // the run of fully visible tiles, begin = end = t_lo if there is none
+    template <int kRows, int kKeys>
+    static __device__ __forceinline__ TileOrder of(const AttnArgs& a, int q0, int t_lo, int t_hi) {
+        // (rows past the end need no masks: nothing they yield is used)
+        int end = a.sk / kKeys;  // first tile that is incomplete or hidden from some query
+        if (a.causal) end = min(end, (q0 + 1) / kKeys);
+        end = min(end, t_hi);
+        // the last query sees keys >= q0 + kRows - window
+        int begin = a.window > 0 ? (max(q0 + kRows - a.window, 0) + kKeys - 1) / kKeys : 0;
+        begin = max(begin, t_lo);
+        return begin < end ? TileOrder{t_lo, begin, end} : TileOrder{t_lo, t_lo, t_lo};
+    }
+    __device__ __forceinline__ int first() const { return begin; }
+    // what follows fast tile t, and any other one
+    __device__ __forceinline__ int after_fast(int t) const {
+        return t + 1 < end || begin == t_lo ? t + 1 : t_lo;
+    }
+    __device__ __forceinline__ int after(int t) const { return t + 1 == begin ? end : t + 1; }
+};
+// Bit c (0..31): lo <= c <= hi.
+__device__ __forceinline__ uint32_t visible_bits(int lo, int hi) {
+    const uint32_t below = hi < 0 ? 0u : hi >= 31 ? ~0u : (2u << hi) - 1u;
+    return lo <= 0 ? below : lo > 31 ? 0u : below & (~0u << lo);
+}
+
 // First / one-past-last query that can see any key in [k_lo, k_hi).
 __device__ __forceinline__ void query_range(const AttnArgs& a, int k_lo, int k_hi, int& i_lo,
                                             int& i_hi) {

@@ -11,9 +11,10 @@
 //                                 permutation of the K reads makes them ordered k-slots), A = V^T
 //                                 read from the row-major V tile with the transposing LDS read.
 // The loop is deliberately NOT software pipelined across tiles inside a wavefront: one tile is in
-// flight per wavefront and leading tiles that no query of the workgroup needs masks for run as
-// one straight block.  That keeps the kernel inside 168 registers at head_dim <= 64 (THREE
-// workgroups per CU) and inside 256 above (two), and on this hardware resident wavefronts hide
+// flight per wavefront.  Tiles that no query of the workgroup needs masks for come first, as one
+// straight block; all others share one body (TileOrder, visible_bits).  That keeps the kernel inside
+// 168 registers at head_dim <= 64 (three workgroups per CU; four in 128 without bias and dropout) and
+// inside 256 above (two), and on this hardware resident wavefronts hide
 // more latency than a deeper pipeline inside one wavefront does: a pipelined variant with twice
 // the registers measured 12 % slower at head_dim 64 and 35-80 % slower at 80 / 128.
 //
@@ -32,13 +33,16 @@ constexpr int kBM = kWaves * 32;
 constexpr int kBN = 64;
 constexpr float kMaxSlack = 8.0f;  // hysteresis of the softmax reference, log2 units
 
-// Workgroups per CU: three in 168 registers without dropout or a per-score bias up to head_dim 64.
-constexpr int fwd_per_cu(int dpad, int bias, int drop) {
-    return dpad <= 64 && drop == 0 && bias != 3 ? 3 : 2;
-}
+// Workgroups per CU: three in 168 registers up to head_dim 64, two above (three at 96 spill 2 to 54
+// registers: bf16 B2 S3000 H20 D80 padded 147 -> 185 us).
+constexpr int fwd_per_cu(int dpad) { return dpad <= 64 ? 3 : 2; }
+// Without bias and dropout four fit in 128 registers, which pays where the launch fills them: from the
+// first workgroup that three a CU would not hold on (fp16 B8 S1024 H16 D64 causal, 1024 workgroups:
+// 30.9 -> 29.8 us, bf16 B2 S4096 H16 D64 causal 88.4 -> 83.5; bf16 B1 S8192 H8 D64, 512: 167 -> 169).
+constexpr int kFwdFour = 4;
 
-template <typename T, int DPAD, int kBias, int kDrop, int kWin, int kSteps>
-__global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn_fwd_kernel(
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu>
+__global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     const AttnArgs a_in) {
     // kBias: 0 = no additive bias, 1 = any layout (read from memory per score), 2 = the bias
     // depends on the key only (stride 0 over the queries, e.g. a [B,1,1,Sk] padding mask): the 64
@@ -47,16 +51,10 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     // with the per-score reads against 169 us without a bias), 3 = a prepared bias
     // (bias_prepare_kernel): fp32 rows in log2 units, padded and in accumulator order, so that a
     // lane reads its sixteen values of a half with four 16-byte loads and nothing else.
-    // kWin: 0 = the launcher guarantees window <= 0, 1 = it guarantees window > 0, 2 = either.
-    // Folding "no window" in removes the two-sided mask body and the window tests from the
-    // kernel, and with them the register spills of the bias-free builds (head_dim 64: 24 spilled
-    // registers -> none, 37.8 -> 35.7 us at fp16 B8 S1024 H16 causal; head_dim 128: 69 -> 4,
-    // 116 -> 96-109 us at bf16 B4 S2048 H16 causal); folding "window" in leaves one masked body.
     // 4 = like 2 for a bias of any type (16-bit masks at inference; the selects of the conversion cost
     // the forward 2 %, so that training, whose backward kernels read fp32 anyway, keeps 2).
     constexpr bool kKeyBias = kBias == 2 || kBias == 4;
     AttnArgs a = a_in;
-    if constexpr (kWin == 0) a.window = 0;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     typedef typename Mma<T>::frag frag_t;
     typedef TileStage<T, DPAD, kBN, kThreads> Stage;
@@ -105,6 +103,8 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     int t_hi = (j_hi + kBN - 1) / kBN;
     if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
     const int n_tiles = t_hi - t_lo;
+    const TileOrder order = TileOrder::of<kBM, kBN>(a, q0, t_lo, t_hi);
+    const int first = order.first() * kBN;  // first key of the first tile
 
     // Start-up loads, all issued before any is used: the Q^T fragments (column i = this lane's
     // query, k-slots = 8 consecutive head-dim elements) and the first K / V tile.  Addresses are
@@ -120,8 +120,8 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
         for (int t = 0; t < DK; ++t)
             q_raw[t] = *reinterpret_cast<const u32x4_t*>(q_base + (int64_t)qr * a.qs[1] +
                                                          min(16 * t + 8 * g, a.d - 8));
-        ks.load(k_base, a.ks[1], t_lo * kBN, a.sk, a.d);
-        vs.load(v_base, a.vs[1], t_lo * kBN, a.sk, a.d);
+        ks.load(k_base, a.ks[1], first, a.sk, a.d);
+        vs.load(v_base, a.vs[1], first, a.sk, a.d);
         // Q is multiplied by scale * log2(e) once, here: the scores leave the matrix pipe in log2
         // units and no per-score multiplication is left in the tile body.
 #pragma unroll
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     // a bias could not: the masking value -FLT_MAX is no number of T; and the build for the other mask
     // geometries rounds as the one that reads stored bits does, which stands in for it wherever
     // there is a buffer for them.)
-    constexpr bool kRefInMma = kBias == 0 && kDrop == 1 && kWin == 0 && DPAD > 96;
+    constexpr bool kRefInMma = kBias == 0 && kDrop == 1 && DPAD > 96;
     constexpr float kRefUnit = std::is_same<T, f16_t>::value ? 64.f : 1.f;
     frag_t ones_frag, ref_frag;
 #pragma unroll
@@ -169,9 +169,9 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     if constexpr (kDrop != 0)
         drop_row_base = ((uint64_t)bh * a.sq + (uint64_t)q_row) * (uint64_t)a.sk;
     const float* bias_row = nullptr;
-    if constexpr (kBias == 1 || kBias == 3)  // (prepared rows exist past the end)
+    if constexpr (kBias == 1 || kBias == 3)  // (rows past the end: the last one)
         bias_row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1] +
-                   (int64_t)(kBias == 3 ? q_row : min(q_row, a.sq - 1)) * a.bs[2];
+                   (int64_t)min(q_row, a.sq - 1) * a.bs[2];
     // kKeyBias: thread (x & 63) carries key j0 + (x & 63) of the requested tile (all four
     // wavefronts alike, so that neither request nor store needs a branch)
     const float* bias_keys = nullptr;
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
         if constexpr (kKeyBias) bias_lds[slot * kBN + row_slot(lane)] = bias_log2(bias_stage);
     };
     const float* bias_tile = bias_lds;  // the slot of the tile in process
-    request_bias(t_lo * kBN);
+    request_bias(first);
 
     // per-lane LDS offsets (elements) that do not change from tile to tile
     const int k_off = pi_row(i_loc) * kPitch + 8 * g;
@@ -204,12 +204,6 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
         if (a.window > 0 && wq0 - (j0 + kBN - 1) >= a.window) return false;
         return true;
     };
-    auto tile_needs_mask = [&](int t) __attribute__((always_inline)) {
-        const int j0 = t * kBN;
-        return (j0 + kBN > a.sk) || (a.causal && j0 + kBN - 1 > wq0) ||
-               (a.window > 0 && wq_last - j0 >= a.window);
-    };
-
     // S^T half = K_half Q^T, in log2 units
     auto half_scores = [&](const T* kt, int kb, f32x16_t& s) __attribute__((always_inline)) {
 #pragma unroll
@@ -219,19 +213,20 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
         for (int x = 0; x < DK; ++x)
             s = Mma<T>::mma32(lds_frag<T>(kt + kb * 32 * kPitch + k_off + 16 * x), qf[x], s);
     };
-    // bias, masks and maximum of one half; mask_tag: 0 = every key visible, 1 = upper bound only
-    // (causal / key tail), 2 = both bounds (local window).  Returns this lane's maximum.
+    // bias, masks and maximum of one half; mask_tag: 0 = every key visible, 1 = the causal, window
+    // and tail bounds, as one bit per key: two instructions per score whatever the bounds are, so
+    // that one masked tile body serves every call.  Returns this lane's maximum.
     auto finish_half = [&](f32x16_t& s, int t, int kb, auto mask_tag)
                            __attribute__((always_inline)) -> float {
         constexpr int kMask = decltype(mask_tag)::value;
         const int j0 = t * kBN + 32 * kb;
-        // register r is key j0 + acc_row(r, g) = j0 + kAccGroupStep g + c with c = acc_row(r, 0);
-        // visible iff c_lo <= c <= c_hi
-        int c_lo = 0, c_hi = 0;
+        // register r is key j0 + acc_row(r, g) = j0 + kAccGroupStep g + c with c = acc_row(r, 0)
+        uint32_t visible = 0u;
         if constexpr (kMask != 0) {
             const int k_max = a.causal ? min(a.sk - 1, q_row) : a.sk - 1;
-            c_hi = k_max - j0 - kAccGroupStep * g;
-            if constexpr (kMask == 2) c_lo = q_row - a.window + 1 - j0 - kAccGroupStep * g;
+            const int k_min = a.window > 0 ? q_row - a.window + 1 : 0;
+            const int at = j0 + kAccGroupStep * g;
+            visible = visible_bits(k_min - at, k_max - at);
         }
         if constexpr (kBias == 1) {
             // Registers 8 h + e and 8 h + 4 + e are keys 2 g and 2 g + 1 of the aligned group of
@@ -272,14 +267,8 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
             }
             if constexpr (kMask != 0) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int c = acc_row(4 * r4 + e, 0);
-                    if constexpr (kMask == 2) {
-                        if (c > c_hi || c < c_lo) s[4 * r4 + e] = -INFINITY;
-                    } else {
-                        if (c > c_hi) s[4 * r4 + e] = -INFINITY;
-                    }
-                }
+                for (int e = 0; e < 4; ++e)
+                    s[4 * r4 + e] = keep_or_hide(s[4 * r4 + e], visible, acc_row(4 * r4 + e, 0));
             }
             mx = fmaxf(mx, fmaxf(fmaxf(s[4 * r4], s[4 * r4 + 1]),
                                  fmaxf(s[4 * r4 + 2], s[4 * r4 + 3])));
@@ -445,82 +434,49 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     };
 
     // ---- prologue: tile 0 into LDS ----
-    ks.fix(t_lo * kBN, a.sk, a.d);
-    vs.fix(t_lo * kBN, a.sk, a.d);
+    ks.fix(first, a.sk, a.d);
+    vs.fix(first, a.sk, a.d);
     ks.store(k_lds);
     vs.store(v_lds);
     store_bias(0);
     __syncthreads();
 
-    // Iteration r: request tile r+1, process tile r, write tile r+1 into the other slot.
-    // kFast iterations hold tiles that every wavefront of the workgroup sees in full.
+    // Iteration r: request the next tile, process tile r of the order, write the next tile into the
+    // other slot.  kFast iterations hold tiles that every wavefront of the workgroup sees in full.
+    int t = order.first();
     auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
         constexpr bool kFast = decltype(fast_tag)::value;
-        const int t = t_lo + r;
+        const int t_next = kFast ? order.after_fast(t) : order.after(t), next = t_next * kBN;
         const bool have_next = r + 1 < n_tiles;
         // the next tile is requested unconditionally (rows are clamped into the tensor; after the
         // last tile the request is wasted) so that it stays straight-line code.  Requesting it
         // later in the body saves no registers and measures slower.  (Addresses: a scalar tile
         // base plus a per-lane 32-bit offset that is selected, not multiplied out: 2 % faster than
         // the multiplied-out form now that the tile body has no other address arithmetic.)
-        ks.load(k_base, a.ks[1], (t + 1) * kBN, a.sk, a.d);
-        vs.load(v_base, a.vs[1], (t + 1) * kBN, a.sk, a.d);
-        request_bias((t + 1) * kBN);
+        ks.load(k_base, a.ks[1], next, a.sk, a.d);
+        vs.load(v_base, a.vs[1], next, a.sk, a.d);
+        request_bias(next);
         const T* kt = k_lds + (r & 1) * kTileElems;
         const T* vt = v_lds + (r & 1) * kTileElems;
         bias_tile = bias_lds + (r & 1) * kBN;
         if constexpr (kFast) {
             tile_body(kt, vt, t, std::integral_constant<int, 0>{});
         } else {
-            if (tile_active(t)) {
-                if (!tile_needs_mask(t))
-                    tile_body(kt, vt, t, std::integral_constant<int, 0>{});
-                else if constexpr (kWin == 1)  // one masked body per build: both bounds
-                    tile_body(kt, vt, t, std::integral_constant<int, 2>{});
-                else if (kWin == 2 && a.window > 0)
-                    tile_body(kt, vt, t, std::integral_constant<int, 2>{});
-                else
-                    tile_body(kt, vt, t, std::integral_constant<int, 1>{});
-            }
+            if (tile_active(t)) tile_body(kt, vt, t, std::integral_constant<int, 1>{});
         }
         if (have_next) {
-            ks.fix((t + 1) * kBN, a.sk, a.d);
-            vs.fix((t + 1) * kBN, a.sk, a.d);
+            ks.fix(next, a.sk, a.d);
+            vs.fix(next, a.sk, a.d);
             ks.store(k_lds + ((r + 1) & 1) * kTileElems);
             vs.store(v_lds + ((r + 1) & 1) * kTileElems);
             store_bias((r + 1) & 1);
         }
         __syncthreads();
+        t = t_next;
     };
-    // tiles that need neither mask nor activity test for any of the 128 queries: the leading
-    // ones without a local window, a run in the middle of the key range with one
-    if constexpr (kWin != 1) {
-        int n_fast = 0;
-        if (a.window <= 0 && q0 + kBM <= a.sq) {
-            n_fast = a.sk / kBN;
-            if (a.causal) n_fast = min(n_fast, (q0 + 1) / kBN);
-            n_fast = min(n_fast - t_lo, n_tiles);
-        }
-        int r = 0;
-        for (; r < n_fast; ++r) iteration(r, std::true_type{});
-        for (; r < n_tiles; ++r) iteration(r, std::false_type{});
-    } else {
-        int f_lo = 0, f_hi = 0;  // iterations [f_lo, f_hi) are fast
-        if (q0 + kBM <= a.sq) {
-            int t_end = a.sk / kBN;  // first tile that is incomplete or hidden from some query
-            if (a.causal) t_end = min(t_end, (q0 + 1) / kBN);
-            // the last query of the workgroup sees keys >= q0 + kBM - window
-            const int t_begin = (max(q0 + kBM - a.window, 0) + kBN - 1) / kBN;
-            f_lo = min(max(t_begin - t_lo, 0), n_tiles);
-            f_hi = min(max(t_end - t_lo, f_lo), n_tiles);
-        }
-        for (int r = 0; r < n_tiles; ++r) {
-            if (r >= f_lo && r < f_hi)
-                iteration(r, std::true_type{});
-            else
-                iteration(r, std::false_type{});
-        }
-    }
+    int r = 0;
+    for (; r < order.end - order.begin; ++r) iteration(r, std::true_type{});
+    for (; r < n_tiles; ++r) iteration(r, std::false_type{});
 
     // ---- epilogue ----
     const float l_tot = sum_xor32(l_run);
@@ -553,7 +509,7 @@ __global__ __launch_bounds__(kThreads, fwd_per_cu(DPAD, kBias, kDrop)) void attn
     }
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, int kWin, int kSteps>
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu = fwd_per_cu(DPAD)>
 int launch(const AttnArgs& a, hipStream_t st) {
     typedef TileStage<T, DPAD, kBN, kThreads> Stage;
     const size_t smem = (size_t)4 * kBN * Stage::kPitch * sizeof(T) +
@@ -561,7 +517,11 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const int n_qt = (a.sq + kBM - 1) / kBM;
     const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    auto kern = attn_fwd_kernel<T, DPAD, kBias, kDrop, kWin, kSteps>;
+    if constexpr (DPAD <= 64 && kBias == 0 && kDrop == 0 && kPerCu < kFwdFour) {
+        if (blocks > (int64_t)kPerCu * a.n_cus)
+            return launch<T, DPAD, kBias, kDrop, kSteps, kFwdFour>(a, st);
+    }
+    auto kern = attn_fwd_kernel<T, DPAD, kBias, kDrop, kSteps, kPerCu>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
@@ -570,51 +530,26 @@ int launch(const AttnArgs& a, hipStream_t st) {
     // long there and a group's late heavy ones become the tail: 314 -> 350 us at bf16 B4 S2048 H32
     // D80 causal, p 0.1, 588 -> 667 us at fp16 B2 S4096 H32 D96)
     if (a.n_split == 1)
-        set_dispatch_order(&ordered, blocks, fwd_per_cu(DPAD, kBias, kDrop), kDrop == 0);
+        set_dispatch_order(&ordered, blocks, kPerCu, kDrop == 0);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, ordered);
     return check_launch();
 }
 
-template <typename T, int DPAD, int kWin, int kSteps>
-int dispatch_nobias(const AttnArgs& a, hipStream_t st) {
-    if (a.dropout == 1) return launch<T, DPAD, 0, 1, kWin, kSteps>(a, st);
-    if (a.dropout == 2) return launch<T, DPAD, 0, 2, kWin, kSteps>(a, st);
-    if (a.dropout == 3) return launch<T, DPAD, 0, 3, kWin, kSteps>(a, st);
-    return launch<T, DPAD, 0, 0, kWin, kSteps>(a, st);
+template <typename T, int DPAD, int kBias, int kSteps>
+int dispatch_drop(const AttnArgs& a, hipStream_t st) {
+    if (a.dropout == 1) return launch<T, DPAD, kBias, 1, kSteps>(a, st);
+    if (a.dropout == 2) return launch<T, DPAD, kBias, 2, kSteps>(a, st);
+    if (a.dropout == 3) return launch<T, DPAD, kBias, 3, kSteps>(a, st);
+    return launch<T, DPAD, kBias, 0, kSteps>(a, st);
 }
 template <typename T, int DPAD, int kSteps = DPAD / 16>
 int dispatch_flags(const AttnArgs& a, hipStream_t st) {
-    if (a.has_bias) {
-        // one build for both: with a bias the window-free build measured slower (it spills more
-        // at head_dim 64 and 96: 266 against 185 us at bf16 B4 S2048 H32 D80 with a padding mask)
-        if (a.bias_type == SLAPO_BIAS_PREPARED) {
-            if (a.dropout == 1) return launch<T, DPAD, 3, 1, 2, kSteps>(a, st);
-            if (a.dropout == 2) return launch<T, DPAD, 3, 2, 2, kSteps>(a, st);
-            if (a.dropout == 3) return launch<T, DPAD, 3, 3, 2, kSteps>(a, st);
-            return a.window <= 0 ? launch<T, DPAD, 3, 0, 0, kSteps>(a, st)
-                                 : launch<T, DPAD, 3, 0, 2, kSteps>(a, st);
-        }
-        if (a.bias_type != SLAPO_F32)  // one value per key, no dropout (checked by the caller)
-            return a.window <= 0 ? launch<T, DPAD, 4, 0, 0, kSteps>(a, st)
-                                 : launch<T, DPAD, 4, 0, 2, kSteps>(a, st);
-        if (a.bs[2] == 0) {  // the bias depends on the key only
-            if (a.dropout == 1)
-                return a.window <= 0 ? launch<T, DPAD, 2, 1, 0, kSteps>(a, st)
-                                     : launch<T, DPAD, 2, 1, 2, kSteps>(a, st);
-            if (a.dropout == 2) return launch<T, DPAD, 2, 2, 2, kSteps>(a, st);
-            if (a.dropout == 3)
-                return a.window <= 0 ? launch<T, DPAD, 2, 3, 0, kSteps>(a, st)
-                                     : launch<T, DPAD, 2, 3, 2, kSteps>(a, st);
-            if (a.window <= 0) return launch<T, DPAD, 2, 0, 0, kSteps>(a, st);
-            return launch<T, DPAD, 2, 0, 2, kSteps>(a, st);
-        }
-        if (a.dropout == 1) return launch<T, DPAD, 1, 1, 2, kSteps>(a, st);
-        if (a.dropout == 2) return launch<T, DPAD, 1, 2, 2, kSteps>(a, st);
-        if (a.dropout == 3) return launch<T, DPAD, 1, 3, 2, kSteps>(a, st);
-        return launch<T, DPAD, 1, 0, 2, kSteps>(a, st);
-    }
-    return a.window > 0 ? dispatch_nobias<T, DPAD, 1, kSteps>(a, st)
-                        : dispatch_nobias<T, DPAD, 0, kSteps>(a, st);
+    if (!a.has_bias) return dispatch_drop<T, DPAD, 0, kSteps>(a, st);
+    if (a.bias_type == SLAPO_BIAS_PREPARED) return dispatch_drop<T, DPAD, 3, kSteps>(a, st);
+    // one value per key of a 16-bit type, no dropout (checked by the caller)
+    if (a.bias_type != SLAPO_F32) return launch<T, DPAD, 4, 0, kSteps>(a, st);
+    return a.bs[2] == 0 ? dispatch_drop<T, DPAD, 2, kSteps>(a, st)  // it depends on the key only
+                        : dispatch_drop<T, DPAD, 1, kSteps>(a, st);
 }
 
 template <typename T>

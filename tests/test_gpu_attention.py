@@ -535,6 +535,34 @@ def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
     return ref, qf.grad, kf.grad, vf.grad
 
 
+@pytest.mark.parametrize("mask", ["none", "key", "square"])
+@pytest.mark.parametrize("shape,causal,window,p", [
+    ((2, 450, 3, 64), True, 0, 0.0),     # wavefronts past the last row and key in full tiles
+    ((1, 193, 2, 80), False, 0, 0.1),    # ... of every tile
+    ((2, 700, 2, 128), True, 200, 0.1),  # a run of full tiles in the middle, masked ones on both sides
+    ((1, 449, 2, 96), True, 70, 0.0),    # a window without full tiles
+    ((1, 330, 2, 32), False, 100, 0.0),  # a window without a causal mask
+    ((2, 450, 40, 96), True, 0, 0.1),    # more key blocks than CUs: two workgroups of dK/dV per CU
+    ((5, 770, 24, 64), True, 0, 0.0),    # more than three workgroups of the forward per CU
+])
+def test_order_and_masks_of_the_tiles(shape, causal, window, p, mask):
+    """Full tiles first, one masked body for the others: outputs and gradients against the fp32 kernels
+    on the same 16-bit values and seed, at sizes with remainders on either side."""
+    b, s, h, d = shape
+    q, k, v, do, g = _inputs(b, s, h, d, torch.bfloat16)
+    q, k, v, do = (t.cuda() for t in (q, k, v, do))
+    m = None
+    if mask != "none":
+        m = torch.randn(b, 1, 1 if mask == "key" else s, s, generator=g).bfloat16().cuda()
+    qh, kh, vh = (t.clone().requires_grad_(True) for t in (q, k, v))
+    torch.cuda.manual_seed(3)
+    out = op.hip_attention(qh, kh, vh, m, causal=causal, p=p, window=window)
+    out.backward(do)
+    ref, rq, rk, rv = _fp32_twin(q, k, v, do, m, causal, window, p, 3)
+    for a, r in ((out, ref), (qh.grad, rq), (kh.grad, rk), (vh.grad, rv)):
+        assert rel_err(a, r) <= 2e-2
+
+
 def test_full_size_cfg4_properties():
     """bf16, B 4, S 2048, 32 x 80, causal + key padding with valid lengths ~ U[512, 2048], at full
     size: rows of P sum to one (V = 1 returns 1, also for queries in the padded region); query 0
