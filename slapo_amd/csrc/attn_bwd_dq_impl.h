@@ -35,14 +35,17 @@ constexpr int kBN = 64;
 constexpr int kKRing = 2;
 constexpr int kVRing = 2;
 
-// kStagger (see the tile bodies below): up to head_dim 64; above, sequential halves are what fits two
-// workgroups per CU.
+// kStagger (see the tile bodies below): at head_dim 33-64; above, sequential halves are what fits two
+// workgroups per CU, and below, three (fp16 B8 S1024 H16 D32 padded, forward and backward: 144 -> 129
+// us, the staggered build spills 20 registers; with stored dropout bits it spills none and is the
+// faster one, bf16 B3 S1845 H6 D32, p 0.1: 212 -> 205).
+constexpr int dq_per_cu(int dpad) { return dpad <= 32 ? 3 : 2; }
 // kBias: 0 = no additive bias, 1 = any layout (read from memory per score), 2 = the bias depends on
 // the key only (stride 0 over the queries): its 64 values per key tile travel through LDS beside
 // the K / V tile, and the tile bodies have neither global loads nor branches for them.
 template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
-__global__ __launch_bounds__(kThreads, 2) void attn_bwd_dq_kernel(const AttnArgs a_in) {
-    constexpr bool kStagger = DPAD <= 64;
+__global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(const AttnArgs a_in) {
+    constexpr bool kStagger = DPAD == 64 || (DPAD == 32 && kDrop == 3 && kBias == 0);
     AttnArgs a = a_in;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     typedef typename Mma<T>::frag frag_t;
@@ -532,7 +535,7 @@ int launch(const AttnArgs& a, hipStream_t st) {
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
-    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, 2);
+    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, dq_per_cu(DPAD));
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kThreads), smem, st, ordered);
     return check_launch();
 }
@@ -565,6 +568,7 @@ int dispatch_flags(const AttnArgs& a, hipStream_t st) {
 
 template <typename T>
 int dispatch(const AttnArgs& a, hipStream_t st) {
+    if (a.d <= 32) return dispatch_flags<T, 32>(a, st);
     if (a.d <= 64) return dispatch_flags<T, 64>(a, st);
     if (a.d <= 80) return dispatch_flags<T, 96, 5>(a, st);  // five k-steps cover head_dim 80
     if (a.d <= 96) return dispatch_flags<T, 96>(a, st);

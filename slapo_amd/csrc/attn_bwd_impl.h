@@ -47,19 +47,19 @@ struct BwdSmem {
     static constexpr size_t kBytes = 2 * kQBytes + kStatBytes + kMaskBytes;
 };
 
-// Two workgroups per CU up to DPAD 96, one at 128 (192 resident accumulator / fragment registers).  At
+// Workgroups per CU: three up to DPAD 32, two up to 96, one at 128 (192 resident accumulator / fragment registers).  At
 // 96 with the forward's keep bits both are built: two where a call has more key blocks than CUs
 // (fp16 B5 S920 H31 D80 window 356, p 0.1, forward and backward 256 -> 226 us; bf16 B4 S2048 H12 D96
 // causal, p 0.1 322 -> 292), else one, whose staggered body is the faster of the two (fp16 B2 S1600 H8
 // D96 padded, p 0.1, 208 blocks dealt to 416 workgroups: 168 against 173 us; B1 S2048 H12 D96 175
 // against 181).
-constexpr bool bwd_two_per_cu(int dpad, int kb) { return kb == 1 && dpad <= 96; }
+constexpr int bwd_per_cu(int dpad) { return dpad <= 32 ? 3 : dpad <= 96 ? 2 : 1; }
 
 // KB = blocks of 32 keys per wavefront.  KB = 2 halves the LDS operand traffic per matrix
 // instruction (every Q / dO fragment read feeds two MFMAs) at the price of twice the resident
 // fragments and accumulators, i.e. one wavefront per SIMD instead of two.
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, bool kTwo>
-__global__ __launch_bounds__(kBwdThreads, (kTwo ? 2 : 1)) void attn_bwd_kernel(
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
+__global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(
     const AttnArgs a_in) {
     AttnArgs a = a_in;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
@@ -557,7 +557,7 @@ __global__ __launch_bounds__(kBwdThreads, (kTwo ? 2 : 1)) void attn_bwd_kernel(
     auto fast_iteration = [&](int t) __attribute__((always_inline)) {
         constexpr bool kLateRequest = DPAD <= 64;  // two workgroups share a CU: registers scarce
         if constexpr (!kLateRequest) request_tile(regs, t + 1);
-        if constexpr (DPAD == 96 && kTwo)
+        if constexpr (DPAD == 96 && kPerCu == 2)
             sequential_tile(t);
         else
             staggered_tile(t, std::integral_constant<int, 0>{},
@@ -653,7 +653,7 @@ __global__ __launch_bounds__(kBwdThreads, (kTwo ? 2 : 1)) void attn_bwd_kernel(
     }
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, bool kTwo>
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
 int launch(const AttnArgs& a, hipStream_t st) {
     typedef BwdSmem<T, DPAD> SM;
     const size_t smem = SM::kBytes;
@@ -661,12 +661,12 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const int n_kt = (a.sk + kBN - 1) / kBN;
     const int64_t blocks = (int64_t)n_kt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps, kTwo>;
+    auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps, kPerCu>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
-    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, kTwo ? 2 : 1);
+    if (a.n_split == 1) set_dispatch_order(&ordered, blocks, kPerCu);
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBwdThreads), smem, st, ordered);
     return check_launch();
 }
@@ -679,9 +679,9 @@ int launch_kb(const AttnArgs& a, hipStream_t st) {
     if constexpr (DPAD == 96 && kDrop == 3) {
         const int64_t blocks =
             (int64_t)((a.sk + kBwdWaves * 32 - 1) / (kBwdWaves * 32)) * a.batch * a.heads;
-        if (blocks <= a.n_cus) return launch<T, DPAD, kBias, kDrop, 1, kSteps, false>(a, st);
+        if (blocks <= a.n_cus) return launch<T, DPAD, kBias, kDrop, 1, kSteps, 1>(a, st);
     }
-    return launch<T, DPAD, kBias, kDrop, 1, kSteps, bwd_two_per_cu(DPAD, 1)>(a, st);
+    return launch<T, DPAD, kBias, kDrop, 1, kSteps, bwd_per_cu(DPAD)>(a, st);
 }
 
 template <typename T, int DPAD, int kBias, int kSteps>
@@ -702,6 +702,7 @@ int dispatch_flags(const AttnArgs& a, hipStream_t st) {
 
 template <typename T>
 int dispatch(const AttnArgs& a, hipStream_t st) {
+    if (a.d <= 32) return dispatch_flags<T, 32>(a, st);
     if (a.d <= 64) return dispatch_flags<T, 64>(a, st);
     if (a.d <= 80) return dispatch_flags<T, 96, 5>(a, st);  // five k-steps cover head_dim 80
     if (a.d <= 96) return dispatch_flags<T, 96>(a, st);

@@ -33,10 +33,10 @@ constexpr int kBM = kWaves * 32;
 constexpr int kBN = 64;
 constexpr float kMaxSlack = 8.0f;  // hysteresis of the softmax reference, log2 units
 
-// Workgroups per CU: three in 168 registers up to head_dim 64, two above (three at 96 spill 2 to 54
+// Workgroups per CU: four in 128 registers up to head_dim 32, three in 168 up to 64, two above (three at 96 spill 2 to 54
 // registers: bf16 B2 S3000 H20 D80 padded 147 -> 185 us).
-constexpr int fwd_per_cu(int dpad) { return dpad <= 64 ? 3 : 2; }
-// Without bias and dropout four fit in 128 registers, which pays where the launch fills them: from the
+constexpr int fwd_per_cu(int dpad) { return dpad <= 32 ? 4 : dpad <= 64 ? 3 : 2; }
+// At 64 without bias and dropout four fit in 128 registers, which pays where the launch fills them: from the
 // first workgroup that three a CU would not hold on (fp16 B8 S1024 H16 D64 causal, 1024 workgroups:
 // 30.9 -> 29.8 us, bf16 B2 S4096 H16 D64 causal 88.4 -> 83.5; bf16 B1 S8192 H8 D64, 512: 167 -> 169).
 constexpr int kFwdFour = 4;
@@ -554,6 +554,9 @@ int dispatch_flags(const AttnArgs& a, hipStream_t st) {
 
 template <typename T>
 int dispatch(const AttnArgs& a, hipStream_t st) {
+    // (head_dim 32 in the 64-wide kernels multiplies zeros half the time and holds them in registers and
+    // LDS; forward and backward fp16 B8 S1024 H16 D32 causal 110 -> 82 us, bf16 B2 S4096 310 -> 214)
+    if (a.d <= 32) return dispatch_flags<T, 32>(a, st);
     if (a.d <= 64) return dispatch_flags<T, 64>(a, st);
     if (a.d <= 80) return dispatch_flags<T, 96, 5>(a, st);  // five k-steps cover head_dim 80
     if (a.d <= 96) return dispatch_flags<T, 96>(a, st);

@@ -542,6 +542,7 @@ def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
     ((2, 700, 2, 128), True, 200, 0.1),  # a run of full tiles in the middle, masked ones on both sides
     ((1, 449, 2, 96), True, 70, 0.0),    # a window without full tiles
     ((1, 330, 2, 32), False, 100, 0.0),  # a window without a causal mask
+    ((3, 201, 3, 24), True, 0, 0.1),     # the kernels for head_dim 32 with columns to spare
     ((2, 450, 40, 96), True, 0, 0.1),    # more key blocks than CUs: two workgroups of dK/dV per CU
     ((5, 770, 24, 64), True, 0, 0.0),    # more than three workgroups of the forward per CU
 ])
