@@ -319,15 +319,19 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
         }
     };
     // dS^T half = P^T (dP^T - delta), packed to T
-    // kDrop == 3: the keep bits of this lane's query for one half of 32 keys, as the forward
-    // stored them (requested at the top of a tile body, used in half_ds)
-    auto mask_word = [&](int t, int kb) __attribute__((always_inline)) -> uint32_t {
+    // kDrop == 3: the keep bits of this lane's query for the two halves of a tile, as the forward stored
+    // them.  Requested a tile ahead and before the tile's K / V: loads return in order, so that a word
+    // requested after them would make dS wait for the whole next tile.
+    uint32_t tile_bits[2] = {0u, 0u}, next_bits[2] = {0u, 0u};
+    auto request_bits = [&](int t) __attribute__((always_inline)) {
         if constexpr (kDrop == 3) {
-            const int w = min(2 * t + kb, a.mask_words - 1);
-            return a.keep_mask[((int64_t)bh * a.mask_words + w) * a.mask_pitch +
-                               min(q_row, a.sq - 1)];
+            const int64_t base = (int64_t)bh * a.mask_words;
+            const int row = min(q_row, a.sq - 1);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                next_bits[kb] =
+                    a.keep_mask[(base + min(2 * t + kb, a.mask_words - 1)) * a.mask_pitch + row];
         }
-        return 0u;
     };
     auto half_ds = [&](const f32x16_t& p, const f32x16_t& dp, int t, int kb, uint32_t mword,
                        uint32_t (&dw)[8]) __attribute__((always_inline)) {
@@ -373,27 +377,25 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
             uint32_t dw0[8];
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb) {
-                const uint32_t mw = mask_word(t, kb);
                 half_s(kt, kb, s0);
                 half_dp(vt, kb, p0);
                 half_exp(s0, t, kb, mask_tag);
-                half_ds(s0, p0, t, kb, mw, dw0);
+                half_ds(s0, p0, t, kb, tile_bits[kb], dw0);
                 half_dq(kt, kb, dw0);
             }
             return;
         }
         f32x16_t s0, s1, p0, p1;
         uint32_t dw0[8], dw1[8];
-        const uint32_t mw0 = mask_word(t, 0), mw1 = mask_word(t, 1);
         half_s(kt, 0, s0);
         half_dp(vt, 0, p0);
         half_exp(s0, t, 0, mask_tag);
         half_s(kt, 1, s1);
-        half_ds(s0, p0, t, 0, mw0, dw0);
+        half_ds(s0, p0, t, 0, tile_bits[0], dw0);
         half_dp(vt, 1, p1);
         half_exp(s1, t, 1, mask_tag);
         half_dq(kt, 0, dw0);
-        half_ds(s1, p1, t, 1, mw1, dw1);
+        half_ds(s1, p1, t, 1, tile_bits[1], dw1);
         half_dq(kt, 1, dw1);
     };
 
@@ -435,7 +437,6 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
                     dq_acc[x] = Mma<T>::mma32(f[s2 * DV + x], df, dq_acc[x]);
             }
         };
-        const uint32_t mw0 = mask_word(t, 0), mw1 = mask_word(t, 1);
         rows(kt, 0, kr0);
         rows(vt, 0, vr0);
         __builtin_amdgcn_sched_barrier(0);
@@ -451,11 +452,11 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
         __builtin_amdgcn_sched_barrier(0);
         cols(1, kq1);
         mma_rows(vr1, gf, dp_init, p1);
-        half_ds(s0, p0, t, 0, mw0, dw0);
+        half_ds(s0, p0, t, 0, tile_bits[0], dw0);
         __builtin_amdgcn_sched_barrier(0);
         mma_cols(kq0, dw0);
         half_exp(s1, t, 1, mask_tag);
-        half_ds(s1, p1, t, 1, mw1, dw1);
+        half_ds(s1, p1, t, 1, tile_bits[1], dw1);
         __builtin_amdgcn_sched_barrier(0);
         mma_cols(kq1, dw1);
     };
@@ -474,10 +475,13 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
     // other ring slot.  kFast iterations hold tiles that every wavefront of the workgroup sees in
     // full; the others test activity per wavefront and mask.
     int t = order.first();
+    request_bits(t);
     auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
         constexpr bool kFast = decltype(fast_tag)::value;
         const int next = kFast ? order.after_fast(t) : order.after(t);
         const bool have_next = r + 1 < n_tiles;
+        tile_bits[0] = next_bits[0], tile_bits[1] = next_bits[1];
+        request_bits(next);
         if (have_next) {
             request(next * kBN);
         }

@@ -547,6 +547,7 @@ __global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(
         half_exp(s1, lse_t + 32, i0 + 32, mask_tag);
         if constexpr (kRequestInside) {
             request_tile(regs, t + 1);
+            pin_requests();
         }
         half_out(qt, gt, 0, pw0, dw0);
         half_ds(s1, p1, delta_t + 32, mask_t + 32, i0 + 32, pw1, dw1);
@@ -556,7 +557,13 @@ __global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(
     // t+1, process tile t as one straight block, write tile t+1 into the other buffer.
     auto fast_iteration = [&](int t) __attribute__((always_inline)) {
         constexpr bool kLateRequest = DPAD <= 64;  // two workgroups share a CU: registers scarce
-        if constexpr (!kLateRequest) request_tile(regs, t + 1);
+        if constexpr (!kLateRequest) {
+            request_tile(regs, t + 1);
+            // (not at head_dim 65-96 without dropout, where the registers that they hold on to spill:
+            // bf16 B10 S577 H16 D80 causal, forward and backward 107.4 -> 109.6 us.  Elsewhere: bf16 B3
+            // S777 H12 D64 padded, p 0.1 87.1 -> 85, bf16 B2 S1024 H12 D80, p 0.1 130.4 -> 126.7)
+            if constexpr (!(DPAD == 96 && kDrop == 0)) pin_requests();
+        }
         if constexpr (DPAD == 96 && kPerCu == 2)
             sequential_tile(t);
         else

@@ -518,6 +518,11 @@ __device__ __forceinline__ void store_partial(const f32x16_t (&acc)[DPAD / 32], 
         }
 }
 
+// Keeps loads that have been requested above this point from sinking below it.  Where what they return
+// is used in one branch only (the next tile's stores, skipped after the last tile) the compiler moves
+// the requests themselves into that branch, behind the tile body that they were meant to overlap.
+__device__ __forceinline__ void pin_requests() { asm volatile("" ::: "memory"); }
+
 // Stage a [ROWS x DPAD] tile of T (rows row0.., zero beyond n_rows / beyond d) through registers.
 // The global loads are unconditional (out-of-range rows are clamped to the last valid row and
 // zeroed when the tile is written to LDS), so they stay in the caller's basic block and the

@@ -393,20 +393,26 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
                     o_acc[x]);
         }
     };
+    // kDrop == 3: the keep bits of this lane's query for the two halves of a tile, drawn by
+    // keep_mask_kernel.  Requested a tile ahead and before the tile's K / V: loads return in order, so
+    // that a word requested after them would make the probabilities wait for the whole next tile.
+    uint32_t tile_bits[2] = {0u, 0u}, next_bits[2] = {0u, 0u};
+    auto request_bits = [&](int t) __attribute__((always_inline)) {
+        if constexpr (kDrop == 3) {
+            const int64_t base = (int64_t)bh * a.mask_words;
+            const int row = min(q_row, a.sq - 1);
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+                next_bits[kb] =
+                    a.keep_mask[(base + min(2 * t + kb, a.mask_words - 1)) * a.mask_pitch + row];
+        }
+    };
     auto tile_body = [&](const T* kt, const T* vt, int t, auto mask_tag)
                          __attribute__((always_inline)) {
         f32x16_t s0, s1;
         uint32_t pw0[8], pw1[8];
         uint32_t bits0 = 0, bits1 = 0;
-        if constexpr (kDrop == 3) {
-            // the keep bits of this lane's query for the two halves of the tile, drawn by
-            // keep_mask_kernel; requested first, used after the scores
-            const int w = 2 * t;
-            const int64_t base = (int64_t)bh * a.mask_words;
-            const int row = min(q_row, a.sq - 1);
-            bits0 = a.keep_mask[(base + min(w, a.mask_words - 1)) * a.mask_pitch + row];
-            bits1 = a.keep_mask[(base + min(w + 1, a.mask_words - 1)) * a.mask_pitch + row];
-        }
+        if constexpr (kDrop == 3) bits0 = tile_bits[0], bits1 = tile_bits[1];
         half_scores(kt, 0, s0);
         half_scores(kt, 1, s1);
         const float mx =
@@ -444,10 +450,13 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     // Iteration r: request the next tile, process tile r of the order, write the next tile into the
     // other slot.  kFast iterations hold tiles that every wavefront of the workgroup sees in full.
     int t = order.first();
+    request_bits(t);
     auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
         constexpr bool kFast = decltype(fast_tag)::value;
         const int t_next = kFast ? order.after_fast(t) : order.after(t), next = t_next * kBN;
         const bool have_next = r + 1 < n_tiles;
+        tile_bits[0] = next_bits[0], tile_bits[1] = next_bits[1];
+        request_bits(t_next);
         // the next tile is requested unconditionally (rows are clamped into the tensor; after the
         // last tile the request is wasted) so that it stays straight-line code.  Requesting it
         // later in the body saves no registers and measures slower.  (Addresses: a scalar tile
