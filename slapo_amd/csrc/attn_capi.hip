@@ -30,7 +30,7 @@ namespace {
 // kernels: thread (row i, word w) draws the eight Philox blocks of keys 32 w .. 32 w + 31 of
 // query i and stores them as one word, keep_mask[(bh * mask_words + w) * mask_pitch + i], bit j =
 // keep(i, 32 w + j).  The matrix kernels then only test bits; drawing inside the forward kernel
-// costs about seventy vector-ALU cycles per score (61 instructions per block of four) beside
+// costs about fifty vector-ALU cycles per score (47 instructions per block of four) beside
 // thirty-two (head_dim 128) or sixteen (64) of matrix work.  Only words that hold a key the row itself can see are drawn: the kernels read
 // whole words of every 64-key tile that some query of a 32-query group sees, but a bit that
 // belongs to a pair outside the row's own mask meets a probability of zero, so what such words
@@ -43,7 +43,7 @@ namespace {
 // forward and backward 199 us before, 89 us with this kernel ahead of the forward.  The words of
 // padded keys are left as they are too where the other kernels skip their tiles (a third of them in
 // that call's mask).  Units of 64 rows and a word, dealt to the wavefronts one after the other: blocks
-// of 256 rows left a quarter of the launch to nine rows at S777.  That call: 22.1 -> 17.3 us.
+// of 256 rows left a quarter of the launch to nine rows at S777.  That call: 22.1 -> 17.3 us (14.1 with PhiloxCall).
 template <bool kExact>
 __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in, int words) {
     AttnArgs a = a_in;
@@ -75,17 +75,8 @@ __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in, int
         return;  // (without a window: every word of a 64-key tile that the row's group visits)
     }
     const uint64_t row_base = ((uint64_t)bh * a.sq + (uint64_t)i) * (uint64_t)a.sk;
-    uint32_t word = 0;
-    if constexpr (kExact) {
-        word = dropout_keep_run(a.rng, row_base + 32 * (uint64_t)w, 32);
-    } else {
-#pragma unroll
-        for (int blk = 0; blk < 8; ++blk) {
-            const int key0 = 32 * w + 4 * blk;
-            if (key0 < a.sk)
-                word |= dropout_keep4_pow2(a.rng, (row_base + (uint64_t)key0) >> 2) << (4 * blk);
-        }
-    }
+    const uint64_t elem = row_base + 32 * (uint64_t)w;
+    const uint32_t word = dropout_keep_run<32, !kExact>(a.rng, elem);
     a.keep_mask[((int64_t)bh * a.mask_words + w) * a.mask_pitch + i] = word;
 }
 

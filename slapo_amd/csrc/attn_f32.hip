@@ -302,8 +302,7 @@ template <int kKeys>
 __device__ __forceinline__ uint32_t keep_keys(const AttnArgs& a, int bh, int i, int j) {
     const uint64_t e = ((uint64_t)bh * a.sq + (uint64_t)i) * (uint64_t)a.sk + (uint64_t)j;
     if (i >= a.sq || j >= a.sk) return 0;
-    if (a.dropout != 1)
-        return dropout_keep_run(a.rng, e, min(kKeys, a.sk - j)) & ((1u << kKeys) - 1u);
+    if (a.dropout != 1) return dropout_keep_run<kKeys>(a.rng, e);
     uint32_t bits = dropout_keep4_pow2(a.rng, e >> 2);
 #pragma unroll
     for (int k = 4; k < kKeys; k += 4)

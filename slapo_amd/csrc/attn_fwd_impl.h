@@ -328,8 +328,32 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     // Keep bits of this lane's query for the 32 keys from j0 on (bit j = key j0 + j), drawn here:
     // Philox blocks cover four consecutive keys; the two lanes of a query (l, l ^ 32) draw the
     // blocks of keys 8 g .. 8 g + 7 of each 16-key group and exchange them.
+    // Where the 32 rows of the wavefront lie within one call of the generator (all but a few: a call
+    // covers 4 T elements), what the call's blocks share sits in scalar registers (PhiloxCall).
+    bool one_call = false;
+    PhiloxCall call = {};
+    uint32_t row_thread = 0;
+    if constexpr (kDrop == 1) {
+        const uint64_t first = ((uint64_t)bh * a.sq + (uint64_t)min(wq0, a.sq - 1)) * (uint64_t)a.sk >> 2;
+        const uint64_t last = (((uint64_t)bh * a.sq + (uint64_t)wq_last + 1) * (uint64_t)a.sk - 1) >> 2;
+        one_call = philox_call_fits(a.rng) && first >> a.rng.t_shift == last >> a.rng.t_shift;
+        call = philox_call(a.rng.base_counter + (first >> a.rng.t_shift), a.rng.key0, a.rng.key1);
+        row_thread = (uint32_t)(drop_row_base >> 2) & (uint32_t)(a.rng.total_threads - 1);
+    }
     auto draw_half = [&](int j0) __attribute__((always_inline)) -> uint32_t {
         uint32_t mine = 0;
+        if constexpr (kDrop == 1) {
+            if (__builtin_expect(one_call, 1)) {
+#pragma unroll
+                for (int h2 = 1; h2 >= 0; --h2) {
+                    const uint32_t thread = row_thread + (uint32_t)(j0 + 16 * h2 + 8 * g) / 4;
+                    uint32_t bits = push_keep4(0u, philox_block(call, thread + 1), a.rng.keep_max);
+                    bits = push_keep4(bits, philox_block(call, thread), a.rng.keep_max);
+                    mine = mine << 16 | bits;
+                }
+                return or_xor32(mine << (8 * g));
+            }
+        }
 #pragma unroll
         for (int blk = 0; blk < 4; ++blk) {
             const int pos = 16 * (blk >> 1) + 8 * g + 4 * (blk & 1);
