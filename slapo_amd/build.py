@@ -48,6 +48,8 @@ PER_FILE_FLAGS = {
     "attn_bwd_bf16.hip": ["-fno-honor-nans"],
     "attn_bwd_dq_f16.hip": ["-fno-honor-nans"],
     "attn_bwd_dq_bf16.hip": ["-fno-honor-nans"],
+    "attn_bwd_both_f16.hip": ["-fno-honor-nans"],
+    "attn_bwd_both_bf16.hip": ["-fno-honor-nans"],
 }
 
 

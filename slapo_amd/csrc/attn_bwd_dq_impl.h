@@ -43,10 +43,11 @@ constexpr int dq_per_cu(int dpad) { return dpad <= 32 ? 3 : 2; }
 // kBias: 0 = no additive bias, 1 = any layout (read from memory per score), 2 = the bias depends on
 // the key only (stride 0 over the queries): its 64 values per key tile travel through LDS beside
 // the K / V tile, and the tile bodies have neither global loads nor branches for them.
-template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
-__global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(const AttnArgs a_in) {
+// kDelta: computes delta = rowsum(dO * O) of its rows and stores it for the dK / dV kernel; otherwise it
+// has been stored (delta_kernel).  Workgroup `block` of `n_blocks`.
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps, bool kDelta>
+__device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     constexpr bool kStagger = DPAD == 64 || (DPAD == 32 && kDrop == 3 && kBias == 0);
-    AttnArgs a = a_in;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     typedef typename Mma<T>::frag frag_t;
     typedef TileStage<T, DPAD, kBN, kThreads> Stage;
@@ -65,7 +66,7 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
 
     const int n_bh = a.batch * a.heads;
     const int n_qt = (a.sq + kBM - 1) / kBM;
-    int work = work_index(a), split = 0;
+    int work = work_index(a, block, n_blocks), split = 0;
     if (a.n_split > 1) {
         split = work / (n_bh * n_qt);
         work -= split * n_bh * n_qt;
@@ -143,8 +144,10 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
             const int dc = min(16 * t + 8 * g, a.d - 8);
             qv[t] = *reinterpret_cast<const u32x4_t*>(q_base + (int64_t)qr * a.qs[1] + dc);
             gv[t] = *reinterpret_cast<const u32x4_t*>(g_base + (int64_t)qr * a.os[1] + dc);
-            ov[t] = *reinterpret_cast<const u32x4_t*>(o_base + (int64_t)qr * a.os[1] + dc);
+            if constexpr (kDelta)
+                ov[t] = *reinterpret_cast<const u32x4_t*>(o_base + (int64_t)qr * a.os[1] + dc);
         }
+        delta = kDelta ? 0.f : a.delta[(int64_t)bh * a.sq + qr];
         const float lse_raw = a.lse[(int64_t)bh * a.sq + qr];
         request(order.first() * kBN);
         const bool row_ok = q_row < a.sq;
@@ -166,17 +169,21 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
         // kernel scales that row of dO instead).
         lse2 = row_ok ? (kBias ? lse_reference(lse_raw, kLog2e) : lse_raw * kLog2e) : INFINITY;
         if constexpr (kBias) inv_n = lse_row_factor(lse_raw);
-        // delta = sum_d dO * O: lanes i and i + 32 hold complementary head-dim slots of row i
-        float part = 0.f;
+        if constexpr (kDelta) {
+            // delta = sum_d dO * O: lanes i and i + 32 hold complementary head-dim slots of row i
+            float part = 0.f;
 #pragma unroll
-        for (int t = 0; t < DK; ++t) {
-            const frag_t of = __builtin_bit_cast(frag_t, ov[t]);
+            for (int t = 0; t < DK; ++t) {
+                const frag_t of = __builtin_bit_cast(frag_t, ov[t]);
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                part = __builtin_fmaf((float)gf[t][j], (float)of[j], part);
+                for (int j = 0; j < 8; ++j)
+                    part = __builtin_fmaf((float)gf[t][j], (float)of[j], part);
+            }
+            delta = sum_xor32(part);  // masked dO slots are zero: clamped rows / columns add nothing
+            if (row_ok && g == 0) a.delta[(int64_t)bh * a.sq + q_row] = delta * inv_n;
+        } else if constexpr (kBias) {
+            delta /= inv_n;  // (1, but for rows that saw nothing but masked keys)
         }
-        delta = sum_xor32(part);  // masked dO slots are zero, so clamped rows / columns add nothing
-        if (row_ok && g == 0) a.delta[(int64_t)bh * a.sq + q_row] = delta * inv_n;
     }
     // Where the registers allow it the per-row terms enter through the accumulators: S^T starts
     // from -lse (log2 units) and, without dropout, dP^T from -delta, in all sixteen registers of
@@ -527,10 +534,18 @@ __global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(
 }
 
 template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
+__global__ __launch_bounds__(kThreads, dq_per_cu(DPAD)) void attn_bwd_dq_kernel(const AttnArgs a) {
+    dq_block<T, DPAD, kBias, kDrop, kSteps, true>(a, (int)blockIdx.x, (int)gridDim.x);
+}
+
+template <typename T, int DPAD, int kBias>
+constexpr size_t lds_bytes() {
+    return (size_t)(kKRing + kVRing) * kBN * TileStage<T, DPAD, kBN, kThreads>::kPitch * sizeof(T) +
+           (kBias == 2 ? 2 * kBN * sizeof(float) : 0);
+}
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
 int launch(const AttnArgs& a, hipStream_t st) {
-    typedef TileStage<T, DPAD, kBN, kThreads> Stage;
-    const size_t smem = (size_t)(kKRing + kVRing) * kBN * Stage::kPitch * sizeof(T) +
-                        (kBias == 2 ? 2 * kBN * sizeof(float) : 0);
+    const size_t smem = lds_bytes<T, DPAD, kBias>();
     const int n_qt = (a.sq + kBM - 1) / kBM;
     const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;

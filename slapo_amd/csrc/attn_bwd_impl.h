@@ -58,10 +58,9 @@ constexpr int bwd_per_cu(int dpad) { return dpad <= 32 ? 3 : dpad <= 96 ? 2 : 1;
 // KB = blocks of 32 keys per wavefront.  KB = 2 halves the LDS operand traffic per matrix
 // instruction (every Q / dO fragment read feeds two MFMAs) at the price of twice the resident
 // fragments and accumulators, i.e. one wavefront per SIMD instead of two.
+// Workgroup `block` of `n_blocks`.
 template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
-__global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(
-    const AttnArgs a_in) {
-    AttnArgs a = a_in;
+__device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     static_assert(kDrop != 3 || KB == 1, "the keep-bit tile holds one word per wavefront and query");
     typedef typename Mma<T>::frag frag_t;
@@ -82,9 +81,9 @@ __global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(
     uint32_t* mask_lds = reinterpret_cast<uint32_t*>(smem_raw + 2 * SM::kQBytes + SM::kStatBytes);
 
     const int n_bh = a.batch * a.heads;
-    int work = work_index(a), split = 0;
+    int work = work_index(a, block, n_blocks), split = 0;
     if (a.n_split > 1) {
-        const int base = (int)gridDim.x / a.n_split;
+        const int base = n_blocks / a.n_split;
         split = work / base;
         work -= split * base;
     }
@@ -658,6 +657,11 @@ __global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(
                                              g_lds + wave * 32 * kPitch, dv_row0, a.dvs[1],
                                              a.sk - kw0, a.d);
     }
+}
+
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
+__global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(const AttnArgs a) {
+    dkv_block<T, DPAD, kBias, kDrop, KB, kSteps, kPerCu>(a, (int)blockIdx.x, (int)gridDim.x);
 }
 
 template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>

@@ -11,6 +11,8 @@ int attn_bwd_mfma_f16(const AttnArgs& a, hipStream_t st);
 int attn_bwd_mfma_bf16(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_mfma_f16(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_mfma_bf16(const AttnArgs& a, hipStream_t st);
+int attn_bwd_both_mfma_f16(const AttnArgs& a, hipStream_t st);
+int attn_bwd_both_mfma_bf16(const AttnArgs& a, hipStream_t st);
 int attn_fwd_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_dq_f32(const AttnArgs& a, hipStream_t st);
 int attn_bwd_f32(const AttnArgs& a, hipStream_t st);
@@ -409,6 +411,20 @@ extern "C" size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* pr
 }
 
 namespace {
+// Whether a backward runs as one launch (attn_bwd_both_impl.h): while the workgroups of both kernels
+// together are fewer than two such launches would keep resident.  Device time of the backward, two
+// launches -> delta_kernel and one: bf16 B4 S512 H8 D64 (256 workgroups) 25.4 -> 18.6 us, B6 S1187 H4
+// D64 causal (480) 48.5 -> 36.3, B2 S1024 H12 D80 causal (384) 61.9 -> 40.8, B8 S512 H12 D64 (768) 39.9
+// -> 38.1; B8 S1024 H8 D64 (1024) 71.1 -> 69.7, D80 102 -> 104.  At head_dim 128 a CU holds one workgroup
+// of dK/dV: B2 S1024 H12 causal (384) 75.8 -> 51.3, B2 S1024 H16 (512) 82.6 -> 80.9.
+bool one_launch_backward(const AttnArgs& a) {
+    if (a.dropout != 0 && a.dropout != 3) return false;
+    if (a.has_bias && (a.bias_type != SLAPO_F32 || a.bs[2] != 0)) return false;
+    const int64_t n_bh = (int64_t)a.batch * a.heads;
+    const int64_t blocks = n_bh * (((int64_t)a.sq + 127) / 128 + ((int64_t)a.sk + 127) / 128);
+    return blocks < (int64_t)(a.d <= 96 ? 4 : 2) * a.n_cus;
+}
+
 int run_backward(const slapo_attn_params* prm, const void* q, const void* k, const void* v,
                  const void* bias, int bias_type, const void* o, const void* dout,
                  const float* lse, void* dq, void* dk, void* dv, const int64_t dq_strides[3],
@@ -458,6 +474,10 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
         if (splits.dkv > 1) dkv_part = next;
     }
 
+    if (deal && !f32 && stages == SLAPO_BWD_ALL && splits.dq == 1 && splits.dkv == 1 &&
+        one_launch_backward(a))
+        return prm->dtype == SLAPO_F16 ? attn_bwd_both_mfma_f16(a, st)
+                                       : attn_bwd_both_mfma_bf16(a, st);
     // PREPARE has nothing to do (the dQ kernel computes delta for its own rows and stores it for
     // the dK / dV kernel), so DQ runs before DKDV.
     if (stages & SLAPO_BWD_DQ) {

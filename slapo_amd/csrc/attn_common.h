@@ -320,8 +320,7 @@ __device__ __forceinline__ constexpr int prepared_slot(int key) {
 // 34 to 40 tiles (43 to 53 us).  Walking the odd rows backwards (in groups of eight, so that a
 // workgroup stays on the XCD it would have had: workgroup i runs on XCD i % 8, and the heads are
 // spread over the XCDs the same way) evens the sums out.
-__device__ __forceinline__ int work_index(const AttnArgs& a) {
-    int idx = (int)blockIdx.x;
+__device__ __forceinline__ int work_index(const AttnArgs& a, int idx, int n_blocks) {
     if (a.snake_rows > 0) {
         const int row = idx / a.snake_len;
         if (row < a.snake_rows && (row & 1)) {
@@ -336,7 +335,7 @@ __device__ __forceinline__ int work_index(const AttnArgs& a) {
         const int n_bh = a.batch * a.heads;
         const int xcd = idx & 7, j = idx >> 3;
         const int per_xcd = n_bh >> 3;
-        const int n_levels = (int)gridDim.x / n_bh;
+        const int n_levels = n_blocks / n_bh;
         const int full = per_xcd / a.head_group;             // groups of full size
         const int span = a.head_group * n_levels;            // workgroups per full group
         int group = j / span, r = j - group * span, size = a.head_group;

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
 
     const int n_bh = a.batch * a.heads;
     const int n_qt = (a.sq + kBM - 1) / kBM;
-    int work = work_index(a), split = 0;
+    int work = work_index(a, (int)blockIdx.x, (int)gridDim.x), split = 0;
     if (a.n_split > 1) {
         split = work / (n_bh * n_qt);
         work -= split * n_bh * n_qt;
