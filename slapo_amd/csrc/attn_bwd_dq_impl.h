@@ -190,7 +190,7 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // the lane (= one query).  Measured against explicit subtractions: 130 against 150 us at bf16
     // B4 S2048 H16 D128 causal, 43.5 against 45 us at fp16 B8 S1024 H16 D64; at head_dim 80 / 96
     // the 32 registers cost more than the subtractions (189 against 168 us at B4 S2048 H32 D80).
-    constexpr bool kAccInit = DPAD != 96;
+    constexpr bool kAccInit = DPAD != 96 && !(kBias == 3 && DPAD == 64 && (kDrop == 0 || kDrop == 3));
     f32x16_t s_init, dp_init;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -238,6 +238,26 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // hides more latency than the stagger does (measured: 28 % faster at head_dim 80, 2-12 % at
     // 128; with one masked body for all bounds also where a window or stored dropout bits spilled
     // registers before: 90.6 -> 71.3 us at bf16 B4 S2048 H16 D128 window 256, p 0.1).
+
+    // kRowsAhead: the prepared bias of a half tile is requested when that of the same half of the tile
+    // before it has been added, so that it waits neither for itself nor, as loads return in order, for
+    // the K / V tile requested in between (bf16 with a [B,1,Sq,Sk] mask, forward and backward: B4 S500
+    // H9 D64 66.5 -> 60.0 us, D80 79.5 -> 75.4; B8 S1024 H16 D64 306 -> 297).  Above head_dim 96 its
+    // registers spill, and from 81 on or where keep bits are drawn with dropout as well; up to 32 they
+    // cost a workgroup per CU (B8 S1024 H16 causal 171 -> 172).
+    constexpr bool kRowsAhead = kBias == 3 && DPAD > 32 && DPAD <= 96 &&
+                                (kDrop == 0 || (kDrop == 3 && kSteps < 6));
+    f32x4_t bias_ahead[2][4];
+    int next_key = 0;  // first key of the next tile
+    auto request_rows = [&](int kb) __attribute__((always_inline)) {
+        if constexpr (kRowsAhead) {
+            // (rows are padded to 64 keys; past the last tile the request is wasted)
+            const float* p = bias_row + min(next_key, (a.sk - 1) & ~63) + 16 * g + 32 * kb;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+                bias_ahead[kb][r4] = *reinterpret_cast<const f32x4_t*>(p + 4 * r4);
+        }
+    };
 
     // S^T half = K_half Q^T (log2 units)
     auto half_s = [&](const T* kt, int kb, f32x16_t& s) __attribute__((always_inline)) {
@@ -310,8 +330,10 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
                 bv[0] = t4.x, bv[1] = t4.y, bv[2] = t4.z, bv[3] = t4.w;
             }
             if constexpr (kBias == 3) {
-                const f32x4_t t4 =
-                    *reinterpret_cast<const f32x4_t*>(bias_row + j0 + 16 * g + 4 * r4);
+                const f32x4_t t4 = kRowsAhead
+                                       ? bias_ahead[kb][r4]
+                                       : *reinterpret_cast<const f32x4_t*>(bias_row + j0 + 16 * g +
+                                                                           4 * r4);
                 bv[0] = t4.x, bv[1] = t4.y, bv[2] = t4.z, bv[3] = t4.w;
             }
 #pragma unroll
@@ -324,6 +346,7 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
                 s[4 * r4 + e] = p;
             }
         }
+        request_rows(kb);
     };
     // dS^T half = P^T (dP^T - delta), packed to T
     // kDrop == 3: the keep bits of this lane's query for the two halves of a tile, as the forward stored
@@ -483,12 +506,16 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // full; the others test activity per wavefront and mask.
     int t = order.first();
     request_bits(t);
+    next_key = t * kBN;
+    request_rows(0);
+    request_rows(1);
     auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
         constexpr bool kFast = decltype(fast_tag)::value;
         const int next = kFast ? order.after_fast(t) : order.after(t);
         const bool have_next = r + 1 < n_tiles;
         tile_bits[0] = next_bits[0], tile_bits[1] = next_bits[1];
         request_bits(next);
+        next_key = next * kBN;
         if (have_next) {
             request(next * kBN);
         }
@@ -502,6 +529,9 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
                 tile_body(kt, vt, t, std::integral_constant<int, 0>{});
         } else if (tile_active(t)) {
             tile_body(kt, vt, t, std::integral_constant<int, 1>{});
+        } else {
+            request_rows(0);
+            request_rows(1);
         }
         if (have_next) {
             ks.fix(next * kBN, a.sk, a.d);

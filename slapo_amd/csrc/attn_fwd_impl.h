@@ -204,6 +204,28 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
         if (a.window > 0 && wq0 - (j0 + kBN - 1) >= a.window) return false;
         return true;
     };
+    // kRowsAhead: the prepared bias of a tile is requested when that of the tile before it has been
+    // added, so that it waits neither for itself nor, as loads return in order, for the K / V tile
+    // requested in between (bf16 B2 S500 H9 with a [B,1,Sq,Sk] mask, its preparation included: D64
+    // 23.9 -> 18.3 us, D80 26.1 -> 22.3; B8 S1024 H16 D80 121 -> 112).  Above head_dim 96 its 32
+    // registers spill, and elsewhere than at 64 where the kernel draws keep bits as well (p 0.1 D32 37.2
+    // -> 41.6 us, D80 42.5 -> 47.6); up to 64 they cost a workgroup per CU (launch).
+    constexpr bool kRowsAhead = kBias == 3 && DPAD <= 96 &&
+                                (DPAD > 64 || kPerCu < fwd_per_cu(DPAD)) &&
+                                (DPAD == 64 || (kDrop != 1 && kDrop != 2));
+    f32x4_t bias_ahead[2][4];
+    auto request_rows = [&](int j0) __attribute__((always_inline)) {
+        if constexpr (kRowsAhead) {
+            // (rows are padded to 64 keys; past the last tile the request is wasted)
+            const float* p = bias_row + min(j0, (a.sk - 1) & ~63) + 16 * g;
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4)
+                    bias_ahead[kb][r4] = *reinterpret_cast<const f32x4_t*>(p + 32 * kb + 4 * r4);
+        }
+    };
+
     // S^T half = K_half Q^T, in log2 units
     auto half_scores = [&](const T* kt, int kb, f32x16_t& s) __attribute__((always_inline)) {
 #pragma unroll
@@ -252,8 +274,10 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             if constexpr (kBias == 3) {
-                const f32x4_t t4 =
-                    *reinterpret_cast<const f32x4_t*>(bias_row + j0 + 16 * g + 4 * r4);
+                const f32x4_t t4 = kRowsAhead
+                                       ? bias_ahead[kb][r4]
+                                       : *reinterpret_cast<const f32x4_t*>(bias_row + j0 + 16 * g +
+                                                                           4 * r4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) s[4 * r4 + e] += t4[e];
             }
@@ -431,7 +455,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
                     a.keep_mask[(base + min(2 * t + kb, a.mask_words - 1)) * a.mask_pitch + row];
         }
     };
-    auto tile_body = [&](const T* kt, const T* vt, int t, auto mask_tag)
+    auto tile_body = [&](const T* kt, const T* vt, int t, int next, auto mask_tag)
                          __attribute__((always_inline)) {
         f32x16_t s0, s1;
         uint32_t pw0[8], pw1[8];
@@ -441,6 +465,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
         half_scores(kt, 1, s1);
         const float mx =
             max_xor32(fmaxf(finish_half(s0, t, 0, mask_tag), finish_half(s1, t, 1, mask_tag)));
+        request_rows(next);
         update_reference(mx, s0, s1);
         half_prob(s0, t, 0, pw0, bits0);
         half_accumulate(vt, 0, pw0);
@@ -475,6 +500,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     // other slot.  kFast iterations hold tiles that every wavefront of the workgroup sees in full.
     int t = order.first();
     request_bits(t);
+    request_rows(t * kBN);
     auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
         constexpr bool kFast = decltype(fast_tag)::value;
         const int t_next = kFast ? order.after_fast(t) : order.after(t), next = t_next * kBN;
@@ -493,9 +519,12 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
         const T* vt = v_lds + (r & 1) * kTileElems;
         bias_tile = bias_lds + (r & 1) * kBN;
         if constexpr (kFast) {
-            tile_body(kt, vt, t, std::integral_constant<int, 0>{});
+            tile_body(kt, vt, t, next, std::integral_constant<int, 0>{});
         } else {
-            if (tile_active(t)) tile_body(kt, vt, t, std::integral_constant<int, 1>{});
+            if (tile_active(t))
+                tile_body(kt, vt, t, next, std::integral_constant<int, 1>{});
+            else
+                request_rows(next);
         }
         if (have_next) {
             ks.fix(next, a.sk, a.d);
@@ -550,6 +579,14 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const int n_qt = (a.sq + kBM - 1) / kBM;
     const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
+    // kRowsAhead against one workgroup more per CU (bf16 B8 S1024 H16, 1024 workgroups): without the
+    // causal mask D64 100.8 -> 96.7 us, D32 98.5 -> 95.9; with it, whose workgroups differ in length,
+    // 65.8 -> 66.3 and 60.0 -> 64.5, so there only in launches that need not the one more
+    if constexpr (DPAD <= 64 && kBias == 3 && kPerCu == fwd_per_cu(DPAD) &&
+                  (DPAD == 64 || (kDrop != 1 && kDrop != 2))) {
+        if (!a.causal || blocks <= (int64_t)(kPerCu - 1) * a.n_cus)
+            return launch<T, DPAD, kBias, kDrop, kSteps, kPerCu - 1>(a, st);
+    }
     if constexpr (DPAD <= 64 && kBias == 0 && kDrop == 0 && kPerCu < kFwdFour) {
         if (blocks > (int64_t)kPerCu * a.n_cus)
             return launch<T, DPAD, kBias, kDrop, kSteps, kFwdFour>(a, st);
