@@ -17,7 +17,8 @@ other_attention  forward and backward time of the OPT-2.7B-shaped (padding mask)
           GPT-Neo-1.3B-shaped (global / window 256, dropout 0.1) attention calls, bf16
 bert_large_fp32  BASELINE configuration 1, which is DEFINED as the native CPU path: the oracle's
           fp32 forward of B 4, S 512, 16 x 64 on the host cores, and beside it the fp32 kernel
-          of this library on the same tensors against the fp32 vector peak (reported, not a target)
+          of this library on the same tensors (on bf16 matrix instructions, six products for one)
+          against the fp32 vector peak (reported, not a target)
 cpu_baseline  the oracle's native-PyTorch restatement (fp32 CPU, autograd backward) timed on the
           host cores on a bounded sample of the same workload; every epilogue / other_attention
           entry carries a cpu_baseline of its own (a bounded chunk of its tensors)
@@ -670,7 +671,7 @@ def main():
                    "heads": cfg["heads"], "head_dim": cfg["head_dim"], "causal": cfg["causal"],
                    "dropout_p": cfg["p"], "flops_per_step": 14 * d * n_pairs},
         "frac_of_mfma_peak": value / MFMA_PEAK_TFLOPS,
-        "roofline": {"bound": "mfma", "kernel": "attn_bwd_kernel<f16,64,0,0,1,4> (dK/dV)",
+        "roofline": {"bound": "mfma", "kernel": "attn_bwd_kernel<f16,64,0,0,1,4,2> (dK/dV)",
                      "achieved": achieved,
                      "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / MFMA_PEAK_TFLOPS, "traffic": DKDV_TRAFFIC_BYTES,
@@ -679,9 +680,9 @@ def main():
                           "raw_event_intervals_ms": seg_raw,
                           "sum_of_kernels_ms": sum(seg_ms)},
     }
-    result["kernels"] = [kern("attn_fwd_kernel<f16,64,0,0,0,4>", 4 * d * n_pairs, seg_ms[0]),
-                         kern("attn_bwd_kernel<f16,64,0,0,1,4> (dK/dV)", bwd_flops, seg_ms[2]),
-                         kern("attn_bwd_dq_kernel<f16,64,0,0,true,4>", 6 * d * n_pairs, seg_ms[1])]
+    result["kernels"] = [kern("attn_fwd_kernel<f16,64,0,0,4,4>", 4 * d * n_pairs, seg_ms[0]),
+                         kern("attn_bwd_kernel<f16,64,0,0,1,4,2> (dK/dV)", bwd_flops, seg_ms[2]),
+                         kern("attn_bwd_dq_kernel<f16,64,0,0,4>", 6 * d * n_pairs, seg_ms[1])]
     with_cpu = not args.no_cpu_baseline
     if not args.no_epilogues:
         result["epilogue"] = bench_epilogues(device)
