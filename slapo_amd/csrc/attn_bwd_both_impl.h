@@ -82,9 +82,14 @@ template <typename T, int DPAD, int kSteps = DPAD / 16>
 int dispatch_flags(const AttnArgs& a, hipStream_t st) {
     if (!a.has_bias)
         return a.dropout ? launch<T, DPAD, 0, 3, kSteps>(a, st) : launch<T, DPAD, 0, 0, kSteps>(a, st);
+    if (a.bias_type == SLAPO_BIAS_PREPARED) {
+        if (!a.dropout) return launch<T, DPAD, 3, 0, kSteps>(a, st);
+        if constexpr (kSteps != 6) return launch<T, DPAD, 3, 3, kSteps>(a, st);
+        return SLAPO_ERR_SHAPE;  // (one_launch_backward)
+    }
     return a.dropout ? launch<T, DPAD, 2, 3, kSteps>(a, st) : launch<T, DPAD, 2, 0, kSteps>(a, st);
 }
-// Calls without bias or with one value per key, without dropout or with stored bits.
+// Calls without bias, with one value per key or with a prepared bias, without dropout or with stored bits.
 template <typename T>
 int dispatch(const AttnArgs& a, hipStream_t st) {
     if (a.d <= 32) return dispatch_flags<T, 32>(a, st);

@@ -535,7 +535,7 @@ def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
     return ref, qf.grad, kf.grad, vf.grad
 
 
-@pytest.mark.parametrize("mask", ["none", "key", "hidden"])
+@pytest.mark.parametrize("mask", ["none", "key", "hidden", "square"])
 @pytest.mark.parametrize("shape,sk,causal,window", [
     ((2, 130, 3, 64), 130, True, 0),
     ((1, 257, 5, 32), 257, False, 0),
@@ -546,7 +546,8 @@ def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
 ])
 def test_backward_in_one_launch_equals_the_two_kernels(shape, sk, causal, window, mask):
     """The op's backward of a small call runs as one launch behind a delta kernel; bit for bit what the
-    entry point with the two kernels gives, also for rows that see only masked keys."""
+    two kernels give, also for rows that see only masked keys: those of the entry point that always runs
+    them, or, with a mask that the op prepares, those of a call of so many copies that it runs them."""
     from slapo_amd.op import _kernels as K
 
     b, s, h, d = shape
@@ -554,13 +555,23 @@ def test_backward_in_one_launch_equals_the_two_kernels(shape, sk, causal, window
     q, k, v, do = (t.cuda() for t in (q, k, v, do))
     m = None
     if mask != "none":
-        m = torch.randn(b, 1, 1, sk, generator=g)
+        m = torch.randn(b, 1, s if mask == "square" else 1, sk, generator=g)
+        if mask == "square":
+            m[:, :, s // 2] = torch.finfo(torch.float32).min
         if mask == "hidden":
             m[0] = torch.finfo(torch.float32).min
         m = m.cuda()
     qh, kh, vh = (t.clone().requires_grad_(True) for t in (q, k, v))
     out = op.hip_attention(qh, kh, vh, m, causal=causal, window=window)
     out.backward(do)
+    if mask == "square":
+        n = -(-1024 // (b * h * (-(-s // 128) + -(-sk // 128))))
+        qn, kn, vn = (t.repeat(n, 1, 1, 1).requires_grad_(True) for t in (q, k, v))
+        op.hip_attention(qn, kn, vn, m.repeat(n, 1, 1, 1), causal=causal,
+                         window=window).backward(do.repeat(n, 1, 1, 1))
+        for a, r in ((qh, qn), (kh, kn), (vh, vn)):
+            assert torch.equal(a.grad, r.grad[:b])
+        return
     bias = None if m is None else m.expand(b, h, s, sk)
     o, lse, _ = K.attn_fwd(q, k, v, bias, causal, window, d ** -0.5, 0.0, 1, 0, None)
     assert torch.equal(o, out)
