@@ -321,6 +321,23 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     };
 
     // ---- stages of one half tile (32 queries at ih0 = i0 + 32 hf) ----
+    // The prepared bias of a half tile is requested before the products whose result it is added to
+    // (bf16 with a [B,1,Sq,Sk] mask, forward and backward: B8 S1024 H16 D64 297 -> 289 us, D80 causal 277
+    // -> 248, D96 causal, p 0.1 429 -> 308, where its loads in the masked body spilled).  Up to head_dim
+    // 32 each value comes where it is added (B8 S1024 H16 D32 causal 171.1 against 173.5).  At 81-96
+    // without dropout the masked body gains (B2 S1024 H12 D96 causal 110.7 -> 99.5) and full tiles alone
+    // do not (104.0 -> 104.7; with the values where they are added in those only, 105.9).
+    constexpr bool kRowsEarly = kBias == 3 && DPAD > 32;
+    float bias_rows[16];
+    auto bias_at = [&](int ih0, int r) __attribute__((always_inline)) {
+        static_assert(kBias != 3 || KB == 1, "one key block per wavefront");
+        return (bias_tile + (int64_t)(ih0 + acc_row(r, 0)) * a.bs[2])[bias_lane];
+    };
+    auto request_rows = [&](int ih0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bias_rows[r] = bias_at(ih0, r);
+        pin_requests();
+    };
     // S = Q_h K_w^T, dP = dO_h V_w^T: every Q / dO fragment read feeds KB matrix instructions
     auto half_sp = [&](const T* qt, const T* gt, const float* lse_h, const float* delta_h, int hf,
                        f32x16_t (&s)[KB], f32x16_t (&dp)[KB]) __attribute__((always_inline)) {
@@ -348,6 +365,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     };
     // scores -> probabilities in place.  mask_tag: 0 = all visible, 1 = the causal and window bounds, as
     // one bit per query: two instructions per score whatever they are
+    // (kRowsEarly: the prepared bias is in bias_rows)
     auto half_exp = [&](f32x16_t (&s)[KB], const float* lse_h, int ih0, auto mask_tag)
                         __attribute__((always_inline)) {
         constexpr int kMask = decltype(mask_tag)::value;
@@ -373,9 +391,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
                             a.bias)[b * a.bs[0] + h * a.bs[1] + (int64_t)i * a.bs[2] +
                                     (int64_t)key[kb] * a.bs[3]]);
                 } else if constexpr (kBias == 3) {
-                    static_assert(KB == 1, "one key block per wavefront");
-                    const float* row = bias_tile + (int64_t)(ih0 + acc_row(r, 0)) * a.bs[2];
-                    x += row[bias_lane];
+                    x += kRowsEarly ? bias_rows[r] : bias_at(ih0, r);
                 }
                 float p = fast_exp2(x);
                 if constexpr (kMask != 0) p = keep_or_zero(p, visible[kb], acc_row(r, 0));
@@ -511,6 +527,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
             const uint32_t* mask_h = mask_lds + buf * kBwdThreads + wave * kBwdBM + 32 * hf;
             f32x16_t s[KB], dp[KB];
             uint32_t pw[KB][8], dw[KB][8];
+            if constexpr (kRowsEarly) request_rows(ih0);
             half_sp(qt, gt, lse_h, delta_h, hf, s, dp);
             half_exp(s, lse_h, ih0, std::integral_constant<int, 0>{});
             half_ds(s, dp, delta_h, mask_h, ih0, pw, dw);
@@ -539,8 +556,10 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
         const int i0 = t * kBwdBM;
         f32x16_t s0[KB], s1[KB], p0[KB], p1[KB];
         uint32_t pw0[KB][8], dw0[KB][8], pw1[KB][8], dw1[KB][8];
+        if constexpr (kRowsEarly) request_rows(i0);
         half_sp(qt, gt, lse_t, delta_t, 0, s0, p0);
         half_exp(s0, lse_t, i0, mask_tag);
+        if constexpr (kRowsEarly) request_rows(i0 + 32);
         half_sp(qt, gt, lse_t + 32, delta_t + 32, 1, s1, p1);
         half_ds(s0, p0, delta_t, mask_t, i0, pw0, dw0);
         half_exp(s1, lse_t + 32, i0 + 32, mask_tag);
@@ -589,6 +608,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
             const uint32_t* mask_h = mask_lds + buf * kBwdThreads + wave * kBwdBM + 32 * hf;
             f32x16_t s[KB], dp[KB];
             uint32_t pw[KB][8], dw[KB][8];
+            if constexpr (kRowsEarly) request_rows(ih0);
             half_sp(qt, gt, lse_h, delta_h, hf, s, dp);
             // (a second copy without masks pays only up to head_dim 64, where registers are left: fp16
             // B8 S1024 H16 D64 causal 120.4 -> 119.9 us forward and backward; bf16 B4 S2048 H16 D128
