@@ -5,6 +5,11 @@
 // of three bf16 numbers, x = h + m + l (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 8 + 8 + 8
 // mantissa bits, fp32's exponent range), and x y = hh + (hm + mh) + (mm + hl + lh) + O(2^-25 |x y|),
 // six v_mfma_f32_16x16x32_bf16 with exact products and fp32 sums.
+// Infinities have no such parts, and numbers that bf16 rounds to infinity none that are finite.  A
+// workgroup that meets a magnitude above kTop, or whose results are not all finite, writes nothing and
+// runs its rows again on v_mfma_f32_16x16x4_f32 (Full8), whose products are fp32's own: infinity times
+// infinity is one.  It costs such a call two to three times the time and the others nothing (B4 S512 H16
+// D64 33 us before and after; forward and backward 125).
 //
 // v_mfma_f32_16x16x32_bf16 (one wavefront, lane l, i = l % 16, g = l / 16):
 //   A operand: lane holds A[row i][k-slots 8 g .. 8 g + 7];   B operand: the same slots of column i;
@@ -33,6 +38,8 @@
 //
 //
 // Reference semantics: slapo/op/attention.py:163-181 (attention_bmk) and its autograd.
+#include <type_traits>
+
 #include "attn_common.h"
 
 using namespace slapo;
@@ -55,14 +62,26 @@ constexpr int64_t kWideBwd = 512;   // in units of 64 rows: B4 S512 H16 D64 (512
 constexpr int64_t kHalvesBelow = 128;
 // LDS and registers leave a SIMD four of a forward's wavefronts up to head_dim 64, else two.
 constexpr int per_simd(int db, int waves) { return db <= 4 && waves >= 8 ? 4 : 2; }
-constexpr float kReserve = 8.0f;  // of the softmax reference above the maximum, log2 units
+constexpr float kPartsReserve = 8.0f;  // of the softmax reference above the maximum, log2 units
 
 typedef Mma<bf16_t>::frag frag_t;
 __device__ __forceinline__ f32x4_t splat(float v) { return f32x4_t{v, v, v, v}; }
-// Eight fp32 numbers as their bf16 parts.
+// The two forms of eight fp32 numbers: their bf16 parts, and themselves.
 struct Split8 {
     u32x4_t h, m, l;
 };
+struct Full8 {
+    f32x4_t a, b;
+};
+// (see read_again)
+template <bool kParts>
+__device__ __forceinline__ int thread_of() {
+    int t = threadIdx.x;
+    if constexpr (!kParts) asm("" : "+v"(t));
+    return t;
+}
+template <bool kParts>
+using operand_t = std::conditional_t<kParts, Split8, Full8>;
 __device__ __forceinline__ frag_t frag(u32x4_t v) { return __builtin_bit_cast(frag_t, v); }
 // c (and, in `small`, the five smaller products) += A B of fp32 operands
 __device__ __forceinline__ void mma(const Split8& a, const Split8& b, f32x4_t& c, f32x4_t& small) {
@@ -73,60 +92,66 @@ __device__ __forceinline__ void mma(const Split8& a, const Split8& b, f32x4_t& c
     small = Mma<bf16_t>::mma16(frag(a.h), frag(b.m), small);
     c = Mma<bf16_t>::mma16(frag(a.h), frag(b.h), c);
 }
+// c += A B over four k-slots, slot g of this lane's column
+__device__ __forceinline__ void mma4(float a, float b, f32x4_t& c) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
 __device__ __forceinline__ float low_half(uint32_t v) { return __builtin_bit_cast(float, v << 16); }
 __device__ __forceinline__ float high_half(uint32_t v) {
     return __builtin_bit_cast(float, v & 0xFFFF0000u);
 }
-// The parts of two finite numbers below 3.38e38 (NaN: stays one)
 __device__ __forceinline__ void split2(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
     h = pack2<bf16_t>(x, y);
     x -= low_half(h), y -= high_half(h);
     m = pack2<bf16_t>(x, y);
     l = pack2<bf16_t>(x - low_half(m), y - high_half(m));
 }
-// ... of any two.  What bf16 would round to infinity is cut instead; an infinity stands in the last
-// part alone, which meets nothing but the other operand's first one (its rest may have any sign).
-__device__ __forceinline__ void split2_any(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
-    const float v[2] = {x, y};
-    float hi[2], mid[2], lo[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const bool inf = __builtin_isinf(v[e]);
-        const float finite = inf ? 0.f : v[e];
-        hi[e] = low_half(pack2<bf16_t>(finite, 0.f));
-        if (__builtin_isinf(hi[e])) hi[e] = high_half(__builtin_bit_cast(uint32_t, finite));
-        mid[e] = low_half(pack2<bf16_t>(finite - hi[e], 0.f));
-        lo[e] = inf ? v[e] : finite - hi[e] - mid[e];
-    }
-    h = pack2<bf16_t>(hi[0], hi[1]);
-    m = pack2<bf16_t>(mid[0], mid[1]);
-    l = pack2<bf16_t>(lo[0], lo[1]);
-}
-__device__ __forceinline__ void split4(const f32x4_t& v, uint32_t* h, uint32_t* m, uint32_t* l) {
-    const float top = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(top > 3.38e38f) != 0, 0)) {
-        split2_any(v[0], v[1], h[0], m[0], l[0]);
-        split2_any(v[2], v[3], h[1], m[1], l[1]);
-    } else {
-        split2(v[0], v[1], h[0], m[0], l[0]);
-        split2(v[2], v[3], h[1], m[1], l[1]);
-    }
-}
-// kSmall: probabilities, whose size needs no look
-template <bool kSmall = false>
-__device__ __forceinline__ Split8 split8(const f32x4_t& a, const f32x4_t& b) {
-    uint32_t h[4], m[4], l[4];
-    if constexpr (kSmall) {
+template <bool kParts>
+__device__ __forceinline__ operand_t<kParts> operand(const f32x4_t& a, const f32x4_t& b) {
+    if constexpr (kParts) {
+        uint32_t h[4], m[4], l[4];
         split2(a[0], a[1], h[0], m[0], l[0]);
         split2(a[2], a[3], h[1], m[1], l[1]);
         split2(b[0], b[1], h[2], m[2], l[2]);
         split2(b[2], b[3], h[3], m[3], l[3]);
+        return {u32x4_t{h[0], h[1], h[2], h[3]}, u32x4_t{m[0], m[1], m[2], m[3]},
+                u32x4_t{l[0], l[1], l[2], l[3]}};
     } else {
-        split4(a, h, m, l);
-        split4(b, h + 2, m + 2, l + 2);
+        return {a, b};
     }
-    return {u32x4_t{h[0], h[1], h[2], h[3]}, u32x4_t{m[0], m[1], m[2], m[3]},
-            u32x4_t{l[0], l[1], l[2], l[3]}};
+}
+// What a pass in bf16 parts has to see below kTop: then every part, every score and every dO v is finite,
+// and a result that went wrong on the way (a sum past fp32's range) is not.
+constexpr float kTop = 0x1p60f;
+// top = the largest magnitude so far (not of NaN, which reaches the results)
+__device__ __forceinline__ void track(float& top, const f32x4_t& v) {
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(v[0]), "v"(v[1]));
+    asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(top) : "v"(v[2]), "v"(v[3]));
+}
+// 0, or NaN once a result is not finite
+template <int DB>
+__device__ __forceinline__ float not_finite(const f32x4_t (&acc)[DB], float so_far = 0.f) {
+#pragma unroll
+    for (int x = 0; x < DB; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) so_far = __builtin_fmaf(acc[x][e], 0.f, so_far);
+    return so_far;
+}
+// 2^x: of parts, zero below 2^-126
+template <bool kParts>
+__device__ __forceinline__ float exp2_of(float x) {
+    return kParts ? fast_exp2(x) : __builtin_exp2f(x);
+}
+// Whether `ok` holds in every thread of the workgroup's kWaves wavefronts; `votes` is theirs alone.
+template <int kWaves>
+__device__ __forceinline__ bool everywhere(bool ok, int* votes) {
+    const bool wave_ok = __builtin_amdgcn_ballot_w64(!ok) == 0;
+    if ((threadIdx.x & 63) == 0) votes[threadIdx.x >> 6] = wave_ok;
+    __syncthreads();
+    int all = 1;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) all &= votes[w];
+    return __builtin_amdgcn_readfirstlane(all) != 0;
 }
 // Tile row (of a group of 16) of accumulator register r of lane-group g: 4 r + lane_row(g).
 __device__ __forceinline__ int lane_row(int g) { return (g & 1) * 2 + (g >> 1); }
@@ -157,19 +182,22 @@ template <int DB>
 constexpr int kStepsOf = (DB + 1) / 2;
 template <int DB>
 constexpr int kPitchOf = 32 * kStepsOf<DB> + 8;
+template <int DB>
+constexpr int kFullPitchOf = 32 * kStepsOf<DB> + 4;  // of a tile of fp32 numbers, in floats
 
 // Builds of each kernel: kMode & 1 = with a bias, kMode & 2 = with dropout, for tensors whose rows are
 // 16-byte aligned with d % 4 == 0; kGeneral serves every other layout element by element and decides
 // about bias and dropout when it runs.
 constexpr int kGeneral = 4;
 
-// A tile of kTileRows rows on its way from global memory to LDS, where it stands as three bf16 planes.
-// Rows past the end are clamped, columns past d read as zero.
-template <int DB, bool kVec, int kTileRows, int kBlock>
+// A tile of kTileRows rows on its way from global memory to LDS, where it stands as three bf16 planes or,
+// in less of the same place, as it is.  Rows past the end are clamped, columns past d read as zero.
+template <int DB, bool kVec, int kTileRows, int kBlock, bool kParts>
 struct Tile {
     static constexpr int kPitch = kPitchOf<DB>;
     static constexpr int kPlane = kTileRows * kPitch;
     static constexpr int kElems = 3 * kPlane;
+    static_assert(sizeof(float) * kFullPitchOf<DB> <= 3 * sizeof(bf16_t) * kPitch);
     static constexpr int kPerRow = 8 * kStepsOf<DB>;
     static constexpr int kChunks = kTileRows * kPerRow;
     static constexpr int kPer = (kChunks + kBlock - 1) / kBlock;
@@ -179,7 +207,7 @@ struct Tile {
                                          int d) {
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int c = threadIdx.x + u * kBlock;
+            const int c = thread_of<kParts>() + u * kBlock;
             if (kChunks % kBlock != 0 && c >= kChunks) continue;
             const float* row = base + (int64_t)min(row0 + c / kPerRow, n_rows - 1) * stride;
             const int col = 4 * (c % kPerRow);
@@ -191,11 +219,11 @@ struct Tile {
             }
         }
     }
-    __device__ __forceinline__ void store(bf16_t* lds, int row0, int n_rows, int d) {
+    __device__ __forceinline__ void store(bf16_t* lds, int row0, int n_rows, int d, float& top) {
         if (row0 + kTileRows > n_rows || d < 32 * kStepsOf<DB>) {  // uniform
 #pragma unroll
             for (int u = 0; u < kPer; ++u) {
-                const int c = threadIdx.x + u * kBlock;
+                const int c = thread_of<kParts>() + u * kBlock;
                 const int row = c / kPerRow, col = 4 * (c % kPerRow);
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -204,23 +232,31 @@ struct Tile {
         }
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
-            const int c = threadIdx.x + u * kBlock;
+            const int c = thread_of<kParts>() + u * kBlock;
             if (kChunks % kBlock != 0 && c >= kChunks) continue;
-            uint32_t h[2], m[2], l[2];
-            split4(r[u], h, m, l);
-            bf16_t* p = lds + c / kPerRow * kPitch + 4 * (c % kPerRow);
-            *reinterpret_cast<u32x2_t*>(p) = u32x2_t{h[0], h[1]};
-            *reinterpret_cast<u32x2_t*>(p + kPlane) = u32x2_t{m[0], m[1]};
-            *reinterpret_cast<u32x2_t*>(p + 2 * kPlane) = u32x2_t{l[0], l[1]};
+            const int row = c / kPerRow, col = 4 * (c % kPerRow);
+            if constexpr (kParts) {
+                uint32_t h[2], m[2], l[2];
+                track(top, r[u]);
+                split2(r[u][0], r[u][1], h[0], m[0], l[0]);
+                split2(r[u][2], r[u][3], h[1], m[1], l[1]);
+                bf16_t* p = lds + row * kPitch + col;
+                *reinterpret_cast<u32x2_t*>(p) = u32x2_t{h[0], h[1]};
+                *reinterpret_cast<u32x2_t*>(p + kPlane) = u32x2_t{m[0], m[1]};
+                *reinterpret_cast<u32x2_t*>(p + 2 * kPlane) = u32x2_t{l[0], l[1]};
+            } else {
+                float* p = reinterpret_cast<float*>(lds) + row * kFullPitchOf<DB> + col;
+                *reinterpret_cast<f32x4_t*>(p) = r[u];
+            }
         }
     }
 };
 
 // Row `row` of a tensor as this lane holds it: elements 32 t + 8 g .. + 7 in f[2 t], f[2 t + 1].
-template <bool kVec, int KS>
+template <bool kParts, bool kVec, int KS>
 __device__ __forceinline__ void load_row(f32x4_t (&f)[2 * KS], const float* base, int64_t stride,
                                          int row, int n_rows, int d, float scale) {
-    const int g = (threadIdx.x & 63) >> 4;
+    const int g = (thread_of<kParts>() & 63) >> 4;
     const float* p = base + (int64_t)min(row, n_rows - 1) * stride;
 #pragma unroll
     for (int t = 0; t < 2 * KS; ++t) {
@@ -236,10 +272,14 @@ __device__ __forceinline__ void load_row(f32x4_t (&f)[2 * KS], const float* base
             f[t][e] = (row < n_rows && col + e < d) ? f[t][e] * scale : 0.f;
     }
 }
-template <int KS>
-__device__ __forceinline__ void split_row(Split8 (&f)[KS], const f32x4_t (&v)[2 * KS]) {
+template <bool kParts, int KS>
+__device__ __forceinline__ void hold_row(operand_t<kParts> (&f)[KS], const f32x4_t (&v)[2 * KS],
+                                         float& top) {
 #pragma unroll
-    for (int t = 0; t < KS; ++t) f[t] = split8(v[2 * t], v[2 * t + 1]);
+    for (int t = 0; t < KS; ++t) {
+        if constexpr (kParts) track(top, v[2 * t]), track(top, v[2 * t + 1]);
+        f[t] = operand<kParts>(v[2 * t], v[2 * t + 1]);
+    }
 }
 
 // small + A B over the head dimension: A = 16 tile rows from row `r0` on, B = this lane's fragments.
@@ -247,7 +287,7 @@ template <int DB, int kPlane>
 __device__ __forceinline__ f32x4_t dot_rows(const bf16_t* tile, int r0,
                                             const Split8 (&f)[kStepsOf<DB>],
                                             f32x4_t small = f32x4_t{0.f, 0.f, 0.f, 0.f}) {
-    const int lane = threadIdx.x & 63, i = lane & 15;
+    const int lane = thread_of<true>() & 63, i = lane & 15;
     const bf16_t* p = tile + (r0 + 4 * (i & 3) + lane_row(i >> 2)) * kPitchOf<DB> + 8 * (lane >> 4);
     f32x4_t c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -260,12 +300,31 @@ __device__ __forceinline__ f32x4_t dot_rows(const bf16_t* tile, int r0,
     }
     return c + small;
 }
+template <int DB, int kPlane>
+__device__ __forceinline__ f32x4_t dot_rows(const bf16_t* tile, int r0,
+                                            const Full8 (&f)[kStepsOf<DB>],
+                                            f32x4_t small = f32x4_t{0.f, 0.f, 0.f, 0.f}) {
+    const int lane = thread_of<false>() & 63, i = lane & 15;
+    const float* p = reinterpret_cast<const float*>(tile) +
+                     (r0 + 4 * (i & 3) + lane_row(i >> 2)) * kFullPitchOf<DB> + 8 * (lane >> 4);
+    f32x4_t c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < kStepsOf<DB>; ++t) {
+        const f32x4_t a = *reinterpret_cast<const f32x4_t*>(p + 32 * t);
+        const f32x4_t b = *reinterpret_cast<const f32x4_t*>(p + 32 * t + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mma4(a[e], f[t].a[e], c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mma4(b[e], f[t].b[e], c);
+    }
+    return c + small;
+}
 // acc[x] += A B over the 32 tile rows: A = columns 16 x .. 16 x + 15 of those rows (transposed), B =
 // w, slots r and 4 + r of it being rows 4 r + lane_row(g) and 16 more of this lane's column.
 template <int DB, int kPlane>
 __device__ __forceinline__ void add_rows(const bf16_t* tile, const Split8& w, f32x4_t (&acc)[DB],
                                          f32x4_t (&small)[DB]) {
-    const int lane = threadIdx.x & 63;
+    const int lane = thread_of<true>() & 63;
     const bf16_t* p = tile +
                       (4 * ((lane & 15) >> 2) + lane_row(lane >> 4)) * kPitchOf<DB> + 4 * (lane & 3);
     auto columns = [&](const bf16_t* q) __attribute__((always_inline)) {
@@ -280,10 +339,25 @@ __device__ __forceinline__ void add_rows(const bf16_t* tile, const Split8& w, f3
     }
 }
 
+template <int DB, int kPlane>
+__device__ __forceinline__ void add_rows(const bf16_t* tile, const Full8& w, f32x4_t (&acc)[DB],
+                                         f32x4_t (&)[DB]) {
+    const int lane = thread_of<false>() & 63;
+    const float* p = reinterpret_cast<const float*>(tile) +
+                     lane_row(lane >> 4) * kFullPitchOf<DB> + (lane & 15);
+#pragma unroll
+    for (int r = 0; r < 4; ++r, p += 4 * kFullPitchOf<DB>)
+#pragma unroll
+        for (int x = 0; x < DB; ++x) {
+            mma4(p[16 * x], w.a[r], acc[x]);
+            mma4(p[16 * kFullPitchOf<DB> + 16 * x], w.b[r], acc[x]);
+        }
+}
+
 // Writes this lane's column of acc (element 16 x + 4 g + r in acc[x][r]) times mul as row `row`.
-template <bool kVec, int DB>
+template <bool kParts, bool kVec, int DB>
 __device__ __forceinline__ void store_row(const f32x4_t (&acc)[DB], float mul, float* row, int d) {
-    const int g = (threadIdx.x & 63) >> 4;
+    const int g = (thread_of<kParts>() & 63) >> 4;
 #pragma unroll
     for (int x = 0; x < DB; ++x) {
         const int col = 16 * x + 4 * g;
@@ -311,8 +385,9 @@ __device__ __forceinline__ uint32_t keep_keys(const AttnArgs& a, int bh, int i, 
 }
 // Keep bits of query i (the lane's column) and the 32 keys from j0 on: a Philox block covers four
 // consecutive keys, so each of the four lanes of a query draws eight keys and they exchange them.
+template <bool kParts>
 __device__ __forceinline__ uint32_t keep_keys32(const AttnArgs& a, int bh, int i, int j0) {
-    const int at = 8 * ((threadIdx.x & 63) >> 4);
+    const int at = 8 * ((thread_of<kParts>() & 63) >> 4);
     uint32_t bits = keep_keys<8>(a, bh, i, j0 + at) << at;
     bits |= (uint32_t)__shfl_xor((int)bits, 16, 64);
     return bits | (uint32_t)__shfl_xor((int)bits, 32, 64);
@@ -324,8 +399,9 @@ __device__ __forceinline__ uint32_t dpp(uint32_t v) {
 // The same for a lane whose registers are the queries i + 4 r and whose key is j0 + l % 16 (bit r:
 // query i + 4 r): a Philox block covers four consecutive keys, i.e. the four lanes of a quad, so
 // lane c of a quad draws the block of query i + 4 c and the quad exchanges them.
+template <bool kParts>
 __device__ __forceinline__ uint32_t keep_queries(const AttnArgs& a, int bh, int i, int j0) {
-    const int c = threadIdx.x & 3, j = j0 + (threadIdx.x & 15);
+    const int c = thread_of<kParts>() & 3, j = j0 + (thread_of<kParts>() & 15);
     const uint32_t mine = keep_keys<4>(a, bh, i + 4 * c, j - c);
     return ((dpp<0x00>(mine) >> c) & 1u) | (((dpp<0x55>(mine) >> c) & 1u) << 1) |
            (((dpp<0xAA>(mine) >> c) & 1u) << 2) | (((dpp<0xFF>(mine) >> c) & 1u) << 3);
@@ -350,6 +426,23 @@ struct Place {
     }
 };
 
+// The kernel's arguments once more, for the pass on fp32 instructions (thread_of: likewise).  What the
+// compiler knows to be the same it would compute once and hold in registers through the first pass,
+// which has none left for a pass that hardly ever follows.
+__device__ __forceinline__ AttnArgs read_again() {
+    typedef const __attribute__((address_space(4))) uint32_t* words_t;
+    words_t p = (words_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    uint32_t w[sizeof(AttnArgs) / sizeof(uint32_t)];
+    static_assert(sizeof(AttnArgs) % sizeof(uint32_t) == 0);
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(w) / sizeof(w[0]); ++i) w[i] = p[i];
+    AttnArgs a;
+    __builtin_memcpy(&a, w, sizeof(a));
+    if (a.dropout) resolve_device_state(a.rng);
+    return a;
+}
+
 // Which elements c of a lane's run are visible: lo <= c <= hi.
 struct Visible {
     int lo, hi;
@@ -366,24 +459,23 @@ __device__ __forceinline__ Visible queries_of_key(const AttnArgs& a, int j, int 
             (a.window > 0 ? min(j + a.window, a.sq) - 1 : a.sq - 1) - first};
 }
 
-template <int DB, int kMode, int kWaves, int kHalves>
-__global__ __launch_bounds__(kHalves* kWaves * 64, per_simd(DB, kHalves* kWaves)) void
-attn_f32_fwd_kernel(const AttnArgs a_in) {
+// One pass of a workgroup over its rows, tiles t_lo .. t_hi - 1.  false (of kParts alone): nothing is
+// written, the caller has the other form do it.
+template <int DB, int kMode, int kWaves, int kHalves, bool kParts>
+__device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int t_lo, int t_hi,
+                                         float* lds) {
     constexpr int kFwdThreads = kHalves * kWaves * 64, kFwdTile = kHalves * kTile;
-    constexpr int kRows = 16 * kWaves, KS = kStepsOf<DB>;
-    AttnArgs a = a_in;
+    constexpr int KS = kStepsOf<DB>;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
-    if (dropout) resolve_device_state(a.rng);
-    extern __shared__ __align__(16) float lds[];
-    typedef Tile<DB, kVec, kFwdTile, kFwdThreads> tile_t;
+    constexpr float kReserve = kParts ? kPartsReserve : 0.f;
+    typedef Tile<DB, kVec, kFwdTile, kFwdThreads, kParts> tile_t;
     constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
     bf16_t* ks = reinterpret_cast<bf16_t*>(lds);  // K[2][tile]
     bf16_t* vs = ks + 2 * kElems;                 // V[2][tile]
-    const Place at(a, a.sq, kRows, true);
-    const int lane = threadIdx.x & 63, g = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = thread_of<kParts>() & 63, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(thread_of<kParts>() >> 6);
     const int wq0 = at.row0 + 16 * (wave % kWaves);
     const int half = wave / kWaves;  // of every tile's keys
     const int row_g = lane_row(g);
@@ -392,35 +484,30 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
     const float* kp = reinterpret_cast<const float*>(a.k) + at.b * a.ks[0] + at.h * a.ks[2];
     const float* vp = reinterpret_cast<const float*>(a.v) + at.b * a.vs[0] + at.h * a.vs[2];
 
-    int j_lo, j_hi;
-    key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
-    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kFwdThreads, true>(a, at.b, at.h, lds) : a.sk));
-    int t_lo = j_lo / kFwdTile, t_hi = (j_hi + kFwdTile - 1) / kFwdTile;
-    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
-
+    float top = 0.f;
     tile_t kt, vt;
-    Split8 qf[KS];
+    operand_t<kParts> qf[KS];
     f32x4_t o[DB], o_small[DB];  // (mma)
     kt.load(kp, a.ks[1], t_lo * kFwdTile, a.sk, a.d);
     vt.load(vp, a.vs[1], t_lo * kFwdTile, a.sk, a.d);
     {
         f32x4_t q[2 * KS];
-        load_row<kVec, KS>(q, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
-        split_row<KS>(qf, q);
+        load_row<kParts, kVec, KS>(q, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
+        hold_row<kParts, KS>(qf, q, top);
     }
 #pragma unroll
     for (int x = 0; x < DB; ++x) o[x] = o_small[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;  // m: in log2 units, as the scores are; l: this lane's share of the row sum
-    kt.store(ks, t_lo * kFwdTile, a.sk, a.d);
-    vt.store(vs, t_lo * kFwdTile, a.sk, a.d);
+    kt.store(ks, t_lo * kFwdTile, a.sk, a.d, top);
+    vt.store(vs, t_lo * kFwdTile, a.sk, a.d, top);
     __syncthreads();
 
     const int wq_last = min(wq0 + 15, a.sq - 1);
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
-        const int part = half * kTile * tile_t::kPitch;
+        const int part = half * kTile * (kParts ? tile_t::kPitch : 2 * kFullPitchOf<DB>);
         const bf16_t *kb = ks + slot * kElems + part, *vb = vs + slot * kElems + part;
-        if (t + 1 < t_hi) {
+        if (kParts && t + 1 < t_hi) {
             kt.load(kp, a.ks[1], (t + 1) * kFwdTile, a.sk, a.d);
             vt.load(vp, a.vs[1], (t + 1) * kFwdTile, a.sk, a.d);
         }
@@ -457,7 +544,7 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
             const bool move = mx > m;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(move) != 0, 0)) {
                 const float m_new = move ? mx + kReserve : m;
-                const float alpha = m == -INFINITY ? 0.f : fast_exp2(m - m_new);
+                const float alpha = m == -INFINITY ? 0.f : exp2_of<kParts>(m - m_new);
                 m = m_new;
                 l *= alpha;
 #pragma unroll
@@ -465,27 +552,34 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
             }
             const float m_ref = m == -INFINITY ? 0.f : m;
             uint32_t bits = 0u;
-            if (dropout) bits = keep_keys32(a, at.bh, i, j0) >> row_g;
+            if (dropout) bits = keep_keys32<kParts>(a, at.bh, i, j0) >> row_g;
 #pragma unroll
             for (int h2 = 0; h2 < 2; ++h2)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float p = fast_exp2(s[h2][r] - m_ref);
+                    float p = exp2_of<kParts>(s[h2][r] - m_ref);
                     l += p;
                     if (dropout) p = (bits >> (16 * h2 + 4 * r)) & 1u ? p * a.rng.inv_keep : 0.f;
                     s[h2][r] = p;
                 }
-            add_rows<DB, kPlane>(vb, split8<true>(s[0], s[1]), o, o_small);
+            add_rows<DB, kPlane>(vb, operand<kParts>(s[0], s[1]), o, o_small);
         }
         if (t + 1 < t_hi) {
-            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d);
-            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d);
+            if (!kParts) kt.load(kp, a.ks[1], (t + 1) * kFwdTile, a.sk, a.d);
+            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d, top);
+            if (!kParts) vt.load(vp, a.vs[1], (t + 1) * kFwdTile, a.sk, a.d);
+            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d, top);
         }
         __syncthreads();
     }
     float l_tot = column_sum(l);
 #pragma unroll
     for (int x = 0; x < DB; ++x) o[x] += o_small[x];
+    if constexpr (kParts) {  // (the votes lie behind the halves' states)
+        const bool ok = top <= kTop && not_finite(o) == 0.f;
+        int* votes = reinterpret_cast<int*>(ks + 4 * kElems) - kHalves * kWaves;
+        if (!everywhere<kHalves * kWaves>(ok, votes)) return false;
+    }
     if constexpr (kHalves == 2) {
         // the second half's state joins the first's through LDS (every wavefront is past the loop's
         // last barrier): lane by lane, the two hold the same rows and columns
@@ -498,10 +592,10 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
             state[4 * DB * 64] = m, state[(4 * DB + 1) * 64] = l_tot;
         }
         __syncthreads();
-        if (half != 0) return;
+        if (half != 0) return true;
         const float m2 = state[4 * DB * 64], m_all = fmaxf(m, m2);
-        const float w1 = m == -INFINITY ? 0.f : fast_exp2(m - m_all);
-        const float w2 = m2 == -INFINITY ? 0.f : fast_exp2(m2 - m_all);
+        const float w1 = m == -INFINITY ? 0.f : exp2_of<kParts>(m - m_all);
+        const float w2 = m2 == -INFINITY ? 0.f : exp2_of<kParts>(m2 - m_all);
         l_tot = l_tot * w1 + state[(4 * DB + 1) * 64] * w2;
         m = m_all;
 #pragma unroll
@@ -509,43 +603,64 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[x][e] = o[x][e] * w1 + state[(4 * x + e) * 64] * w2;
     }
-    if (i >= a.sq) return;
+    if (i >= a.sq) return true;
     if (a.n_split > 1) {
-        store_row<kVec>(o, 1.0f, a.part + (at.part_row0 + i) * a.d, a.d);
+        store_row<kParts, kVec>(o, 1.0f, a.part + (at.part_row0 + i) * a.d, a.d);
         if (g == 0) {
             float* ml = a.part + (int64_t)a.n_split * a.batch * a.heads * a.sq * a.d +
                         2 * (at.part_row0 + i);
             ml[0] = m, ml[1] = l_tot;
         }
-        return;
+        return true;
     }
     float* op = reinterpret_cast<float*>(a.o) + at.b * a.os[0] + (int64_t)i * a.os[1] +
                 at.h * a.os[2];
-    store_row<kVec>(o, 1.0f / l_tot, op, a.d);
+    store_row<kParts, kVec>(o, 1.0f / l_tot, op, a.d);
     // a row that saw nothing but masked keys: see canonical_bias
     if (g == 0)
         a.lse[(int64_t)at.bh * a.sq + i] = m == -kFltMax ? l_tot * kMaskedRowLse
                                                          : __builtin_fmaf(m, kLn2, logf(l_tot));
+    return true;
+}
+template <int DB, int kMode, int kWaves, int kHalves>
+__global__ __launch_bounds__(kHalves* kWaves * 64, per_simd(DB, kHalves* kWaves)) void
+attn_f32_fwd_kernel(const AttnArgs a_in) {
+    constexpr int kFwdThreads = kHalves * kWaves * 64, kFwdTile = kHalves * kTile;
+    constexpr int kRows = 16 * kWaves;
+    AttnArgs a = a_in;
+    constexpr bool kVec = kMode != kGeneral;
+    if (kVec ? (kMode & 2) != 0 : a.dropout != 0) resolve_device_state(a.rng);
+    extern __shared__ __align__(16) float lds[];
+    const Place at(a, a.sq, kRows, true);
+    const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
+                          ? padded_key_limit<kFwdThreads, true>(a, at.b, at.h, lds)
+                          : a.sk;
+    int j_lo, j_hi;
+    key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
+    j_hi = max(j_lo + 1, min(j_hi, limit));
+    int t_lo = j_lo / kFwdTile, t_hi = (j_hi + kFwdTile - 1) / kFwdTile;
+    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
+    if (fwd_pass<DB, kMode, kWaves, kHalves, true>(a, at, t_lo, t_hi, lds)) return;
+    __syncthreads();
+    a = read_again();
+    fwd_pass<DB, kMode, kWaves, kHalves, false>(a, Place(a, a.sq, kRows, true), t_lo, t_hi, lds);
 }
 
 // dQ: dq_i = scale * sum_j ds_ij k_j,  ds = p (dp - delta),  dp = dO_i . v_j.  Also computes
 // delta = rowsum(dO * O) of its rows and stores it for the dK / dV kernel, which runs second.
-template <int DB, int kMode, int kWaves>
-__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnArgs a_in) {
-    constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves, KS = kStepsOf<DB>;
-    AttnArgs a = a_in;
+template <int DB, int kMode, int kWaves, bool kParts>
+__device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int t_lo, int t_hi,
+                                        float* lds) {
+    constexpr int kThreads = kWaves * 64, KS = kStepsOf<DB>;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
-    if (dropout) resolve_device_state(a.rng);
-    extern __shared__ __align__(16) float lds[];
-    typedef Tile<DB, kVec, kTile, kThreads> tile_t;
+    typedef Tile<DB, kVec, kTile, kThreads, kParts> tile_t;
     constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
     bf16_t* ks = reinterpret_cast<bf16_t*>(lds);
     bf16_t* vs = ks + 2 * kElems;
-    const Place at(a, a.sq, kRows, true);
-    const int lane = threadIdx.x & 63, g = lane >> 4, row_g = lane_row(g);
-    const int wq0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = thread_of<kParts>() & 63, g = lane >> 4, row_g = lane_row(g);
+    const int wq0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(thread_of<kParts>() >> 6);
     const int i = wq0 + (lane & 15);
     const float* qp = reinterpret_cast<const float*>(a.q) + at.b * a.qs[0] + at.h * a.qs[2];
     const float* kp = reinterpret_cast<const float*>(a.k) + at.b * a.ks[0] + at.h * a.ks[2];
@@ -553,25 +668,20 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnA
     const float* gp = reinterpret_cast<const float*>(a.dout) + at.b * a.os[0] + at.h * a.os[2];
     const float* op = reinterpret_cast<const float*>(a.o) + at.b * a.os[0] + at.h * a.os[2];
 
-    int j_lo, j_hi;
-    key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
-    j_hi = max(j_lo + 1, min(j_hi, has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk));
-    int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
-    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
-
+    float top = 0.f;
     tile_t kt, vt;
-    Split8 qf[KS], gf[KS];
+    operand_t<kParts> qf[KS], gf[KS];
     f32x4_t dq[DB];
     kt.load(kp, a.ks[1], t_lo * kTile, a.sk, a.d);
     vt.load(vp, a.vs[1], t_lo * kTile, a.sk, a.d);
     float delta = 0.f;
     {
         f32x4_t row[2 * KS], out[2 * KS];
-        load_row<kVec, KS>(row, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
-        split_row<KS>(qf, row);
-        load_row<kVec, KS>(row, gp, a.os[1], i, a.sq, a.d, 1.0f);
-        load_row<kVec, KS>(out, op, a.os[1], i, a.sq, a.d, 1.0f);
-        split_row<KS>(gf, row);
+        load_row<kParts, kVec, KS>(row, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
+        hold_row<kParts, KS>(qf, row, top);
+        load_row<kParts, kVec, KS>(row, gp, a.os[1], i, a.sq, a.d, 1.0f);
+        load_row<kParts, kVec, KS>(out, op, a.os[1], i, a.sq, a.d, 1.0f);
+        hold_row<kParts, KS>(gf, row, top);
 #pragma unroll
         for (int x = 0; x < 2 * KS; ++x)
 #pragma unroll
@@ -584,15 +694,15 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnA
     const float lse = lse_reference(lse_raw, kLog2e), inv_n = lse_row_factor(lse_raw);
     const float rest = masked_row_lse(lse_raw) ? 0.f : __builtin_fmaf(lse_raw, -kLog2e, lse);
     if (g == 0 && i < a.sq) a.delta[(int64_t)at.bh * a.sq + i] = delta;
-    kt.store(ks, t_lo * kTile, a.sk, a.d);
-    vt.store(vs, t_lo * kTile, a.sk, a.d);
+    kt.store(ks, t_lo * kTile, a.sk, a.d, top);
+    vt.store(vs, t_lo * kTile, a.sk, a.d, top);
     __syncthreads();
 
     const int wq_last = min(wq0 + 15, a.sq - 1);
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
         const bf16_t *kb = ks + slot * kElems, *vb = vs + slot * kElems;
-        if (t + 1 < t_hi) {
+        if (kParts && t + 1 < t_hi) {
             kt.load(kp, a.ks[1], (t + 1) * kTile, a.sk, a.d);
             vt.load(vp, a.vs[1], (t + 1) * kTile, a.sk, a.d);
         }
@@ -603,7 +713,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnA
             const bool masked = j0 + kTile > a.sk || (a.causal && j0 + kTile - 1 > wq0) ||
                                 (a.window > 0 && wq_last - j0 >= a.window);
             uint32_t bits = 0u;
-            if (dropout) bits = keep_keys32(a, at.bh, i, j0) >> row_g;
+            if (dropout) bits = keep_keys32<kParts>(a, at.bh, i, j0) >> row_g;
             f32x4_t ds[2];
 #pragma unroll
             for (int h2 = 0; h2 < 2; ++h2) {
@@ -618,7 +728,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnA
                     if (dropout) y = (bits >> (16 * h2 + 4 * r)) & 1u ? y * a.rng.inv_keep : 0.f;
                     y -= delta;
                     if (has_bias) y *= inv_n;  // (1 without a bias)
-                    ds[h2][r] = fast_exp2(x - lse) * y;
+                    ds[h2][r] = exp2_of<kParts>(x - lse) * y;
                 }
             }
             if (masked) {  // uniform
@@ -629,76 +739,95 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnA
                     for (int r = 0; r < 4; ++r)
                         if (!vis(16 * h2 + 4 * r)) ds[h2][r] = 0.f;
             }
-            add_rows<DB, kPlane>(kb, split8(ds[0], ds[1]), dq, dq);
+            add_rows<DB, kPlane>(kb, operand<kParts>(ds[0], ds[1]), dq, dq);
         }
         if (t + 1 < t_hi) {
-            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d);
-            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d);
+            if (!kParts) kt.load(kp, a.ks[1], (t + 1) * kTile, a.sk, a.d);
+            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d, top);
+            if (!kParts) vt.load(vp, a.vs[1], (t + 1) * kTile, a.sk, a.d);
+            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d, top);
         }
         __syncthreads();
     }
-    if (i >= a.sq) return;
+    if constexpr (kParts) {
+        const bool ok = top <= kTop && not_finite(dq) == 0.f;
+        if (!everywhere<kWaves>(ok, reinterpret_cast<int*>(lds))) return false;
+    }
+    if (i >= a.sq) return true;
     if (a.n_split > 1) {
-        store_row<kVec>(dq, a.scale, a.part + (at.part_row0 + i) * a.d, a.d);
-        return;
+        store_row<kParts, kVec>(dq, a.scale, a.part + (at.part_row0 + i) * a.d, a.d);
+        return true;
     }
     float* dqp = reinterpret_cast<float*>(a.dq) + at.b * a.dqs[0] + (int64_t)i * a.dqs[1] +
                  at.h * a.dqs[2];
-    store_row<kVec>(dq, a.scale, dqp, a.d);
+    store_row<kParts, kVec>(dq, a.scale, dqp, a.d);
+    return true;
+}
+template <int DB, int kMode, int kWaves>
+__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnArgs a_in) {
+    constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves;
+    AttnArgs a = a_in;
+    constexpr bool kVec = kMode != kGeneral;
+    if (kVec ? (kMode & 2) != 0 : a.dropout != 0) resolve_device_state(a.rng);
+    extern __shared__ __align__(16) float lds[];
+    const Place at(a, a.sq, kRows, true);
+    const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
+                          ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds)
+                          : a.sk;
+    int j_lo, j_hi;
+    key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
+    j_hi = max(j_lo + 1, min(j_hi, limit));
+    int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
+    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
+    if (dq_pass<DB, kMode, kWaves, true>(a, at, t_lo, t_hi, lds)) return;
+    __syncthreads();
+    a = read_again();
+    dq_pass<DB, kMode, kWaves, false>(a, Place(a, a.sq, kRows, true), t_lo, t_hi, lds);
 }
 
 // dK and dV: a wavefront owns 16 keys, queries stream through LDS.
 //   dv_j = sum_i pdrop_ij dO_i          dk_j = scale * sum_i ds_ij q_i
-template <int DB, int kMode, int kWaves>
-__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const AttnArgs a_in) {
-    constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves, KS = kStepsOf<DB>;
-    AttnArgs a = a_in;
+template <int DB, int kMode, int kWaves, bool kParts>
+__device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int t_lo, int t_hi,
+                                         float* lds) {
+    constexpr int kThreads = kWaves * 64, KS = kStepsOf<DB>;
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
-    if (dropout) resolve_device_state(a.rng);
-    extern __shared__ __align__(16) float lds[];
-    typedef Tile<DB, kVec, kTile, kThreads> tile_t;
+    typedef Tile<DB, kVec, kTile, kThreads, kParts> tile_t;
     constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
     bf16_t* qs = reinterpret_cast<bf16_t*>(lds);
     bf16_t* gs = qs + 2 * kElems;
     // [2][4][kTile]: lse reference and its rest, its factor, delta; rows in the order of the accumulators (row
     // 16 h + 4 r + e at 16 h + 4 e + r)
     float* rows = reinterpret_cast<float*>(gs + 2 * kElems);
-    const Place at(a, a.sk, kRows, false);
-    const int lane = threadIdx.x & 63, g = lane >> 4, row_g = lane_row(g);
-    const int wk0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = thread_of<kParts>() & 63, g = lane >> 4, row_g = lane_row(g);
+    const int wk0 = at.row0 + 16 * __builtin_amdgcn_readfirstlane(thread_of<kParts>() >> 6);
     const int j = wk0 + (lane & 15);
     const float* qp = reinterpret_cast<const float*>(a.q) + at.b * a.qs[0] + at.h * a.qs[2];
     const float* kp = reinterpret_cast<const float*>(a.k) + at.b * a.ks[0] + at.h * a.ks[2];
     const float* vp = reinterpret_cast<const float*>(a.v) + at.b * a.vs[0] + at.h * a.vs[2];
     const float* gp = reinterpret_cast<const float*>(a.dout) + at.b * a.os[0] + at.h * a.os[2];
 
-    int i_lo, i_hi;
-    query_range(a, at.row0, min(at.row0 + kRows, a.sk), i_lo, i_hi);
-    // keys past the last unpadded one get no probability from any row
-    if (at.row0 >= (has_bias ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds) : a.sk)) i_hi = i_lo;
-    int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
-    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
-
+    float top = 0.f;
     tile_t qt, gt;
-    Split8 kf[KS], vf[KS];
+    operand_t<kParts> kf[KS], vf[KS];
     f32x4_t dk[DB], dv[DB];
     float lse_r = 0.f, delta_r = 0.f;  // thread x < kTile: row x of the tile on its way
     auto request = [&](int t) __attribute__((always_inline)) {
         qt.load(qp, a.qs[1], t * kTile, a.sq, a.d);
         gt.load(gp, a.os[1], t * kTile, a.sq, a.d);
-        if (threadIdx.x < kTile) {
-            const int64_t row = (int64_t)at.bh * a.sq + min(t * kTile + (int)threadIdx.x, a.sq - 1);
+        if (thread_of<kParts>() < kTile) {
+            const int64_t row = (int64_t)at.bh * a.sq + min(t * kTile + (int)thread_of<kParts>(), a.sq - 1);
             lse_r = a.lse[row];
             delta_r = a.delta[row];
         }
     };
     auto publish = [&](int t, int slot) __attribute__((always_inline)) {
-        qt.store(qs + slot * kElems, t * kTile, a.sq, a.d);
-        gt.store(gs + slot * kElems, t * kTile, a.sq, a.d);
-        if (threadIdx.x < kTile) {
-            const int x = threadIdx.x;
+        qt.store(qs + slot * kElems, t * kTile, a.sq, a.d, top);
+        gt.store(gs + slot * kElems, t * kTile, a.sq, a.d, top);
+        if (thread_of<kParts>() < kTile) {
+            const int x = thread_of<kParts>();
             float* r = rows + slot * 4 * kTile + ((x & 16) | (x & 3) << 2 | (x >> 2 & 3));
             const float lse = lse_reference(lse_r, kLog2e);
             r[0] = lse;
@@ -709,10 +838,10 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const Attn
     };
     {
         f32x4_t row[2 * KS];
-        load_row<kVec, KS>(row, kp, a.ks[1], j, a.sk, a.d, a.scale_log2);
-        split_row<KS>(kf, row);
-        load_row<kVec, KS>(row, vp, a.vs[1], j, a.sk, a.d, 1.0f);
-        split_row<KS>(vf, row);
+        load_row<kParts, kVec, KS>(row, kp, a.ks[1], j, a.sk, a.d, a.scale_log2);
+        hold_row<kParts, KS>(kf, row, top);
+        load_row<kParts, kVec, KS>(row, vp, a.vs[1], j, a.sk, a.d, 1.0f);
+        hold_row<kParts, KS>(vf, row, top);
     }
 #pragma unroll
     for (int x = 0; x < DB; ++x) dk[x] = dv[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -727,7 +856,7 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const Attn
         const int slot = (t - t_lo) & 1;
         const bf16_t *qb = qs + slot * kElems, *gb = gs + slot * kElems;
         const float* rb = rows + slot * 4 * kTile;
-        if (t + 1 < t_hi) request(t + 1);
+        if (kParts && t + 1 < t_hi) request(t + 1);
         const int i0 = t * kTile;
         const bool active = wk0 < a.sk && (!a.causal || i0 + kTile - 1 >= wk0) &&
                             (a.window <= 0 || i0 - wk_last < a.window);
@@ -745,14 +874,14 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const Attn
                 const f32x4_t s = dot_rows<DB, kPlane>(qb, 16 * h2, kf, rest);
                 const f32x4_t dp = dot_rows<DB, kPlane>(gb, 16 * h2, vf);
                 uint32_t bits = 0u;
-                if (dropout) bits = keep_queries(a, at.bh, i0 + 16 * h2 + row_g, wk0);
+                if (dropout) bits = keep_queries<kParts>(a, at.bh, i0 + 16 * h2 + row_g, wk0);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int i = i0 + 16 * h2 + 4 * r + row_g;
                     float x = s[r];
                     if (has_bias)
                         x += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
-                    float p = fast_exp2(x - lse[r]);
+                    float p = exp2_of<kParts>(x - lse[r]);
                     if (has_bias) p *= rb[3 * kTile + r0 + r];  // (1 without a bias)
                     const float keep = dropout ? ((bits >> r) & 1u ? a.rng.inv_keep : 0.f) : 1.f;
                     pd[h2][r] = p * keep;
@@ -767,26 +896,56 @@ __global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const Attn
                     for (int r = 0; r < 4; ++r)
                         if (!vis(16 * h2 + 4 * r)) pd[h2][r] = ds[h2][r] = 0.f;
             }
-            add_rows<DB, kPlane>(gb, split8<true>(pd[0], pd[1]), dv, dv);
-            add_rows<DB, kPlane>(qb, split8(ds[0], ds[1]), dk, dk);
+            add_rows<DB, kPlane>(gb, operand<kParts>(pd[0], pd[1]), dv, dv);
+            add_rows<DB, kPlane>(qb, operand<kParts>(ds[0], ds[1]), dk, dk);
         }
-        if (t + 1 < t_hi) publish(t + 1, slot ^ 1);
+        if (t + 1 < t_hi) {
+            if (!kParts) request(t + 1);
+            publish(t + 1, slot ^ 1);
+        }
         __syncthreads();
     }
-    if (j >= a.sk) return;
+    if constexpr (kParts) {
+        const bool ok = top <= kTop && not_finite(dv, not_finite(dk)) == 0.f;
+        if (!everywhere<kWaves>(ok, reinterpret_cast<int*>(lds))) return false;
+    }
+    if (j >= a.sk) return true;
     if (a.n_split > 1) {
         float* part = a.part + (at.part_row0 + j) * a.d;
-        store_row<kVec>(dk, a.scale, part, a.d);
-        store_row<kVec>(dv, 1.0f,
+        store_row<kParts, kVec>(dk, a.scale, part, a.d);
+        store_row<kParts, kVec>(dv, 1.0f,
                         part + (int64_t)a.n_split * a.batch * a.heads * a.sk * a.d, a.d);
-        return;
+        return true;
     }
     float* dkp = reinterpret_cast<float*>(a.dk) + at.b * a.dks[0] + (int64_t)j * a.dks[1] +
                  at.h * a.dks[2];
     float* dvp = reinterpret_cast<float*>(a.dv) + at.b * a.dvs[0] + (int64_t)j * a.dvs[1] +
                  at.h * a.dvs[2];
-    store_row<kVec>(dk, a.scale, dkp, a.d);
-    store_row<kVec>(dv, 1.0f, dvp, a.d);
+    store_row<kParts, kVec>(dk, a.scale, dkp, a.d);
+    store_row<kParts, kVec>(dv, 1.0f, dvp, a.d);
+    return true;
+}
+template <int DB, int kMode, int kWaves>
+__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const AttnArgs a_in) {
+    constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves;
+    AttnArgs a = a_in;
+    constexpr bool kVec = kMode != kGeneral;
+    if (kVec ? (kMode & 2) != 0 : a.dropout != 0) resolve_device_state(a.rng);
+    extern __shared__ __align__(16) float lds[];
+    const Place at(a, a.sk, kRows, false);
+    const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
+                          ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds)
+                          : a.sk;
+    int i_lo, i_hi;
+    query_range(a, at.row0, min(at.row0 + kRows, a.sk), i_lo, i_hi);
+    // keys past the last unpadded one get no probability from any row
+    if (at.row0 >= limit) i_hi = i_lo;
+    int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
+    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
+    if (dkv_pass<DB, kMode, kWaves, true>(a, at, t_lo, t_hi, lds)) return;
+    __syncthreads();
+    a = read_again();
+    dkv_pass<DB, kMode, kWaves, false>(a, Place(a, a.sk, kRows, false), t_lo, t_hi, lds);
 }
 
 enum class Which { kFwd, kDq, kDkv };

@@ -825,6 +825,85 @@ def test_fp32_values_at_the_ends_of_the_range(head_dim):
     assert err <= 1e-5, err  # the fp32 bar of unit-scale values, per column
 
 
+def _plain_fwd_bwd(q, k, v, do):
+    """Attention without a mask and its gradients in 64 bits, as sums of products (infinities times zero
+    included), delta as rowsum(dO * O)."""
+    q, k, v, do = (t.double().transpose(1, 2) for t in (q, k, v, do))
+    prod = lambda x, y: (x.unsqueeze(3) * y.unsqueeze(2)).sum(-1)
+    scale = q.shape[-1] ** -0.5
+    p = torch.softmax(prod(q, k) * scale, -1)
+    out = prod(p, v.transpose(2, 3))
+    ds = p * (prod(do, v) - (do * out).sum(-1, keepdim=True))
+    dq = prod(ds, k.transpose(2, 3)) * scale
+    dk = prod(ds.transpose(2, 3), q.transpose(2, 3)) * scale
+    dv = prod(p.transpose(2, 3), do.transpose(2, 3))
+    return [t.transpose(1, 2) for t in (out, dq, dk, dv)]
+
+
+@pytest.mark.parametrize("head_dim", [64, 80, 128])
+def test_fp32_gradients_at_the_ends_of_the_range(head_dim):
+    """Infinities, NaN and values that bf16 rounds to infinity in each operand of the backward, a head
+    for each: finite, infinite and NaN where 64-bit sums of products are."""
+    q, k, v, do, _ = _inputs(1, 70, 9, head_dim, torch.float32)
+    top, inf = torch.finfo(torch.float32).max, float("inf")
+    v[0, 60, 0, 0], do[0, :, 0, 0] = top, 0.0
+    v[0, 4, 1, 1] = inf
+    v[0, 4, 2, 1], do[0, 9, 2, 1] = -inf, inf
+    do[0, 6, 3, 3] = -inf
+    do[0, 6, 4, 3], v[0, :, 4, 3] = top, 0.0
+    k[0, 7, 5, 5] = -inf
+    q[0, 69, 6, 5] = float("nan")
+    q[0, 3, 7, 2], k[0, :, 7, 2] = -top, 0.0
+    k[0, 3, 8, 2], q[0, :, 8, 2] = top, 0.0
+    do[0, :, 7:] *= 1e-3  # (the sums stay below the largest number before they are scaled)
+    got = _run(q, k, v, do, None, False)
+    for name, a, r in zip(("out", "dq", "dk", "dv"), got, _plain_fwd_bwd(q, k, v, do)):
+        a, big = a.detach().cpu().double(), r.abs() > top  # what fp32 cannot hold
+        r = r.where(~big, r.sign() * inf)
+        assert torch.equal(a.isnan(), r.isnan()), name
+        assert torch.equal(a.isinf(), r.isinf()), name
+        ok = r.isfinite()
+        scale = r.where(ok, torch.zeros_like(r)).abs().amax(dim=1, keepdim=True).clamp(min=1.0)
+        err = ((a - r).where(ok, torch.zeros_like(r)).abs() / scale).max().item()
+        assert err <= 2e-5, (name, err)
+
+
+@pytest.mark.parametrize("mask", ["none", "key", "square"])
+@pytest.mark.parametrize("shape,sk,causal,window,p", [
+    ((2, 70, 3, 64), 70, True, 0, 0.1),
+    ((1, 130, 2, 80), 97, False, 0, 0.0),
+    ((1, 257, 2, 128), 257, True, 33, 0.1),
+    ((1, 63, 2, 30), 100, False, 0, 0.3),    # rows that are not 16-byte aligned
+    ((1, 300, 1, 24), 300, True, 0, 0.0),
+    ((1, 640, 1, 64), 640, True, 0, 0.1),    # dealt tiles
+    ((8, 530, 9, 64), 530, False, 0, 0.0),   # eight wavefronts in the backward as well
+    ((1, 90, 2, 96), 300, False, 0, 0.1),
+])
+def test_fp32_values_too_large_for_bf16_parts(shape, sk, causal, window, p, mask):
+    """One value of 1e19 in each operand, against a column of zeros in the other factor of its product:
+    the workgroups that meet it run their rows again on fp32 instructions, and everything but the
+    column that it scales is as it was.  Errors are measured by the column's largest value; a column that
+    is scaled holds one ds (or p) times 1e19, whose error of 1e-6 stands against values from 0.02 up."""
+    q, k, v, do, g = _inputs(*shape, torch.float32, sk=sk)
+    m = None
+    if mask != "none":
+        m = torch.randn(shape[0], 1, 1 if mask == "key" else shape[1], sk, generator=g)
+    i, j, huge = shape[1] // 3, min(sk, shape[1]) // 4, 1e19
+    v[:, j, :, 0], do[..., 0] = huge, 0.0
+    k[:, j, :, 1], q[..., 1] = huge, 0.0
+    q[:, i, :, 2], k[..., 2] = -huge, 0.0
+    do[:, i, :, 3], v[..., 3] = huge, 0.0
+    got = _run(q, k, v, do, m, causal, window, p)
+    keep = _torch_keep(shape[0], shape[2], shape[1], sk, p) if p > 0 else None
+    ref = OA.attention_fwd_bwd(q, k, v, do, m, causal, window, p, keep, None, torch.float64)
+    for name, scaled, a, r in zip(("out", "dq", "dk", "dv"), range(4), got, ref):
+        a, r = a.detach().cpu().double(), r.double()
+        err = (a - r).abs().amax(dim=(0, 1, 2)) / r.abs().amax(dim=(0, 1, 2)).clamp(min=1.0)
+        assert err[scaled].item() <= 5e-5, (name, err[scaled])
+        err[scaled] = 0.0
+        assert err.max().item() <= 1e-5, (name, err.max())
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("b,h,d,sk,layout", [
     (1, 1, 8, 1, None),            # one key
