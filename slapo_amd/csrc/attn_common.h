@@ -156,6 +156,14 @@ __device__ __forceinline__ float bias_log2(float b) {
 __device__ __forceinline__ bool masked_row_lse(float lse) {
     return lse >= 0.5f * kMaskedRowLse && lse < INFINITY;
 }
+// Log-sum-exp of a row with reference point m in log2 units and row sum l, rounded once (l near 1 after
+// the powers of two are taken out of it): what is lost here every probability of the row loses in the
+// backward.
+__device__ __forceinline__ float row_lse(float m, float l) {
+    int e;
+    const float f = __builtin_frexpf(l, &e);
+    return (float)__builtin_fma((double)m + e, 0.69314718055994531, (double)logf(f));
+}
 // The reference point that exp subtracts for a stored log-sum-exp, times `unit` (1 for natural
 // units, log2(e) for log2 units), and the factor 1 / n that goes with it (1 for ordinary rows).
 __device__ __forceinline__ float lse_reference(float lse, float unit) {

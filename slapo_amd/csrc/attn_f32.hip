@@ -1,15 +1,20 @@
 // Attention forward and backward for fp32 tensors, the kernels behind dtype == SLAPO_F32, whose
 // parity bar is 1e-5 absolute.
 //
-// Products run on the bf16 matrix instructions without giving up fp32: an operand is the exact sum
-// of three bf16 numbers, x = h + m + l (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 8 + 8 + 8
-// mantissa bits, fp32's exponent range), and x y = hh + (hm + mh) + (mm + hl + lh) + O(2^-25 |x y|),
-// six v_mfma_f32_16x16x32_bf16 with exact products and fp32 sums.
-// Infinities have no such parts, and numbers that bf16 rounds to infinity none that are finite.  A
-// workgroup that meets a magnitude above kTop, or whose results are not all finite, writes nothing and
-// runs its rows again on v_mfma_f32_16x16x4_f32 (Full8), whose products are fp32's own: infinity times
-// infinity is one.  It costs such a call two to three times the time and the others nothing (B4 S512 H16
-// D64 33 us before and after; forward and backward 125).
+// Products run on the bf16 matrix instructions without giving up fp32: an operand is the sum of three
+// bf16 numbers, x = h + m + l (h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 8 + 8 + 8 mantissa
+// bits), and x y = hh + (hm + mh) + (mm + hl + lh) + O(2^-25 |x y|), six v_mfma_f32_16x16x32_bf16 with
+// exact products and fp32 sums.  The parts have the three ranges that fp32's has not:
+//  * l's last bit is 2^-24 x: below 2^-102 it leaves bf16's normal numbers.  V, K, Q, dO, the
+//    probabilities and dS are therefore split at 2^24 times their size (kUp), exactly, and the results
+//    are lowered again: every normal fp32 number is the exact sum of its parts.  Only scores need no such
+//    care: what their operands lose is at most 2^-125 each, 2^-58 of a score beside numbers below 2^60.
+//  * What bf16 rounds to infinity, and infinities, have no finite parts.  A workgroup that meets a
+//    magnitude above 2^36 (2^60 at the size held: kTop), or whose results are not all finite, writes
+//    nothing and runs its rows again on v_mfma_f32_16x16x4_f32 (Full8), whose products are fp32's own:
+//    infinity times infinity is one.  Where all do, a call takes 2.4 times as long (forward and
+//    backward of B4 S512 H16 D64 133 -> 317 us).
+//  * Probabilities below 2^-126 are zero in the first pass (v_exp_f32).
 //
 // v_mfma_f32_16x16x32_bf16 (one wavefront, lane l, i = l % 16, g = l / 16):
 //   A operand: lane holds A[row i][k-slots 8 g .. 8 g + 7];   B operand: the same slots of column i;
@@ -30,12 +35,14 @@
 // cycles -- the fp32 matrix instructions take 2048 --, about 200 vector instructions (half of them
 // the splitting of the tile and of the probabilities) and 24 KB of LDS reads: no one of the three
 // binds, their sum does.  fp32 matrix instructions in the same layout -> these: forward B4 S512
-// H16 D64 50.9 -> 33.2 us (83 -> 129 TFLOP/s), B16 S512 H16 D64 184 -> 103, B2 S2048 H16 D128 701 -> 356
-// (193 TFLOP/s; the fp32 instructions stop at 157); forward and backward B4 S512 H16 D64 210 -> 125, B4
-// S1024 H8 D80 554 -> 337, B1 S1024 H8 D128 causal 233 -> 146.  Errors against 64 bits (2-norm) at B4
-// S512 H16 D64: output 4.1e-7 -> 2.0e-7, gradients 6.2e-7 -> 5.3e-7; at B2 S2048 H16 D128 output
-// 9.3e-7 -> 3.7e-7.
-//
+// H16 D64 50.9 -> 33.1 us (83 -> 130 TFLOP/s), B16 S512 H16 D64 184 -> 102, B2 S2048 H16 D128 701 -> 357
+// (193 TFLOP/s; the fp32 instructions stop at 157, six bf16 products for one at about 222); forward and
+// backward B4 S512 H16 D64 210 -> 124, B4 S1024 H8 D80 554 -> 334, B1 S1024 H8 D128 causal 233 -> 146.
+// Errors against 64 bits (2-norm) at B4 S512 H16 D64: output 4.1e-7 -> 2.0e-7, gradients 6.2e-7 ->
+// 4.3e-7; at B2 S2048 H16 D128 output 9.3e-7 -> 3.7e-7.
+// What the sizes held above (kUp) and the largest magnitude cost: B4 S512 H16 D64 32.7 -> 33.1 us
+// forward, 150.0 -> 152.5 with a padding mask and backward; what it gave, by fewer branches: B4 S700 H12
+// D80 causal and padded 67.9 -> 66.0 forward, B2 S1000 H6 D96 window 200 85.8 -> 82.3 with backward.
 //
 // Reference semantics: slapo/op/attention.py:163-181 (attention_bmk) and its autograd.
 #include <type_traits>
@@ -62,7 +69,10 @@ constexpr int64_t kWideBwd = 512;   // in units of 64 rows: B4 S512 H16 D64 (512
 constexpr int64_t kHalvesBelow = 128;
 // LDS and registers leave a SIMD four of a forward's wavefronts up to head_dim 64, else two.
 constexpr int per_simd(int db, int waves) { return db <= 4 && waves >= 8 ? 4 : 2; }
-constexpr float kPartsReserve = 8.0f;  // of the softmax reference above the maximum, log2 units
+// ... of a backward kernel's four up to head_dim 32 where no dropout is drawn for columns, else two.
+constexpr int per_simd_bwd(int db, bool draws) { return db <= 2 && !draws ? 4 : 2; }
+// The forward moves its softmax reference when a score stands more than this above it, in log2 units.
+constexpr float kPartsAhead = 8.0f;
 
 typedef Mma<bf16_t>::frag frag_t;
 __device__ __forceinline__ f32x4_t splat(float v) { return f32x4_t{v, v, v, v}; }
@@ -120,8 +130,13 @@ __device__ __forceinline__ operand_t<kParts> operand(const f32x4_t& a, const f32
         return {a, b};
     }
 }
-// What a pass in bf16 parts has to see below kTop: then every part, every score and every dO v is finite,
-// and a result that went wrong on the way (a sum past fp32's range) is not.
+// In parts everything but the scores' own operands is held kUp times its size: the last part of a number of
+// 2^-126 is then one of 2^-126, where bf16 has all its bits, instead of one of 2^-150, where it has none.
+constexpr float kUp = 0x1p24f;
+template <bool kParts>
+constexpr float lift = kParts ? kUp : 1.0f;
+// What a pass in bf16 parts may see, at the size held: up to it every part, every score and every dO v is
+// finite, and a result that went wrong on the way (a sum past fp32's range) is not.
 constexpr float kTop = 0x1p60f;
 // top = the largest magnitude so far (not of NaN, which reaches the results)
 __device__ __forceinline__ void track(float& top, const f32x4_t& v) {
@@ -219,6 +234,8 @@ struct Tile {
             }
         }
     }
+    // times kUp where kLift; `top` tracked where kScores (an operand of the scores)
+    template <bool kLift, bool kScores>
     __device__ __forceinline__ void store(bf16_t* lds, int row0, int n_rows, int d, float& top) {
         if (row0 + kTileRows > n_rows || d < 32 * kStepsOf<DB>) {  // uniform
 #pragma unroll
@@ -237,7 +254,8 @@ struct Tile {
             const int row = c / kPerRow, col = 4 * (c % kPerRow);
             if constexpr (kParts) {
                 uint32_t h[2], m[2], l[2];
-                track(top, r[u]);
+                if (kLift) r[u] *= kUp;
+                if (kScores) track(top, r[u]);
                 split2(r[u][0], r[u][1], h[0], m[0], l[0]);
                 split2(r[u][2], r[u][3], h[1], m[1], l[1]);
                 bf16_t* p = lds + row * kPitch + col;
@@ -273,13 +291,14 @@ __device__ __forceinline__ void load_row(f32x4_t (&f)[2 * KS], const float* base
     }
 }
 template <bool kParts, int KS>
-__device__ __forceinline__ void hold_row(operand_t<kParts> (&f)[KS], const f32x4_t (&v)[2 * KS],
-                                         float& top) {
+__device__ __forceinline__ void hold_row(operand_t<kParts> (&f)[KS], const f32x4_t (&v)[2 * KS]) {
 #pragma unroll
-    for (int t = 0; t < KS; ++t) {
-        if constexpr (kParts) track(top, v[2 * t]), track(top, v[2 * t + 1]);
-        f[t] = operand<kParts>(v[2 * t], v[2 * t + 1]);
-    }
+    for (int t = 0; t < KS; ++t) f[t] = operand<kParts>(v[2 * t], v[2 * t + 1]);
+}
+template <int N>
+__device__ __forceinline__ void track_row(float& top, const f32x4_t (&v)[N]) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) track(top, v[t]);
 }
 
 // small + A B over the head dimension: A = 16 tile rows from row `r0` on, B = this lane's fragments.
@@ -354,19 +373,21 @@ __device__ __forceinline__ void add_rows(const bf16_t* tile, const Full8& w, f32
         }
 }
 
-// Writes this lane's column of acc (element 16 x + 4 g + r in acc[x][r]) times mul as row `row`.
+// Writes this lane's column of acc (element 16 x + 4 g + r in acc[x][r]), lowered by `down` (a power of
+// two, so that mul meets what fp32 sums would be), times mul as row `row`.
 template <bool kParts, bool kVec, int DB>
-__device__ __forceinline__ void store_row(const f32x4_t (&acc)[DB], float mul, float* row, int d) {
+__device__ __forceinline__ void store_row(const f32x4_t (&acc)[DB], float down, float mul,
+                                          float* row, int d) {
     const int g = (thread_of<kParts>() & 63) >> 4;
 #pragma unroll
     for (int x = 0; x < DB; ++x) {
         const int col = 16 * x + 4 * g;
         if constexpr (kVec) {
-            if (col < d) *reinterpret_cast<f32x4_t*>(row + col) = acc[x] * mul;
+            if (col < d) *reinterpret_cast<f32x4_t*>(row + col) = acc[x] * down * mul;
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (col + e < d) row[col + e] = acc[x][e] * mul;
+                if (col + e < d) row[col + e] = acc[x][e] * down * mul;
         }
     }
 }
@@ -469,7 +490,7 @@ __device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int
     constexpr bool kVec = kMode != kGeneral;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
-    constexpr float kReserve = kParts ? kPartsReserve : 0.f;
+    constexpr float kAhead = kParts ? kPartsAhead : 0.f, kLift = lift<kParts>;
     typedef Tile<DB, kVec, kFwdTile, kFwdThreads, kParts> tile_t;
     constexpr int kElems = tile_t::kElems, kPlane = tile_t::kPlane;
     bf16_t* ks = reinterpret_cast<bf16_t*>(lds);  // K[2][tile]
@@ -493,16 +514,18 @@ __device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int
     {
         f32x4_t q[2 * KS];
         load_row<kParts, kVec, KS>(q, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
-        hold_row<kParts, KS>(qf, q, top);
+        if (kParts) track_row(top, q);
+        hold_row<kParts, KS>(qf, q);
     }
 #pragma unroll
     for (int x = 0; x < DB; ++x) o[x] = o_small[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;  // m: in log2 units, as the scores are; l: this lane's share of the row sum
-    kt.store(ks, t_lo * kFwdTile, a.sk, a.d, top);
-    vt.store(vs, t_lo * kFwdTile, a.sk, a.d, top);
+    kt.template store<false, true>(ks, t_lo * kFwdTile, a.sk, a.d, top);
+    vt.template store<kParts, true>(vs, t_lo * kFwdTile, a.sk, a.d, top);
     __syncthreads();
 
     const int wq_last = min(wq0 + 15, a.sq - 1);
+    const float kept = dropout ? a.rng.inv_keep * kLift : kLift;
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
         const int part = half * kTile * (kParts ? tile_t::kPitch : 2 * kFullPitchOf<DB>);
@@ -540,10 +563,10 @@ __device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int
 #pragma unroll
             for (int r = 0; r < 4; ++r) mx = fmaxf(mx, fmaxf(s[0][r], s[1][r]));
             mx = column_max(mx);
-            // moved lazily, to kReserve above the maximum: probabilities stay at or below 1
-            const bool move = mx > m;
+            // moved lazily: probabilities stay at or below 2^kAhead
+            const bool move = mx - m > kAhead;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(move) != 0, 0)) {
-                const float m_new = move ? mx + kReserve : m;
+                const float m_new = move ? mx : m;
                 const float alpha = m == -INFINITY ? 0.f : exp2_of<kParts>(m - m_new);
                 m = m_new;
                 l *= alpha;
@@ -559,16 +582,16 @@ __device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int
                 for (int r = 0; r < 4; ++r) {
                     float p = exp2_of<kParts>(s[h2][r] - m_ref);
                     l += p;
-                    if (dropout) p = (bits >> (16 * h2 + 4 * r)) & 1u ? p * a.rng.inv_keep : 0.f;
-                    s[h2][r] = p;
+                    const bool drop = dropout && ((bits >> (16 * h2 + 4 * r)) & 1u) == 0;
+                    s[h2][r] = drop ? 0.f : p * kept;
                 }
             add_rows<DB, kPlane>(vb, operand<kParts>(s[0], s[1]), o, o_small);
         }
         if (t + 1 < t_hi) {
             if (!kParts) kt.load(kp, a.ks[1], (t + 1) * kFwdTile, a.sk, a.d);
-            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d, top);
+            kt.template store<false, true>(ks + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d, top);
             if (!kParts) vt.load(vp, a.vs[1], (t + 1) * kFwdTile, a.sk, a.d);
-            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d, top);
+            vt.template store<kParts, true>(vs + (slot ^ 1) * kElems, (t + 1) * kFwdTile, a.sk, a.d, top);
         }
         __syncthreads();
     }
@@ -605,7 +628,7 @@ __device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int
     }
     if (i >= a.sq) return true;
     if (a.n_split > 1) {
-        store_row<kParts, kVec>(o, 1.0f, a.part + (at.part_row0 + i) * a.d, a.d);
+        store_row<kParts, kVec>(o, 1.0f / (kLift * kLift), 1.0f, a.part + (at.part_row0 + i) * a.d, a.d);
         if (g == 0) {
             float* ml = a.part + (int64_t)a.n_split * a.batch * a.heads * a.sq * a.d +
                         2 * (at.part_row0 + i);
@@ -615,11 +638,11 @@ __device__ __forceinline__ bool fwd_pass(const AttnArgs& a, const Place& at, int
     }
     float* op = reinterpret_cast<float*>(a.o) + at.b * a.os[0] + (int64_t)i * a.os[1] +
                 at.h * a.os[2];
-    store_row<kParts, kVec>(o, 1.0f / l_tot, op, a.d);
+    store_row<kParts, kVec>(o, 1.0f / (kLift * kLift), 1.0f / l_tot, op, a.d);
     // a row that saw nothing but masked keys: see canonical_bias
     if (g == 0)
         a.lse[(int64_t)at.bh * a.sq + i] = m == -kFltMax ? l_tot * kMaskedRowLse
-                                                         : __builtin_fmaf(m, kLn2, logf(l_tot));
+                                                         : row_lse(m, l_tot);
     return true;
 }
 template <int DB, int kMode, int kWaves, int kHalves>
@@ -653,6 +676,7 @@ __device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int 
                                         float* lds) {
     constexpr int kThreads = kWaves * 64, KS = kStepsOf<DB>;
     constexpr bool kVec = kMode != kGeneral;
+    constexpr float kLift = lift<kParts>;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
     typedef Tile<DB, kVec, kTile, kThreads, kParts> tile_t;
@@ -677,15 +701,18 @@ __device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int 
     float delta = 0.f;
     {
         f32x4_t row[2 * KS], out[2 * KS];
-        load_row<kParts, kVec, KS>(row, qp, a.qs[1], i, a.sq, a.d, a.scale_log2);
-        hold_row<kParts, KS>(qf, row, top);
+        load_row<kParts, kVec, KS>(row, qp, a.qs[1], i, a.sq, a.d, a.scale_log2 / kLift);
+        if (kParts) track_row(top, row);
+        hold_row<kParts, KS>(qf, row);
         load_row<kParts, kVec, KS>(row, gp, a.os[1], i, a.sq, a.d, 1.0f);
         load_row<kParts, kVec, KS>(out, op, a.os[1], i, a.sq, a.d, 1.0f);
-        hold_row<kParts, KS>(gf, row, top);
 #pragma unroll
-        for (int x = 0; x < 2 * KS; ++x)
+        for (int x = 0; x < 2 * KS; ++x) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) delta = __builtin_fmaf(out[x][e], row[x][e], delta);
+            row[x] *= kLift;
+        }
+        hold_row<kParts, KS>(gf, row);
         delta = column_sum(delta);
 #pragma unroll
         for (int x = 0; x < DB; ++x) dq[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -694,8 +721,9 @@ __device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int 
     const float lse = lse_reference(lse_raw, kLog2e), inv_n = lse_row_factor(lse_raw);
     const float rest = masked_row_lse(lse_raw) ? 0.f : __builtin_fmaf(lse_raw, -kLog2e, lse);
     if (g == 0 && i < a.sq) a.delta[(int64_t)at.bh * a.sq + i] = delta;
-    kt.store(ks, t_lo * kTile, a.sk, a.d, top);
-    vt.store(vs, t_lo * kTile, a.sk, a.d, top);
+    delta *= kLift;
+    kt.template store<kParts, true>(ks, t_lo * kTile, a.sk, a.d, top);
+    vt.template store<kParts, true>(vs, t_lo * kTile, a.sk, a.d, top);
     __syncthreads();
 
     const int wq_last = min(wq0 + 15, a.sq - 1);
@@ -726,7 +754,7 @@ __device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int 
                     if (has_bias)
                         x += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
                     if (dropout) y = (bits >> (16 * h2 + 4 * r)) & 1u ? y * a.rng.inv_keep : 0.f;
-                    y -= delta;
+                    y = y * (1.0f / kLift) - delta;  // (dO v: kLift^2 times itself)
                     if (has_bias) y *= inv_n;  // (1 without a bias)
                     ds[h2][r] = exp2_of<kParts>(x - lse) * y;
                 }
@@ -743,9 +771,9 @@ __device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int 
         }
         if (t + 1 < t_hi) {
             if (!kParts) kt.load(kp, a.ks[1], (t + 1) * kTile, a.sk, a.d);
-            kt.store(ks + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d, top);
+            kt.template store<kParts, true>(ks + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d, top);
             if (!kParts) vt.load(vp, a.vs[1], (t + 1) * kTile, a.sk, a.d);
-            vt.store(vs + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d, top);
+            vt.template store<kParts, true>(vs + (slot ^ 1) * kElems, (t + 1) * kTile, a.sk, a.d, top);
         }
         __syncthreads();
     }
@@ -755,16 +783,17 @@ __device__ __forceinline__ bool dq_pass(const AttnArgs& a, const Place& at, int 
     }
     if (i >= a.sq) return true;
     if (a.n_split > 1) {
-        store_row<kParts, kVec>(dq, a.scale, a.part + (at.part_row0 + i) * a.d, a.d);
+        store_row<kParts, kVec>(dq, 1.0f / (kLift * kLift), a.scale, a.part + (at.part_row0 + i) * a.d, a.d);
         return true;
     }
     float* dqp = reinterpret_cast<float*>(a.dq) + at.b * a.dqs[0] + (int64_t)i * a.dqs[1] +
                  at.h * a.dqs[2];
-    store_row<kParts, kVec>(dq, a.scale, dqp, a.d);
+    store_row<kParts, kVec>(dq, 1.0f / (kLift * kLift), a.scale, dqp, a.d);
     return true;
 }
 template <int DB, int kMode, int kWaves>
-__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dq_kernel(const AttnArgs a_in) {
+__global__ __launch_bounds__(kWaves * 64, per_simd_bwd(DB, false)) void
+attn_f32_dq_kernel(const AttnArgs a_in) {
     constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves;
     AttnArgs a = a_in;
     constexpr bool kVec = kMode != kGeneral;
@@ -792,6 +821,7 @@ __device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int
                                          float* lds) {
     constexpr int kThreads = kWaves * 64, KS = kStepsOf<DB>;
     constexpr bool kVec = kMode != kGeneral;
+    constexpr float kLift = lift<kParts>;
     const bool has_bias = kVec ? (kMode & 1) != 0 : a.has_bias != 0;
     const bool dropout = kVec ? (kMode & 2) != 0 : a.dropout != 0;
     typedef Tile<DB, kVec, kTile, kThreads, kParts> tile_t;
@@ -824,24 +854,26 @@ __device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int
         }
     };
     auto publish = [&](int t, int slot) __attribute__((always_inline)) {
-        qt.store(qs + slot * kElems, t * kTile, a.sq, a.d, top);
-        gt.store(gs + slot * kElems, t * kTile, a.sq, a.d, top);
+        qt.template store<kParts, true>(qs + slot * kElems, t * kTile, a.sq, a.d, top);
+        gt.template store<kParts, true>(gs + slot * kElems, t * kTile, a.sq, a.d, top);
         if (thread_of<kParts>() < kTile) {
             const int x = thread_of<kParts>();
             float* r = rows + slot * 4 * kTile + ((x & 16) | (x & 3) << 2 | (x >> 2 & 3));
             const float lse = lse_reference(lse_r, kLog2e);
             r[0] = lse;
             r[kTile] = masked_row_lse(lse_r) ? 0.f : __builtin_fmaf(lse_r, -kLog2e, lse);
-            r[2 * kTile] = delta_r;
+            r[2 * kTile] = delta_r * (kLift * kLift * kLift);  // (as dO v p below)
             r[3 * kTile] = lse_row_factor(lse_r);
         }
     };
     {
         f32x4_t row[2 * KS];
-        load_row<kParts, kVec, KS>(row, kp, a.ks[1], j, a.sk, a.d, a.scale_log2);
-        hold_row<kParts, KS>(kf, row, top);
-        load_row<kParts, kVec, KS>(row, vp, a.vs[1], j, a.sk, a.d, 1.0f);
-        hold_row<kParts, KS>(vf, row, top);
+        load_row<kParts, kVec, KS>(row, kp, a.ks[1], j, a.sk, a.d, a.scale_log2 / kLift);
+        if (kParts) track_row(top, row);
+        hold_row<kParts, KS>(kf, row);
+        load_row<kParts, kVec, KS>(row, vp, a.vs[1], j, a.sk, a.d, kLift);
+        if (kParts) track_row(top, row);
+        hold_row<kParts, KS>(vf, row);
     }
 #pragma unroll
     for (int x = 0; x < DB; ++x) dk[x] = dv[x] = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -851,15 +883,26 @@ __device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int
     }
     __syncthreads();
 
+    // Above head_dim 64 the keep bits are drawn ahead of the next tile's requests, whose registers they would
+    // push out to memory (B2 S900 H8 D96 padded, p 0.1, forward and backward 262 -> 250 us, B2 S512 H8 D128 with
+    // a per-query mask and p 0.1 163 -> 147); below, the requests have the time of the drawing (B2 S777 H12 D64
+    // padded, p 0.1 269 against 291).
+    constexpr bool kDrawFirst = DB > 4;
+    auto draw = [&](int first) __attribute__((always_inline)) {
+        return keep_queries<kParts>(a, at.bh, first + row_g, wk0);
+    };
     const int wk_last = min(wk0 + 15, a.sk - 1);
+    const float kept = dropout ? a.rng.inv_keep * kLift : kLift;
     for (int t = t_lo; t < t_hi; ++t) {
         const int slot = (t - t_lo) & 1;
         const bf16_t *qb = qs + slot * kElems, *gb = gs + slot * kElems;
         const float* rb = rows + slot * 4 * kTile;
-        if (kParts && t + 1 < t_hi) request(t + 1);
         const int i0 = t * kTile;
         const bool active = wk0 < a.sk && (!a.causal || i0 + kTile - 1 >= wk0) &&
                             (a.window <= 0 || i0 - wk_last < a.window);
+        uint32_t drawn[2] = {0u, 0u};
+        if (kDrawFirst && dropout && active) drawn[0] = draw(i0), drawn[1] = draw(i0 + 16);
+        if (kParts && t + 1 < t_hi) request(t + 1);
         if (active) {
             const bool masked = i0 + kTile > a.sq || wk0 + 16 > a.sk ||
                                 (a.causal && i0 < wk0 + 15) ||
@@ -873,8 +916,8 @@ __device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int
                 const f32x4_t delta = *reinterpret_cast<const f32x4_t*>(rb + 2 * kTile + r0);
                 const f32x4_t s = dot_rows<DB, kPlane>(qb, 16 * h2, kf, rest);
                 const f32x4_t dp = dot_rows<DB, kPlane>(gb, 16 * h2, vf);
-                uint32_t bits = 0u;
-                if (dropout) bits = keep_queries<kParts>(a, at.bh, i0 + 16 * h2 + row_g, wk0);
+                uint32_t bits = drawn[h2];
+                if (!kDrawFirst && dropout) bits = draw(i0 + 16 * h2);
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int i = i0 + 16 * h2 + 4 * r + row_g;
@@ -883,7 +926,7 @@ __device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int
                         x += bias_at(a, at.b, at.h, min(i, a.sq - 1), min(j, a.sk - 1));
                     float p = exp2_of<kParts>(x - lse[r]);
                     if (has_bias) p *= rb[3 * kTile + r0 + r];  // (1 without a bias)
-                    const float keep = dropout ? ((bits >> r) & 1u ? a.rng.inv_keep : 0.f) : 1.f;
+                    const float keep = dropout && ((bits >> r) & 1u) == 0 ? 0.f : kept;
                     pd[h2][r] = p * keep;
                     ds[h2][r] = p * (dp[r] * keep - delta[r]);
                 }
@@ -910,23 +953,25 @@ __device__ __forceinline__ bool dkv_pass(const AttnArgs& a, const Place& at, int
         if (!everywhere<kWaves>(ok, reinterpret_cast<int*>(lds))) return false;
     }
     if (j >= a.sk) return true;
+    constexpr float kDownV = 1.0f / (kLift * kLift), kDownK = kDownV * kDownV;
     if (a.n_split > 1) {
         float* part = a.part + (at.part_row0 + j) * a.d;
-        store_row<kParts, kVec>(dk, a.scale, part, a.d);
-        store_row<kParts, kVec>(dv, 1.0f,
-                        part + (int64_t)a.n_split * a.batch * a.heads * a.sk * a.d, a.d);
+        store_row<kParts, kVec>(dk, kDownK, a.scale, part, a.d);
+        store_row<kParts, kVec>(dv, kDownV, 1.0f,
+                                part + (int64_t)a.n_split * a.batch * a.heads * a.sk * a.d, a.d);
         return true;
     }
     float* dkp = reinterpret_cast<float*>(a.dk) + at.b * a.dks[0] + (int64_t)j * a.dks[1] +
                  at.h * a.dks[2];
     float* dvp = reinterpret_cast<float*>(a.dv) + at.b * a.dvs[0] + (int64_t)j * a.dvs[1] +
                  at.h * a.dvs[2];
-    store_row<kParts, kVec>(dk, a.scale, dkp, a.d);
-    store_row<kParts, kVec>(dv, 1.0f, dvp, a.d);
+    store_row<kParts, kVec>(dk, kDownK, a.scale, dkp, a.d);
+    store_row<kParts, kVec>(dv, kDownV, 1.0f, dvp, a.d);
     return true;
 }
 template <int DB, int kMode, int kWaves>
-__global__ __launch_bounds__(kWaves * 64, 2) void attn_f32_dkv_kernel(const AttnArgs a_in) {
+__global__ __launch_bounds__(kWaves * 64, per_simd_bwd(DB, kMode >= 2)) void
+attn_f32_dkv_kernel(const AttnArgs a_in) {
     constexpr int kThreads = kWaves * 64, kRows = 16 * kWaves;
     AttnArgs a = a_in;
     constexpr bool kVec = kMode != kGeneral;

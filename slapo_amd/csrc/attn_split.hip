@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kThreads) void merge_fwd_kernel(const AttnArgs a) {
         for (int e = 0; e < n; ++e) out[e] = Elem<T>::from_f32(o[e] * inv);
     }
     if (c == 0) {
-        const float lse = kF32 ? __builtin_fmaf(m, kLn2, logf(l)) : (m + __builtin_log2f(l)) * kLn2;
+        const float lse = kF32 ? row_lse(m, l) : (m + __builtin_log2f(l)) * kLn2;
         a.lse[row] = m == -kFltMax ? l * kMaskedRowLse : lse;
     }
 }

@@ -868,6 +868,63 @@ def test_fp32_gradients_at_the_ends_of_the_range(head_dim):
         assert err <= 2e-5, (name, err)
 
 
+@pytest.mark.parametrize("shape,sk,causal,p", [
+    ((2, 70, 3, 64), 70, True, 0.1),
+    ((1, 130, 2, 80), 97, False, 0.0),
+    ((1, 257, 2, 128), 257, True, 0.0),
+    ((1, 63, 2, 30), 100, False, 0.3),
+    ((1, 640, 1, 24), 640, True, 0.0),
+    ((8, 530, 9, 64), 530, False, 0.0),
+])
+@pytest.mark.parametrize("mask", [False, True])
+def test_fp32_results_follow_powers_of_two(shape, sk, causal, p, mask):
+    """A power of two on a column of V, K, Q or dO, or on all of dO, is one on what depends on it and changes
+    no bit, down to the smallest normal numbers (2^-110 times numbers and results above 2^-16)."""
+    q, k, v, do, g = _inputs(*shape, torch.float32, sk=sk)
+    m = torch.randn(shape[0], 1, 1, sk, generator=g) if mask else None
+    q[..., 1] = k[..., 2] = 0.0  # (the scores stay as they are)
+    normal = lambda t: t.where(t.abs() >= 2.0 ** -16, torch.zeros_like(t))
+    q, k, v, do = (normal(t) for t in (q, k, v, do))
+    base = _run(q, k, v, do, m, causal, 0, p)
+    tiny = 2.0 ** -110
+    same = lambda a, r: torch.equal(normal(r), a.detach().where(r.abs() >= 2.0 ** -16, torch.zeros_like(r)))
+    v2, k2, q2, do2 = (t.clone() for t in (v, k, q, do))
+    v2[..., 0] *= tiny
+    k2[..., 1] *= tiny
+    q2[..., 2] *= tiny
+    do2[..., 3] *= tiny
+    out = _run(q, k, v2, do, m, causal, 0, p)[0].detach().clone()
+    out[..., 0] /= tiny
+    assert same(out, base[0].detach())
+    for pos, col, got in ((1, 1, _run(q, k2, v, do, m, causal, 0, p)),
+                          (2, 2, _run(q2, k, v, do, m, causal, 0, p)),
+                          (3, 3, _run(q, k, v, do2, m, causal, 0, p))):
+        got = got[pos].clone()
+        got[..., col] /= tiny
+        assert same(got, base[pos]), pos
+    tiny = 2.0 ** -100  # (the first sums of delta, of two small factors, stay normal too)
+    for scaled in ((v, do * tiny), (v * tiny, do)):
+        got = _run(q, k, *scaled, m, causal, 0, p)
+        for a, r in zip(got[1:3], base[1:3]):
+            assert same(a / tiny, r)
+
+
+def test_fp32_probabilities_near_the_smallest_number():
+    """A key that every row gives 2^-124: what it adds, where nothing else adds anything, and its own
+    gradients.  Bar: the rounding of an exponent of 124 (3 ulp of 2^-18, 2^-17 ln 2 each) and fp32 sums."""
+    q, k, v, do, _ = _inputs(1, 40, 2, 64, torch.float32, sk=8)
+    q, k = q * 0.1, k * 0.1
+    m = torch.zeros(1, 1, 1, 8)
+    m[..., 5] = -84.0
+    v[:, :5, :, 0] = v[:, 6:, :, 0] = 0.0
+    out, dq, dk, dv = _run(q, k, v, do, m, False)
+    ro, rq, rk, rv = OA.attention_fwd_bwd(q, k, v, do, m, False, 0, 0.0, None, None, torch.float64)
+    for a, r in ((out[..., 0], ro[..., 0]), (dk[:, 5], rk[:, 5]), (dv[:, 5], rv[:, 5])):
+        assert r.abs().max().item() < 1e-35
+        a = a.detach().cpu().double()
+        assert ((a - r).norm() / r.norm()).item() <= 2e-5
+
+
 @pytest.mark.parametrize("mask", ["none", "key", "square"])
 @pytest.mark.parametrize("shape,sk,causal,window,p", [
     ((2, 70, 3, 64), 70, True, 0, 0.1),
