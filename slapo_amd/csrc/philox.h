@@ -233,11 +233,21 @@ SLAPO_HD uint32_t dropout_keep_any(const DropoutState& s, uint64_t elem, int n) 
 
 // Keep-bits of the kN (a multiple of four, at most 32) consecutive elements starting at elem (bit j <->
 // element elem + j), for any launch geometry and alignment.  The split of the element index, a division
-// where the thread count is no power of two, is taken once.  At vec 4 kN / 4 + 1 blocks are drawn
-// (kAligned, elem % 4 == 0: one fewer), at vec 2 kN / 2 + 1, at vec 1 kN.
+// where the thread count is no power of two, is taken once (at vec 8 and 16 per block).  From vec 4 on
+// kN / 4 + 1 blocks are drawn (kAligned, elem % 4 == 0: one fewer), at vec 2 kN / 2 + 1, at vec 1 kN.
 template <int kN, bool kAligned = false>
 SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem) {
-    if (s.vec > 4) return dropout_keep_any(s, elem, kN);
+    constexpr int kBlocks = kN / 4 + (kAligned ? 0 : 1);
+    constexpr uint32_t kMask = kN == 32 ? ~0u : (1u << (kN & 31)) - 1u;
+    if (s.vec > 4) {  // (plans of one- and two-byte tensors: C ABI callers only)
+        uint64_t all = 0;
+#if defined(__HIPCC__)
+#pragma unroll 1
+#endif
+        for (int blk = 0; blk < kBlocks; ++blk)
+            all |= (uint64_t)dropout_keep4(s, (elem >> 2) + (uint64_t)blk) << (4 * blk);
+        return (uint32_t)(all >> (kAligned ? 0 : elem & 3u)) & kMask;
+    }
     const uint32_t shift = s.vec == 4 ? 2u : s.vec == 2 ? 1u : 0u;
     const uint64_t v = elem >> shift;
     uint64_t thread, trip;
@@ -247,7 +257,6 @@ SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem) {
     } else {
         split_by_threads(s, v, thread, trip);
     }
-    constexpr int kBlocks = kN / 4 + (kAligned ? 0 : 1);
     bool one_call = philox_call_fits(s) && thread + kBlocks <= s.total_threads;
 #if defined(__HIP_DEVICE_COMPILE__)
     one_call = __builtin_amdgcn_ballot_w64(!one_call) == 0;
@@ -279,7 +288,7 @@ SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem) {
         }
         all = run;
     }
-    return (uint32_t)all & (kN == 32 ? ~0u : (1u << (kN & 31)) - 1u);
+    return (uint32_t)all & kMask;
 }
 
 }  // namespace slapo

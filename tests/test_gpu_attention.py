@@ -368,6 +368,25 @@ def test_dropout_keep_bits_saved_by_the_forward(dtype, shape, causal, window, ma
                 assert torch.equal(got[bi * h + hi][sel], keep[bi * h + hi][sel])
 
 
+@pytest.mark.parametrize("elem_bytes", [1, 2])
+@pytest.mark.parametrize("h,sk", [(4, 512), (4, 498), (2, 500)])
+def test_keep_bits_drawn_ahead_under_wide_plans(elem_bytes, h, sk):
+    """The plan of a one- or two-byte tensor (a C ABI caller's): keep bits drawn ahead of a windowed
+    forward, or of a length that is no multiple of four, are those of the mask generator."""
+    from slapo_amd.op import _kernels as K
+
+    b, sq, d, p, window = 1, 320, 64, 0.3, 100
+    q, k, v, _, _ = (t if i == 4 else t.cuda()
+                     for i, t in enumerate(_inputs(b, sq, h, d, torch.bfloat16, sk=sk)))
+    plan = K.dropout_plan(b * h * sq * sk, elem_bytes, q.device)
+    assert plan.vec > 4
+    o = K.attn_fwd(q, k, v, None, True, window, d ** -0.5, p, 77, 8, plan, save_mask=True)[0]
+    keep = K.dropout_mask(plan.numel, elem_bytes, p, 77, 8, q.device).view(b * h, sq, sk).bool()
+    ref = OA.xformers_ref(q.cpu(), k.cpu(), v.cpu(), None, True, window, p, keep.cpu(),
+                          compute_dtype=torch.float64)
+    assert_parity(o, ref, torch.bfloat16)
+
+
 def test_strided_views_of_fused_qkv_are_read_in_place():
     b, s, h, d = 2, 160, 4, 64
     g = torch.Generator().manual_seed(1)

@@ -60,13 +60,49 @@ int main() {
 """
 
 
+def _compile_and_run(tmp_path, text):
+    source = tmp_path / "philox.cpp"
+    source.write_text(text)
+    exe = tmp_path / "philox"
+    subprocess.run(["g++", "-O2", "-std=c++17", str(source), "-o", str(exe)], check=True, timeout=120)
+    return subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+
+
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
 def test_runs_and_shared_rounds_equal_the_single_elements(tmp_path):
     """Runs of keep bits for every vec, thread count, alignment and wrap; blocks whose first rounds are
     shared by a call."""
-    source = tmp_path / "philox.cpp"
-    source.write_text(SOURCE % HEADER)
-    exe = tmp_path / "philox"
-    subprocess.run(["g++", "-O2", "-std=c++17", str(source), "-o", str(exe)], check=True, timeout=120)
-    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    out = _compile_and_run(tmp_path, SOURCE % HEADER)
     assert out.returncode == 0 and out.stdout.strip() == "0", out.stdout + out.stderr
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs a host compiler")
+@pytest.mark.parametrize("vec", [8, 16])
+@pytest.mark.parametrize("threads", [524288, 256 * 7])
+def test_wide_plans_draw_a_block_per_four_elements(tmp_path, vec, threads):
+    """A run of 32 elements under the plan of a one- or two-byte tensor: eight blocks, nine where it
+    does not start at a multiple of four."""
+    with open(HEADER, encoding="utf-8") as f:
+        header = f.read()
+    start = "uint32_t k1) {\n#pragma unroll\n"  # of philox4x32_10
+    assert header.count(start) == 1
+    counted = tmp_path / "philox_counted.h"
+    counted.write_text(header.replace("SLAPO_HD u32x4 philox4x32_10(",
+                                      "static int blocks;\nSLAPO_HD u32x4 philox4x32_10(")
+                       .replace(start, "uint32_t k1) {\n++blocks;\n"))
+    out = _compile_and_run(tmp_path, f"""
+#include "{counted}"
+#include <cstdio>
+using namespace slapo;
+int main() {{
+    DropoutState s{{}};
+    s.total_threads = {threads}, s.vec = {vec}, s.calls_per_iter = {vec // 4};
+    s.keep_max = 3865470566u, s.t_shift = {threads.bit_length() - 1 if threads == 524288 else -1};
+    s.g_shift = {1 if vec == 8 else 2};
+    dropout_keep_run<32, true>(s, 1024);
+    const int aligned = blocks;
+    dropout_keep_run<32, false>(s, 1023);
+    std::printf("%d %d\\n", aligned, blocks - aligned);
+}}
+""")
+    assert out.stdout.split() == ["8", "9"], out.stdout + out.stderr
