@@ -37,8 +37,8 @@ namespace {
 // whole words of every 64-key tile that some query of a 32-query group sees, but a bit that
 // belongs to a pair outside the row's own mask meets a probability of zero, so what such words
 // hold does not matter and they are left as they are.  With a local window the word columns count
-// from the first word of the row's window (window / 32 + 1 of them, not seqlen_k / 32: every thread
-// then has a word to draw); without one they are the words themselves.
+// from the first word of the row's window (under a causal mask window / 32 + 2 of them, not seqlen_k /
+// 32: every thread then has a word to draw); without one they are the words themselves.
 // kExact: any launch geometry of the dropout plan and any seqlen_k (dropout_keep_run).  Drawn per
 // word this costs 9 Philox blocks per 32 scores where the forward kernel, whose lanes hold single
 // groups of four, drew one block per score: bf16 B3 S777 H12 D64 without a causal mask, p 0.1,
@@ -90,8 +90,10 @@ bool keep_mask_kernel_fits(const AttnArgs& a) {
 int draw_keep_mask(const AttnArgs& a, hipStream_t st) {
     const int64_t bh = (int64_t)a.batch * a.heads;
     if (!keep_mask_kernel_fits(a)) return SLAPO_ERR_SHAPE;
-    // with a window: the words of a row's own window (it spans window / 32 + 1 words at most)
-    const int words = a.window > 0 ? min(a.mask_words, a.window / 32 + 2) : a.mask_words;
+    // with a window: the words of a row's own window (it spans window / 32 + 1 words at most), and where
+    // nothing hides the keys behind the query, those as well
+    const int words =
+        a.window > 0 && a.causal ? min(a.mask_words, a.window / 32 + 2) : a.mask_words;
     const int units = (a.sq + 63) / 64 * words;
     const dim3 grid((unsigned)((units + 3) / 4), (unsigned)bh);
     if (a.dropout == 1)

@@ -387,6 +387,16 @@ def test_keep_bits_drawn_ahead_under_wide_plans(elem_bytes, h, sk):
     assert_parity(o, ref, torch.bfloat16)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,sk,window", [((2, 320, 2, 64), 320, 100), ((1, 200, 3, 80), 333, 40),
+                                             ((1, 300, 2, 128), 290, 33)])
+def test_dropout_with_a_window_that_leaves_later_keys_visible(dtype, shape, sk, window):
+    """A window without a causal mask bounds the keys before a query, not those behind it: the keep bits
+    of all of these are drawn."""
+    q, k, v, do, _ = _inputs(*shape, dtype, sk=sk)
+    _check(q, k, v, do, None, False, window, dtype, p=0.2)
+
+
 def test_strided_views_of_fused_qkv_are_read_in_place():
     b, s, h, d = 2, 160, 4, 64
     g = torch.Generator().manual_seed(1)
