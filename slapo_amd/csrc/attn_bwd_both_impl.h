@@ -12,7 +12,8 @@ namespace slapo {
 namespace bwd_both {
 
 // delta of every row, times the factor that the dK / dV kernel wants on it (lse_row_factor), in the order
-// of dq_block's own sum, so that both give the same bits: two lanes a row, lane g on columns 16 t + 8 g.
+// of dq_block's own sum, so that both give the same bits (rows that saw only masked keys aside: dq_block
+// divides their factor out again, equal within a rounding): two lanes a row, lane g on columns 16 t + 8 g.
 // Heads are the fastest index, as in memory.  Bound by reading dO and O once.
 template <typename T, int kSteps, bool kBias>
 __global__ __launch_bounds__(256) void delta_kernel(const AttnArgs a, int64_t n_rows) {

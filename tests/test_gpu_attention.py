@@ -609,6 +609,82 @@ def test_backward_in_one_launch_equals_the_two_kernels(shape, sk, causal, window
         assert torch.equal(a, r)
 
 
+@pytest.mark.parametrize("mask", ["none", "key", "hidden", "square"])
+@pytest.mark.parametrize("shape,sk,causal,window", [
+    ((2, 130, 3, 64), 130, True, 0),
+    ((1, 257, 5, 32), 257, False, 0),
+    ((2, 65, 3, 80), 300, False, 0),
+    ((1, 300, 3, 96), 66, False, 0),
+    ((3, 200, 2, 128), 200, True, 70),
+])
+def test_backward_in_one_launch_with_stored_keep_bits(shape, sk, causal, window, mask):
+    """The builds with stored keep bits: slapo_amd_attn_bwd_ex on a small call, and on as many copies of
+    it (with copies of its bits) as make it run the two kernels."""
+    import ctypes
+
+    from slapo_amd import _lib
+    from slapo_amd.op import _kernels as K
+
+    lib = _lib.load()
+    b, s, h, d = shape
+    q, k, v, do, g = _inputs(b, s, h, d, torch.bfloat16, sk=sk)
+    q, k, v, do = (t.cuda() for t in (q, k, v, do))
+    m = None
+    if mask != "none":
+        m = torch.randn(b, 1, s if mask == "square" else 1, sk, generator=g)
+        if mask == "square":
+            m[:, :, s // 2] = torch.finfo(torch.float32).min
+        if mask == "hidden":
+            m[0] = torch.finfo(torch.float32).min
+        m = m.cuda()
+    bias = None if m is None else m.expand(b, h, s, sk)
+    p, plan = 0.2, K.dropout_plan(b * h * s * sk, 4, q.device)
+    o, lse, _, bits = K.attn_fwd(q, k, v, bias, causal, window, d ** -0.5, p, 5, 0, plan,
+                                 save_mask=True)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    P = lambda t: ctypes.c_void_p(t.data_ptr() if t is not None else None)
+
+    def backward(n):
+        rep = lambda t: t.repeat(n, *[1] * (t.ndim - 1))
+        qn, kn, vn, dn, on, ln = (rep(t) for t in (q, k, v, do, o, lse))
+        mn, kind, strides = None, _lib.SLAPO_F32, None
+        if m is not None:
+            mn = rep(m)
+            strides = mn.expand(n * b, h, s, sk).stride()
+        if mask == "square":
+            pitch = -(-sk // 64) * 64
+            plane = -(-s // 64) * 64 * pitch
+            rows = torch.empty(n * b * plane, device="cuda")
+            assert lib.slapo_amd_attn_prepare_bias(
+                P(mn), kind, (ctypes.c_int64 * 4)(*strides), n * b, 1, s, sk, P(rows), st) == 0
+            mn, kind, strides = rows, 3, (plane, 0, pitch, 1)  # SLAPO_BIAS_PREPARED
+        prm = K.make_attn_params(qn, kn, vn, on, None, causal, window, d ** -0.5, p, 5, 0,
+                                 K.dropout_plan(n * b * h * s * sk, 4, q.device))
+        if strides is not None:
+            prm.bias_strides = (ctypes.c_int64 * 4)(*strides)
+        kept = bits.repeat(n)
+        prm.keep_mask = kept.data_ptr()
+        grads = [torch.empty_like(t) for t in (qn, kn, vn)]
+        nbytes = lib.slapo_amd_attn_bwd_workspace_bytes(ctypes.byref(prm))  # (no room to deal tiles)
+        ws = torch.empty(nbytes // 4, device="cuda")
+        assert lib.slapo_amd_attn_bwd_ex(
+            ctypes.byref(prm), P(qn), P(kn), P(vn), P(mn), kind, P(on), P(dn), P(ln), *map(P, grads),
+            *map(K._bshd_strides, grads), P(ws), nbytes, st) == 0
+        torch.cuda.synchronize()
+        return [t[:b] for t in grads]
+
+    one = backward(1)
+    two = backward(-(-1024 // (b * h * (-(-s // 128) + -(-sk // 128)))))
+    for a, r in zip(one, two):
+        assert torch.equal(a, r)
+    # and they are the gradients of that mask
+    keep = K.dropout_mask(plan.numel, 4, p, 5, 0, q.device).view(b * h, s, sk).bool().cpu()
+    ref = OA.attention_fwd_bwd(q.cpu(), k.cpu(), v.cpu(), do.cpu(), None if m is None else m.cpu(),
+                               causal, window, p, keep, None, torch.float64)
+    for a, r in zip(one, ref[1:]):
+        assert_parity(a, r, torch.bfloat16)
+
+
 @pytest.mark.parametrize("mask", ["none", "key", "square"])
 @pytest.mark.parametrize("shape,causal,window,p", [
     ((2, 450, 3, 64), True, 0, 0.0),     # wavefronts past the last row and key in full tiles
