@@ -17,8 +17,8 @@ other_attention  forward and backward time of the OPT-2.7B-shaped (padding mask)
           GPT-Neo-1.3B-shaped (global / window 256, dropout 0.1) attention calls, bf16
 bert_large_fp32  BASELINE configuration 1, which is DEFINED as the native CPU path: the oracle's
           fp32 forward of B 4, S 512, 16 x 64 on the host cores, and beside it the fp32 kernel
-          of this library on the same tensors (on bf16 matrix instructions, six products for one)
-          against the fp32 vector peak (reported, not a target)
+          of this library on the same tensors against the peak of what it runs on: bf16 matrix
+          instructions, six products for one (reported, not a target)
 cpu_baseline  the oracle's native-PyTorch restatement (fp32 CPU, autograd backward) timed on the
           host cores on a bounded sample of the same workload; every epilogue / other_attention
           entry carries a cpu_baseline of its own (a bounded chunk of its tensors)
@@ -46,12 +46,12 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 / bf16
-FP32_VECTOR_PEAK_TFLOPS = 157.3
+FP32_PEAK_TFLOPS = MFMA_PEAK_TFLOPS / 6  # an fp32 product is six bf16 ones (csrc/attn_f32.hip)
 # HBM bytes per launch of the dK/dV kernel on WORKLOAD, from rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (KiB per dispatch), each scaled by the same counter's reading for a 256 MiB copy
 # (FETCH_SIZE reads half the copied bytes: factor 2.0; WRITE_SIZE factor 1.0):
-# (43.93e3 * 2.0 + 32.77e3) KiB = 123.5 MB against 101.7 MB algorithmic.  Summary under profiles/.
-DKDV_TRAFFIC_BYTES = (43.46e3 * 2.0 + 32.77e3) * 1024
+# (43.39e3 * 2.0 + 32.77e3) KiB = 122.4 MB against 101.7 MB algorithmic.  Summary under profiles/.
+DKDV_TRAFFIC_BYTES = (43.39e3 * 2.0 + 32.77e3) * 1024
 HBM_PEAK_GBS = 8000.0      # MI355X HBM3E
 
 WORKLOAD = dict(name="gpt2-medium causal attention fwd+bwd", dtype="fp16", batch=8, seq=1024,
@@ -441,9 +441,8 @@ def bench_bert_large_fp32(device, iters=10):
             "cpu": {"ms": cpu_sec * 1e3, "TFLOPs": flops / cpu_sec / 1e12, "cores": threads,
                     "kind": "port", "sample": "the whole configuration, median of 3"},
             "gpu_fp32_kernel": {"ms": gpu_sec * 1e3, "TFLOPs": flops / gpu_sec / 1e12,
-                                "peak": FP32_VECTOR_PEAK_TFLOPS,
-                                "frac_of_fp32_vector_peak":
-                                    flops / gpu_sec / 1e12 / FP32_VECTOR_PEAK_TFLOPS,
+                                "peak": FP32_PEAK_TFLOPS,
+                                "frac_of_peak": flops / gpu_sec / 1e12 / FP32_PEAK_TFLOPS,
                                 "note": "parity kernel (1e-5 bar), not a performance target"}}
 
 
