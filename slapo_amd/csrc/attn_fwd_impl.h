@@ -38,7 +38,7 @@ constexpr float kMaxSlack = 8.0f;  // hysteresis of the softmax reference, log2 
 constexpr int fwd_per_cu(int dpad) { return dpad <= 32 ? 4 : dpad <= 64 ? 3 : 2; }
 // At 64 without bias and dropout four fit in 128 registers, which pays where the launch fills them: from the
 // first workgroup that three a CU would not hold on (fp16 B8 S1024 H16 D64 causal, 1024 workgroups:
-// 30.9 -> 29.8 us, bf16 B2 S4096 H16 D64 causal 88.4 -> 83.5; bf16 B1 S8192 H8 D64, 512: 167 -> 169).
+// 30.8 -> 29.5 us, bf16 B2 S4096 H16 D64 causal 88.5 -> 83.1; bf16 B1 S8192 H8 D64, 512: 167 -> 169).
 constexpr int kFwdFour = 4;
 
 template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu>
