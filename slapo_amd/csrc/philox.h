@@ -233,23 +233,11 @@ SLAPO_HD uint32_t dropout_keep_any(const DropoutState& s, uint64_t elem, int n) 
 
 // Keep-bits of the kN (a multiple of four, at most 32) consecutive elements starting at elem (bit j <->
 // element elem + j), for any launch geometry and alignment.  The split of the element index, a division
-// where the thread count is no power of two, is taken once (at vec 8 and 16 per block).  From vec 4 on
-// kN / 4 + 1 blocks are drawn (kAligned, elem % 4 == 0: one fewer), at vec 2 kN / 2 + 1, at vec 1 kN.
+// where the thread count is no power of two, is taken once.  From vec 4 on kN / 4 + 1 blocks are drawn
+// (kAligned, elem % 4 == 0: one fewer), at vec 2 kN / 2 + 1, at vec 1 kN.
 template <int kN, bool kAligned = false>
 SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem) {
-    constexpr int kBlocks = kN / 4 + (kAligned ? 0 : 1);
-    constexpr uint32_t kMask = kN == 32 ? ~0u : (1u << (kN & 31)) - 1u;
-    if (s.vec > 4) {  // (plans of one- and two-byte tensors: C ABI callers only)
-        uint64_t all = 0;
-#if defined(__HIPCC__)
-#pragma unroll 1
-#endif
-        for (int blk = 0; blk < kBlocks; ++blk)
-            all |= (uint64_t)dropout_keep4(s, (elem >> 2) + (uint64_t)blk) << (4 * blk);
-        return (uint32_t)(all >> (kAligned ? 0 : elem & 3u)) & kMask;
-    }
-    const uint32_t shift = s.vec == 4 ? 2u : s.vec == 2 ? 1u : 0u;
-    const uint64_t v = elem >> shift;
+    const uint64_t v = elem >> __builtin_ctz(s.vec);
     uint64_t thread, trip;
     if (((v | s.total_threads) >> 32) == 0 && s.t_shift < 0) {
         trip = (uint32_t)v / (uint32_t)s.total_threads;
@@ -257,6 +245,7 @@ SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem) {
     } else {
         split_by_threads(s, v, thread, trip);
     }
+    constexpr int kBlocks = kN / 4 + (kAligned ? 0 : 1);
     bool one_call = philox_call_fits(s) && thread + kBlocks <= s.total_threads;
 #if defined(__HIP_DEVICE_COMPILE__)
     one_call = __builtin_amdgcn_ballot_w64(!one_call) == 0;
@@ -272,23 +261,27 @@ SLAPO_HD uint32_t dropout_keep_run(const DropoutState& s, uint64_t elem) {
         for (int blk = kN / 4 - 1; blk >= 0; --blk)
             bits = push_keep4(bits, philox_block(call, t + blk), s.keep_max);
         all = (((uint64_t)last << kN) | bits) >> (kAligned ? 0 : elem & 3u);
-    } else {  // fewer words a block, or a run that wraps to the next call
-        const int skip = (int)(elem & ((1u << shift) - 1u));  // elements of the first block before elem
-        uint32_t run = 0;
+    } else {  // other words a block or blocks a trip, or a run that wraps to the next call
+        const int step = s.vec < 4 ? (int)s.vec : 4;  // elements a block serves
+        const int skip = (int)elem & (step - 1);      // ... of the first one before elem
+        uint32_t sub = (uint32_t)(elem >> 2) & (s.calls_per_iter - 1u), run = 0;
 #if defined(__HIPCC__)
 #pragma unroll 1
 #endif
-        for (int at = -skip; at < kN; at += 1 << shift) {
-            const u32x4 r = philox_block(s, thread, shift ? trip : trip >> 2);
+        for (int at = -skip; at < kN; at += step) {
+            const u32x4 r =
+                philox_block(s, thread, s.vec == 1 ? trip >> 2 : trip * s.calls_per_iter + sub);
             uint32_t four = s.keep_none ? 0u : push_keep4(0u, r, s.keep_max);
-            if (shift == 0) four = (four >> (trip & 3)) & 1u;
-            if (shift == 1) four &= 3u;
+            if (step == 1) four = (four >> (trip & 3)) & 1u;
+            if (step == 2) four &= 3u;
             run |= at < 0 ? four >> -at : four << at;
+            if (++sub < s.calls_per_iter) continue;
+            sub = 0;
             if (++thread == s.total_threads) thread = 0, ++trip;
         }
         all = run;
     }
-    return (uint32_t)all & kMask;
+    return (uint32_t)all & (kN == 32 ? ~0u : (1u << (kN & 31)) - 1u);
 }
 
 }  // namespace slapo
