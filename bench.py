@@ -670,7 +670,7 @@ def main():
                    "heads": cfg["heads"], "head_dim": cfg["head_dim"], "causal": cfg["causal"],
                    "dropout_p": cfg["p"], "flops_per_step": 14 * d * n_pairs},
         "frac_of_mfma_peak": value / MFMA_PEAK_TFLOPS,
-        "roofline": {"bound": "mfma", "kernel": "attn_bwd_kernel<f16,64,0,0,1,4,2> (dK/dV)",
+        "roofline": {"bound": "mfma", "kernel": "attn_bwd_kernel<f16,64,0,0,1,4,2,0> (dK/dV)",
                      "achieved": achieved,
                      "peak": MFMA_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / MFMA_PEAK_TFLOPS, "traffic": DKDV_TRAFFIC_BYTES,
@@ -680,7 +680,7 @@ def main():
                           "sum_of_kernels_ms": sum(seg_ms)},
     }
     result["kernels"] = [kern("attn_fwd_kernel<f16,64,0,0,4,4>", 4 * d * n_pairs, seg_ms[0]),
-                         kern("attn_bwd_kernel<f16,64,0,0,1,4,2> (dK/dV)", bwd_flops, seg_ms[2]),
+                         kern("attn_bwd_kernel<f16,64,0,0,1,4,2,0> (dK/dV)", bwd_flops, seg_ms[2]),
                          kern("attn_bwd_dq_kernel<f16,64,0,0,4>", 6 * d * n_pairs, seg_ms[1])]
     with_cpu = not args.no_cpu_baseline
     if not args.no_epilogues:

@@ -50,7 +50,7 @@ __global__ __launch_bounds__(256, bwd::bwd_per_cu(DPAD)) void attn_bwd_both_kern
     const AttnArgs dkv, const AttnArgs dq, int n_dkv) {
     const int block = (int)blockIdx.x;
     if (block < n_dkv)
-        bwd::dkv_block<T, DPAD, kBias, kDrop, 1, kSteps, bwd::bwd_per_cu(DPAD)>(dkv, block, n_dkv);
+        bwd::dkv_block<T, DPAD, kBias, kDrop, 1, kSteps, bwd::bwd_per_cu(DPAD), false>(dkv, block, n_dkv);
     else
         bwd_dq::dq_block<T, DPAD, kBias, kDrop, kSteps, false>(dq, block - n_dkv,
                                                                (int)gridDim.x - n_dkv);
@@ -63,7 +63,7 @@ int launch(const AttnArgs& a, hipStream_t st) {
     const int64_t n_rows = n_bh * a.sq;
     const int64_t delta_blocks = (n_rows * 2 + 255) / 256;
     if (n_dkv + n_dq > 0x7FFFFFFF || delta_blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    const size_t lds_dkv = bwd::BwdSmem<T, DPAD>::kBytes, lds_dq = bwd_dq::lds_bytes<T, DPAD, kBias>();
+    const size_t lds_dkv = bwd::BwdSmem<T, DPAD, false>::kBytes, lds_dq = bwd_dq::lds_bytes<T, DPAD, kBias>();
     const size_t smem = lds_dkv > lds_dq ? lds_dkv : lds_dq;
     auto kern = attn_bwd_both_kernel<T, DPAD, kBias, kDrop, kSteps>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device

@@ -1,7 +1,7 @@
 // Flash-attention backward, dK / dV half, for gfx950 (fp16 / bf16 inputs, fp32 accumulation).
 //
-// One workgroup (4 wavefronts) owns 128 consecutive keys of one (batch, head); wavefront w owns
-// 32 of them and keeps their K and V fragments in registers for the whole kernel, together with
+// One workgroup (4 wavefronts; 8 with kPair, see BwdSmem) owns 128 consecutive keys of one (batch,
+// head); wavefront w owns 32 of them and keeps their K and V fragments in registers for the whole kernel, together with
 // its dK^T and dV^T accumulators.  Query tiles of 64 rows (Q, dO, lse, delta) stream through LDS,
 // double buffered and staged through registers.  Per 32-query half tile and wavefront (lane l,
 // g = l / 32):
@@ -31,23 +31,39 @@
 namespace slapo {
 namespace bwd {
 
-constexpr int kBwdWaves = 4;
-constexpr int kBwdThreads = kBwdWaves * 64;
-constexpr int kBwdBM = 64;  // queries per tile
+constexpr int kBwdBM = 64;       // queries per tile
+constexpr int kBwdKeys = 128;    // keys per workgroup
+constexpr int kKeyBlocks = kBwdKeys / 32;
 
-template <typename T, int DPAD>
+// kPair (head_dim 97-128 in a launch of its own): two wavefronts per 32 keys, eight a workgroup.  There the
+// K and V fragments and both accumulators of a wavefront are 192 registers, which leaves room for one
+// wavefront per SIMD, and nothing runs beside its waits; a pair needs 250 each, so two fit.  Both hold the
+// fragments; either accumulates one of dV and dK (64 registers instead of 128) and computes one half of
+// every query tile, so no product is done twice; what crosses LDS are 16-bit words that a wavefront on its
+// own would have kept (2 KB written and read per half tile beside 32 KB of operands).
+// Forward and backward, before -> after: bf16 B1 S16384 H16 D128 causal 4.65 -> 4.49 ms (the matrix pipe
+// busy 41 -> 50 % of dK/dV), B4 S2048 H16 causal 361 -> 351 us, window 256 with p 0.1 222 -> 216, B2 S1024
+// with a [B,1,Sq,Sk] mask 169.7 -> 163.2.  (The two roles as one body with selects in place of two bodies:
+// window 217, long 4.48 -> 4.55; each wavefront adding its own half first, which gives other bits than
+// the one-launch backward: 1 % less.)
+template <typename T, int DPAD, bool kPair>
 struct BwdSmem {
-    typedef TileStage<T, DPAD, kBwdBM, kBwdThreads> QStage;
+    static constexpr int kThreads = (kPair ? 2 : 1) * kKeyBlocks * 64;
+    typedef TileStage<T, DPAD, kBwdBM, kThreads> QStage;
     static constexpr int kPitch = QStage::kPitch;
-    static constexpr int kQTile = kBwdBM * kPitch;            // elements
-    static constexpr size_t kQBytes = 2 * kQTile * sizeof(T);   // double buffered
-    static constexpr size_t kStatBytes = 2 * 2 * kBwdBM * sizeof(float);  // lse, delta; x2 buffers
-    // dropout keep bits of a query tile: one word per wavefront (32 keys) and query; x2 buffers
-    static constexpr size_t kMaskBytes = 2 * kBwdWaves * kBwdBM * sizeof(uint32_t);
-    static constexpr size_t kBytes = 2 * kQBytes + kStatBytes + kMaskBytes;
+    static constexpr int kBufs = kPair ? 3 : 2;
+    static constexpr int kQTile = kBwdBM * kPitch;                // elements
+    static constexpr size_t kQBytes = kBufs * kQTile * sizeof(T);
+    static constexpr size_t kStatBytes = kBufs * 2 * kBwdBM * sizeof(float);  // lse, delta
+    // dropout keep bits of a query tile: one word per 32 keys and query
+    static constexpr size_t kMaskBytes = kBufs * kKeyBlocks * kBwdBM * sizeof(uint32_t);
+    // kPair: the 32 x 32 words of P or dS that a wavefront hands to its partner, two tiles deep
+    static constexpr size_t kHandBlock = 32 * 32 * sizeof(T);
+    static constexpr size_t kHandBytes = kPair ? 2 * 2 * kKeyBlocks * kHandBlock : 0;
+    static constexpr size_t kBytes = 2 * kQBytes + kStatBytes + kMaskBytes + kHandBytes;
 };
 
-// Workgroups per CU: three up to DPAD 32, two up to 96, one at 128 (192 resident accumulator / fragment registers).  At
+// Workgroups per CU: three up to DPAD 32, two up to 96, one at 128.  At
 // 96 with the forward's keep bits both are built: two where a call has more key blocks than CUs
 // (fp16 B5 S920 H31 D80 window 356, p 0.1, forward and backward 256 -> 226 us; bf16 B4 S2048 H12 D96
 // causal, p 0.1 322 -> 292), else one, whose staggered body is the faster of the two (fp16 B2 S1600 H8
@@ -59,20 +75,22 @@ constexpr int bwd_per_cu(int dpad) { return dpad <= 32 ? 3 : dpad <= 96 ? 2 : 1;
 // instruction (every Q / dO fragment read feeds two MFMAs) at the price of twice the resident
 // fragments and accumulators, i.e. one wavefront per SIMD instead of two.
 // Workgroup `block` of `n_blocks`.
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu, bool kPair>
 __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     static_assert(kDrop != 3 || KB == 1, "the keep-bit tile holds one word per wavefront and query");
     typedef typename Mma<T>::frag frag_t;
-    typedef BwdSmem<T, DPAD> SM;
+    static_assert(!kPair || KB == 1, "two wavefronts per 32 keys");
+    typedef BwdSmem<T, DPAD, kPair> SM;
     typedef typename SM::QStage QStage;
+    constexpr int kThreads = SM::kThreads;
     constexpr int kPitch = SM::kPitch;
     // k-steps over the head dimension: DPAD / 16, or one fewer where the launcher guarantees
     // head_dim <= 16 * kSteps (head_dim 80 in the 96-wide build)
     constexpr int DK = kSteps;
     constexpr int DV = DPAD / 32;          // 32-row blocks of dK^T / dV^T
     constexpr int kWaveKeys = 32 * KB;
-    constexpr int kBN = kBwdWaves * kWaveKeys;  // keys per workgroup
+    constexpr int kBN = kKeyBlocks * kWaveKeys;  // keys per workgroup
 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     T* q_lds = reinterpret_cast<T*>(smem_raw);
@@ -94,7 +112,9 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     const int k0 = kt * kBN;
 
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wavefront-uniform
+    // wavefront-uniform: the 32 keys and, of a pair, the half of every query tile that it computes
+    const int wave_id = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = kPair ? wave_id & (kKeyBlocks - 1) : wave_id, role = kPair ? wave_id / kKeyBlocks : 0;
     const int g = lane >> 5;
     const int c_loc = lane & 31;
     const int kw0 = k0 + wave * kWaveKeys;  // first key of this wavefront
@@ -128,6 +148,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
         }
     }
 
+    // (a wavefront of a pair accumulates one of the two: dV where role = 0, else dK, in dv_acc)
     f32x16_t dk_acc[KB][DV], dv_acc[KB][DV];
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
@@ -139,7 +160,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     int i_lo, i_hi;
     query_range(a, k0, min(k0 + kBN, a.sk), i_lo, i_hi);
     if constexpr (kBias) {  // a workgroup that owns nothing but padded keys has dK = dV = 0
-        if (k0 >= padded_key_limit<kBwdThreads, false>(a, b, h, reinterpret_cast<float*>(smem_raw)))
+        if (k0 >= padded_key_limit<kThreads, false>(a, b, h, reinterpret_cast<float*>(smem_raw)))
             i_hi = i_lo;
     }
     int t_lo = i_lo / kBwdBM;
@@ -188,7 +209,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     regs.g.init(a.os[1], a.d);
     regs.stat = 0.f, regs.mask = 0u;
     regs.row_lse = 0.f;
-    int masked_pending = 0, masked_tile[2] = {0, 0};  // staged tiles that sync_staged must fix
+    int masked_pending = 0, masked_tile[SM::kBufs] = {};  // staged tiles that sync_staged must fix
     // lse / delta of a query tile: threads 0..63 fetch lse, threads 64..127 delta.
     const float* stat_src = (threadIdx.x < kBwdBM) ? lse_base : delta_base;
     // Requests tile t.  Unconditional: rows are clamped into the tensor (past the last tile the
@@ -201,23 +222,27 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
         // a branch here would end the basic block in the middle of a tile body, and the
         // exponentials of the body then sink below it, away from the matrix instructions that
         // are meant to run beside them (bf16 B4 S2048 H32 D80 causal: 289 -> 263 us; head_dim 128
-        // with dropout: 236 -> 221 us; head_dim 64: 1-3 %).  Only head_dim 128 without dropout,
-        // which requests at the top of the body, measured better with the branch (659 against
-        // 697 us at S 4096) and keeps it.
-        if (!(DPAD > 96 && kDrop == 0) || threadIdx.x < 2 * kBwdBM)
+        // with dropout: 236 -> 221 us; head_dim 64: 1-3 %).  Only head_dim 128 without dropout in
+        // four wavefronts, which requests at the top of the body, measured better with the branch
+        // (659 against 697 us at S 4096) and keeps it.
+        if (kPair || !(DPAD > 96 && kDrop == 0) || threadIdx.x < 2 * kBwdBM)
             r.stat = stat_src[min(i0 + (int)(threadIdx.x & (kBwdBM - 1)), a.sq - 1)];
         if constexpr (kBias) r.row_lse = lse_base[min(i0 + (int)(threadIdx.x & 63), a.sq - 1)];
         if constexpr (kDrop == 3) {
             // the keep bits that the forward stored: thread (w, row) of the workgroup fetches the
             // word of query row i0 + row for the 32 keys of wavefront w
-            const int w = min((k0 >> 5) + (int)(threadIdx.x >> 6), a.mask_words - 1);
+            const int w = min((k0 >> 5) + (int)(kPair ? threadIdx.x >> 6 & (kKeyBlocks - 1) : threadIdx.x >> 6), a.mask_words - 1);
             const int row = min(i0 + (int)(threadIdx.x & 63), a.mask_pitch - 1);
             r.mask = a.keep_mask[((int64_t)bh * a.mask_words + w) * a.mask_pitch + row];
         }
     };
-    // Writes the requested tile t into its LDS buffer (tiles alternate between two buffers).
+    // The LDS buffer of tile t.
+    auto buf_of = [&](int t) __attribute__((always_inline)) {
+        return kPair ? (int)((uint32_t)(t - t_lo) % SM::kBufs) : (t - t_lo) & 1;
+    };
+    // Writes the requested tile t into its LDS buffer.
     auto stage_tile = [&](TileRegs& r, int t) __attribute__((always_inline)) {
-        const int buf = (t - t_lo) & 1;
+        const int buf = buf_of(t);
         const int i0 = t * kBwdBM;
         r.q.fix(i0, a.sq, a.d);
         r.g.fix(i0, a.sq, a.d);
@@ -241,8 +266,8 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
                                 : (ok ? (kDrop == 0 ? -r.stat : r.stat * keep_prob) : 0.f);
             stat_lds[buf * 2 * kBwdBM + (threadIdx.x & kBwdBM) + row_slot(threadIdx.x & (kBwdBM - 1))] = v;
         }
-        if constexpr (kDrop == 3)
-            mask_lds[buf * kBwdThreads + (threadIdx.x & ~63) + row_slot(threadIdx.x & 63)] = r.mask;
+        if (kDrop == 3 && (!kPair || threadIdx.x < kKeyBlocks * 64))
+            mask_lds[buf * kKeyBlocks * 64 + (threadIdx.x & ~63) + row_slot(threadIdx.x & 63)] = r.mask;
     };
     // The barrier after a stage_tile.  Rows that saw nothing but masked keys (bias_log2) have
     // probabilities exp2(x + FLT_MAX) / n: the division goes onto their row of dO (and, in the dQ
@@ -254,14 +279,14 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
         if constexpr (kBias) {
             if (__builtin_expect(masked_pending != 0, 0)) {
 #pragma unroll 1
-                for (int buf = 0; buf < 2; ++buf) {
+                for (int buf = 0; buf < SM::kBufs; ++buf) {
                     if (!(masked_pending >> buf & 1)) continue;
                     const int i0 = masked_tile[buf] * kBwdBM;
                     T* tile = g_lds + buf * SM::kQTile;
 #pragma unroll
                     for (int u = 0; u < QStage::kPerThread; ++u) {
-                        const int c = threadIdx.x + u * kBwdThreads;
-                        if (QStage::kChunks % kBwdThreads != 0 && c >= QStage::kChunks) continue;
+                        const int c = threadIdx.x + u * kThreads;
+                        if (QStage::kChunks % kThreads != 0 && c >= QStage::kChunks) continue;
                         const int row = c / QStage::kChunksPerRow, cc = c % QStage::kChunksPerRow;
                         const float f = lse_row_factor(lse_base[min(i0 + row, a.sq - 1)]);
                         u32x4_t* p = reinterpret_cast<u32x4_t*>(tile + row * kPitch + cc * 8);
@@ -285,7 +310,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     // the kernel starts with such a pair, both tiles are requested at once.
     // (Measured: 3.5 % on the kernel at head_dim 128, 15 % with a local window; at 64 the second
     // register set spills and costs more than the pairing saves, at 80 it is a wash.)
-    constexpr bool kPairGeneric = DPAD > 96;
+    constexpr bool kPairGeneric = DPAD > 96 && !kPair;
     const bool pair_first =
         kPairGeneric && t_lo + 1 < t_hi && !tile_fast(t_lo) && !tile_fast(t_lo + 1);
     TileRegs second = regs;  // same lane offsets
@@ -516,7 +541,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     // per CU, and the second one is worth more than the stagger (319 -> 287 us at bf16 B4 S2048 H32 D80
     // causal, 638 -> 503 us when the backward regenerates the dropout mask).
     auto sequential_tile = [&](int t) __attribute__((always_inline)) {
-        const int buf = (t - t_lo) & 1;
+        const int buf = buf_of(t);
         const T* qt = q_lds + buf * SM::kQTile;
         const T* gt = g_lds + buf * SM::kQTile;
 #pragma unroll
@@ -524,7 +549,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
             const int ih0 = t * kBwdBM + 32 * hf;
             const float* lse_h = stat_lds + buf * 2 * kBwdBM + 32 * hf;
             const float* delta_h = lse_h + kBwdBM;
-            const uint32_t* mask_h = mask_lds + buf * kBwdThreads + wave * kBwdBM + 32 * hf;
+            const uint32_t* mask_h = mask_lds + buf * kKeyBlocks * 64 + wave * kBwdBM + 32 * hf;
             f32x16_t s[KB], dp[KB];
             uint32_t pw[KB][8], dw[KB][8];
             if constexpr (kRowsEarly) request_rows(ih0);
@@ -547,12 +572,12 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     auto staggered_tile = [&](int t, auto mask_tag, auto request_inside)
                               __attribute__((always_inline)) {
         constexpr bool kRequestInside = decltype(request_inside)::value;
-        const int buf = (t - t_lo) & 1;
+        const int buf = buf_of(t);
         const T* qt = q_lds + buf * SM::kQTile;
         const T* gt = g_lds + buf * SM::kQTile;
         const float* lse_t = stat_lds + buf * 2 * kBwdBM;
         const float* delta_t = lse_t + kBwdBM;
-        const uint32_t* mask_t = mask_lds + buf * kBwdThreads + wave * kBwdBM;
+        const uint32_t* mask_t = mask_lds + buf * kKeyBlocks * 64 + wave * kBwdBM;
         const int i0 = t * kBwdBM;
         f32x16_t s0[KB], s1[KB], p0[KB], p1[KB];
         uint32_t pw0[KB][8], dw0[KB][8], pw1[KB][8], dw1[KB][8];
@@ -600,12 +625,12 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
             const int tt = t + (j >> 1), hf = j & 1;
             const int ih0 = tt * kBwdBM + 32 * hf;
             if (!half_active(ih0)) continue;
-            const int buf = (tt - t_lo) & 1;
+            const int buf = buf_of(tt);
             const T* qt = q_lds + buf * SM::kQTile;
             const T* gt = g_lds + buf * SM::kQTile;
             const float* lse_h = stat_lds + buf * 2 * kBwdBM + 32 * hf;
             const float* delta_h = lse_h + kBwdBM;
-            const uint32_t* mask_h = mask_lds + buf * kBwdThreads + wave * kBwdBM + 32 * hf;
+            const uint32_t* mask_h = mask_lds + buf * kKeyBlocks * 64 + wave * kBwdBM + 32 * hf;
             f32x16_t s[KB], dp[KB];
             uint32_t pw[KB][8], dw[KB][8];
             if constexpr (kRowsEarly) request_rows(ih0);
@@ -644,6 +669,101 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     // rounds: with a copy for each side, three ways to mask in each, the live values of all of
     // them cost registers in the fast body too.
     int t = t_lo;
+    if constexpr (kPair) {
+        // ---- two wavefronts per 32 keys ----
+        // Of every query tile, role 0 computes P and dS of the first half and role 1 those of the second;
+        // each hands the other what it does not accumulate itself (16-bit words, through LDS) and adds up
+        // one of the two results, role 0 dV and role 1 dK.  Both add the first half before the second, as
+        // a wavefront on its own does: the results are the same bits.
+        // One barrier per tile, behind which every wavefront still reads tile t and its partner's words,
+        // hence three tile buffers and two of words.
+        unsigned char* hand = smem_raw + 2 * SM::kQBytes + SM::kStatBytes + SM::kMaskBytes +
+                              wave * SM::kHandBlock + lane * 16;
+        // acc += (tile rows of half hf)^T words: dV from dO and P, dK from Q and dS
+        auto pair_out = [&](const T* tile, int hf, const u32x4_t (&w)[2]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int hh = 0; hh < 2; ++hh) {
+                const T* rows = tile + (32 * hf + 16 * hh) * kPitch + t_off;
+#pragma unroll
+                for (int x = 0; x < DV; ++x)
+                    dv_acc[0][x] = Mma<T>::mma32(lds_frag_tr<T>(rows + 32 * x, kPitch),
+                                                 __builtin_bit_cast(frag_t, w[hh]), dv_acc[0][x]);
+            }
+        };
+        auto pair_iteration = [&](int t, auto role_tag, auto fast_tag) __attribute__((always_inline)) {
+            constexpr int kRole = decltype(role_tag)::value;
+            constexpr bool kFast = decltype(fast_tag)::value;
+            const int buf = buf_of(t);
+            const T* qt = q_lds + buf * SM::kQTile;
+            const T* gt = g_lds + buf * SM::kQTile;
+            const T* out_tile = kRole ? qt : gt;
+            // words of the halves: [tile parity][half][key block]
+            unsigned char* words = hand + ((t - t_lo) & 1) * (2 * kKeyBlocks * SM::kHandBlock);
+            unsigned char* mine = words + kRole * (kKeyBlocks * SM::kHandBlock);
+            const unsigned char* other = words + (1 - kRole) * (kKeyBlocks * SM::kHandBlock);
+            const int ih0 = t * kBwdBM + 32 * kRole;
+            const bool active = kFast || half_active(ih0);
+            u32x4_t own[2];
+            request_tile(regs, t + 1);
+            pin_requests();
+            if (active) {
+                const float* lse_h = stat_lds + buf * 2 * kBwdBM + 32 * kRole;
+                const float* delta_h = lse_h + kBwdBM;
+                const uint32_t* mask_h = mask_lds + buf * kKeyBlocks * 64 + wave * kBwdBM + 32 * kRole;
+                f32x16_t s[KB], dp[KB];
+                uint32_t pw[KB][8], dw[KB][8];
+                if constexpr (kRowsEarly) request_rows(ih0);
+                half_sp(qt, gt, lse_h, delta_h, kRole, s, dp);
+                half_exp(s, lse_h, ih0, std::integral_constant<int, kFast ? 0 : 1>{});
+                half_ds(s, dp, delta_h, mask_h, ih0, pw, dw);
+                const uint32_t(&kept)[8] = kRole ? dw[0] : pw[0];
+                const uint32_t(&sent)[8] = kRole ? pw[0] : dw[0];
+#pragma unroll
+                for (int hh = 0; hh < 2; ++hh) {
+                    *reinterpret_cast<u32x4_t*>(mine + hh * 1024) = u32x4_t{
+                        sent[4 * hh], sent[4 * hh + 1], sent[4 * hh + 2], sent[4 * hh + 3]};
+                    own[hh] = u32x4_t{kept[4 * hh], kept[4 * hh + 1], kept[4 * hh + 2], kept[4 * hh + 3]};
+                }
+                if constexpr (kRole == 0) pair_out(out_tile, 0, own);
+            }
+            if (t + 1 < t_hi) stage_tile(regs, t + 1);
+            sync_staged();
+            if (kFast || half_active(t * kBwdBM + 32 - 32 * kRole)) {
+                const u32x4_t theirs[2] = {*reinterpret_cast<const u32x4_t*>(other),
+                                           *reinterpret_cast<const u32x4_t*>(other + 1024)};
+                pair_out(out_tile, 1 - kRole, theirs);
+            }
+            if (kRole == 1 && active) pair_out(out_tile, 1, own);
+        };
+        auto pair_loop = [&](auto role_tag) __attribute__((always_inline)) {
+#pragma unroll 1
+            for (int round = 0; round < 2; ++round) {
+                for (; t < t_hi && !tile_fast(t); ++t) pair_iteration(t, role_tag, std::false_type{});
+                for (; t < t_hi && tile_fast(t); ++t) pair_iteration(t, role_tag, std::true_type{});
+            }
+        };
+        if (role == 0)
+            pair_loop(std::integral_constant<int, 0>{});
+        else
+            pair_loop(std::integral_constant<int, 1>{});
+        __syncthreads();  // the last tile has been read: every wavefront may write over it
+        if (kw0 < a.sk) {
+            const float mul = (role ? a.scale : 1.0f) * (kDrop != 0 ? a.rng.inv_keep : 1.0f);
+            if (a.n_split > 1) {
+                const int64_t rows = (int64_t)n_bh * a.sk;
+                store_partial<DPAD>(dv_acc[0], mul,
+                                    a.part + ((role ? split : a.n_split + split) * rows +
+                                              (int64_t)bh * a.sk + kw0) * a.d,
+                                    a.sk - kw0, a.d);
+                return;
+            }
+            const int64_t* st = role ? a.dks : a.dvs;
+            T* out = reinterpret_cast<T*>(role ? a.dk : a.dv) + b * st[0] + (int64_t)kw0 * st[1] + h * st[2];
+            store_block_via_lds<T, DPAD, kPitch>(dv_acc[0], mul, q_lds + wave_id * 32 * kPitch, out, st[1],
+                                                 a.sk - kw0, a.d);
+        }
+        return;
+    }
 #pragma unroll 1
     for (int round = 0; round < 2; ++round) {
         while (t < t_hi && !tile_fast(t)) t += generic_step(t);
@@ -679,26 +799,27 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     }
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
-__global__ __launch_bounds__(kBwdThreads, kPerCu) void attn_bwd_kernel(const AttnArgs a) {
-    dkv_block<T, DPAD, kBias, kDrop, KB, kSteps, kPerCu>(a, (int)blockIdx.x, (int)gridDim.x);
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu, bool kPair>
+__global__ __launch_bounds__((BwdSmem<T, DPAD, kPair>::kThreads), (kPair ? 2 : 1) * kPerCu) void attn_bwd_kernel(
+    const AttnArgs a) {
+    dkv_block<T, DPAD, kBias, kDrop, KB, kSteps, kPerCu, kPair>(a, (int)blockIdx.x, (int)gridDim.x);
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu>
+template <typename T, int DPAD, int kBias, int kDrop, int KB, int kSteps, int kPerCu, bool kPair>
 int launch(const AttnArgs& a, hipStream_t st) {
-    typedef BwdSmem<T, DPAD> SM;
+    typedef BwdSmem<T, DPAD, kPair> SM;
     const size_t smem = SM::kBytes;
-    constexpr int kBN = kBwdWaves * 32 * KB;
+    constexpr int kBN = kKeyBlocks * 32 * KB;
     const int n_kt = (a.sk + kBN - 1) / kBN;
     const int64_t blocks = (int64_t)n_kt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
-    auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps, kPerCu>;
+    auto kern = attn_bwd_kernel<T, DPAD, kBias, kDrop, KB, kSteps, kPerCu, kPair>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;
     AttnArgs ordered = a;
     if (a.n_split == 1) set_dispatch_order(&ordered, blocks, kPerCu);
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBwdThreads), smem, st, ordered);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(SM::kThreads), smem, st, ordered);
     return check_launch();
 }
 
@@ -709,10 +830,10 @@ template <typename T, int DPAD, int kBias, int kDrop, int kSteps>
 int launch_kb(const AttnArgs& a, hipStream_t st) {
     if constexpr (DPAD == 96 && kDrop == 3) {
         const int64_t blocks =
-            (int64_t)((a.sk + kBwdWaves * 32 - 1) / (kBwdWaves * 32)) * a.batch * a.heads;
-        if (blocks <= a.n_cus) return launch<T, DPAD, kBias, kDrop, 1, kSteps, 1>(a, st);
+            (int64_t)((a.sk + kBwdKeys - 1) / kBwdKeys) * a.batch * a.heads;
+        if (blocks <= a.n_cus) return launch<T, DPAD, kBias, kDrop, 1, kSteps, 1, false>(a, st);
     }
-    return launch<T, DPAD, kBias, kDrop, 1, kSteps, bwd_per_cu(DPAD)>(a, st);
+    return launch<T, DPAD, kBias, kDrop, 1, kSteps, bwd_per_cu(DPAD), (DPAD > 96)>(a, st);
 }
 
 template <typename T, int DPAD, int kBias, int kSteps>

@@ -609,6 +609,31 @@ def test_backward_in_one_launch_equals_the_two_kernels(shape, sk, causal, window
         assert torch.equal(a, r)
 
 
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("sq,sk,d,causal,window", [
+    (1, 129, 128, False, 0),      # one row of the first half tile, one key of the second workgroup
+    (32, 128, 104, False, 0),     # the second halves have no rows
+    (33, 31, 128, False, 0),      # ... and one; wavefronts without keys
+    (65, 97, 128, True, 0),
+    (191, 257, 128, False, 0),    # three tile buffers in turn
+    (320, 320, 112, True, 0),     # diagonal tiles, then full ones
+    (321, 300, 128, True, 40),    # halves outside the window
+])
+def test_dkv_of_wavefront_pairs(sq, sk, d, causal, window, masked):
+    """dK / dV above head_dim 96 in a launch of its own (two wavefronts per 32 keys) against the oracle."""
+    from slapo_amd.op import _kernels as K
+
+    q, k, v, do, g = _inputs(2, sq, 3, d, torch.bfloat16, sk=sk)
+    mask = _padding_mask(2, sk, torch.bfloat16, g, sk // 2 + 1)[0] if masked else None
+    qd, kd, vd, dod = (t.cuda() for t in (q, k, v, do))
+    bias = mask.float().cuda().expand(2, 3, sq, sk) if masked else None
+    o, lse, _ = K.attn_fwd(qd, kd, vd, bias, causal, window, d ** -0.5, 0.0, 1, 0, None)
+    got = K.attn_bwd(dod, qd, kd, vd, bias, o, lse, causal, window, d ** -0.5, 0.0, 1, 0, None)
+    want = OA.attention_fwd_bwd(q, k, v, do, mask, causal, window, 0.0, None, None, torch.float64)[1:]
+    for name, a, r in zip(("dq", "dk", "dv"), got, want):
+        assert_parity(a, r, torch.bfloat16, name)
+
+
 @pytest.mark.parametrize("mask", ["none", "key", "hidden", "square"])
 @pytest.mark.parametrize("shape,sk,causal,window", [
     ((2, 130, 3, 64), 130, True, 0),
