@@ -124,9 +124,12 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     };
     int j_lo, j_hi;
     key_range(a, q0, min(q0 + kBM, a.sq), j_lo, j_hi);
-    if constexpr (kBias)  // skip the tiles that hold nothing but padded keys
-        j_hi = max(j_lo + 1, min(j_hi, padded_key_limit<kThreads, false>(
-                                           a, b, h, reinterpret_cast<float*>(smem_raw))));
+    int bias_from = j_lo;  // keys before this one have a bias of zero
+    if constexpr (kBias == 2) {  // skip the tiles that hold nothing but padded keys
+        const KeyBiasSpan span =
+            key_bias_span<kThreads, false>(a, b, h, j_lo, j_hi, reinterpret_cast<int*>(smem_raw));
+        j_hi = span.limit, bias_from = span.zeros;
+    }
     int t_lo = j_lo / kBN;
     int t_hi = (j_hi + kBN - 1) / kBN;
     if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
@@ -289,13 +292,14 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // scores -> probabilities, in place
     // mask_tag: 0 = every key visible, 1 = the causal, window and tail bounds, as one bit per key:
     // two instructions per score whatever the bounds are (a compare and a select for each bound
-    // before), so that one masked tile body serves every call
+    // before), so that one masked tile body serves every call, 2 = every key visible and with a bias of
+    // zero
     auto half_exp = [&](f32x16_t& s, int t, int kb, auto mask_tag) __attribute__((always_inline)) {
         constexpr int kMask = decltype(mask_tag)::value;
         const int j0 = t * kBN + kb * 32;
         // register r is key j0 + acc_row(r, g) = j0 + kAccGroupStep g + c with c = acc_row(r, 0)
         uint32_t visible = 0u;
-        if constexpr (kMask != 0) {
+        if constexpr (kMask == 1) {
             const int k_max = a.causal ? min(a.sk - 1, q_row) : a.sk - 1;
             const int k_min = a.window > 0 ? q_row - a.window + 1 : 0;
             const int at = j0 + kAccGroupStep * g;
@@ -324,7 +328,7 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             float bv[4] = {0.f, 0.f, 0.f, 0.f};
-            if constexpr (kBias == 2) {  // already in log2 units
+            if constexpr (kBias == 2 && kMask != 2) {  // already in log2 units
                 const f32x4_t t4 = *reinterpret_cast<const f32x4_t*>(bias_tile + 32 * kb +
                                                                      quad_slot(r4, g));
                 bv[0] = t4.x, bv[1] = t4.y, bv[2] = t4.z, bv[3] = t4.w;
@@ -340,9 +344,9 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
             for (int e = 0; e < 4; ++e) {
                 float x = s[4 * r4 + e];  // the scale is in already
                 if constexpr (!kAccInit) x -= lse_sub;
-                if constexpr (kBias == 2 || kBias == 3) x += bv[e];
+                if constexpr ((kBias == 2 && kMask != 2) || kBias == 3) x += bv[e];
                 float p = fast_exp2(x);
-                if constexpr (kMask != 0) p = keep_or_zero(p, visible, acc_row(4 * r4 + e, 0));
+                if constexpr (kMask == 1) p = keep_or_zero(p, visible, acc_row(4 * r4 + e, 0));
                 s[4 * r4 + e] = p;
             }
         }
@@ -432,8 +436,8 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // Hand-scheduled version of tile_body for tiles without masks: the LDS operands of each group
     // of matrix instructions are requested one phase before the group runs, and scheduling fences
     // keep the compiler from sinking the requests back down to their uses.
-    auto tile_body_fast = [&](const T* kt, const T* vt, int t) __attribute__((always_inline)) {
-        constexpr std::integral_constant<int, 0> mask_tag{};
+    auto tile_body_fast = [&](const T* kt, const T* vt, int t, auto mask_tag)
+                              __attribute__((always_inline)) {
         frag_t kr0[DK], vr0[DK], kr1[DK], vr1[DK], kq0[2 * DV], kq1[2 * DV];
         f32x16_t s0, s1, p0, p1;
         uint32_t dw0[8], dw1[8];
@@ -502,15 +506,15 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     __syncthreads();
 
     // Iteration r: request the next tile, process tile r of the order, write the next tile into the
-    // other ring slot.  kFast iterations hold tiles that every wavefront of the workgroup sees in
-    // full; the others test activity per wavefront and mask.
+    // other ring slot.  kMask != 1: tiles that every wavefront of the workgroup sees in full; the
+    // others test activity per wavefront and mask.
     int t = order.first();
     request_bits(t);
     next_key = t * kBN;
     request_rows(0);
     request_rows(1);
-    auto iteration = [&](int r, auto fast_tag) __attribute__((always_inline)) {
-        constexpr bool kFast = decltype(fast_tag)::value;
+    auto iteration = [&](int r, auto mask_tag) __attribute__((always_inline)) {
+        constexpr bool kFast = decltype(mask_tag)::value != 1;
         const int next = kFast ? order.after_fast(t) : order.after(t);
         const bool have_next = r + 1 < n_tiles;
         tile_bits[0] = next_bits[0], tile_bits[1] = next_bits[1];
@@ -524,11 +528,11 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
         bias_tile = bias_lds + (r & 1) * kBN;
         if constexpr (kFast) {
             if constexpr (kStagger)
-                tile_body_fast(kt, vt, t);
+                tile_body_fast(kt, vt, t, mask_tag);
             else
-                tile_body(kt, vt, t, std::integral_constant<int, 0>{});
+                tile_body(kt, vt, t, mask_tag);
         } else if (tile_active(t)) {
-            tile_body(kt, vt, t, std::integral_constant<int, 1>{});
+            tile_body(kt, vt, t, mask_tag);
         } else {
             request_rows(0);
             request_rows(1);
@@ -544,8 +548,14 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
         t = next;
     };
     int r = 0;
-    for (; r < order.end - order.begin; ++r) iteration(r, std::true_type{});
-    for (; r < n_tiles; ++r) iteration(r, std::false_type{});
+    if constexpr (kBias == 2) {
+        // a padding mask is zero up to the padding: no bias to add there (bf16 B8 S1024 H16 D64 causal
+        // 49.3 -> 45.8 us, without the causal mask, p 0.1 85.0 -> 78.0)
+        const int zeros = min(order.end, bias_from / kBN) - order.begin;
+        for (; r < zeros; ++r) iteration(r, std::integral_constant<int, 2>{});
+    }
+    for (; r < order.end - order.begin; ++r) iteration(r, std::integral_constant<int, 0>{});
+    for (; r < n_tiles; ++r) iteration(r, std::integral_constant<int, 1>{});
     // ---- epilogue: dQ = scale * dQ^T^T ----
     // every wavefront is past the last barrier of the loop: the K buffers are free, and each
     // wavefront routes its 32 rows through its own quarter of them

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void keep_mask_kernel(const AttnArgs a_in, int
     const int bh = blockIdx.y;
     int w = unit % words;
     if (a.has_bias && a.bs[2] == 0 && a.window <= 0) {  // (of type fp32: see set_bias)
-        // from the first tile on that holds nothing but padded keys: not read (padded_key_limit)
+        // from the first tile on that holds nothing but padded keys: not read (key_bias_span)
         const float* row = reinterpret_cast<const float*>(a.bias) + bh / a.heads * a.bs[0] +
                            bh % a.heads * a.bs[1];
         bool padded = row[0] > kMaskedBias;  // uniform

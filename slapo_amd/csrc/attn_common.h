@@ -9,6 +9,8 @@
 // the A operand is free as well; both freedoms are used below to keep every fragment a plain
 // 128-bit LDS read or two transposing 64-bit reads.
 #pragma once
+#include <type_traits>
+
 #include "common.h"
 
 namespace slapo {
@@ -436,40 +438,76 @@ __device__ __forceinline__ void query_range(const AttnArgs& a, int k_lo, int k_h
 }
 
 // Key-padding masks arrive as an additive bias that does not depend on the query
-// ([B,1,1,Sk] with a large negative value on padded keys).  Keys past the last unmasked one
-// contribute exp(-huge) = 0 exactly to every row that sees at least one unmasked key, so whole
-// tiles of them can be skipped.  Returns one past the last key worth visiting (a.sk when the
-// shortcut does not apply): only per-key biases, no local window, and key 0 unmasked, which
-// guarantees an unmasked visible key for every query row under a causal or full mask.
-// Called by all threads of the workgroup; `scratch` is 4 floats of LDS that nothing else uses
-// until the call returns.
+// ([B,1,1,Sk] with a large negative value on padded keys, zero on the others).  What a workgroup needs to
+// know of it over its keys [j_lo, j_hi):
+//  * limit: one past the last key worth visiting.  Keys past the last unmasked one contribute
+//    exp(-huge) = 0 exactly to every row that sees at least one unmasked key, so whole tiles of them
+//    can be skipped: without a local window and with key 0 unmasked, which guarantees an unmasked visible
+//    key for every query row under a causal or full mask.
+//  * zeros: the first key from j_lo on whose bias is not zero.  The full tiles before it take a body
+//    that adds no bias.
+// (j_hi and j_lo where the bias does depend on the query.)  Called by all threads of the workgroup;
+// `scratch` is 2 * THREADS / 64 words of LDS that nothing else uses until the call returns.  The values
+// are read eight at a time per thread, all of them in flight together (one by one they took the forward
+// of bf16 B2 S7744 H7 D64 a twentieth of its time).
 constexpr float kMaskedBias = -30000.f;  // below fp16's most negative value, far beyond any score
+struct KeyBiasSpan {
+    int limit, zeros;
+    bool hidden;  // nothing but padded keys, which get no probability from any row
+};
 // kTyped: the bias may be of any type; the 16-bit backward kernels take fp32 only (their registers are
 // all spoken for: the selects of bias_value cost them 10 %).
 template <int THREADS, bool kTyped>
-__device__ __forceinline__ int padded_key_limit(const AttnArgs& a, int b, int h, float* scratch) {
-    if (!a.has_bias || a.bs[2] != 0 || a.window > 0) return a.sk;  // (a prepared one: pitch)
-    int last = 0;
-    if constexpr (kTyped) {
-        const int64_t row = b * a.bs[0] + h * a.bs[1];
-        if (!(bias_load(a, row) > kMaskedBias)) return a.sk;
-        for (int j = threadIdx.x; j < a.sk; j += THREADS)
-            if (bias_load(a, row + j * a.bs[3]) > kMaskedBias) last = j;
-    } else {
-        const float* row = reinterpret_cast<const float*>(a.bias) + b * a.bs[0] + h * a.bs[1];
-        if (!(row[0] > kMaskedBias)) return a.sk;
-        for (int j = threadIdx.x; j < a.sk; j += THREADS)
-            if (row[(int64_t)j * a.bs[3]] > kMaskedBias) last = j;
+__device__ __forceinline__ KeyBiasSpan key_bias_span(const AttnArgs& a, int b, int h, int j_lo, int j_hi,
+                                                     int* scratch) {
+    if (!a.has_bias || a.bs[2] != 0) return {j_hi, j_lo, false};  // (a prepared one: pitch)
+    const int64_t row = b * a.bs[0] + h * a.bs[1];
+    auto value = [&](int j) __attribute__((always_inline)) {
+        if constexpr (kTyped)
+            return bias_load(a, row + j * a.bs[3]);
+        else
+            return reinterpret_cast<const float*>(a.bias)[row + j * a.bs[3]];
+    };
+    const float first_value = value(0);
+    int last = j_lo - 1, nonzero = j_hi;  // wavefront-uniform
+    // n * THREADS keys from j0 on, this lane's the first of them at j
+    auto scan = [&](int j0, auto n_tag) __attribute__((always_inline)) {
+        constexpr int kN = decltype(n_tag)::value;
+        float v[kN];
+        const int j = j0 + (int)threadIdx.x;
+#pragma unroll
+        for (int u = 0; u < kN; ++u) v[u] = value(min(j + u * THREADS, j_hi - 1));
+#pragma unroll
+        for (int u = 0; u < kN; ++u) {
+            const bool in = j + u * THREADS < j_hi;
+            // (as bits: the 16-bit kernels are compiled without NaNs, and a NaN is not zero)
+            const bool any = (__builtin_bit_cast(uint32_t, v[u]) & 0x7FFFFFFFu) != 0u;
+            const uint64_t seen = __builtin_amdgcn_ballot_w64(in && v[u] > kMaskedBias);
+            const uint64_t set = __builtin_amdgcn_ballot_w64(in && any);
+            const int first = j0 + u * THREADS + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
+            if (seen) last = first + 63 - __builtin_clzll(seen);
+            if (set) nonzero = min(nonzero, first + __builtin_ctzll(set));
+        }
+    };
+    int j0 = j_lo;
+    for (; j_hi - j0 > THREADS; j0 += 8 * THREADS) scan(j0, std::integral_constant<int, 8>{});
+    if (j0 < j_hi) scan(j0, std::integral_constant<int, 1>{});
+    constexpr int kWaves = THREADS / 64;
+    if ((threadIdx.x & 63) == 0) {
+        scratch[threadIdx.x >> 6] = last;
+        scratch[kWaves + (threadIdx.x >> 6)] = nonzero;
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) last = max(last, __shfl_xor(last, off, 64));
-    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = __int_as_float(last);
     __syncthreads();
-    int limit = 0;
 #pragma unroll
-    for (int w = 0; w < THREADS / 64; ++w) limit = max(limit, __float_as_int(scratch[w]));
+    for (int w = 0; w < kWaves; ++w) {
+        last = max(last, scratch[w]);
+        nonzero = min(nonzero, scratch[kWaves + w]);
+    }
     __syncthreads();
-    return limit + 1;
+    last = __builtin_amdgcn_readfirstlane(last);
+    const bool skip = a.window <= 0 && first_value > kMaskedBias;
+    return {skip ? max(last, j_lo) + 1 : j_hi, __builtin_amdgcn_readfirstlane(nonzero),
+            skip && last < j_lo};
 }
 
 // Writes a wavefront's 32 x d block of results to global memory with full-line stores.  The

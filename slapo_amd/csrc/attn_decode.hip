@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kThreads) void attn_decode_kernel(const AttnArgs a,
 
     if (bias && bias_load(a, bias_at) > kMaskedBias) {
         // Padding at the end of the share contributes exactly zero to a row that sees key 0 (see
-        // padded_key_limit): its keys are not read.
+        // key_bias_span): its keys are not read.
         int last = k_lo - 1;
         for (int j = k_lo + (int)threadIdx.x; j < k_hi; j += kThreads)
             if (bias_load(a, bias_at + (int64_t)j * a.bs[3]) > kMaskedBias) last = j;

@@ -656,7 +656,8 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
     extern __shared__ __align__(16) float lds[];
     const Place at(a, a.sq, kRows, true);
     const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
-                          ? padded_key_limit<kFwdThreads, true>(a, at.b, at.h, lds)
+                          ? key_bias_span<kFwdThreads, true>(a, at.b, at.h, 0, a.sk,
+                                                             reinterpret_cast<int*>(lds)).limit
                           : a.sk;
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
@@ -801,7 +802,8 @@ attn_f32_dq_kernel(const AttnArgs a_in) {
     extern __shared__ __align__(16) float lds[];
     const Place at(a, a.sq, kRows, true);
     const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
-                          ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds)
+                          ? key_bias_span<kThreads, true>(a, at.b, at.h, 0, a.sk,
+                                                          reinterpret_cast<int*>(lds)).limit
                           : a.sk;
     int j_lo, j_hi;
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
@@ -979,7 +981,8 @@ attn_f32_dkv_kernel(const AttnArgs a_in) {
     extern __shared__ __align__(16) float lds[];
     const Place at(a, a.sk, kRows, false);
     const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
-                          ? padded_key_limit<kThreads, true>(a, at.b, at.h, lds)
+                          ? key_bias_span<kThreads, true>(a, at.b, at.h, 0, a.sk,
+                                                          reinterpret_cast<int*>(lds)).limit
                           : a.sk;
     int i_lo, i_hi;
     query_range(a, at.row0, min(at.row0 + kRows, a.sk), i_lo, i_hi);

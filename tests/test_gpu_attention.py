@@ -564,6 +564,39 @@ def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
     return ref, qf.grad, kf.grad, vf.grad
 
 
+@pytest.mark.parametrize("rest", ["padded", "soft", "hole"])
+@pytest.mark.parametrize("sq,sk,d,causal,window,zeros", [
+    (130, 200, 64, False, 0, 0),      # no key without a bias
+    (130, 200, 64, False, 0, 63),     # one short of a tile
+    (130, 257, 128, False, 0, 64),
+    (257, 257, 80, True, 0, 65),
+    (300, 2500, 64, False, 0, 2111),  # more keys than one round of the scan reads
+    (400, 400, 128, True, 0, 399),
+    (400, 400, 64, True, 130, 256),   # a window whose full tiles start behind key 0
+    (300, 300, 32, True, 0, 300),     # zero throughout
+])
+def test_key_bias_that_is_zero_up_to_a_key(sq, sk, d, causal, window, zeros, rest):
+    """Key masks whose leading tiles need no addition, what follows padded, of any value, or zero again
+    behind one hidden key, in training (fp32 copy of the mask) and at inference (16-bit)."""
+    q, k, v, do, g = _inputs(2, sq, 2, d, torch.bfloat16, sk=sk)
+    mask = torch.zeros(2, 1, 1, sk)
+    if rest == "padded":
+        mask[..., zeros:] = torch.finfo(torch.bfloat16).min
+    elif rest == "soft":
+        mask[..., zeros:] = torch.randn(2, 1, 1, sk - zeros, generator=g)
+    else:
+        mask[..., zeros:zeros + 1] = torch.finfo(torch.bfloat16).min
+    if zeros > 2:
+        mask[1, ..., zeros // 2:] = mask[1, ..., zeros - 1:zeros]  # another length in the second sequence
+        mask[1, ..., zeros // 2] = -3.0
+    mask = mask.to(torch.bfloat16)
+    _check(q, k, v, do, mask, causal, window, torch.bfloat16)
+    with torch.no_grad():
+        out = op.hip_attention(q.cuda(), k.cuda(), v.cuda(), mask.cuda(), causal=causal, window=window)
+    want = OA.attention_fwd_bwd(q, k, v, do, mask, causal, window, 0.0, None, None, torch.float64)[0]
+    assert_parity(out, want, torch.bfloat16, "out")
+
+
 @pytest.mark.parametrize("mask", ["none", "key", "hidden", "square"])
 @pytest.mark.parametrize("shape,sk,causal,window", [
     ((2, 130, 3, 64), 130, True, 0),
