@@ -132,7 +132,7 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     }
     int t_lo = j_lo / kBN;
     int t_hi = (j_hi + kBN - 1) / kBN;
-    if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
+    if (a.n_split > 1) split_tiles(a.n_split, split, t_lo, t_hi);
     const int n_tiles = t_hi - t_lo;
     const TileOrder order = TileOrder::of<kBM, kBN>(a, q0, t_lo, t_hi);
 

@@ -168,7 +168,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     }
     int t_lo = i_lo / kBwdBM;
     int t_hi = (i_hi + kBwdBM - 1) / kBwdBM;
-    if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
+    if (a.n_split > 1) split_tiles(a.n_split, split, t_lo, t_hi);
 
     // kBias: 0 = none, 1 = any layout (read from memory per score), 2 = the launcher guarantees a
     // bias that does not depend on the query (stride 0 over the queries, the compact [B,1,1,Sk]

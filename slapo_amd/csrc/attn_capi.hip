@@ -290,6 +290,11 @@ Splits plan_splits(const slapo_attn_params* p) {
     };
     const bool causal = p->causal && p->window <= 0;
     s.fwd = s.dq = attn_splits(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), f32, causal);
+    // (groups of wavefronts in a workgroup do the same without partial results in memory)
+    const int groups = f32 ? 1
+                           : attn_fwd_groups(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), p->head_dim,
+                                             causal);
+    if (s.fwd <= groups && !(p->head_dim > 64 && tiles(p->seqlen_k) > 40)) s.fwd = 1;
     s.dkv = attn_splits(blocks(p->seqlen_k), cus, tiles(p->seqlen_q), f32, causal);
     return s;
 }

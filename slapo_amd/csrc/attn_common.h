@@ -275,11 +275,14 @@ struct AttnArgs {
     float* part;
 };
 
-// The share of tiles [t_lo, t_hi) that workgroup number `split` of its row block takes.
-__device__ __forceinline__ void split_tiles(const AttnArgs& a, int split, int& t_lo, int& t_hi) {
+// Groups of wavefronts that share the key tiles of a 16-bit forward call (attn_split.hip).
+int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal);
+
+// The share of tiles [t_lo, t_hi) that number `split` of n_split takes.
+__device__ __forceinline__ void split_tiles(int n_split, int split, int& t_lo, int& t_hi) {
     const int n = t_hi - t_lo;
-    t_hi = t_lo + n * (split + 1) / a.n_split;
-    t_lo += n * split / a.n_split;
+    t_hi = t_lo + n * (split + 1) / n_split;
+    t_lo += n * split / n_split;
 }
 
 // One value of the additive bias in the type it is stored in.  Split into the read -- one aligned
@@ -572,8 +575,12 @@ __device__ __forceinline__ void pin_requests() { asm volatile("" ::: "memory"); 
 // The global loads are unconditional (out-of-range rows are clamped to the last valid row and
 // zeroed when the tile is written to LDS), so they stay in the caller's basic block and the
 // compiler can leave them in flight across the math that follows.
+// THREADS below the workgroup's 256: every group of that many threads stages a tile of its own.
 template <typename T, int DPAD, int ROWS, int THREADS>
 struct TileStage {
+    static __device__ __forceinline__ int tid() {
+        return THREADS < 256 ? (int)threadIdx.x & (THREADS - 1) : (int)threadIdx.x;
+    }
     static constexpr int kChunksPerRow = DPAD / 8;
     static constexpr int kChunks = ROWS * kChunksPerRow;
     static constexpr int kPerThread = (kChunks + THREADS - 1) / THREADS;
@@ -594,7 +601,7 @@ struct TileStage {
         const uint32_t stride_b = (uint32_t)row_stride * (uint32_t)sizeof(T);
 #pragma unroll
         for (int u = 0; u < kOffsets; ++u) {
-            const int c = threadIdx.x + u * THREADS;
+            const int c = tid() + u * THREADS;
             col[u] = (uint32_t)min((c % kChunksPerRow) * 8, d - 8) * (uint32_t)sizeof(T);
             own[u] = (uint32_t)(c / kChunksPerRow) * stride_b + col[u];
             // opaque to the optimiser, which would otherwise turn the select in `load` back into
@@ -617,7 +624,7 @@ struct TileStage {
         const uint32_t last_b = (uint32_t)last * stride_b;
 #pragma unroll
         for (int u = 0; u < kPerThread; ++u) {
-            const int c = threadIdx.x + u * THREADS;
+            const int c = tid() + u * THREADS;
             const int row = c / kChunksPerRow;
             uint32_t off;
             if constexpr (kOneColumn)
@@ -635,7 +642,7 @@ struct TileStage {
                                                  int n_rows, int d) {
 #pragma unroll
         for (int u = 0; u < kPerThread; ++u) {
-            const int c = threadIdx.x + u * THREADS;
+            const int c = tid() + u * THREADS;
             const int row = c / kChunksPerRow;
             const int cc = c % kChunksPerRow;
             const int gr = min(row0 + row, n_rows - 1);
@@ -649,7 +656,7 @@ struct TileStage {
         if (row0 + ROWS <= n_rows && d == DPAD) return;  // uniform: whole tile valid
 #pragma unroll
         for (int u = 0; u < kPerThread; ++u) {
-            const int c = threadIdx.x + u * THREADS;
+            const int c = tid() + u * THREADS;
             const int row = c / kChunksPerRow;
             const int cc = c % kChunksPerRow;
             if (row0 + row >= n_rows || cc * 8 >= d) r[u] = u32x4_t{0u, 0u, 0u, 0u};
@@ -663,12 +670,12 @@ struct TileStage {
     }
     // Tile row of chunk u of this thread.
     static __device__ __forceinline__ int row_of(int u) {
-        return (threadIdx.x + u * THREADS) / kChunksPerRow;
+        return (tid() + u * THREADS) / kChunksPerRow;
     }
     __device__ __forceinline__ void store(T* lds) const {
 #pragma unroll
         for (int u = 0; u < kPerThread; ++u) {
-            const int c = threadIdx.x + u * THREADS;
+            const int c = tid() + u * THREADS;
             if (kChunks % THREADS != 0 && c >= kChunks) continue;
             const int row = c / kChunksPerRow;
             const int cc = c % kChunksPerRow;

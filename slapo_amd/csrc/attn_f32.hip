@@ -663,7 +663,7 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
     j_hi = max(j_lo + 1, min(j_hi, limit));
     int t_lo = j_lo / kFwdTile, t_hi = (j_hi + kFwdTile - 1) / kFwdTile;
-    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
+    if (a.n_split > 1) split_tiles(a.n_split, at.split, t_lo, t_hi);
     if (fwd_pass<DB, kMode, kWaves, kHalves, true>(a, at, t_lo, t_hi, lds)) return;
     __syncthreads();
     a = read_again();
@@ -809,7 +809,7 @@ attn_f32_dq_kernel(const AttnArgs a_in) {
     key_range(a, at.row0, min(at.row0 + kRows, a.sq), j_lo, j_hi);
     j_hi = max(j_lo + 1, min(j_hi, limit));
     int t_lo = j_lo / kTile, t_hi = (j_hi + kTile - 1) / kTile;
-    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
+    if (a.n_split > 1) split_tiles(a.n_split, at.split, t_lo, t_hi);
     if (dq_pass<DB, kMode, kWaves, true>(a, at, t_lo, t_hi, lds)) return;
     __syncthreads();
     a = read_again();
@@ -989,7 +989,7 @@ attn_f32_dkv_kernel(const AttnArgs a_in) {
     // keys past the last unpadded one get no probability from any row
     if (at.row0 >= limit) i_hi = i_lo;
     int t_lo = i_lo / kTile, t_hi = (i_hi + kTile - 1) / kTile;
-    if (a.n_split > 1) split_tiles(a, at.split, t_lo, t_hi);
+    if (a.n_split > 1) split_tiles(a.n_split, at.split, t_lo, t_hi);
     if (dkv_pass<DB, kMode, kWaves, true>(a, at, t_lo, t_hi, lds)) return;
     __syncthreads();
     a = read_again();

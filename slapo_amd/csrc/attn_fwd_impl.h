@@ -41,7 +41,28 @@ constexpr int fwd_per_cu(int dpad) { return dpad <= 32 ? 4 : dpad <= 64 ? 3 : 2;
 // 30.8 -> 29.5 us, bf16 B2 S4096 H16 D64 causal 88.5 -> 83.1; bf16 B1 S8192 H8 D64, 512: 167 -> 169).
 constexpr int kFwdFour = 4;
 
-template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu>
+// Small launches: kGroups groups of wavefronts, each with an equal share of the key tiles of the same
+// 128 / kGroups queries, merged through LDS at the end.  A launch that leaves CUs idle takes as long as one
+// workgroup needs for all its tiles (0.9 us each at head_dim 64, 1.3 at 128, and 4 to start and end), and
+// kGroups as many workgroups walk a kGroups-th each.  With four groups a wavefront stages its own tiles
+// and meets no barrier.  What it costs is K / V traffic, kGroups times as much from L2.
+constexpr int group_rows(int groups) { return kBM / groups; }
+// LDS slots of a group's K and of its V tiles: one where a group is a single wavefront, whose LDS accesses
+// are in order anyway, or where two would leave one workgroup per CU.
+constexpr int group_slots(int groups, int dpad) { return groups == 1 || (groups == 2 && dpad <= 64) ? 2 : 1; }
+template <typename T, int DPAD, int kBias, int kGroups>
+constexpr size_t group_lds() {
+    return (size_t)2 * group_slots(kGroups, DPAD) * kBN * (DPAD + 8) * sizeof(T) +
+           (kBias == 2 || kBias == 4 ? 2 * kBN * sizeof(float) : 0);
+}
+// Workgroups per CU: two where that spills nothing.
+constexpr int group_per_cu(int groups, int dpad, int bias) {
+    return dpad <= 32 || (groups == 4 ? dpad <= 64 && bias != 3 : dpad <= 64 || (dpad <= 96 && bias != 3))
+               ? 2
+               : 1;
+}
+
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu, int kGroups>
 __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     const AttnArgs a_in) {
     // kBias: 0 = no additive bias, 1 = any layout (read from memory per score), 2 = the bias
@@ -57,7 +78,9 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     AttnArgs a = a_in;
     if constexpr (kDrop == 1 || kDrop == 2) resolve_device_state(a.rng);
     typedef typename Mma<T>::frag frag_t;
-    typedef TileStage<T, DPAD, kBN, kThreads> Stage;
+    constexpr int kRowWaves = kWaves / kGroups, kRows = group_rows(kGroups);
+    constexpr int kSlots = group_slots(kGroups, DPAD);
+    typedef TileStage<T, DPAD, kBN, kRowWaves * 64> Stage;
     constexpr int kPitch = Stage::kPitch;
     constexpr int kTileElems = kBN * kPitch;
     // k-steps of S^T = K Q^T: DPAD / 16, or one fewer where the launcher guarantees head_dim <=
@@ -66,14 +89,18 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     constexpr int DV = DPAD / 32;  // 32-row blocks of O^T
 
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    T* k_lds = reinterpret_cast<T*>(smem_raw);  // K[2][tile]
-    T* v_lds = k_lds + 2 * kTileElems;          // V[2][tile]
-    float* bias_lds = reinterpret_cast<float*>(v_lds + 2 * kTileElems);  // [2][kBN], kKeyBias
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wavefront-uniform
+    const int group = kGroups == 1 ? 0 : wave / kRowWaves;
+    const int row_wave = kGroups == 1 ? wave : wave % kRowWaves;
+    T* k_lds = reinterpret_cast<T*>(smem_raw + group * group_lds<T, DPAD, kBias, kGroups>());
+    T* v_lds = k_lds + kSlots * kTileElems;  // K[kSlots][tile], V[kSlots][tile]
+    float* bias_lds = reinterpret_cast<float*>(v_lds + kSlots * kTileElems);  // [2][kBN], kKeyBias
 
     const int n_bh = a.batch * a.heads;
-    const int n_qt = (a.sq + kBM - 1) / kBM;
+    const int n_qt = (a.sq + kRows - 1) / kRows;
     int work = work_index(a, (int)blockIdx.x, (int)gridDim.x), split = 0;
-    if (a.n_split > 1) {
+    if (kGroups == 1 && a.n_split > 1) {
         split = work / (n_bh * n_qt);
         work -= split * n_bh * n_qt;
     }
@@ -81,13 +108,11 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     const int qt = n_qt - 1 - work / n_bh;  // heaviest (latest) query tiles first
     const int b = bh / a.heads;
     const int h = bh % a.heads;
-    const int q0 = qt * kBM;
+    const int q0 = qt * kRows;
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wavefront-uniform
     const int g = lane >> 5;
     const int i_loc = lane & 31;
-    const int wq0 = q0 + wave * 32;  // first query of this wavefront
+    const int wq0 = q0 + row_wave * 32;  // first query of this wavefront
     const int q_row = wq0 + i_loc;
 
     const T* q_base = reinterpret_cast<const T*>(a.q) + b * a.qs[0] + h * a.qs[2];
@@ -95,7 +120,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     const T* v_base = reinterpret_cast<const T*>(a.v) + b * a.vs[0] + h * a.vs[2];
 
     int j_lo, j_hi;
-    key_range(a, q0, min(q0 + kBM, a.sq), j_lo, j_hi);
+    key_range(a, q0, min(q0 + kRows, a.sq), j_lo, j_hi);
     int bias_from = j_lo;  // keys before this one have a bias of zero
     if constexpr (kKeyBias) {  // skip the tiles that hold nothing but padded keys
         const KeyBiasSpan span = key_bias_span<kThreads, kBias == 4>(a, b, h, j_lo, j_hi,
@@ -104,9 +129,13 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     }
     int t_lo = j_lo / kBN;
     int t_hi = (j_hi + kBN - 1) / kBN;
-    if (a.n_split > 1) split_tiles(a, split, t_lo, t_hi);
+    const int n_longest = (t_hi - t_lo + kGroups - 1) / kGroups;  // tiles of the group with most
+    if constexpr (kGroups > 1)
+        split_tiles(kGroups, group, t_lo, t_hi);
+    else if (a.n_split > 1)
+        split_tiles(a.n_split, split, t_lo, t_hi);
     const int n_tiles = t_hi - t_lo;
-    const TileOrder order = TileOrder::of<kBM, kBN>(a, q0, t_lo, t_hi);
+    const TileOrder order = TileOrder::of<kRows, kBN>(a, q0, t_lo, t_hi);
     const int first = order.first() * kBN;  // first key of the first tile
 
     // Start-up loads, all issued before any is used: the Q^T fragments (column i = this lane's
@@ -495,10 +524,21 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     // ---- prologue: tile 0 into LDS ----
     ks.fix(first, a.sk, a.d);
     vs.fix(first, a.sk, a.d);
+    // The wavefronts of a group see each other's stores to LDS (all of the workgroup where there are two
+    // groups: they walk the same number of barriers).
+    auto group_sync = [&]() __attribute__((always_inline)) {
+        if constexpr (kRowWaves > 1) {
+            __syncthreads();
+        } else {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    };
     ks.store(k_lds);
     vs.store(v_lds);
     store_bias(0);
-    __syncthreads();
+    group_sync();
 
     // Iteration r: request the next tile, process tile r of the order, write the next tile into the
     // other slot.  kMask != 1: tiles that every wavefront of the workgroup sees in full.
@@ -519,8 +559,8 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
         ks.load(k_base, a.ks[1], next, a.sk, a.d);
         vs.load(v_base, a.vs[1], next, a.sk, a.d);
         request_bias(next);
-        const T* kt = k_lds + (r & 1) * kTileElems;
-        const T* vt = v_lds + (r & 1) * kTileElems;
+        const T* kt = k_lds + (r & (kSlots - 1)) * kTileElems;
+        const T* vt = v_lds + (r & (kSlots - 1)) * kTileElems;
         bias_tile = bias_lds + (r & 1) * kBN;
         if constexpr (kFast) {
             tile_body(kt, vt, t, next, mask_tag);
@@ -530,14 +570,15 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
             else
                 request_rows(next);
         }
+        if constexpr (kSlots == 1) group_sync();
         if (have_next) {
             ks.fix(next, a.sk, a.d);
             vs.fix(next, a.sk, a.d);
-            ks.store(k_lds + ((r + 1) & 1) * kTileElems);
-            vs.store(v_lds + ((r + 1) & 1) * kTileElems);
+            ks.store(k_lds + ((r + 1) & (kSlots - 1)) * kTileElems);
+            vs.store(v_lds + ((r + 1) & (kSlots - 1)) * kTileElems);
             store_bias((r + 1) & 1);
         }
-        __syncthreads();
+        group_sync();
         t = t_next;
     };
     int r = 0;
@@ -552,8 +593,55 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     for (; r < n_tiles; ++r) iteration(r, std::integral_constant<int, 1>{});
 
     // ---- epilogue ----
+    if constexpr (kGroups > 1) {
+        if constexpr (kRowWaves > 1)
+            for (; r < n_longest; ++r) {  // (the other group's barriers)
+                if constexpr (kSlots == 1) group_sync();
+                group_sync();
+            }
+        // The first group adds up: the others leave m, l and O^T in LDS as they sit in registers, a word
+        // of 64 lanes after the other.
+        constexpr int kWords = 16 * DV + 2;
+        float* mine = reinterpret_cast<float*>(smem_raw) + row_wave * (kGroups - 1) * 64 * kWords + lane;
+        __syncthreads();
+        if (group > 0) {
+            float* p = mine + (group - 1) * 64 * kWords;
+            p[0] = m_run, p[64] = l_run;
+#pragma unroll
+            for (int x = 0; x < DV; ++x)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) p[64 * (2 + 16 * x + e)] = o_acc[x][e];
+        }
+        __syncthreads();
+        if (group > 0) return;
+        float m = m_run;
+#pragma unroll
+        for (int k = 0; k < kGroups - 1; ++k) m = fmaxf(m, mine[k * 64 * kWords]);
+        // (an unset reference weighs nothing)
+        auto weight = [&](float mk) __attribute__((always_inline)) {
+            return mk == -INFINITY ? 0.f : fast_exp2(mk - m);
+        };
+        const float w0 = weight(m_run);
+        l_run *= w0;
+#pragma unroll
+        for (int x = 0; x < DV; ++x)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o_acc[x][e] *= w0;
+#pragma unroll
+        for (int k = 0; k < kGroups - 1; ++k) {
+            const float* p = mine + k * 64 * kWords;
+            const float w = weight(p[0]);
+            l_run = __builtin_fmaf(p[64], w, l_run);
+#pragma unroll
+            for (int x = 0; x < DV; ++x)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    o_acc[x][e] = __builtin_fmaf(p[64 * (2 + 16 * x + e)], w, o_acc[x][e]);
+        }
+        m_run = m;
+    }
     const float l_tot = sum_xor32(l_run);
-    if (a.n_split > 1) {
+    if (kGroups == 1 && a.n_split > 1) {
         const int64_t rows = (int64_t)n_bh * a.sq;
         const int64_t row0 = (int64_t)bh * a.sq + wq0;
         if (wq0 < a.sq)
@@ -566,11 +654,16 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     }
     const float inv_l = kDrop != 0 ? a.rng.inv_keep / l_tot : 1.0f / l_tot;
     // every wavefront is past the last barrier of the loop: the K buffers are free, and each
-    // wavefront routes its 32 output rows through its own quarter of them
+    // wavefront routes its 32 output rows through its own quarter of them (with groups: through what the
+    // others left for it, which it has read)
     if (wq0 < a.sq) {
         T* o_row0 = reinterpret_cast<T*>(a.o) + b * a.os[0] + (int64_t)wq0 * a.os[1] + h * a.os[2];
-        store_block_via_lds<T, DPAD, kPitch>(o_acc, inv_l, k_lds + wave * 32 * kPitch, o_row0,
-                                             a.os[1], a.sq - wq0, a.d);
+        T* rows_lds = reinterpret_cast<T*>(smem_raw);
+        if constexpr (kGroups == 1)
+            rows_lds += wave * 32 * kPitch;
+        else
+            rows_lds += row_wave * (kGroups - 1) * 64 * (16 * DV + 2) * 2;
+        store_block_via_lds<T, DPAD, kPitch>(o_acc, inv_l, rows_lds, o_row0, a.os[1], a.sq - wq0, a.d);
     }
     if (q_row < a.sq) {
         // A row that met nothing but masked keys (bias_log2) sits at -FLT_MAX with l_tot = their
@@ -582,27 +675,36 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     }
 }
 
-template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu = fwd_per_cu(DPAD)>
+template <typename T, int DPAD, int kBias, int kDrop, int kSteps, int kPerCu = fwd_per_cu(DPAD),
+          int kGroups = 1>
 int launch(const AttnArgs& a, hipStream_t st) {
-    typedef TileStage<T, DPAD, kBN, kThreads> Stage;
-    const size_t smem = (size_t)4 * kBN * Stage::kPitch * sizeof(T) +
-                        (kBias == 2 || kBias == 4 ? 2 * kBN * sizeof(float) : 0);
-    const int n_qt = (a.sq + kBM - 1) / kBM;
+    const size_t smem = kGroups * group_lds<T, DPAD, kBias, kGroups>();
+    const int n_qt = (a.sq + group_rows(kGroups) - 1) / group_rows(kGroups);
     const int64_t blocks = (int64_t)n_qt * a.batch * a.heads * a.n_split;
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
+    if constexpr (kGroups == 1 && kBias != 1) {
+        const int64_t keys = a.window > 0 ? min(a.sk, a.window + kBM) : a.sk;
+        const int groups = a.n_split > 1 ? 1
+                                         : attn_fwd_groups(blocks, a.n_cus, (keys + kBN - 1) / kBN, a.d,
+                                                           a.causal && a.window <= 0);
+        if (groups == 4)
+            return launch<T, DPAD, kBias, kDrop, kSteps, group_per_cu(4, DPAD, kBias), 4>(a, st);
+        if (groups == 2)
+            return launch<T, DPAD, kBias, kDrop, kSteps, group_per_cu(2, DPAD, kBias), 2>(a, st);
+    }
     // kRowsAhead against one workgroup more per CU (bf16 B8 S1024 H16, 1024 workgroups): without the
     // causal mask D64 100.8 -> 96.7 us, D32 98.5 -> 95.9; with it, whose workgroups differ in length,
     // 65.8 -> 66.3 and 60.0 -> 64.5, so there only in launches that need not the one more
-    if constexpr (DPAD <= 64 && kBias == 3 && kPerCu == fwd_per_cu(DPAD) &&
+    if constexpr (kGroups == 1 && DPAD <= 64 && kBias == 3 && kPerCu == fwd_per_cu(DPAD) &&
                   (DPAD == 64 || (kDrop != 1 && kDrop != 2))) {
         if (!a.causal || blocks <= (int64_t)(kPerCu - 1) * a.n_cus)
             return launch<T, DPAD, kBias, kDrop, kSteps, kPerCu - 1>(a, st);
     }
-    if constexpr (DPAD <= 64 && kBias == 0 && kDrop == 0 && kPerCu < kFwdFour) {
+    if constexpr (kGroups == 1 && DPAD <= 64 && kBias == 0 && kDrop == 0 && kPerCu < kFwdFour) {
         if (blocks > (int64_t)kPerCu * a.n_cus)
             return launch<T, DPAD, kBias, kDrop, kSteps, kFwdFour>(a, st);
     }
-    auto kern = attn_fwd_kernel<T, DPAD, kBias, kDrop, kSteps, kPerCu>;
+    auto kern = attn_fwd_kernel<T, DPAD, kBias, kDrop, kSteps, kPerCu, kGroups>;
     static std::atomic<uint64_t> lds_ready{0};  // per instantiation, one bit per device
     if (allow_dynamic_lds(reinterpret_cast<const void*>(kern), smem, lds_ready) != SLAPO_OK)
         return SLAPO_ERR_LAUNCH;

@@ -148,6 +148,36 @@ int attn_splits(int64_t blocks, int64_t cus, int64_t tiles, bool f32, bool causa
     return n < 2 ? 1 : (int)n;
 }
 
+// Into how many groups of wavefronts a forward workgroup of the 16-bit kernels is divided (attn_fwd_impl.h),
+// for `blocks` undivided workgroups of 128 queries: four, two or one, so that their number comes near what
+// the chip holds.  Four groups of a wavefront each bring the 32-query workgroups to four times as many; above
+// head_dim 64 their LDS leaves one a CU.  Under a causal mask the workgroups have half the longest one's
+// tiles on average, so more of them pay.  Forward, undivided (or by attn_splits) / two / four groups, bf16
+// without a mask:
+//   D64   B1 S1024 H4 (32 blocks) 17.8 / 12.1 / 9.7 us, H16 (128) 18.3 / 13.1 / 14.6, causal 18.3 / 13.0 /
+//         11.1, H32 (256) 20.1 / 18.5 / 25.1, causal 19.4 / 13.8 / 19.1; B4 S512 H16 (256) 11.8 / 11.9 /
+//         17.6, causal 11.9 / 9.3 / 15.5; B1 S8192 H4 causal (256) 93.8 / 72.6 / 68.1; with drawn dropout B1
+//         S1024 H16 causal 39.3 / 24.1 / 16.5
+//   D80   B1 S512 H16 (64) 13.6 / 11.8 / 12.5, S1024 H8 (64) 22.7 / 18.0 / 17.6, H16 (128) 23.4 / 19.1 /
+//         32.5, H32 (256) 25.5 / 27.0 / 62.6, causal 24.2 / 20.5 / 48.7
+//   D128  B1 S256 H16 (32) 9.9 / 10.4 / 9.9, S1024 H8 (64) 26.2 / 23.2 / 18.8, H16 (128) 27.2 / 24.9 / 34.8,
+//         H32 causal (256) 27.7 / 31.7 / 49.8, S2048 H16 causal (256) 56.1 / 47.5 / 68.1
+// Below six tiles there is nothing to divide (B1 S256 H16 D64 7.2 / 7.0 / 6.8).
+int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal) {
+    if (cus <= 0 || blocks > cus || tiles < 6) return 1;
+    const bool half = 2 * blocks <= cus, quarter = 4 * blocks <= cus;
+    if (d <= 64) {
+        if (quarter || (half && causal)) return 4;
+        return half || causal || tiles >= 16 ? 2 : 1;
+    }
+    if (d <= 96) {
+        if (quarter && tiles >= 16) return 4;
+        return half || causal ? 2 : 1;
+    }
+    if (quarter) return tiles >= 8 ? 4 : 1;
+    return tiles >= (half ? 8 : 24) && (half || causal) ? 2 : 1;
+}
+
 int attn_merge_fwd(const AttnArgs& a, int dtype, hipStream_t st) {
     const int64_t threads = (int64_t)a.batch * a.heads * a.sq * ((a.d + 3) / 4);
     const int64_t blocks = (threads + kThreads - 1) / kThreads;

@@ -564,6 +564,36 @@ def _fp32_twin(q, k, v, do, mask, causal, window, p, seed):
     return ref, qf.grad, kf.grad, vf.grad
 
 
+@pytest.mark.parametrize("mask", ["none", "key", "square"])
+@pytest.mark.parametrize("shape,sk,causal,window,p", [
+    # four groups: 32 queries, one wavefront per share of the tiles
+    ((1, 330, 2, 64), 330, True, 0, 0.1),       # six tiles, shares of one and two
+    ((2, 33, 2, 64), 449, False, 0, 0.0),       # the second workgroup has one query
+    ((1, 400, 2, 32), 500, True, 0, 0.0),       # workgroups with fewer tiles than groups
+    ((1, 700, 2, 64), 700, True, 300, 0.1),     # a window: shares that none of the queries sees
+    ((1, 520, 2, 128), 520, True, 0, 0.0),
+    ((1, 1025, 1, 80), 1025, False, 0, 0.1),
+    # two groups: 64 queries, two wavefronts each
+    ((1, 700, 12, 64), 700, False, 0, 0.0),
+    ((1, 330, 3, 96), 400, False, 0, 0.1),
+    ((1, 641, 13, 128), 641, True, 0, 0.0),
+    ((1, 641, 13, 104), 577, False, 0, 0.2),
+])
+def test_forward_in_groups_of_wavefronts(shape, sk, causal, window, p, mask):
+    """Small launches, whose workgroups deal the key tiles to groups of their wavefronts."""
+    b, s, h, d = shape
+    q, k, v, do, g = _inputs(b, s, h, d, torch.bfloat16, sk=sk)
+    m = None
+    if mask == "key":
+        m = _padding_mask(b, sk, torch.bfloat16, g, sk // 2)[0]
+    elif mask == "square":
+        m = torch.randn(b, 1, s, sk, generator=g)
+        m[:, :, s // 2] = torch.finfo(torch.bfloat16).min  # a row of masked keys
+        m[:, :, 3, : sk // 2] = torch.finfo(torch.bfloat16).min  # ... and half a row
+        m = m.to(torch.bfloat16)
+    _check(q, k, v, do, m, causal, window, torch.bfloat16, p)
+
+
 @pytest.mark.parametrize("rest", ["padded", "soft", "hole"])
 @pytest.mark.parametrize("sq,sk,d,causal,window,zeros", [
     (130, 200, 64, False, 0, 0),      # no key without a bias
