@@ -501,8 +501,8 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
 
     // ---- prologue: tile 0 into LDS ----
     if (n_tiles > 0) {
-        ks.fix(order.first() * kBN, a.sk, a.d);
-        vs.fix(order.first() * kBN, a.sk, a.d);
+        ks.fix(order.first() * kBN, a.sk, a.d, 16 * DK);
+        vs.fix(order.first() * kBN, a.sk, a.d, 16 * DK);
         ks.store(k_lds);
         vs.store(v_lds);
         store_bias(0);
@@ -542,8 +542,8 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
             request_rows(1);
         }
         if (have_next) {
-            ks.fix(next * kBN, a.sk, a.d);
-            vs.fix(next * kBN, a.sk, a.d);
+            ks.fix(next * kBN, a.sk, a.d, 16 * DK);
+            vs.fix(next * kBN, a.sk, a.d, 16 * DK);
             ks.store(k_lds + ((r + 1) % kKRing) * kTileElems);
             vs.store(v_lds + ((r + 1) % kVRing) * kTileElems);
             store_bias((r + 1) & 1);

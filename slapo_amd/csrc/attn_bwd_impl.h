@@ -247,8 +247,8 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     auto stage_tile = [&](TileRegs& r, int t) __attribute__((always_inline)) {
         const int buf = buf_of(t);
         const int i0 = t * kBwdBM;
-        r.q.fix(i0, a.sq, a.d);
-        r.g.fix(i0, a.sq, a.d);
+        r.q.fix(i0, a.sq, a.d, 16 * DK);
+        r.g.fix(i0, a.sq, a.d, 16 * DK);
         if constexpr (kBias) {
             // Every wavefront holds the 64 lse values of the tile, one per lane, so all of them
             // agree on whether the tile has a row that saw nothing but masked keys; see

@@ -522,8 +522,8 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     };
 
     // ---- prologue: tile 0 into LDS ----
-    ks.fix(first, a.sk, a.d);
-    vs.fix(first, a.sk, a.d);
+    ks.fix(first, a.sk, a.d, 16 * DK);
+    vs.fix(first, a.sk, a.d, 16 * DK);
     // The wavefronts of a group see each other's stores to LDS (all of the workgroup where there are two
     // groups: they walk the same number of barriers).
     auto group_sync = [&]() __attribute__((always_inline)) {
@@ -572,8 +572,8 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
         }
         if constexpr (kSlots == 1) group_sync();
         if (have_next) {
-            ks.fix(next, a.sk, a.d);
-            vs.fix(next, a.sk, a.d);
+            ks.fix(next, a.sk, a.d, 16 * DK);
+            vs.fix(next, a.sk, a.d, 16 * DK);
             ks.store(k_lds + ((r + 1) & (kSlots - 1)) * kTileElems);
             vs.store(v_lds + ((r + 1) & (kSlots - 1)) * kTileElems);
             store_bias((r + 1) & 1);
