@@ -488,7 +488,12 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
         if (splits.dkv > 1) dkv_part = next;
     }
 
-    if (deal && !f32 && stages == SLAPO_BWD_ALL && splits.dq == 1 && splits.dkv == 1 &&
+    // In two shares the partial results cost more than the one launch, whose two kernels fill each other's
+    // idle CUs.  Backward, two shares / one launch, bf16: B1 S2048 H8 D64 (128 blocks) 68.0 / 49.2 us, H16
+    // causal (256) 89.7 / 57.3, S8192 H4 causal 234 / 189; H16 causal D80 117 / 79.6; H8 D128 112 / 87.4, B2
+    // S1600 H9 D128 causal 119 / 80.3.  In four, with 64 blocks, they do not: S2048 H4 D64 48.8 / 45.8, S4096
+    // H2 64.7 / 82.1, D128 105 / 145.
+    if (deal && !f32 && stages == SLAPO_BWD_ALL && splits.dq <= 2 && splits.dkv <= 2 &&
         one_launch_backward(a))
         return prm->dtype == SLAPO_F16 ? attn_bwd_both_mfma_f16(a, st)
                                        : attn_bwd_both_mfma_bf16(a, st);
