@@ -679,7 +679,7 @@ def main():
                           "raw_event_intervals_ms": seg_raw,
                           "sum_of_kernels_ms": sum(seg_ms)},
     }
-    result["kernels"] = [kern("attn_fwd_kernel<f16,64,0,0,4,4>", 4 * d * n_pairs, seg_ms[0]),
+    result["kernels"] = [kern("attn_fwd_kernel<f16,64,0,0,4,4,1>", 4 * d * n_pairs, seg_ms[0]),
                          kern("attn_bwd_kernel<f16,64,0,0,1,4,2,0> (dK/dV)", bwd_flops, seg_ms[2]),
                          kern("attn_bwd_dq_kernel<f16,64,0,0,4>", 6 * d * n_pairs, seg_ms[1])]
     with_cpu = not args.no_cpu_baseline
