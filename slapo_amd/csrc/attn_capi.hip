@@ -276,7 +276,9 @@ namespace {
 struct Splits {
     int fwd = 1, dq = 1, dkv = 1;
 };
-Splits plan_splits(const slapo_attn_params* p) {
+// grouped: the forward can be divided into groups of wavefronts (every build but the one that reads a bias
+// of any layout per score).
+Splits plan_splits(const slapo_attn_params* p, bool grouped) {
     Splits s;
     if (!p || p->batch <= 0 || p->heads <= 0 || p->seqlen_q <= 0 || p->seqlen_k <= 0 ||
         p->head_dim <= 0)
@@ -291,10 +293,11 @@ Splits plan_splits(const slapo_attn_params* p) {
     const bool causal = p->causal && p->window <= 0;
     s.fwd = s.dq = attn_splits(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), f32, causal);
     // (groups of wavefronts in a workgroup do the same without partial results in memory)
-    const int groups = f32 ? 1
+    const int groups = f32 || !grouped
+                           ? 1
                            : attn_fwd_groups(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), p->head_dim,
                                              causal);
-    if (s.fwd <= groups && !(p->head_dim > 64 && tiles(p->seqlen_k) > 40)) s.fwd = 1;
+    if (groups > 1 && s.fwd <= groups && !(p->head_dim > 64 && tiles(p->seqlen_k) > 40)) s.fwd = 1;
     s.dkv = attn_splits(blocks(p->seqlen_k), cus, tiles(p->seqlen_q), f32, causal);
     return s;
 }
@@ -309,14 +312,14 @@ extern "C" size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* pr
         return shares == 1 ? 0
                            : (size_t)shares * prm->batch * prm->heads * (2 + prm->head_dim) *
                                  sizeof(float);
-    const Splits s = plan_splits(prm);
+    const Splits s = plan_splits(prm, prm && prm->bias_strides[2] == 0);
     if (s.fwd == 1) return 0;
     return (size_t)s.fwd * prm->batch * prm->heads * prm->seqlen_q * (2 + prm->head_dim) *
            sizeof(float);
 }
 
 extern "C" size_t slapo_amd_attn_bwd_ex_workspace_bytes(const slapo_attn_params* prm) {
-    const Splits s = plan_splits(prm);
+    const Splits s = plan_splits(prm, true);
     if (s.dq == 1 && s.dkv == 1) return slapo_amd_attn_bwd_workspace_bytes(prm);
     const size_t row = (size_t)prm->batch * prm->heads * prm->head_dim * sizeof(float);
     return delta_bytes(prm) + (s.dq > 1 ? row * prm->seqlen_q * s.dq : 0) +
@@ -382,7 +385,7 @@ extern "C" int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q
     const size_t split_bytes = slapo_amd_attn_fwd_workspace_bytes(prm);
     if (workspace && split_bytes > 0 && workspace_bytes >= split_bytes &&
         decode_shares(prm) == 0) {
-        a.n_split = plan_splits(prm).fwd;
+        a.n_split = plan_splits(prm, !a.has_bias || bias_type != SLAPO_F32 || a.bs[2] == 0).fwd;
         a.part = static_cast<float*>(workspace);
     }
     auto merged = [&](int status) {
@@ -479,7 +482,7 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
     Splits splits;
     float *dq_part = nullptr, *dkv_part = nullptr;
     if (deal && workspace_bytes >= slapo_amd_attn_bwd_ex_workspace_bytes(prm)) {
-        splits = plan_splits(prm);
+        splits = plan_splits(prm, true);
         float* next = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(prm));
         if (splits.dq > 1) {
             dq_part = next;

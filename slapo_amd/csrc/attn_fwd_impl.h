@@ -18,6 +18,8 @@
 // more latency than a deeper pipeline inside one wavefront does: a pipelined variant with twice
 // the registers measured 12 % slower at head_dim 64 and 35-80 % slower at 80 / 128.
 //
+// Launches that leave CUs idle take workgroups of 64 or 32 queries whose wavefronts share the keys (kGroups).
+//
 // Reference semantics: slapo/op/attention.py:163-181 (attention_bmk), :97-131 (flash_attn_ref).
 #pragma once
 #include <type_traits>

@@ -137,7 +137,8 @@ namespace slapo {
 // forward 49 -> 29 us, forward + backward 206 -> 109 us; at B2 S1024 H8 D64 the same split costs
 // (forward 19 -> 26 us).  fp32 B1 S1971 H2 D72 forward + backward 629 -> 170 us.
 // Under a causal mask the blocks have half the longest one's tiles on average, so that even a launch
-// with a workgroup for every CU gains from two shares (bf16 B1 S8192 H4 D64: 378 -> 315 us).
+// with a workgroup for every CU gains from two shares (bf16 B1 S8192 H4 D128 backward 457 -> 339 us; where
+// groups of wavefronts or the one-launch backward apply they take the place of two, attn_capi.hip).
 int attn_splits(int64_t blocks, int64_t cus, int64_t tiles, bool f32, bool causal) {
     const int64_t slots = f32 ? 2 * cus : cus, least = f32 ? 4 : 6;
     if (blocks <= 0 || tiles < (f32 ? 12 : 24)) return 1;
