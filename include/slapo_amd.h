@@ -283,7 +283,11 @@ int slapo_amd_attn_fwd(const slapo_attn_params* prm, const void* q, const void* 
  * several workgroups, whose partial results meet there; with a smaller one or none every block of
  * rows keeps to one workgroup. */
 #define SLAPO_BIAS_PREPARED 3
+#define SLAPO_BIAS_NONE (-1)
 size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm);
+/* What the call needs with this type of bias (SLAPO_BIAS_NONE: with none) and no more; the function
+ * above answers for the type that needs most. */
+size_t slapo_amd_attn_fwd_workspace_bytes_for(const slapo_attn_params* prm, int bias_type);
 int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
                           const void* v, const void* bias, int bias_type, void* o, float* lse,
                           void* workspace, size_t workspace_bytes, void* stream);
@@ -316,6 +320,9 @@ int slapo_amd_attn_bwd(const slapo_attn_params* prm, const void* q, const void* 
  * the sums of such a call are formed in another order than slapo_amd_attn_bwd's, which deals nothing
  * whatever its workspace holds. */
 size_t slapo_amd_attn_bwd_ex_workspace_bytes(const slapo_attn_params* prm);
+/* What the call needs with this type of bias (SLAPO_BIAS_NONE: with none) and, with dropout, with the
+ * keep bits in prm or without: calls that run as one launch need only delta. */
+size_t slapo_amd_attn_bwd_ex_workspace_bytes_for(const slapo_attn_params* prm, int bias_type);
 int slapo_amd_attn_bwd_ex(const slapo_attn_params* prm, const void* q, const void* k,
                           const void* v, const void* bias, int bias_type, const void* o,
                           const void* dout, const float* lse, void* dq, void* dk, void* dv,

@@ -134,6 +134,8 @@ PROTOTYPES = {
         ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp]
     ),
     "slapo_amd_attn_fwd_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
+    "slapo_amd_attn_fwd_workspace_bytes_for": (ctypes.c_size_t, [ctypes.POINTER(AttnParams),
+                                                                 ctypes.c_int]),
     "slapo_amd_attn_fwd_ex": (
         ctypes.c_int, [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, ctypes.c_int, c_vp,
                        c_vp, c_vp, ctypes.c_size_t, c_vp]
@@ -144,6 +146,8 @@ PROTOTYPES = {
                        c_vp, c_vp]
     ),
     "slapo_amd_attn_bwd_ex_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(AttnParams)]),
+    "slapo_amd_attn_bwd_ex_workspace_bytes_for": (ctypes.c_size_t, [ctypes.POINTER(AttnParams),
+                                                                    ctypes.c_int]),
     "slapo_amd_attn_bwd_ex": (
         ctypes.c_int,
         [ctypes.POINTER(AttnParams), c_vp, c_vp, c_vp, c_vp, ctypes.c_int, c_vp, c_vp, c_vp, c_vp,

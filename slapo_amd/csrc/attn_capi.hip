@@ -1,5 +1,6 @@
 // C-ABI entry points of the attention path: argument validation, kernel selection (MFMA kernels
 // for fp16 / bf16 and for fp32) and the kernel that draws dropout masks ahead of the forward.
+#include <algorithm>
 #include <mutex>
 
 #include "attn_common.h"
@@ -272,58 +273,133 @@ int decode_shares(const slapo_attn_params* p) {
 
 namespace {
 
-// Splits of the three kernels of a call (attn_splits), for the current device.
-struct Splits {
-    int fwd = 1, dq = 1, dkv = 1;
+BiasKind bias_kind(const slapo_attn_params* p, int bias_type) {
+    if (bias_type == SLAPO_BIAS_NONE) return kNoBias;
+    if (bias_type == SLAPO_BIAS_PREPARED) return kPreparedBias;
+    return p->seqlen_q == 1 || p->bias_strides[2] == 0 ? kKeyBias : kScoreBias;
+}
+BiasKind bias_kind(const slapo_attn_params* p, const AttnArgs& a) {
+    return bias_kind(p, a.has_bias ? a.bias_type : SLAPO_BIAS_NONE);
+}
+
+// Row blocks and tiles of a call, for the current device.
+struct Extent {
+    int64_t cus, blocks_q, blocks_k, tiles_q, tiles_k;
+    bool f32, causal;
+    explicit Extent(const slapo_attn_params* p) {
+        cus = cus_of_current_device();
+        f32 = p->dtype == SLAPO_F32;
+        causal = p->causal && p->window <= 0;
+        const int64_t n_bh = (int64_t)p->batch * p->heads, rows = f32 ? 64 : 128, tile = f32 ? 32 : 64;
+        auto blocks = [&](int64_t n) { return n_bh * ((n + rows - 1) / rows); };
+        auto tiles = [&](int64_t n) {
+            return ((p->window > 0 && p->window + rows < n ? p->window + rows : n) + tile - 1) / tile;
+        };
+        blocks_q = blocks(p->seqlen_q), blocks_k = blocks(p->seqlen_k);
+        tiles_q = tiles(p->seqlen_q), tiles_k = tiles(p->seqlen_k);
+    }
+    static bool known(const slapo_attn_params* p) {
+        return p && p->batch > 0 && p->heads > 0 && p->seqlen_q > 0 && p->seqlen_k > 0 && p->head_dim > 0;
+    }
 };
-// grouped: the forward can be divided into groups of wavefronts (every build but the one that reads a bias
-// of any layout per score).
-Splits plan_splits(const slapo_attn_params* p, bool grouped) {
-    Splits s;
-    if (!p || p->batch <= 0 || p->heads <= 0 || p->seqlen_q <= 0 || p->seqlen_k <= 0 ||
-        p->head_dim <= 0)
-        return s;
-    const int64_t cus = cus_of_current_device();
-    const bool f32 = p->dtype == SLAPO_F32;
-    const int64_t n_bh = (int64_t)p->batch * p->heads, rows = f32 ? 64 : 128, tile = f32 ? 32 : 64;
-    auto blocks = [&](int64_t n) { return n_bh * ((n + rows - 1) / rows); };
-    auto tiles = [&](int64_t n) {
-        return ((p->window > 0 && p->window + rows < n ? p->window + rows : n) + tile - 1) / tile;
-    };
-    const bool causal = p->causal && p->window <= 0;
-    s.fwd = s.dq = attn_splits(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), f32, causal);
-    // (groups of wavefronts in a workgroup do the same without partial results in memory)
-    const int groups = f32 || !grouped
-                           ? 1
-                           : attn_fwd_groups(blocks(p->seqlen_q), cus, tiles(p->seqlen_k), p->head_dim,
-                                             causal);
-    if (groups > 1 && s.fwd <= groups && !(p->head_dim > 64 && tiles(p->seqlen_k) > 40)) s.fwd = 1;
-    s.dkv = attn_splits(blocks(p->seqlen_k), cus, tiles(p->seqlen_q), f32, causal);
-    return s;
+
+// Into how many shares the forward of a call deals the tiles of a row block.
+int plan_forward(const slapo_attn_params* p, BiasKind kind) {
+    const Extent e(p);
+    const int shares = attn_splits(e.blocks_q, e.cus, e.tiles_k, e.f32, e.causal);
+    if (e.f32 || kind == kScoreBias) return shares;
+    // groups of wavefronts in a workgroup do the same without partial results in memory
+    const int groups = attn_fwd_groups(e.blocks_q, e.cus, e.tiles_k, p->head_dim, e.causal);
+    if (groups > 1 && shares <= groups && !(p->head_dim > 64 && e.tiles_k > 40)) return 1;
+    return shares;
+}
+size_t forward_bytes(const slapo_attn_params* p, BiasKind kind) {
+    const size_t shares = plan_forward(p, kind);
+    return shares == 1 ? 0
+                       : shares * p->batch * p->heads * p->seqlen_q * (2 + p->head_dim) * sizeof(float);
+}
+
+// Whether a backward runs as one launch (attn_bwd_both_impl.h): while the workgroups of both kernels
+// together are fewer than two such launches would keep resident.  Device time of the backward, two
+// launches -> delta_kernel and one: bf16 B4 S512 H8 D64 (256 workgroups) 25.4 -> 18.6 us, B6 S1187 H4
+// D64 causal (480) 48.5 -> 36.3, B2 S1024 H12 D80 causal (384) 61.9 -> 40.8, B8 S512 H12 D64 (768) 39.9
+// -> 38.1; B8 S1024 H8 D64 (1024) 71.1 -> 69.7, D80 102 -> 104.  At head_dim 128 a CU holds one workgroup
+// of dK/dV: B2 S1024 H12 causal (384) 75.8 -> 51.3, B2 S1024 H16 (512) 82.6 -> 80.9.
+// With a prepared bias, forward and backward at bf16 B2 S1024 H12: D64 97.2 -> 85.0 us, causal 97.7 -> 81.9,
+// D80 causal 140 -> 111, D128 causal 170 -> 108; with stored keep bits as well D128 202 -> 138, but at
+// head_dim 81-96 the one kernel spills (174 -> 263).
+bool one_launch_backward(const slapo_attn_params* p, const Extent& e, BiasKind kind, int dropout) {
+    if (dropout != 0 && dropout != 3) return false;
+    if (kind == kScoreBias) return false;
+    if (kind == kPreparedBias && dropout && p->head_dim > 80 && p->head_dim <= 96) return false;
+    return e.blocks_q + e.blocks_k < (p->head_dim <= 96 ? 4 : 2) * e.cus;
+}
+
+// How a backward runs: in how many shares each kernel deals its tiles, or as one launch
+// (attn_bwd_both_impl.h), which deals none.
+struct BackwardPlan {
+    int dq = 1, dkv = 1;
+    bool one_launch = false;
+};
+// dropout: as in AttnArgs.  deal: whether there is room for partial results.
+BackwardPlan plan_backward(const slapo_attn_params* p, BiasKind kind, int dropout, bool deal) {
+    const Extent e(p);
+    BackwardPlan plan;
+    if (deal) {
+        plan.dq = attn_splits(e.blocks_q, e.cus, e.tiles_k, e.f32, e.causal);
+        plan.dkv = attn_splits(e.blocks_k, e.cus, e.tiles_q, e.f32, e.causal);
+    }
+    // In two shares the partial results cost more than the one launch, whose two kernels fill each other's
+    // idle CUs.  Backward, two shares / one launch, bf16: B1 S2048 H8 D64 (128 blocks) 68.0 / 49.2 us, H16
+    // causal (256) 89.7 / 57.3, S8192 H4 causal 234 / 189; H16 causal D80 117 / 79.6; H8 D128 112 / 87.4, B2
+    // S1600 H9 D128 causal 119 / 80.3.  In four, with 64 blocks, they do not: S2048 H4 D64 48.8 / 45.8, S4096
+    // H2 64.7 / 82.1, D128 105 / 145.
+    if (!e.f32 && plan.dq <= 2 && plan.dkv <= 2 && one_launch_backward(p, e, kind, dropout)) {
+        plan.dq = plan.dkv = 1;
+        plan.one_launch = true;
+    }
+    return plan;
 }
 size_t delta_bytes(const slapo_attn_params* p) {  // rounded: the partial results follow
     return (slapo_amd_attn_bwd_workspace_bytes(p) + 255) & ~size_t(255);
 }
+size_t backward_bytes(const slapo_attn_params* p, const BackwardPlan& plan) {
+    if (plan.dq == 1 && plan.dkv == 1) return slapo_amd_attn_bwd_workspace_bytes(p);
+    const size_t row = (size_t)p->batch * p->heads * p->head_dim * sizeof(float);
+    return delta_bytes(p) + (plan.dq > 1 ? row * p->seqlen_q * plan.dq : 0) +
+           (plan.dkv > 1 ? 2 * row * p->seqlen_k * plan.dkv : 0);
+}
 
 }  // namespace
 
-extern "C" size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm) {
+extern "C" size_t slapo_amd_attn_fwd_workspace_bytes_for(const slapo_attn_params* prm, int bias_type) {
+    if (!Extent::known(prm)) return 0;
     if (const int shares = decode_shares(prm))
         return shares == 1 ? 0
                            : (size_t)shares * prm->batch * prm->heads * (2 + prm->head_dim) *
                                  sizeof(float);
-    const Splits s = plan_splits(prm, prm && prm->bias_strides[2] == 0);
-    if (s.fwd == 1) return 0;
-    return (size_t)s.fwd * prm->batch * prm->heads * prm->seqlen_q * (2 + prm->head_dim) *
-           sizeof(float);
+    return forward_bytes(prm, bias_kind(prm, bias_type));
+}
+
+extern "C" size_t slapo_amd_attn_bwd_ex_workspace_bytes_for(const slapo_attn_params* prm, int bias_type) {
+    if (!Extent::known(prm)) return slapo_amd_attn_bwd_workspace_bytes(prm);
+    const int dropout = !(prm->p_drop > 0.f) ? 0 : prm->keep_mask ? 3 : 1;
+    return backward_bytes(prm, plan_backward(prm, bias_kind(prm, bias_type), dropout, true));
+}
+
+// Without the type: what is enough for every one of them.
+extern "C" size_t slapo_amd_attn_fwd_workspace_bytes(const slapo_attn_params* prm) {
+    size_t most = 0;
+    for (int type : {SLAPO_BIAS_NONE, SLAPO_F32, SLAPO_BIAS_PREPARED})
+        most = std::max(most, slapo_amd_attn_fwd_workspace_bytes_for(prm, type));
+    return most;
 }
 
 extern "C" size_t slapo_amd_attn_bwd_ex_workspace_bytes(const slapo_attn_params* prm) {
-    const Splits s = plan_splits(prm, true);
-    if (s.dq == 1 && s.dkv == 1) return slapo_amd_attn_bwd_workspace_bytes(prm);
-    const size_t row = (size_t)prm->batch * prm->heads * prm->head_dim * sizeof(float);
-    return delta_bytes(prm) + (s.dq > 1 ? row * prm->seqlen_q * s.dq : 0) +
-           (s.dkv > 1 ? 2 * row * prm->seqlen_k * s.dkv : 0);
+    size_t most = 0;
+    for (int type : {SLAPO_BIAS_NONE, SLAPO_F32, SLAPO_BIAS_PREPARED})
+        most = std::max(most, slapo_amd_attn_bwd_ex_workspace_bytes_for(prm, type));
+    return most;
 }
 
 extern "C" size_t slapo_amd_attn_prepared_bias_bytes(int64_t batch, int64_t heads,
@@ -378,14 +454,13 @@ extern "C" int slapo_amd_attn_fwd_ex(const slapo_attn_params* prm, const void* q
         const bool rows_ok = !f32 || (a.d % 4 == 0 && strides_ok(prm->q_strides, 4) &&
                                       strides_ok(prm->k_strides, 4) &&
                                       strides_ok(prm->v_strides, 4) && half_ptrs_ok({q, k, v}));
-        if (!workspace || workspace_bytes < slapo_amd_attn_fwd_workspace_bytes(prm)) shares = 1;
+        if (!workspace || workspace_bytes < slapo_amd_attn_fwd_workspace_bytes_for(prm, bias_type)) shares = 1;
         if (rows_ok && bias_type != SLAPO_BIAS_PREPARED)
             return attn_decode(a, prm->dtype, shares, static_cast<float*>(workspace), st);
     }
-    const size_t split_bytes = slapo_amd_attn_fwd_workspace_bytes(prm);
-    if (workspace && split_bytes > 0 && workspace_bytes >= split_bytes &&
-        decode_shares(prm) == 0) {
-        a.n_split = plan_splits(prm, !a.has_bias || bias_type != SLAPO_F32 || a.bs[2] == 0).fwd;
+    if (workspace && decode_shares(prm) == 0) {
+        const BiasKind kind = bias_kind(prm, a);
+        if (workspace_bytes >= forward_bytes(prm, kind)) a.n_split = plan_forward(prm, kind);
         a.part = static_cast<float*>(workspace);
     }
     auto merged = [&](int status) {
@@ -421,27 +496,6 @@ extern "C" size_t slapo_amd_attn_bwd_workspace_bytes(const slapo_attn_params* pr
 }
 
 namespace {
-// Whether a backward runs as one launch (attn_bwd_both_impl.h): while the workgroups of both kernels
-// together are fewer than two such launches would keep resident.  Device time of the backward, two
-// launches -> delta_kernel and one: bf16 B4 S512 H8 D64 (256 workgroups) 25.4 -> 18.6 us, B6 S1187 H4
-// D64 causal (480) 48.5 -> 36.3, B2 S1024 H12 D80 causal (384) 61.9 -> 40.8, B8 S512 H12 D64 (768) 39.9
-// -> 38.1; B8 S1024 H8 D64 (1024) 71.1 -> 69.7, D80 102 -> 104.  At head_dim 128 a CU holds one workgroup
-// of dK/dV: B2 S1024 H12 causal (384) 75.8 -> 51.3, B2 S1024 H16 (512) 82.6 -> 80.9.
-// With a prepared bias, forward and backward at bf16 B2 S1024 H12: D64 97.2 -> 85.0 us, causal 97.7 -> 81.9,
-// D80 causal 140 -> 111, D128 causal 170 -> 108; with stored keep bits as well D128 202 -> 138, but at
-// head_dim 81-96 the one kernel spills (174 -> 263).
-bool one_launch_backward(const AttnArgs& a) {
-    if (a.dropout != 0 && a.dropout != 3) return false;
-    if (a.has_bias && a.bias_type == SLAPO_BIAS_PREPARED) {
-        if (a.dropout && a.d > 80 && a.d <= 96) return false;
-    } else if (a.has_bias && (a.bias_type != SLAPO_F32 || a.bs[2] != 0)) {
-        return false;
-    }
-    const int64_t n_bh = (int64_t)a.batch * a.heads;
-    const int64_t blocks = n_bh * (((int64_t)a.sq + 127) / 128 + ((int64_t)a.sk + 127) / 128);
-    return blocks < (int64_t)(a.d <= 96 ? 4 : 2) * a.n_cus;
-}
-
 int run_backward(const slapo_attn_params* prm, const void* q, const void* k, const void* v,
                  const void* bias, int bias_type, const void* o, const void* dout,
                  const float* lse, void* dq, void* dk, void* dv, const int64_t dq_strides[3],
@@ -479,45 +533,41 @@ int run_backward(const slapo_attn_params* prm, const void* q, const void* k, con
             return SLAPO_ERR_ALIGN;
     }
     // Partial results need room.  Both kernels' are merged in one launch at the end.
-    Splits splits;
+    BackwardPlan plan;
     float *dq_part = nullptr, *dkv_part = nullptr;
-    if (deal && workspace_bytes >= slapo_amd_attn_bwd_ex_workspace_bytes(prm)) {
-        splits = plan_splits(prm, true);
+    if (deal) {
+        const BiasKind kind = bias_kind(prm, a);
+        plan = plan_backward(prm, kind, a.dropout, true);
+        if (workspace_bytes < backward_bytes(prm, plan)) plan = plan_backward(prm, kind, a.dropout, false);
         float* next = reinterpret_cast<float*>(static_cast<char*>(workspace) + delta_bytes(prm));
-        if (splits.dq > 1) {
+        if (plan.dq > 1) {
             dq_part = next;
-            next += (int64_t)splits.dq * a.batch * a.heads * a.sq * a.d;
+            next += (int64_t)plan.dq * a.batch * a.heads * a.sq * a.d;
         }
-        if (splits.dkv > 1) dkv_part = next;
+        if (plan.dkv > 1) dkv_part = next;
     }
 
-    // In two shares the partial results cost more than the one launch, whose two kernels fill each other's
-    // idle CUs.  Backward, two shares / one launch, bf16: B1 S2048 H8 D64 (128 blocks) 68.0 / 49.2 us, H16
-    // causal (256) 89.7 / 57.3, S8192 H4 causal 234 / 189; H16 causal D80 117 / 79.6; H8 D128 112 / 87.4, B2
-    // S1600 H9 D128 causal 119 / 80.3.  In four, with 64 blocks, they do not: S2048 H4 D64 48.8 / 45.8, S4096
-    // H2 64.7 / 82.1, D128 105 / 145.
-    if (deal && !f32 && stages == SLAPO_BWD_ALL && splits.dq <= 2 && splits.dkv <= 2 &&
-        one_launch_backward(a))
+    if (plan.one_launch)
         return prm->dtype == SLAPO_F16 ? attn_bwd_both_mfma_f16(a, st)
                                        : attn_bwd_both_mfma_bf16(a, st);
     // PREPARE has nothing to do (the dQ kernel computes delta for its own rows and stores it for
     // the dK / dV kernel), so DQ runs before DKDV.
     if (stages & SLAPO_BWD_DQ) {
-        a.n_split = splits.dq, a.part = dq_part;
+        a.n_split = plan.dq, a.part = dq_part;
         rc = f32                        ? attn_bwd_dq_f32(a, st)
              : prm->dtype == SLAPO_F16 ? attn_bwd_dq_mfma_f16(a, st)
                                        : attn_bwd_dq_mfma_bf16(a, st);
         if (rc != SLAPO_OK) return rc;
     }
     if (stages & SLAPO_BWD_DKDV) {
-        a.n_split = splits.dkv, a.part = dkv_part;
+        a.n_split = plan.dkv, a.part = dkv_part;
         rc = f32                        ? attn_bwd_f32(a, st)
              : prm->dtype == SLAPO_F16 ? attn_bwd_mfma_f16(a, st)
                                        : attn_bwd_mfma_bf16(a, st);
         if (rc != SLAPO_OK) return rc;
     }
     return dq_part || dkv_part
-               ? attn_merge_bwd(a, prm->dtype, dq_part, splits.dq, dkv_part, splits.dkv, st)
+               ? attn_merge_bwd(a, prm->dtype, dq_part, plan.dq, dkv_part, plan.dkv, st)
                : SLAPO_OK;
 }
 

@@ -275,6 +275,10 @@ struct AttnArgs {
     float* part;
 };
 
+// How the additive bias of a call reaches the kernels: not at all, as one value per key, laid out by
+// slapo_amd_attn_prepare_bias, or read per score.
+enum BiasKind { kNoBias, kKeyBias, kPreparedBias, kScoreBias };
+
 // Groups of wavefronts that share the key tiles of a 16-bit forward call (attn_split.hip).
 int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal);
 

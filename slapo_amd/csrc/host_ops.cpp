@@ -351,7 +351,8 @@ AttnResult launch_attn_fwd(AttnProblem& a, const Operands& x, at::IntArrayRef ou
             prm.keep_mask = r.keep_mask.mutable_data_ptr();
         }
     }
-    const size_t ws_bytes = slapo_amd_attn_fwd_workspace_bytes(&prm);
+    const size_t ws_bytes =
+        slapo_amd_attn_fwd_workspace_bytes_for(&prm, a.bias.defined() ? a.bias_type : SLAPO_BIAS_NONE);
     const Tensor ws = ws_bytes ? floats((int64_t)(ws_bytes / 4)) : Tensor();
     check(slapo_amd_attn_fwd_ex(&prm, x.ptr[0], x.ptr[1], x.ptr[2], cptr(a.bias), a.bias_type,
                                 mptr(r.out), static_cast<float*>(mptr(r.lse)), mptr(ws), ws_bytes,
@@ -367,7 +368,8 @@ void launch_attn_bwd(AttnProblem& a, const Operands& x, const Tensor& out, const
     Tensor dout = cast(grad, a.dtype).contiguous();
     if (!aligned(dout)) dout = dout.clone();
     a.prm.keep_mask = mptr(keep_mask);
-    const size_t ws_bytes = slapo_amd_attn_bwd_ex_workspace_bytes(&a.prm);
+    const size_t ws_bytes = slapo_amd_attn_bwd_ex_workspace_bytes_for(
+        &a.prm, a.bias.defined() ? a.bias_type : SLAPO_BIAS_NONE);
     const Tensor ws = floats((int64_t)(ws_bytes / 4));
     check(slapo_amd_attn_bwd_ex(&a.prm, x.ptr[0], x.ptr[1], x.ptr[2], cptr(a.bias), a.bias_type,
                                 cptr(out), cptr(dout), static_cast<const float*>(cptr(lse)),

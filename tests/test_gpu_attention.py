@@ -2,6 +2,7 @@
 same seeded inputs, forward and backward.  Bars: fp32 max-abs 1e-5; fp16 / bf16 relative 2e-2
 with dropout off; with dropout on, the mask is torch's own (bit exact) and values follow the
 oracle evaluated with that mask."""
+import ctypes
 import math
 
 import pytest
@@ -968,6 +969,62 @@ def test_backward_forms_agree_where_tiles_could_be_dealt(dtype):
     assert not all(torch.equal(a, r) for a, r in zip(dealt, whole))
     for a, r in zip(dealt, whole):
         assert_parity(a, r, dtype)
+
+
+def _geometry(b, s, h, d, dtype, bias_strides=(0, 0, 0, 0), causal=False, p=0.0, keep=False):
+    """The parameters of a call as the workspace queries read them."""
+    from slapo_amd import _lib
+
+    prm = _lib.AttnParams()
+    prm.dtype, prm.batch, prm.heads, prm.head_dim = _lib.dtype_code(dtype), b, h, d
+    prm.seqlen_q = prm.seqlen_k = s
+    prm.causal, prm.p_drop = int(causal), p
+    prm.bias_strides = (ctypes.c_int64 * 4)(*bias_strides)
+    if keep:
+        prm.keep_mask = 16  # (not read)
+    return prm
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_workspace_is_what_the_plan_uses(dtype):
+    """Calls that could be dealt but run as one launch, or in groups of wavefronts, have no partial
+    results: neither the queries nor the op ask for room for them."""
+    from slapo_amd import _lib
+
+    lib = _lib.load()
+    none, f32, prepared = -1, _lib.SLAPO_F32, 3
+    delta = 2048 * 8 * 4
+
+    def sizes(prm, kind):
+        ref = ctypes.byref(prm)
+        one = (lib.slapo_amd_attn_fwd_workspace_bytes_for(ref, kind),
+               lib.slapo_amd_attn_bwd_ex_workspace_bytes_for(ref, kind))
+        every = (lib.slapo_amd_attn_fwd_workspace_bytes(ref),
+                 lib.slapo_amd_attn_bwd_ex_workspace_bytes(ref))
+        assert one[0] <= every[0] and one[1] <= every[1]
+        return one
+
+    plain = _geometry(1, 2048, 8, 64, dtype)
+    assert sizes(plain, none) == sizes(plain, f32) == (0, delta)
+    assert lib.slapo_amd_attn_bwd_ex_workspace_bytes(ctypes.byref(plain)) == delta
+    rows = _geometry(1, 2048, 8, 64, dtype, (0, 0, 2048, 1))
+    assert sizes(rows, prepared) == (0, delta)
+    fwd, bwd = sizes(rows, f32)  # read per score: neither groups nor the one launch take it
+    assert fwd > 0 and bwd > delta
+    # dropout: the one launch reads stored keep bits
+    assert sizes(_geometry(1, 2048, 8, 64, dtype, p=0.1, keep=True), none)[1] == delta
+    assert sizes(_geometry(1, 2048, 8, 64, dtype, p=0.1), none)[1] > delta
+
+    q, k, v = (torch.randn(1, 8192, 4, 64, dtype=dtype, device="cuda", requires_grad=True)
+               for _ in range(3))
+    out = op.hip_attention(q, k, v, causal=True)
+    do = torch.randn_like(out)
+    torch.autograd.grad(out, (q, k, v), do, retain_graph=True)
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    grads = torch.autograd.grad(out, (q, k, v), do)
+    results = sum(t.numel() * t.element_size() for t in grads)
+    assert torch.cuda.max_memory_allocated() - before <= results + (1 << 20)
 
 
 @pytest.mark.parametrize("shape,sk,causal,window,p", [
