@@ -1027,6 +1027,37 @@ def test_workspace_is_what_the_plan_uses(dtype):
     assert torch.cuda.max_memory_allocated() - before <= results + (1 << 20)
 
 
+@pytest.mark.parametrize("s,h,d,causal,kind,p,dealt", [
+    (8192, 2, 64, False, "key", 0.0, True), (2048, 8, 64, False, "key", 0.0, False),
+    (8192, 3, 128, True, "key", 0.0, True), (4096, 6, 128, True, "key", 0.0, False),
+    (16384, 1, 64, False, None, 0.0, True), (6144, 2, 64, False, None, 0.0, False),
+    (16384, 1, 128, True, None, 0.0, True), (8192, 4, 64, True, None, 0.0, False),
+    (4096, 4, 64, False, "prepared", 0.0, True), (4096, 4, 128, False, "prepared", 0.0, False),
+    (2432, 6, 96, False, "key", 0.1, True), (2048, 8, 128, False, "key", 0.1, False),
+    (1600, 9, 80, False, "prepared", 0.1, True),
+    (8192, 4, 64, True, "key", 0.1, False), (8192, 4, 80, True, "key", 0.1, True),
+    (2048, 12, 96, True, "key", 0.1, False), (2048, 6, 96, True, "key", 0.1, True),
+])
+def test_long_backward_calls_are_dealt_again(s, h, d, causal, kind, p, dealt):
+    """Two shares of the tiles against one launch: the latter up to a length that masks, dropout and the
+    number of blocks decide."""
+    from slapo_amd import _lib
+
+    prm = _geometry(1, s, h, d, torch.bfloat16, (0, 0, s if kind == "prepared" else 0, 1), causal, p, p > 0)
+    code = {None: -1, "key": _lib.SLAPO_F32, "prepared": 3}[kind]
+    size = _lib.load().slapo_amd_attn_bwd_ex_workspace_bytes_for(ctypes.byref(prm), code)
+    assert (size > h * s * 4) == dealt
+
+
+@pytest.mark.parametrize("layout", [None, "padding"])
+@pytest.mark.parametrize("s,h,d", [(4160, 3, 64), (3136, 4, 128)])
+def test_backward_in_two_shares_beside_padding(s, h, d, layout):
+    """65 and 49 tiles: with a padding mask dealt to two shares, without one in one launch."""
+    q, k, v, do, g = _inputs(1, s, h, d, torch.bfloat16)
+    mask = None if layout is None else _padding_mask(1, s, torch.bfloat16, g, s // 2)[0]
+    _check(q, k, v, do, mask, False, 0, torch.bfloat16)
+
+
 @pytest.mark.parametrize("shape,sk,causal,window,p", [
     ((1, 1, 2, 20), 33, False, 0, 0.0),       # one query, head_dim no multiple of four
     ((1, 15, 1, 72), 16, True, 0, 0.0),       # less than a wavefront's rows
