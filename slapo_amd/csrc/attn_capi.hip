@@ -308,10 +308,21 @@ int plan_forward(const slapo_attn_params* p, BiasKind kind) {
     const Extent e(p);
     const int shares = attn_splits(e.blocks_q, e.cus, e.tiles_k, e.f32, e.causal);
     if (e.f32 || kind == kScoreBias) return shares;
-    // groups of wavefronts in a workgroup do the same without partial results in memory
-    const int groups = attn_fwd_groups(e.blocks_q, e.cus, e.tiles_k, p->head_dim, e.causal);
-    if (groups > 1 && shares <= groups && !(p->head_dim > 64 && e.tiles_k > 40)) return 1;
-    return shares;
+    // Groups of wavefronts in a workgroup do the same without partial results in memory.  (Which dropout it is
+    // matters to calls of few tiles only, which are not dealt.)
+    const int groups = attn_fwd_groups(e.blocks_q, e.cus, e.tiles_k, p->head_dim, e.causal, kind,
+                                       p->p_drop > 0.f ? 1 : 0);
+    if (groups == 1 || shares > groups) return shares;
+    // Dealt all the same, above head_dim 64: beyond 40 tiles, where the merge is the smaller part, and, above 96,
+    // where two groups read a bias for one workgroup a CU (dealt / two groups: causal B1 S2048 H16 with a padding
+    // mask 51.2 / 53.2 us, p 0.1 74.5 / 77.7, without a mask 56.1 / 47.5; H8 with a [B,1,Sq,Sk] mask 54.1 / 60.8, causal
+    // 50.8 / 57.9, with p 0.1 both the same).
+    if (p->head_dim > 64 && e.tiles_k > 40) return shares;
+    const bool half = 2 * e.blocks_q <= e.cus;
+    if (p->head_dim > 96 && groups == 2 &&
+        (kind == kKeyBias ? !half : kind == kPreparedBias && half && !(p->p_drop > 0.f)))
+        return shares;
+    return 1;
 }
 size_t forward_bytes(const slapo_attn_params* p, BiasKind kind) {
     const size_t shares = plan_forward(p, kind);

@@ -280,7 +280,8 @@ struct AttnArgs {
 enum BiasKind { kNoBias, kKeyBias, kPreparedBias, kScoreBias };
 
 // Groups of wavefronts that share the key tiles of a 16-bit forward call (attn_split.hip).
-int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal);
+int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal, BiasKind bias,
+                    int dropout);
 
 // The share of tiles [t_lo, t_hi) that number `split` of n_split takes.
 __device__ __forceinline__ void split_tiles(int n_split, int split, int& t_lo, int& t_hi) {

@@ -686,9 +686,10 @@ int launch(const AttnArgs& a, hipStream_t st) {
     if (blocks <= 0 || blocks > 0x7FFFFFFF) return SLAPO_ERR_SHAPE;
     if constexpr (kGroups == 1 && kBias != 1) {
         const int64_t keys = a.window > 0 ? min(a.sk, a.window + kBM) : a.sk;
+        constexpr BiasKind kKind = kBias == 0 ? kNoBias : kBias == 3 ? kPreparedBias : kKeyBias;
         const int groups = a.n_split > 1 ? 1
                                          : attn_fwd_groups(blocks, a.n_cus, (keys + kBN - 1) / kBN, a.d,
-                                                           a.causal && a.window <= 0);
+                                                           a.causal && a.window <= 0, kKind, kDrop);
         if (groups == 4)
             return launch<T, DPAD, kBias, kDrop, kSteps, group_per_cu(4, DPAD, kBias), 4>(a, st);
         if (groups == 2)

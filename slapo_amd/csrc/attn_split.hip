@@ -164,18 +164,28 @@ int attn_splits(int64_t blocks, int64_t cus, int64_t tiles, bool f32, bool causa
 //   D128  B1 S256 H16 (32) 9.9 / 10.4 / 9.9, S1024 H8 (64) 26.2 / 23.2 / 18.8, H16 (128) 27.2 / 24.9 / 34.8,
 //         H32 causal (256) 27.7 / 31.7 / 49.8, S2048 H16 causal (256) 56.1 / 47.5 / 68.1
 // Below six tiles there is nothing to divide (B1 S256 H16 D64 7.2 / 7.0 / 6.8).
-int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal) {
+// A prepared bias is read from memory by every workgroup, a second one per CU only where the chip has room:
+// without drawn dropout two groups lose where it has little (undivided / two groups: D64 B1 S1024 H32 23.8 / 27.2,
+// S8192 H4 197 / 227; D96 causal B4 S512 H16 17.8 / 22.1, B3 S777 H12 24.8 / 27.1, but B1 S1472 H16 (192 blocks)
+// 37.9 / 31.6).  A padding mask leaves fewer tiles than the keys have (D128 B1 S512 H8, five of eight tiles valid,
+// 12.6 / 13.6 / 13.5); drawing keep bits is worth dividing all the same (there 21.0 / - / 15.6).
+int attn_fwd_groups(int64_t blocks, int64_t cus, int64_t tiles, int64_t d, bool causal, BiasKind bias,
+                    int dropout) {
     if (cus <= 0 || blocks > cus || tiles < 6) return 1;
     const bool half = 2 * blocks <= cus, quarter = 4 * blocks <= cus;
+    const bool rows = bias == kPreparedBias, drawn = dropout == 1 || dropout == 2;
     if (d <= 64) {
         if (quarter || (half && causal)) return 4;
+        if (rows && !dropout && !half && !causal) return 1;
         return half || causal || tiles >= 16 ? 2 : 1;
     }
     if (d <= 96) {
         if (quarter && tiles >= 16) return 4;
+        if (rows && !drawn && 4 * blocks > 3 * cus && tiles + (dropout != 0) <= 16)
+            return 1;
         return half || causal ? 2 : 1;
     }
-    if (quarter) return tiles >= 8 ? 4 : 1;
+    if (quarter) return tiles >= (bias == kKeyBias && !drawn ? 12 : 8) ? 4 : 1;
     return tiles >= (half ? 8 : 24) && (half || causal) ? 2 : 1;
 }
 

@@ -595,6 +595,49 @@ def test_forward_in_groups_of_wavefronts(shape, sk, causal, window, p, mask):
     _check(q, k, v, do, m, causal, window, torch.bfloat16, p)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,sk,causal", [
+    ((1, 1100, 3, 80), 1100, False),   # four groups
+    ((1, 1100, 3, 96), 1030, True),
+    ((1, 800, 4, 128), 800, False),
+    ((2, 330, 2, 32), 397, False),
+    ((1, 700, 12, 64), 700, False),    # two groups
+    ((1, 330, 3, 80), 400, False),
+    ((1, 513, 17, 96), 513, True),
+    ((1, 641, 13, 128), 577, True),
+])
+def test_forward_in_groups_with_a_16_bit_key_mask(dtype, shape, sk, causal):
+    """At inference a padding mask is read in its own type, by builds of their own; in training as fp32."""
+    q, k, v, _, g = _inputs(*shape, dtype, sk=sk)
+    mask, _ = _padding_mask(shape[0], sk, dtype, g, sk // 3)
+    mask[..., 1:9] = torch.randn(8, generator=g).to(dtype)
+    with torch.no_grad():
+        out = op.hip_attention(q.cuda(), k.cuda(), v.cuda(), mask.cuda(), causal=causal)
+    train = op.hip_attention(q.cuda().requires_grad_(), k.cuda(), v.cuda(), mask.cuda(), causal=causal)
+    want = OA.attention_fwd_bwd(q, k, v, torch.zeros_like(q), mask, causal, 0, 0.0, None, None,
+                                torch.float64)[0]
+    assert_parity(out, want, dtype, "inference")
+    assert_parity(train, want, dtype, "training")
+
+
+@pytest.mark.parametrize("b,s,h,d,causal,mask", [
+    (1, 1024, 32, 64, False, "square"), (1, 1024, 32, 32, False, "square"),
+    (4, 512, 16, 96, True, "square"), (4, 512, 16, 80, True, "square"),
+    (1, 512, 8, 128, False, "key"), (1, 512, 8, 128, True, "key"),
+])
+def test_forward_calls_that_stay_undivided(b, s, h, d, causal, mask):
+    """Masked calls for which groups of wavefronts do not pay: the bits of a launch of many blocks."""
+    q, k, v, _, g = _inputs(b, s, h, d, torch.bfloat16)
+    m = (_padding_mask(b, s, torch.bfloat16, g, s // 2)[0] if mask == "key"
+         else torch.randn(b, 1, s, s, generator=g).to(torch.bfloat16))
+    q, k, v, m = (t.cuda() for t in (q, k, v, m))
+    n = 256 // (b * h * -(-s // 128)) + 1
+    with torch.no_grad():
+        one = op.hip_attention(q, k, v, m, causal=causal)
+        many = op.hip_attention(*(t.repeat(n, 1, 1, 1) for t in (q, k, v, m)), causal=causal)
+    assert torch.equal(one, many[:b])
+
+
 @pytest.mark.parametrize("rest", ["padded", "soft", "hole"])
 @pytest.mark.parametrize("sq,sk,d,causal,window,zeros", [
     (130, 200, 64, False, 0, 0),      # no key without a bias
@@ -1038,7 +1081,7 @@ def test_workspace_is_what_the_plan_uses(dtype):
     (8192, 4, 64, True, "key", 0.1, False), (8192, 4, 80, True, "key", 0.1, True),
     (2048, 12, 96, True, "key", 0.1, False), (2048, 6, 96, True, "key", 0.1, True),
 ])
-def test_long_backward_calls_are_dealt_again(s, h, d, causal, kind, p, dealt):
+def test_long_backward_calls_are_dealt(s, h, d, causal, kind, p, dealt):
     """Two shares of the tiles against one launch: the latter up to a length that masks, dropout and the
     number of blocks decide."""
     from slapo_amd import _lib
@@ -1047,6 +1090,22 @@ def test_long_backward_calls_are_dealt_again(s, h, d, causal, kind, p, dealt):
     code = {None: -1, "key": _lib.SLAPO_F32, "prepared": 3}[kind]
     size = _lib.load().slapo_amd_attn_bwd_ex_workspace_bytes_for(ctypes.byref(prm), code)
     assert (size > h * s * 4) == dealt
+
+
+@pytest.mark.parametrize("s,h,d,causal,kind,p,dealt", [
+    (2048, 16, 128, True, "key", 0.0, True), (2048, 8, 128, True, "key", 0.0, False),
+    (2048, 8, 128, False, "prepared", 0.0, True), (2048, 8, 128, False, "prepared", 0.1, False),
+    (2048, 16, 128, True, None, 0.0, False), (2048, 8, 64, False, "prepared", 0.0, False),
+    (2624, 5, 80, False, None, 0.0, True), (2048, 2, 64, False, None, 0.0, True),
+])
+def test_forward_calls_that_are_dealt(s, h, d, causal, kind, p, dealt):
+    """Shares of the tiles for several workgroups against groups of wavefronts in one."""
+    from slapo_amd import _lib
+
+    prm = _geometry(1, s, h, d, torch.bfloat16, (0, 0, s if kind == "prepared" else 0, 1), causal, p)
+    code = {None: -1, "key": _lib.SLAPO_F32, "prepared": 3}[kind]
+    size = _lib.load().slapo_amd_attn_fwd_workspace_bytes_for(ctypes.byref(prm), code)
+    assert (size > 0) == dealt
 
 
 @pytest.mark.parametrize("layout", [None, "padding"])
