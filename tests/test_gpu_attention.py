@@ -1343,7 +1343,8 @@ def test_one_query_with_an_infinite_value_at_the_last_key(dtype):
     ((1, 700, 1, 32), 1600, False, 0, 0.0, "square"),    # per-query mask, more keys than queries
 ])
 def test_few_rows_dealt_to_many_workgroups(dtype, shape, sk, causal, window, p, layout):
-    """Calls too small to fill the device: partial results of shares of the tiles, merged."""
+    """Calls too small to fill the device: the backward, and in fp32 the forward, as partial results of
+    shares of the tiles, merged; the 16-bit forward in four groups of wavefronts."""
     q, k, v, do, g = _inputs(*shape, dtype, sk=sk)
     mask = None
     if layout == "padding":
@@ -1356,9 +1357,10 @@ def test_few_rows_dealt_to_many_workgroups(dtype, shape, sk, causal, window, p, 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("causal", [False, True])
 def test_nan_keys_reach_every_row_that_sees_them(dtype, causal):
-    """Dealt tiles: a share whose visible scores are all NaN has no maximum and still counts.  One
+    """Divided tiles: a share whose visible scores are all NaN has no maximum and still counts.  One
     key at a time, the first of every share of every block among them, and whole shares; the call
-    without a workspace, which deals nothing, gives the same."""
+    without a workspace gives the same.  (fp32 deals the shares to workgroups where there is one; the
+    16-bit types take groups of wavefronts either way.)"""
     from slapo_amd.op import _kernels as K
     s, d = 1536, 64
     q, k, v, _, _ = _inputs(1, s, 1, d, dtype)
@@ -1371,6 +1373,60 @@ def test_nan_keys_reach_every_row_that_sees_them(dtype, causal):
         alone = K.attn_fwd(q, bad, v, None, causal, 0, d ** -0.5, 0.0, 0, 0, None)[0]
         for out in (dealt, alone):
             assert torch.equal(out.isnan(), sees.expand_as(out)), (lo, hi)
+
+
+def _forward_room(shape, sk, dtype, mask, causal, window, p):
+    """Bytes of partial results that the forward of a call writes: 0 unless it is dealt."""
+    from slapo_amd import _lib
+
+    prm = _geometry(*shape, dtype, (0, 0, 0 if mask is None or mask.shape[2] == 1 else 64, 1), causal, p)
+    prm.seqlen_k, prm.window = sk or shape[1], window
+    kind = -1 if mask is None else _lib.SLAPO_F32 if mask.shape[2] == 1 else 3
+    return _lib.load().slapo_amd_attn_fwd_workspace_bytes_for(ctypes.byref(prm), kind)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,sk,causal,window,p,layout", [
+    ((1, 1920, 1, 64), None, True, 0, 0.0, None),        # fewest tiles, causal: unequal shares
+    ((1, 1921, 1, 128), None, False, 0, 0.0, None),      # one row in the last block
+    ((1, 1924, 2, 72), None, True, 0, 0.1, "padding"),   # padded keys: shares that hold nothing else
+    ((1, 2100, 1, 80), None, True, 1800, 0.1, None),     # local window
+    ((1, 700, 1, 32), 1930, False, 0, 0.0, "square"),    # per-query mask, more keys than queries
+    ((1, 300, 3, 128), 2700, False, 0, 0.1, "square"),   # ... above 40 tiles
+    ((1, 2625, 5, 96), None, True, 0, 0.0, "padding"),   # two shares
+])
+def test_forward_dealt_to_many_workgroups(dtype, shape, sk, causal, window, p, layout):
+    """The 16-bit forward where it writes partial results, which a kernel of their own merges."""
+    q, k, v, do, g = _inputs(*shape, dtype, sk=sk)
+    mask = None
+    if layout == "padding":
+        mask, _ = _padding_mask(shape[0], shape[1], dtype, g, shape[1] // 4)
+    elif layout == "square":
+        mask = torch.randn(1, 1, shape[1], sk, generator=g)
+        mask[:, :, 5, : sk // 2] = torch.finfo(dtype).min  # (shares of nothing but masked keys)
+        mask = mask.to(dtype)
+    assert _forward_room(shape, sk, dtype, mask, causal, window, p) > 0
+    _check(q, k, v, do, mask, causal, window, dtype, p=p)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,causal,layout", [(64, False, None), (64, True, "square"), (128, True, None),
+                                             (128, False, "square"), (80, True, "key")])
+def test_nan_keys_in_a_dealt_forward(dtype, d, causal, layout):
+    """Five shares of six tiles: single NaN keys and shares of nothing else reach every row that sees
+    them through the merge of partial results."""
+    s = 1920
+    q, k, v, _, g = _inputs(1, s, 1, d, dtype)
+    mask = None if layout is None else torch.randn(1, 1, s if layout == "square" else 1, s,
+                                                   generator=g).to(dtype).cuda()
+    assert _forward_room((1, s, 1, d), None, dtype, mask, causal, 0, 0.0) > 0
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    for lo, hi in [(j, j + 1) for j in range(0, s, 96)] + [(0, 384), (768, 1152), (0, s)]:
+        bad = k.clone()
+        bad[:, lo:hi] = float("nan")
+        sees = (torch.arange(s, device="cuda") >= (lo if causal else 0)).view(1, s, 1, 1)
+        out = op.hip_attention(q, bad, v, mask, causal=causal)
+        assert torch.equal(out.isnan(), sees.expand_as(out)), (lo, hi)
 
 
 @pytest.mark.parametrize("causal", [False, True])
