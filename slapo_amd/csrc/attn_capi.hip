@@ -350,8 +350,8 @@ bool one_launch_backward(const slapo_attn_params* p, const Extent& e, BiasKind k
 // other's idle CUs and write no partial results, but it lasts as long as an undivided dK/dV block: what it
 // saves (the partial results and their merge, 12 to 35 us) does not grow with the length, what it costs
 // does, and more so where the blocks differ (keys that are padded) or a tile takes longer.  Where two of its
-// workgroups share a CU, above half as many blocks as CUs, the line lies twice as far out, and four times
-// where nearly all CUs have two.  Backward, two shares / one launch, bf16, B1:
+// workgroups share a CU, above half as many blocks as CUs, the line lies twice as far out, and farther where
+// nearly all CUs have two.  Backward, two shares / one launch, bf16, B1:
 //   S2048 H8 (128 blocks, 32 tiles)  D64 66.7 / 49.8 us, padded keys 64.4 / 52.3, [B,1,Sq,Sk] 82.9 / 76.8, p 0.1
 //                                    72.2 / 58.6; D80 85.6 / 65.7; D128 109 / 83.1, padded keys 91.5 / 81.2
 //   S4096 H4 (128, 64 tiles)         D64 99.2 / 86.0, all keys valid 1 / 0.89, padded 1 / 0.97 to 1, [B,1,Sq,Sk]
@@ -359,26 +359,26 @@ bool one_launch_backward(const slapo_attn_params* p, const Extent& e, BiasKind k
 //                                    [B,1,Sq,Sk] 1 / 0.87
 //   S8192 H2 (128, 128 tiles)        D64 160 / 157, D80 236 / 239, D128 297 / 294; p 0.1 D64 1 / 1.06, D128 1 / 0.92;
 //                                    padded 1 / 1.13 to 1.25
-//   S16384 H1 (128, 256 tiles)       D64 274 / 287, D80 406 / 428, D128 519 / 539; padded 1 / 1.22 to 1.38
+//   S16384 H1 (128, 256 tiles)       D32 1 / 0.96, D64 274 / 287, D80 406 / 428, D128 519 / 539; padded 1 / 1.22 to 1.38
 //   causal, 192 blocks               S4096 H6 D64 105 / 89.1, padded 1 / 0.89; S8192 H3 171 / 163, padded 1 / 1.02
 //   causal, 256 blocks               S2048 H16 D64 86.8 / 55.0, D80 110 / 74.4; S8192 H4 D64 217 / 175, padded 1 /
 //                                    0.89, p 0.1 1 / 0.80, both 1 / 0.92
 // With dropout at head_dim 65 to 96 the two kernels have builds of their own for few blocks, which the one launch
-// has not: its line lies nearer (192 blocks causal, D96: p 0.1 64 tiles 1 / 1.07; with padded keys as well 32 tiles
-// 1 / 0.95, 64 1 / 1.13, and 96 blocks, 32 tiles, 1 / 1.06), with a prepared bias there is none (D80 25 tiles 1 /
-// 1.03).  In three and four shares, whose line would lie
-// below 32 tiles, nothing is replaced: S2048 H5 (80 blocks) D64 48.5 / 46.2, D80 66.4 / 68.6; H4 (64) D64 49.5 / 45.6,
-// D80 57.6 / 62.9, S4096 H2 D64 62.3 / 78.6.
-int64_t one_launch_tiles(const slapo_attn_params* p, const Extent& e, BiasKind kind, int dropout) {
-    // [head_dim][dropout][bias: none, per key, prepared]
-    static constexpr int kTiles[3][2][3] = {{{128, 64, 40}, {64, 40, 32}},
-                                            {{128, 48, 40}, {48, 26, 0}},
-                                            {{128, 48, 96}, {128, 48, 40}}};
-    const int width = p->head_dim <= 64 ? 0 : p->head_dim <= 96 ? 1 : 2;
-    const int64_t blocks = e.blocks_q + e.blocks_k;
-    int times = 4 * blocks > 7 * e.cus ? 4 : blocks > e.cus ? 2 : 1;
-    if (width == 1 && dropout) times = kind != kNoBias ? std::min(times, 2) : times == 2 ? 1 : times;
-    return times * kTiles[width][dropout != 0][kind];
+// has not: its line lies nearer (D80 causal, two shares / one launch: p 0.1 S3072 H7 (168 blocks) 1 / 0.95, H10
+// (240) 1 / 0.83; with padded keys S2048 H12 (192) 1 / 0.92, S3072 H7 1 / 1.07; with a [B,1,Sq,Sk] mask S1536 H18
+// (216) 1 / 0.88, S2048 H12 1 / 1.03).  In three and four shares, whose line would lie below 32 tiles, nothing is
+// replaced: S2048 H5 (80 blocks) D64 48.5 / 46.2, D80 66.4 / 68.6; H4 (64) D64 49.5 / 45.6, D80 57.6 / 62.9, S4096 H2
+// D64 62.3 / 78.6.
+int one_launch_tiles(const slapo_attn_params* p, const Extent& e, BiasKind kind, int dropout) {
+    // [head_dim][dropout][bias: none, per key, prepared][blocks: up to half of the CUs, 0.8, more]
+    static constexpr int kTiles[4][2][3][3] = {
+        {{{256, 384, 384}, {48, 96, 192}, {64, 80, 120}}, {{48, 96, 256}, {32, 64, 128}, {32, 64, 96}}},
+        {{{128, 256, 384}, {64, 128, 192}, {40, 80, 120}}, {{64, 128, 192}, {40, 80, 128}, {32, 64, 96}}},
+        {{{128, 256, 384}, {48, 96, 144}, {40, 80, 120}}, {{48, 48, 192}, {26, 32, 60}, {0, 24, 32}}},
+        {{{128, 256, 384}, {48, 96, 144}, {96, 192, 288}}, {{128, 256, 384}, {48, 96, 144}, {64, 128, 192}}}};
+    const int width = p->head_dim <= 32 ? 0 : p->head_dim <= 64 ? 1 : p->head_dim <= 96 ? 2 : 3;
+    const int64_t blocks = (e.blocks_q + e.blocks_k) / 2;
+    return kTiles[width][dropout != 0][kind][10 * blocks > 8 * e.cus ? 2 : 2 * blocks > e.cus ? 1 : 0];
 }
 
 // How a backward runs: in how many shares each kernel deals its tiles, or as one launch

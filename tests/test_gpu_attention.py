@@ -1080,6 +1080,7 @@ def test_workspace_is_what_the_plan_uses(dtype):
     (1600, 9, 80, False, "prepared", 0.1, True),
     (8192, 4, 64, True, "key", 0.1, False), (8192, 4, 80, True, "key", 0.1, True),
     (2048, 12, 96, True, "key", 0.1, False), (2048, 6, 96, True, "key", 0.1, True),
+    (1536, 18, 80, True, "prepared", 0.1, False), (2048, 12, 80, True, "prepared", 0.1, True),
 ])
 def test_long_backward_calls_are_dealt(s, h, d, causal, kind, p, dealt):
     """Two shares of the tiles against one launch: the latter up to a length that masks, dropout and the
