@@ -125,10 +125,12 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     int j_lo, j_hi;
     key_range(a, q0, min(q0 + kBM, a.sq), j_lo, j_hi);
     int bias_from = j_lo;  // keys before this one have a bias of zero
-    // Skip the tiles that hold nothing but padded keys.  (Other layouts than kBias == 2 return at once; that
-    // the builds for them contain the call measures faster, bf16 B1 S7040 H24 D32 with a [B,1,Sq,Sk] mask
-    // 793 against 815 us.)
-    if constexpr (kBias != 0) {
+    // Skip the tiles that hold nothing but padded keys.  (Other layouts than kBias == 2 return at once.  The
+    // compiler schedules their tile bodies another way where the call is there, though none spills for it:
+    // without dropout better, bf16 B2 S2048 H16 D128 with a [B,1,Sq,Sk] mask 249 against 270 us, per head 317
+    // against 351, B1 S7040 H24 D32 805 against 823; with it worse, p 0.1 causal D128 194 against 182, drawn
+    // bits D96 247 against 238, D64 228 against 222.)
+    if constexpr (kBias == 2 || (kBias != 0 && kDrop == 0)) {
         const KeyBiasSpan span =
             key_bias_span<kThreads, false>(a, b, h, j_lo, j_hi, reinterpret_cast<int*>(smem_raw));
         j_hi = span.limit, bias_from = span.zeros;
@@ -557,9 +559,10 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
         t = next;
     };
     int r = 0;
-    if constexpr (kBias == 2) {
+    if constexpr (kBias == 2 && !(DPAD == 96 && kDrop == 1)) {
         // a padding mask is zero up to the padding: no bias to add there (bf16 B8 S1024 H16 D64 causal
-        // 49.3 -> 45.8 us, without the causal mask, p 0.1 85.0 -> 78.0)
+        // 49.3 -> 45.8 us, without the causal mask, p 0.1 85.0 -> 78.0; at 65 to 96 with drawn bits a second
+        // loop costs more than it saves, B2 S2048 H16 D96 128 against 125, causal D80 101 against 98)
         const int zeros = min(order.end, bias_from / kBN) - order.begin;
         for (; r < zeros; ++r) iteration(r, std::integral_constant<int, 2>{});
     }
