@@ -132,7 +132,7 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // bits D96 247 against 238, D64 228 against 222.)
     if constexpr (kBias == 2 || (kBias != 0 && kDrop == 0)) {
         const KeyBiasSpan span =
-            key_bias_span<kThreads, false>(a, b, h, j_lo, j_hi, reinterpret_cast<int*>(smem_raw));
+            key_bias_span<kThreads, false, true>(a, b, h, j_lo, j_hi, reinterpret_cast<int*>(smem_raw));
         j_hi = span.limit, bias_from = span.zeros;
     }
     int t_lo = j_lo / kBN;

@@ -162,7 +162,7 @@ __device__ __forceinline__ void dkv_block(AttnArgs a, int block, int n_blocks) {
     if constexpr (kBias) {
         // a workgroup that owns nothing but padded keys has dK = dV = 0 (its own keys are all it looks
         // at; the whole mask took bf16 B2 S2048 H16 D128 causal 102 us instead of 92)
-        if (key_bias_span<kThreads, false>(a, b, h, k0, min(k0 + kBN, a.sk),
+        if (key_bias_span<kThreads, false, false>(a, b, h, k0, min(k0 + kBN, a.sk),
                                            reinterpret_cast<int*>(smem_raw)).hidden)
             i_hi = i_lo;
     }

@@ -459,16 +459,23 @@ __device__ __forceinline__ void query_range(const AttnArgs& a, int k_lo, int k_h
 // are read eight at a time per thread, all of them in flight together (one by one they took the forward
 // of bf16 B2 S7744 H7 D64 a twentieth of its time).
 constexpr float kMaskedBias = -30000.f;  // below fp16's most negative value, far beyond any score
+// Local windows that are worth the scan, which hides no keys there: narrower ones have too few full tiles
+// (bf16 B4 S2048 H16, window 256, with / without it: forward D64 27.7 / 26.4 us, D128 44.8 / 42.2, dQ D64 37.9 /
+// 34.7; B2 S4096 H8 D64, 1024: forward 34.3 / 35.0, dQ 39.1 / 39.9).
+constexpr int kScannedWindow = 1024;
 struct KeyBiasSpan {
     int limit, zeros;
     bool hidden;  // nothing but padded keys, which get no probability from any row
 };
 // kTyped: the bias may be of any type; the 16-bit backward kernels take fp32 only (their registers are
 // all spoken for: the selects of bias_value cost them 10 %).
-template <int THREADS, bool kTyped>
+// kZeros: whether `zeros` is wanted as well.
+template <int THREADS, bool kTyped, bool kZeros>
 __device__ __forceinline__ KeyBiasSpan key_bias_span(const AttnArgs& a, int b, int h, int j_lo, int j_hi,
                                                      int* scratch) {
-    if (!a.has_bias || a.bs[2] != 0) return {j_hi, j_lo, false};  // (a prepared one: pitch)
+    // (a prepared bias: pitch)
+    if (!a.has_bias || a.bs[2] != 0 || (a.window > 0 && (!kZeros || a.window < kScannedWindow)))
+        return {j_hi, j_lo, false};
     const int64_t row = b * a.bs[0] + h * a.bs[1];
     auto value = [&](int j) __attribute__((always_inline)) {
         if constexpr (kTyped)
@@ -491,7 +498,7 @@ __device__ __forceinline__ KeyBiasSpan key_bias_span(const AttnArgs& a, int b, i
             // (as bits: the 16-bit kernels are compiled without NaNs, and a NaN is not zero)
             const bool any = (__builtin_bit_cast(uint32_t, v[u]) & 0x7FFFFFFFu) != 0u;
             const uint64_t seen = __builtin_amdgcn_ballot_w64(in && v[u] > kMaskedBias);
-            const uint64_t set = __builtin_amdgcn_ballot_w64(in && any);
+            const uint64_t set = kZeros ? __builtin_amdgcn_ballot_w64(in && any) : 0u;
             const int first = j0 + u * THREADS + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u);
             if (seen) last = first + 63 - __builtin_clzll(seen);
             if (set) nonzero = min(nonzero, first + __builtin_ctzll(set));
@@ -503,13 +510,13 @@ __device__ __forceinline__ KeyBiasSpan key_bias_span(const AttnArgs& a, int b, i
     constexpr int kWaves = THREADS / 64;
     if ((threadIdx.x & 63) == 0) {
         scratch[threadIdx.x >> 6] = last;
-        scratch[kWaves + (threadIdx.x >> 6)] = nonzero;
+        if constexpr (kZeros) scratch[kWaves + (threadIdx.x >> 6)] = nonzero;
     }
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
         last = max(last, scratch[w]);
-        nonzero = min(nonzero, scratch[kWaves + w]);
+        if constexpr (kZeros) nonzero = min(nonzero, scratch[kWaves + w]);
     }
     __syncthreads();
     last = __builtin_amdgcn_readfirstlane(last);

@@ -656,7 +656,7 @@ attn_f32_fwd_kernel(const AttnArgs a_in) {
     extern __shared__ __align__(16) float lds[];
     const Place at(a, a.sq, kRows, true);
     const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
-                          ? key_bias_span<kFwdThreads, true>(a, at.b, at.h, 0, a.sk,
+                          ? key_bias_span<kFwdThreads, true, false>(a, at.b, at.h, 0, a.sk,
                                                              reinterpret_cast<int*>(lds)).limit
                           : a.sk;
     int j_lo, j_hi;
@@ -802,7 +802,7 @@ attn_f32_dq_kernel(const AttnArgs a_in) {
     extern __shared__ __align__(16) float lds[];
     const Place at(a, a.sq, kRows, true);
     const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
-                          ? key_bias_span<kThreads, true>(a, at.b, at.h, 0, a.sk,
+                          ? key_bias_span<kThreads, true, false>(a, at.b, at.h, 0, a.sk,
                                                           reinterpret_cast<int*>(lds)).limit
                           : a.sk;
     int j_lo, j_hi;
@@ -981,7 +981,7 @@ attn_f32_dkv_kernel(const AttnArgs a_in) {
     extern __shared__ __align__(16) float lds[];
     const Place at(a, a.sk, kRows, false);
     const int limit = (kVec ? (kMode & 1) != 0 : a.has_bias != 0)
-                          ? key_bias_span<kThreads, true>(a, at.b, at.h, 0, a.sk,
+                          ? key_bias_span<kThreads, true, false>(a, at.b, at.h, 0, a.sk,
                                                           reinterpret_cast<int*>(lds)).limit
                           : a.sk;
     int i_lo, i_hi;

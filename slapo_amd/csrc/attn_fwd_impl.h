@@ -125,7 +125,7 @@ __global__ __launch_bounds__(kThreads, kPerCu) void attn_fwd_kernel(
     key_range(a, q0, min(q0 + kRows, a.sq), j_lo, j_hi);
     int bias_from = j_lo;  // keys before this one have a bias of zero
     if constexpr (kKeyBias) {  // skip the tiles that hold nothing but padded keys
-        const KeyBiasSpan span = key_bias_span<kThreads, kBias == 4>(a, b, h, j_lo, j_hi,
+        const KeyBiasSpan span = key_bias_span<kThreads, kBias == 4, true>(a, b, h, j_lo, j_hi,
                                                                      reinterpret_cast<int*>(smem_raw));
         j_hi = span.limit, bias_from = span.zeros;
     }

@@ -646,7 +646,9 @@ def test_forward_calls_that_stay_undivided(b, s, h, d, causal, mask):
     (257, 257, 80, True, 0, 65),
     (300, 2500, 64, False, 0, 2111),  # more keys than one round of the scan reads
     (400, 400, 128, True, 0, 399),
-    (400, 400, 64, True, 130, 256),   # a window whose full tiles start behind key 0
+    (400, 400, 64, True, 130, 256),   # a window too narrow for the scan
+    (1300, 1300, 64, True, 1100, 1000),  # one whose full tiles start behind key 0
+    (1290, 1290, 128, True, 1024, 300),
     (300, 300, 32, True, 0, 300),     # zero throughout
 ])
 def test_key_bias_that_is_zero_up_to_a_key(sq, sk, d, causal, window, zeros, rest):
