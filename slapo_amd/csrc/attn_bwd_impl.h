@@ -37,15 +37,18 @@ constexpr int kKeyBlocks = kBwdKeys / 32;
 
 // kPair (head_dim 97-128 in a launch of its own): two wavefronts per 32 keys, eight a workgroup.  There the
 // K and V fragments and both accumulators of a wavefront are 192 registers, which leaves room for one
-// wavefront per SIMD, and nothing runs beside its waits; a pair needs 250 each, so two fit.  Both hold the
-// fragments; either accumulates one of dV and dK (64 registers instead of 128) and computes one half of
-// every query tile, so no product is done twice; what crosses LDS are 16-bit words that a wavefront on its
-// own would have kept (2 KB written and read per half tile beside 32 KB of operands).
-// Forward and backward, before -> after: bf16 B1 S16384 H16 D128 causal 4.65 -> 4.49 ms (the matrix pipe
-// busy 41 -> 50 % of dK/dV), B4 S2048 H16 causal 361 -> 351 us, window 256 with p 0.1 222 -> 216, B2 S1024
-// with a [B,1,Sq,Sk] mask 169.7 -> 163.2.  (The two roles as one body with selects in place of two bodies:
-// window 217, long 4.48 -> 4.55; each wavefront adding its own half first, which gives other bits than
-// the one-launch backward: 1 % less.)
+// wavefront per SIMD, and nothing runs beside its waits.  Of a pair both hold the fragments; either
+// accumulates one of dV and dK (64 registers instead of 128) and computes one half of every query tile, so
+// no product is done twice and two fit a SIMD; what crosses LDS are 16-bit words that a wavefront on its own
+// would have kept (2 KB written and read per half tile beside 32 KB of operands).
+// In 256 registers five of the sixteen builds spill nothing (without dropout, and drawn bits without a bias),
+// the others 2 to 46; all of them are faster than four wavefronts.  dK/dV alone, pair / four wavefronts, bf16 B2
+// S2048 H16 D128 causal: no bias 88 / 96 us, stored bits 88 / 98, drawn 121 / 163, any geometry 344 / 479; key mask
+// 85 / 95, 89 / 97, 121 / 167, 333 / 475; prepared bias 244 / 406, 261 / 420, 282 / 469, 506 / 811; per score 334 /
+// 565, 353 / 584, 372 / 634, 596 / 967; without the causal mask and with a window of 256 between 1.05 and 1.73.
+// Forward and backward: B1 S16384 H16 causal 4.65 -> 4.49 ms, B4 S2048 H16 causal 361 -> 351 us, window 256 with p
+// 0.1 222 -> 216.  (The two roles as one body with selects in place of two bodies: window 217, long 4.48 -> 4.55;
+// each wavefront adding its own half first, which gives other bits than the one-launch backward: 1 % less.)
 template <typename T, int DPAD, bool kPair>
 struct BwdSmem {
     static constexpr int kThreads = (kPair ? 2 : 1) * kKeyBlocks * 64;

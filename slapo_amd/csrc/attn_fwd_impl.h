@@ -57,7 +57,13 @@ constexpr size_t group_lds() {
     return (size_t)2 * group_slots(kGroups, DPAD) * kBN * (DPAD + 8) * sizeof(T) +
            (kBias == 2 || kBias == 4 ? 2 * kBN * sizeof(float) : 0);
 }
-// Workgroups per CU: two where that spills nothing.
+// Workgroups per CU: two where the second hides more than the registers cost that the build spills for it (up
+// to 26, at head_dim 65 to 96 with a key mask or bits of any geometry).  One / two per CU, bf16:
+//   two groups   D64 B1 S1024 H16 14.1 / 13.1 us; D80 S1024 H8 with a 16-bit key mask 15.3 / 14.7, B4 S512 H16 bits of
+//                any geometry 115 / 75.7; with a prepared bias D80 B2 S777 H12 causal 19.8 / 39.2; above 96 S1024 H16
+//                24.2 / 23.8, stored bits 25.8 / 27.4, with a prepared bias 36.5 / 49.0
+//   four groups  D64 S1024 H16 18.9 / 14.4, with a prepared bias and drawn bits S1024 H8 causal 16.6 / 23.8; D80 S1024
+//                H8 with a 16-bit key mask 15.7 / 26.2
 constexpr int group_per_cu(int groups, int dpad, int bias) {
     return dpad <= 32 || (groups == 4 ? dpad <= 64 && bias != 3 : dpad <= 64 || (dpad <= 96 && bias != 3))
                ? 2
