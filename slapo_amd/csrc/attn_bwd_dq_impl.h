@@ -198,13 +198,11 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // the lane (= one query).  Measured against explicit subtractions: 130 against 150 us at bf16
     // B4 S2048 H16 D128 causal, 43.5 against 45 us at fp16 B8 S1024 H16 D64; at head_dim 80 / 96
     // the 32 registers cost more than the subtractions (189 against 168 us at B4 S2048 H32 D80).
-    // Above head_dim 96 with a bias and without dropout they spill as well (14 and 28 registers; none with the
-    // subtractions): bf16 B2 S2048 H16 D128 causal 94 -> 79 us with a [B,1,1,Sk] mask, 138 -> 109 with a
-    // [B,1,Sq,Sk] one, B9 S1216 H9 D128 with that one 213 -> 169.  With stored keep bits, where only lse is
-    // in the accumulators, a launch of this kernel takes 183 us either way (B2 S2048 H16, [B,1,Sq,Sk]) and
-    // the one with dK/dV, B1 S2048 H12, 217 against 248.
-    constexpr bool kAccInit = DPAD != 96 && !(kBias == 3 && DPAD == 64 && (kDrop == 0 || kDrop == 3)) &&
-                              !((kBias == 2 || kBias == 3) && DPAD == 128 && kDrop == 0);
+    // Above head_dim 96 with a bias they spill as well (14 to 33 registers; none with the subtractions):
+    // bf16 B2 S2048 H16 D128 causal 94 -> 79 us with a [B,1,1,Sk] mask, 138 -> 109 with a [B,1,Sq,Sk]
+    // one, B9 S1216 H9 D128 with that one 213 -> 169, B4 S1024 H16, p 0.1 96 -> 88.
+    constexpr bool kAccInit = DPAD != 96 && !(kBias == 3 && DPAD >= 64 && (kDrop == 0 || kDrop == 3)) &&
+                              !(kBias == 2 && DPAD == 128 && kDrop == 0);
     f32x16_t s_init, dp_init;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
