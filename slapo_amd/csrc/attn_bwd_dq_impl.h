@@ -200,7 +200,11 @@ __device__ __forceinline__ void dq_block(AttnArgs a, int block, int n_blocks) {
     // the 32 registers cost more than the subtractions (189 against 168 us at B4 S2048 H32 D80).
     // Above head_dim 96 with a bias they spill as well (14 to 33 registers; none with the subtractions):
     // bf16 B2 S2048 H16 D128 causal 94 -> 79 us with a [B,1,1,Sk] mask, 138 -> 109 with a [B,1,Sq,Sk]
-    // one, B9 S1216 H9 D128 with that one 213 -> 169, B4 S1024 H16, p 0.1 96 -> 88.
+    // one, B9 S1216 H9 D128 with that one 213 -> 169, B4 S1024 H16, p 0.1 96 -> 88.  With a [B,1,Sq,Sk] mask
+    // and stored bits the launch together with dK/dV, which has registers to spare, would rather have the
+    // accumulators (B1 S2048 H12, p 0.1: 217 against 245 us), but rows that see fp16's lowest value at every key
+    // are closer to 64 bits with the subtractions (B4 S640 H16: 6.4e-4 against 1.6e-3), and both forms of the
+    // backward give the same bits.
     constexpr bool kAccInit = DPAD != 96 && !(kBias == 3 && DPAD >= 64 && (kDrop == 0 || kDrop == 3)) &&
                               !(kBias == 2 && DPAD == 128 && kDrop == 0);
     f32x16_t s_init, dp_init;

@@ -375,7 +375,7 @@ int one_launch_tiles(const slapo_attn_params* p, const Extent& e, BiasKind kind,
         {{{256, 384, 384}, {48, 96, 192}, {64, 80, 120}}, {{48, 96, 256}, {32, 64, 128}, {32, 64, 96}}},
         {{{128, 256, 384}, {64, 128, 192}, {40, 80, 120}}, {{64, 128, 192}, {40, 80, 128}, {32, 64, 96}}},
         {{{128, 256, 384}, {48, 96, 144}, {40, 80, 120}}, {{48, 48, 192}, {26, 32, 60}, {0, 24, 32}}},
-        {{{128, 256, 384}, {48, 96, 144}, {96, 192, 288}}, {{128, 256, 384}, {48, 96, 144}, {64, 128, 192}}}};
+        {{{128, 256, 384}, {48, 96, 144}, {96, 192, 288}}, {{128, 256, 384}, {48, 96, 144}, {40, 80, 120}}}};
     const int width = p->head_dim <= 32 ? 0 : p->head_dim <= 64 ? 1 : p->head_dim <= 96 ? 2 : 3;
     const int64_t blocks = (e.blocks_q + e.blocks_k) / 2;
     return kTiles[width][dropout != 0][kind][10 * blocks > 8 * e.cus ? 2 : 2 * blocks > e.cus ? 1 : 0];
